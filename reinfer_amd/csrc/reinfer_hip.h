@@ -75,6 +75,13 @@ int ra_act_mul_bounded(const void* gate_up, void* out, int act_dtype, int n_toke
 int ra_gemm_plain(const void* A, const void* W, const void* bias, void* C, int in_dtype, int out_dtype,
                   int M, int N, int K, int lda, int ldc, hipStream_t stream);
 
+// float operands and result on the float matrix cores, for rows that are whole 16-byte pieces (ra_gemm_f32_supports):
+// C[M, N] = A . W^T (+ bias). scratch: ra_gemm_f32_scratch floats (0: none needed).
+int ra_gemm_f32_supports(const void* A, const void* W, int K, int lda);
+long ra_gemm_f32_scratch(int M, int N, int K);
+int ra_gemm_f32(const float* A, const float* W, const float* bias, float* C, int M, int N, int K, int lda, int ldc,
+                float* scratch, long scratch_floats, hipStream_t stream);
+
 // bfloat16, M <= 64, K and lda multiples of 8: weight-streaming MFMA product.
 // epilogue 0: C[M, N] = A . W^T (+ bias); epilogue 1: W rows are gate/up interleaved in runs of 8
 // and C[M, N/2] = silu(gate) * up; epilogue 2: C is float and C += A . W^T (+ bias)

@@ -702,7 +702,8 @@ class HipKernels:
         (crates/cuda/src/gemm.rs:226-292). bfloat16 with more rows and a float
         result (the head's logits for more than 64 wanted rows): the library
         product again, bfloat16 operands and a float result.
-        Everything else, all of float32 included: the plain FMA kernel.
+        float32 whose rows are whole 16-byte pieces: this library's product on the
+        float matrix cores. Everything else: the plain FMA kernel.
         """
         if x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16:
             M, K = x.shape
@@ -723,6 +724,8 @@ class HipKernels:
                 if bias is not None:
                     out.add_(bias)
                 return
+        if x.dtype == torch.float32 and weight.dtype == torch.float32 and out.dtype == torch.float32 and x.is_cuda:
+            return self.linear_f32(x, weight, out, bias)
         self.linear_plain(x, weight, out, bias)
 
     @staticmethod
@@ -744,6 +747,17 @@ class HipKernels:
         library.call("ra_gemm_plain", x.data_ptr(), weight.data_ptr(), _ptr(bias), out.data_ptr(),
                      _tag(x, "linear input"), _tag(out, "linear output"), M, N, K, x.stride(0),
                      out.stride(0), _stream())
+
+    def linear_f32(self, x, weight, out, bias=None) -> None:
+        """The product of three float32 matrices; rows that 16-byte accesses cannot read go to the plain kernel."""
+        M, N, K = self._check_linear(x, weight, out, bias)
+        lib = library.load()
+        if not lib.ra_gemm_f32_supports(x.data_ptr(), weight.data_ptr(), K, x.stride(0)):
+            return self.linear_plain(x, weight, out, bias)
+        need = int(lib.ra_gemm_f32_scratch(M, N, K))
+        scratch = torch.empty(need, dtype=torch.float32, device=x.device) if need else None
+        library.call("ra_gemm_f32", x.data_ptr(), weight.data_ptr(), _ptr(bias), out.data_ptr(), M, N, K, x.stride(0),
+                     out.stride(0), _ptr(scratch), need, _stream())
 
     def linear_skinny(self, x, weight, out, bias=None, accumulate: bool = False, row_sums=None,
                       emit=None, wide: Optional[bool] = None, finish=None, alpha: float = 1.0):
