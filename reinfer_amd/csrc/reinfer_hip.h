@@ -5,7 +5,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
-#define RA_ABI_VERSION 25
+#define RA_ABI_VERSION 26
 
 #ifdef __cplusplus
 extern "C" {
@@ -207,9 +207,11 @@ int ra_sample_static(const float* logits, int n_rows, int vocab, int row_stride,
 // holds one record of 12 x 4 bytes per row: float temperature, top_p, min_p, repeat_penalty,
 // frequency_penalty, presence_penalty; int top_k, window_off, window_len, bias_off, bias_len, pad.
 // `window` holds the requests' recent tokens, row r's at [window_off, window_off + window_len), and
-// its logit bias as bias_len pairs (token id, float bits) from bias_off, each id once.
+// its logit bias as bias_len pairs (token id, float bits) from bias_off, each id once. scratch: ra_filter_scratch bytes on
+// a 16-byte boundary, read and written by this call alone.
+long ra_filter_scratch(int n_rows, int vocab);
 int ra_filter_logits(float* logits, int n_rows, int vocab, int row_stride, const void* rows,
-                     const int* window, hipStream_t stream);
+                     const int* window, void* scratch, long scratch_bytes, hipStream_t stream);
 
 // What the machine gives at best (peaks.hip; for measurement, not on the product path): one read of
 // `bytes` of device memory, and `iters` iterations of bfloat16 matrix-core products on registers

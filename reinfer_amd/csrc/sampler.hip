@@ -206,35 +206,49 @@ extern "C" int ra_sample_static(const float* logits, int n_rows, int vocab, int 
 //     sum_{kept, p >= theta} p >= top_p * (mass kept so far)
 //   (order and boundary rules: sampler_kernel.cu:20-43, 287-372). Removed
 //   tokens get -inf; ra_sample then applies the temperature and draws.
-// One workgroup per row; counts and sums are reduced in a fixed order.
+//
+// A row is cut into slices, a workgroup each, and passes over it follow one another as launches:
+//   1  bias and penalties of the slice's tokens, the slice's maximum of x = logit / T;
+//   2  how many of its tokens, and how much of their mass e = exp(x - max x), fall into each of 512 bins a sixteenth wide
+//      below the maximum (mass as whole numbers, so that sums do not depend on their order);
+//   3  one workgroup a row adds the slices' bins: the bin in which the k-th largest lies, and the few in which the mass
+//      reaches top_p's share, are then known;
+//   4  the tokens of those bins, some dozens to hundreds, are listed;
+//   5  one workgroup a row finds the exact boundaries among them;
+//   6  every slice removes what lies below.
+// One workgroup a row that bisected over the whole row, up to 94 passes, took 3.15 ms for 24 rows of 151936 however many
+// rows there were; the six launches take 73 us for them, each bound by its own start and one trip over the row (the two
+// with one workgroup a row 9 and 21 us).
 // ---------------------------------------------------------------------------
-#define FILTER_THREADS 1024
+#define FILTER_THREADS 256
+#define FILTER_SLICE 4096
+#define FILTER_BINS 512
+#define FILTER_BINS_A_UNIT 16.f
+#define FILTER_ROW_THREADS 1024
+#define FILTER_SHORT 2048        // listed tokens up to which every one is ranked against all others
 
 __device__ __forceinline__ unsigned sortable(float v) {      // ascending order of floats as unsigned
   const unsigned b = __float_as_uint(v);
   return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
 }
+// (value, lower id first) as one number
+__device__ __forceinline__ unsigned long long filter_key(int v, float x) {
+  return ((unsigned long long)sortable(x) << 32) | (unsigned)(~v);
+}
+__device__ __forceinline__ int filter_bin(float x, float mx) {
+  return (int)fminf((mx - x) * FILTER_BINS_A_UNIT, (float)(FILTER_BINS - 1));
+}
 
-template <typename T>
-__device__ __forceinline__ T filter_block_sum(T v, T* red) {
+// Sum over FILTER_ROW_THREADS threads; `red` is LDS for a number a wave.
+__device__ __forceinline__ unsigned long long filter_row_sum(unsigned long long v, unsigned long long* red) {
 #pragma unroll
   for (int m = RA_WAVE / 2; m > 0; m >>= 1) v += __shfl_xor(v, m, RA_WAVE);
   const int lane = threadIdx.x & (RA_WAVE - 1), wave = threadIdx.x / RA_WAVE;
   __syncthreads();
   if (lane == 0) red[wave] = v;
   __syncthreads();
-  T t = 0;
-  for (int i = 0; i < FILTER_THREADS / RA_WAVE; ++i) t += red[i];
-  return t;
-}
-__device__ __forceinline__ float filter_block_max(float v, float* red) {
-  v = wave_max(v);
-  const int lane = threadIdx.x & (RA_WAVE - 1), wave = threadIdx.x / RA_WAVE;
-  __syncthreads();
-  if (lane == 0) red[wave] = v;
-  __syncthreads();
-  float t = -INFINITY;
-  for (int i = 0; i < FILTER_THREADS / RA_WAVE; ++i) t = fmaxf(t, red[i]);
+  unsigned long long t = 0;
+  for (int i = 0; i < FILTER_ROW_THREADS / RA_WAVE; ++i) t += red[i];
   return t;
 }
 
@@ -245,22 +259,33 @@ struct FilterRow {           // one per row, in device memory
   int pad;
 };
 
-__global__ void __launch_bounds__(FILTER_THREADS)
-filter_logits_kernel(float* __restrict__ logits, int vocab, int row_stride, const FilterRow* __restrict__ rows,
-                     const int* __restrict__ window) {
-  __shared__ float redf[FILTER_THREADS / RA_WAVE];
-  __shared__ unsigned long long redu[FILTER_THREADS / RA_WAVE];
-  const FilterRow fr = rows[blockIdx.x];
-  float* lg = logits + (size_t)blockIdx.x * row_stride;
-  const int tid = threadIdx.x;
+// What the passes know of a row. A token is kept if e >= e_min, e >= theta and key >= key_min.
+struct FilterPlan {
+  unsigned long long key_min, mass, mass_before_k, mass_before_p;
+  float mx, e_min, theta;
+  int bin_k, rank_k;           // the k-th largest is number rank_k (from 1) of bin_k; bin_k -1: no such filter
+  int bin_p0, bin_p1;          // top_p's boundary lies in one of these bins; bin_p0 -1: no such filter
+  unsigned listed;
+};
 
+__device__ __forceinline__ bool filter_uses(const FilterRow& fr, int vocab) {
+  return fr.temperature > 0.f && ((fr.top_k > 0 && fr.top_k < vocab) || (fr.top_p > 0.f && fr.top_p < 1.f) || fr.min_p > 0.f);
+}
+
+__global__ void __launch_bounds__(FILTER_THREADS)
+filter_max_kernel(float* __restrict__ logits, int vocab, int row_stride, const FilterRow* __restrict__ rows,
+                  const int* __restrict__ window, float* __restrict__ slice_max) {
+  __shared__ float red[FILTER_THREADS / RA_WAVE];
+  const FilterRow fr = rows[blockIdx.y];
+  float* lg = logits + (size_t)blockIdx.y * row_stride;
+  const int tid = threadIdx.x, from = blockIdx.x * FILTER_SLICE, to = min(vocab, from + FILTER_SLICE);
   // additive bias per token id, before everything else (crates/cuda/kernels/sampler_kernel.cu:189-203);
   // the caller lists every id once
   if (fr.bias_len > 0) {
     const int* bp = window + fr.bias_off;
     for (int b = tid; b < fr.bias_len; b += FILTER_THREADS) {
       const int tok = bp[2 * b];
-      if (tok < 0 || tok >= vocab) continue;
+      if (tok < from || tok >= to) continue;
       const float l = lg[tok];
       if (isfinite(l)) lg[tok] = l + __int_as_float(bp[2 * b + 1]);
     }
@@ -272,7 +297,7 @@ filter_logits_kernel(float* __restrict__ logits, int vocab, int row_stride, cons
     const int* win = window + fr.window_off;
     for (int w = tid; w < fr.window_len; w += FILTER_THREADS) {
       const int tok = win[w];
-      if (tok < 0 || tok >= vocab) continue;
+      if (tok < from || tok >= to) continue;
       bool first = true;
       int cnt = 0;
       for (int x = 0; x < fr.window_len; ++x) {
@@ -290,80 +315,324 @@ filter_logits_kernel(float* __restrict__ logits, int vocab, int row_stride, cons
     }
     __syncthreads();
   }
-  const float T = fr.temperature;
-  const bool use_k = fr.top_k > 0 && fr.top_k < vocab;
-  const bool use_p = fr.top_p > 0.f && fr.top_p < 1.f;
-  const bool use_m = fr.min_p > 0.f;
-  if (!(T > 0.f) || !(use_k || use_p || use_m)) return;
-
-  // x = logit / T; e = exp(x - max x) = p / max p
+  if (!filter_uses(fr, vocab)) return;
   float mx = -INFINITY;
-  for (int v = tid; v < vocab; v += FILTER_THREADS) {
+  for (int v = from + tid; v < to; v += FILTER_THREADS) {
     const float l = lg[v];
-    if (isfinite(l)) mx = fmaxf(mx, l / T);
+    if (isfinite(l)) mx = fmaxf(mx, l / fr.temperature);
   }
-  mx = filter_block_max(mx, redf);
-  if (mx == -INFINITY) return;               // no finite logit: ra_sample reports it
-  // what is kept so far is described by two thresholds: e >= e_min and key >= key_min
-  float e_min = use_m ? fr.min_p : 0.f;      // min_p: p >= min_p * max p  <=>  e >= min_p
-  unsigned long long key_min = 0ull;
-  auto key_of = [&](int v, float x) { return ((unsigned long long)sortable(x) << 32) | (unsigned)(~v); };
-  if (use_k) {
-    // the k-th largest (value, lower id first) pair by bisection on the 64-bit key
-    unsigned long long lo = 0ull, hi = ~0ull;           // count(key >= lo) >= k > count(key >= hi)
-    for (int round = 0; round < 64 && hi - lo > 1ull; ++round) {
-      const unsigned long long mid = lo + (hi - lo) / 2ull;
-      unsigned long long c = 0ull;
-      for (int v = tid; v < vocab; v += FILTER_THREADS) {
-        const float l = lg[v];
-        if (isfinite(l) && key_of(v, l / T) >= mid) ++c;
-      }
-      c = filter_block_sum<unsigned long long>(c, redu);
-      if (c >= (unsigned long long)fr.top_k) lo = mid; else hi = mid;
-    }
-    key_min = lo;
-  }
-  float theta = 0.f;                          // top_p boundary on e
-  if (use_p) {
-    float zs = 0.f;
-    for (int v = tid; v < vocab; v += FILTER_THREADS) {
-      const float l = lg[v];
-      if (!isfinite(l)) continue;
-      const float x = l / T, e = __expf(x - mx);
-      if (e >= e_min && key_of(v, x) >= key_min) zs += e;
-    }
-    zs = filter_block_sum<float>(zs, redf);
-    const float need = fr.top_p * zs;
-    float flo = 0.f, fhi = 1.f;               // mass(e >= flo) >= need; e <= 1 always
-    for (int round = 0; round < 30; ++round) {
-      const float mid = 0.5f * (flo + fhi);
-      float mass = 0.f;
-      for (int v = tid; v < vocab; v += FILTER_THREADS) {
-        const float l = lg[v];
-        if (!isfinite(l)) continue;
-        const float x = l / T, e = __expf(x - mx);
-        if (e >= mid && e >= e_min && key_of(v, x) >= key_min) mass += e;
-      }
-      mass = filter_block_sum<float>(mass, redf);
-      if (mass >= need) flo = mid; else fhi = mid;
-    }
-    theta = flo;
-  }
-  for (int v = tid; v < vocab; v += FILTER_THREADS) {
-    const float l = lg[v];
-    if (!isfinite(l)) continue;
-    const float x = l / T, e = __expf(x - mx);
-    if (!(e >= e_min && e >= theta && key_of(v, x) >= key_min)) lg[v] = -INFINITY;
+  mx = wave_max(mx);
+  if ((tid & (RA_WAVE - 1)) == 0) red[tid / RA_WAVE] = mx;
+  __syncthreads();
+  if (tid == 0) {
+    for (int i = 1; i < FILTER_THREADS / RA_WAVE; ++i) mx = fmaxf(mx, red[i]);
+    slice_max[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = mx;
   }
 }
 
+// every thread gets the row's maximum
+__device__ __forceinline__ float filter_row_max(const float* slice_max, int slices) {
+  float mx = -INFINITY;
+  for (int i = threadIdx.x & (RA_WAVE - 1); i < slices; i += RA_WAVE) mx = fmaxf(mx, slice_max[i]);
+  return wave_max(mx);
+}
+
+__global__ void __launch_bounds__(FILTER_THREADS)
+filter_bins_kernel(const float* __restrict__ logits, int vocab, int row_stride, const FilterRow* __restrict__ rows,
+                   const float* __restrict__ slice_max, unsigned long long* __restrict__ mass,
+                   unsigned* __restrict__ count, float unit) {
+  __shared__ unsigned long long m[FILTER_BINS];
+  __shared__ unsigned c[FILTER_BINS];
+  const FilterRow fr = rows[blockIdx.y];
+  if (!filter_uses(fr, vocab)) return;
+  const float* lg = logits + (size_t)blockIdx.y * row_stride;
+  const int tid = threadIdx.x, from = blockIdx.x * FILTER_SLICE, to = min(vocab, from + FILTER_SLICE);
+  const float mx = filter_row_max(slice_max + (size_t)blockIdx.y * gridDim.x, gridDim.x);
+  if (mx == -INFINITY) return;               // no finite logit: ra_sample reports it
+  const float e_min = fr.min_p > 0.f ? fr.min_p : 0.f;
+  for (int b = tid; b < FILTER_BINS; b += FILTER_THREADS) {
+    m[b] = 0ull;
+    c[b] = 0u;
+  }
+  __syncthreads();
+  for (int v = from + tid; v < to; v += FILTER_THREADS) {
+    const float l = lg[v];
+    if (!isfinite(l)) continue;
+    const float x = l / fr.temperature, e = __expf(x - mx);
+    const int b = filter_bin(x, mx);
+    atomicAdd(&c[b], 1u);
+    if (e >= e_min) atomicAdd(&m[b], (unsigned long long)(e * unit));
+  }
+  __syncthreads();
+  const size_t at = ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * FILTER_BINS;
+  for (int b = tid; b < FILTER_BINS; b += FILTER_THREADS) {
+    mass[at + b] = m[b];
+    count[at + b] = c[b];
+  }
+}
+
+// One workgroup of FILTER_BINS threads a row.
+__global__ void __launch_bounds__(FILTER_BINS)
+filter_plan_kernel(int vocab, const FilterRow* __restrict__ rows, const float* __restrict__ slice_max, int slices,
+                   const unsigned long long* __restrict__ mass, const unsigned* __restrict__ count,
+                   FilterPlan* __restrict__ plans) {
+  __shared__ unsigned long long m[FILTER_BINS];
+  __shared__ unsigned c[FILTER_BINS];
+  __shared__ FilterPlan plan;
+  const FilterRow fr = rows[blockIdx.x];
+  const int b = threadIdx.x;
+  const float mx = filter_uses(fr, vocab) ? filter_row_max(slice_max + (size_t)blockIdx.x * slices, slices) : -INFINITY;
+  if (mx == -INFINITY) {                     // nothing to remove
+    if (b == 0) plans[blockIdx.x].mx = mx;
+    return;
+  }
+  unsigned long long ms = 0ull;
+  unsigned cs = 0u;
+  const size_t at = (size_t)blockIdx.x * slices * FILTER_BINS + b;
+#pragma unroll 8
+  for (int i = 0; i < slices; ++i) {
+    ms += mass[at + (size_t)i * FILTER_BINS];
+    cs += count[at + (size_t)i * FILTER_BINS];
+  }
+  m[b] = ms;
+  c[b] = cs;
+  if (b == 0) plan = {0ull, 0ull, 0ull, 0ull, mx, fr.min_p > 0.f ? fr.min_p : 0.f, 0.f, -1, 0, -1, -1, 0u};
+  __syncthreads();
+  for (int d = 1; d < FILTER_BINS; d <<= 1) {            // m, c: of this bin and all above it
+    const unsigned long long mo = b >= d ? m[b - d] : 0ull;
+    const unsigned co = b >= d ? c[b - d] : 0u;
+    __syncthreads();
+    m[b] += mo;
+    c[b] += co;
+    __syncthreads();
+  }
+  const unsigned k = (unsigned)fr.top_k;
+  const unsigned long long mb = b ? m[b - 1] : 0ull;
+  const unsigned cb = b ? c[b - 1] : 0u;
+  if (fr.top_k > 0 && k < c[FILTER_BINS - 1] && cb < k && k <= c[b]) {
+    plan.bin_k = b;
+    plan.rank_k = (int)(k - cb);
+    plan.mass_before_k = mb;
+  }
+  __syncthreads();
+  if (fr.top_p > 0.f && fr.top_p < 1.f) {
+    // the mass left by top_k lies between these two, and with it what the boundary's bin must reach
+    const int bk = plan.bin_k;
+    const double p = (double)fr.top_p;
+    const double least = p * (double)(bk >= 0 ? plan.mass_before_k : m[FILTER_BINS - 1]);
+    const double most = p * (double)(bk >= 0 ? m[bk] : m[FILTER_BINS - 1]);
+    if ((b == 0 || (double)mb < least) && (double)m[b] >= least) {
+      plan.bin_p0 = b;
+      plan.mass_before_p = mb;
+    }
+    if ((b == 0 || (double)mb < most) && (double)m[b] >= most) plan.bin_p1 = b;
+    if (b == 0) plan.mass = m[FILTER_BINS - 1];
+  }
+  __syncthreads();
+  if (b == 0) plans[blockIdx.x] = plan;
+}
+
+__global__ void __launch_bounds__(FILTER_THREADS)
+filter_list_kernel(const float* __restrict__ logits, int vocab, int row_stride, const FilterRow* __restrict__ rows,
+                   FilterPlan* __restrict__ plans, int* __restrict__ list) {
+  __shared__ unsigned found, base;
+  __shared__ int mine[FILTER_SLICE];
+  const FilterPlan p = plans[blockIdx.y];
+  if (p.mx == -INFINITY || (p.bin_k < 0 && p.bin_p0 < 0)) return;
+  const float* lg = logits + (size_t)blockIdx.y * row_stride;
+  const float T = rows[blockIdx.y].temperature;
+  const int tid = threadIdx.x, from = blockIdx.x * FILTER_SLICE, to = min(vocab, from + FILTER_SLICE);
+  if (tid == 0) found = 0u;
+  __syncthreads();
+  for (int v = from + tid; v < to; v += FILTER_THREADS) {
+    const float l = lg[v];
+    if (!isfinite(l)) continue;
+    const int b = filter_bin(l / T, p.mx);
+    if (b == p.bin_k || (p.bin_p0 >= 0 && b >= p.bin_p0 && b <= p.bin_p1)) mine[atomicAdd(&found, 1u)] = v;
+  }
+  __syncthreads();
+  if (found == 0u) return;
+  if (tid == 0) base = atomicAdd(&plans[blockIdx.y].listed, found);
+  __syncthreads();
+  for (unsigned i = tid; i < found; i += FILTER_THREADS) list[(size_t)blockIdx.y * vocab + base + i] = mine[i];
+}
+
+// One workgroup a row: the boundaries among the listed tokens, whose order on the list means nothing.
+__global__ void __launch_bounds__(FILTER_ROW_THREADS)
+filter_select_kernel(const float* __restrict__ logits, int vocab, int row_stride, const FilterRow* __restrict__ rows,
+                     FilterPlan* __restrict__ plans, const int* __restrict__ list, float unit) {
+  __shared__ unsigned long long red[FILTER_ROW_THREADS / RA_WAVE];
+  __shared__ unsigned long long keys[FILTER_SHORT], masses[FILTER_SHORT];
+  __shared__ float es[FILTER_SHORT];
+  __shared__ short bins[FILTER_SHORT];
+  __shared__ unsigned long long key_min;
+  __shared__ unsigned theta_bits;
+  const FilterPlan p = plans[blockIdx.x];
+  if (p.mx == -INFINITY || (p.bin_k < 0 && p.bin_p0 < 0)) return;
+  const FilterRow fr = rows[blockIdx.x];
+  const float* lg = logits + (size_t)blockIdx.x * row_stride;
+  const int* mine = list + (size_t)blockIdx.x * vocab;
+  const int tid = threadIdx.x, n = (int)p.listed;
+  const bool is_short = n <= FILTER_SHORT;
+  struct Item {
+    unsigned long long key, mass;
+    float e;
+    int bin;
+  };
+  auto read = [&](int i) {                   // listed token i, from memory
+    const int v = mine[i];
+    const float x = lg[v] / fr.temperature, e = __expf(x - p.mx);
+    return Item{filter_key(v, x), e >= p.e_min ? (unsigned long long)(e * unit) : 0ull, e, filter_bin(x, p.mx)};
+  };
+  if (tid == 0) {
+    key_min = 0ull;
+    theta_bits = 0u;
+  }
+  if (is_short)
+    for (int i = tid; i < n; i += FILTER_ROW_THREADS) {
+      const Item it = read(i);
+      keys[i] = it.key;
+      masses[i] = it.mass;
+      es[i] = it.e;
+      bins[i] = (short)it.bin;
+    }
+  __syncthreads();
+  if (p.bin_k >= 0) {
+    if (is_short) {
+      for (int i = tid; i < n; i += FILTER_ROW_THREADS) {
+        if (bins[i] != p.bin_k) continue;
+        int above = 0;
+        for (int j = 0; j < n; ++j) above += bins[j] == p.bin_k && keys[j] > keys[i];
+        if (above == p.rank_k - 1) key_min = keys[i];      // keys differ: one thread
+      }
+    } else {
+      unsigned long long lo = 0ull, hi = ~0ull;            // count(key >= lo) >= rank > count(key >= hi)
+      while (hi - lo > 1ull) {
+        const unsigned long long mid = lo + (hi - lo) / 2ull;
+        unsigned long long c = 0ull;
+        for (int i = tid; i < n; i += FILTER_ROW_THREADS) {
+          const Item it = read(i);
+          c += it.bin == p.bin_k && it.key >= mid;
+        }
+        if (filter_row_sum(c, red) >= (unsigned long long)p.rank_k) lo = mid; else hi = mid;
+      }
+      if (tid == 0) key_min = lo;
+    }
+    __syncthreads();
+  }
+  if (p.bin_p0 >= 0) {
+    const unsigned long long kmin = key_min;
+    unsigned long long left = p.mass;                      // the mass that top_k and min_p leave
+    if (p.bin_k >= 0) {
+      unsigned long long s = 0ull;
+      for (int i = tid; i < n; i += FILTER_ROW_THREADS) {
+        const Item it = is_short ? Item{keys[i], masses[i], es[i], bins[i]} : read(i);
+        if (it.bin == p.bin_k && it.key >= kmin) s += it.mass;
+      }
+      left = p.mass_before_k + filter_row_sum(s, red);
+    }
+    const double need = (double)fr.top_p * (double)left;
+    auto counts = [&](int bin, unsigned long long key) { return bin >= p.bin_p0 && bin <= p.bin_p1 && key >= kmin; };
+    if (is_short) {
+      for (int i = tid; i < n; i += FILTER_ROW_THREADS) {
+        if (!counts(bins[i], keys[i]) || es[i] < p.e_min) continue;
+        unsigned long long s = p.mass_before_p;
+        for (int j = 0; j < n; ++j) s += es[j] >= es[i] && counts(bins[j], keys[j]) ? masses[j] : 0ull;
+        if ((double)s >= need) atomicMax(&theta_bits, __float_as_uint(es[i]));
+      }
+    } else {
+      unsigned lo = 0u, hi = 0x3F800001u;                  // mass(e >= lo) >= need > mass(e >= hi); e is at most 1
+      while (hi - lo > 1u) {
+        const unsigned mid = lo + (hi - lo) / 2u;
+        unsigned long long s = 0ull;
+        for (int i = tid; i < n; i += FILTER_ROW_THREADS) {
+          const Item it = read(i);
+          if (counts(it.bin, it.key) && __float_as_uint(it.e) >= mid) s += it.mass;
+        }
+        if ((double)(p.mass_before_p + filter_row_sum(s, red)) >= need) lo = mid; else hi = mid;
+      }
+      if (tid == 0) theta_bits = lo;
+    }
+    __syncthreads();
+  }
+  if (tid == 0) {
+    plans[blockIdx.x].key_min = key_min;
+    plans[blockIdx.x].theta = __uint_as_float(theta_bits);
+  }
+}
+
+__global__ void __launch_bounds__(FILTER_THREADS)
+filter_remove_kernel(float* __restrict__ logits, int vocab, int row_stride, const FilterRow* __restrict__ rows,
+                     const FilterPlan* __restrict__ plans) {
+  const FilterPlan p = plans[blockIdx.y];
+  if (p.mx == -INFINITY) return;
+  float* lg = logits + (size_t)blockIdx.y * row_stride;
+  const float T = rows[blockIdx.y].temperature;
+  const int from = blockIdx.x * FILTER_SLICE, to = min(vocab, from + FILTER_SLICE);
+  for (int v = from + threadIdx.x; v < to; v += FILTER_THREADS) {
+    const float l = lg[v];
+    if (!isfinite(l)) continue;
+    const float x = l / T, e = __expf(x - p.mx);
+    if (!(e >= p.e_min && e >= p.theta && filter_key(v, x) >= p.key_min)) lg[v] = -INFINITY;
+  }
+}
+
+// Scratch of a call, in the order of its parts: plans, the slices' bins (mass, count), their maxima, the lists.
+static size_t filter_parts(int n_rows, int vocab, size_t (&off)[5]) {
+  const size_t slices = (vocab + FILTER_SLICE - 1) / FILTER_SLICE, n = (size_t)n_rows;
+  const size_t bytes[5] = {n * sizeof(FilterPlan), n * slices * FILTER_BINS * 8, n * slices * FILTER_BINS * 4,
+                           n * slices * 4, n * (size_t)vocab * 4};
+  size_t at = 0;
+  for (int i = 0; i < 5; ++i) {
+    off[i] = at;
+    at += (bytes[i] + 15) / 16 * 16;
+  }
+  return at;
+}
+
+extern "C" long ra_filter_scratch(int n_rows, int vocab) {
+  size_t off[5];
+  return n_rows > 0 && vocab > 0 ? (long)filter_parts(n_rows, vocab, off) : 0;
+}
+
 extern "C" int ra_filter_logits(float* logits, int n_rows, int vocab, int row_stride, const void* rows,
-                                const int* window, hipStream_t stream) {
+                                const int* window, void* scratch, long scratch_bytes, hipStream_t stream) {
   RA_CHECK(n_rows > 0 && vocab > 0, "filter_logits: empty input (%d rows, vocabulary %d)", n_rows, vocab);
   RA_CHECK(row_stride >= vocab, "filter_logits: row stride %d below the vocabulary %d", row_stride, vocab);
   RA_CHECK(n_rows <= 65535, "filter_logits: %d rows in one launch (max 65535)", n_rows);
   RA_CHECK(rows != nullptr, "filter_logits: no row parameters");
-  filter_logits_kernel<<<n_rows, FILTER_THREADS, 0, stream>>>(logits, vocab, row_stride, (const FilterRow*)rows, window);
-  RA_LAUNCH_CHECK("filter_logits");
+  size_t off[5];
+  const size_t need = filter_parts(n_rows, vocab, off);
+  RA_CHECK(scratch != nullptr && scratch_bytes >= (long)need && (uintptr_t)scratch % 16 == 0,
+           "filter_logits: scratch of %ld bytes, needs %zu on a 16-byte boundary", scratch_bytes, need);
+  char* s = (char*)scratch;
+  FilterPlan* plans = (FilterPlan*)(s + off[0]);
+  unsigned long long* mass = (unsigned long long*)(s + off[1]);
+  unsigned* count = (unsigned*)(s + off[2]);
+  float* slice_max = (float*)(s + off[3]);
+  int* list = (int*)(s + off[4]);
+  const FilterRow* fr = (const FilterRow*)rows;
+  const int slices = (vocab + FILTER_SLICE - 1) / FILTER_SLICE;
+  // e = 1 in whole numbers: a whole row of ones stays below 2^63
+  float unit = 1.f;
+  for (int bits = 62, v = vocab; bits > 0; --bits, v >>= 1)
+    if (v <= 1) {
+      unit = (float)(1ull << bits);
+      break;
+    }
+  unit *= 0.5f;
+  const dim3 grid(slices, n_rows);
+  filter_max_kernel<<<grid, FILTER_THREADS, 0, stream>>>(logits, vocab, row_stride, fr, window, slice_max);
+  RA_LAUNCH_CHECK("filter_logits (maximum)");
+  filter_bins_kernel<<<grid, FILTER_THREADS, 0, stream>>>(logits, vocab, row_stride, fr, slice_max, mass, count, unit);
+  RA_LAUNCH_CHECK("filter_logits (bins)");
+  filter_plan_kernel<<<n_rows, FILTER_BINS, 0, stream>>>(vocab, fr, slice_max, slices, mass, count, plans);
+  RA_LAUNCH_CHECK("filter_logits (plan)");
+  filter_list_kernel<<<grid, FILTER_THREADS, 0, stream>>>(logits, vocab, row_stride, fr, plans, list);
+  RA_LAUNCH_CHECK("filter_logits (list)");
+  filter_select_kernel<<<n_rows, FILTER_ROW_THREADS, 0, stream>>>(logits, vocab, row_stride, fr, plans, list, unit);
+  RA_LAUNCH_CHECK("filter_logits (boundaries)");
+  filter_remove_kernel<<<grid, FILTER_THREADS, 0, stream>>>(logits, vocab, row_stride, fr, plans);
+  RA_LAUNCH_CHECK("filter_logits (removal)");
   return 0;
 }

@@ -15,7 +15,7 @@ import torch  # noqa: F401  (loads the HIP runtime the library links against)
 
 from ..csrc import build as _build
 
-ABI_VERSION = 25
+ABI_VERSION = 26
 
 
 class KernelLibraryError(RuntimeError):
@@ -49,7 +49,7 @@ _SIGNATURES = {
     "ra_gemm_f32": [P, P, P, P, I, I, I, I, I, P, c_long, P],
     "ra_sample": [P, I, I, I, P, P, P, P, P, P, P],
     "ra_sample_static": [P, I, I, I, P, P, P, P, P],
-    "ra_filter_logits": [P, I, I, I, P, P, P],
+    "ra_filter_logits": [P, I, I, I, P, P, P, c_long, P],
     "ra_pair_hash_add": [P, P, I, P, P, P, P, P, P, I, c_longlong, c_longlong, I, I, P],
     "ra_stream_add": [P, P, I, P, P, I, I, I, F, P],
     "ra_tanh_cap": [P, I, I, I, F, P],
@@ -129,6 +129,8 @@ def load() -> ctypes.CDLL:
             getattr(lib, name).argtypes = [c_int, c_int, c_int]
         lib.ra_attention_prefill_part_floats.restype = c_long
         lib.ra_attention_prefill_part_floats.argtypes = [c_int, c_int, c_int, c_int, c_int]
+        lib.ra_filter_scratch.restype = c_long
+        lib.ra_filter_scratch.argtypes = [I, I]
         lib.ra_sample_static_max_pairs.restype = c_long
         lib.ra_sample_static_max_pairs.argtypes = []
         lib.ra_sample_static_prepare.restype = c_int

@@ -1791,8 +1791,10 @@ class HipKernels:
                 off += 2 * len(bias)
         rows_t = torch.from_numpy(rec).to(logits.device)
         win_t = torch.tensor(window or [0], dtype=torch.int32).to(logits.device)
+        need = int(library.load().ra_filter_scratch(n, V))
+        scratch = torch.empty(need, dtype=torch.uint8, device=logits.device)
         library.call("ra_filter_logits", logits.data_ptr(), n, V, logits.stride(0), rows_t.data_ptr(),
-                     win_t.data_ptr(), _stream())
+                     win_t.data_ptr(), scratch.data_ptr(), need, _stream())
 
     # ------------------------------------------------------------ measurement
     def measure_peaks(self, device="cuda:0", read_bytes: int = 4 << 30) -> dict:

@@ -1,0 +1,59 @@
+"""The filters' boundaries where their slices, bins and lists end, against the plain chain."""
+import pytest
+import torch
+
+import plain_qwen3 as plain
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def filtered(rows, params):
+    from reinfer_amd import kernels
+    from reinfer_amd.sampling import SamplingParams
+    logits = torch.stack(rows).to(DEV)
+    kernels.current().filter_logits(logits, [SamplingParams(**p) for p in params], [[1, 2, 3]] * len(rows))
+    return logits.cpu()
+
+
+FILTERS = [dict(temperature=0.7, top_k=1), dict(temperature=1.0, top_k=300), dict(temperature=0.9, top_p=0.9),
+           dict(temperature=1.0, top_k=40, top_p=0.7), dict(temperature=1.2, top_k=2000, top_p=0.99, min_p=1e-3),
+           dict(temperature=0.5, min_p=0.2), dict(temperature=1.0, top_k=10 ** 6), dict(temperature=1.0)]
+
+
+@pytest.mark.parametrize("V", [1, 63, 4095, 4096, 4097, 12289])
+@pytest.mark.parametrize("spread", [0.01, 1.0, 40.0])     # one bin, a bell over many, most beyond the last
+def test_filters_at_the_edges_of_slices_and_bins(V, spread):
+    g = torch.Generator().manual_seed(V)
+    # values a clear step apart, in a random order: no boundary hangs on the last bit
+    row = (torch.linspace(-3.0, 3.0, V) * spread)[torch.randperm(V, generator=g)]
+    got = filtered([row] * len(FILTERS), FILTERS)
+    for i, f in enumerate(FILTERS):
+        kw = {k: v for k, v in f.items() if k != "temperature"}
+        kept = torch.isfinite(plain.filter_logits(row, f["temperature"], **kw))
+        mine = torch.isfinite(got[i])
+        assert torch.equal(got[i][mine], row[mine])
+        if f.get("top_p") and spread < 1.0:
+            # neighbours' shares of the mass differ by less than the rounding of their exponentials (a few units of 2^-24
+            # each): the boundary may lie that share of the row further
+            assert abs(int(mine.sum()) - int(kept.sum())) <= 1 + V * 2.0 ** -20, (i, int(mine.sum()), int(kept.sum()))
+            assert row[mine].min() > row[~mine].max() if (~mine).any() else True
+        else:
+            assert torch.equal(kept, mine), (i, int(kept.sum()), int(mine.sum()))
+
+
+def test_filters_over_equal_logits_and_rows_with_few_finite_ones():
+    V = 10000
+    equal = torch.full((V,), 1.5)
+    few = torch.full((V,), float("-inf"))
+    few[[7, 4096, 9999]] = torch.tensor([1.0, 3.0, 2.0])
+    few[11] = float("nan")
+    none = torch.full((V,), float("nan"))
+    got = filtered([equal, equal, few, few, none],
+                   [dict(temperature=1.0, top_k=5000), dict(temperature=1.0, top_p=0.4), dict(temperature=1.0, top_k=2),
+                    dict(temperature=1.0, top_k=50, top_p=0.6), dict(temperature=1.0, top_k=3, top_p=0.5)])
+    assert torch.isfinite(got[0]).nonzero()[:, 0].tolist() == list(range(5000))      # the lower id first among equals
+    assert torch.isfinite(got[1]).all()                                              # ties at the boundary all stay
+    assert torch.isfinite(got[2]).nonzero()[:, 0].tolist() == [4096, 9999]
+    assert torch.isfinite(got[3]).nonzero()[:, 0].tolist() == [4096]                 # 0.67 of the mass
+    assert not torch.isfinite(got[4]).any()
