@@ -75,6 +75,17 @@ int ra_act_mul_bounded(const void* gate_up, void* out, int act_dtype, int n_toke
 int ra_gemm_plain(const void* A, const void* W, const void* bias, void* C, int in_dtype, int out_dtype,
                   int M, int N, int K, int lda, int ldc, hipStream_t stream);
 
+// Experts over tokens sorted by expert (bfloat16; moe_grouped.hip): w_up [experts ff, width], with a gate [2 experts ff,
+// width] an expert's gate rows before its up rows, w_down [width, ld_down] an expert's ff columns side by side, ids and
+// weights [n_tokens, top] (an id of `experts` or more: its weight times the token's row). more (float [n_tokens, width], or
+// null) is added, times sigmoid(more_logit[t * ld_logit]) where that is given. Exactly one of resid (float, += alpha times
+// the sum) and out (bfloat16). scratch: ra_moe_grouped_scratch bytes on a 256-byte boundary.
+long ra_moe_grouped_scratch(int n_tokens, int top, int experts, int ff, int width);
+int ra_moe_grouped(const void* x, int ldx, const void* w_up, const void* w_down, int ld_down, const int* ids,
+                   const float* weights, int top, int experts, int ff, int gated, int n_tokens, int width,
+                   const float* more, const float* more_logit, int ld_logit, float* resid, void* out, float alpha,
+                   void* scratch, long scratch_bytes, hipStream_t stream);
+
 // float operands and result on the float matrix cores, for rows that are whole 16-byte pieces (ra_gemm_f32_supports):
 // C[M, N] = A . W^T (+ bias). scratch: ra_gemm_f32_scratch floats (0: none needed).
 int ra_gemm_f32_supports(const void* A, const void* W, int K, int lda);

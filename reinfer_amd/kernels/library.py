@@ -46,6 +46,7 @@ _SIGNATURES = {
     "ra_gemm_skinny_scaled": [P, P, P, I, I, I, I, I, F, P],
     "ra_gemm_wide_scaled": [P, P, P, I, I, I, I, I, P, c_long, F, P],
     "ra_gemm_plain": [P, P, P, P, I, I, I, I, I, I, I, P],
+    "ra_moe_grouped": [P, I, P, P, I, P, P, I, I, I, I, I, I, P, P, I, P, P, F, P, c_long, P],
     "ra_gemm_f32": [P, P, P, P, I, I, I, I, I, P, c_long, P],
     "ra_sample": [P, I, I, I, P, P, P, P, P, P, P],
     "ra_sample_static": [P, I, I, I, P, P, P, P, P],
@@ -139,6 +140,8 @@ def load() -> ctypes.CDLL:
         lib.ra_chunk_scratch_floats.argtypes = [c_int, c_int, c_int, c_int, c_int]
         lib.ra_scan_state_floats.restype = c_long
         lib.ra_scan_state_floats.argtypes = [c_int, c_int, c_int, c_int]
+        lib.ra_moe_grouped_scratch.restype = c_long
+        lib.ra_moe_grouped_scratch.argtypes = [I, I, I, I, I]
         lib.ra_gemm_f32_supports.restype = c_int
         lib.ra_gemm_f32_supports.argtypes = [P, P, I, I]
         lib.ra_gemm_f32_scratch.restype = c_long

@@ -1646,6 +1646,57 @@ class HipKernels:
         ``moe_down_chosen``): its token-expert pairs are few against the experts there are."""
         return n_tokens <= self.MOE_CHOSEN_TOKENS and n_tokens * top <= self.MOE_CHOSEN_SHARE * experts
 
+    # Rows from which a token's rows meet its chosen experts alone, its pairs sorted by expert, and the share of the
+    # experts that a token may choose at most for that. Up to 64 rows the products that read every expert once are bound by
+    # those reads in either form; with half of the experts chosen the products over all of them, at twice the rate, cost
+    # the same.
+    MOE_GROUPED_FROM = 65
+    MOE_GROUPED_SHARE = 0.4
+
+    def moe_groups(self, x: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor, top: int, experts: int, ff: int) -> bool:
+        """Whether a step over the rows ``x`` should go through :meth:`moe_grouped`."""
+        T, width = x.shape
+        return self.MOE_GROUPED_FROM <= T <= 65535 and top <= self.MOE_GROUPED_SHARE * experts and experts <= 4096 \
+            and T * top <= 1 << 24 and x.is_cuda and x.dtype == w_up.dtype == w_down.dtype == torch.bfloat16 \
+            and width % 8 == 0 and ff % 8 == 0 and w_down.stride(0) % 8 == 0 and x.stride(0) % 8 == 0 and x.stride(1) == 1 \
+            and all(t.data_ptr() % 16 == 0 for t in (x, w_up, w_down))
+
+    def moe_grouped(self, x: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor, ids: torch.Tensor,
+                    weights: torch.Tensor, experts: int, ff: int, gated: bool, more: Optional[torch.Tensor] = None,
+                    more_logit: Optional[torch.Tensor] = None, resid: Optional[torch.Tensor] = None, alpha: float = 1.0,
+                    out: Optional[torch.Tensor] = None) -> None:
+        """y[t] = sum_j weights[t, j] * (expert ids[t, j] of x[t]) (an id of ``experts`` or more stands for x[t] itself)
+        + ``more``[t] (float32, times sigmoid(more_logit[t]) where that is given); resid += alpha * y, or out = y in
+        bfloat16. An expert is W_down relu(W_up x)^2, or ``gated`` W_down (silu(W_gate x) * (W_up x)). ``w_up`` holds
+        [experts * ff] rows, gated [gate; up] an expert, ``w_down`` [width, at least experts * ff] an expert's columns side
+        by side; rows of either behind the experts' are not read."""
+        _dev(x, w_up, w_down, ids, weights, more, more_logit, resid, out)
+        T, width = x.shape
+        top = ids.shape[1]
+        n_up = (2 if gated else 1) * experts * ff
+        if w_up.dim() != 2 or w_up.shape[0] < n_up or w_up.shape[1] != width or not w_up.is_contiguous() \
+                or w_down.dim() != 2 or w_down.shape[0] != width or w_down.shape[1] < experts * ff or w_down.stride(1) != 1:
+            raise ValueError(f"moe_grouped: x {tuple(x.shape)}, up {tuple(w_up.shape)}, down {tuple(w_down.shape)} for "
+                             f"{experts} experts of {ff}")
+        self._check_choice("moe_grouped", ids, weights, T, top)
+        if more is not None and (more.dtype != torch.float32 or more.shape != (T, width) or not more.is_contiguous()):
+            raise ValueError(f"moe_grouped: the rows to add are contiguous float32 [{T}, {width}]")
+        if more_logit is not None and (more is None or more_logit.dtype != torch.float32 or more_logit.shape[0] != T
+                                       or more_logit.numel() != T):
+            raise ValueError("moe_grouped: the logits of the rows to add are float32, one a token")
+        if (resid is None) == (out is None):
+            raise ValueError("moe_grouped: the result goes into the stream or into out")
+        if resid is not None and (resid.shape != (T, width) or resid.dtype != torch.float32 or not resid.is_contiguous()):
+            raise ValueError("moe_grouped: the residual stream is contiguous float32 [T, width]")
+        if out is not None and (out.shape != (T, width) or out.dtype != torch.bfloat16 or not out.is_contiguous()):
+            raise ValueError("moe_grouped: out is contiguous bfloat16 [T, width]")
+        need = int(library.load().ra_moe_grouped_scratch(T, top, int(experts), int(ff), width))
+        scratch = torch.empty(need, dtype=torch.uint8, device=x.device)
+        library.call("ra_moe_grouped", x.data_ptr(), x.stride(0), w_up.data_ptr(), w_down.data_ptr(), w_down.stride(0),
+                     ids.data_ptr(), weights.data_ptr(), top, int(experts), int(ff), 1 if gated else 0, T, width, _ptr(more),
+                     _ptr(more_logit), more_logit.stride(0) if more_logit is not None else 0, _ptr(resid), _ptr(out),
+                     float(alpha), scratch.data_ptr(), need, _stream())
+
     def moe_up_chosen(self, x: torch.Tensor, w_up: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor,
                       act: torch.Tensor, ff: int) -> None:
         """act[t * top + j] = weights[t, j] * relu(w_up[ids[t, j] * ff : ... + ff] . x[t])^2 for the chosen

@@ -10,7 +10,8 @@ applies the activation and the routing weight in one kernel (0 for experts a tok
 product with the down matrix is then the weighted sum: with few experts of which a good share is chosen, two
 dense products at the matrix cores' rate cost less than gathering tokens by expert would. A step of so few
 tokens that most experts are not asked for at all (one or two requests decoding) reads only the chosen experts'
-rows instead, a wave a row.
+rows instead, a wave a row; a step of more than 64 tokens sorts its token-expert pairs by expert on the device and
+runs each expert over its own.
 
 A second form of the same part (``activation`` "silu_gated", ``weights`` "sigmoid"): an expert is
 W_down (silu(W_gate h) * (W_up h)); a token's score for expert e is sigmoid(z_e); where the experts form
@@ -128,6 +129,8 @@ class MixtureOfExperts:
                 downs.append(weights[prefix + "shared.down"])
             self.w_gate_up = torch.cat(rows, dim=0).contiguous()       # [2 (E ff + shared), width]
             self.w_down = torch.cat(downs, dim=1).contiguous()          # [width, E ff + shared]
+            # the shared expert's columns by themselves, for steps whose tokens go through their own experts alone
+            self.w_shared_down = downs[-1].contiguous() if self.shared else None
             return
         self.w_up = torch.cat([weights[f"{prefix}e{e}.up"] for e in range(self.experts)], dim=0).contiguous()
         self.w_down = torch.cat([weights[f"{prefix}e{e}.down"] for e in range(self.experts)], dim=1).contiguous()
@@ -162,6 +165,9 @@ class MixtureOfExperts:
             out = torch.empty((T, self.spec.hidden), dtype=self.dtype, device=x.device)
             ops.moe_down_gated_chosen(act, self.w_down, ids, weights, x, out, self.experts, self.ff, self.shared)
             return out
+        groups = getattr(ops, "moe_groups", None)
+        if groups is not None and groups(x, self.w_gate_up, self.w_down, self.top, self.experts, self.ff):
+            return self._forward_grouped(ops, x, self.w_gate_up, ids, weights, shared_logit, resid, resid_scale)
         gu = torch.empty((T, 2 * n), dtype=self.dtype, device=x.device)
         ops.linear(x, self.w_gate_up, gu)
         act = torch.empty((T, n), dtype=self.dtype, device=x.device)
@@ -186,6 +192,23 @@ class MixtureOfExperts:
         ops.linear(act, self.w_down, out)
         return out
 
+    def _forward_grouped(self, ops, x, w_up, ids, weights, shared_logit, resid, resid_scale):
+        """Many tokens: each through its chosen experts alone. The shared expert runs over all of them beside, its result
+        kept in float until the sum."""
+        T, width = x.shape
+        more = None
+        if self.gated and self.shared:
+            gu = torch.empty((T, 2 * self.shared), dtype=self.dtype, device=x.device)
+            ops.linear(x, w_up[2 * self.experts * self.ff:], gu)
+            act = torch.empty((T, self.shared), dtype=self.dtype, device=x.device)
+            ops.silu_mul(gu, act)
+            more = torch.empty((T, width), dtype=torch.float32, device=x.device)
+            ops.linear(act, self.w_shared_down, more)
+        out = None if resid is not None else torch.empty((T, width), dtype=self.dtype, device=x.device)
+        ops.moe_grouped(x, w_up, self.w_down, ids, weights, self.experts, self.ff, self.gated, more=more,
+                        more_logit=shared_logit if more is not None else None, resid=resid, alpha=resid_scale, out=out)
+        return out
+
     def forward(self, x, batch, resid: Optional[torch.Tensor] = None, resid_scale: float = 1.0):
         if self.gated:
             return self._forward_gated(x, resid, resid_scale, batch)
@@ -208,6 +231,9 @@ class MixtureOfExperts:
             out = torch.empty((T, self.spec.hidden), dtype=self.dtype, device=x.device)
             ops.moe_down_chosen(act, self.w_down, ids, self.ff, out=out)
             return out
+        groups = getattr(ops, "moe_groups", None)
+        if groups is not None and groups(x, self.w_up, self.w_down, self.top, self.experts, self.ff):
+            return self._forward_grouped(ops, x, self.w_up, ids, weights, None, resid, 1.0)
         up = torch.empty((T, n), dtype=self.dtype, device=x.device)
         ops.linear(x, self.w_up, up)
         act = torch.empty((T, n), dtype=self.dtype, device=x.device)

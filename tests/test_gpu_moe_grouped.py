@@ -1,0 +1,68 @@
+"""Experts over sorted tokens against a plain sum over every token's choices."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def ops():
+    from reinfer_amd import kernels
+    return kernels.current()
+
+
+def choices(kind, T, E, top, g):
+    if kind == "spread":
+        return torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(T)])
+    if kind == "one":                        # every token the same experts, the others none: full tiles and empty experts
+        return torch.arange(top).expand(T, top).clone()
+    ids = torch.stack([torch.randperm(E + 2, generator=g)[:top] for _ in range(T)])      # "identity": ids past the experts
+    ids[0] = E
+    return ids
+
+
+# slots of an expert on both sides of a tile of 128; k and weight rows that end inside a step and a tile, rows in steps of
+# 8 alone; both tile widths (256 needs two tiles a CU)
+@pytest.mark.parametrize("T,E,top,ff,width", [(65, 5, 2, 40, 72), (127, 3, 1, 64, 128), (128, 3, 1, 72, 264),
+                                              (129, 3, 1, 136, 64), (400, 9, 3, 24, 200), (1500, 16, 4, 264, 4104)])
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("kind", ["spread", "one", "identity"])
+def test_experts_over_sorted_tokens(T, E, top, ff, width, gated, kind):
+    g = torch.Generator().manual_seed(T + ff)
+    G = torch.Generator(device=DEV).manual_seed(T + ff)
+    shared = 16
+    x = torch.randn(T, width + 8, generator=G, device=DEV).bfloat16()[:, :width]
+    n_up = 2 if gated else 1
+    w_up = (torch.randn(n_up * (E * ff + shared), width, generator=G, device=DEV) / width ** 0.5).bfloat16()
+    w_down = (torch.randn(width, E * ff + shared, generator=G, device=DEV) / ff ** 0.5).bfloat16()
+    ids = choices(kind, T, E, top, g).to(torch.int32).to(DEV).contiguous()
+    wts = torch.rand(T, top, generator=G, device=DEV)
+    more = torch.randn(T, width, generator=G, device=DEV) if gated else None
+    logit = torch.randn(T, 3, generator=G, device=DEV)[:, 1] if gated else None
+    assert top > 0.4 * E or ops().moe_groups(x, w_up, w_down, top, E, ff)
+    want = torch.zeros(T, width, dtype=torch.float64, device=DEV)
+    size = torch.zeros_like(want)            # of the terms, for the bound
+    xd = x.double()
+    for e in range(E):
+        rows = (ids == e).any(-1).nonzero()[:, 0]
+        p = (wts * (ids == e)).sum(-1)[rows, None].double()
+        u = w_up[n_up * e * ff:n_up * (e + 1) * ff].double()
+        a = torch.nn.functional.silu(xd[rows] @ u[:ff].t()) * (xd[rows] @ u[ff:].t()) if gated else \
+            torch.relu(xd[rows] @ u.t()) ** 2
+        d = w_down[:, e * ff:(e + 1) * ff].double().t()
+        want[rows] += (p * a) @ d
+        size[rows] += (p * a).abs() @ d.abs()
+    same = (wts * (ids >= E)).sum(-1, keepdim=True).double()
+    want += same * xd
+    size += same * xd.abs()
+    if more is not None:
+        want += more.double() * torch.sigmoid(logit[:, None].double())
+    # the activation is rounded once to bfloat16 (2^-9 of each term at most); float sums stay far below that
+    bound = 2.0 ** -8 * size + 1e-4
+    out = torch.full((T, width), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops().moe_grouped(x, w_up, w_down, ids, wts, E, ff, gated, more=more, more_logit=logit, out=out)
+    assert ((out.double() - want).abs() <= bound + 2.0 ** -8 * want.abs()).all()
+    resid = torch.randn(T, width, generator=G, device=DEV)
+    base = resid.double()
+    ops().moe_grouped(x, w_up, w_down, ids, wts, E, ff, gated, more=more, more_logit=logit, resid=resid, alpha=0.5)
+    assert ((resid.double() - (base + 0.5 * want)).abs() <= bound).all()
