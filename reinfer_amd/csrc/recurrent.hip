@@ -707,7 +707,8 @@ extern "C" int ra_matrix_memory_scan(const void* proj, int act_dtype, int ld, in
                                      long slot_stride,
                                      const int* cu_tokens, const int* state_slots, const int* fresh, int n_seqs,
                                      int n_tokens, int max_q_len, int heads, int key_dim, int value_dim,
-                                     float gate_cap, float q_scale, float denom_eps, float* out, hipStream_t stream) {
+                                     float gate_cap, float q_scale, float denom_eps, float* scratch, long scratch_floats,
+                                     float* out, hipStream_t stream) {
   RA_CHECK(n_seqs > 0 && n_tokens > 0 && heads > 0, "matrix_memory_scan: %d requests, %d tokens, %d heads", n_seqs,
            n_tokens, heads);
   ScanGeom g;
@@ -722,6 +723,10 @@ extern "C" int ra_matrix_memory_scan(const void* proj, int act_dtype, int ld, in
       gates, gate_bias, gate_cap, gates3, state, slot_stride, (long)g.waves * g.wave_floats,
       (long)g.NPL * RA_WAVE + (long)g.NPL * g.R, cu_tokens, state_slots, fresh, heads);
   RA_LAUNCH_CHECK("matrix_memory_gates");
+  if (scratch)
+    return ra_matrix_memory_chunks(proj, act_dtype, ld, q_off, k_off, v_off, gates3, state, slot_stride, cu_tokens, state_slots,
+                                   fresh, n_seqs, n_tokens, heads, key_dim, value_dim, q_scale, denom_eps, scratch,
+                                   scratch_floats, out, stream);
   const ScanLaunch L = scan_launch(g, n_seqs, heads, max_q_len);
   const size_t es = act_dtype == RA_F32 ? 4 : 2;
   ScanArgs a = {};
@@ -774,7 +779,8 @@ extern "C" int ra_delta_rule_prepare(const void* proj, int act_dtype, int ld, co
 extern "C" int ra_delta_rule_scan(const float* qkv, int ld, float* gates, const float* a_log, const float* dt_bias,
                                   float* state, long slot_stride, const int* cu_tokens, const int* state_slots,
                                   const int* fresh, int n_seqs, int n_tokens, int max_q_len, int heads, int key_heads,
-                                  int key_dim, int value_dim, float* out, hipStream_t stream) {
+                                  int key_dim, int value_dim, float* scratch, long scratch_floats, float* out,
+                                  hipStream_t stream) {
   RA_CHECK(n_seqs > 0 && n_tokens > 0 && heads > 0 && key_heads > 0 && heads % key_heads == 0,
            "delta_rule_scan: %d requests, %d tokens, %d heads on %d key heads", n_seqs, n_tokens, heads, key_heads);
   ScanGeom g;
@@ -785,6 +791,9 @@ extern "C" int ra_delta_rule_scan(const float* qkv, int ld, float* gates, const 
   const long n = (long)n_tokens * 2 * heads;
   delta_rule_gates_kernel<<<(unsigned)((n + 255) / 256), 256, 0, stream>>>(gates, a_log, dt_bias, heads, n);
   RA_LAUNCH_CHECK("delta_rule_gates");
+  if (scratch)
+    return ra_delta_rule_chunks(qkv, ld, gates, state, slot_stride, cu_tokens, state_slots, fresh, n_seqs, n_tokens, heads,
+                                key_heads, key_dim, value_dim, scratch, scratch_floats, out, stream);
   const ScanLaunch L = scan_launch(g, n_seqs, heads, max_q_len);
   ScanArgs a = {};
   a.q = qkv;

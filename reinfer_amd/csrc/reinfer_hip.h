@@ -355,7 +355,7 @@ int ra_gla_scan(const void* proj, int act_dtype, int ld, int q_off, int k_off, i
                 int value_dim, float* out, hipStream_t stream);
 // The same recurrences (silu: ra_decay_scan's) in chunks of 16 tokens on the float matrix cores, keys up to 256, from and
 // into the same state. Scratch: ra_chunk_scratch_floats(...) floats, 16-byte aligned.
-long ra_chunk_scratch_floats(int n_tokens, int n_seqs, int heads, int key_dim, int value_dim);
+long ra_chunk_scratch_floats(int kind, int n_tokens, int n_seqs, int heads, int key_dim, int value_dim);
 int ra_decay_chunks(const void* proj, int act_dtype, int ld, int q_off, int k_off, int v_off, int silu, const float* decays,
                     const int* positions, const float* inv_freq, int rot_dims, float q_scale, float k_scale, float* state,
                     long slot_stride, const int* cu_tokens, const int* state_slots, const int* fresh, int n_seqs,
@@ -382,8 +382,8 @@ long ra_scan_state_floats(int kind, int heads, int key_dim, int value_dim);
 int ra_matrix_memory_scan(const void* proj, int act_dtype, int ld, int q_off, int k_off, int v_off, const float* gates,
                           float* gates3, const float* gate_bias, float* state, long slot_stride, const int* cu_tokens,
                           const int* state_slots, const int* fresh, int n_seqs, int n_tokens, int max_q_len, int heads,
-                          int key_dim, int value_dim, float gate_cap, float q_scale, float denom_eps, float* out,
-                          hipStream_t stream);
+                          int key_dim, int value_dim, float gate_cap, float q_scale, float denom_eps, float* scratch,
+                          long scratch_floats, float* out, hipStream_t stream);
 // proj rows hold q | k (key_heads x key_dim each) | v (heads x value_dim) from column 0; filt float [channels, taps];
 // the filter's tail lies at tail_off floats in a request's state slot; qkv float [n_tokens, channels]
 int ra_delta_rule_prepare(const void* proj, int act_dtype, int ld, const float* filt, float* state, long slot_stride,
@@ -393,8 +393,8 @@ int ra_delta_rule_prepare(const void* proj, int act_dtype, int ld, const float* 
 // gates [n_tokens, 2 heads] float pre-activations (b | a), turned into (beta | decay) in place
 int ra_delta_rule_scan(const float* qkv, int ld, float* gates, const float* a_log, const float* dt_bias, float* state,
                        long slot_stride, const int* cu_tokens, const int* state_slots, const int* fresh, int n_seqs,
-                       int n_tokens, int max_q_len, int heads, int key_heads, int key_dim, int value_dim, float* out,
-                       hipStream_t stream);
+                       int n_tokens, int max_q_len, int heads, int key_heads, int key_dim, int value_dim, float* scratch,
+                       long scratch_floats, float* out, hipStream_t stream);
 // kind 2 of ra_scan_state_floats. proj rows hold r, k and v (heads x dim each) at the given column offsets; decay
 // float [n_tokens, >= heads dim] holds the decays' pre-activations z, the decay being exp(-exp(z + w0)); u float
 // [heads dim] is the bonus of the current token: o = (S + diag(u) k v^T)^T r, then S <- diag(decay) S + k v^T

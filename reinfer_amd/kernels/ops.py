@@ -1113,11 +1113,12 @@ class HipKernels:
     def matrix_memory_scan(self, proj: torch.Tensor, q_off: int, k_off: int, v_off: int, gates: torch.Tensor,
                            gate_bias: torch.Tensor, state: torch.Tensor, batch, heads: int, key_dim: int,
                            value_dim: int, gate_cap: float, q_scale: float, denom_eps: float,
-                           out: torch.Tensor) -> None:
+                           out: torch.Tensor, chunks: Optional[bool] = None) -> None:
         """The matrix memory over the step's tokens, request by request in order, from and into ``state``
         [slots, floats]. ``proj`` [T, *] holds q and k (heads x key_dim) and v (heads x value_dim) from the
         given columns; ``gates`` float32 [T, 2 heads] holds the input and forget gates' pre-activations;
-        ``out`` float32 [T, heads * value_dim] gets the read-out before its norm."""
+        ``out`` float32 [T, heads * value_dim] gets the read-out before its norm. ``chunks`` forces the form (None: by the
+        step's longest portion)."""
         _dev(proj, gates, gate_bias, state, out)
         T = proj.shape[0]
         self._check_scan("matrix_memory_scan", state, batch, T)
@@ -1130,12 +1131,14 @@ class HipKernels:
         if out.shape != (T, heads * value_dim) or out.dtype != torch.float32 or not out.is_contiguous():
             raise ValueError("matrix_memory_scan: out is contiguous float32 [T, heads * value_dim]")
         factors = torch.empty((T, 3 * heads), dtype=torch.float32, device=proj.device)     # decay, input, threshold
+        scratch = self._scan_scratch(chunks, "matrix_memory", batch, T, heads, key_dim, value_dim, proj.device)
         library.call("ra_matrix_memory_scan", proj.data_ptr(), _tag(proj, "matrix_memory_scan"), proj.stride(0),
                      int(q_off), int(k_off), int(v_off), gates.data_ptr(), factors.data_ptr(), gate_bias.data_ptr(),
                      state.data_ptr(),
                      state.stride(0), batch.cu_tokens.data_ptr(), batch.state_slots.data_ptr(), batch.fresh.data_ptr(),
                      batch.num_seqs, T, int(getattr(batch, "max_q_len", 0) or 0), int(heads), int(key_dim),
-                     int(value_dim), float(gate_cap), float(q_scale), float(denom_eps), out.data_ptr(), _stream())
+                     int(value_dim), float(gate_cap), float(q_scale), float(denom_eps), _ptr(scratch),
+                     scratch.numel() if scratch is not None else 0, out.data_ptr(), _stream())
 
     def delta_rule_prepare(self, proj: torch.Tensor, filt: torch.Tensor, state: torch.Tensor, tail_off: int, batch,
                            key_heads: int, key_dim: int, heads: int, value_dim: int, taps: int, unit_eps: float,
@@ -1164,7 +1167,7 @@ class HipKernels:
 
     def delta_rule_scan(self, qkv: torch.Tensor, gates: torch.Tensor, a_log: torch.Tensor, dt_bias: torch.Tensor,
                         state: torch.Tensor, batch, heads: int, key_heads: int, key_dim: int, value_dim: int,
-                        out: torch.Tensor) -> None:
+                        out: torch.Tensor, chunks: Optional[bool] = None) -> None:
         """The gated delta rule over the step's tokens from and into ``state``. ``qkv`` float32 [T, q | k | v]
         as ``delta_rule_prepare`` left it; ``gates`` float32 [T, 2 heads] holds the pre-activations of beta
         and of the decay and is overwritten with both; ``out`` float32 [T, heads * value_dim]."""
@@ -1181,11 +1184,12 @@ class HipKernels:
                 raise ValueError(f"delta_rule_scan: {what} is float32 [heads]")
         if out.shape != (T, heads * value_dim) or out.dtype != torch.float32 or not out.is_contiguous():
             raise ValueError("delta_rule_scan: out is contiguous float32 [T, heads * value_dim]")
+        scratch = self._scan_scratch(chunks, "delta_rule", batch, T, heads, key_dim, value_dim, qkv.device)
         library.call("ra_delta_rule_scan", qkv.data_ptr(), qkv.stride(0), gates.data_ptr(), a_log.data_ptr(),
                      dt_bias.data_ptr(), state.data_ptr(), state.stride(0), batch.cu_tokens.data_ptr(),
                      batch.state_slots.data_ptr(), batch.fresh.data_ptr(), batch.num_seqs, T,
                      int(getattr(batch, "max_q_len", 0) or 0), int(heads), int(key_heads), int(key_dim), int(value_dim),
-                     out.data_ptr(), _stream())
+                     _ptr(scratch), scratch.numel() if scratch is not None else 0, out.data_ptr(), _stream())
 
     def wkv_scan(self, proj: torch.Tensor, r_off: int, k_off: int, v_off: int, decay: torch.Tensor, w0: torch.Tensor,
                  u: torch.Tensor, state: torch.Tensor, batch, heads: int, dim: int, out: torch.Tensor) -> None:
@@ -1385,9 +1389,15 @@ class HipKernels:
         if out.shape != (T, heads * value_dim) or out.dtype != torch.float32 or not out.is_contiguous():
             raise ValueError(f"{what}: out is contiguous float32 [T, {heads * value_dim}]")
 
-    @staticmethod
-    def _chunk_scratch(T, n_seqs, heads, key_dim, value_dim, device) -> torch.Tensor:
-        n = int(library.load().ra_chunk_scratch_floats(T, n_seqs, int(heads), int(key_dim), int(value_dim)))
+    def _scan_scratch(self, chunks, kind: str, batch, T: int, heads: int, key_dim: int, value_dim: int, device):
+        """Scratch for a scan of ``kind`` in chunks, or None where it goes token by token."""
+        if chunks is None:
+            chunks = int(getattr(batch, "max_q_len", 0) or 0) >= self.CHUNK_FROM and key_dim <= self.CHUNK_KEYS
+        return self._chunk_scratch(T, batch.num_seqs, heads, key_dim, value_dim, device, kind) if chunks else None
+
+    @classmethod
+    def _chunk_scratch(cls, T, n_seqs, heads, key_dim, value_dim, device, kind: str = "decay_memory") -> torch.Tensor:
+        n = int(library.load().ra_chunk_scratch_floats(cls._SCAN_KINDS[kind], T, n_seqs, int(heads), int(key_dim), int(value_dim)))
         if n < 0:
             raise ValueError(f"heads of {key_dim} x {value_dim} are not taken in chunks (keys up to 256)")
         return torch.empty(n, dtype=torch.float32, device=device)
