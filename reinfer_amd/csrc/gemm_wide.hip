@@ -15,9 +15,8 @@
 //
 // Where N gives too few workgroups of 128 features to fill the chip, K is cut into S ranges
 // (grid.y); each writes its float partial result and a second kernel adds them in range order
-// and applies the epilogue: deterministic, no atomics. In that form only, the kernel also takes 65 to
-// 128 rows (six or eight row tiles): a product over a long K that adds into the residual stream is
-// faster so than the library's product followed by the add. Epilogues as in gemm_skinny.hip: plain
+// and applies the epilogue: deterministic, no atomics. Products of 65 to 512 rows that gemm_tile.hip
+// takes come through the same entry points and adding kernels. Epilogues as in gemm_skinny.hip: plain
 // (+ bias), SiLU gate over interleaved gate/up rows (S = 1 only), C += (float).
 //
 // An RMSNorm can ride on these products as on gemm_skinny's (y = rstd[m] * ((x .* w) . W^T)): the
@@ -26,6 +25,7 @@
 // the adding kernel, which such a product then always runs: one partial sum per row and 1024 columns.
 #include "common.h"
 #include "reinfer_hip.h"
+#include "gemm_tile.h"
 
 enum { WEPI_PLAIN = 0, WEPI_SILU_PAIRS = 1, WEPI_ACCUM = 2, WEPI_PARTIAL = 3 };
 
@@ -408,6 +408,17 @@ gemm_wide_reduce_rows_kernel(const float* __restrict__ P, int S, const bf16_t* _
 // give one workgroup a CU or fewer, each range a multiple of the run.
 static void gw_split(int epilogue, int M, int N, int K, int* waves, int* S, int* k_per_split, bool* partial = nullptr,
                      bool emits = false) {
+  if (M > 64) {                                        // gemm_tile.hip's: a gated product is not cut
+    *waves = 4;
+    if (epilogue == WEPI_SILU_PAIRS) {
+      *S = 1;
+      *k_per_split = K;
+    } else {
+      ra_tile_plan(M, N, K, S, k_per_split);
+    }
+    if (partial) *partial = epilogue != WEPI_SILU_PAIRS;
+    return;
+  }
   if (partial) *partial = emits;                       // the adding kernel writes what the next norm needs
   const int cus = ra_cu_count(), fill = cus - cus / 4;  // workgroups that keep the chip busy: three quarters of its CUs
   const int cb8 = (N + 127) / 128;
@@ -453,19 +464,16 @@ static void gw_split(int epilogue, int M, int N, int K, int* waves, int* S, int*
 // except a small product whose K has to be cut (4096 x 4096: the second launch costs more than the
 // shared activations save); from 9 rows for the gated product of a wide feed-forward.
 extern "C" int ra_gemm_wide_preferred(int epilogue, int M, int N, int K) {
-  if (M < 1 || M > 128) return 0;
+  if (M < 1) return 0;
+  // 65 to 128 rows: what adds into the residual stream, cut into ranges, because the norm that follows can ride on it
+  // (the other products of these rows are offered by ra_gemm_tile_takes)
+  if (M > 64) return M <= 128 && epilogue == WEPI_ACCUM ? ra_gemm_tile_takes(epilogue, M, N, K) : 0;
   int waves, S, kps;
   gw_split(epilogue, M, N, K, &waves, &S, &kps);
   // sizes are priced a CU: a product is "large" where every CU has more than 128 KiB of weights to stream
   // (on 256 CUs: more than 4096 x 4096 bfloat16)
   const int cus = ra_cu_count(), fill = cus - cus / 4;
   const bool large = (long)N * K * 2 > 131072L * cus;
-  // 65 to 128 rows: the library's products are as fast or faster (151936 x 4096 at 128 rows: 285 us against
-  // 400) but for a product that adds into the residual stream over a long K, which this kernel cuts into
-  // ranges (4096 x 12288 at 96 / 128 rows: 37 / 43 us against 59 / 70 for the library's product and the add)
-  // (and from exactly 128 KiB a CU on: 4096 x 4096 at 96 / 128 rows 19.7 / 22.0 us with the adding kernel, which
-  // also does the add, against 17.2 / 19.3 for the library's product, whose result the norm kernel then adds)
-  if (M > 64) return (epilogue == WEPI_ACCUM && S > 1 && (long)N * K * 2 >= 131072L * cus) ? 1 : 0;
   // from 9 to 16 rows the gated product of a wide feed-forward (up to 8 rows the other kernel, whose
   // workgroups stay and keep two runs a wave in flight, is ahead: 24576 x 4096 36 us against 37, 51200 x
   // 5120 91 to 97 against 101 to 103): one K range, enough workgroups to fill the
@@ -515,20 +523,6 @@ static int launch_wide_reduce(const void* bias, void* C, int ldc, int out_dtype,
   return 0;
 }
 
-// 65 to 128 rows: only as K ranges and the adding kernel (six or eight row tiles, workgroups of eight waves)
-template <int MT>
-static int launch_wide_ranges(const void* A, int lda, const void* W, const void* bias, void* C, int ldc, int out_dtype,
-                              int epilogue, int M, int N, int K, int S, int kps, float* scratch, const WideNorm& nf,
-                              hipStream_t stream) {
-  RA_CHECK(((size_t)(M - 1) * lda + K) * 2 < 0x7FFFFF00ull && (size_t)128 * K * 2 < 0x7FFFFF00ull,
-           "gemm_wide: rows of %d (stride %d) are too long for this kernel", K, lda);
-  const WideNorm none = {};
-  gemm_wide_kernel<MT, 8, WEPI_PARTIAL, float><<<dim3((N + 127) / 128, S), 8 * RA_WAVE, 0, stream>>>(
-      (const bf16_t*)A, lda, (const bf16_t*)W, nullptr, scratch, N, M, N, K, kps, none);
-  RA_LAUNCH_CHECK("gemm_wide");
-  return launch_wide_reduce(bias, C, ldc, out_dtype, epilogue, M, N, S, scratch, nf, stream);
-}
-
 template <int MT, int WV>
 static int launch_wide(const void* A, int lda, const void* W, const void* bias, void* C, int ldc, int out_dtype,
                        int epilogue, int M, int N, int K, int S, int kps, bool partial, float* scratch,
@@ -566,7 +560,8 @@ static int gemm_wide_impl(const void* A, const void* W, const void* bias, void* 
                           int in_width, const void* out_w, int out_w_dtype, void* out_x, int out_ldx,
                           float* out_ss, float out_eps, float acc_scale, hipStream_t stream) {
   RA_CHECK(M > 0 && N > 0 && K > 0, "gemm_wide: empty product (%d, %d, %d)", M, N, K);
-  RA_CHECK(M <= 128, "gemm_wide: %d rows; this kernel takes at most 128", M);
+  RA_CHECK(M <= 128 || ra_gemm_tile_takes(epilogue, M, N, K),
+           "gemm_wide: %d rows; at most 128, or 512 where the tiled product is ahead", M);
   RA_CHECK(K % 8 == 0 && lda % 8 == 0, "gemm_wide: K (%d) and the row stride (%d) must be multiples of 8", K, lda);
   RA_CHECK(epilogue == WEPI_PLAIN || epilogue == WEPI_SILU_PAIRS || epilogue == WEPI_ACCUM,
            "gemm_wide: unknown epilogue %d", epilogue);
@@ -611,10 +606,13 @@ static int gemm_wide_impl(const void* A, const void* W, const void* bias, void* 
   bool partial;
   gw_split(epilogue, M, N, K, &waves, &S, &kps, &partial, emits);
   if (M > 64) {
-    RA_CHECK(partial && epilogue != WEPI_SILU_PAIRS,
-             "gemm_wide: with %d rows only a product that is cut into K ranges (64 rows otherwise)", M);
-    if (M <= 96) return launch_wide_ranges<6>(A, lda, W, bias, C, ldc, out_dtype, epilogue, M, N, K, S, kps, scratch, nf, stream);
-    return launch_wide_ranges<8>(A, lda, W, bias, C, ldc, out_dtype, epilogue, M, N, K, S, kps, scratch, nf, stream);
+    if (!partial) {
+      RA_CHECK(!in_ss && out_dtype == RA_BF16 && ra_gemm_tile_takes(epilogue, M, N, K),
+               "gemm_wide: with %d rows a gated product only where its tiles fill the chip, with a bfloat16 result and no norm", M);
+      return ra_tile_gated(A, lda, W, C, ldc, M, N, K, stream);
+    }
+    if (int rc = ra_tile_ranges(A, lda, W, scratch, M, N, K, S, kps, stream)) return rc;
+    return launch_wide_reduce(bias, C, ldc, out_dtype, epilogue, M, N, S, scratch, nf, stream);
   }
 #define RA_GWW(MT, WV) launch_wide<MT, WV>(A, lda, W, bias, C, ldc, out_dtype, epilogue, M, N, K, S, kps, partial, scratch, nf, stream)
 #define RA_GWL(MT) return waves == 5 ? RA_GWW(MT, 5) : waves == 6 ? RA_GWW(MT, 6) : waves == 7 ? RA_GWW(MT, 7) : RA_GWW(MT, 8)
@@ -640,7 +638,8 @@ extern "C" int ra_gemm_wide_ranges(int M, int N, int K) {
 extern "C" int ra_gemm_wide_partial(const void* A, const void* W, float* P, long p_floats, int M, int N, int K,
                                     int lda, hipStream_t stream) {
   RA_CHECK(M > 0 && N > 0 && K > 0, "gemm_wide: empty product (%d, %d, %d)", M, N, K);
-  RA_CHECK(M <= 64, "gemm_wide: %d rows; this kernel takes at most 64", M);
+  RA_CHECK(M <= 64 || ra_gemm_tile_takes(WEPI_PLAIN, M, N, K),
+           "gemm_wide: %d rows; at most 64, or 512 where the tiled product is ahead", M);
   RA_CHECK(K % 8 == 0 && lda % 8 == 0 && lda >= K, "gemm_wide: K (%d) and the row stride (%d) must be multiples of 8", K, lda);
   RA_CHECK(((uintptr_t)A % 16) == 0 && ((uintptr_t)W % 16) == 0 && ((uintptr_t)P % 16) == 0,
            "gemm_wide: operands must be 16-byte aligned");
@@ -649,6 +648,7 @@ extern "C" int ra_gemm_wide_partial(const void* A, const void* W, float* P, long
   gw_split(WEPI_PLAIN, M, N, K, &waves, &S, &kps, &partial, true);
   RA_CHECK(P && p_floats >= (long)S * M * N, "gemm_wide: %d ranges of [%d, %d] need %ld floats, got %ld", S, M, N,
            (long)S * M * N, p_floats);
+  if (M > 64) return ra_tile_ranges(A, lda, W, P, M, N, K, S, kps, stream);
   WideNorm nf = {};
   nf.acc_scale = 1.f;
 #define RA_GWP(MT, WV)                                                                                  \

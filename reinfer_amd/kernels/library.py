@@ -156,6 +156,8 @@ def load() -> ctypes.CDLL:
         lib.ra_gemm_wide_row_parts.argtypes = [c_int]
         lib.ra_gemm_wide_ranges.restype = c_int
         lib.ra_gemm_wide_ranges.argtypes = [c_int, c_int, c_int]
+        lib.ra_gemm_tile_takes.restype = c_int
+        lib.ra_gemm_tile_takes.argtypes = [c_int, c_int, c_int, c_int]
         lib.ra_gemm_wide_preferred.restype = c_int
         lib.ra_gemm_wide_preferred.argtypes = [c_int, c_int, c_int, c_int]
         if lib.ra_abi_version() != ABI_VERSION:

@@ -140,19 +140,20 @@ class HipKernels:
     # ---- the q/k/v product left in K ranges for the kernel that consumes it
     def linear_ranges(self, x: torch.Tensor, weight: torch.Tensor):
         """x . weight^T as the float results of the K ranges it was cut into, [ranges, M, N], not yet
-        added, or None where that does not pay: only the products the split kernel takes (bfloat16,
-        17 to 64 rows) and cuts (few output features), whose adding kernel a consumer can save by
-        adding the ranges itself (``qk_norm_rope_cache(..., ranges=)``)."""
+        added, or None where that does not pay: only the products the split kernels take (bfloat16,
+        17 to 64 rows, or 512 where the tiled one is ahead) and cut (few output features), whose adding
+        kernel a consumer can save by adding the ranges itself (``qk_norm_rope_cache(..., ranges=)``)."""
         if not (x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.dim() == 2):
             return None
         M, K = x.shape
         N = weight.shape[0]
-        if not (self.NORM_SKINNY_ROWS < M <= 64) or K % 8 or x.stride(1) != 1 or x.stride(0) % 8 \
+        if not (self.NORM_SKINNY_ROWS < M <= 512) or K % 8 or x.stride(1) != 1 or x.stride(0) % 8 \
                 or weight.shape != (N, K) or not weight.is_contiguous():
             return None
         lib = library.load()
         S = int(lib.ra_gemm_wide_ranges(M, N, K))
-        if S < 2 or not lib.ra_gemm_wide_preferred(0, M, N, K):
+        if S < 2 or not (lib.ra_gemm_wide_preferred if M <= 64 else lib.ra_gemm_tile_takes)(0, M, N, K) \
+                or M > 64 and (not K <= x.stride(0) < 2 ** 21 or x.data_ptr() % 16 or weight.data_ptr() % 16):
             return None
         parts = torch.empty((S, M, N), dtype=torch.float32, device=x.device)
         library.call("ra_gemm_wide_partial", x.data_ptr(), weight.data_ptr(), parts.data_ptr(), parts.numel(),
@@ -696,7 +697,8 @@ class HipKernels:
                bias: Optional[torch.Tensor] = None) -> None:
         """out[M, N] = x[M, K] . weight[N, K]^T (+ bias), float accumulation.
 
-        bfloat16 with up to 64 rows: the weight-streaming MFMA kernel. bfloat16
+        bfloat16 with up to 64 rows: the weight-streaming MFMA kernel; with up to
+        512 rows the tiled one where it is ahead. bfloat16
         with more rows and a bfloat16 result: the library product (hipBLASLt
         through torch), as the reference calls cuBLAS for its prompt products
         (crates/cuda/src/gemm.rs:226-292). bfloat16 with more rows and a float
@@ -709,6 +711,9 @@ class HipKernels:
             M, K = x.shape
             if M <= 64 and K % 8 == 0 and x.stride(0) % 8 == 0 and x.stride(1) == 1:
                 return self.linear_skinny(x, weight, out, bias)
+            if self._tile_takes(0, x, weight, out):
+                self._check_linear(x, weight, out, bias)
+                return self._few_rows("linear output", x, weight, bias, out, 0, M, weight.shape[0], K, True)
             if out.dtype == torch.bfloat16 and x.is_cuda:
                 self._check_linear(x, weight, out, bias)
                 if bias is None:
@@ -727,6 +732,16 @@ class HipKernels:
         if x.dtype == torch.float32 and weight.dtype == torch.float32 and out.dtype == torch.float32 and x.is_cuda:
             return self.linear_f32(x, weight, out, bias)
         self.linear_plain(x, weight, out, bias)
+
+    @staticmethod
+    def _tile_takes(epilogue: int, x, weight, out) -> bool:
+        """Whether the tiled product of 65 to 512 rows takes this one (epilogues as ``ra_gemm_wide``): where it is ahead of
+        the library's, for rows that are whole 16-byte pieces."""
+        M, K = x.shape
+        return 64 < M <= 512 and x.is_cuda and K % 8 == 0 and x.stride(0) % 8 == 0 and K <= x.stride(0) < 2 ** 21 \
+            and x.stride(1) == 1 and out.stride(0) >= out.shape[1] and weight.is_contiguous() and out.stride(1) == 1 \
+            and all(t.data_ptr() % 16 == 0 for t in (x, weight, out)) \
+            and bool(library.load().ra_gemm_tile_takes(epilogue, M, weight.shape[0], K))
 
     @staticmethod
     def _check_linear(x, weight, out, bias):
@@ -780,11 +795,11 @@ class HipKernels:
                     or x.dtype != torch.bfloat16 or out.dtype != torch.float32:
                 raise ValueError("linear_skinny: a factor rides on a plain accumulating bfloat16 product only")
             lib = library.load()
-            if M > 64 and not bool(lib.ra_gemm_wide_preferred(2, M, N, K)):
+            if M > 64 and not self._tile_takes(2, x, weight, out):
                 torch.addmm(out, x, weight.t(), alpha=float(alpha), out_dtype=torch.float32, out=out)
                 return None
             if wide is None:
-                wide = bool(lib.ra_gemm_wide_preferred(2, M, N, K))
+                wide = M > 64 or bool(lib.ra_gemm_wide_preferred(2, M, N, K))
             if not wide:
                 library.call("ra_gemm_skinny_scaled", x.data_ptr(), weight.data_ptr(), out.data_ptr(), M, N, K,
                              x.stride(0), out.stride(0), float(alpha), _stream())
@@ -817,8 +832,9 @@ class HipKernels:
                 return True
             self.linear_skinny(x, weight, out, bias, accumulate=True, wide=wide)
             return False
-        if accumulate and M > 64 and bias is None and row_sums is None and emit is None and wide is None \
-                and not bool(library.load().ra_gemm_wide_preferred(2, M, N, K)):
+        if accumulate and M > 64 and bias is None and row_sums is None and emit is None and wide is None:
+            if self._tile_takes(2, x, weight, out):
+                return self._few_rows("linear output", x, weight, None, out, 2, M, N, K, True)
             # more rows than the weight-streaming kernels take: the library's product, adding in place
             torch.addmm(out, x, weight.t(), out_dtype=torch.float32, out=out)
             return None
@@ -840,7 +856,7 @@ class HipKernels:
 
     def can_finish_norm(self, M: int, N: int, K: int) -> bool:
         """True where ``linear_skinny(..., accumulate=True, finish=)`` writes the finished norm: the rows
-        between the two limits, a product that the kernel with K ranges takes at these rows, rows of up to
+        between the two limits, a product that the tiled kernel takes at these rows, rows of up to
         16384 columns in steps of 8."""
         return self.NORM_ON_PRODUCTS_ROWS < M <= self.NORM_FINISHED_ROWS and N % 8 == 0 and N <= 16384 \
             and K % 8 == 0 and bool(library.load().ra_gemm_wide_preferred(2, M, N, K))
@@ -954,8 +970,8 @@ class HipKernels:
         """out[M, I] = silu(x . Wg^T) * (x . Wu^T) for ``weight`` [2I, K] whose rows alternate in
         runs of GATE_GROUP: 8 gate rows, the 8 up rows of the same features, and so on.
 
-        bfloat16 with up to 64 rows: one kernel, the gate applied in the product's
-        epilogue. Otherwise the product into a [M, 2I] buffer, then the gate kernel."""
+        bfloat16 with up to 64 rows, or 128 where the tiles fill the chip: one kernel, the gate
+        applied in the product's epilogue. Otherwise the product into a [M, 2I] buffer, then the gate kernel."""
         _dev(x, weight, out)
         M, K = x.shape
         I = out.shape[1]
@@ -969,6 +985,9 @@ class HipKernels:
             else:
                 self._skinny_normed(x, weight, None, out, 1, M, 2 * I, K, row_sums, None)
             return
+        if row_sums is None and wide is None and weight.dtype == out.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 \
+                and out.stride(0) % 4 == 0 and self._tile_takes(1, x, weight, out):
+            return self._few_rows("linear output", x, weight, None, out, 1, M, 2 * I, K, True)
         if row_sums is not None:
             raise ValueError("gated_linear: row sums ride on the weight-streaming product only (bfloat16, <= 64 rows)")
         gu = torch.empty((M, 2 * I), dtype=out.dtype, device=x.device)

@@ -1,0 +1,94 @@
+"""The tiled bfloat16 product of 65 to 512 rows against float64, at the edges of its tiles, K ranges and dispatch."""
+import math
+
+import pytest
+import torch
+
+from reinfer_amd import kernels
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def ops():
+    return kernels.current()
+
+
+def operands(M, N, K, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    x = torch.randn(M, K, device=DEV, generator=g).to(torch.bfloat16)
+    w = (torch.randn(N, K, device=DEV, generator=g) / math.sqrt(K)).to(torch.bfloat16)
+    return x, w, g
+
+
+def bound(x, w, K):
+    """Float sums of K exact products in any order: K roundings of at most 2^-24 of the sum of magnitudes, which the
+    matrix cores' own order halves many times over; a twentieth of that worst case still catches a lost or doubled k."""
+    return (x.double().abs() @ w.double().abs().T) * (K * 2.0 ** -24 / 20) + 1e-6
+
+
+# row tiles of 128 at, below and above their edges; feature tiles with 1, 4 and 127 left; K with pieces left of a step of 64
+# and of a range; two ranges and many
+SIZES = [(65, 4096, 4096), (97, 6144, 4096), (128, 4097, 1032), (129, 2564, 4096), (192, 1151, 6152), (256, 4096, 12288),
+         (255, 8128, 1536), (257, 4224, 8192), (512, 2560, 9736), (511, 2049, 8200), (65, 7936, 1024)]
+
+
+@pytest.mark.parametrize("M,N,K", SIZES)
+def test_tiled_product_with_each_epilogue(M, N, K):
+    lib = kernels.library.load()
+    assert lib.ra_gemm_tile_takes(0, M, N, K) == 1
+    x, w, g = operands(M, N, K, M + N)
+    ref, err = x.double() @ w.double().T, bound(x, w, K)
+    bias = torch.randn(N, device=DEV, generator=g).to(torch.bfloat16)
+    out = torch.full((M, N), float("nan"), device=DEV)
+    ops().linear(x, w, out)
+    assert ((out.double() - ref).abs() <= err).all()
+    ops().linear(x, w, out, bias)
+    biased = ref + bias.double()
+    assert ((out.double() - biased).abs() <= err + biased.abs() * 2 ** -23).all()
+    half = torch.full((M, N + 4), float("nan"), device=DEV, dtype=torch.bfloat16)
+    ops().linear(x, w, half[:, :N], bias)               # rows that are not next to one another
+    assert ((half[:, :N].double() - biased).abs() <= err + biased.abs() * 2 ** -8).all()
+    assert torch.isnan(half[:, N:]).all()
+    for alpha in (1.0, 0.25):
+        stream = torch.randn(M, N, device=DEV, generator=g) * 8
+        want = stream.double() + alpha * ref
+        ops().linear_skinny(x, w, stream, accumulate=True, alpha=alpha)
+        assert ((stream.double() - want).abs() <= err + want.abs() * 2 ** -23).all()
+    parts = ops().linear_ranges(x, w)
+    assert parts.shape[0] == lib.ra_gemm_wide_ranges(M, N, K) >= 2
+    assert ((parts.double().sum(0) - ref).abs() <= err).all()
+
+
+@pytest.mark.parametrize("M,I,K", [(65, 9728, 2560), (97, 12288, 4096), (128, 16384, 1024), (128, 8200, 1032)])
+def test_tiled_gated_product(M, I, K):
+    assert kernels.library.load().ra_gemm_tile_takes(1, M, 2 * I, K) == 1
+    x, w, _ = operands(M, 2 * I, K, M + I)
+    out = torch.full((M, I), float("nan"), device=DEV, dtype=torch.bfloat16)
+    ops().gated_linear(x, w, out)
+    prod, err = x.double() @ w.double().T, bound(x, w, K)
+    rows = torch.arange(2 * I, device=DEV).view(-1, 2, 8)
+    gate, up = prod[:, rows[:, 0].reshape(-1)], prod[:, rows[:, 1].reshape(-1)]
+    eg, eu = err[:, rows[:, 0].reshape(-1)], err[:, rows[:, 1].reshape(-1)]
+    want = gate * torch.sigmoid(gate) * up              # silu's slope is at most 1.1
+    assert ((out.double() - want).abs() <= 1.1 * eg * (up.abs() + eu) + gate.abs() * eu + want.abs() * (2 ** -8 + 2 ** -20)).all()
+
+
+def test_tiled_product_takes_only_what_it_can_read():
+    """Sizes past its rule, rows of no whole 16-byte pieces and unaligned pointers stay with the library's product."""
+    lib = kernels.library.load()
+    for epilogue, M, N, K in [(0, 64, 4096, 4096), (0, 513, 4096, 12288), (0, 257, 4096, 4096), (0, 97, 22528, 4096),
+                              (0, 384, 4096, 12288), (0, 97, 512, 1024), (1, 129, 24576, 4096), (1, 97, 4096, 4096)]:
+        assert lib.ra_gemm_tile_takes(epilogue, M, N, K) == 0
+    M, N, K = 97, 4096, 4096
+    x, w, g = operands(M, N, K + 8, 3)
+    odd = torch.empty(M, K + 12, device=DEV, dtype=torch.bfloat16)[:, 1:K + 1]
+    odd.copy_(x[:, :K])
+    rows = torch.randn(1, K, device=DEV, generator=g).to(torch.bfloat16).expand(M, K)
+    w = w[:, :K].contiguous()
+    for a in (odd, rows):
+        assert not ops()._tile_takes(0, a, w, torch.empty(M, N, device=DEV, dtype=torch.bfloat16))
+        out = torch.full((M, N), float("nan"), device=DEV, dtype=torch.bfloat16)
+        ops().linear(a, w, out)
+        want = a.double() @ w.double().T
+        assert ((out.double() - want).abs() <= bound(a, w, K) + want.abs() * 2 ** -8).all()
