@@ -11,21 +11,16 @@
 // took 406 us for the first; with more rows the activations, which every workgroup reads again, cost as much as the weights
 // (19456 x 2560 at 32 rows 96 us, as much as the other kernel at 33).
 //
-// From 33 rows on (gemm_f32_tile_kernel) tiles of both operands go through LDS, 32 k at a time: fetched into registers
-// while the tile before is multiplied, written to the other of two buffers, one barrier a step. The float matrix cores do
-// 256 flops a clock and CU, and a 128 x 128 tile wants 8 bytes a clock from L2, a 64 x 64 one 16, which is what L2 gives:
-// 100 to 107 TFLOP/s of 157 (2048 x 19456 x 2560 1.92 ms; 300 rows 360 us against 561 of the plain kernel, 300 x 2560 x 9728
-// 191 us against 1350).
+// From 33 rows on (gemm_f32_tile_kernel) tiles of both operands go through LDS, 32 k at a time, by loads that go straight
+// there; two stages and one barrier a step. The float matrix cores do 256 flops a clock and CU and bound it: a workgroup
+// alone on a CU keeps them 79 % busy, with others beside it 87 %. Tiles of 64 x 128 leave room in LDS for three workgroups
+// whose waits fall at different times; 128 x 128 with two or four stages had them 70 to 83 % busy, deeper rings changed
+// nothing. 1190 x 19456 x 2560 takes 0.94 ms (127 TFLOP/s of 157; through registers into LDS, in tiles of 128 x 128, 1.18 ms),
+// 2048 x 19456 x 2560 1.52 (1.92), 300 rows 269 us (360), 300 x 2560 x 9728 149 us (191; the plain kernel 1350).
 #include "common.h"
 #include "reinfer_hip.h"
 
 namespace {
-
-__device__ __forceinline__ f32x4_t load4(const float* p, bool ok) {
-  f32x4_t v = *(const f32x4_t*)p;
-  if (!ok) v = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-  return v;
-}
 
 // ------------------------------------------------------------------------------------------------ up to 32 rows
 // Workgroups that stay: tile b, b + grid, ... of 16 features, all M rows (MT tiles of 16), WAVES waves. A wave's loads run
@@ -128,149 +123,189 @@ gemm_f32_stream_kernel(const float* __restrict__ A, const float* __restrict__ W,
 
 // ------------------------------------------------------------------------------------------------ from 33 rows on
 #define F32_BK 32
-// A row of a tile in LDS is 8 pieces of 16 bytes, piece p of row r at place p ^ (r % 8): eight rows' reads of one piece fall
-// on different banks.
-__device__ __forceinline__ int piece_at(int row, int piece) { return row * F32_BK + ((piece ^ (row & 7)) << 2); }
 
-// One workgroup of four waves: rows [B blockIdx.y, +B), features [B blockIdx.x, +B), k of range blockIdx.z.
-// ranges == 1: C with the bias; else the range's float sums into part[blockIdx.z][M][N].
-template <int B>
-__global__ void __launch_bounds__(256)
-gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
-                     float* __restrict__ C, float* __restrict__ part, int M, int N, int K, int lda, int ldc,
-                     int range_k) {
-  constexpr int T = B / 64;                // 32 x 32 tiles a side of a wave's quarter
-  constexpr int L = B * F32_BK / 4 / 256;  // 16-byte pieces a thread and operand
-  __shared__ float lds[4 * B * F32_BK];    // two buffers of both operands: 64 KB at B = 128
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int m0 = blockIdx.y * B, n0 = blockIdx.x * B;
-  const int k0 = blockIdx.z * range_k, k1 = k0 + range_k < K ? k0 + range_k : K;
-  const int steps = (k1 - k0 + F32_BK - 1) / F32_BK;
-  // staging: piece i of a thread is row (tid + 256 i) / 8, k 4 ((tid + 256 i) % 8)
-  const float *ag[L], *wg[L];
-  const int kp = (tid & 7) * 4;
+struct F32Tile {
+  const float* a;
+  const float* w;
+  const float* bias;
+  float* c;                                // ranges > 1: the ranges' sums, [ranges][M][N]
+  int M, N, K, lda, ldc, m_tiles, n_tiles, ranges, range_k;
+};
+
+// One workgroup of four waves a tile of BM rows and BN features and range of k, in 2 x 2 quarters. A stage is 32 k of both
+// operands, rows of 8 pieces of 16 bytes, piece p of row r at place p ^ (r % 8), so that eight rows' reads of one piece fall
+// on different banks; loads that go straight to LDS write it in the order of their lanes, so it is their addresses that are
+// permuted. A tile's operands have descriptors of their own, whose ends are those of the matrices: rows past them are zeros.
+template <int BM, int BN, int STAGES>
+__global__ void __launch_bounds__(256) gemm_f32_tile_kernel(F32Tile g) {
+  constexpr int TM = BM / 64, TN = BN / 64;
+  constexpr int ROWS = BM + BN, PA = BM / 32, PB = BN / 32;       // a wave's loads a stage: 8 rows (1 KB) each
+  constexpr unsigned NOWHERE = 0xFFFFFFF0u;
+  __shared__ __attribute__((aligned(1024))) float lds[STAGES * ROWS * F32_BK];
+  // the row tiles of a panel and range of weights follow one another, and each XCD gets a run of tiles
+  const long total = (long)g.m_tiles * g.n_tiles * g.ranges, each = (total + RA_XCDS - 1) / RA_XCDS;
+  const long at = blockIdx.x / RA_XCDS, tile = blockIdx.x % RA_XCDS * each + at;
+  if (at >= each || tile >= total) return;
+  const int m0 = (int)(tile % g.m_tiles) * BM;
+  const int z = (int)(tile / g.m_tiles % g.ranges), n0 = (int)(tile / g.m_tiles / g.ranges) * BN;
+  const int k0 = z * g.range_k, k1 = min(k0 + g.range_k, g.K), steps = (k1 - k0 + F32_BK - 1) / F32_BK;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int a_rows = min(BM, g.M - m0), w_rows = min(BN, g.N - n0);
+  const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(g.a + (size_t)m0 * g.lda), 0, (int)(((size_t)(a_rows - 1) * g.lda + g.K) * 4), 0x00020000);
+  const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(g.w + (size_t)n0 * g.K), 0, (int)((size_t)w_rows * g.K * 4), 0x00020000);
+  const int piece = (lane & 7) ^ (lane >> 3);
+  unsigned a_off[PA], w_off[PB];
 #pragma unroll
-  for (int i = 0; i < L; ++i) {
-    const int row = (tid + 256 * i) >> 3;
-    ag[i] = A + (size_t)(m0 + row < M ? m0 + row : M - 1) * lda;
-    wg[i] = W + (size_t)(n0 + row < N ? n0 + row : N - 1) * K;
+  for (int i = 0; i < PA; ++i) {
+    const int r = (wave * PA + i) * 8 + (lane >> 3);
+    a_off[i] = r < a_rows ? (unsigned)(((size_t)r * g.lda + piece * 4) * 4) : 0x80000000u;
   }
-  f32x4_t as[L], ws[L];
-  auto fetch = [&](int k) {
-    const bool ok = k + kp < k1;
-    const int at = ok ? k + kp : 0;
 #pragma unroll
-    for (int i = 0; i < L; ++i) {
-      as[i] = load4(ag[i] + at, ok);
-      ws[i] = load4(wg[i] + at, ok);
-    }
+  for (int i = 0; i < PB; ++i) {
+    const int r = (wave * PB + i) * 8 + (lane >> 3);
+    w_off[i] = r < w_rows ? (unsigned)(((size_t)r * g.K + piece * 4) * 4) : 0x80000000u;
+  }
+  auto fetch = [&](int s, int buf) {
+    const int k = k0 + s * F32_BK;
+    const unsigned past = k + piece * 4 < k1 ? 0u : NOWHERE;      // pieces past the range's end become zeros
+    float* to = lds + buf * ROWS * F32_BK;
+#pragma unroll
+    for (int i = 0; i < PA; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          a_rsrc, (__attribute__((address_space(3))) void*)(to + (wave * PA + i) * 8 * F32_BK), 16,
+          (int)((a_off[i] + (unsigned)k * 4u) | past), 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < PB; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          w_rsrc, (__attribute__((address_space(3))) void*)(to + (BM + (wave * PB + i) * 8) * F32_BK), 16,
+          (int)((w_off[i] + (unsigned)k * 4u) | past), 0, 0, 0);
   };
-  auto stage = [&](int buf) {
-    float* a = lds + buf * 2 * B * F32_BK;
-    float* w = a + B * F32_BK;
+  f32x16_t acc[TN][TM];
 #pragma unroll
-    for (int i = 0; i < L; ++i) {
-      const int at = piece_at((tid + 256 * i) >> 3, tid & 7);
-      *(f32x4_t*)(a + at) = as[i];
-      *(f32x4_t*)(w + at) = ws[i];
-    }
-  };
-  f32x16_t acc[T][T];
+  for (int i = 0; i < TN; ++i)
 #pragma unroll
-  for (int i = 0; i < T; ++i)
-#pragma unroll
-    for (int j = 0; j < T; ++j)
+    for (int j = 0; j < TM; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-  const int wm = (wave >> 1) * (B / 2), wn = (wave & 1) * (B / 2);
+  const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BN / 2);
   const int row = lane & 31, half = lane >> 5;
-
-  fetch(k0);
-  stage(0);
-  __syncthreads();
+#pragma unroll
+  for (int s = 0; s < STAGES - 1; ++s) fetch(s, s);
+  int buf = 0;
   for (int s = 0; s < steps; ++s) {
-    if (s + 1 < steps) fetch(k0 + (s + 1) * F32_BK);
-    __builtin_amdgcn_sched_barrier(0);
-    const float* a = lds + (s & 1) * 2 * B * F32_BK + wm * F32_BK;
-    const float* w = lds + ((s & 1) * 2 + 1) * B * F32_BK + wn * F32_BK;
+    // this wave's loads of stage s are done when only those of the stages behind it are left, its reads of the stage that is
+    // asked for next when no LDS read is left
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((PA + PB) * (STAGES - 2)) : "memory");
+    fetch(s + STAGES - 1, buf == 0 ? STAGES - 1 : buf - 1);
+    const float* as = lds + buf * ROWS * F32_BK + (wm + row) * F32_BK;
+    const float* ws = lds + buf * ROWS * F32_BK + (BM + wn + row) * F32_BK;
 #pragma unroll
-    for (int kk = 0; kk < F32_BK; kk += 8) {
-      f32x4_t x[T], y[T];
+    for (int kk = 0; kk < F32_BK / 8; ++kk) {
+      f32x4_t x[TM], y[TN];
+      const int p = ((kk * 2 + half) ^ (row & 7)) * 4;
 #pragma unroll
-      for (int i = 0; i < T; ++i) {
-        x[i] = *(const f32x4_t*)(a + piece_at(i * 32 + row, kk / 4 + half));
-        y[i] = *(const f32x4_t*)(w + piece_at(i * 32 + row, kk / 4 + half));
-      }
+      for (int j = 0; j < TM; ++j) x[j] = *(const f32x4_t*)(as + j * 32 * F32_BK + p);
+#pragma unroll
+      for (int i = 0; i < TN; ++i) y[i] = *(const f32x4_t*)(ws + i * 32 * F32_BK + p);
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int i = 0; i < T; ++i)
+        for (int i = 0; i < TN; ++i)
 #pragma unroll
-          for (int j = 0; j < T; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(y[j][e], x[i][e], acc[i][j], 0, 0, 0);
+          for (int j = 0; j < TM; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(y[i][e], x[j][e], acc[i][j], 0, 0, 0);
     }
-    if (s + 1 < steps) stage((s + 1) & 1);
-    __syncthreads();
+    buf = buf + 1 == STAGES ? 0 : buf + 1;
   }
   // a lane holds row lane % 32 of the tile, features 8 (e / 4) + 4 (lane / 32) + e % 4
-  float* out = part ? part + (size_t)blockIdx.z * M * N : C;
-  const int ld = part ? N : ldc;
-  const float* b = part ? nullptr : bias;
+  const bool cut = g.ranges > 1;
+  float* out = cut ? g.c + (size_t)z * g.M * g.N : g.c;
+  const int ld = cut ? g.N : g.ldc;
+  const float* b = cut ? nullptr : g.bias;
+  const bool whole = g.N % 4 == 0 && ld % 4 == 0 && (uintptr_t)g.c % 16 == 0;
 #pragma unroll
-  for (int i = 0; i < T; ++i) {
-    const int m = m0 + wm + i * 32 + row;
-    if (m >= M) continue;
+  for (int j = 0; j < TM; ++j) {
+    const int m = m0 + wm + j * 32 + row;
+    if (m >= g.M) continue;
 #pragma unroll
-    for (int j = 0; j < T; ++j)
+    for (int i = 0; i < TN; ++i)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int n = n0 + wn + j * 32 + g * 8 + half * 4;
+      for (int q = 0; q < 4; ++q) {
+        const int n = n0 + wn + i * 32 + q * 8 + half * 4;
+        if (n >= g.N) continue;
+        f32x4_t v;
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (n + e < N) out[(size_t)m * ld + n + e] = b ? acc[i][j][g * 4 + e] + b[n + e] : acc[i][j][g * 4 + e];
+        for (int e = 0; e < 4; ++e) {
+          v[e] = acc[i][j][q * 4 + e];
+          if (b && n + e < g.N) v[e] += b[n + e];
+        }
+        if (whole) {
+          *(f32x4_t*)(out + (size_t)m * ld + n) = v;
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (n + e < g.N) out[(size_t)m * ld + n + e] = v[e];
+        }
       }
   }
 }
 
+// C = the ranges' sums added in range order (+ bias): a workgroup takes 1024 features of a row, four a thread, read 16 bytes at
+// a time where rows allow it. It is bound by reading the planes.
 __global__ void __launch_bounds__(256)
 gemm_f32_add_kernel(const float* __restrict__ part, int ranges, const float* __restrict__ bias, float* __restrict__ C,
-                    int M, int N, int ldc) {
-  const size_t size = (size_t)M * N, i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= size) return;
-  const int m = i / N, n = i % N;
-  float v = part[i];
-  for (int r = 1; r < ranges; ++r) v += part[r * size + i];
-  C[(size_t)m * ldc + n] = bias ? v + bias[n] : v;
+                    int M, int N, int ldc, bool whole) {
+  const int n = (blockIdx.y * 256 + threadIdx.x) * 4;
+  if (n >= N) return;
+  const size_t m = blockIdx.x, size = (size_t)M * N;
+  const float* p = part + m * N + n;
+  float* c = C + m * ldc + n;
+  if (whole) {
+    f32x4_t v = *(const f32x4_t*)p;
+    for (int r = 1; r < ranges; ++r) v += *(const f32x4_t*)(p + r * size);
+    if (bias)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] += bias[n + e];
+    *(f32x4_t*)c = v;
+    return;
+  }
+  for (int e = 0; e < 4 && n + e < N; ++e) {
+    float v = p[e];
+    for (int r = 1; r < ranges; ++r) v += p[r * size + e];
+    c[e] = bias ? v + bias[n + e] : v;
+  }
 }
 
-// The tile kernel's plan: 128 x 128 tiles where there are four a CU and more (2048 x 19456 x 2560: 1.91 ms against 2.02 ms),
-// else 64 x 64 ones with K cut into as many ranges of at least 256 k as price lowest: a CU's share of the workgroups at the
-// share of the matrix cores' rate that so many side by side reach (measured: one workgroup waits for memory most of the
-// time), and the ranges' sums written and read again. (300 x 2560 x 9728: uncut 459 us, in 12 ranges 190; 33 x 19456 x
-// 2560: 157 us, in 3 ranges 92.)
+// The tile kernel's plan: tiles of 64 x 128 or 64 x 64 and as many K ranges of at least 256 k as price lowest: a CU's share
+// of the workgroups at the share of the matrix cores' rate that so many side by side reach (measured), and the ranges' sums
+// written and read again. (300 x 2560 x 9728: 64 x 64 uncut 185 us, in 5 ranges 149; 48 x 19456 x 2560: uncut 86 us, in 5 68.)
 struct TilePlan {
-  int side, ranges, range_k;
+  int bn, ranges, range_k;
 };
 TilePlan tile_plan(int M, int N, int K) {
-  const int cus = ra_cu_count();
-  const long big = (long)((M + 127) / 128) * ((N + 127) / 128);
-  if (big >= 4L * cus) return {128, 1, K};
-  const long tiles = (long)((M + 63) / 64) * ((N + 63) / 64);
-  const double reached[5] = {0.28, 0.48, 0.62, 0.72, 0.76};
-  const double tile_us = 64.0 * 64.0 * 2.0 * K / 600e3;                       // one tile at a CU's full rate
-  int best = 1;
+  const long cus = ra_cu_count();
+  const double reached[2][3] = {{0.70, 0.78, 0.81}, {0.79, 0.85, 0.87}};
+  TilePlan best = {};
   double best_us = 0.0;
-  for (int r = 1; r <= 16 && (r == 1 || K / r >= 256); ++r) {
-    const long load = (tiles * r + cus - 1) / cus;
-    double us = (double)load / r * tile_us / reached[load < 5 ? load - 1 : 4];
-    if (r > 1) us += 3.0 + (double)r * M * N * 8.0 / 5e6;
-    if (r == 1 || us < best_us) {
-      best = r;
-      best_us = us;
+  for (int wide = 0; wide < 2; ++wide) {
+    const int bn = wide ? 128 : 64;
+    const long tiles = (long)((M + 63) / 64) * ((N + bn - 1) / bn);
+    const double tile_us = 64.0 * bn * 2.0 * K / 614e3;                       // one tile at a CU's full rate
+    for (int r = 1; r <= 16 && (r == 1 || K / r >= 256); ++r) {
+      const long load = (tiles * r + cus - 1) / cus;
+      double us = (double)load / r * tile_us / reached[wide][load < 3 ? load - 1 : 2];
+      if (r > 1) us += 3.0 + (double)r * M * N * 8.0 / 5e6;
+      if (best.bn == 0 || us < best_us) {
+        const int range_k = ((K + r - 1) / r + F32_BK - 1) / F32_BK * F32_BK;
+        best = {bn, (K + range_k - 1) / range_k, range_k};
+        best_us = us;
+      }
     }
   }
-  const int range_k = ((K + best - 1) / best + F32_BK - 1) / F32_BK * F32_BK;
-  return {64, (K + range_k - 1) / range_k, range_k};
+  return best;
 }
 
 }  // namespace
@@ -278,7 +313,8 @@ TilePlan tile_plan(int M, int N, int K) {
 #define F32_STREAM_ROWS 32
 
 extern "C" int ra_gemm_f32_supports(const void* A, const void* W, int K, int lda) {
-  return K > 0 && K % 4 == 0 && ra_rows_16b(A, lda, 4) && ra_rows_16b(W, K, 4);
+  // a tile's rows are addressed from its first one in 31 bits
+  return K > 0 && K % 4 == 0 && lda < (1 << 21) && K < (1 << 21) && ra_rows_16b(A, lda, 4) && ra_rows_16b(W, K, 4);
 }
 
 extern "C" long ra_gemm_f32_scratch(int M, int N, int K) {
@@ -317,15 +353,15 @@ extern "C" int ra_gemm_f32(const float* A, const float* W, const float* bias, fl
   const bool cut = p.ranges > 1;
   RA_CHECK(!cut || (scratch && scratch_floats >= (long)p.ranges * M * N), "gemm_f32: scratch of %ld floats, needs %ld",
            scratch_floats, (long)p.ranges * M * N);
-  const dim3 grid((N + p.side - 1) / p.side, (M + p.side - 1) / p.side, p.ranges);
-  RA_CHECK(grid.y <= 65535, "gemm_f32: %d rows in one launch", M);
-  float* part = cut ? scratch : nullptr;
-  if (p.side == 128) gemm_f32_tile_kernel<128><<<grid, 256, 0, stream>>>(A, W, bias, C, part, M, N, K, lda, ldc, p.range_k);
-  else gemm_f32_tile_kernel<64><<<grid, 256, 0, stream>>>(A, W, bias, C, part, M, N, K, lda, ldc, p.range_k);
+  F32Tile g = {A, W, bias, cut ? scratch : C, M, N, K, lda, ldc, (M + 63) / 64, (N + p.bn - 1) / p.bn, p.ranges, p.range_k};
+  const long total = (long)g.m_tiles * g.n_tiles * g.ranges, blocks = (total + RA_XCDS - 1) / RA_XCDS * RA_XCDS;
+  RA_CHECK(blocks <= 0x7FFFFFFFL, "gemm_f32: [%d, %d] in one launch", M, N);
+  if (p.bn == 128) gemm_f32_tile_kernel<64, 128, 2><<<(unsigned)blocks, 256, 0, stream>>>(g);
+  else gemm_f32_tile_kernel<64, 64, 2><<<(unsigned)blocks, 256, 0, stream>>>(g);
   RA_LAUNCH_CHECK("gemm_f32");
   if (cut) {
-    const size_t blocks = ((size_t)M * N + 255) / 256;
-    gemm_f32_add_kernel<<<blocks, 256, 0, stream>>>(scratch, p.ranges, bias, C, M, N, ldc);
+    const bool whole = N % 4 == 0 && ldc % 4 == 0 && (uintptr_t)C % 16 == 0 && (uintptr_t)scratch % 16 == 0;
+    gemm_f32_add_kernel<<<dim3(M, (N + 1023) / 1024), 256, 0, stream>>>(scratch, p.ranges, bias, C, M, N, ldc, whole);
     RA_LAUNCH_CHECK("gemm_f32 (ranges)");
   }
   return 0;

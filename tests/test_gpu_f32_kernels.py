@@ -11,10 +11,10 @@ def ops():
     return kernels.current()
 
 
-# rows on both sides of the two kernels' edges (16, 32, 64, 128), features off every tile, k with a part piece of 32, a last
+# rows on both sides of the two kernels' edges (16, 32, 64, 128), features off every tile (of 64 and, with many, of 128), k with a part piece of 32, a last
 # range shorter than the others, and rows that are no 16-byte pieces (the plain kernel's)
 @pytest.mark.parametrize("M", [1, 16, 17, 32, 33, 64, 65, 129, 300])
-@pytest.mark.parametrize("N,K", [(16, 32), (7, 4), (100, 68), (333, 2052), (1030, 1120), (40, 6144), (24, 70)])
+@pytest.mark.parametrize("N,K", [(16, 32), (7, 4), (100, 68), (333, 2052), (1030, 1120), (40, 6144), (24, 70), (4100, 2052), (8193, 516)])
 @pytest.mark.parametrize("bias", [False, True])
 def test_product_of_float_matrices(M, N, K, bias):
     g = torch.Generator(device=DEV).manual_seed(M * N + K)
