@@ -7,11 +7,13 @@ parts call these through :func:`reinfer_amd.kernels.current`.
 from __future__ import annotations
 
 import heapq
+import struct
 from typing import Optional
 
 import torch
 
 from . import library
+from .upload import to_device
 
 _TAG = {torch.float32: 0, torch.bfloat16: 1}
 
@@ -1846,31 +1848,28 @@ class HipKernels:
         n, V = logits.shape
         if logits.dtype != torch.float32 or logits.stride(1) != 1:
             raise TypeError("filter_logits: logits are float32 rows")
-        rec = np.zeros((n, 12), dtype=np.float32)
-        irec = rec.view(np.int32)
-        window, off = [], 0
-        for i, (p, hist) in enumerate(zip(params, histories)):
-            rec[i, 0] = max(0.0, float(p.temperature))
-            rec[i, 1] = float(p.top_p or 0.0)
-            rec[i, 2] = float(p.min_p or 0.0)
-            rec[i, 3] = float(p.repeat_penalty or 0.0)
-            rec[i, 4] = max(0.0, float(p.frequency_penalty or 0.0))
-            rec[i, 5] = max(0.0, float(p.presence_penalty or 0.0))
-            irec[i, 6] = int(p.top_k or 0)
-            win = list(hist[-p.repeat_last_n:]) if (p.penalties and p.repeat_last_n > 0) else []
-            irec[i, 7], irec[i, 8] = off, len(win)
-            window += win
-            off += len(win)
+        floats, ints, window = [], [], []
+        for p, hist in zip(params, histories):
+            repeat, frequency, presence = p.repeat_penalty or 0.0, p.frequency_penalty or 0.0, p.presence_penalty or 0.0
+            floats.append((max(0.0, p.temperature), p.top_p or 0.0, p.min_p or 0.0, repeat, max(0.0, frequency),
+                           max(0.0, presence)))
+            at = len(window)
+            if p.repeat_last_n > 0 and (repeat > 1.0 or frequency > 0.0 or presence > 0.0):
+                window.extend(hist[-p.repeat_last_n:])
+            end = len(window)
             bias = getattr(p, "logit_bias", ())
             if bias:
-                pairs = np.zeros((len(bias), 2), dtype=np.int32)
+                pairs = np.empty((len(bias), 2), dtype=np.int32)
                 pairs[:, 0] = [int(t) for t, _ in bias]
                 pairs[:, 1] = np.asarray([float(b) for _, b in bias], dtype=np.float32).view(np.int32)
-                irec[i, 9], irec[i, 10] = off, len(bias)
                 window += pairs.reshape(-1).tolist()
-                off += 2 * len(bias)
-        rows_t = torch.from_numpy(rec).to(logits.device)
-        win_t = torch.tensor(window or [0], dtype=torch.int32).to(logits.device)
+            ints.append((int(p.top_k or 0), at, end - at, end if bias else 0, len(bias), 0))
+        rec = np.empty((n, 12), dtype=np.float32)
+        rec[:, :6], rec.view(np.int32)[:, 6:] = floats, ints
+        window.append(0)                     # never empty
+        packed = np.frombuffer(struct.pack(f"{len(window)}i", *window), dtype=np.int32)     # half the time of an array of the list
+        both = to_device(np.concatenate([rec.view(np.int32).reshape(-1), packed]), logits.device)
+        rows_t, win_t = both[:12 * n], both[12 * n:]
         need = int(library.load().ra_filter_scratch(n, V))
         scratch = torch.empty(need, dtype=torch.uint8, device=logits.device)
         library.call("ra_filter_logits", logits.data_ptr(), n, V, logits.stride(0), rows_t.data_ptr(),

@@ -13,9 +13,11 @@ from __future__ import annotations
 
 from typing import List, Optional, Sequence
 
+import numpy as np
 import torch
 
 from .. import kernels
+from ..kernels.upload import to_device
 from .params import SamplingParams
 
 _MASK63 = (1 << 63) - 1
@@ -55,11 +57,15 @@ class Sampler:
                 raise ValueError("penalties need the requests' tokens")
             logits = logits.clone()
             ops.filter_logits(logits, params, histories)
-        temp = torch.tensor([max(0.0, float(p.temperature)) for p in params], dtype=torch.float32)
-        seeds_t = torch.tensor([as_int64(int(s)) for s in seeds], dtype=torch.int64)
-        pos_t = torch.tensor([int(p) for p in positions], dtype=torch.int32)
+        # one transfer: seeds, temperatures, positions
+        rows = np.empty(16 * n, dtype=np.uint8)
+        rows[:8 * n].view(np.int64)[:] = [as_int64(int(s)) for s in seeds]
+        rows[8 * n:12 * n].view(np.float32)[:] = [max(0.0, float(p.temperature)) for p in params]
+        rows[12 * n:].view(np.int32)[:] = [int(p) for p in positions]
+        rows_t = to_device(rows, self.device)
         tokens = torch.empty(n, dtype=torch.int32, device=self.device)
-        ops.sample(logits, temp.to(self.device), seeds_t.to(self.device), pos_t.to(self.device), tokens)
+        ops.sample(logits, rows_t[8 * n:12 * n].view(torch.float32), rows_t[:8 * n].view(torch.int64),
+                   rows_t[12 * n:].view(torch.int32), tokens)
         out = tokens.tolist()
         for i, t in enumerate(out):
             if t < 0:
