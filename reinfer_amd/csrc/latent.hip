@@ -122,14 +122,16 @@ extern "C" int ra_latent_prep(const void* proj, int act_dtype, int ld, int q_off
 // owns 16 output columns of one head for MT tiles of 16 tokens and walks K in steps of 32; both operands come
 // straight from memory in operand layout (lane (r, g): row r, elements 8g .. 8g + 7 of the step, one 16-byte
 // load), the weights of a head being small enough to stay in the caches while the token tiles pass. The four
-// waves of a workgroup take four column tiles. Lane (r, g) ends with out[token r][column 4g .. 4g + 3].
+// waves of a workgroup take four column tiles. Lane (r, g) ends with out[token r][column 4g .. 4g + 3], stored as one 8-byte
+// piece where rows allow it. Bound by memory: the rows in and out (1900 tokens, 16 heads, 128 -> 192 and back, 20 MB a
+// product: 22 us; with two-byte stores and each step's loads waited for, 30).
 // Anything else (float, odd sizes): a plain kernel, 16 tokens of one head a workgroup, x in LDS as float.
 // ---------------------------------------------------------------------------
 template <int MT>
 __global__ void __launch_bounds__(256)
 head_linear_mfma_kernel(const bf16_t* __restrict__ x, int ldx, int x_head, const bf16_t* __restrict__ W,
                         bf16_t* __restrict__ out, int ldo, int o_head, const bf16_t* __restrict__ gate, int ldg,
-                        int gate_per_head, int T, int N, int K) {
+                        int gate_per_head, int T, int N, int K, bool whole) {
   const int lane = threadIdx.x & (RA_WAVE - 1);
   const int wave = threadIdx.x / RA_WAVE;
   const int r = lane & 15, g = lane >> 4;
@@ -137,44 +139,64 @@ head_linear_mfma_kernel(const bf16_t* __restrict__ x, int ldx, int x_head, const
   const int n0 = (blockIdx.x * 4 + wave) * 16;
   const int t0 = blockIdx.y * 16 * MT;
   if (n0 >= N) return;
+  // rows past the end are a row that is there: nobody stores what becomes of them
   const bf16_t* wrow = W + ((size_t)h * N + (n0 + r < N ? n0 + r : 0)) * K;
-  const bool w_ok = n0 + r < N;
   const bf16_t* xrow[MT];
-  bool x_ok[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     const int t = t0 + mt * 16 + r;
-    x_ok[mt] = t < T;
-    xrow[mt] = x + (size_t)(x_ok[mt] ? t : 0) * ldx + (size_t)h * x_head;
+    xrow[mt] = x + (size_t)(t < T ? t : 0) * ldx + (size_t)h * x_head;
   }
   f32x4_t acc[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) acc[mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   const bf16x8_t zero = {0, 0, 0, 0, 0, 0, 0, 0};
-  for (int k0 = 0; k0 < K; k0 += 32) {
-    const int k = k0 + g * 8;
-    const bool k_ok = k < K;                          // K is a multiple of 8: a chunk is whole or absent
-    const bf16x8_t a = (w_ok && k_ok) ? *(const bf16x8_t*)(wrow + k) : zero;
+  for (int k0 = 0; k0 < K; k0 += 64) {                // two steps' loads are on their way together
+    bf16x8_t a[2], b[2][MT];
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const bf16x8_t b = (x_ok[mt] && k_ok) ? *(const bf16x8_t*)(xrow[mt] + k) : zero;
-      acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[mt], 0, 0, 0);
+    for (int s = 0; s < 2; ++s) {
+      const int k = k0 + s * 32 + g * 8;
+      const bool k_ok = k < K;                        // K is a multiple of 8: a chunk is whole or absent
+      const int at = k_ok ? k : 0;
+      a[s] = *(const bf16x8_t*)(wrow + at);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) b[s][mt] = *(const bf16x8_t*)(xrow[mt] + at);
+      if (!k_ok) {
+        a[s] = zero;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) b[s][mt] = zero;
+      }
     }
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[s], b[s][mt], acc[mt], 0, 0, 0);
   }
+  const int n = n0 + 4 * g;
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     const int t = t0 + mt * 16 + r;
     if (t >= T) continue;
+    bf16_t* o = out + (size_t)t * ldo + (size_t)h * o_head + n;
+    const bf16_t* gt = gate ? gate + (size_t)t * ldg + (gate_per_head ? (size_t)h : (size_t)h * N + n) : nullptr;
+    if (whole && n < N) {
+      f32x4_t v = acc[mt];
+      if (gate) {
+        bf16x4_t gv;
+        if (gate_per_head) gv = (bf16x4_t){gt[0], gt[0], gt[0], gt[0]};
+        else gv = *(const bf16x4_t*)gt;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] *= 1.f / (1.f + expf(-to_f32((bf16_t)gv[i])));
+      }
+      *(bf16x4_t*)o = (bf16x4_t){from_f32<bf16_t>(v[0]), from_f32<bf16_t>(v[1]), from_f32<bf16_t>(v[2]), from_f32<bf16_t>(v[3])};
+      continue;
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int n = n0 + 4 * g + i;
-      if (n >= N) continue;
+      if (n + i >= N) continue;
       float v = acc[mt][i];
-      if (gate) {
-        const float gv = to_f32(gate[(size_t)t * ldg + (gate_per_head ? (size_t)h : (size_t)h * N + n)]);
-        v *= 1.f / (1.f + expf(-gv));
-      }
-      out[(size_t)t * ldo + (size_t)h * o_head + n] = from_f32<bf16_t>(v);
+      if (gate) v *= 1.f / (1.f + expf(-to_f32(gt[gate_per_head ? 0 : i])));
+      o[i] = from_f32<bf16_t>(v);
     }
   }
 }
@@ -236,18 +258,21 @@ extern "C" int ra_head_linear(const void* x, int ldx, int x_head, const void* W,
   if (act_dtype == RA_BF16 && K % 8 == 0 && ldx % 8 == 0 && x_head % 8 == 0 && ((uintptr_t)x % 16) == 0 &&
       ((uintptr_t)W % 16) == 0) {
     const int col_groups = (N + 63) / 64;
+    // four columns of a result and of the gate in one access
+    const bool whole = N % 4 == 0 && ldo % 4 == 0 && o_head % 4 == 0 && (uintptr_t)out % 8 == 0 &&
+                       (gate == nullptr || gate_per_head || (ldg % 4 == 0 && (uintptr_t)gate % 8 == 0));
     if (n_tokens <= 16) {
       dim3 grid(col_groups, 1, H);
       head_linear_mfma_kernel<1><<<grid, 256, 0, stream>>>((const bf16_t*)x, ldx, x_head, (const bf16_t*)W,
                                                            (bf16_t*)out, ldo, o_head, (const bf16_t*)gate, ldg,
-                                                           gate_per_head, n_tokens, N, K);
+                                                           gate_per_head, n_tokens, N, K, whole);
     } else {
       const int tiles = (n_tokens + 63) / 64;
       RA_CHECK(tiles <= 65535, "head_linear: %d tokens in one launch", n_tokens);
       dim3 grid(col_groups, tiles, H);
       head_linear_mfma_kernel<4><<<grid, 256, 0, stream>>>((const bf16_t*)x, ldx, x_head, (const bf16_t*)W,
                                                            (bf16_t*)out, ldo, o_head, (const bf16_t*)gate, ldg,
-                                                           gate_per_head, n_tokens, N, K);
+                                                           gate_per_head, n_tokens, N, K, whole);
     }
     RA_LAUNCH_CHECK("head_linear");
     return 0;
