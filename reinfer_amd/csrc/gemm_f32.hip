@@ -128,8 +128,9 @@ struct F32Tile {
   const float* a;
   const float* w;
   const float* bias;
-  float* c;                                // ranges > 1: the ranges' sums, [ranges][M][N]
-  int M, N, K, lda, ldc, m_tiles, n_tiles, ranges, range_k;
+  float* c;                                // ranges > 1: the blocks' sums, [blocks][M][N]
+  int M, N, K, lda, ldc, m_tiles, n_tiles, ranges;
+  int block_k, range_blocks;               // k of a block (a multiple of 32), blocks of a range
 };
 
 // One workgroup of four waves a tile of BM rows and BN features and range of k, in 2 x 2 quarters. A stage is 32 k of both
@@ -148,7 +149,8 @@ __global__ void __launch_bounds__(256) gemm_f32_tile_kernel(F32Tile g) {
   if (at >= each || tile >= total) return;
   const int m0 = (int)(tile % g.m_tiles) * BM;
   const int z = (int)(tile / g.m_tiles % g.ranges), n0 = (int)(tile / g.m_tiles / g.ranges) * BN;
-  const int k0 = z * g.range_k, k1 = min(k0 + g.range_k, g.K), steps = (k1 - k0 + F32_BK - 1) / F32_BK;
+  const int range_k = g.block_k * g.range_blocks, block_steps = g.block_k / F32_BK;
+  const int k0 = z * range_k, k1 = min(k0 + range_k, g.K), steps = (k1 - k0 + F32_BK - 1) / F32_BK;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int a_rows = min(BM, g.M - m0), w_rows = min(BN, g.N - n0);
@@ -183,20 +185,25 @@ __global__ void __launch_bounds__(256) gemm_f32_tile_kernel(F32Tile g) {
           w_rsrc, (__attribute__((address_space(3))) void*)(to + (BM + (wave * PB + i) * 8) * F32_BK), 16,
           (int)((w_off[i] + (unsigned)k * 4u) | past), 0, 0, 0);
   };
-  f32x16_t acc[TN][TM];
+  f32x16_t acc[TN][TM], sum[TN][TM];         // of the block; of the blocks before it
 #pragma unroll
   for (int i = 0; i < TN; ++i)
 #pragma unroll
     for (int j = 0; j < TM; ++j)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = sum[i][j][e] = 0.f;
   const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BN / 2);
   const int row = lane & 31, half = lane >> 5;
 #pragma unroll
   for (int s = 0; s < STAGES - 1; ++s) fetch(s, s);
-  int buf = 0;
+  const bool cut = g.ranges > 1;
+  const int ld = cut ? g.N : g.ldc;
+  const float* b = cut ? nullptr : g.bias;
+  const bool whole = g.N % 4 == 0 && ld % 4 == 0 && (uintptr_t)g.c % 16 == 0;
+  int buf = 0, in_block = 0;
   for (int s = 0; s < steps; ++s) {
-    // this wave's loads of stage s are done when only those of the stages behind it are left, its reads of the stage that is
+    // this wave's loads of stage s are done when only those of the stages behind it are left (and, behind a block's end, its
+    // stores), its reads of the stage that is
     // asked for next when no LDS read is left
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((PA + PB) * (STAGES - 2)) : "memory");
     fetch(s + STAGES - 1, buf == 0 ? STAGES - 1 : buf - 1);
@@ -219,41 +226,57 @@ __global__ void __launch_bounds__(256) gemm_f32_tile_kernel(F32Tile g) {
             acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(y[i][e], x[j][e], acc[i][j], 0, 0, 0);
     }
     buf = buf + 1 == STAGES ? 0 : buf + 1;
-  }
-  // a lane holds row lane % 32 of the tile, features 8 (e / 4) + 4 (lane / 32) + e % 4
-  const bool cut = g.ranges > 1;
-  float* out = cut ? g.c + (size_t)z * g.M * g.N : g.c;
-  const int ld = cut ? g.N : g.ldc;
-  const float* b = cut ? nullptr : g.bias;
-  const bool whole = g.N % 4 == 0 && ld % 4 == 0 && (uintptr_t)g.c % 16 == 0;
+    if (++in_block < block_steps && s + 1 < steps) continue;
+    in_block = 0;
+    const int block = z * g.range_blocks + s / block_steps;
+    const bool first = s < block_steps, last = s + 1 == steps;
+    if (!cut) {                              // the blocks are added here, as the adding kernel does it
 #pragma unroll
-  for (int j = 0; j < TM; ++j) {
-    const int m = m0 + wm + j * 32 + row;
-    if (m >= g.M) continue;
+      for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int j = 0; j < TM; ++j)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) sum[i][j][e] = first ? acc[i][j][e] : sum[i][j][e] + acc[i][j][e];
+    }
+    if (cut || last) {
+      // a lane holds row lane % 32 of the tile, features 8 (e / 4) + 4 (lane / 32) + e % 4
+      float* out = cut ? g.c + (size_t)block * g.M * g.N : g.c;
+#pragma unroll
+      for (int j = 0; j < TM; ++j) {
+        const int m = m0 + wm + j * 32 + row;
+        if (m >= g.M) continue;
+#pragma unroll
+        for (int i = 0; i < TN; ++i)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const int n = n0 + wn + i * 32 + q * 8 + half * 4;
+            if (n >= g.N) continue;
+            f32x4_t v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              v[e] = cut ? acc[i][j][q * 4 + e] : sum[i][j][q * 4 + e];
+              if (b && n + e < g.N) v[e] += b[n + e];
+            }
+            if (whole) {
+              *(f32x4_t*)(out + (size_t)m * ld + n) = v;
+            } else {
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                if (n + e < g.N) out[(size_t)m * ld + n + e] = v[e];
+            }
+          }
+      }
+    }
 #pragma unroll
     for (int i = 0; i < TN; ++i)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int n = n0 + wn + i * 32 + q * 8 + half * 4;
-        if (n >= g.N) continue;
-        f32x4_t v;
+      for (int j = 0; j < TM; ++j)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          v[e] = acc[i][j][q * 4 + e];
-          if (b && n + e < g.N) v[e] += b[n + e];
-        }
-        if (whole) {
-          *(f32x4_t*)(out + (size_t)m * ld + n) = v;
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (n + e < g.N) out[(size_t)m * ld + n + e] = v[e];
-        }
-      }
+        for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
   }
 }
 
-// C = the ranges' sums added in range order (+ bias): a workgroup takes 1024 features of a row, four a thread, read 16 bytes at
+// C = the blocks' sums added in their order (+ bias): a workgroup takes 1024 features of a row, four a thread, read 16 bytes at
 // a time where rows allow it. It is bound by reading the planes.
 __global__ void __launch_bounds__(256)
 gemm_f32_add_kernel(const float* __restrict__ part, int ranges, const float* __restrict__ bias, float* __restrict__ C,
@@ -279,28 +302,34 @@ gemm_f32_add_kernel(const float* __restrict__ part, int ranges, const float* __r
   }
 }
 
-// The tile kernel's plan: tiles of 64 x 128 or 64 x 64 and as many K ranges of at least 256 k as price lowest: a CU's share
-// of the workgroups at the share of the matrix cores' rate that so many side by side reach (measured), and the ranges' sums
-// written and read again. (300 x 2560 x 9728: 64 x 64 uncut 185 us, in 5 ranges 149; 48 x 19456 x 2560: uncut 86 us, in 5 68.)
+// The tile kernel's plan. K is summed in up to eight blocks of at least 512 k whose number follows from K alone, and their sums
+// are added in order, in the registers of one workgroup or from planes by the adding kernel: a row's result does not depend on
+// how many rows stand beside it. What depends on them is the price: tiles of 64 x 128 or 64 x 64, and how many blocks a
+// workgroup takes; a CU's share of the workgroups at the share of the matrix cores' rate that so many side by side reach
+// (measured), and the planes written and read again.
 struct TilePlan {
-  int bn, ranges, range_k;
+  int bn, blocks, block_k, range_blocks, ranges;
 };
 TilePlan tile_plan(int M, int N, int K) {
   const long cus = ra_cu_count();
   const double reached[2][3] = {{0.70, 0.78, 0.81}, {0.79, 0.85, 0.87}};
+  int blocks = K / 512;
+  blocks = blocks < 1 ? 1 : blocks > 8 ? 8 : blocks;
+  const int block_k = ((K + blocks - 1) / blocks + F32_BK - 1) / F32_BK * F32_BK;
+  blocks = (K + block_k - 1) / block_k;
   TilePlan best = {};
   double best_us = 0.0;
   for (int wide = 0; wide < 2; ++wide) {
     const int bn = wide ? 128 : 64;
     const long tiles = (long)((M + 63) / 64) * ((N + bn - 1) / bn);
-    const double tile_us = 64.0 * bn * 2.0 * K / 614e3;                       // one tile at a CU's full rate
-    for (int r = 1; r <= 16 && (r == 1 || K / r >= 256); ++r) {
-      const long load = (tiles * r + cus - 1) / cus;
-      double us = (double)load / r * tile_us / reached[wide][load < 3 ? load - 1 : 2];
-      if (r > 1) us += 3.0 + (double)r * M * N * 8.0 / 5e6;
+    const double block_us = 64.0 * bn * 2.0 * block_k / 614e3;                // one tile's block at a CU's full rate
+    for (int take = blocks; take >= 1; --take) {
+      const int ranges = (blocks + take - 1) / take;
+      const long load = (tiles * ranges + cus - 1) / cus;
+      double us = (double)load * take * block_us / reached[wide][load < 3 ? load - 1 : 2];
+      if (ranges > 1) us += 3.0 + (double)blocks * M * N * 8.0 / 5e6;
       if (best.bn == 0 || us < best_us) {
-        const int range_k = ((K + r - 1) / r + F32_BK - 1) / F32_BK * F32_BK;
-        best = {bn, (K + range_k - 1) / range_k, range_k};
+        best = {bn, blocks, block_k, take, ranges};
         best_us = us;
       }
     }
@@ -313,14 +342,16 @@ TilePlan tile_plan(int M, int N, int K) {
 #define F32_STREAM_ROWS 32
 
 extern "C" int ra_gemm_f32_supports(const void* A, const void* W, int K, int lda) {
-  // a tile's rows are addressed from its first one in 31 bits
-  return K > 0 && K % 4 == 0 && lda < (1 << 21) && K < (1 << 21) && ra_rows_16b(A, lda, 4) && ra_rows_16b(W, K, 4);
+  // Sums of fewer than 512 k stay in the plain kernel's one chain: they belong to layers so small that a launch is most of
+  // either's time, and a read-out that divides by a sum with cancellation shows the order of theirs a thousandfold. A tile's
+  // rows are addressed from its first one in 31 bits.
+  return K >= 512 && K % 4 == 0 && lda < (1 << 21) && K < (1 << 21) && ra_rows_16b(A, lda, 4) && ra_rows_16b(W, K, 4);
 }
 
 extern "C" long ra_gemm_f32_scratch(int M, int N, int K) {
   if (M <= F32_STREAM_ROWS) return 0;
   const TilePlan p = tile_plan(M, N, K);
-  return p.ranges > 1 ? (long)p.ranges * M * N : 0;
+  return p.ranges > 1 ? (long)p.blocks * M * N : 0;
 }
 
 extern "C" int ra_gemm_f32(const float* A, const float* W, const float* bias, float* C, int M, int N, int K, int lda,
@@ -351,9 +382,10 @@ extern "C" int ra_gemm_f32(const float* A, const float* W, const float* bias, fl
   }
   const TilePlan p = tile_plan(M, N, K);
   const bool cut = p.ranges > 1;
-  RA_CHECK(!cut || (scratch && scratch_floats >= (long)p.ranges * M * N), "gemm_f32: scratch of %ld floats, needs %ld",
-           scratch_floats, (long)p.ranges * M * N);
-  F32Tile g = {A, W, bias, cut ? scratch : C, M, N, K, lda, ldc, (M + 63) / 64, (N + p.bn - 1) / p.bn, p.ranges, p.range_k};
+  RA_CHECK(!cut || (scratch && scratch_floats >= (long)p.blocks * M * N), "gemm_f32: scratch of %ld floats, needs %ld",
+           scratch_floats, (long)p.blocks * M * N);
+  F32Tile g = {A, W, bias, cut ? scratch : C, M, N, K, lda, ldc, (M + 63) / 64, (N + p.bn - 1) / p.bn, p.ranges,
+               p.block_k, p.range_blocks};
   const long total = (long)g.m_tiles * g.n_tiles * g.ranges, blocks = (total + RA_XCDS - 1) / RA_XCDS * RA_XCDS;
   RA_CHECK(blocks <= 0x7FFFFFFFL, "gemm_f32: [%d, %d] in one launch", M, N);
   if (p.bn == 128) gemm_f32_tile_kernel<64, 128, 2><<<(unsigned)blocks, 256, 0, stream>>>(g);
@@ -361,7 +393,7 @@ extern "C" int ra_gemm_f32(const float* A, const float* W, const float* bias, fl
   RA_LAUNCH_CHECK("gemm_f32");
   if (cut) {
     const bool whole = N % 4 == 0 && ldc % 4 == 0 && (uintptr_t)C % 16 == 0 && (uintptr_t)scratch % 16 == 0;
-    gemm_f32_add_kernel<<<dim3(M, (N + 1023) / 1024), 256, 0, stream>>>(scratch, p.ranges, bias, C, M, N, ldc, whole);
+    gemm_f32_add_kernel<<<dim3(M, (N + 1023) / 1024), 256, 0, stream>>>(scratch, p.blocks, bias, C, M, N, ldc, whole);
     RA_LAUNCH_CHECK("gemm_f32 (ranges)");
   }
   return 0;
