@@ -15,8 +15,9 @@
 // there; two stages and one barrier a step. The float matrix cores do 256 flops a clock and CU and bound it: a workgroup
 // alone on a CU keeps them 79 % busy, with others beside it 87 %. Tiles of 64 x 128 leave room in LDS for three workgroups
 // whose waits fall at different times; 128 x 128 with two or four stages had them 70 to 83 % busy, deeper rings changed
-// nothing. 1190 x 19456 x 2560 takes 0.94 ms (127 TFLOP/s of 157; through registers into LDS, in tiles of 128 x 128, 1.18 ms),
-// 2048 x 19456 x 2560 1.52 (1.92), 300 rows 269 us (360), 300 x 2560 x 9728 149 us (191; the plain kernel 1350).
+// nothing. 1119 x 19456 x 2560 takes 0.97 ms inside a prompt (115 TFLOP/s of 157; through registers into LDS, in tiles of
+// 128 x 128, 1.18 ms), the other three products of such a layer 441 us on average (480). K is summed in blocks (below), which
+// costs a second set of sums: uncut and in one chain the first took 0.94 ms.
 #include "common.h"
 #include "reinfer_hip.h"
 
