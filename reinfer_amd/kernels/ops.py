@@ -1138,10 +1138,13 @@ class HipKernels:
         """The matrix memory over the step's tokens, request by request in order, from and into ``state``
         [slots, floats]. ``proj`` [T, *] holds q and k (heads x key_dim) and v (heads x value_dim) from the
         given columns; ``gates`` float32 [T, 2 heads] holds the input and forget gates' pre-activations;
-        ``out`` float32 [T, heads * value_dim] gets the read-out before its norm. ``chunks`` forces the form (None: by the
-        step's longest portion)."""
+        ``out`` float32 [T, heads * value_dim] gets the read-out before its norm. ``chunks`` forces the form (None: float32
+        rows token by token, else by the step's longest portion). The read-out divides by a sum that may cancel a thousandfold
+        and shows every change in the order of sums by as much: the 32-bit path keeps one order."""
         _dev(proj, gates, gate_bias, state, out)
         T = proj.shape[0]
+        if chunks is None and proj.dtype == torch.float32:
+            chunks = False
         self._check_scan("matrix_memory_scan", state, batch, T)
         if proj.dim() != 2 or proj.stride(1) != 1 or max(q_off, k_off) + heads * key_dim > proj.shape[1] \
                 or v_off + heads * value_dim > proj.shape[1]:
@@ -1191,7 +1194,8 @@ class HipKernels:
                         out: torch.Tensor, chunks: Optional[bool] = None) -> None:
         """The gated delta rule over the step's tokens from and into ``state``. ``qkv`` float32 [T, q | k | v]
         as ``delta_rule_prepare`` left it; ``gates`` float32 [T, 2 heads] holds the pre-activations of beta
-        and of the decay and is overwritten with both; ``out`` float32 [T, heads * value_dim]."""
+        and of the decay and is overwritten with both; ``out`` float32 [T, heads * value_dim]. ``chunks`` forces the form
+        (None: by the step's longest portion)."""
         _dev(qkv, gates, a_log, dt_bias, state, out)
         T = qkv.shape[0]
         C = 2 * key_heads * key_dim + heads * value_dim
