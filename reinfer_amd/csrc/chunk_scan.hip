@@ -118,10 +118,11 @@ __global__ void __launch_bounds__(256) chunk_prepare_kernel(ChunkArgs p) {
   float* Lm = Am + CS_C * CS_VP;
   float* Tm = Lm + CS_C * CS_VP;
   float* Mm = Tm + CS_C * CS_VP;
-  // TOKEN: log2 of the factors' products, in 64 bits (behind a few factors near zero the difference of two of them keeps its
-  // place behind the point), and the weight of a token's write
+  // TOKEN: log2 of the factors' products, in 64 bits from the factors on (behind a few factors near zero the difference of two
+  // of them keeps its place behind the point), the products B_r / B_j and B_r, rounded to float once, and the weight of a
+  // token's write
   __shared__ double log_b[CS_C];
-  __shared__ float beta[CS_C];
+  __shared__ float ratio[CS_C][CS_C], b_to[CS_C], beta[CS_C];
   const int tid = threadIdx.x, lane = tid & (RA_WAVE - 1), wave = tid / RA_WAVE;
   const int r = lane & 15, g = lane >> 4;
   const int place = blockIdx.x / p.H, head = blockIdx.x % p.H;
@@ -144,8 +145,9 @@ __global__ void __launch_bounds__(256) chunk_prepare_kernel(ChunkArgs p) {
   if (TOKEN && tid < CS_C) {
     const int ng = MEMORY ? 3 : 2;
     const float* gt = p.gates + (size_t)(t0 + tid) * ng * p.H + head;
-    // a factor that is zero in float: 2^-1000 is, too, and its logarithms can be added and subtracted
-    double l = tid < n ? fmaxf(log2f(gt[DELTA ? p.H : 0]), -1000.f) : 0.f;
+    // a factor that is zero in float: 2^-1000 is, too, and its logarithms can be added and subtracted; NaN stays
+    const float factor = tid < n ? gt[DELTA ? p.H : 0] : 1.f;
+    double l = factor == 0.f ? -1000.0 : log2((double)factor);
     beta[tid] = tid < n ? gt[DELTA ? 0 : p.H] : 0.f;
     if (MEMORY) W[L.w + tid] = tid < n ? gt[2 * p.H] : 1.f;
 #pragma unroll
@@ -275,7 +277,11 @@ __global__ void __launch_bounds__(256) chunk_prepare_kernel(ChunkArgs p) {
     float s = 0.f;
 #pragma unroll
     for (int w = 0; w < 4; ++w) s += red[(w * CS_C + j) * CS_VP + r];
-    const float f = CHANNEL ? 1.f : TOKEN ? __builtin_amdgcn_exp2f((float)(log_b[r] - log_b[j < r ? j : r])) : power(d, r - j);
+    const float f = CHANNEL ? 1.f : TOKEN ? (float)exp2(log_b[r] - log_b[j < r ? j : r]) : power(d, r - j);
+    if (TOKEN) {
+      ratio[r][j] = f;
+      if (tid < CS_C) b_to[tid] = (float)exp2(log_b[tid]);
+    }
     s = r >= j ? s * f : 0.f;
     W[L.a + tid] = s;
     if (DELTA) {
@@ -286,8 +292,8 @@ __global__ void __launch_bounds__(256) chunk_prepare_kernel(ChunkArgs p) {
       Lm[r * CS_VP + j] = j < r ? beta[r] * f * l : 0.f;
     }
   }
+  if (TOKEN) __syncthreads();
   if (DELTA) {
-    __syncthreads();
     float t[CS_C];
     if (tid < CS_C) {                                // a thread a column of T = (I + L)^-1
 #pragma unroll
@@ -300,7 +306,7 @@ __global__ void __launch_bounds__(256) chunk_prepare_kernel(ChunkArgs p) {
     }
     __syncthreads();
     if (tid < CS_C) {
-      const float b = beta[tid], bb = b * __builtin_amdgcn_exp2f((float)log_b[tid]);
+      const float b = beta[tid], bb = b * b_to[tid];
 #pragma unroll
       for (int i = 0; i < CS_C; ++i) {
         Lm[i * CS_VP + tid] = t[i] * b;              // L itself is done with
@@ -318,11 +324,11 @@ __global__ void __launch_bounds__(256) chunk_prepare_kernel(ChunkArgs p) {
 
   // ---- operands in the products' order: a wave's lane (r, g) holds row r, columns 4 g + i of a tile of q, rows 4 g + i,
   // column r of one of k or v
-  const float fq = CHANNEL ? 1.f : TOKEN ? __builtin_amdgcn_exp2f((float)log_b[r]) : power(d, r + 1);
+  const float fq = CHANNEL ? 1.f : TOKEN ? b_to[r] : power(d, r + 1);
   float fk[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i)                        // rows past n are zeros
-    fk[i] = CHANNEL ? 1.f : TOKEN ? __builtin_amdgcn_exp2f((float)(log_b[CS_C - 1] - log_b[4 * g + i])) : power(d, max(n - 1 - (4 * g + i), 0));
+    fk[i] = CHANNEL ? 1.f : TOKEN ? ratio[CS_C - 1][4 * g + i] : power(d, max(n - 1 - (4 * g + i), 0));
   f32x4_t tb = {0.f, 0.f, 0.f, 0.f}, mm = tb, tv = tb;      // CS_DELTA: row r, columns 4 g + i of the 16 x 16 matrices
   if (DELTA) {
     tb = *(const f32x4_t*)(Tm + r * CS_VP + 4 * g);
@@ -354,7 +360,7 @@ __global__ void __launch_bounds__(256) chunk_prepare_kernel(ChunkArgs p) {
     if (DELTA) *(f32x4_t*)(W + L.w + (nt * RA_WAVE + lane) * 4) = w;
     *(f32x4_t*)(W + (nt * RA_WAVE + lane) * 4) = q;
     *(f32x4_t*)(W + L.k + (nt * RA_WAVE + lane) * 4) = k;
-    if (lane < 16) W[L.b + nt * 16 + r] = CHANNEL ? __builtin_amdgcn_exp2f(bc) : TOKEN ? __builtin_amdgcn_exp2f((float)log_b[CS_C - 1]) : power(d, n);
+    if (lane < 16) W[L.b + nt * 16 + r] = CHANNEL ? __builtin_amdgcn_exp2f(bc) : TOKEN ? b_to[CS_C - 1] : power(d, n);
   }
   for (int cg = wave; cg < (p.dv + p.group - 1) / p.group; cg += 4) {
     const int col = r < p.group ? cg * p.group + r : p.dv;

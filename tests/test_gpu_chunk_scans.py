@@ -101,3 +101,52 @@ def test_delta_rule_in_chunks(H, G, dk, dv, spread):
         close(out, out_ref, 3e-5, f"call {n}")
         untouched = [s for s in range(4) if s not in slots]
         assert torch.equal(torch.nan_to_num(st_gpu[untouched], nan=7.0), torch.nan_to_num(before[untouched], nan=7.0))
+
+
+@pytest.mark.parametrize("kind", ["memory", "delta"])
+@pytest.mark.parametrize("gate", [0, 1])                 # input and forget gate; beta and decay
+@pytest.mark.parametrize("at", [0, 20, 47])
+def test_a_gate_that_is_no_number_stays_one(kind, gate, at):
+    """From its token on, and in the state it leaves, as in the token-by-token scans; the chunks before it and the other head
+    know nothing of it (tokens before it in its own chunk may: they share its products)."""
+    ops = kernels.current()
+    g = torch.Generator().manual_seed(at)
+    H, dk, dv, T = 2, 64, 24, 50
+    rows = torch.randn(T, 2 * H * dk + H * dv, generator=g) * 0.5
+    gates = torch.randn(T, 2 * H, generator=g)
+    gates[at, gate * H] = float("nan")
+    found = []
+    for chunks in (True, False):
+        batch, out = make_batch([T], [0], [1], DEV), torch.zeros(T, H * dv, device=DEV)
+        st = torch.zeros(1, ops.scan_state_floats("matrix_memory" if kind == "memory" else "delta_rule", H, dk, dv), device=DEV)
+        more = [torch.full((n,), 0.1, device=DEV) for n in (2 * H, H, H)]
+        if kind == "memory":
+            ops.matrix_memory_scan(rows.to(DEV), 0, H * dk, 2 * H * dk, gates.to(DEV), more[0], st, batch, H, dk, dv, 15.0,
+                                   dk ** -0.5, 1e-6, out, chunks=chunks)
+        else:
+            ops.delta_rule_scan(rows.to(DEV), gates.to(DEV), more[1], more[2], st, batch, H, H, dk, dv, out, chunks=chunks)
+        found.append((torch.isnan(out).cpu().view(T, H, dv), torch.isnan(st).cpu()))
+    (chunked, chunked_state), (single, single_state) = found
+    assert torch.equal(chunked_state, single_state)
+    assert single[at:, 0].all() and not single[:at].any() and chunked[at:, 0].all()
+    assert not chunked[:at // 16 * 16].any() and not chunked[:, 1].any()
+
+
+def test_errors_in_chunks_are_those_of_single_tokens():
+    """Over gates from mild to vanishing, 400 tokens: the read-outs' errors in units of one rounding of their terms' sizes."""
+    ops = kernels.current()
+    for H, dk, dv in ((2, 128, 64), (1, 20, 12)):
+        for spread, base in ((1.0, 3.0), (3.0, 0.0), (30.0, 0.0)):
+            g = torch.Generator().manual_seed(dk)
+            T, off = 400, (0, H * dk, 2 * H * dk)
+            proj = (torch.randn(T, 2 * H * dk + H * dv, generator=g) * 0.7).to(torch.bfloat16)
+            gates, bias = torch.randn(T, 2 * H, generator=g) * spread, torch.cat([torch.zeros(H), torch.full((H,), base)])
+            want, size = matrix_memory(proj, *off, gates, bias, {}, make_batch([T], [0], [1], "cpu"), H, dk, dv, 15.0, 1e-6)
+            errs = []
+            for chunks in (True, False):
+                out, st = torch.empty(T, H * dv, device=DEV), torch.zeros(1, ops.scan_state_floats("matrix_memory", H, dk, dv), device=DEV)
+                ops.matrix_memory_scan(proj.to(DEV), *off, gates.to(DEV), bias.to(DEV), st, make_batch([T], [0], [1], DEV), H,
+                                       dk, dv, 15.0, dk ** -0.5, 1e-6, out, chunks=chunks)
+                errs.append(float(((out.double().cpu() - want) / (size * 2.0 ** -24 + 1e-30)).pow(2).mean().sqrt()))
+            # both are sums of some thousands of independent roundings: their root mean squares are known to a few percent
+            assert errs[0] <= 1.15 * errs[1], (H, dk, spread, errs)
