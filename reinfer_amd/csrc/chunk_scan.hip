@@ -67,6 +67,7 @@ struct ChunkArgs {
   int group;                                         // columns of v a workgroup: 16, or 12 or 8 and the normaliser
   float* state; long slot_stride;
   const int* cu_tokens; const int* state_slots; const int* fresh;
+  int from;                                          // tokens of a portion from which it is taken so: shorter ones are left alone
   int n_seqs, n_tokens, H, dk, dv, dkp, waves_per_head, wave_floats, R, NPL, CPW;
   int vec;                                           // rows of q and k in whole 16-byte pieces of 8 elements
   float* ops;                                        // the prepared operands
@@ -133,7 +134,8 @@ __global__ void __launch_bounds__(256) chunk_prepare_kernel(ChunkArgs p) {
     else hi = mid - 1;
   }
   const int t0 = p.cu_tokens[lo] + (place - chunk_base(p.cu_tokens, lo)) * CS_C, last = p.cu_tokens[lo + 1];
-  if (t0 >= last || p.state_slots[lo] < 0) return;   // a place nobody has, or a padding row
+  // a place nobody has, a portion that goes token by token, or a padding row
+  if (t0 >= last || last - p.cu_tokens[lo] < p.from || p.state_slots[lo] < 0) return;
   const int n = min(CS_C, last - t0);
   const ChunkLayout L = chunk_layout(dkp, p.dv, p.group, DELTA);
   float* W = p.ops + ((size_t)place * p.H + head) * L.floats;
@@ -399,6 +401,7 @@ __global__ void __launch_bounds__(WAVES * RA_WAVE) chunk_carry_kernel(ChunkArgs 
   if (unit >= p.n_seqs * p.H) return;
   const int seq = unit / p.H, head = unit % p.H;
   const int first = p.cu_tokens[seq], last = p.cu_tokens[seq + 1];
+  if (last - first < p.from) return;
   const int slot = p.state_slots[seq];
   const size_t ow = (size_t)p.H * p.dv;
   float* out = p.out + (size_t)head * p.dv + cg * GC;
@@ -552,6 +555,7 @@ __global__ void __launch_bounds__(WAVES * RA_WAVE) chunk_carry_delta_kernel(Chun
   if (unit >= p.n_seqs * p.H) return;
   const int seq = unit / p.H, head = unit % p.H;
   const int first = p.cu_tokens[seq], last = p.cu_tokens[seq + 1];
+  if (last - first < p.from) return;
   const int slot = p.state_slots[seq];
   const size_t ow = (size_t)p.H * p.dv;
   float* out = p.out + (size_t)head * p.dv + cg * 16;
@@ -726,8 +730,9 @@ extern "C" long ra_chunk_scratch_floats(int kind, int n_tokens, int n_seqs, int 
 int ra_matrix_memory_chunks(const void* proj, int act_dtype, int ld, int q_off, int k_off, int v_off, const float* gates3,
                             float* state, long slot_stride, const int* cu_tokens, const int* state_slots, const int* fresh,
                             int n_seqs, int n_tokens, int heads, int key_dim, int value_dim, float q_scale, float denom_eps,
-                            float* scratch, long scratch_floats, float* out, hipStream_t stream) {
+                            float* scratch, long scratch_floats, int from, float* out, hipStream_t stream) {
   ChunkArgs a = {};
+  a.from = from;
   a.n_seqs = n_seqs; a.n_tokens = n_tokens; a.H = heads; a.dk = key_dim; a.dv = value_dim;
   a.cu_tokens = cu_tokens; a.state_slots = state_slots; a.fresh = fresh; a.ops = scratch; a.out = out;
   a.q_scale = q_scale; a.k_scale = 1.f; a.gates = gates3; a.denom_eps = denom_eps;
@@ -739,8 +744,9 @@ int ra_matrix_memory_chunks(const void* proj, int act_dtype, int ld, int q_off, 
 
 int ra_delta_rule_chunks(const float* qkv, int ld, const float* gates, float* state, long slot_stride, const int* cu_tokens,
                          const int* state_slots, const int* fresh, int n_seqs, int n_tokens, int heads, int key_heads,
-                         int key_dim, int value_dim, float* scratch, long scratch_floats, float* out, hipStream_t stream) {
+                         int key_dim, int value_dim, float* scratch, long scratch_floats, int from, float* out, hipStream_t stream) {
   ChunkArgs a = {};
+  a.from = from;
   a.n_seqs = n_seqs; a.n_tokens = n_tokens; a.H = heads; a.dk = key_dim; a.dv = value_dim; a.q_heads = key_heads;
   a.cu_tokens = cu_tokens; a.state_slots = state_slots; a.fresh = fresh; a.ops = scratch; a.out = out;
   a.q_scale = 1.f; a.k_scale = 1.f; a.gates = gates;

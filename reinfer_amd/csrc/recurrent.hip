@@ -70,6 +70,7 @@ struct ScanArgs {
   float* state; long slot_stride;
   const int* cu_tokens; const int* state_slots; const int* fresh;
   int H, dk, dv, waves_per_head, wave_floats, chunk;
+  int below;                                         // portions of so many tokens and more are left alone (0: none are)
   float q_scale, denom_eps;
   float* out;
   // wkv: the decays' pre-activations, float [T, H dk] with rows ldw apart, their bias w0 [H dk] and the bonus u [H dk]
@@ -101,6 +102,7 @@ __global__ __launch_bounds__(256) void scan_kernel(ScanArgs p) {
   const int col = w * CPW + c;
   const bool col_ok = active && col < p.dv;
   const int first = p.cu_tokens[seq], last = p.cu_tokens[seq + 1];
+  if (p.below > 0 && last - first >= p.below) return;
   const int slot = p.state_slots[seq];
   const int ow = p.H * p.dv;
   const int H = p.H, dk = p.dk, dv = p.dv, CT = p.chunk;
@@ -776,7 +778,7 @@ extern "C" int ra_matrix_memory_scan(const void* proj, int act_dtype, int ld, in
                                      const int* cu_tokens, const int* state_slots, const int* fresh, int n_seqs,
                                      int n_tokens, int max_q_len, int heads, int key_dim, int value_dim,
                                      float gate_cap, float q_scale, float denom_eps, float* scratch, long scratch_floats,
-                                     float* out, hipStream_t stream) {
+                                     int chunk_from, float* out, hipStream_t stream) {
   RA_CHECK(n_seqs > 0 && n_tokens > 0 && heads > 0, "matrix_memory_scan: %d requests, %d tokens, %d heads", n_seqs,
            n_tokens, heads);
   ScanGeom g;
@@ -791,10 +793,13 @@ extern "C" int ra_matrix_memory_scan(const void* proj, int act_dtype, int ld, in
       gates, gate_bias, gate_cap, gates3, state, slot_stride, (long)g.waves * g.wave_floats,
       (long)g.NPL * RA_WAVE + (long)g.NPL * g.R, cu_tokens, state_slots, fresh, heads);
   RA_LAUNCH_CHECK("matrix_memory_gates");
-  if (scratch)
-    return ra_matrix_memory_chunks(proj, act_dtype, ld, q_off, k_off, v_off, gates3, state, slot_stride, cu_tokens, state_slots,
-                                   fresh, n_seqs, n_tokens, heads, key_dim, value_dim, q_scale, denom_eps, scratch,
-                                   scratch_floats, out, stream);
+  if (scratch) {
+    const int rc = ra_matrix_memory_chunks(proj, act_dtype, ld, q_off, k_off, v_off, gates3, state, slot_stride, cu_tokens,
+                                           state_slots, fresh, n_seqs, n_tokens, heads, key_dim, value_dim, q_scale, denom_eps,
+                                           scratch, scratch_floats, chunk_from, out, stream);
+    if (rc != 0 || chunk_from <= 1) return rc;
+    if (max_q_len <= 0 || max_q_len >= chunk_from) max_q_len = chunk_from - 1;
+  }
   const ScanLaunch L = scan_launch(g, n_seqs, heads, max_q_len);
   const size_t es = act_dtype == RA_F32 ? 4 : 2;
   ScanArgs a = {};
@@ -804,7 +809,7 @@ extern "C" int ra_matrix_memory_scan(const void* proj, int act_dtype, int ld, in
   a.ld = ld; a.q_heads = heads; a.gates = gates3; a.state = state; a.slot_stride = slot_stride;
   a.cu_tokens = cu_tokens; a.state_slots = state_slots; a.fresh = fresh;
   a.H = heads; a.dk = key_dim; a.dv = value_dim; a.waves_per_head = g.waves; a.wave_floats = g.wave_floats;
-  a.chunk = L.chunk; a.q_scale = q_scale; a.denom_eps = denom_eps; a.out = out;
+  a.chunk = L.chunk; a.below = scratch ? chunk_from : 0; a.q_scale = q_scale; a.denom_eps = denom_eps; a.out = out;
   if (act_dtype == RA_F32) scan_dispatch<float, SCAN_MEMORY>(g, L, a, stream);
   else scan_dispatch<bf16_t, SCAN_MEMORY>(g, L, a, stream);
   RA_LAUNCH_CHECK("matrix_memory_scan");
@@ -862,8 +867,8 @@ extern "C" int ra_delta_rule_prepare(const void* proj, int act_dtype, int ld, co
 extern "C" int ra_delta_rule_scan(const float* qkv, int ld, float* gates, const float* a_log, const float* dt_bias,
                                   float* state, long slot_stride, const int* cu_tokens, const int* state_slots,
                                   const int* fresh, int n_seqs, int n_tokens, int max_q_len, int heads, int key_heads,
-                                  int key_dim, int value_dim, float* scratch, long scratch_floats, float* out,
-                                  hipStream_t stream) {
+                                  int key_dim, int value_dim, float* scratch, long scratch_floats, int chunk_from,
+                                  float* out, hipStream_t stream) {
   RA_CHECK(n_seqs > 0 && n_tokens > 0 && heads > 0 && key_heads > 0 && heads % key_heads == 0,
            "delta_rule_scan: %d requests, %d tokens, %d heads on %d key heads", n_seqs, n_tokens, heads, key_heads);
   ScanGeom g;
@@ -874,9 +879,12 @@ extern "C" int ra_delta_rule_scan(const float* qkv, int ld, float* gates, const 
   const long n = (long)n_tokens * 2 * heads;
   delta_rule_gates_kernel<<<(unsigned)((n + 255) / 256), 256, 0, stream>>>(gates, a_log, dt_bias, heads, n);
   RA_LAUNCH_CHECK("delta_rule_gates");
-  if (scratch)
-    return ra_delta_rule_chunks(qkv, ld, gates, state, slot_stride, cu_tokens, state_slots, fresh, n_seqs, n_tokens, heads,
-                                key_heads, key_dim, value_dim, scratch, scratch_floats, out, stream);
+  if (scratch) {
+    const int rc = ra_delta_rule_chunks(qkv, ld, gates, state, slot_stride, cu_tokens, state_slots, fresh, n_seqs, n_tokens,
+                                        heads, key_heads, key_dim, value_dim, scratch, scratch_floats, chunk_from, out, stream);
+    if (rc != 0 || chunk_from <= 1) return rc;
+    if (max_q_len <= 0 || max_q_len >= chunk_from) max_q_len = chunk_from - 1;
+  }
   const ScanLaunch L = scan_launch(g, n_seqs, heads, max_q_len);
   ScanArgs a = {};
   a.q = qkv;
@@ -885,7 +893,7 @@ extern "C" int ra_delta_rule_scan(const float* qkv, int ld, float* gates, const 
   a.ld = ld; a.q_heads = key_heads; a.gates = gates; a.state = state; a.slot_stride = slot_stride;
   a.cu_tokens = cu_tokens; a.state_slots = state_slots; a.fresh = fresh;
   a.H = heads; a.dk = key_dim; a.dv = value_dim; a.waves_per_head = g.waves; a.wave_floats = g.wave_floats;
-  a.chunk = L.chunk; a.q_scale = 1.f; a.denom_eps = 0.f; a.out = out;
+  a.chunk = L.chunk; a.below = scratch ? chunk_from : 0; a.q_scale = 1.f; a.denom_eps = 0.f; a.out = out;
   scan_dispatch<float, SCAN_DELTA>(g, L, a, stream);
   RA_LAUNCH_CHECK("delta_rule_scan");
   return 0;

@@ -5,7 +5,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
-#define RA_ABI_VERSION 26
+#define RA_ABI_VERSION 27
 
 #ifdef __cplusplus
 extern "C" {
@@ -378,23 +378,24 @@ long ra_scan_state_floats(int kind, int heads, int key_dim, int value_dim);
 // max_q_len: the most tokens a request brings (0: unknown; it only sizes the chunks that are staged)
 // gates [n_tokens, 2 heads] float pre-activations (input | forget); gates3 [n_tokens, 3 heads] scratch for the
 // decay, input and threshold factors made from them; proj rows hold q, k (heads x key_dim) and v (heads x value_dim)
-// at the given column offsets; out float [n_tokens, heads * value_dim]
+// at the given column offsets; out float [n_tokens, heads * value_dim]. scratch (ra_chunk_scratch_floats, or null): portions of
+// at least chunk_from tokens go in chunks of 16 tokens, the others, or all without scratch, token by token
 int ra_matrix_memory_scan(const void* proj, int act_dtype, int ld, int q_off, int k_off, int v_off, const float* gates,
                           float* gates3, const float* gate_bias, float* state, long slot_stride, const int* cu_tokens,
                           const int* state_slots, const int* fresh, int n_seqs, int n_tokens, int max_q_len, int heads,
                           int key_dim, int value_dim, float gate_cap, float q_scale, float denom_eps, float* scratch,
-                          long scratch_floats, float* out, hipStream_t stream);
+                          long scratch_floats, int chunk_from, float* out, hipStream_t stream);
 // proj rows hold q | k (key_heads x key_dim each) | v (heads x value_dim) from column 0; filt float [channels, taps];
 // the filter's tail lies at tail_off floats in a request's state slot; qkv float [n_tokens, channels]
 int ra_delta_rule_prepare(const void* proj, int act_dtype, int ld, const float* filt, float* state, long slot_stride,
                           long tail_off, const int* seq_of_token, const int* cu_tokens, const int* state_slots,
                           const int* fresh, int n_seqs, int n_tokens, int key_heads, int key_dim, int heads,
                           int value_dim, int taps, float unit_eps, float q_scale, float* qkv, hipStream_t stream);
-// gates [n_tokens, 2 heads] float pre-activations (b | a), turned into (beta | decay) in place
+// gates [n_tokens, 2 heads] float pre-activations (b | a), turned into (beta | decay) in place; scratch and chunk_from as above
 int ra_delta_rule_scan(const float* qkv, int ld, float* gates, const float* a_log, const float* dt_bias, float* state,
                        long slot_stride, const int* cu_tokens, const int* state_slots, const int* fresh, int n_seqs,
                        int n_tokens, int max_q_len, int heads, int key_heads, int key_dim, int value_dim, float* scratch,
-                       long scratch_floats, float* out, hipStream_t stream);
+                       long scratch_floats, int chunk_from, float* out, hipStream_t stream);
 // kind 2 of ra_scan_state_floats. proj rows hold r, k and v (heads x dim each) at the given column offsets; decay
 // float [n_tokens, >= heads dim] holds the decays' pre-activations z, the decay being exp(-exp(z + w0)); u float
 // [heads dim] is the bonus of the current token: o = (S + diag(u) k v^T)^T r, then S <- diag(decay) S + k v^T

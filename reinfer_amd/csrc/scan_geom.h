@@ -56,11 +56,11 @@ __device__ __forceinline__ void ra_sincos(float x, float* sn, float* cs) {
   *cs = ((q + 1) & 2) ? -b : b;
 }
 
-// chunk_scan.hip
+// chunk_scan.hip: portions of at least `from` tokens
 int ra_matrix_memory_chunks(const void* proj, int act_dtype, int ld, int q_off, int k_off, int v_off, const float* gates3,
                             float* state, long slot_stride, const int* cu_tokens, const int* state_slots, const int* fresh,
                             int n_seqs, int n_tokens, int heads, int key_dim, int value_dim, float q_scale, float denom_eps,
-                            float* scratch, long scratch_floats, float* out, hipStream_t stream);
+                            float* scratch, long scratch_floats, int from, float* out, hipStream_t stream);
 int ra_delta_rule_chunks(const float* qkv, int ld, const float* gates, float* state, long slot_stride, const int* cu_tokens,
                          const int* state_slots, const int* fresh, int n_seqs, int n_tokens, int heads, int key_heads,
-                         int key_dim, int value_dim, float* scratch, long scratch_floats, float* out, hipStream_t stream);
+                         int key_dim, int value_dim, float* scratch, long scratch_floats, int from, float* out, hipStream_t stream);

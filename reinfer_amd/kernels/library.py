@@ -15,7 +15,7 @@ import torch  # noqa: F401  (loads the HIP runtime the library links against)
 
 from ..csrc import build as _build
 
-ABI_VERSION = 26
+ABI_VERSION = 27
 
 
 class KernelLibraryError(RuntimeError):
@@ -74,9 +74,9 @@ _SIGNATURES = {
     "ra_moe_down_gated_chosen": [P, P, P, P, P, I, P, I, I, I, I, I, I, I, P],
     "ra_moe_route_sigmoid": [P, I, I, I, I, I, I, F, P, P, I, P],
     "ra_moe_silu_gate_scale": [P, P, I, P, P, I, I, I, I, I, P],
-    "ra_matrix_memory_scan": [P, I, I, I, I, I, P, P, P, P, c_long, P, P, P, I, I, I, I, I, I, F, F, F, P, c_long, P, P],
+    "ra_matrix_memory_scan": [P, I, I, I, I, I, P, P, P, P, c_long, P, P, P, I, I, I, I, I, I, F, F, F, P, c_long, I, P, P],
     "ra_delta_rule_prepare": [P, I, I, P, P, c_long, c_long, P, P, P, P, I, I, I, I, I, I, I, F, F, P, P],
-    "ra_delta_rule_scan": [P, I, P, P, P, P, c_long, P, P, P, I, I, I, I, I, I, I, P, c_long, P, P],
+    "ra_delta_rule_scan": [P, I, P, P, P, P, c_long, P, P, P, I, I, I, I, I, I, I, P, c_long, I, P, P],
     "ra_head_norm_gate": [P, P, I, P, I, I, I, F, I, I, I, P, P],
     "ra_normed_mean": [P, P, I, I, F, I, I, P, P, F, P],
     "ra_attention_plain_mod": [P, I, P, I, P, P, I, P, I, P, P, P, I, I, I, I, I, F, I, I, I, F, P, P, P, P, I, P],

@@ -1139,7 +1139,7 @@ class HipKernels:
         [slots, floats]. ``proj`` [T, *] holds q and k (heads x key_dim) and v (heads x value_dim) from the
         given columns; ``gates`` float32 [T, 2 heads] holds the input and forget gates' pre-activations;
         ``out`` float32 [T, heads * value_dim] gets the read-out before its norm. ``chunks`` forces the form (None: float32
-        rows token by token, else by the step's longest portion). The read-out divides by a sum that may cancel a thousandfold
+        rows token by token, else by a request's own portion). The read-out divides by a sum that may cancel a thousandfold
         and shows every change in the order of sums by as much: the 32-bit path keeps one order."""
         _dev(proj, gates, gate_bias, state, out)
         T = proj.shape[0]
@@ -1155,14 +1155,14 @@ class HipKernels:
         if out.shape != (T, heads * value_dim) or out.dtype != torch.float32 or not out.is_contiguous():
             raise ValueError("matrix_memory_scan: out is contiguous float32 [T, heads * value_dim]")
         factors = torch.empty((T, 3 * heads), dtype=torch.float32, device=proj.device)     # decay, input, threshold
-        scratch = self._scan_scratch(chunks, "matrix_memory", batch, T, heads, key_dim, value_dim, proj.device)
+        scratch, chunk_from = self._scan_scratch(chunks, "matrix_memory", batch, T, heads, key_dim, value_dim, proj.device)
         library.call("ra_matrix_memory_scan", proj.data_ptr(), _tag(proj, "matrix_memory_scan"), proj.stride(0),
                      int(q_off), int(k_off), int(v_off), gates.data_ptr(), factors.data_ptr(), gate_bias.data_ptr(),
                      state.data_ptr(),
                      state.stride(0), batch.cu_tokens.data_ptr(), batch.state_slots.data_ptr(), batch.fresh.data_ptr(),
                      batch.num_seqs, T, int(getattr(batch, "max_q_len", 0) or 0), int(heads), int(key_dim),
                      int(value_dim), float(gate_cap), float(q_scale), float(denom_eps), _ptr(scratch),
-                     scratch.numel() if scratch is not None else 0, out.data_ptr(), _stream())
+                     scratch.numel() if scratch is not None else 0, chunk_from, out.data_ptr(), _stream())
 
     def delta_rule_prepare(self, proj: torch.Tensor, filt: torch.Tensor, state: torch.Tensor, tail_off: int, batch,
                            key_heads: int, key_dim: int, heads: int, value_dim: int, taps: int, unit_eps: float,
@@ -1195,7 +1195,7 @@ class HipKernels:
         """The gated delta rule over the step's tokens from and into ``state``. ``qkv`` float32 [T, q | k | v]
         as ``delta_rule_prepare`` left it; ``gates`` float32 [T, 2 heads] holds the pre-activations of beta
         and of the decay and is overwritten with both; ``out`` float32 [T, heads * value_dim]. ``chunks`` forces the form
-        (None: by the step's longest portion)."""
+        (None: by a request's own portion)."""
         _dev(qkv, gates, a_log, dt_bias, state, out)
         T = qkv.shape[0]
         C = 2 * key_heads * key_dim + heads * value_dim
@@ -1209,12 +1209,12 @@ class HipKernels:
                 raise ValueError(f"delta_rule_scan: {what} is float32 [heads]")
         if out.shape != (T, heads * value_dim) or out.dtype != torch.float32 or not out.is_contiguous():
             raise ValueError("delta_rule_scan: out is contiguous float32 [T, heads * value_dim]")
-        scratch = self._scan_scratch(chunks, "delta_rule", batch, T, heads, key_dim, value_dim, qkv.device)
+        scratch, chunk_from = self._scan_scratch(chunks, "delta_rule", batch, T, heads, key_dim, value_dim, qkv.device)
         library.call("ra_delta_rule_scan", qkv.data_ptr(), qkv.stride(0), gates.data_ptr(), a_log.data_ptr(),
                      dt_bias.data_ptr(), state.data_ptr(), state.stride(0), batch.cu_tokens.data_ptr(),
                      batch.state_slots.data_ptr(), batch.fresh.data_ptr(), batch.num_seqs, T,
                      int(getattr(batch, "max_q_len", 0) or 0), int(heads), int(key_heads), int(key_dim), int(value_dim),
-                     _ptr(scratch), scratch.numel() if scratch is not None else 0, out.data_ptr(), _stream())
+                     _ptr(scratch), scratch.numel() if scratch is not None else 0, chunk_from, out.data_ptr(), _stream())
 
     def wkv_scan(self, proj: torch.Tensor, r_off: int, k_off: int, v_off: int, decay: torch.Tensor, w0: torch.Tensor,
                  u: torch.Tensor, state: torch.Tensor, batch, heads: int, dim: int, out: torch.Tensor) -> None:
@@ -1415,10 +1415,14 @@ class HipKernels:
             raise ValueError(f"{what}: out is contiguous float32 [T, {heads * value_dim}]")
 
     def _scan_scratch(self, chunks, kind: str, batch, T: int, heads: int, key_dim: int, value_dim: int, device):
-        """Scratch for a scan of ``kind`` in chunks, or None where it goes token by token."""
+        """(scratch, tokens of a portion from which it goes in chunks) for a scan of ``kind``; scratch is None where all go token
+        by token. A request's form follows from its own portion: its result does not depend on the requests beside it."""
+        least = 1
         if chunks is None:
             chunks = int(getattr(batch, "max_q_len", 0) or 0) >= self.CHUNK_FROM and key_dim <= self.CHUNK_KEYS
-        return self._chunk_scratch(T, batch.num_seqs, heads, key_dim, value_dim, device, kind) if chunks else None
+            if min(batch.q_lens, default=0) < self.CHUNK_FROM:
+                least = self.CHUNK_FROM
+        return (self._chunk_scratch(T, batch.num_seqs, heads, key_dim, value_dim, device, kind) if chunks else None), least
 
     @classmethod
     def _chunk_scratch(cls, T, n_seqs, heads, key_dim, value_dim, device, kind: str = "decay_memory") -> torch.Tensor:

@@ -7,8 +7,10 @@ import torch
 
 from helpers import random_tokens, run_plan
 from kobolix_helpers import _attn, _delta, _dense, _memory, draw_weights
+from reinfer_amd import kernels
 from reinfer_amd.engine import ModelRunner
 from reinfer_amd.weights.safetensors_io import write_safetensors
+from test_gpu_kobolix_kernels import DEV, make_batch
 
 pytestmark = pytest.mark.gpu
 
@@ -35,3 +37,33 @@ def test_32_bit_results_do_not_depend_on_the_requests_beside(tmp_path):
     alone = run_plan(runner, {"a": a}, [[("a", n)] for n in mine])["a"]
     beside = run_plan(runner, {"a": a, "b": b}, [[("a", n), ("b", m)] for n, m in zip(mine, [17, 50, 1, 33, 16, 30, 3])])["a"]
     assert torch.equal(alone, beside)
+
+
+@pytest.mark.parametrize("kind", ["memory", "delta"])
+@pytest.mark.parametrize("mine,others", [(1, [64]), (16, [17]), (17, [1, 1]), (40, [3, 200])])
+def test_a_scan_does_not_depend_on_the_requests_beside(kind, mine, others):
+    """bfloat16 rows, the form left to the call: a request's read-out and state alone and in the middle of a step."""
+    ops = kernels.current()
+    H, dk, dv = 3, 128, 40
+    g = torch.Generator().manual_seed(mine)
+    lens = [others[0], mine] + others[1:]
+    T, at, width = sum(lens), others[0], 2 * H * dk + H * dv
+    rows = (torch.randn(T, width, generator=g) * 0.3).to(torch.bfloat16).to(DEV)
+    gates, bias = torch.randn(T, 2 * H, generator=g).to(DEV), torch.randn(2 * H, generator=g).to(DEV)
+    floats = ops.scan_state_floats("matrix_memory" if kind == "memory" else "delta_rule", H, dk, dv)
+    state = torch.zeros(4, floats, device=DEV)
+    state[:, :] = torch.rand(4, 1, generator=g).to(DEV) * 0.1
+    found = []
+    for q_lens, slots, run in ((lens, [0, 2, 3][:len(lens)], slice(0, T)), ([mine], [2], slice(at, at + mine))):
+        batch = make_batch(q_lens, slots, [0] * len(q_lens), DEV)
+        batch.max_q_len = max(q_lens)
+        n, st = sum(q_lens), state.clone()
+        out = torch.full((n, H * dv), float("nan"), device=DEV)
+        x, z = rows[run].clone(), gates[run].clone()
+        if kind == "memory":
+            ops.matrix_memory_scan(x, 0, H * dk, 2 * H * dk, z, bias, st, batch, H, dk, dv, 15.0, dk ** -0.5, 1e-6, out)
+        else:
+            ops.delta_rule_scan(x.float(), z, bias[:H].contiguous(), bias[H:].contiguous(), st, batch, H, H, dk, dv, out)
+        assert torch.isfinite(out).all()
+        found.append((out[at:at + mine] if n == T else out, st[2]))
+    assert torch.equal(found[0][0], found[1][0]) and torch.equal(found[0][1], found[1][1])
