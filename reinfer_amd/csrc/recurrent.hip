@@ -453,11 +453,11 @@ __global__ void delta_rule_prepare_kernel(const TA* __restrict__ proj, int ld, c
         float x;
         if (rel >= 0) x = to_f32(proj[(size_t)(first + rel) * ld + ch]);
         else x = zero ? 0.f : tail[(size_t)(taps - 1 + rel) * C + ch];
-        acc += filt[(size_t)ch * taps + p] * x;
+        acc = fmaf(filt[(size_t)ch * taps + p], x, acc);
       }
       acc = acc / (1.f + expf(-acc));
       y[j] = acc;
-      ss += acc * acc;
+      ss = fmaf(acc, acc, ss);
     }
   }
   float f = 1.f;
@@ -475,8 +475,9 @@ __global__ void delta_rule_prepare_kernel(const TA* __restrict__ proj, int ld, c
 
 // The same for prompts: heads of up to 256 in steps of 4, filters of up to four taps, rows that 4-channel accesses can read. A
 // lane takes four channels and PREP_RUN tokens: its filter is loaded once, and a row of the run is read once and not once a
-// tap. A head's LANES lanes are a group of a wave, so that the sum of its squares stays inside it. Bound by its rows in and
-// results out: 1859 tokens of 8192 channels, four taps, 106 us in the kernel above, 40 here.
+// tap. A head's LANES lanes are a group of a wave, so that the sum of its squares stays inside it; the squares are added in the
+// order of the kernel above, so that a token's inputs do not depend on how many tokens stand beside it. Bound by its rows in and
+// results out: 1859 tokens of 8192 channels, four taps, 106 us in the kernel above, 43 here (40 with one sum a lane).
 #define PREP_RUN 8
 #define PREP_TAPS 4
 template <typename TA, int LANES>
@@ -518,23 +519,31 @@ delta_rule_prepare_run_kernel(const TA* __restrict__ proj, int ld, const float* 
         if (p >= taps) continue;
         if (since >= p) {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) y[i] += w[i][p] * to_f32((TA)row[r + PREP_TAPS - 1 - p][i]);
+          for (int i = 0; i < 4; ++i) y[i] = fmaf(w[i][p], to_f32((TA)row[r + PREP_TAPS - 1 - p][i]), y[i]);
         } else if (fresh[seq] == 0) {                    // a row before the portion: the request's tail
           const float* x = state + (size_t)slot * slot_stride + tail_off + (size_t)(taps - 1 + since - p) * C + ch;
 #pragma unroll
-          for (int i = 0; i < 4; ++i) y[i] += w[i][p] * x[i];
+          for (int i = 0; i < 4; ++i) y[i] = fmaf(w[i][p], x[i], y[i]);
         }
       }
-      float ss = 0.f;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        y[i] = y[i] / (1.f + expf(-y[i]));
-        ss += y[i] * y[i];
+      for (int i = 0; i < 4; ++i) y[i] = e < width ? y[i] / (1.f + expf(-y[i])) : 0.f;
+      if (!is_v) {
+        // channels 64 apart first, one after the other, then a butterfly over the bits of a channel's place in its 64
+        float ss[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          ss[i] = 0.f;
+#pragma unroll
+          for (int j = 0; j < LANES / 16; ++j) {
+            const float c = LANES == 16 ? y[i] : __shfl(y[i], (int)threadIdx.x % RA_WAVE / LANES * LANES + j * 16 + (int)threadIdx.x % 16, RA_WAVE);
+            ss[i] = fmaf(c, c, ss[i]);
+          }
+#pragma unroll
+          for (int d = 8; d > 0; d >>= 1) ss[i] += __shfl_xor(ss[i], d, RA_WAVE);
+        }
+        f = 1.f / sqrtf((ss[0] + ss[2]) + (ss[1] + ss[3]) + unit_eps);
       }
-      if (e >= width) ss = 0.f;
-#pragma unroll
-      for (int d = LANES / 2; d > 0; d >>= 1) ss += __shfl_xor(ss, d, RA_WAVE);
-      if (!is_v) f = 1.f / sqrtf(ss + unit_eps);
       if (unit < G) f *= q_scale;
     }
     if (e < width) *(f32x4_t*)(qkv + (size_t)t * C + ch) = y * f;

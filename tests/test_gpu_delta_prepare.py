@@ -36,3 +36,29 @@ def test_delta_rule_prepare_in_runs(H, G, dk, dv, taps, rows, dtype):
     st, other = state.to(DEV), torch.full((rows, C), float("nan"), device=DEV)
     ops.delta_rule_prepare(odd, filt.to(DEV), st, 8, make_batch(q_lens, slots, fresh, DEV), *args, other)
     assert ((got - other).abs() <= 1e-5 * other.abs().max()).all()
+
+
+@pytest.mark.parametrize("H,G,dk,dv", [(64, 32, 16, 20), (16, 8, 64, 48), (16, 8, 68, 96), (16, 8, 128, 128), (16, 8, 132, 256), (8, 8, 256, 40)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_a_token_alone_and_in_a_prompt_has_the_same_inputs(H, G, dk, dv, dtype):
+    """Tokens one a step, which a wave a head takes, against the same tokens as one portion in runs: the same bits."""
+    ops = kernels.current()
+    g = torch.Generator().manual_seed(dk)
+    C, rows, taps, last = 2 * G * dk + H * dv, 1203, 4, 6
+    filt = (torch.randn(C, taps, generator=g) * 0.6).to(DEV)
+    proj = torch.randn(rows, C + 4, generator=g).to(dtype).to(DEV)
+    args = (G, dk, H, dv, taps, 1e-6, 0.25)
+    st, whole = torch.zeros(1, (taps - 1) * C, device=DEV), torch.empty(rows, C, device=DEV)
+    ops.delta_rule_prepare(proj, filt, st, 0, make_batch([rows], [0], [1], DEV), *args, whole)
+    one = torch.zeros(1, (taps - 1) * C, device=DEV)
+    first = torch.empty(rows - last, C, device=DEV)
+    ops.delta_rule_prepare(proj[:-last], filt, one, 0, make_batch([rows - last], [0], [1], DEV), *args, first)
+    assert torch.equal(first, whole[:-last])
+    for t in range(rows - last, rows):
+        got = torch.empty(1, C, device=DEV)
+        ops.delta_rule_prepare(proj[t:t + 1], filt, one, 0, make_batch([1], [0], [0], DEV), *args, got)
+        assert torch.equal(got[0], whole[t]), t
+    assert torch.equal(one, st)
+    few = torch.empty(5, C, device=DEV)
+    ops.delta_rule_prepare(proj[:5], filt, torch.zeros_like(st), 0, make_batch([5], [0], [1], DEV), *args, few)
+    assert torch.equal(few, whole[:5])
