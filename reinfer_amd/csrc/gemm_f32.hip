@@ -1,44 +1,60 @@
 // Matrix products of the 32-bit path, C[M,N] = A[M,K] . W[N,K]^T (+ bias[N]), on the float matrix cores: the products are
 // full float ones and the sums are float, as in gemm_plain.hip, which keeps the rows that 16-byte accesses cannot read.
 //
-// An operand of the 16x16x4 and 32x32x2 products is one float a lane at (row, k slot). Which k a slot stands for is free as
-// long as both operands agree, so a lane reads four neighbouring k with one 16-byte access and the four products that
-// follow take one element of it each.
+// An operand of a 16x16x4 product is one float a lane at (row, k slot). Which k a slot stands for is free as long as both
+// operands agree, so a lane reads four neighbouring k with one 16-byte access and the four products that follow take one
+// element of it each.
 //
 // Up to 32 rows (gemm_f32_stream_kernel) the product is bound by reading the weights once. A workgroup has 16 features, its
 // waves share K out and add their sums through LDS in a fixed order; both operands go from memory to the matrix cores
-// without LDS. At 4 rows 19456 x 2560 takes 41 us (4.8 TB/s) and 151936 x 2560 281 us (5.5 TB/s), where the plain kernel
+// without LDS. At 4 rows 19456 x 2560 takes 41 us (4.8 TB/s) and 151936 x 2560 277 us (5.6 TB/s), where the plain kernel
 // took 406 us for the first; with more rows the activations, which every workgroup reads again, cost as much as the weights
-// (19456 x 2560 at 32 rows 96 us, as much as the other kernel at 33).
+// (19456 x 2560 at 32 rows 93 us).
 //
 // From 33 rows on (gemm_f32_tile_kernel) tiles of both operands go through LDS, 32 k at a time, by loads that go straight
-// there; two stages and one barrier a step. The float matrix cores do 256 flops a clock and CU and bound it: a workgroup
-// alone on a CU keeps them 79 % busy, with others beside it 87 %. Tiles of 64 x 128 leave room in LDS for three workgroups
-// whose waits fall at different times; 128 x 128 with two or four stages had them 70 to 83 % busy, deeper rings changed
-// nothing. 1119 x 19456 x 2560 takes 0.97 ms inside a prompt (115 TFLOP/s of 157; through registers into LDS, in tiles of
-// 128 x 128, 1.18 ms), the other three products of such a layer 441 us on average (480). K is summed in blocks (below), which
-// costs a second set of sums: uncut and in one chain the first took 0.94 ms.
+// there; two stages and one barrier a step. The float matrix cores do 256 flops a clock and CU and bound it. Tiles of 64 x 128
+// leave room in LDS for three workgroups whose waits fall at different times; 128 x 128 with two or four stages had the
+// matrix cores 70 to 83 % busy, deeper rings changed nothing. In a loop over other weights 1119 x 19456 x 2560 takes 0.87 ms
+// (128 TFLOP/s of 157), 1119 x 2560 x 9728 0.47, 300 x 2560 x 9728 0.144; with 32x32x2 products, whose order of sums is
+// another one than the other kernel's, 0.89, 0.51 and 0.155.
 #include "common.h"
 #include "reinfer_hip.h"
 
 namespace {
 
+// ------------------------------------------------------------------------------------------------ the order of the sums
+// K is summed in up to eight blocks of at least 512 k, whose number and length follow from K alone. A block is one chain of
+// 16x16x4 products over its pieces of 16 k: the four products of a piece take k 0, 4, 8, 12, then 1, 5, 9, 13, ... The blocks'
+// sums are added in their order, then the bias. Both kernels keep this order, so a row's result does not depend on how many
+// rows stand beside it: a request's 32-bit results are the same bits alone and in any step.
+struct KBlocks {
+  int n, k;                                // how many, and k of one (a multiple of 32)
+};
+KBlocks k_blocks(int K) {
+  int n = K / 512;
+  n = n < 1 ? 1 : n > 8 ? 8 : n;
+  const int k = ((K + n - 1) / n + 31) / 32 * 32;
+  return {(K + k - 1) / k, k};
+}
+
 // ------------------------------------------------------------------------------------------------ up to 32 rows
-// Workgroups that stay: tile b, b + grid, ... of 16 features, all M rows (MT tiles of 16), WAVES waves. A wave's loads run
-// DEPTH runs of 32 U k ahead, on across the ends of tiles, and are unconditional: through a buffer descriptor a load past
-// its end returns zeros and touches no memory, so rows past N or M, pieces past K and runs past the last tile count like any
-// other load and cost nothing. A tile's runs are padded to a multiple of DEPTH, so that it ends where a round of the
+// Workgroups that stay: tile b, b + grid, ... of 16 features, all M rows (MT tiles of 16), a wave a block of K. A wave's loads
+// run DEPTH runs of 32 U k ahead, on across the ends of tiles, and are unconditional: through a buffer descriptor a load past
+// its end returns zeros and touches no memory, so rows past N or M, pieces past the block and runs past the last tile count
+// like any other load and cost nothing. A tile's runs are padded to a multiple of DEPTH, so that it ends where a round of the
 // ring does.
-template <int WAVES, int MT, int U, int DEPTH>
-__global__ void __launch_bounds__(WAVES * RA_WAVE, 4)
+template <int MT, int U, int DEPTH>
+__global__ void __launch_bounds__(8 * RA_WAVE, 4)
 gemm_f32_stream_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
-                       float* __restrict__ C, int M, int N, int K, int lda, int ldc) {
-  constexpr int SPAN = WAVES * U * 32;     // k of one run of all waves
+                       float* __restrict__ C, int M, int N, int K, int lda, int ldc, int block_k) {
+  constexpr int SPAN = U * 32;             // k of one run of a wave
   constexpr unsigned NOWHERE = 0xFFFFFFF0u;
-  __shared__ f32x4_t sums[2][WAVES][MT][RA_WAVE];        // of one tile while the next one's may already be written
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  __shared__ f32x4_t sums[2][8][MT][RA_WAVE];            // of one tile while the next one's may already be written
+  const int lane = threadIdx.x & 63, waves = blockDim.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, q = lane >> 4;
-  const int n_steps = (K + SPAN - 1) / SPAN;
+  const int k0 = wave * block_k, k1 = min(k0 + block_k, K);
+  const int n_steps = (block_k + SPAN - 1) / SPAN;       // the same for every wave: all meet at a tile's end
   const int n_steps_p = (n_steps + DEPTH - 1) / DEPTH * DEPTH;
   const int n_tiles = (N + 15) / 16;
   const int n_mine = (n_tiles - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;
@@ -54,8 +70,8 @@ gemm_f32_stream_kernel(const float* __restrict__ A, const float* __restrict__ W,
     const bool live_ = l_q < total && l_step < n_steps;                                                       \
     _Pragma("unroll") for (int u = 0; u < U; ++u)                                                             \
       _Pragma("unroll") for (int j = 0; j < 2; ++j) {                                                         \
-        const int k_ = l_step * SPAN + (wave * U + u) * 32 + j * 16 + q * 4;                                  \
-        const bool ok_ = live_ && k_ < K;            /* K is a multiple of 4 */                               \
+        const int k_ = k0 + l_step * SPAN + u * 32 + j * 16 + q * 4;                                          \
+        const bool ok_ = live_ && k_ < k1;           /* a multiple of 4 */                                    \
         const unsigned off_ = ok_ && l_n < N ? (unsigned)(((size_t)l_n * K + k_) * 4) : NOWHERE;              \
         w[d][u][j] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, off_, 0, 0));  \
         _Pragma("unroll") for (int t = 0; t < MT; ++t) {                                                      \
@@ -102,11 +118,12 @@ gemm_f32_stream_kernel(const float* __restrict__ A, const float* __restrict__ W,
       acc[t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
     }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (wave < MT) {
-      f32x4_t v = sums[buf][0][wave][lane];
+    for (int t = wave; t < MT; t += waves) {
+      f32x4_t v = sums[buf][0][t][lane];
 #pragma unroll
-      for (int x = 1; x < WAVES; ++x) v += sums[buf][x][wave][lane];
-      const int m = wave * 16 + r;
+      for (int x = 1; x < 8; ++x)
+        if (x < waves) v += sums[buf][x][t][lane];
+      const int m = t * 16 + r;
       if (m < M) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -138,9 +155,9 @@ struct F32Tile {
 // operands, rows of 8 pieces of 16 bytes, piece p of row r at place p ^ (r % 8), so that eight rows' reads of one piece fall
 // on different banks; loads that go straight to LDS write it in the order of their lanes, so it is their addresses that are
 // permuted. A tile's operands have descriptors of their own, whose ends are those of the matrices: rows past them are zeros.
-template <int BM, int BN, int STAGES>
+template <int BM, int BN, int STAGES, bool CUT>
 __global__ void __launch_bounds__(256) gemm_f32_tile_kernel(F32Tile g) {
-  constexpr int TM = BM / 64, TN = BN / 64;
+  constexpr int TM = BM / 32, TN = BN / 32;                       // 16 x 16 tiles a side of a wave's quarter
   constexpr int ROWS = BM + BN, PA = BM / 32, PB = BN / 32;       // a wave's loads a stage: 8 rows (1 KB) each
   constexpr unsigned NOWHERE = 0xFFFFFFF0u;
   __shared__ __attribute__((aligned(1024))) float lds[STAGES * ROWS * F32_BK];
@@ -186,94 +203,90 @@ __global__ void __launch_bounds__(256) gemm_f32_tile_kernel(F32Tile g) {
           w_rsrc, (__attribute__((address_space(3))) void*)(to + (BM + (wave * PB + i) * 8) * F32_BK), 16,
           (int)((w_off[i] + (unsigned)k * 4u) | past), 0, 0, 0);
   };
-  f32x16_t acc[TN][TM], sum[TN][TM];         // of the block; of the blocks before it
+  f32x4_t sum[TN][TM];                       // of the blocks before this one
 #pragma unroll
   for (int i = 0; i < TN; ++i)
 #pragma unroll
-    for (int j = 0; j < TM; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = sum[i][j][e] = 0.f;
+    for (int j = 0; j < TM; ++j) sum[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
   const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BN / 2);
-  const int row = lane & 31, half = lane >> 5;
+  const int row = lane & 15, quarter = lane >> 4;
 #pragma unroll
   for (int s = 0; s < STAGES - 1; ++s) fetch(s, s);
-  const bool cut = g.ranges > 1;
-  const int ld = cut ? g.N : g.ldc;
-  const float* b = cut ? nullptr : g.bias;
+  const int ld = CUT ? g.N : g.ldc;
+  const float* b = CUT ? nullptr : g.bias;
   const bool whole = g.N % 4 == 0 && ld % 4 == 0 && (uintptr_t)g.c % 16 == 0;
-  int buf = 0, in_block = 0;
-  for (int s = 0; s < steps; ++s) {
-    // this wave's loads of stage s are done when only those of the stages behind it are left (and, behind a block's end, its
-    // stores), its reads of the stage that is
-    // asked for next when no LDS read is left
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((PA + PB) * (STAGES - 2)) : "memory");
-    fetch(s + STAGES - 1, buf == 0 ? STAGES - 1 : buf - 1);
-    const float* as = lds + buf * ROWS * F32_BK + (wm + row) * F32_BK;
-    const float* ws = lds + buf * ROWS * F32_BK + (BM + wn + row) * F32_BK;
+  int buf = 0;
+  for (int s = 0, block = z * g.range_blocks; s < steps; ++block) {
+    f32x4_t acc[TN][TM];
 #pragma unroll
-    for (int kk = 0; kk < F32_BK / 8; ++kk) {
-      f32x4_t x[TM], y[TN];
-      const int p = ((kk * 2 + half) ^ (row & 7)) * 4;
+    for (int i = 0; i < TN; ++i)
 #pragma unroll
-      for (int j = 0; j < TM; ++j) x[j] = *(const f32x4_t*)(as + j * 32 * F32_BK + p);
+      for (int j = 0; j < TM; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    const int end = min(s + block_steps, steps);
+    for (; s < end; ++s) {
+      // this wave's loads of stage s are done when only those of the stages behind it are left (and, behind a block's end, its
+      // stores), its reads of the stage that is
+      // asked for next when no LDS read is left
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((PA + PB) * (STAGES - 2)) : "memory");
+      fetch(s + STAGES - 1, buf == 0 ? STAGES - 1 : buf - 1);
+      const float* as = lds + buf * ROWS * F32_BK + (wm + row) * F32_BK;
+      const float* ws = lds + buf * ROWS * F32_BK + (BM + wn + row) * F32_BK;
 #pragma unroll
-      for (int i = 0; i < TN; ++i) y[i] = *(const f32x4_t*)(ws + i * 32 * F32_BK + p);
+      for (int kk = 0; kk < F32_BK / 16; ++kk) {
+        f32x4_t x[TM], y[TN];
+        const int p = ((kk * 4 + quarter) ^ (row & 7)) * 4;
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
+        for (int j = 0; j < TM; ++j) x[j] = *(const f32x4_t*)(as + j * 16 * F32_BK + p);
 #pragma unroll
-        for (int i = 0; i < TN; ++i)
+        for (int i = 0; i < TN; ++i) y[i] = *(const f32x4_t*)(ws + i * 16 * F32_BK + p);
 #pragma unroll
-          for (int j = 0; j < TM; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(y[i][e], x[j][e], acc[i][j], 0, 0, 0);
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int i = 0; i < TN; ++i)
+#pragma unroll
+            for (int j = 0; j < TM; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(y[i][e], x[j][e], acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);     // one piece's operands at a time: three workgroups a CU have registers for no more
+      }
+      buf = buf + 1 == STAGES ? 0 : buf + 1;
     }
-    buf = buf + 1 == STAGES ? 0 : buf + 1;
-    if (++in_block < block_steps && s + 1 < steps) continue;
-    in_block = 0;
-    const int block = z * g.range_blocks + s / block_steps;
-    const bool first = s < block_steps, last = s + 1 == steps;
-    if (!cut) {                              // the blocks are added here, as the adding kernel does it
+    if (!CUT) {                              // the blocks are added here, as the adding kernel does it
 #pragma unroll
       for (int i = 0; i < TN; ++i)
 #pragma unroll
         for (int j = 0; j < TM; ++j)
 #pragma unroll
-          for (int e = 0; e < 16; ++e) sum[i][j][e] = first ? acc[i][j][e] : sum[i][j][e] + acc[i][j][e];
+          for (int e = 0; e < 4; ++e) sum[i][j][e] += acc[i][j][e];
     }
-    if (cut || last) {
-      // a lane holds row lane % 32 of the tile, features 8 (e / 4) + 4 (lane / 32) + e % 4
-      float* out = cut ? g.c + (size_t)block * g.M * g.N : g.c;
+    if (CUT || s == steps) {
+      // a lane holds row lane % 16 of the tile, features 4 (lane / 16) .. + 3
+      float* out = CUT ? g.c + (size_t)block * g.M * g.N : g.c;
+      int m_at = m0 + wm + row;
+      asm volatile("" : "+v"(m_at));         // addresses are worked out here and not kept in registers through the steps
 #pragma unroll
       for (int j = 0; j < TM; ++j) {
-        const int m = m0 + wm + j * 32 + row;
+        const int m = m_at + j * 16;
         if (m >= g.M) continue;
 #pragma unroll
-        for (int i = 0; i < TN; ++i)
+        for (int i = 0; i < TN; ++i) {
+          const int n = n0 + wn + i * 16 + quarter * 4;
+          if (n >= g.N) continue;
+          f32x4_t v;
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int n = n0 + wn + i * 32 + q * 8 + half * 4;
-            if (n >= g.N) continue;
-            f32x4_t v;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              v[e] = cut ? acc[i][j][q * 4 + e] : sum[i][j][q * 4 + e];
-              if (b && n + e < g.N) v[e] += b[n + e];
-            }
-            if (whole) {
-              *(f32x4_t*)(out + (size_t)m * ld + n) = v;
-            } else {
-#pragma unroll
-              for (int e = 0; e < 4; ++e)
-                if (n + e < g.N) out[(size_t)m * ld + n + e] = v[e];
-            }
+          for (int e = 0; e < 4; ++e) {
+            v[e] = CUT ? acc[i][j][e] : sum[i][j][e];
+            if (b && n + e < g.N) v[e] += b[n + e];
           }
+          if (whole) {
+            *(f32x4_t*)(out + (size_t)m * ld + n) = v;
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (n + e < g.N) out[(size_t)m * ld + n + e] = v[e];
+          }
+        }
       }
     }
-#pragma unroll
-    for (int i = 0; i < TN; ++i)
-#pragma unroll
-      for (int j = 0; j < TM; ++j)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
   }
 }
 
@@ -303,21 +316,16 @@ gemm_f32_add_kernel(const float* __restrict__ part, int ranges, const float* __r
   }
 }
 
-// The tile kernel's plan. K is summed in up to eight blocks of at least 512 k whose number follows from K alone, and their sums
-// are added in order, in the registers of one workgroup or from planes by the adding kernel: a row's result does not depend on
-// how many rows stand beside it. What depends on them is the price: tiles of 64 x 128 or 64 x 64, and how many blocks a
-// workgroup takes; a CU's share of the workgroups at the share of the matrix cores' rate that so many side by side reach
-// (measured), and the planes written and read again.
+// The tile kernel's plan: tiles of 64 x 128 or 64 x 64, and how many of K's blocks a workgroup takes (it adds them in its
+// registers; several ranges of blocks go to planes that the adding kernel adds). The price is a CU's share of the workgroups at
+// the share of the matrix cores' rate that so many side by side reach (measured), and the planes written and read again.
 struct TilePlan {
   int bn, blocks, block_k, range_blocks, ranges;
 };
 TilePlan tile_plan(int M, int N, int K) {
   const long cus = ra_cu_count();
   const double reached[2][3] = {{0.70, 0.78, 0.81}, {0.79, 0.85, 0.87}};
-  int blocks = K / 512;
-  blocks = blocks < 1 ? 1 : blocks > 8 ? 8 : blocks;
-  const int block_k = ((K + blocks - 1) / blocks + F32_BK - 1) / F32_BK * F32_BK;
-  blocks = (K + block_k - 1) / block_k;
+  const int blocks = k_blocks(K).n, block_k = k_blocks(K).k;
   TilePlan best = {};
   double best_us = 0.0;
   for (int wide = 0; wide < 2; ++wide) {
@@ -362,20 +370,20 @@ extern "C" int ra_gemm_f32(const float* A, const float* W, const float* bias, fl
   RA_CHECK(ra_gemm_f32_supports(A, W, K, lda), "gemm_f32: rows of %d (stride %d) are not 16-byte pieces", K, lda);
   if (M <= F32_STREAM_ROWS) {
     // a descriptor covers less than 4 GiB of weights: a larger matrix goes in runs of features
+    const KBlocks kb = k_blocks(K);
     const long most = 0xFFFFFF00L / ((long)K * 4) / 16 * 16;
     RA_CHECK(most > 0 && ((long)(M - 1) * lda + K) * 4 < 0xFFFFFF00L, "gemm_f32: rows of %d (stride %d) are too long", K, lda);
     for (long n0 = 0; n0 < N; n0 += most) {
       const int n = (int)(N - n0 < most ? N - n0 : most);
       const int tiles = (n + 15) / 16, cus = ra_cu_count();
       const float *w = W + (size_t)n0 * K, *b = bias ? bias + n0 : nullptr;
-#define RA_GO(WAVES, MT, U, DEPTH, GRID) \
-  gemm_f32_stream_kernel<WAVES, MT, U, DEPTH><<<(GRID) < tiles ? (GRID) : tiles, WAVES * RA_WAVE, 0, stream>>>( \
-      A, w, b, C + n0, M, n, K, lda, ldc)
-      // four waves and four workgroups a CU share many tiles out most evenly (6144 x 2560 at 4 rows: 19.0 us against 21.1
-      // with eight waves and two), eight waves keep more in flight where a CU has one tile (2560 x 9728: 30.5 against 32.9)
-      if (M > 16) RA_GO(8, 2, 1, 3, 2 * cus);
-      else if (tiles <= cus) RA_GO(8, 1, 2, 2, cus);
-      else RA_GO(4, 1, 2, 2, 4 * cus);
+#define RA_GO(MT, U, DEPTH, GRID) \
+  gemm_f32_stream_kernel<MT, U, DEPTH><<<(GRID) < tiles ? (GRID) : tiles, kb.n * RA_WAVE, 0, stream>>>( \
+      A, w, b, C + n0, M, n, K, lda, ldc, kb.k)
+      // as many workgroups as the registers hold, 16 waves a CU
+      const int grid = 16 / kb.n * cus;
+      if (M > 16) RA_GO(2, 1, 3, grid);
+      else RA_GO(1, 2, 2, grid);
 #undef RA_GO
       RA_LAUNCH_CHECK("gemm_f32");
     }
@@ -389,8 +397,10 @@ extern "C" int ra_gemm_f32(const float* A, const float* W, const float* bias, fl
                p.block_k, p.range_blocks};
   const long total = (long)g.m_tiles * g.n_tiles * g.ranges, blocks = (total + RA_XCDS - 1) / RA_XCDS * RA_XCDS;
   RA_CHECK(blocks <= 0x7FFFFFFFL, "gemm_f32: [%d, %d] in one launch", M, N);
-  if (p.bn == 128) gemm_f32_tile_kernel<64, 128, 2><<<(unsigned)blocks, 256, 0, stream>>>(g);
-  else gemm_f32_tile_kernel<64, 64, 2><<<(unsigned)blocks, 256, 0, stream>>>(g);
+  if (p.bn == 128 && cut) gemm_f32_tile_kernel<64, 128, 2, true><<<(unsigned)blocks, 256, 0, stream>>>(g);
+  else if (p.bn == 128) gemm_f32_tile_kernel<64, 128, 2, false><<<(unsigned)blocks, 256, 0, stream>>>(g);
+  else if (cut) gemm_f32_tile_kernel<64, 64, 2, true><<<(unsigned)blocks, 256, 0, stream>>>(g);
+  else gemm_f32_tile_kernel<64, 64, 2, false><<<(unsigned)blocks, 256, 0, stream>>>(g);
   RA_LAUNCH_CHECK("gemm_f32");
   if (cut) {
     const bool whole = N % 4 == 0 && ldc % 4 == 0 && (uintptr_t)C % 16 == 0 && (uintptr_t)scratch % 16 == 0;
