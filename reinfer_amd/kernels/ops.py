@@ -709,6 +709,8 @@ class HipKernels:
         float32 whose rows are whole 16-byte pieces: this library's product on the
         float matrix cores. Everything else: the plain FMA kernel.
         """
+        if bias is not None:
+            bias = bias.contiguous()         # the kernels here read it as it lies
         if x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16:
             M, K = x.shape
             if M <= 64 and K % 8 == 0 and x.stride(0) % 8 == 0 and x.stride(1) == 1:

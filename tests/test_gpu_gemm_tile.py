@@ -92,3 +92,15 @@ def test_tiled_product_takes_only_what_it_can_read():
         ops().linear(a, w, out)
         want = a.double() @ w.double().T
         assert ((out.double() - want).abs() <= bound(a, w, K) + want.abs() * 2 ** -8).all()
+
+
+@pytest.mark.parametrize("dtype,M,K", [(torch.bfloat16, M, 4096) for M in (8, 97, 200, 600)] + [(torch.float32, M, 512) for M in (8, 97)])
+def test_a_bias_that_is_a_column_of_a_matrix(dtype, M, K):
+    N = 4096
+    x, w, g = operands(M, N, K, M)
+    x, w = x.to(dtype), w.to(dtype)
+    biases = torch.randn(N, 3, device=DEV, generator=g).to(dtype)
+    out, want = torch.empty(M, N, device=DEV, dtype=dtype), torch.empty(M, N, device=DEV, dtype=dtype)
+    ops().linear(x, w, out, biases[:, 1])
+    ops().linear(x, w, want, biases[:, 1].clone())
+    assert torch.equal(out, want)
