@@ -1874,10 +1874,14 @@ class HipKernels:
                 pairs[:, 1] = np.asarray([float(b) for _, b in bias], dtype=np.float32).view(np.int32)
                 window += pairs.reshape(-1).tolist()
             ints.append((int(p.top_k or 0), at, end - at, end if bias else 0, len(bias), 0))
-        rec = np.empty((n, 12), dtype=np.float32)
-        rec[:, :6], rec.view(np.int32)[:, 6:] = floats, ints
+        rec = np.zeros((n, 12), dtype=np.float32)      # rows without options stay as they are
+        if floats:
+            rec[:len(floats), :6], rec.view(np.int32)[:len(floats), 6:] = floats, ints
         window.append(0)                     # never empty
-        packed = np.frombuffer(struct.pack(f"{len(window)}i", *window), dtype=np.int32)     # half the time of an array of the list
+        try:
+            packed = np.frombuffer(struct.pack(f"{len(window)}i", *window), dtype=np.int32)     # half the time of an array of the list
+        except struct.error:                 # numbers of another kind among the tokens
+            packed = torch.tensor(window, dtype=torch.int32).numpy()
         both = to_device(np.concatenate([rec.view(np.int32).reshape(-1), packed]), logits.device)
         rows_t, win_t = both[:12 * n], both[12 * n:]
         need = int(library.load().ra_filter_scratch(n, V))

@@ -57,3 +57,31 @@ def test_filters_over_equal_logits_and_rows_with_few_finite_ones():
     assert torch.isfinite(got[2]).nonzero()[:, 0].tolist() == [4096, 9999]
     assert torch.isfinite(got[3]).nonzero()[:, 0].tolist() == [4096]                 # 0.67 of the mass
     assert not torch.isfinite(got[4]).any()
+
+
+@pytest.mark.parametrize("given", [0, 1, 2])
+def test_rows_without_options_or_tokens_stay_as_they_are(given):
+    """Fewer options, or fewer token lists, than rows: the rows behind them keep their logits."""
+    from reinfer_amd import kernels
+    from reinfer_amd.sampling import SamplingParams
+    row = torch.linspace(-3.0, 3.0, 500)
+    p = SamplingParams(temperature=1.0, top_k=7)
+    for params, histories in (([p] * given, [[1, 2]] * 3), ([p] * 3, [[1, 2]] * given)):
+        logits = torch.stack([row] * 3).to(DEV)
+        kernels.current().filter_logits(logits, params, histories)
+        kept = torch.isfinite(logits).sum(-1).tolist()
+        assert kept == [7] * given + [500] * (3 - given)
+
+
+def test_tokens_of_other_number_kinds():
+    """Histories that hold numpy numbers, floats among them, count as the whole numbers that they are."""
+    import numpy as np
+    from reinfer_amd import kernels
+    from reinfer_amd.sampling import SamplingParams
+    p = [SamplingParams(temperature=1.0, presence_penalty=2.0)]
+    want = None
+    for history in ([3, 5], np.array([3, 5]), np.array([3.0, 5.0]), torch.tensor([3, 5]), (3, 5)):
+        logits = torch.zeros(1, 16, device=DEV)
+        kernels.current().filter_logits(logits, p, [history])
+        want = logits.clone() if want is None else want
+        assert torch.equal(logits, want) and logits[0, 3] == -2.0 and logits[0, 4] == 0.0
