@@ -5,7 +5,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
-#define RA_ABI_VERSION 27
+#define RA_ABI_VERSION 28
 
 #ifdef __cplusplus
 extern "C" {
@@ -77,12 +77,13 @@ int ra_gemm_plain(const void* A, const void* W, const void* bias, void* C, int i
 
 // Experts over tokens sorted by expert (bfloat16; moe_grouped.hip): w_up [experts ff, width], with a gate [2 experts ff,
 // width] an expert's gate rows before its up rows, w_down [width, ld_down] an expert's ff columns side by side, ids and
-// weights [n_tokens, top] (an id of `experts` or more: its weight times the token's row). more (float [n_tokens, width], or
+// weights [n_tokens, top] (an id of `experts` or more: its weight times the token's row; of an expert's mentions by one token the
+// last one counts; distinct: there are no two). more (float [n_tokens, width], or
 // null) is added, times sigmoid(more_logit[t * ld_logit]) where that is given. Exactly one of resid (float, += alpha times
 // the sum) and out (bfloat16). scratch: ra_moe_grouped_scratch bytes on a 256-byte boundary.
 long ra_moe_grouped_scratch(int n_tokens, int top, int experts, int ff, int width);
 int ra_moe_grouped(const void* x, int ldx, const void* w_up, const void* w_down, int ld_down, const int* ids,
-                   const float* weights, int top, int experts, int ff, int gated, int n_tokens, int width,
+                   const float* weights, int top, int distinct, int experts, int ff, int gated, int n_tokens, int width,
                    const float* more, const float* more_logit, int ld_logit, float* resid, void* out, float alpha,
                    void* scratch, long scratch_bytes, hipStream_t stream);
 

@@ -15,7 +15,7 @@ import torch  # noqa: F401  (loads the HIP runtime the library links against)
 
 from ..csrc import build as _build
 
-ABI_VERSION = 27
+ABI_VERSION = 28
 
 
 class KernelLibraryError(RuntimeError):
@@ -46,7 +46,7 @@ _SIGNATURES = {
     "ra_gemm_skinny_scaled": [P, P, P, I, I, I, I, I, F, P],
     "ra_gemm_wide_scaled": [P, P, P, I, I, I, I, I, P, c_long, F, P],
     "ra_gemm_plain": [P, P, P, P, I, I, I, I, I, I, I, P],
-    "ra_moe_grouped": [P, I, P, P, I, P, P, I, I, I, I, I, I, P, P, I, P, P, F, P, c_long, P],
+    "ra_moe_grouped": [P, I, P, P, I, P, P, I, I, I, I, I, I, I, P, P, I, P, P, F, P, c_long, P],
     "ra_gemm_f32": [P, P, P, P, I, I, I, I, I, P, c_long, P],
     "ra_sample": [P, I, I, I, P, P, P, P, P, P, P],
     "ra_sample_static": [P, I, I, I, P, P, P, P, P],

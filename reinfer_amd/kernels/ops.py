@@ -1705,8 +1705,9 @@ class HipKernels:
     def moe_grouped(self, x: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor, ids: torch.Tensor,
                     weights: torch.Tensor, experts: int, ff: int, gated: bool, more: Optional[torch.Tensor] = None,
                     more_logit: Optional[torch.Tensor] = None, resid: Optional[torch.Tensor] = None, alpha: float = 1.0,
-                    out: Optional[torch.Tensor] = None) -> None:
-        """y[t] = sum_j weights[t, j] * (expert ids[t, j] of x[t]) (an id of ``experts`` or more stands for x[t] itself)
+                    out: Optional[torch.Tensor] = None, distinct: bool = False) -> None:
+        """y[t] = sum_j weights[t, j] * (expert ids[t, j] of x[t]) (an id of ``experts`` or more stands for x[t] itself; of an
+        expert that a token names twice the last weight counts, as in ``moe_silu_gate_scale``; ``distinct``: none is)
         + ``more``[t] (float32, times sigmoid(more_logit[t]) where that is given); resid += alpha * y, or out = y in
         bfloat16. An expert is W_down relu(W_up x)^2, or ``gated`` W_down (silu(W_gate x) * (W_up x)). ``w_up`` holds
         [experts * ff] rows, gated [gate; up] an expert, ``w_down`` [width, at least experts * ff] an expert's columns side
@@ -1734,7 +1735,8 @@ class HipKernels:
         need = int(library.load().ra_moe_grouped_scratch(T, top, int(experts), int(ff), width))
         scratch = torch.empty(need, dtype=torch.uint8, device=x.device)
         library.call("ra_moe_grouped", x.data_ptr(), x.stride(0), w_up.data_ptr(), w_down.data_ptr(), w_down.stride(0),
-                     ids.data_ptr(), weights.data_ptr(), top, int(experts), int(ff), 1 if gated else 0, T, width, _ptr(more),
+                     ids.data_ptr(), weights.data_ptr(), top, 1 if distinct else 0, int(experts), int(ff), 1 if gated else 0,
+                     T, width, _ptr(more),
                      _ptr(more_logit), more_logit.stride(0) if more_logit is not None else 0, _ptr(resid), _ptr(out),
                      float(alpha), scratch.data_ptr(), need, _stream())
 

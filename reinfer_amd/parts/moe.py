@@ -206,7 +206,8 @@ class MixtureOfExperts:
             ops.linear(act, self.w_shared_down, more)
         out = None if resid is not None else torch.empty((T, width), dtype=self.dtype, device=x.device)
         ops.moe_grouped(x, w_up, self.w_down, ids, weights, self.experts, self.ff, self.gated, more=more,
-                        more_logit=shared_logit if more is not None else None, resid=resid, alpha=resid_scale, out=out)
+                        more_logit=shared_logit if more is not None else None, resid=resid, alpha=resid_scale, out=out,
+                        distinct=self.table is None)       # a router chooses an expert once
         return out
 
     def forward(self, x, batch, resid: Optional[torch.Tensor] = None, resid_scale: float = 1.0):

@@ -66,3 +66,43 @@ def test_experts_over_sorted_tokens(T, E, top, ff, width, gated, kind):
     base = resid.double()
     ops().moe_grouped(x, w_up, w_down, ids, wts, E, ff, gated, more=more, more_logit=logit, resid=resid, alpha=0.5)
     assert ((resid.double() - (base + 0.5 * want)).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("T,E,top,ff,width", [(65, 8, 3, 40, 72), (300, 16, 4, 64, 128)])
+def test_an_expert_that_a_token_names_twice(T, E, top, ff, width):
+    """Its last weight counts, as in the products over all experts side by side."""
+    g, G = torch.Generator().manual_seed(T), torch.Generator(device=DEV).manual_seed(T)
+    x = torch.randn(T, width, generator=G, device=DEV).bfloat16()
+    w_up = (torch.randn(2 * E * ff, width, generator=G, device=DEV) / width ** 0.5).bfloat16()
+    w_down = (torch.randn(width, E * ff, generator=G, device=DEV) / ff ** 0.5).bfloat16()
+    ids = choices("spread", T, E, top, g)
+    ids[::3, 0] = ids[::3, top - 1]
+    ids[1::3, 1] = ids[1::3, 0]
+    ids[5] = ids[5, 0]
+    ids = ids.to(torch.int32).to(DEV)
+    wts = torch.rand(T, top, generator=G, device=DEV)
+    gu, act = torch.empty(T, 2 * E * ff, device=DEV).bfloat16(), torch.empty(T, E * ff, device=DEV).bfloat16()
+    ops().linear(x, w_up, gu)
+    ops().moe_silu_gate_scale(gu, act, ids, wts, E, ff)
+    want = act.double() @ w_down.double().t()
+    size = act.double().abs() @ w_down.double().abs().t()
+    out = torch.empty(T, width, dtype=torch.bfloat16, device=DEV)
+    ops().moe_grouped(x, w_up, w_down, ids, wts, E, ff, True, out=out)
+    # the products before the activation are rounded to bfloat16 on one side alone, the activations on both
+    assert ((out.double() - want).abs() <= 2.0 ** -6 * size + 2.0 ** -8 * want.abs() + 1e-4).all()
+
+
+def test_an_id_below_zero_names_nothing():
+    T, E, top, ff, width = 70, 8, 3, 40, 72
+    G = torch.Generator(device=DEV).manual_seed(T)
+    x = torch.randn(T, width, generator=G, device=DEV).bfloat16()
+    w_up = (torch.randn(E * ff, width, generator=G, device=DEV) / width ** 0.5).bfloat16()
+    w_down = (torch.randn(width, E * ff, generator=G, device=DEV) / ff ** 0.5).bfloat16()
+    ids = torch.arange(top, device=DEV, dtype=torch.int32).repeat(T, 1)
+    wts = torch.rand(T, top, generator=G, device=DEV)
+    wts[7, 0] = 0.0
+    out, want = (torch.empty(T, width, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    ops().moe_grouped(x, w_up, w_down, ids, wts, E, ff, False, out=want)
+    ids[7, 0] = -5
+    ops().moe_grouped(x, w_up, w_down, ids, wts, E, ff, False, out=out)
+    assert torch.equal(out, want)
