@@ -1688,16 +1688,27 @@ class HipKernels:
         return n_tokens <= self.MOE_CHOSEN_TOKENS and n_tokens * top <= self.MOE_CHOSEN_SHARE * experts
 
     # Rows from which a token's rows meet its chosen experts alone, its pairs sorted by expert, and the share of the
-    # experts that a token may choose at most for that. Up to 64 rows the products that read every expert once are bound by
-    # those reads in either form; with half of the experts chosen the products over all of them, at twice the rate, cost
-    # the same.
-    MOE_GROUPED_FROM = 65
+    # experts that a token may choose at most for that (with half of them chosen the products over all of them, at twice the
+    # rate, cost the same). Up to some 256 rows the products over all experts are bound by reading every matrix once, which
+    # the sorted form does too, with its sorting, part-filled tiles and last sum on top; beyond, the library's products double
+    # their time. Experts x chosen x ff x width, all / sorted, at 65, 128, 256, 320 and 1024 rows: 16 x 4 x 1024 x 4096 and a
+    # shared one 125 / 154, 139 / 162, 160 / 176, 257 / 183, 477 / 311 us; 16 x 4 x 1536 x 4096 without gate 108 / 130,
+    # 118 / 133, 153 / 137, 239 / 143, 451 / 214; 8 x 2 x 2048 x 4096 115 / 137, 120 / 141, 150 / 146, 184 / 142, 355 / 226.
+    # Where few are chosen, what lies between the products is large for nothing as well: 64 x 6 x 512 x 2048 138 / 135,
+    # 142 / 136, 169 / 141; 128 x 8 x 768 x 2048 323 / 274, 346 / 271, 408 / 275.
+    MOE_GROUPED_FROM = 257
     MOE_GROUPED_SHARE = 0.4
+    MOE_GROUPED_FEW = 0.1            # of the experts chosen: sorted from MOE_GROUPED_LEAST rows on
+    MOE_GROUPED_LEAST = 65
+
+    def moe_groups_pay(self, n_tokens: int, top: int, experts: int) -> bool:
+        """Whether a step that :meth:`moe_grouped` can take is faster there than in products over all experts."""
+        return n_tokens >= (self.MOE_GROUPED_LEAST if top <= self.MOE_GROUPED_FEW * experts else self.MOE_GROUPED_FROM)
 
     def moe_groups(self, x: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor, top: int, experts: int, ff: int) -> bool:
-        """Whether a step over the rows ``x`` should go through :meth:`moe_grouped`."""
+        """Whether :meth:`moe_grouped` can take a step over the rows ``x`` (see :meth:`moe_groups_pay`)."""
         T, width = x.shape
-        return self.MOE_GROUPED_FROM <= T <= 65535 and top <= self.MOE_GROUPED_SHARE * experts and experts <= 4096 \
+        return self.MOE_GROUPED_LEAST <= T <= 65535 and top <= self.MOE_GROUPED_SHARE * experts and experts <= 4096 \
             and T * top <= 1 << 24 and x.is_cuda and x.dtype == w_up.dtype == w_down.dtype == torch.bfloat16 \
             and width % 8 == 0 and ff % 8 == 0 and w_down.stride(0) % 8 == 0 and x.stride(0) % 8 == 0 and x.stride(1) == 1 \
             and all(t.data_ptr() % 16 == 0 for t in (x, w_up, w_down))

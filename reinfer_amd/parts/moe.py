@@ -10,8 +10,8 @@ applies the activation and the routing weight in one kernel (0 for experts a tok
 product with the down matrix is then the weighted sum: with few experts of which a good share is chosen, two
 dense products at the matrix cores' rate cost less than gathering tokens by expert would. A step of so few
 tokens that most experts are not asked for at all (one or two requests decoding) reads only the chosen experts'
-rows instead, a wave a row; a step of more than 64 tokens sorts its token-expert pairs by expert on the device and
-runs each expert over its own.
+rows instead, a wave a row; a step of many tokens (``moe_groups_pay``) sorts its token-expert pairs by expert on the
+device and runs each expert over its own.
 
 A second form of the same part (``activation`` "silu_gated", ``weights`` "sigmoid"): an expert is
 W_down (silu(W_gate h) * (W_up h)); a token's score for expert e is sigmoid(z_e); where the experts form
@@ -165,8 +165,7 @@ class MixtureOfExperts:
             out = torch.empty((T, self.spec.hidden), dtype=self.dtype, device=x.device)
             ops.moe_down_gated_chosen(act, self.w_down, ids, weights, x, out, self.experts, self.ff, self.shared)
             return out
-        groups = getattr(ops, "moe_groups", None)
-        if groups is not None and groups(x, self.w_gate_up, self.w_down, self.top, self.experts, self.ff):
+        if self._grouped(ops, x, self.w_gate_up, routed):
             return self._forward_grouped(ops, x, self.w_gate_up, ids, weights, shared_logit, resid, resid_scale)
         gu = torch.empty((T, 2 * n), dtype=self.dtype, device=x.device)
         ops.linear(x, self.w_gate_up, gu)
@@ -191,6 +190,11 @@ class MixtureOfExperts:
         out = torch.empty((T, self.spec.hidden), dtype=self.dtype, device=x.device)
         ops.linear(act, self.w_down, out)
         return out
+
+    def _grouped(self, ops, x, w_up, routed: int) -> bool:
+        groups = getattr(ops, "moe_groups", None)
+        return groups is not None and ops.moe_groups_pay(x.shape[0], self.top, routed) \
+            and groups(x, w_up, self.w_down, self.top, self.experts, self.ff)
 
     def _forward_grouped(self, ops, x, w_up, ids, weights, shared_logit, resid, resid_scale):
         """Many tokens: each through its chosen experts alone. The shared expert runs over all of them beside, its result
@@ -232,8 +236,7 @@ class MixtureOfExperts:
             out = torch.empty((T, self.spec.hidden), dtype=self.dtype, device=x.device)
             ops.moe_down_chosen(act, self.w_down, ids, self.ff, out=out)
             return out
-        groups = getattr(ops, "moe_groups", None)
-        if groups is not None and groups(x, self.w_up, self.w_down, self.top, self.experts, self.ff):
+        if self._grouped(ops, x, self.w_up, self.experts):
             return self._forward_grouped(ops, x, self.w_up, ids, weights, None, resid, 1.0)
         up = torch.empty((T, n), dtype=self.dtype, device=x.device)
         ops.linear(x, self.w_up, up)

@@ -106,3 +106,46 @@ def test_an_id_below_zero_names_nothing():
     ids[7, 0] = -5
     ops().moe_grouped(x, w_up, w_down, ids, wts, E, ff, False, out=out)
     assert torch.equal(out, want)
+
+
+def test_where_sorting_pays():
+    """Decode steps of up to 128 requests and short mixed steps stay with the products over all experts unless few are chosen."""
+    pay = ops().moe_groups_pay
+    assert not any(pay(T, 4, 16) or pay(T, 2, 8) for T in (65, 128, 256)) and pay(257, 4, 16) and pay(1900, 4, 16)
+    assert not pay(64, 6, 64) and pay(65, 6, 64) and pay(65, 8, 128)
+
+
+def test_captured_steps_over_sorted_tokens(tmp_path):
+    """A decode step of 70 requests whose tokens choose 2 of 32 experts: replays between other work against eager steps."""
+    import json
+    import os
+    from helpers import random_tokens
+    from kobolix_helpers import _dense, _memory, _moe, draw_weights
+    from reinfer_amd.engine import ModelRunner, StepEntry
+    from reinfer_amd.weights.safetensors_io import write_safetensors
+    raw = {"architecture": "Kobolix", "vocab": 90, "width": 64, "norm": {"eps": 1e-5},
+           "layers": [{"type": "mlstm", "mixer": _memory(2, 16, 24, 12.0), "mlp": _moe(32, 2, 24, shared=16)},
+                      {"type": "mlstm", "mixer": _memory(1, 32, 16, 12.0), "mlp": _dense(40)}]}
+    with open(os.path.join(str(tmp_path), "config.json"), "w") as f:
+        json.dump(raw, f)
+    write_safetensors(os.path.join(str(tmp_path), "model.safetensors"), draw_weights(raw, 5, torch.bfloat16), metadata={"format": "pt"})
+    n, tokens = 70, random_tokens(70 * 8, 90, 3)
+    found, calls = [], []
+    kind = type(ops())
+    real = kind.moe_grouped
+    kind.moe_grouped = lambda *a, **k: (calls.append(1), real(*a, **k))[1]
+    try:
+        for graphs in (True, False):
+            runner = ModelRunner.from_folder(str(tmp_path), dtype="bfloat16", device=DEV, max_seqs=n, max_model_len=64, use_graphs=graphs)
+            out, seen = [], len(calls)
+            for r in range(n):
+                runner.add_request(r)
+            for s in range(7):
+                out.append(runner.step([StepEntry(r, [tokens[s * n + r]], [0]) for r in range(n)]).clone())
+                torch.randn(500, 500, device=DEV).sum().item()
+            assert len(calls) > seen
+            found.append(out)
+    finally:
+        kind.moe_grouped = real
+    for s, (a, b) in enumerate(zip(*found)):
+        assert torch.isfinite(a).all() and torch.equal(a, b), s
