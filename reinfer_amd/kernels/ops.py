@@ -1406,6 +1406,11 @@ class HipKernels:
     # token; either form goes on from the state that the other left.
     CHUNK_FROM = 17
     CHUNK_KEYS = 256
+    # The same for the matrix memory and the delta rule, whose chunks take a preparation and, beside shorter portions, a scan
+    # of their own: a portion alone, in chunks / token by token, at 17, 32, 64 and 128 tokens 22 / 16, 22 / 21, 22 / 33 and
+    # 26 / 56 us (16 heads of 128 x 256) and 18 / 13, 18 / 18, 18 / 28 and 23 / 50 (32 of 128 x 128); beside 32 single tokens
+    # 75 / 53, 74 / 59, 74 / 75 and 76 / 106 and 59 / 45, 58 / 51, 59 / 66 and 62 / 94.
+    MEMORY_CHUNK_FROM = 64
 
     @staticmethod
     def _check_linear_scan(what: str, proj, q_off, k_off, v_off, heads, key_dim, value_dim, out) -> None:
@@ -1421,9 +1426,9 @@ class HipKernels:
         by token. A request's form follows from its own portion: its result does not depend on the requests beside it."""
         least = 1
         if chunks is None:
-            chunks = int(getattr(batch, "max_q_len", 0) or 0) >= self.CHUNK_FROM and key_dim <= self.CHUNK_KEYS
-            if min(batch.q_lens, default=0) < self.CHUNK_FROM:
-                least = self.CHUNK_FROM
+            chunks = int(getattr(batch, "max_q_len", 0) or 0) >= self.MEMORY_CHUNK_FROM and key_dim <= self.CHUNK_KEYS
+            if min(batch.q_lens, default=0) < self.MEMORY_CHUNK_FROM:
+                least = self.MEMORY_CHUNK_FROM
         return (self._chunk_scratch(T, batch.num_seqs, heads, key_dim, value_dim, device, kind) if chunks else None), least
 
     @classmethod

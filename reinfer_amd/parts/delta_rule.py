@@ -90,7 +90,7 @@ class GatedDeltaRule:
                                self.unit_eps, dk ** -0.5, qkv)
         read = torch.empty((T, H * dv), dtype=torch.float32, device=x.device)
         # the 32-bit path goes token by token: one order of sums, which does not depend on the requests beside
-        form = {"chunks": False} if self.dtype == torch.float32 and hasattr(ops, "CHUNK_FROM") else {}
+        form = {"chunks": False} if self.dtype == torch.float32 and hasattr(ops, "MEMORY_CHUNK_FROM") else {}
         ops.delta_rule_scan(qkv, ba, self.a_log, self.dt_bias, cache.state, batch, H, G, dk, dv, read, **form)
         act = torch.empty((T, H * dv), dtype=self.dtype, device=x.device)
         ops.head_norm_gate(read, self.norm_weight, False, proj[:, self.channels:], "silu", self.norm_eps, H, dv, act)

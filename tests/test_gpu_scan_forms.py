@@ -40,7 +40,7 @@ def test_32_bit_results_do_not_depend_on_the_requests_beside(tmp_path):
 
 
 @pytest.mark.parametrize("kind", ["memory", "delta"])
-@pytest.mark.parametrize("mine,others", [(1, [64]), (16, [17]), (17, [1, 1]), (40, [3, 200])])
+@pytest.mark.parametrize("mine,others", [(1, [64]), (16, [17]), (17, [1, 1]), (40, [3, 200]), (63, [64]), (64, [63, 1]), (100, [1, 65])])
 def test_a_scan_does_not_depend_on_the_requests_beside(kind, mine, others):
     """bfloat16 rows, the form left to the call: a request's read-out and state alone and in the middle of a step."""
     ops = kernels.current()
@@ -67,3 +67,25 @@ def test_a_scan_does_not_depend_on_the_requests_beside(kind, mine, others):
         assert torch.isfinite(out).all()
         found.append((out[at:at + mine] if n == T else out, st[2]))
     assert torch.equal(found[0][0], found[1][0]) and torch.equal(found[0][1], found[1][1])
+
+
+@pytest.mark.parametrize("kind", ["memory", "delta"])
+@pytest.mark.parametrize("mine,least", [(63, 64), (64, 64), (17, 64)])
+def test_where_chunks_begin(kind, mine, least):
+    """bfloat16 portions below the edge are walked token by token, from it on in chunks: the forced forms' bits."""
+    ops = kernels.current()
+    H, dk, dv = 2, 64, 24
+    g = torch.Generator().manual_seed(mine)
+    rows, z = (torch.randn(mine, 2 * H * dk + H * dv, generator=g) * 0.3).to(torch.bfloat16).to(DEV), torch.randn(mine, 2 * H, generator=g).to(DEV)
+    bias, found = torch.randn(2 * H, generator=g).to(DEV), []
+    for form in (None, mine >= least):
+        batch = make_batch([mine], [0], [1], DEV)
+        batch.max_q_len = mine
+        out, st = torch.empty(mine, H * dv, device=DEV), torch.zeros(1, ops.scan_state_floats("matrix_memory", H, dk, dv), device=DEV)
+        if kind == "memory":
+            ops.matrix_memory_scan(rows, 0, H * dk, 2 * H * dk, z, bias, st, batch, H, dk, dv, 15.0, dk ** -0.5, 1e-6, out, chunks=form)
+        else:
+            ops.delta_rule_scan(rows.float(), z.clone(), bias[:H].contiguous(), bias[H:].contiguous(), st, batch, H, H, dk, dv, out,
+                                chunks=form)
+        found.append(out)
+    assert torch.equal(found[0], found[1])
