@@ -737,15 +737,26 @@ class HipKernels:
             return self.linear_f32(x, weight, out, bias)
         self.linear_plain(x, weight, out, bias)
 
-    @staticmethod
-    def _tile_takes(epilogue: int, x, weight, out) -> bool:
+    # Weights (elements) from which a product that is cut, and then added up by a kernel of its own, is worth that: at 65 to 256
+    # rows, tiled / library, 8192 x 2048 14 to 22 / 11 to 20 us, 6144 x 2560 14 to 23 / 13 to 25, 2560 x 4096 14 to 20 / 10 to 18,
+    # 4096 x 4096 14 to 22 / 14 to 26 in no order, but 4096 x 6144 17 to 28 / 19 to 43, 2560 x 9728 18 to 29 / 22 to 36. Above 256
+    # rows 5120 x 8192 50 / 44, 4096 x 11008 and 12288 67 to 76 / 76 to 79. A gated product is not cut, and what adds into the
+    # stream with up to 128 rows saves the norm behind it its add.
+    TILE_ADDED_WEIGHTS = 20 << 20
+    TILE_LONG_K = 8192
+
+    @classmethod
+    def _tile_takes(cls, epilogue: int, x, weight, out) -> bool:
         """Whether the tiled product of 65 to 512 rows takes this one (epilogues as ``ra_gemm_wide``): where it is ahead of
         the library's, for rows that are whole 16-byte pieces."""
         M, K = x.shape
+        N = weight.shape[0]
+        added = epilogue == 0 or (epilogue == 2 and M > 128)
         return 64 < M <= 512 and x.is_cuda and K % 8 == 0 and x.stride(0) % 8 == 0 and K <= x.stride(0) < 2 ** 21 \
+            and not (added and (N * K < cls.TILE_ADDED_WEIGHTS or (M > 256 and K <= cls.TILE_LONG_K))) \
             and x.stride(1) == 1 and out.stride(0) >= out.shape[1] and weight.is_contiguous() and out.stride(1) == 1 \
             and all(t.data_ptr() % 16 == 0 for t in (x, weight, out)) \
-            and bool(library.load().ra_gemm_tile_takes(epilogue, M, weight.shape[0], K))
+            and bool(library.load().ra_gemm_tile_takes(epilogue, M, N, K))
 
     @staticmethod
     def _check_linear(x, weight, out, bias):

@@ -104,3 +104,32 @@ def test_a_bias_that_is_a_column_of_a_matrix(dtype, M, K):
     ops().linear(x, w, out, biases[:, 1])
     ops().linear(x, w, want, biases[:, 1].clone())
     assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("M,N,K", SIZES)
+def test_tiled_product_where_the_library_is_asked_first(M, N, K):
+    """The kernel itself at every size it takes, also where ``linear`` prefers the library's product."""
+    x, w, g = operands(M, N, K, M * 3 + N)
+    ref, err = x.double() @ w.double().T, bound(x, w, K)
+    bias = torch.randn(N, device=DEV, generator=g).to(torch.bfloat16)
+    biased = ref + bias.double()
+    for kind, ulp in ((torch.float32, 2.0 ** -23), (torch.bfloat16, 2.0 ** -8)):
+        buf = torch.full((M, N + 8), float("nan"), device=DEV, dtype=kind)
+        ops()._few_rows("linear output", x, w, bias, buf[:, :N], 0, M, N, K, True)
+        assert ((buf[:, :N].double() - biased).abs() <= err + biased.abs() * ulp).all()
+        assert torch.isnan(buf[:, N:]).all()
+    stream = torch.randn(M, N, device=DEV, generator=g) * 8
+    want = stream.double() + ref
+    ops()._few_rows("linear output", x, w, None, stream, 2, M, N, K, True)
+    assert ((stream.double() - want).abs() <= err + want.abs() * 2 ** -23).all()
+
+
+def test_small_cut_products_stay_with_the_library():
+    def takes(epilogue, M, N, K):
+        x, w = torch.empty(M, K, device=DEV, dtype=torch.bfloat16), torch.empty(N, K, device=DEV, dtype=torch.bfloat16)
+        return ops()._tile_takes(epilogue, x, w, torch.empty(M, N, device=DEV, dtype=torch.float32 if epilogue == 2 else torch.bfloat16))
+    for M in (65, 128, 256):
+        assert not any(takes(0, M, N, K) for N, K in ((8192, 2048), (6144, 2560), (4096, 4096)))
+        assert takes(0, M, 6144, 4096) and takes(0, M, 4096, 6144)
+    assert takes(2, 97, 2560, 4096) and not takes(2, 160, 2560, 4096) and takes(2, 160, 2560, 9728)
+    assert not takes(2, 320, 5120, 8192) and takes(2, 320, 5120, 25600) and takes(1, 97, 24576, 4096)
