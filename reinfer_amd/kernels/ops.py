@@ -738,12 +738,11 @@ class HipKernels:
         self.linear_plain(x, weight, out, bias)
 
     # Weights (elements) from which a product that is cut, and then added up by a kernel of its own, is worth that: at 65 to 256
-    # rows, tiled / library, 8192 x 2048 14 to 22 / 11 to 20 us, 6144 x 2560 14 to 23 / 13 to 25, 2560 x 4096 14 to 20 / 10 to 18,
-    # 4096 x 4096 14 to 22 / 14 to 26 in no order, but 4096 x 6144 17 to 28 / 19 to 43, 2560 x 9728 18 to 29 / 22 to 36. Above 256
-    # rows 5120 x 8192 50 / 44, 4096 x 11008 and 12288 67 to 76 / 76 to 79. A gated product is not cut, and what adds into the
-    # stream with up to 128 rows saves the norm behind it its add.
+    # rows, tiled / library, 8192 x 2048 14 to 22 / 11 to 20 us, 6144 x 2560 14 to 23 / 13 to 25, 4096 x 4096 14 to 22 / 14 to 26 in
+    # no order, but 6144 x 4096 18 to 30 / 18 to 40 and 4096 x 6144 17 to 28 / 19 to 43. A gated product is not cut, and what adds
+    # into the stream is launched here in a fraction of the host's time for the library's product (a 4b prompt of 160 rows with
+    # its 2560 x 4096 in the library 1.70 ms, tiled 1.63).
     TILE_ADDED_WEIGHTS = 20 << 20
-    TILE_LONG_K = 8192
 
     @classmethod
     def _tile_takes(cls, epilogue: int, x, weight, out) -> bool:
@@ -751,9 +750,8 @@ class HipKernels:
         the library's, for rows that are whole 16-byte pieces."""
         M, K = x.shape
         N = weight.shape[0]
-        added = epilogue == 0 or (epilogue == 2 and M > 128)
         return 64 < M <= 512 and x.is_cuda and K % 8 == 0 and x.stride(0) % 8 == 0 and K <= x.stride(0) < 2 ** 21 \
-            and not (added and (N * K < cls.TILE_ADDED_WEIGHTS or (M > 256 and K <= cls.TILE_LONG_K))) \
+            and (epilogue != 0 or N * K >= cls.TILE_ADDED_WEIGHTS) \
             and x.stride(1) == 1 and out.stride(0) >= out.shape[1] and weight.is_contiguous() and out.stride(1) == 1 \
             and all(t.data_ptr() % 16 == 0 for t in (x, weight, out)) \
             and bool(library.load().ra_gemm_tile_takes(epilogue, M, N, K))
@@ -1712,14 +1710,19 @@ class HipKernels:
     # 118 / 133, 153 / 137, 239 / 143, 451 / 214; 8 x 2 x 2048 x 4096 115 / 137, 120 / 141, 150 / 146, 184 / 142, 355 / 226.
     # Where few are chosen, what lies between the products is large for nothing as well: 64 x 6 x 512 x 2048 138 / 135,
     # 142 / 136, 169 / 141; 128 x 8 x 768 x 2048 323 / 274, 346 / 271, 408 / 275.
-    MOE_GROUPED_FROM = 257
+    # A step that is not captured costs the host less in the sorted form: a prompt of 16 x 4 x 1536 x 4096 over 129 to 256 rows is
+    # 5 % faster in it, a mixed step with the first sizes, whose shared expert takes three launches of its own, 2 % slower.
+    MOE_GROUPED_FROM = 129
+    MOE_GROUPED_FROM_SHARED = 257    # beside a shared expert
     MOE_GROUPED_SHARE = 0.4
     MOE_GROUPED_FEW = 0.1            # of the experts chosen: sorted from MOE_GROUPED_LEAST rows on
     MOE_GROUPED_LEAST = 65
 
-    def moe_groups_pay(self, n_tokens: int, top: int, experts: int) -> bool:
+    def moe_groups_pay(self, n_tokens: int, top: int, experts: int, shared: bool = False) -> bool:
         """Whether a step that :meth:`moe_grouped` can take is faster there than in products over all experts."""
-        return n_tokens >= (self.MOE_GROUPED_LEAST if top <= self.MOE_GROUPED_FEW * experts else self.MOE_GROUPED_FROM)
+        if top <= self.MOE_GROUPED_FEW * experts:
+            return n_tokens >= self.MOE_GROUPED_LEAST
+        return n_tokens >= (self.MOE_GROUPED_FROM_SHARED if shared else self.MOE_GROUPED_FROM)
 
     def moe_groups(self, x: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor, top: int, experts: int, ff: int) -> bool:
         """Whether :meth:`moe_grouped` can take a step over the rows ``x`` (see :meth:`moe_groups_pay`)."""

@@ -193,7 +193,7 @@ class MixtureOfExperts:
 
     def _grouped(self, ops, x, w_up, routed: int) -> bool:
         groups = getattr(ops, "moe_groups", None)
-        return groups is not None and ops.moe_groups_pay(x.shape[0], self.top, routed) \
+        return groups is not None and ops.moe_groups_pay(x.shape[0], self.top, routed, self.gated and self.shared > 0) \
             and groups(x, w_up, self.w_down, self.top, self.experts, self.ff)
 
     def _forward_grouped(self, ops, x, w_up, ids, weights, shared_logit, resid, resid_scale):

@@ -109,9 +109,11 @@ def test_an_id_below_zero_names_nothing():
 
 
 def test_where_sorting_pays():
-    """Decode steps of up to 128 requests and short mixed steps stay with the products over all experts unless few are chosen."""
+    """Decode steps of up to 128 requests, and short steps beside a shared expert, stay with the products over all experts unless
+    few are chosen."""
     pay = ops().moe_groups_pay
-    assert not any(pay(T, 4, 16) or pay(T, 2, 8) for T in (65, 128, 256)) and pay(257, 4, 16) and pay(1900, 4, 16)
+    assert not any(pay(T, 4, 16) or pay(T, 2, 8) for T in (65, 128)) and pay(129, 4, 16) and pay(1900, 4, 16)
+    assert not pay(256, 4, 16, True) and pay(257, 4, 16, True)
     assert not pay(64, 6, 64) and pay(65, 6, 64) and pay(65, 8, 128)
 
 
