@@ -129,8 +129,6 @@ class MixtureOfExperts:
                 downs.append(weights[prefix + "shared.down"])
             self.w_gate_up = torch.cat(rows, dim=0).contiguous()       # [2 (E ff + shared), width]
             self.w_down = torch.cat(downs, dim=1).contiguous()          # [width, E ff + shared]
-            # the shared expert's columns by themselves, for steps whose tokens go through their own experts alone
-            self.w_shared_down = downs[-1].contiguous() if self.shared else None
             return
         self.w_up = torch.cat([weights[f"{prefix}e{e}.up"] for e in range(self.experts)], dim=0).contiguous()
         self.w_down = torch.cat([weights[f"{prefix}e{e}.down"] for e in range(self.experts)], dim=1).contiguous()
@@ -207,7 +205,7 @@ class MixtureOfExperts:
             act = torch.empty((T, self.shared), dtype=self.dtype, device=x.device)
             ops.silu_mul(gu, act)
             more = torch.empty((T, width), dtype=torch.float32, device=x.device)
-            ops.linear(act, self.w_shared_down, more)
+            ops.linear_columns(act, self.w_down, self.experts * self.ff, more)
         out = None if resid is not None else torch.empty((T, width), dtype=self.dtype, device=x.device)
         ops.moe_grouped(x, w_up, self.w_down, ids, weights, self.experts, self.ff, self.gated, more=more,
                         more_logit=shared_logit if more is not None else None, resid=resid, alpha=resid_scale, out=out,

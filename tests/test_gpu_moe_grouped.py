@@ -151,3 +151,16 @@ def test_captured_steps_over_sorted_tokens(tmp_path):
         kind.moe_grouped = real
     for s, (a, b) in enumerate(zip(*found)):
         assert torch.isfinite(a).all() and torch.equal(a, b), s
+
+
+def test_weights_are_held_once():
+    from kobolix_helpers import _memory, _moe, draw_weights
+    from reinfer_amd.config import config_from_dict
+    from reinfer_amd.parts.moe import MixtureOfExperts
+    raw = {"architecture": "Kobolix", "vocab": 90, "width": 64, "norm": {"eps": 1e-5},
+           "layers": [{"type": "mlstm", "mixer": _memory(2, 16, 24, 12.0), "mlp": _moe(8, 2, 24, shared=16)}]}
+    weights = {n: t.to(DEV) for n, t in draw_weights(raw, 5, torch.bfloat16).items() if ".mlp." in n}
+    spec = config_from_dict(raw).to_spec().blocks[0].ffn
+    part = MixtureOfExperts(spec, weights, "l0.mlp.", torch.bfloat16, torch.device(DEV))
+    held = {t.untyped_storage().data_ptr(): t.untyped_storage().nbytes() for t in vars(part).values() if isinstance(t, torch.Tensor)}
+    assert sum(held.values()) == sum(t.numel() * t.element_size() for t in weights.values())
