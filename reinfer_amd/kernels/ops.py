@@ -155,7 +155,7 @@ class HipKernels:
         lib = library.load()
         S = int(lib.ra_gemm_wide_ranges(M, N, K))
         if S < 2 or not (lib.ra_gemm_wide_preferred if M <= 64 else lib.ra_gemm_tile_takes)(0, M, N, K) \
-                or M > 64 and (not K <= x.stride(0) < 2 ** 21 or x.data_ptr() % 16 or weight.data_ptr() % 16):
+                or M > 64 and (not K <= x.stride(0) < self.TILE_ROW_STRIDE or x.data_ptr() % 16 or weight.data_ptr() % 16):
             return None
         parts = torch.empty((S, M, N), dtype=torch.float32, device=x.device)
         library.call("ra_gemm_wide_partial", x.data_ptr(), weight.data_ptr(), parts.data_ptr(), parts.numel(),
@@ -754,6 +754,8 @@ class HipKernels:
     # into the stream is launched here in a fraction of the host's time for the library's product (a 4b prompt of 160 rows with
     # its 2560 x 4096 in the library 1.70 ms, tiled 1.63).
     TILE_ADDED_WEIGHTS = 20 << 20
+    # Elements from one row to the next up to which 512 rows, addressed in 31 bits from the first one, surely fit.
+    TILE_ROW_STRIDE = 1 << 20
 
     @classmethod
     def _tile_takes(cls, epilogue: int, x, weight, out) -> bool:
@@ -761,7 +763,7 @@ class HipKernels:
         the library's, for rows that are whole 16-byte pieces."""
         M, K = x.shape
         N = weight.shape[0]
-        return 64 < M <= 512 and x.is_cuda and K % 8 == 0 and x.stride(0) % 8 == 0 and K <= x.stride(0) < 2 ** 21 \
+        return 64 < M <= 512 and x.is_cuda and K % 8 == 0 and x.stride(0) % 8 == 0 and K <= x.stride(0) < cls.TILE_ROW_STRIDE \
             and (epilogue != 0 or N * K >= cls.TILE_ADDED_WEIGHTS) \
             and x.stride(1) == 1 and out.stride(0) >= out.shape[1] and weight.is_contiguous() and out.stride(1) == 1 \
             and all(t.data_ptr() % 16 == 0 for t in (x, weight, out)) \

@@ -132,3 +132,13 @@ def test_small_cut_products_stay_with_the_library():
         assert not any(takes(0, M, N, K) for N, K in ((8192, 2048), (6144, 2560), (4096, 4096)))
         assert takes(0, M, 6144, 4096) and takes(0, M, 4096, 6144)
     assert takes(2, 97, 2560, 4096) and takes(2, 160, 2560, 4096) and takes(2, 160, 2560, 9728) and takes(1, 97, 24576, 4096)
+
+
+def test_rows_too_far_apart_to_address_stay_with_the_library():
+    """512 rows of 2^21 elements are more than a descriptor covers: such calls went to the library's product, and still do."""
+    M, N, K = 512, 4096, 12288
+    w = torch.empty(N, K, device=DEV, dtype=torch.bfloat16)
+    for stride, taken in ((K, True), (2 ** 20 - 8, True), (2 ** 20, False), (2 ** 21 - 8, False)):
+        x = torch.empty((M - 1) * stride + K, device=DEV, dtype=torch.bfloat16).as_strided((M, K), (stride, 1))
+        assert ops()._tile_takes(2, x, w, torch.empty(M, N, device=DEV)) == taken
+        assert taken or ops().linear_ranges(x, w) is None
