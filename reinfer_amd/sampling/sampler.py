@@ -1,9 +1,10 @@
 """Sampling on the GPU from the step's float32 logits.
 
 Greedy takes the first maximum. Temperature > 0 draws by Gumbel-max with noise
-that is a pure function of (request seed, position, token id), so a request
-gets the same tokens whatever else is in the batch, however its prompt was cut
-and whether or not it was preempted and recomputed
+that is a pure function of (request seed, position, token id), so equal logits
+give a request the same tokens whatever else is in the batch, however its prompt
+was cut and whether or not it was preempted and recomputed (that the logits are
+equal to the last bit is a matter of the kernels that the steps went through)
 (crates/scheduler/src/rng.rs:52-66; crates/cuda/kernels/sampler_kernel.cu:61-77).
 Filters and penalties, if asked for, mask or shift the logits first, in the
 reference's order: repeat, frequency/presence, top-k, top-p, min-p, then
