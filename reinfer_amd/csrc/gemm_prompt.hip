@@ -1,0 +1,571 @@
+// Products of many rows in bfloat16, C[M,N] = A[M,K] . W[N,K]^T: the projections of prompts. They are bound by the matrix cores
+// (and behind those by the chip's power: on operands of zeros the same instructions run a quarter faster), so what counts is that
+// the matrix cores never wait and that every CU has work until the end.
+//
+// A workgroup of four waves, one a SIMD with all of its registers, takes tiles of 128 to 256 rows and 128 or 256 weight rows, 64 k a
+// step; a wave holds a quarter of the tile's sums. Operands go straight to LDS by loads of whole 128-byte lines, two or three steps
+// ahead (as LDS allows), and from there to registers half a step ahead, so that in the middle of a step there is one barrier, with
+// products of the first half still to issue behind it, and nowhere else a wait. Reads and fetches stand between the products, one
+// to two products apart: a wave issues in order, and a fetch holds the issue while the CU's other waves' fetches are taken (all of
+// a step's fetches in one place: 1.14 PFLOP/s at 2048 x 24576 x 4096; spread out 1.26; with the barrier moved in among the
+// products, no scalar work at the seam and the sums kept in their registers 1.39, and 1.45 at 8192 x 10240 x 5120; without any
+// fetches 1.65 and 1.76). Weights through registers instead of straight to LDS: 5 to 15 % slower. Loads past the caches' usual
+// policy (non-temporal): 2 to 50 % slower. The workgroups stay (one a CU) and ask for the next tile's first stages before they
+// write a tile's sums.
+//
+// The tile and the K ranges are chosen for the fewest part-filled rounds of workgroups, which is what the library's own product
+// loses on: with the gate 3000 x 24576 x 4096 466 us against 614 with the library and the gate's kernel, 2048 x 19456 x 2560 166
+// against 203, 512 x 51200 x 5120 234 against 288; 3000 x 6144 x 4096 127 against 146, but 8000 x 6144 x 4096, whose rounds are full
+// in any tile, 281 against 272. Weight rows of a tile are permuted (gp_row) so that a lane's sums are stored 16 bytes at a time.
+#include <type_traits>
+#include <utility>
+
+#include "common.h"
+#include "gemm_prompt.h"
+#include "reinfer_hip.h"
+
+namespace {
+
+#define GP_BK 64
+#define GP_LDS (160 * 1024)
+#define GP_STEPS 4                 // least steps of a tile
+
+enum { GP_PLAIN = 0, GP_GATED = 1, GP_ADD = 2, GP_FLOAT = 3 };
+
+struct PromptArgs {
+  const bf16_t* a;
+  const bf16_t* w;
+  void* c;
+  int M, N, K, lda, ldc;
+  float alpha;
+  int m_tiles, n_tiles, band;
+  int ranges, range_steps;        // GP_FLOAT: c is [ranges][M][N], a range of range_steps * 64 k in each
+};
+
+template <class F, int... I>
+__device__ __forceinline__ void gp_each(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+// f(0) ... f(N - 1) with the number as a constant
+template <int N, class F>
+__device__ __forceinline__ void gp_for(F&& f) {
+  gp_each(f, std::make_integer_sequence<int, N>{});
+}
+
+// The instructions stay in the order that they are written in: operand reads and fetches between the products.
+#define GP_ORDER __builtin_amdgcn_sched_barrier(0)
+
+// Written by hand so that a sum stays in its registers: of 64 sums that fill the accumulation registers the compiler moves
+// a few to and fro in every step.
+__device__ __forceinline__ void gp_mfma(f32x4_t& c, const bf16x8_t& w, const bf16x8_t& a) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(w), "v"(a));
+}
+// The wait states between a product and an ordinary access to its sums, which the compiler does not see in the assembly.
+template <int TN, int TM>
+__device__ __forceinline__ void gp_settle(f32x4_t (&acc)[TN][TM]) {
+  f32x4_t* p = &acc[0][0];
+#pragma unroll
+  for (int i = 0; i < TN * TM; i += 4)
+    asm volatile("s_nop 15\n\ts_nop 3" : "+a"(p[i]), "+a"(p[i + 1]), "+a"(p[i + 2]), "+a"(p[i + 3]));
+}
+
+// The weight row (of a wave's columns) that row r of 16-wide tile i stands for, chosen so that a lane's sums of neighbouring
+// tiles are eight features side by side, one 16-byte store: plain in pairs of tiles; gated in fours, the gate and up rows of
+// four features and of the next four (weight rows alternate in runs of eight).
+template <int EPI>
+__device__ __forceinline__ constexpr int gp_row(int i, int r) {
+  if (EPI == GP_PLAIN) return (i >> 1) * 32 + (r >> 2) * 8 + (i & 1) * 4 + (r & 3);
+  if (EPI == GP_GATED) return (i >> 2) * 64 + (r >> 2) * 16 + (i & 1) * 8 + ((i >> 1) & 1) * 4 + (r & 3);
+  return i * 16 + r;
+}
+// Piece p of 16 bytes of row r lies at place p ^ key(r): the 16 rows of a tile that are read together, two to 256 bytes, then
+// fall on all banks.
+template <int EPI>
+__device__ __forceinline__ constexpr int gp_key(int r) {
+  if (EPI == GP_PLAIN) return ((r >> 1) & 1) | ((r >> 3) & 3) << 1;
+  if (EPI == GP_GATED) return ((r >> 1) & 1) | ((r >> 4) & 3) << 1;
+  return (r >> 1) & 7;
+}
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t gp_rsrc(const bf16_t* p, size_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(p), 0,
+                                           (int)(bytes > 0xFFFFFF00ull ? 0xFFFFFF00u : (unsigned)bytes), 0x00020000);
+}
+
+// Operation t of OPS between MF products, L of which (evenly spread) are fetches, the rest operand reads: whether it is a
+// fetch, the number among its kind, and the product that it stands behind (all of them in the first 9/10, and before the last
+// seven, behind which the slots move on).
+template <int MF, int OPS, int L>
+struct GpOps {
+  static constexpr int SPAN = MF * 9 / 10 < MF - 7 ? MF * 9 / 10 : MF - 7;
+  static constexpr int fetches(int t) { return t * L / OPS; }
+  static constexpr bool fetch(int t) { return fetches(t) != fetches(t + 1); }
+  static constexpr int place(int t) { return t * SPAN / OPS; }
+  // operations that stand behind products before m
+  static constexpr int before(int m) {
+    int t = 0;
+    while (t < OPS && place(t) < m) ++t;
+    return t;
+  }
+};
+
+template <int TM, int TN, int EPI>
+__global__ void __launch_bounds__(256, 1) gemm_prompt_kernel(PromptArgs g) {
+  constexpr int BM = 32 * TM, BN = 32 * TN, PA = TM, PB = TN;      // a wave's fetches a step: 8 rows (1 KB) each
+  constexpr int SA = BM * GP_BK, SW = BN * GP_BK;                  // elements of a slot
+  // Stages that the fetches run ahead, and slots: three where LDS holds them (the weights first, which come from memory), else two.
+  // The rows' slot of stage s + DA is written in the first half of step s, when that of stage s - 1 is the last one free; the
+  // weights' of stage s + DW in the second half, when that of stage s is.
+  constexpr int DW = (3 * SA + 3 * SW) * 2 <= GP_LDS ? 3 : 2, DA = DW == 3 && (4 * SA + 3 * SW) * 2 <= GP_LDS ? 3 : 2;
+  constexpr int NA = DA + 1, NW = DW;
+  // fetches that may be under way when stage s + 1 has to be there, in the middle of step s
+  constexpr int ROWS_AHEAD = (DA - 1) * (PA + PB), WEIGHTS_AHEAD = (DW - 1) * PA + (DW - 2) * PB;
+  constexpr int UNDER_WAY = ROWS_AHEAD < WEIGHTS_AHEAD ? ROWS_AHEAD : WEIGHTS_AHEAD;
+  __shared__ __attribute__((aligned(1024))) bf16_t lds[NA * SA + NW * SW];
+  const int total = g.m_tiles * g.n_tiles * g.ranges, each = (total + RA_XCDS - 1) / RA_XCDS;
+  const int xcd = (int)blockIdx.x % RA_XCDS, stride = (int)gridDim.x / RA_XCDS;
+  const int end = min(each, total - xcd * each);
+  int at = (int)blockIdx.x / RA_XCDS;
+  if (at >= end) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  unsigned a_off[PA], w_off[PB];
+#pragma unroll
+  for (int i = 0; i < PA; ++i) {
+    const int r = (wave * PA + i) * 8 + (lane >> 3), p = (lane & 7) ^ ((r >> 1) & 7);
+    a_off[i] = ((unsigned)r * (unsigned)g.lda + p * 8) * 2u;
+  }
+#pragma unroll
+  for (int i = 0; i < PB; ++i) {
+    const int r = (wave * PB + i) * 8 + (lane >> 3), p = (lane & 7) ^ gp_key<EPI>(r);
+    w_off[i] = ((unsigned)r * (unsigned)g.K + p * 8) * 2u;
+  }
+  bf16_t* const la = lds + wave * PA * 8 * GP_BK;
+  bf16_t* const lw = lds + NA * SA + wave * PB * 8 * GP_BK;
+  auto fetch_a = [&](int i, int slot, __amdgpu_buffer_rsrc_t rs, int k) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        rs, (__attribute__((address_space(3))) void*)(la + slot + i * 8 * GP_BK), 16, (int)a_off[i], k, 0, 0);
+  };
+  auto fetch_w = [&](int i, int slot, __amdgpu_buffer_rsrc_t rs, int k) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        rs, (__attribute__((address_space(3))) void*)(lw + slot + i * 8 * GP_BK), 16, (int)w_off[i], k, 0, 0);
+  };
+  // range by range, in a range bands of `band` row tiles, inside a band column by column
+  auto place = [&](int at, int& m0, int& n0, int& z) {
+    int tile = xcd * each + at;
+    z = 0;
+    if (g.ranges > 1) {
+      z = tile / (g.m_tiles * g.n_tiles);
+      tile -= z * (g.m_tiles * g.n_tiles);
+    }
+    const int per = g.band * g.n_tiles, b = tile / per, in = tile % per;
+    const int rows = min(g.band, g.m_tiles - b * g.band);
+    m0 = (b * g.band + in % rows) * BM;
+    n0 = in / rows * BN;
+  };
+  auto steps_of = [&](int z) { return min(g.range_steps, g.K / GP_BK - z * g.range_steps); };
+  // from a tile's first row to the end of the matrix: rows past the end become zeros and cost no fetch
+  auto a_of = [&](int m0) { return gp_rsrc(g.a + (size_t)m0 * g.lda, ((size_t)(g.M - 1 - m0) * g.lda + g.K) * 2); };
+  auto w_of = [&](int n0) { return gp_rsrc(g.w + (size_t)n0 * g.K, (size_t)(g.N - n0) * g.K * 2); };
+  const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BN / 2);
+  const int lr = lane & 15, lc = lane >> 4;
+  const int ax0 = (lc ^ (lr >> 1)) * 8, ax1 = ((4 + lc) ^ (lr >> 1)) * 8;
+  const int key = gp_key<EPI>(gp_row<EPI>(0, lr));       // the same in every tile
+  const int wx0 = (lc ^ key) * 8, wx1 = ((4 + lc) ^ key) * 8;
+  const bf16_t* const ab = lds + (wm + lr) * GP_BK;
+  const bf16_t* const wb = lds + NA * SA + (wn + gp_row<EPI>(0, lr)) * GP_BK;
+  bf16x8_t x0[TM], y0[TN], x1[TM], y1[TN];
+  int m0, n0, z;
+  place(at, m0, n0, z);
+  __amdgpu_buffer_rsrc_t ar = a_of(m0), wr = w_of(n0);
+  // where along K (bytes) the next stage of rows and of weights lies
+  int ka = z * g.range_steps * GP_BK * 2, kw = ka, a_step = GP_BK * 2, w_step = GP_BK * 2;
+#pragma unroll
+  for (int s = 0; s < DW; ++s) {            // in the order of their steps: rows first
+    if (s < DA) {
+#pragma unroll
+      for (int i = 0; i < PA; ++i) fetch_a(i, s * SA, ar, ka);
+      ka += a_step;
+    }
+#pragma unroll
+    for (int i = 0; i < PB; ++i) fetch_w(i, s * SW, wr, kw);
+    kw += w_step;
+  }
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((DA - 1) * PA + (DW - 1) * PB) : "memory");
+#pragma unroll
+  for (int i = 0; i < TN; ++i) y0[i] = *(const bf16x8_t*)(wb + gp_row<EPI>(i, 0) * GP_BK + wx0);
+#pragma unroll
+  for (int j = 0; j < TM; ++j) x0[j] = *(const bf16x8_t*)(ab + j * 16 * GP_BK + ax0);
+  // the slots (elements) of stage s and of those behind it, the last one the next to be written, and the next reads
+  int as[NA], ws[NW];
+#pragma unroll
+  for (int i = 0; i < NA; ++i) as[i] = i * SA;
+#pragma unroll
+  for (int i = 0; i < NW; ++i) ws[i] = i * SW;
+  const bf16_t *ra1 = ab + ax1, *rw1 = wb + wx1, *ra0 = ab + SA + ax0, *rw0 = wb + SW + wx0;
+  while (true) {
+    f32x4_t acc[TN][TM];
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    gp_settle(acc);
+    const int next = at + stride;
+    int next_m = 0, next_n = 0, next_z = 0;
+    if (next < end) place(next, next_m, next_n, next_z);
+    const int steps = steps_of(z);       // GP_STEPS or more, so that fetches are one tile ahead at most
+    for (int s = 0; s < steps; ++s) {
+      // the first 32 k's products, the second 32 k's operand reads; the last row of products is left for behind the barrier
+      {
+        constexpr int MF = TM * (TN - 1);
+        using Ops = GpOps<MF, TM + TN + PA, PA>;
+        gp_for<MF>([&](auto mc) {
+          constexpr int m = mc, t0 = Ops::before(m);
+          gp_mfma(acc[m / TM][m % TM], y0[m / TM], x0[m % TM]);
+          GP_ORDER;
+          gp_for<Ops::before(m + 1) - t0>([&](auto tc) {
+            constexpr int t = t0 + tc, f = Ops::fetches(t), r = t - f;
+            if constexpr (Ops::fetch(t)) fetch_a(f, as[DA], ar, ka);
+            else if constexpr (r < TN) y1[r] = *(const bf16x8_t*)(rw1 + gp_row<EPI>(r, 0) * GP_BK);
+            else x1[r - TN] = *(const bf16x8_t*)(ra1 + (r - TN) * 16 * GP_BK);
+            GP_ORDER;
+          });
+        });
+      }
+      // This wave's reads of stage s are done, and of its fetches all but those of the rows of stage s + 2; the barrier makes
+      // that true of all waves: stage s + 1 is there, and the weights' slot of stage s may be written.
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(UNDER_WAY) : "memory");
+      GP_ORDER;
+      {
+        constexpr int MF = TM * (TN + 1);
+        using Ops = GpOps<MF, TM + TN + PB, PB>;
+        // the last weights and all rows are in use until the first TM products are out: with reads at their places the last
+        // row's operands are the TN-th read, and the first products behind the barrier come before it
+        gp_for<MF>([&](auto mc) {
+          constexpr int m = mc, t0 = Ops::before(m);
+          if constexpr (m < TM) gp_mfma(acc[TN - 1][m], y0[TN - 1], x0[m]);
+          else gp_mfma(acc[m / TM - 1][m % TM], y1[m / TM - 1], x1[m % TM]);
+          GP_ORDER;
+          gp_for<Ops::before(m + 1) - t0>([&](auto tc) {
+            constexpr int t = t0 + tc, f = Ops::fetches(t), r = t - f;
+            static_assert(Ops::fetch(t) || r < TN - 1 || m >= TM - 1, "a read of a register that a product behind it needs");
+            if constexpr (Ops::fetch(t)) fetch_w(f, ws[0], wr, kw);
+            else if constexpr (r < TN) y0[r] = *(const bf16x8_t*)(rw0 + gp_row<EPI>(r, 0) * GP_BK);
+            else x0[r - TN] = *(const bf16x8_t*)(ra0 + (r - TN) * 16 * GP_BK);
+            GP_ORDER;
+          });
+          if constexpr (m == MF - 6) {         // the slots move on by one stage
+            const int ta = as[0], tw = ws[0];
+#pragma unroll
+            for (int i = 0; i + 1 < NA; ++i) as[i] = as[i + 1];
+#pragma unroll
+            for (int i = 0; i + 1 < NW; ++i) ws[i] = ws[i + 1];
+            as[NA - 1] = ta;
+            ws[NW - 1] = tw;
+            ka += a_step;
+            kw += w_step;
+            GP_ORDER;
+          }
+          if constexpr (m == MF - 5) { ra1 = ab + as[0] + ax1; GP_ORDER; }
+          if constexpr (m == MF - 4) { rw1 = wb + ws[0] + wx1; GP_ORDER; }
+          if constexpr (m == MF - 3) { ra0 = ab + as[1] + ax0; GP_ORDER; }
+          if constexpr (m == MF - 2) { rw0 = wb + ws[1] + wx0; GP_ORDER; }
+        });
+      }
+      // from its last stage on the next tile's are asked for; behind the last tile nothing (and the place along K stays 0)
+      if (s + 1 + DA == steps) {
+        ar = next < end ? a_of(next_m) : gp_rsrc(g.a, 0);
+        ka = next_z * g.range_steps * GP_BK * 2;
+        if (next >= end) a_step = 0;
+      }
+      if (s + 1 + DW == steps) {
+        wr = next < end ? w_of(next_n) : gp_rsrc(g.w, 0);
+        kw = next_z * g.range_steps * GP_BK * 2;
+        if (next >= end) w_step = 0;
+      }
+    }
+    gp_settle(acc);
+    GP_ORDER;
+    // a lane holds row lane % 16 of a tile, weight rows gp_row(i, 4 (lane / 16) + e)
+    if constexpr (EPI == GP_ADD) {
+      // a part of a row of tiles at a time, the next part's old values asked for before this one's are touched
+      constexpr int H = TM * TN < 64 ? TN / 2 : TN / 4, P = TN / H;
+      f32x4_t old[2][H];
+      auto ask = [&](int u) {
+        const int m = m0 + wm + u / P * 16 + lr;
+#pragma unroll
+        for (int i = 0; i < H; ++i) {
+          const int n = n0 + wn + (u % P * H + i) * 16 + lc * 4;
+          if (m < g.M && n < g.N) old[u & 1][i] = *(const f32x4_t*)((const float*)g.c + (size_t)m * g.ldc + n);
+        }
+      };
+      ask(0);
+#pragma unroll
+      for (int u = 0; u < P * TM; ++u) {
+        if (u + 1 < P * TM) ask(u + 1);
+        GP_ORDER;
+        const int m = m0 + wm + u / P * 16 + lr;
+#pragma unroll
+        for (int i = 0; i < H; ++i) {
+          const int n = n0 + wn + (u % P * H + i) * 16 + lc * 4;
+          f32x4_t v;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = fmaf(g.alpha, acc[u % P * H + i][u / P][e], old[u & 1][i][e]);
+          if (m < g.M && n < g.N) *(f32x4_t*)((float*)g.c + (size_t)m * g.ldc + n) = v;
+        }
+        GP_ORDER;
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < TM; ++j) {
+        const int m = m0 + wm + j * 16 + lr;
+        if (EPI == GP_GATED) {
+#pragma unroll
+          for (int i = 0; i < TN; i += 4) {
+            bf16x8_t o;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              const float u = acc[i + (e >> 2) * 2][j][e & 3];
+              o[e] = (bf16_t)(u / (1.f + expf(-u)) * acc[i + (e >> 2) * 2 + 1][j][e & 3]);
+            }
+            const int n = (n0 + wn + (i >> 2) * 64) / 2 + lc * 8;
+            if (m < g.M && n < g.N / 2) *(bf16x8_t*)((bf16_t*)g.c + (size_t)m * g.ldc + n) = o;
+          }
+        } else if (EPI == GP_PLAIN) {
+#pragma unroll
+          for (int i = 0; i < TN; i += 2) {
+            bf16x8_t o;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o[e] = (bf16_t)acc[i + (e >> 2)][j][e & 3];
+            const int n = n0 + wn + (i >> 1) * 32 + lc * 8;
+            if (m < g.M && n < g.N) *(bf16x8_t*)((bf16_t*)g.c + (size_t)m * g.ldc + n) = o;
+          }
+        } else {
+#pragma unroll
+          for (int i = 0; i < TN; ++i) {
+            const int n = n0 + wn + i * 16 + lc * 4;
+            if (m < g.M && n < g.N) *(f32x4_t*)((float*)g.c + ((size_t)z * g.M + m) * g.ldc + n) = acc[i][j];
+          }
+        }
+        GP_ORDER;
+      }
+    }
+    if (next >= end) break;
+    at = next; m0 = next_m; n0 = next_n; z = next_z;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+template <int TM, int TN, int EPI>
+int prompt_launch(PromptArgs g, hipStream_t stream) {
+  g.m_tiles = (g.M + 32 * TM - 1) / (32 * TM);
+  g.n_tiles = (g.N + 32 * TN - 1) / (32 * TN);
+  const long total = (long)g.m_tiles * g.n_tiles * g.ranges, blocks = (total + RA_XCDS - 1) / RA_XCDS * RA_XCDS;
+  const long room = ra_cu_count() / RA_XCDS * RA_XCDS;
+  g.band = TM >= 2 * TN ? 4 : 8;
+  gemm_prompt_kernel<TM, TN, EPI><<<(unsigned)(blocks < room ? blocks : room), 256, 0, stream>>>(g);
+  RA_LAUNCH_CHECK("gemm_prompt");
+  return 0;
+}
+
+template <int TM, int TN>
+int prompt_epilogue(const PromptArgs& g, int epilogue, hipStream_t stream) {
+  switch (epilogue) {
+    case GP_PLAIN: return prompt_launch<TM, TN, GP_PLAIN>(g, stream);
+    case GP_GATED: return prompt_launch<TM, TN, GP_GATED>(g, stream);
+    case GP_ADD: return prompt_launch<TM, TN, GP_ADD>(g, stream);
+    default: return prompt_launch<TM, TN, GP_FLOAT>(g, stream);
+  }
+}
+
+// C[m] += alpha * (the ranges' planes, in order), and with norm_x the RMSNorm of the new row beside it. A row a workgroup, CH
+// chunks of 1024 columns; a plane's chunks are asked for together.
+template <int CH, typename TW>
+__global__ void __launch_bounds__(256) prompt_add_kernel(const float* __restrict__ planes, int ranges, float* __restrict__ C,
+                                                         int ldc, int M, int N, float alpha, const TW* __restrict__ norm_w,
+                                                         bf16_t* __restrict__ norm_x, int norm_ldx, float eps) {
+  __shared__ float red[17];
+  const int m = blockIdx.x;
+  f32x4_t v[CH], c[CH];
+#pragma unroll
+  for (int h = 0; h < CH; ++h) {
+    const int n = (h * 256 + threadIdx.x) * 4;
+    v[h] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    c[h] = n < N ? *(const f32x4_t*)(C + (size_t)m * ldc + n) : v[h];
+  }
+#pragma unroll 2
+  for (int z = 0; z < ranges; ++z)
+#pragma unroll
+    for (int h = 0; h < CH; ++h) {
+      const int n = (h * 256 + threadIdx.x) * 4;
+      if (n < N) v[h] += *(const f32x4_t*)(planes + ((size_t)z * M + m) * N + n);
+    }
+  float ss = 0.f;
+#pragma unroll
+  for (int h = 0; h < CH; ++h) {
+    const int n = (h * 256 + threadIdx.x) * 4;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      c[h][i] = fmaf(alpha, v[h][i], c[h][i]);
+      ss += c[h][i] * c[h][i];
+    }
+    if (n < N) *(f32x4_t*)(C + (size_t)m * ldc + n) = c[h];
+  }
+  if (!norm_x) return;
+  const float rstd = rsqrtf(block_sum(ss, red) / (float)N + eps);
+#pragma unroll
+  for (int h = 0; h < CH; ++h) {
+    const int n = (h * 256 + threadIdx.x) * 4;
+    if (n >= N) continue;
+    bf16x4_t o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = (bf16_t)(c[h][i] * rstd * to_f32(norm_w[n + i]));
+    *(bf16x4_t*)(norm_x + (size_t)m * norm_ldx + n) = o;
+  }
+}
+
+template <typename TW>
+int prompt_add(const float* planes, int ranges, float* C, int ldc, int M, int N, float alpha, const void* norm_w, void* norm_x,
+               int norm_ldx, float eps, hipStream_t stream) {
+#define RA_PA(CH)                                                                                                            \
+  prompt_add_kernel<CH, TW><<<M, 256, 0, stream>>>(planes, ranges, C, ldc, M, N, alpha, (const TW*)norm_w, (bf16_t*)norm_x, \
+                                                   norm_ldx, eps)
+  if (N <= 2048) RA_PA(2);
+  else if (N <= 3072) RA_PA(3);
+  else if (N <= 4096) RA_PA(4);
+  else if (N <= 5120) RA_PA(5);
+  else if (N <= 8192) RA_PA(8);
+  else RA_PA(16);
+#undef RA_PA
+  RA_LAUNCH_CHECK("gemm_prompt add");
+  return 0;
+}
+
+// Bytes that a plane costs beside its product, in us: written with it, read by the adding kernel.
+float plane_cost(int M, int N) { return (float)M * N * 4.f / 4.5e6f; }
+
+}  // namespace
+
+// What a tile of `rows` x `cols` costs, measured on MI355X over products of 128 to 3000 rows (4096 to 25600 k, one to eight
+// ranges; the tile so chosen is within 4 % of the fastest at each of 23 shapes): a start, then for each round of workgroups an
+// end that grows with the tile and the steps, each a part of its own (barrier, first operands) and one that grows with the tile,
+// the more the fuller the chip is (power and fetches).
+static RaPromptPlan prompt_plan(int M, int N, int K, int least, int most, float plane_us, int slots) {
+  static const int sides[10][2] = {{256, 256}, {224, 256}, {192, 256}, {160, 256}, {128, 256},
+                                   {256, 128}, {224, 128}, {192, 128}, {160, 128}, {128, 128}};
+  RaPromptPlan best = {0, 0, 0, 0, 1e30f};
+  const int steps = K / GP_BK;
+  for (const auto& side : sides)
+    for (int s = least; s <= most; ++s) {
+      const int each = (steps + s - 1) / s;
+      if ((long)(s - 1) * each + GP_STEPS > steps) break;
+      const long tiles = (long)((M + side[0] - 1) / side[0]) * ((N + side[1] - 1) / side[1]) * s;
+      const long rounds = ((tiles + RA_XCDS - 1) / RA_XCDS + slots - 1) / slots;
+      const float fill = (float)tiles / (float)(rounds * slots * RA_XCDS), area = (float)side[0] * side[1] / 65536.f;
+      const float us = 6.f + rounds * (11.2f * area + each * (0.227f + 0.623f * area + fill * (0.027f + 0.282f * area))) +
+                       s * plane_us;
+      if (us < best.us) best = {side[0], side[1], s, each * GP_BK, us};
+    }
+  return best;
+}
+
+// A step asks for the same few plans layer after layer, several times a product (which kernel, how much scratch, the launch), and
+// a plan is up to 150 prices: a thread keeps those of the last shapes, 0.1 us instead of 2 (a prompt of 97 rows through 8 layers
+// lasts 1.3 ms).
+RaPromptPlan ra_prompt_plan(int M, int N, int K, int least, int most, float plane_us) {
+  struct Kept {
+    int M, N, K, least, most, slots;
+    float plane_us;
+    RaPromptPlan plan;
+  };
+  static thread_local Kept kept[64];
+  const int slots = ra_cu_count() / RA_XCDS;
+  const unsigned h = (unsigned)M * 2654435761u ^ (unsigned)N * 2246822519u ^ (unsigned)K * 3266489917u ^
+                     (unsigned)(least * 31 + most) * 668265263u;
+  Kept& k = kept[h >> 26];
+  if (k.M != M || k.N != N || k.K != K || k.least != least || k.most != most || k.slots != slots || k.plane_us != plane_us)
+    k = {M, N, K, least, most, slots, plane_us, prompt_plan(M, N, K, least, most, plane_us, slots)};
+  return k.plan;
+}
+
+int ra_prompt_product(const RaPromptPlan& plan, int epilogue, const void* A, const void* W, void* C, int M, int N, int K, int lda,
+                      int ldc, float alpha, hipStream_t stream) {
+  RA_CHECK(M > 0 && ra_prompt_shape(N, K) && lda % 8 == 0 && lda >= K && lda <= (1 << 22) && (uintptr_t)A % 16 == 0 &&
+               (uintptr_t)W % 16 == 0 && (uintptr_t)C % 16 == 0 && ldc % 8 == 0 && ldc >= (epilogue == GP_GATED ? N / 2 : N),
+           "gemm_prompt: [%d, %d, %d] with rows of strides %d and %d", M, N, K, lda, ldc);
+  const int range_steps = plan.range_k / GP_BK;
+  RA_CHECK(plan.ranges >= 1 && plan.range_k % GP_BK == 0 && (long)(plan.ranges - 1) * range_steps + GP_STEPS <= K / GP_BK &&
+               (long)plan.ranges * plan.range_k >= K && (plan.ranges == 1 || (epilogue == GP_FLOAT && ldc == N)),
+           "gemm_prompt: %d ranges of %d k for %d", plan.ranges, plan.range_k, K);
+  PromptArgs g = {(const bf16_t*)A, (const bf16_t*)W, C, M, N, K, lda, ldc, alpha, 0, 0, 0, plan.ranges, range_steps};
+  switch (plan.rows * 1000 + plan.cols) {
+    case 256256: return prompt_epilogue<8, 8>(g, epilogue, stream);
+    case 224256: return prompt_epilogue<7, 8>(g, epilogue, stream);
+    case 192256: return prompt_epilogue<6, 8>(g, epilogue, stream);
+    case 160256: return prompt_epilogue<5, 8>(g, epilogue, stream);
+    case 128256: return prompt_epilogue<4, 8>(g, epilogue, stream);
+    case 256128: return prompt_epilogue<8, 4>(g, epilogue, stream);
+    case 224128: return prompt_epilogue<7, 4>(g, epilogue, stream);
+    case 192128: return prompt_epilogue<6, 4>(g, epilogue, stream);
+    case 160128: return prompt_epilogue<5, 4>(g, epilogue, stream);
+    case 128128: return prompt_epilogue<4, 4>(g, epilogue, stream);
+  }
+  return ra_fail("gemm_prompt: no tiles of %d x %d", plan.rows, plan.cols);
+}
+
+// The K ranges of a product that adds into the stream (1: it adds in its epilogue), 1 for the others, 0 where the product is not
+// this kernel's. Up to 128 rows the weights' way from memory is the bound, and gemm_tile.hip's smaller stages are ahead. With a gate
+// it is ahead of the library and the gate's kernel from there on (160 rows of 24576 x 4096, weights from memory, 57 us against 60;
+// 512 rows of 19456 x 2560 60 / 65; 4096 rows of 24576 x 4096, the one size where it is not, 626 / 608). A plain product of up to
+// 512 rows, which the library cuts, is not (512 rows of 6144 x 4096 38 / 36; 700 rows of 6144 x 2560 29 / 31). One that adds into the
+// stream is priced beside the library's, whose time over 23 shapes of 300 to 2048 rows is within 20 % of its products at 1.45 PFLOP/s
+// and 12 us and 1.4 ns a k: ahead where K is long (1024 rows of 2560 x 9728 in three ranges 48 us + 10 of the adding kernel against
+// 64 + 7 of the norm's; 600 rows of 5120 x 25600 138 + 15 / 270 + 7), behind for 2048 rows of 2560 x 4096 (54 / 50); above 3072 rows
+// the library multiplies without adding.
+extern "C" int ra_gemm_prompt_ranges(int epilogue, int M, int N, int K) {
+  if (M <= 128 || !ra_prompt_shape(N, K) || (size_t)N * K < (4u << 20)) return 0;
+  if (epilogue == GP_GATED) return 1;
+  if (epilogue == GP_PLAIN) return M > 512;
+  if (epilogue != GP_ADD || M <= 256 || M > 3072 || N > 16384) return 0;
+  // the uncut product reads and writes the stream at its end; the cut one's adding kernel reads the planes, reads and writes the
+  // stream and saves the norm kernel's launch and reading; the library's
+  const float plane = plane_cost(M, N);
+  const RaPromptPlan one = ra_prompt_plan(M, N, K, 1, 1, 0.f), cut = ra_prompt_plan(M, N, K, 2, 16, plane);
+  const float whole = one.us + 1.5f * plane, parts = cut.us + plane - 3.f;
+  const float library = (float)((double)M * N * K * 2.0 / 1.45e9) + 12.f + 0.0014f * K;
+  if ((whole < parts ? whole : parts) > library) return 0;
+  return whole <= parts ? 1 : cut.ranges;
+}
+
+// bfloat16, many rows (ra_gemm_prompt_ranges): epilogue 0 C = A . W^T in bfloat16; 1 bfloat16 silu(gate) * up; 2 float C += alpha *
+// (A . W^T); 3 float C = A . W^T. A cut product needs ranges * M * N floats of scratch and may finish the RMSNorm that follows:
+// norm_x = bf16(C * rsqrt(mean(C^2) + eps) * norm_w). tile_rows 0: the plan's own choice.
+extern "C" int ra_gemm_prompt(const void* A, const void* W, void* C, int epilogue, int M, int N, int K, int lda, int ldc,
+                              float alpha, float* scratch, long scratch_floats, const void* norm_w, int norm_w_dtype,
+                              void* norm_x, int norm_ldx, float norm_eps, int tile_rows, int tile_cols, int ranges,
+                              hipStream_t stream) {
+  RA_CHECK(epilogue >= 0 && epilogue <= 3, "gemm_prompt: epilogue %d", epilogue);
+  RA_CHECK(M > 0 && ra_prompt_shape(N, K), "gemm_prompt: a product of [%d, %d, %d]", M, N, K);
+  if (ranges < 1) ranges = epilogue == GP_ADD ? ra_gemm_prompt_ranges(epilogue, M, N, K) : 1;
+  if (ranges < 1) ranges = 1;
+  RA_CHECK(ranges == 1 || epilogue == GP_ADD, "gemm_prompt: only a product that adds is cut (%d ranges)", ranges);
+  RaPromptPlan plan = ra_prompt_plan(M, N, K, ranges, ranges, 0.f);
+  if (tile_rows) {
+    plan.rows = tile_rows;
+    plan.cols = tile_cols;
+  }
+  RA_CHECK(plan.ranges == ranges, "gemm_prompt: K of %d does not cut into %d ranges", K, ranges);
+  if (ranges == 1) {
+    RA_CHECK(!norm_x, "gemm_prompt: only a cut product finishes a norm");
+    return ra_prompt_product(plan, epilogue, A, W, C, M, N, K, lda, ldc, alpha, stream);
+  }
+  RA_CHECK(scratch && scratch_floats >= (long)ranges * M * N && (uintptr_t)scratch % 16 == 0 && N <= 16384 && ldc % 4 == 0 &&
+               ldc >= N && (uintptr_t)C % 16 == 0,
+           "gemm_prompt: %d ranges of [%d, %d] need %ld floats, got %ld", ranges, M, N, (long)ranges * M * N, scratch_floats);
+  RA_CHECK(!norm_x || (norm_w && norm_ldx >= N && norm_ldx % 4 == 0 && (uintptr_t)norm_x % 8 == 0 &&
+                       (norm_w_dtype == RA_F32 || norm_w_dtype == RA_BF16)),
+           "gemm_prompt: the norm that follows takes a weight and rows of %d", N);
+  if (int rc = ra_prompt_product(plan, GP_FLOAT, A, W, scratch, M, N, K, lda, N, 1.f, stream)) return rc;
+  return norm_w_dtype == RA_F32
+             ? prompt_add<float>(scratch, ranges, (float*)C, ldc, M, N, alpha, norm_w, norm_x, norm_ldx, norm_eps, stream)
+             : prompt_add<bf16_t>(scratch, ranges, (float*)C, ldc, M, N, alpha, norm_w, norm_x, norm_ldx, norm_eps, stream);
+}

@@ -1,4 +1,5 @@
-// Products of 65 to 512 rows in bfloat16, C[M,N] = A[M,K] . W[N,K]^T: short prompts and the largest decode steps. They are
+// Products of 65 to 128 rows in bfloat16, C[M,N] = A[M,K] . W[N,K]^T: short prompts and the largest decode steps (and of up to 512
+// rows where N or K does not fit gemm_prompt.hip's steps). They are
 // bound by reading the weights once, and by how many CUs a few tiles of 128 x 128 can be spread over: K is cut into ranges
 // until the tiles fill the chip once, each range's float sums go to a plane of their own, and the adding kernels of
 // gemm_wide.hip add the planes in order and do what stands behind the product (bias, the float stream, the norm that
@@ -20,6 +21,7 @@
 #include "common.h"
 #include "reinfer_hip.h"
 #include "gemm_tile.h"
+#include "gemm_prompt.h"
 
 namespace {
 
@@ -187,13 +189,23 @@ static long tile_count(int M, int N) { return (long)((M + GT_SIDE - 1) / GT_SIDE
 
 // As many K ranges as fill the chip once, of at least 512 k (shorter ones are all start and end), at most 16 (each is a float
 // plane to write and read again).
-void ra_tile_plan(int M, int N, int K, int* ranges, int* range_k) {
+static void tile_plan(int M, int N, int K, int* ranges, int* range_k) {
   long s = ra_cu_count() / tile_count(M, N);
   if (s > K / 512) s = K / 512;
   if (s > 16) s = 16;
   if (s < 1) s = 1;
   *range_k = ((K + (int)s - 1) / (int)s + GT_BK - 1) / GT_BK * GT_BK;
   *ranges = (K + *range_k - 1) / *range_k;
+}
+
+// The ranges of a product: above one row of tiles those of gemm_prompt.hip's, where its shape allows them (weights from memory,
+// with the adding kernel, these tiles / those: 160 rows of 6144 x 4096 32 / 25 us, 4096 x 12288 43 / 37; 300 rows 72 / 50; 256 rows
+// of 2560 x 9728 32.2 / 31.6; but 128 rows of 2560 x 4096 18.9 / 20.4, and of 24576 x 4096 with its gate 51 / 54).
+void ra_tile_plan(int M, int N, int K, int* ranges, int* range_k) {
+  const RaPromptPlan p = M > GT_SIDE && ra_prompt_shape(N, K) ? ra_prompt_plan(M, N, K, 2, 16, (float)M * N * 4.f / 4.5e6f) : RaPromptPlan();
+  if (p.ranges < 2) return tile_plan(M, N, K, ranges, range_k);
+  *ranges = p.ranges;
+  *range_k = p.range_k;
 }
 
 // Products that are cut and whose ranges fill three quarters of the chip, or that are small (the library has too few tiles for
@@ -209,7 +221,7 @@ extern "C" int ra_gemm_tile_takes(int epilogue, int M, int N, int K) {
   const long cus = ra_cu_count(), tiles = tile_count(M, N);
   if (epilogue == 1) return M <= GT_SIDE && tiles <= cus && tiles * 2 > cus;
   int ranges, range_k;
-  ra_tile_plan(M, N, K, &ranges, &range_k);
+  tile_plan(M, N, K, &ranges, &range_k);
   if (ranges < 2) return 0;
   if (M > 256) return K >= 8192 && tiles * ranges * 4 > cus * 3;
   return (epilogue == 2 && M <= GT_SIDE) || tiles * 4 <= cus || tiles * ranges * 4 >= cus * 3;
@@ -226,6 +238,11 @@ static int tile_check(const void* A, int lda, const void* W, int M, int N, int K
 int ra_tile_ranges(const void* A, int lda, const void* W, float* planes, int M, int N, int K, int ranges, int range_k,
                    hipStream_t stream) {
   if (int rc = tile_check(A, lda, W, M, N, K)) return rc;
+  if (M > GT_SIDE && ra_prompt_shape(N, K)) {
+    const RaPromptPlan p = ra_prompt_plan(M, N, K, ranges, ranges, 0.f);
+    if (p.ranges == ranges && p.range_k == range_k)
+      return ra_prompt_product(p, 3, A, W, planes, M, N, K, lda, N, 1.f, stream);
+  }
   TileArgs g = tile_args(A, lda, W, M, N, K, ranges, range_k);
   g.c = planes;
   return tile_launch<GT_SIDE, GT_PART>(g, stream);

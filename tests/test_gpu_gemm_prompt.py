@@ -1,0 +1,147 @@
+"""The bfloat16 product of many rows against float64: every tile at its edges, with each epilogue, in K ranges, and its rule."""
+import math
+
+import pytest
+import torch
+
+from reinfer_amd import kernels
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+TILES = [(m, n) for n in (256, 128) for m in (256, 224, 192, 160, 128)]
+
+
+def ops():
+    return kernels.current()
+
+
+def operands(M, N, K, seed, stride=0):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    x = torch.randn(M, K + stride, device=DEV, generator=g).to(torch.bfloat16)[:, :K]
+    w = (torch.randn(N, K, device=DEV, generator=g) / math.sqrt(K)).to(torch.bfloat16)
+    return x, w, g
+
+
+def bound(x, w, K):
+    """Float sums of K exact products in any order: K roundings of at most 2^-24 of the sum of magnitudes, which the
+    matrix cores' own order halves many times over; a twentieth of that worst case still catches a lost or doubled k."""
+    return (x.double().abs() @ w.double().abs().T) * (K * 2.0 ** -24 / 20) + 1e-6
+
+
+def gated(prod, err):
+    rows = torch.arange(prod.shape[1], device=DEV).view(-1, 2, 8)
+    gate, up = prod[:, rows[:, 0].reshape(-1)], prod[:, rows[:, 1].reshape(-1)]
+    eg, eu = err[:, rows[:, 0].reshape(-1)], err[:, rows[:, 1].reshape(-1)]
+    want = gate * torch.sigmoid(gate) * up              # silu's slope is at most 1.1
+    return want, 1.1 * eg * (up.abs() + eu) + gate.abs() * eu + want.abs() * (2 ** -8 + 2 ** -20)
+
+
+# one row and one run of weight rows; a row less and more than tiles of every height, the least K; weight rows that end inside a
+# tile; more tiles than workgroups, so that one takes several (five rows of 128 x 128 tiles in 66 columns)
+SIZES = [(1, 16, 256), (129, 1040, 256), (255, 528, 320), (449, 272, 4096), (600, 8432, 384)]
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("M,N,K", SIZES)
+def test_every_tile_with_each_epilogue(M, N, K, tile):
+    x, w, g = operands(M, N, K, M + N, stride=8)
+    ref, err = x.double() @ w.double().T, bound(x, w, K)
+    buf = torch.full((M + 1, N + 8), float("nan"), device=DEV, dtype=torch.bfloat16)
+    ops()._prompt(0, x, w, buf[:M, :N], tile=tile)
+    assert ((buf[:M, :N].double() - ref).abs() <= err + ref.abs() * 2 ** -8).all()
+    assert torch.isnan(buf[M]).all() and torch.isnan(buf[:, N:]).all()
+    buf = torch.full((M + 1, N // 2 + 8), float("nan"), device=DEV, dtype=torch.bfloat16)
+    ops()._prompt(1, x, w, buf[:M, :N // 2], tile=tile)
+    want, tol = gated(ref, err)
+    assert ((buf[:M, :N // 2].double() - want).abs() <= tol).all()
+    assert torch.isnan(buf[M]).all() and torch.isnan(buf[:, N // 2:]).all()
+    stream = torch.randn(M + 1, N + 8, device=DEV, generator=g) * 8
+    was, want = stream.clone(), stream[:M, :N].double() + 0.25 * ref
+    ops()._prompt(2, x, w, stream[:M, :N], alpha=0.25, tile=tile)
+    assert ((stream[:M, :N].double() - want).abs() <= err + want.abs() * 2 ** -23).all()
+    assert torch.equal(stream[M], was[M]) and torch.equal(stream[:, N:], was[:, N:])
+    buf = torch.full((M + 1, N + 8), float("nan"), device=DEV)
+    ops()._prompt(3, x, w, buf[:M, :N], tile=tile)
+    assert ((buf[:M, :N].double() - ref).abs() <= err).all()
+    assert torch.isnan(buf[M]).all() and torch.isnan(buf[:, N:]).all()
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("M,N,K,ranges", [(300, 1040, 1024, 4), (129, 2064, 832, 2), (513, 4112, 2560, 3), (70, 16384, 512, 2)])
+def test_ranges_are_added_and_finish_the_norm(M, N, K, ranges, tile):
+    """Ranges of the least steps and of unlike numbers of steps; every width of the adding kernel's rows."""
+    x, w, g = operands(M, N, K, M + N)
+    ref, err = x.double() @ w.double().T, bound(x, w, K)
+    norm = (torch.rand(N, device=DEV, generator=g) + 0.5)
+    for weight in (None, norm, norm.to(torch.bfloat16)):
+        stream = torch.randn(M, N, device=DEV, generator=g)
+        want = stream.double() + 0.5 * ref
+        normed = torch.full((M, N + 8), float("nan"), device=DEV, dtype=torch.bfloat16)[:, :N]
+        ops()._prompt(2, x, w, stream, 0.5, ranges, None if weight is None else (weight, normed, 1e-5), tile)
+        assert ((stream.double() - want).abs() <= err + want.abs() * 2 ** -23).all()
+        if weight is None:
+            continue
+        got = stream.double()
+        want = got * torch.rsqrt((got * got).mean(1, keepdim=True) + 1e-5) * weight.double()
+        assert ((normed.double() - want).abs() <= want.abs() * (2 ** -8 + 2 ** -18)).all()      # a rounding, and float sums
+
+
+@pytest.mark.parametrize("M,N,K", [(129, 4096, 1024), (300, 2560, 9728), (700, 2560, 4096), (1024, 2560, 9728), (3072, 1024, 4096),
+                                   (3073, 1024, 4096), (700, 4096, 1032), (700, 1048, 4096)])
+def test_calls_that_may_take_it(M, N, K):
+    """The entry points on both sides of the rule (rows, K in steps of 64, weight rows in runs of 16) and for rows that cannot be
+    read in 16-byte pieces."""
+    x, w, g = operands(M, N, K, M)
+    ref, err = x.double() @ w.double().T, bound(x, w, K)
+    odd = torch.empty(M, K + 12, device=DEV, dtype=torch.bfloat16)[:, 1:K + 1]
+    odd.copy_(x)
+    for a in (x, odd):
+        out = torch.full((M, N), float("nan"), device=DEV, dtype=torch.bfloat16)
+        ops().linear(a, w, out)
+        assert ((out.double() - ref).abs() <= err + ref.abs() * 2 ** -8).all()
+        for alpha in (1.0, 0.5):
+            stream = torch.randn(M, N, device=DEV, generator=g)
+            want = stream.double() + alpha * ref
+            ops().linear_skinny(a, w, stream, accumulate=True, alpha=alpha)
+            assert ((stream.double() - want).abs() <= err + want.abs() * 2 ** -23).all()
+        if N % 16 == 0:
+            out = torch.full((M, N // 2), float("nan"), device=DEV, dtype=torch.bfloat16)
+            ops().gated_linear(a, w, out)
+            want, tol = gated(ref, err)
+            # the library's product is rounded before its gate
+            tol = tol + (want.abs() + ref.abs().amax() * 0.1) * 2 ** -7
+            assert ((out.double() - want).abs() <= tol).all()
+        norm = torch.rand(N, device=DEV, generator=g).to(torch.bfloat16)
+        stream, normed = torch.randn(M, N, device=DEV, generator=g), torch.zeros(M, N, device=DEV, dtype=torch.bfloat16)
+        want = stream.double() + ref
+        done = ops().linear_skinny(a, w, stream, accumulate=True, finish=(norm, normed, 1e-6))
+        assert ((stream.double() - want).abs() <= err + want.abs() * 2 ** -23).all()
+        assert done == (a is x and kernels.library.load().ra_gemm_prompt_ranges(2, M, N, K) > 1)
+        if done:
+            got = stream.double()
+            want = got * torch.rsqrt((got * got).mean(1, keepdim=True) + 1e-6) * norm.double()
+            assert ((normed.double() - want).abs() <= want.abs() * (2 ** -8 + 2 ** -18)).all()
+
+
+def test_a_row_s_sums_do_not_depend_on_the_tile():
+    x, w, _ = operands(600, 1040, 2560, 5)
+    outs = []
+    for tile in TILES:
+        outs.append(torch.empty(600, 1040, device=DEV))
+        ops()._prompt(3, x, w, outs[-1], tile=tile)
+    assert all(torch.equal(o, outs[0]) for o in outs)
+
+
+def test_what_it_refuses():
+    """Sizes that it cannot read or cut are errors of the library, not launches."""
+    M, N, K = 256, 1040, 1024
+    x, w, _ = operands(M, N, K, 1)
+    out = torch.zeros(M, N, device=DEV)
+    for args in [dict(tile=(96, 128)), dict(ranges=5), dict(ranges=17)]:
+        with pytest.raises(kernels.KernelLibraryError):
+            ops()._prompt(2, x, w, out, **args)
+    for n, k in [(1048, 1024), (1040, 1000), (1040, 192)]:
+        with pytest.raises(kernels.KernelLibraryError):
+            ops()._prompt(3, x[:, :k], w[:min(n, N), :k].contiguous() if n <= N else torch.zeros(n, k, device=DEV, dtype=torch.bfloat16),
+                          torch.zeros(M, n, device=DEV))
+    assert out.abs().max() == 0
