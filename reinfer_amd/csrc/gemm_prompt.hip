@@ -30,6 +30,8 @@ namespace {
 #define GP_LDS (160 * 1024)
 #define GP_STEPS 4                 // least steps of a tile
 
+typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
+
 enum { GP_PLAIN = 0, GP_GATED = 1, GP_ADD = 2, GP_FLOAT = 3 };
 
 struct PromptArgs {
@@ -285,39 +287,46 @@ __global__ void __launch_bounds__(256, 1) gemm_prompt_kernel(PromptArgs g) {
     }
     gp_settle(acc);
     GP_ORDER;
-    // a lane holds row lane % 16 of a tile, weight rows gp_row(i, 4 (lane / 16) + e)
+    // A lane holds row lane % 16 of a tile, weight rows gp_row(i, 4 (lane / 16) + e). What lies past the last row or column is past
+    // the descriptor, which spans the result from the tile's first value on.
+    constexpr int SIZE = EPI == GP_PLAIN || EPI == GP_GATED ? 2 : 4;
+    const int cols = EPI == GP_GATED ? g.N / 2 : g.N, c0 = EPI == GP_GATED ? n0 / 2 : n0;
+    const int left = min(g.M - m0, BM);
+    const __amdgpu_buffer_rsrc_t cr = __builtin_amdgcn_make_buffer_rsrc(
+        (char*)g.c + (((size_t)(EPI == GP_FLOAT ? z : 0) * g.M + m0) * g.ldc + c0) * SIZE, 0,
+        (int)(((unsigned)(left - 1) * (unsigned)g.ldc + (cols - c0)) * SIZE), 0x00020000);
+    const unsigned row0 = (unsigned)(wm + lr) * (unsigned)g.ldc * SIZE, row_step = 16u * (unsigned)g.ldc * SIZE;
+    // where the value in column n (from the tile's first) of row tile j lies
+    auto spot = [&](int j, int n) { return (int)(c0 + n < cols ? row0 + j * row_step + n * SIZE : 0xFFFFFFF0u); };
     if constexpr (EPI == GP_ADD) {
-      // a part of a row of tiles at a time, the next part's old values asked for before this one's are touched
-      constexpr int H = TM * TN < 64 ? TN / 2 : TN / 4, P = TN / H;
-      f32x4_t old[2][H];
+      // half a row of tiles at a time; as many of the stream's old values as there are registers for are asked for ahead (the
+      // next half alone: 1733 x 4096 x 4096 62.4 us, so 58.6)
+      constexpr int H = TN / 2, AHEAD = (TM * TN <= 32 ? 32 : TM * TN < 64 ? 16 : 8) / H;
+      f32x4_t old[AHEAD][H];
       auto ask = [&](int u) {
-        const int m = m0 + wm + u / P * 16 + lr;
 #pragma unroll
-        for (int i = 0; i < H; ++i) {
-          const int n = n0 + wn + (u % P * H + i) * 16 + lc * 4;
-          if (m < g.M && n < g.N) old[u & 1][i] = *(const f32x4_t*)((const float*)g.c + (size_t)m * g.ldc + n);
-        }
+        for (int i = 0; i < H; ++i)
+          old[u % AHEAD][i] = __builtin_bit_cast(
+              f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(cr, spot(u >> 1, wn + ((u & 1) * H + i) * 16 + lc * 4), 0, 0));
       };
-      ask(0);
 #pragma unroll
-      for (int u = 0; u < P * TM; ++u) {
-        if (u + 1 < P * TM) ask(u + 1);
+      for (int u = 0; u < AHEAD && u < 2 * TM; ++u) ask(u);
+#pragma unroll
+      for (int u = 0; u < 2 * TM; ++u) {
         GP_ORDER;
-        const int m = m0 + wm + u / P * 16 + lr;
 #pragma unroll
         for (int i = 0; i < H; ++i) {
-          const int n = n0 + wn + (u % P * H + i) * 16 + lc * 4;
           f32x4_t v;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] = fmaf(g.alpha, acc[u % P * H + i][u / P][e], old[u & 1][i][e]);
-          if (m < g.M && n < g.N) *(f32x4_t*)((float*)g.c + (size_t)m * g.ldc + n) = v;
+          for (int e = 0; e < 4; ++e) v[e] = fmaf(g.alpha, acc[(u & 1) * H + i][u >> 1][e], old[u % AHEAD][i][e]);
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), cr,
+                                                 spot(u >> 1, wn + ((u & 1) * H + i) * 16 + lc * 4), 0, 0);
         }
-        GP_ORDER;
+        if (u + AHEAD < 2 * TM) ask(u + AHEAD);
       }
     } else {
 #pragma unroll
       for (int j = 0; j < TM; ++j) {
-        const int m = m0 + wm + j * 16 + lr;
         if (EPI == GP_GATED) {
 #pragma unroll
           for (int i = 0; i < TN; i += 4) {
@@ -327,8 +336,8 @@ __global__ void __launch_bounds__(256, 1) gemm_prompt_kernel(PromptArgs g) {
               const float u = acc[i + (e >> 2) * 2][j][e & 3];
               o[e] = (bf16_t)(u / (1.f + expf(-u)) * acc[i + (e >> 2) * 2 + 1][j][e & 3]);
             }
-            const int n = (n0 + wn + (i >> 2) * 64) / 2 + lc * 8;
-            if (m < g.M && n < g.N / 2) *(bf16x8_t*)((bf16_t*)g.c + (size_t)m * g.ldc + n) = o;
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, o), cr,
+                                                   spot(j, wn / 2 + (i >> 2) * 32 + lc * 8), 0, 0);
           }
         } else if (EPI == GP_PLAIN) {
 #pragma unroll
@@ -336,15 +345,13 @@ __global__ void __launch_bounds__(256, 1) gemm_prompt_kernel(PromptArgs g) {
             bf16x8_t o;
 #pragma unroll
             for (int e = 0; e < 8; ++e) o[e] = (bf16_t)acc[i + (e >> 2)][j][e & 3];
-            const int n = n0 + wn + (i >> 1) * 32 + lc * 8;
-            if (m < g.M && n < g.N) *(bf16x8_t*)((bf16_t*)g.c + (size_t)m * g.ldc + n) = o;
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, o), cr,
+                                                   spot(j, wn + (i >> 1) * 32 + lc * 8), 0, 0);
           }
         } else {
 #pragma unroll
-          for (int i = 0; i < TN; ++i) {
-            const int n = n0 + wn + i * 16 + lc * 4;
-            if (m < g.M && n < g.N) *(f32x4_t*)((float*)g.c + ((size_t)z * g.M + m) * g.ldc + n) = acc[i][j];
-          }
+          for (int i = 0; i < TN; ++i)
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, acc[i][j]), cr, spot(j, wn + i * 16 + lc * 4), 0, 0);
         }
         GP_ORDER;
       }
@@ -490,7 +497,8 @@ RaPromptPlan ra_prompt_plan(int M, int N, int K, int least, int most, float plan
 int ra_prompt_product(const RaPromptPlan& plan, int epilogue, const void* A, const void* W, void* C, int M, int N, int K, int lda,
                       int ldc, float alpha, hipStream_t stream) {
   RA_CHECK(M > 0 && ra_prompt_shape(N, K) && lda % 8 == 0 && lda >= K && lda <= (1 << 22) && (uintptr_t)A % 16 == 0 &&
-               (uintptr_t)W % 16 == 0 && (uintptr_t)C % 16 == 0 && ldc % 8 == 0 && ldc >= (epilogue == GP_GATED ? N / 2 : N),
+               (uintptr_t)W % 16 == 0 && (uintptr_t)C % 16 == 0 && ldc % 8 == 0 && ldc <= (1 << 21) &&
+               ldc >= (epilogue == GP_GATED ? N / 2 : N),
            "gemm_prompt: [%d, %d, %d] with rows of strides %d and %d", M, N, K, lda, ldc);
   const int range_steps = plan.range_k / GP_BK;
   RA_CHECK(plan.ranges >= 1 && plan.range_k % GP_BK == 0 && (long)(plan.ranges - 1) * range_steps + GP_STEPS <= K / GP_BK &&
@@ -517,10 +525,10 @@ int ra_prompt_product(const RaPromptPlan& plan, int epilogue, const void* A, con
 // it is ahead of the library and the gate's kernel from there on (160 rows of 24576 x 4096, weights from memory, 57 us against 60;
 // 512 rows of 19456 x 2560 60 / 65; 4096 rows of 24576 x 4096, the one size where it is not, 626 / 608). A plain product of up to
 // 512 rows, which the library cuts, is not (512 rows of 6144 x 4096 38 / 36; 700 rows of 6144 x 2560 29 / 31). One that adds into the
-// stream is priced beside the library's, whose time over 23 shapes of 300 to 2048 rows is within 20 % of its products at 1.45 PFLOP/s
-// and 12 us and 1.4 ns a k: ahead where K is long (1024 rows of 2560 x 9728 in three ranges 48 us + 10 of the adding kernel against
-// 64 + 7 of the norm's; 600 rows of 5120 x 25600 138 + 15 / 270 + 7), behind for 2048 rows of 2560 x 4096 (54 / 50); above 3072 rows
-// the library multiplies without adding.
+// stream is priced beside the library's, whose time for weights from memory is its products at 1.45 PFLOP/s, 14 us and 2.5 ns a k,
+// within a tenth over 20 shapes of 600 to 3000 rows: 1024 rows of 2560 x 9728 in three ranges, with the adding kernel, 64 us against
+// 85, 1733 rows of 4096 x 12288 149 / 173, 2048 rows of 2560 x 4096 uncut 50 / 53, 3000 rows of 4096 x 4096 88 / 90. Above 3072 rows
+// the library multiplies without adding, which it does faster (4096 rows of 4096 x 4096 95 us; adding 117, here 121).
 extern "C" int ra_gemm_prompt_ranges(int epilogue, int M, int N, int K) {
   if (M <= 128 || !ra_prompt_shape(N, K) || (size_t)N * K < (4u << 20)) return 0;
   if (epilogue == GP_GATED) return 1;
@@ -530,8 +538,8 @@ extern "C" int ra_gemm_prompt_ranges(int epilogue, int M, int N, int K) {
   // stream and saves the norm kernel's launch and reading; the library's
   const float plane = plane_cost(M, N);
   const RaPromptPlan one = ra_prompt_plan(M, N, K, 1, 1, 0.f), cut = ra_prompt_plan(M, N, K, 2, 16, plane);
-  const float whole = one.us + 1.5f * plane, parts = cut.us + plane - 3.f;
-  const float library = (float)((double)M * N * K * 2.0 / 1.45e9) + 12.f + 0.0014f * K;
+  const float whole = one.us + plane, parts = cut.us + plane - 3.f;
+  const float library = (float)((double)M * N * K * 2.0 / 1.45e9) + 14.f + 0.0025f * K;
   if ((whole < parts ? whole : parts) > library) return 0;
   return whole <= parts ? 1 : cut.ranges;
 }

@@ -779,7 +779,7 @@ class HipKernels:
         M, K = x.shape
         if not (M > 128 and x.is_cuda and x.dtype == weight.dtype == torch.bfloat16 and x.stride(1) == 1 and x.stride(0) % 8 == 0
                 and K <= x.stride(0) < cls.TILE_ROW_STRIDE and weight.is_contiguous() and out.stride(1) == 1
-                and out.stride(0) % 8 == 0 and out.stride(0) >= out.shape[1]
+                and out.stride(0) % 8 == 0 and out.shape[1] <= out.stride(0) < cls.TILE_ROW_STRIDE
                 and all(t.data_ptr() % 16 == 0 for t in (x, weight, out))):
             return 0
         return int(library.load().ra_gemm_prompt_ranges(epilogue, M, weight.shape[0], K))
