@@ -145,3 +145,12 @@ def test_what_it_refuses():
             ops()._prompt(3, x[:, :k], w[:min(n, N), :k].contiguous() if n <= N else torch.zeros(n, k, device=DEV, dtype=torch.bfloat16),
                           torch.zeros(M, n, device=DEV))
     assert out.abs().max() == 0
+
+
+@pytest.mark.parametrize("M", [17, 48, 64])
+@pytest.mark.parametrize("N,K", [(6144, 2560), (1536, 1024), (4099, 4096)])
+def test_small_products_are_left_in_ranges(M, N, K):
+    x, w, _ = operands(M, N, K, M + N)
+    parts = ops().linear_ranges(x, w)
+    assert parts.shape[0] == kernels.library.load().ra_gemm_wide_ranges(M, N, K) >= 2
+    assert ((parts.double().sum(0) - x.double() @ w.double().T).abs() <= bound(x, w, K)).all()
