@@ -16,3 +16,16 @@ RaPromptPlan ra_prompt_plan(int M, int N, int K, int least, int most, float plan
 // 3 float, with more than one range a plane [M, N] for each
 int ra_prompt_product(const RaPromptPlan& plan, int epilogue, const void* A, const void* W, void* C, int M, int N, int K, int lda,
                       int ldc, float alpha, hipStream_t stream);
+
+// Experts over pairs sorted by expert (moe_grouped.hip). plan: [0] tiles in all, from [4] on four ints a tile: expert | pairs << 16,
+// the first pair, the expert's first tile, the expert's tiles. slots: pair (token * top + choice) by place in the sorted run.
+struct RaExpertsPlan {
+  int rows, up_cols, down_cols;  // of a tile: sorted pairs, and weight rows of the up (and gate) and the down product
+};
+// false: not a shape of this kernel (widths in steps of 64, operands within reach of a descriptor)
+bool ra_prompt_experts_plan(int pairs, int experts, int ff, int width, int gated, long tokens, long ldx, long ld_down,
+                            RaExpertsPlan* plan);
+// kind 0: relu(a . w^T)^2, 1: silu(gate) * up of an expert's gate rows and its up rows behind them, both of tokens' rows and times
+// the pair's weight, in bfloat16; 2: a . w^T of pairs' rows in float, an expert's K columns of w's rows side by side
+int ra_prompt_experts(int rows, int cols, int kind, const void* a, long tokens, int lda, const void* w, int ldw, void* out, int N,
+                      int K, const int* plan, const int* slots, const float* weights, int top, long most, hipStream_t stream);

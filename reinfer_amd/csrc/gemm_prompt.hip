@@ -19,6 +19,7 @@
 // in any tile, 281 against 272. Weight rows of a tile are permuted (gp_row) so that a lane's sums are stored 16 bytes at a time.
 #include <type_traits>
 #include <utility>
+#include <math.h>
 
 #include "common.h"
 #include "gemm_prompt.h"
@@ -32,16 +33,24 @@ namespace {
 
 typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
 
-enum { GP_PLAIN = 0, GP_GATED = 1, GP_ADD = 2, GP_FLOAT = 3 };
+enum { GP_PLAIN = 0, GP_GATED = 1, GP_ADD = 2, GP_FLOAT = 3, GP_MOE_RELU2 = 4, GP_MOE_GATED = 5, GP_MOE_DOWN = 6 };
+// what decides where a tile's weight rows lie and how its sums are stored
+__host__ __device__ constexpr int gp_form(int epi) {
+  return epi == GP_MOE_RELU2 ? GP_PLAIN : epi == GP_MOE_GATED ? GP_GATED : epi == GP_MOE_DOWN ? GP_FLOAT : epi;
+}
 
 struct PromptArgs {
   const bf16_t* a;
   const bf16_t* w;
   void* c;
-  int M, N, K, lda, ldc;
+  int M, N, K, lda, ldw, ldc;
   float alpha;
   int m_tiles, n_tiles, band;
   int ranges, range_steps;        // GP_FLOAT: c is [ranges][M][N], a range of range_steps * 64 k in each
+  // experts (gemm_prompt.h): M is the tokens, a tile one of the plan's by a panel of columns
+  const int *plan, *slots;
+  const float* weights;
+  int top;
 };
 
 template <class F, int... I>
@@ -111,8 +120,10 @@ struct GpOps {
   }
 };
 
-template <int TM, int TN, int EPI>
+template <int TM, int TN, int KIND>
 __global__ void __launch_bounds__(256, 1) gemm_prompt_kernel(PromptArgs g) {
+  constexpr bool MOE = KIND >= GP_MOE_RELU2;
+  constexpr int EPI = gp_form(KIND);
   constexpr int BM = 32 * TM, BN = 32 * TN, PA = TM, PB = TN;      // a wave's fetches a step: 8 rows (1 KB) each
   constexpr int SA = BM * GP_BK, SW = BN * GP_BK;                  // elements of a slot
   // Stages that the fetches run ahead, and slots: three where LDS holds them (the weights first, which come from memory), else two.
@@ -124,22 +135,45 @@ __global__ void __launch_bounds__(256, 1) gemm_prompt_kernel(PromptArgs g) {
   constexpr int ROWS_AHEAD = (DA - 1) * (PA + PB), WEIGHTS_AHEAD = (DW - 1) * PA + (DW - 2) * PB;
   constexpr int UNDER_WAY = ROWS_AHEAD < WEIGHTS_AHEAD ? ROWS_AHEAD : WEIGHTS_AHEAD;
   __shared__ __attribute__((aligned(1024))) bf16_t lds[NA * SA + NW * SW];
-  const int total = g.m_tiles * g.n_tiles * g.ranges, each = (total + RA_XCDS - 1) / RA_XCDS;
+  const int total = (MOE ? g.plan[0] : g.m_tiles) * g.n_tiles * g.ranges, each = (total + RA_XCDS - 1) / RA_XCDS;
   const int xcd = (int)blockIdx.x % RA_XCDS, stride = (int)gridDim.x / RA_XCDS;
   const int end = min(each, total - xcd * each);
   int at = (int)blockIdx.x / RA_XCDS;
   if (at >= end) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // a tile of experts: whose, the sorted pairs from `first` on, and the panel of columns; an expert's tiles run along the pairs of
+  // a panel, then along panels
+  int expert = 0, pairs = 0;
+  auto moe_place = [&](int at, int& m0, int& n0) {
+    const int tile = xcd * each + at;
+    const int* t = g.plan + 4 + 4 * (tile / g.n_tiles);
+    const int first = t[2], n = t[3], in = tile - first * g.n_tiles;
+    t = g.plan + 4 + 4 * (first + in % n);
+    expert = t[0] & 0xFFFF;
+    pairs = t[0] >> 16;
+    m0 = t[1];
+    n0 = in / n * BN;
+  };
+  int m0, n0, z = 0;
+  if (MOE) moe_place(at, m0, n0);
   unsigned a_off[PA], w_off[PB];
 #pragma unroll
   for (int i = 0; i < PA; ++i) {
     const int r = (wave * PA + i) * 8 + (lane >> 3), p = (lane & 7) ^ ((r >> 1) & 7);
-    a_off[i] = ((unsigned)r * (unsigned)g.lda + p * 8) * 2u;
+    int row = r;
+    if (MOE && KIND != GP_MOE_DOWN) row = g.slots[m0 + min(r, pairs - 1)] / g.top;         // the pair's token
+    a_off[i] = ((unsigned)row * (unsigned)g.lda + p * 8) * 2u;
   }
 #pragma unroll
   for (int i = 0; i < PB; ++i) {
     const int r = (wave * PB + i) * 8 + (lane >> 3), p = (lane & 7) ^ gp_key<EPI>(r);
-    w_off[i] = ((unsigned)r * (unsigned)g.K + p * 8) * 2u;
+    const int row = KIND == GP_MOE_GATED ? ((r >> 3) & 1) * g.N + (r >> 4) * 8 + (r & 7) : r;  // gate rows, then all up rows
+    w_off[i] = ((unsigned)row * (unsigned)g.ldw + p * 8) * 2u;
+  }
+  float share[TM];                          // what the pairs of this lane's sums weigh
+  if (KIND == GP_MOE_RELU2 || KIND == GP_MOE_GATED) {
+#pragma unroll
+    for (int j = 0; j < TM; ++j) share[j] = g.weights[g.slots[m0 + min((wave >> 1) * (BM / 2) + j * 16 + (lane & 15), pairs - 1)]];
   }
   bf16_t* const la = lds + wave * PA * 8 * GP_BK;
   bf16_t* const lw = lds + NA * SA + wave * PB * 8 * GP_BK;
@@ -166,8 +200,17 @@ __global__ void __launch_bounds__(256, 1) gemm_prompt_kernel(PromptArgs g) {
   };
   auto steps_of = [&](int z) { return min(g.range_steps, g.K / GP_BK - z * g.range_steps); };
   // from a tile's first row to the end of the matrix: rows past the end become zeros and cost no fetch
-  auto a_of = [&](int m0) { return gp_rsrc(g.a + (size_t)m0 * g.lda, ((size_t)(g.M - 1 - m0) * g.lda + g.K) * 2); };
-  auto w_of = [&](int n0) { return gp_rsrc(g.w + (size_t)n0 * g.K, (size_t)(g.N - n0) * g.K * 2); };
+  auto a_of = [&](int m0) {
+    if (KIND == GP_MOE_DOWN) return gp_rsrc(g.a + (size_t)m0 * g.lda, ((size_t)(pairs - 1) * g.lda + g.K) * 2);
+    if (MOE) return gp_rsrc(g.a, ((size_t)(g.M - 1) * g.lda + g.K) * 2);
+    return gp_rsrc(g.a + (size_t)m0 * g.lda, ((size_t)(g.M - 1 - m0) * g.lda + g.K) * 2);
+  };
+  auto w_of = [&](int n0) {
+    if (KIND == GP_MOE_DOWN) return gp_rsrc(g.w + (size_t)n0 * g.ldw + (size_t)expert * g.K, ((size_t)(g.N - 1 - n0) * g.ldw + g.K) * 2);
+    if (KIND == GP_MOE_GATED) return gp_rsrc(g.w + ((size_t)expert * 2 * g.N + n0 / 2) * g.ldw, (size_t)(2 * g.N - n0 / 2) * g.ldw * 2);
+    if (MOE) return gp_rsrc(g.w + ((size_t)expert * g.N + n0) * g.ldw, (size_t)(g.N - n0) * g.ldw * 2);
+    return gp_rsrc(g.w + (size_t)n0 * g.ldw, (size_t)(g.N - n0) * g.ldw * 2);
+  };
   const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BN / 2);
   const int lr = lane & 15, lc = lane >> 4;
   const int ax0 = (lc ^ (lr >> 1)) * 8, ax1 = ((4 + lc) ^ (lr >> 1)) * 8;
@@ -176,8 +219,7 @@ __global__ void __launch_bounds__(256, 1) gemm_prompt_kernel(PromptArgs g) {
   const bf16_t* const ab = lds + (wm + lr) * GP_BK;
   const bf16_t* const wb = lds + NA * SA + (wn + gp_row<EPI>(0, lr)) * GP_BK;
   bf16x8_t x0[TM], y0[TN], x1[TM], y1[TN];
-  int m0, n0, z;
-  place(at, m0, n0, z);
+  if (!MOE) place(at, m0, n0, z);
   __amdgpu_buffer_rsrc_t ar = a_of(m0), wr = w_of(n0);
   // where along K (bytes) the next stage of rows and of weights lies
   int ka = z * g.range_steps * GP_BK * 2, kw = ka, a_step = GP_BK * 2, w_step = GP_BK * 2;
@@ -211,7 +253,7 @@ __global__ void __launch_bounds__(256, 1) gemm_prompt_kernel(PromptArgs g) {
 #pragma unroll
       for (int j = 0; j < TM; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
     gp_settle(acc);
-    const int next = at + stride;
+    const int next = MOE ? end : at + stride;      // experts: a tile a workgroup
     int next_m = 0, next_n = 0, next_z = 0;
     if (next < end) place(next, next_m, next_n, next_z);
     const int steps = steps_of(z);       // GP_STEPS or more, so that fetches are one tile ahead at most
@@ -290,8 +332,8 @@ __global__ void __launch_bounds__(256, 1) gemm_prompt_kernel(PromptArgs g) {
     // A lane holds row lane % 16 of a tile, weight rows gp_row(i, 4 (lane / 16) + e). What lies past the last row or column is past
     // the descriptor, which spans the result from the tile's first value on.
     constexpr int SIZE = EPI == GP_PLAIN || EPI == GP_GATED ? 2 : 4;
-    const int cols = EPI == GP_GATED ? g.N / 2 : g.N, c0 = EPI == GP_GATED ? n0 / 2 : n0;
-    const int left = min(g.M - m0, BM);
+    const int cols = KIND == GP_GATED ? g.N / 2 : g.N, c0 = EPI == GP_GATED ? n0 / 2 : n0;
+    const int left = MOE ? pairs : min(g.M - m0, BM);
     const __amdgpu_buffer_rsrc_t cr = __builtin_amdgcn_make_buffer_rsrc(
         (char*)g.c + (((size_t)(EPI == GP_FLOAT ? z : 0) * g.M + m0) * g.ldc + c0) * SIZE, 0,
         (int)(((unsigned)(left - 1) * (unsigned)g.ldc + (cols - c0)) * SIZE), 0x00020000);
@@ -334,7 +376,8 @@ __global__ void __launch_bounds__(256, 1) gemm_prompt_kernel(PromptArgs g) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
               const float u = acc[i + (e >> 2) * 2][j][e & 3];
-              o[e] = (bf16_t)(u / (1.f + expf(-u)) * acc[i + (e >> 2) * 2 + 1][j][e & 3]);
+              const float gate = u / (1.f + expf(-u));
+              o[e] = (bf16_t)((MOE ? share[j] * gate : gate) * acc[i + (e >> 2) * 2 + 1][j][e & 3]);
             }
             __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, o), cr,
                                                    spot(j, wn / 2 + (i >> 2) * 32 + lc * 8), 0, 0);
@@ -344,7 +387,10 @@ __global__ void __launch_bounds__(256, 1) gemm_prompt_kernel(PromptArgs g) {
           for (int i = 0; i < TN; i += 2) {
             bf16x8_t o;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) o[e] = (bf16_t)acc[i + (e >> 2)][j][e & 3];
+            for (int e = 0; e < 8; ++e) {
+              const float u = acc[i + (e >> 2)][j][e & 3], r = fmaxf(u, 0.f);
+              o[e] = (bf16_t)(MOE ? share[j] * (r * r) : u);
+            }
             __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, o), cr,
                                                    spot(j, wn + (i >> 1) * 32 + lc * 8), 0, 0);
           }
@@ -371,6 +417,18 @@ int prompt_launch(PromptArgs g, hipStream_t stream) {
   g.band = TM >= 2 * TN ? 4 : 8;
   gemm_prompt_kernel<TM, TN, EPI><<<(unsigned)(blocks < room ? blocks : room), 256, 0, stream>>>(g);
   RA_LAUNCH_CHECK("gemm_prompt");
+  return 0;
+}
+
+template <int TM, int TN>
+int prompt_experts(PromptArgs g, int kind, long most, hipStream_t stream) {
+  const int rows = kind == GP_MOE_GATED ? 2 * g.N : g.N;        // weight rows of an expert
+  g.n_tiles = (rows + 32 * TN - 1) / (32 * TN);
+  const unsigned blocks = (unsigned)((most * g.n_tiles + RA_XCDS - 1) / RA_XCDS * RA_XCDS);
+  if (kind == GP_MOE_RELU2) gemm_prompt_kernel<TM, TN, GP_MOE_RELU2><<<blocks, 256, 0, stream>>>(g);
+  else if (kind == GP_MOE_GATED) gemm_prompt_kernel<TM, TN, GP_MOE_GATED><<<blocks, 256, 0, stream>>>(g);
+  else gemm_prompt_kernel<TM, TN, GP_MOE_DOWN><<<blocks, 256, 0, stream>>>(g);
+  RA_LAUNCH_CHECK("gemm_prompt (experts)");
   return 0;
 }
 
@@ -504,7 +562,7 @@ int ra_prompt_product(const RaPromptPlan& plan, int epilogue, const void* A, con
   RA_CHECK(plan.ranges >= 1 && plan.range_k % GP_BK == 0 && (long)(plan.ranges - 1) * range_steps + GP_STEPS <= K / GP_BK &&
                (long)plan.ranges * plan.range_k >= K && (plan.ranges == 1 || (epilogue == GP_FLOAT && ldc == N)),
            "gemm_prompt: %d ranges of %d k for %d", plan.ranges, plan.range_k, K);
-  PromptArgs g = {(const bf16_t*)A, (const bf16_t*)W, C, M, N, K, lda, ldc, alpha, 0, 0, 0, plan.ranges, range_steps};
+  PromptArgs g = {(const bf16_t*)A, (const bf16_t*)W, C, M, N, K, lda, K, ldc, alpha, 0, 0, 0, plan.ranges, range_steps};
   switch (plan.rows * 1000 + plan.cols) {
     case 256256: return prompt_epilogue<8, 8>(g, epilogue, stream);
     case 224256: return prompt_epilogue<7, 8>(g, epilogue, stream);
@@ -518,6 +576,52 @@ int ra_prompt_product(const RaPromptPlan& plan, int epilogue, const void* A, con
     case 128128: return prompt_epilogue<4, 4>(g, epilogue, stream);
   }
   return ra_fail("gemm_prompt: no tiles of %d x %d", plan.rows, plan.cols);
+}
+
+// As ra_prompt_plan, of a product of `tiles` row tiles known beforehand
+static float experts_cost(long tiles, int rows, int weight_rows, int K, int cols) {
+  const int slots = ra_cu_count() / RA_XCDS;
+  const long all = tiles * ((weight_rows + cols - 1) / cols), rounds = ((all + RA_XCDS - 1) / RA_XCDS + slots - 1) / slots;
+  const float fill = (float)all / (float)(rounds * slots * RA_XCDS), area = (float)rows * cols / 65536.f;
+  return 6.f + rounds * (11.2f * area + (K / GP_BK) * (0.227f + 0.623f * area + fill * (0.027f + 0.282f * area)));
+}
+
+bool ra_prompt_experts_plan(int pairs, int experts, int ff, int width, int gated, long tokens, long ldx, long ld_down,
+                            RaExpertsPlan* plan) {
+  if (ff % 64 || width % 64 || ff < 256 || width < 256 || experts > 0xFFFF || ((tokens - 1) * ldx + width) * 2 > 0xFFFFFF00l ||
+      2l * ff * width * 2 > 0xFFFFFF00l || 256l * ld_down * 2 > 0xFFFFFF00l)
+    return false;
+  const float mean = (float)pairs / experts;
+  float best = 1e30f;
+  for (int rows = 128; rows <= 256; rows += 64) {
+    // an expert's pairs, a deviation above the mean, in whole tiles
+    const long tiles = (long)experts * (long)ceilf((mean + sqrtf(mean)) / rows);
+    const int up = gated ? 2 * ff : ff;
+    const float u[2] = {experts_cost(tiles, rows, up, width, 128), experts_cost(tiles, rows, up, width, 256)};
+    const float d[2] = {experts_cost(tiles, rows, width, ff, 128), experts_cost(tiles, rows, width, ff, 256)};
+    const float us = fminf(u[0], u[1]) + fminf(d[0], d[1]);
+    if (us < best) {
+      best = us;
+      *plan = {rows, u[0] < u[1] ? 128 : 256, d[0] < d[1] ? 128 : 256};
+    }
+  }
+  return true;
+}
+
+int ra_prompt_experts(int rows, int cols, int kind, const void* a, long tokens, int lda, const void* w, int ldw, void* out, int N,
+                      int K, const int* plan, const int* slots, const float* weights, int top, long most, hipStream_t stream) {
+  PromptArgs g = {(const bf16_t*)a, (const bf16_t*)w, out, (int)tokens, N, K, lda, ldw, N, 1.f, 0, 0, 1, 1, K / GP_BK,
+                  plan, slots, weights, top};
+  const int k = GP_MOE_RELU2 + kind;
+  switch (rows * 1000 + cols) {
+    case 256256: return prompt_experts<8, 8>(g, k, most, stream);
+    case 192256: return prompt_experts<6, 8>(g, k, most, stream);
+    case 128256: return prompt_experts<4, 8>(g, k, most, stream);
+    case 256128: return prompt_experts<8, 4>(g, k, most, stream);
+    case 192128: return prompt_experts<6, 4>(g, k, most, stream);
+    case 128128: return prompt_experts<4, 4>(g, k, most, stream);
+  }
+  return ra_fail("gemm_prompt: no tiles of %d x %d for experts", rows, cols);
 }
 
 // The K ranges of a product that adds into the stream (1: it adds in its epilogue), 1 for the others, 0 where the product is not

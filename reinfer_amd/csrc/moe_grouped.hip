@@ -5,17 +5,21 @@
 // for the most tiles there can be, and workgroups without one leave.
 //
 // Running every expert over every token instead (two library products, experts laid side by side) executes experts / top
-// times the flops at twice the rate. 1900 tokens of width 4096, 4 of 16 experts of 1536: up 280 + 29 us and down 501 us there,
-// 144 and 152 us here, with sorting and the last sum 331 us in all against 810. What bounds the products (560 to 730 TFLOP/s)
-// is LDS: every product's operands are read from it by two waves each, and written from registers between two barriers.
+// times the flops at twice the rate: 1900 tokens of width 4096, 4 of 16 experts of 1536, 810 us in all against 274 here.
+// The products of widths in steps of 64 run on gemm_prompt.hip's tiles (405 -> 274 us in all with weights from memory; 1859 tokens
+// and gated experts of 1024 312 -> 228; 300 tokens of the first 143 -> 110), the others on the kernel below, which is bound by LDS
+// (560 to 730 TFLOP/s): every product's operands are read from it by two waves each, and written from registers between two
+// barriers.
 #include "common.h"
+#include "gemm_prompt.h"
 #include "reinfer_hip.h"
 
 namespace {
 
 #define MOE_SORT_THREADS 1024
 
-// plan: [0] tiles in all, then from [4] four ints a tile: expert, first slot, slots (1..tile_rows), 0.
+// plan: [0] tiles in all, then from [4] four ints a tile: expert | slots (1..tile_rows) << 16, first slot, the expert's first tile
+// and its tiles.
 // slots[slot] = pair (token * top + choice), place[pair] = slot, or -1 for an id past the experts (the token's row itself), or
 // -2 for a pair that counts for nothing: an expert that the token names again further on weighs what it weighs there, as where
 // all experts run over all tokens. distinct: no token names one twice, nobody looks (8192 tokens, 4 choices: 50 us less).
@@ -55,10 +59,10 @@ moe_sort_kernel(const int* __restrict__ ids, int pairs, int top, bool distinct, 
         tile0[e] = tile + ns - n;
         for (int i = 0; i < n; ++i) {
           int* t = plan + 4 + 4 * (tile0[e] + i);
-          t[0] = e;
+          t[0] = e | (c - i * tile_rows < tile_rows ? c - i * tile_rows : tile_rows) << 16;
           t[1] = first + i * tile_rows;
-          t[2] = c - i * tile_rows < tile_rows ? c - i * tile_rows : tile_rows;
-          t[3] = 0;
+          t[2] = tile0[e];
+          t[3] = n;
         }
         count[e] = first;                    // from here on: the expert's next free slot
       }
@@ -113,17 +117,13 @@ __global__ void __launch_bounds__(256, 2) moe_grouped_kernel(GroupedArgs g) {
   int expert, slot0, rows, panel;
   {
     // an expert's tiles stand side by side in the plan: its panels are walked tile by tile
-    int lo = tile_no / panels;
-    const int* t = g.plan + 4 + 4 * lo;
-    expert = t[0];
-    int first = lo, last = lo;
-    while (first > 0 && g.plan[4 + 4 * (first - 1)] == expert) --first;
-    while (last + 1 < g.plan[0] && g.plan[4 + 4 * (last + 1)] == expert) ++last;
-    const int n = last - first + 1, within = tile_no - first * panels;
+    const int* t = g.plan + 4 + 4 * (tile_no / panels);
+    const int first = t[2], n = t[3], within = tile_no - first * panels;
     panel = within / n;
     t = g.plan + 4 + 4 * (first + within % n);
+    expert = t[0] & 0xFFFF;
+    rows = t[0] >> 16;
     slot0 = t[1];
-    rows = t[2];
   }
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int piece = tid & 7, srow = tid >> 3;              // staging: rows srow + 32 i
@@ -330,13 +330,23 @@ extern "C" int ra_moe_grouped(const void* x, int ldx, const void* w_up, const vo
   const GroupedScratch at = grouped_scratch(n_tokens, top, experts, ff, width);
   RA_CHECK(scratch && (uintptr_t)scratch % 256 == 0 && scratch_bytes >= (long)at.all,
            "moe_grouped: scratch of %ld bytes, needs %zu", scratch_bytes, at.all);
+  RaExpertsPlan tile;
+  const bool tiled = ra_prompt_experts_plan(n_tokens * top, experts, ff, width, gated, n_tokens, ldx, ld_down, &tile);
   char* s = (char*)scratch;
   int *plan = (int*)(s + at.plan), *slots = (int*)(s + at.slots), *place = (int*)(s + at.place);
   const int pairs = n_tokens * top;
-  moe_sort_kernel<<<1, MOE_SORT_THREADS, (size_t)experts * 8, stream>>>(ids, pairs, top, distinct != 0, experts, MOE_TILE, plan, slots,
-                                                                               place);
+  moe_sort_kernel<<<1, MOE_SORT_THREADS, (size_t)experts * 8, stream>>>(ids, pairs, top, distinct != 0, experts,
+                                                                        tiled ? tile.rows : MOE_TILE, plan, slots, place);
   RA_LAUNCH_CHECK("moe_grouped (sort)");
   const long most = most_tiles(pairs, experts);
+  if (tiled) {
+    if (int rc = ra_prompt_experts(tile.rows, tile.up_cols, gated ? 1 : 0, x, n_tokens, ldx, w_up, width, s + at.act, ff, width, plan,
+                                   slots, weights, top, most, stream))
+      return rc;
+    if (int rc = ra_prompt_experts(tile.rows, tile.down_cols, 2, s + at.act, pairs, ff, w_down, ld_down, s + at.rows, width, ff, plan,
+                                   slots, weights, top, most, stream))
+      return rc;
+  } else {
   // 256 weight rows a tile where that still leaves every CU two workgroups: half the reads of the slots' rows (gate and up
   // 1859 tokens, experts of 1024, width 4096: 171 us against 208; down 100 against 115; but up 7600 x 4096 x 1536, 384 tiles
   // of the larger kind, 157 against 144)
@@ -355,6 +365,7 @@ extern "C" int ra_moe_grouped(const void* x, int ldx, const void* w_up, const vo
   if (most * ((width + 255) / 256) >= fill) launch<128, 256, MOE_DOWN>(down, most, stream);
   else launch<128, 128, MOE_DOWN>(down, most, stream);
   RA_LAUNCH_CHECK("moe_grouped (down)");
+  }
   moe_sum_kernel<<<dim3((width / 4 + 255) / 256, n_tokens), 256, 0, stream>>>(
       (const float*)(s + at.rows), place, weights, top, (const bf16_t*)x, ldx, more, more_logit, ld_logit, resid,
       (bf16_t*)out, alpha, width);

@@ -6,6 +6,8 @@ import torch
 
 from reinfer_amd import kernels
 
+import test_gpu_moe_grouped as grouped
+
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 TILES = [(m, n) for n in (256, 128) for m in (256, 224, 192, 160, 128)]
@@ -154,3 +156,13 @@ def test_small_products_are_left_in_ranges(M, N, K):
     parts = ops().linear_ranges(x, w)
     assert parts.shape[0] == kernels.library.load().ra_gemm_wide_ranges(M, N, K) >= 2
     assert ((parts.double().sum(0) - x.double() @ w.double().T).abs() <= bound(x, w, K)).all()
+
+
+# experts in whole steps of 64: pairs of an expert on both sides of every tile height (128, 192 and 256 by the mean), experts without
+# pairs, weight rows that end inside a tile (320 and 576 columns), both tile widths; the least widths
+@pytest.mark.parametrize("T,E,top,ff,width", [(129, 3, 1, 256, 256), (100, 5, 2, 320, 576), (575, 9, 3, 320, 1088),
+                                              (640, 3, 1, 576, 320), (1500, 16, 4, 1024, 512), (3000, 5, 2, 256, 2112)])
+@pytest.mark.parametrize("gated_kind", [False, True])
+@pytest.mark.parametrize("kind", ["spread", "one", "identity"])
+def test_experts_in_whole_steps(T, E, top, ff, width, gated_kind, kind):
+    grouped.test_experts_over_sorted_tokens(T, E, top, ff, width, gated_kind, kind)
