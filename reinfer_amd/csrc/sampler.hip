@@ -221,7 +221,8 @@ extern "C" int ra_sample_static(const float* logits, int n_rows, int vocab, int 
 // with one workgroup a row 9 and 21 us).
 // ---------------------------------------------------------------------------
 #define FILTER_THREADS 256
-#define FILTER_SLICE 4096
+#define FILTER_SLICE 4096        // 16 tokens a thread
+#define FILTER_WINDOW 1024       // tokens of a window that are counted in LDS
 #define FILTER_BINS 512
 #define FILTER_BINS_A_UNIT 16.f
 #define FILTER_ROW_THREADS 1024
@@ -272,55 +273,90 @@ __device__ __forceinline__ bool filter_uses(const FilterRow& fr, int vocab) {
   return fr.temperature > 0.f && ((fr.top_k > 0 && fr.top_k < vocab) || (fr.top_p > 0.f && fr.top_p < 1.f) || fr.min_p > 0.f);
 }
 
+// A thread's 16 values of a slice, all asked for at once: value 4 q + e is token filter_at(from, q) + e. Past the row's end they
+// are no numbers, which every pass leaves alone. Rows on a 16-byte boundary are read 16 bytes at a time.
+__device__ __forceinline__ int filter_at(int from, int q) { return from + (q * FILTER_THREADS + (int)threadIdx.x) * 4; }
+__device__ __forceinline__ void filter_read(const float* lg, int from, int to, float (&l)[16]) {
+  const bool whole = (uintptr_t)lg % 16 == 0;            // `from` is a multiple of FILTER_SLICE
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int v = filter_at(from, q);
+    if (whole && v + 3 < to) {
+      const f32x4_t x = *(const f32x4_t*)(lg + v);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) l[4 * q + e] = x[e];
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) l[4 * q + e] = v + e < to ? lg[v + e] : NAN;
+    }
+  }
+}
+
 __global__ void __launch_bounds__(FILTER_THREADS)
 filter_max_kernel(float* __restrict__ logits, int vocab, int row_stride, const FilterRow* __restrict__ rows,
                   const int* __restrict__ window, float* __restrict__ slice_max) {
   __shared__ float red[FILTER_THREADS / RA_WAVE];
+  __shared__ int near_window[FILTER_WINDOW];
+  __shared__ float slice[FILTER_SLICE];
   const FilterRow fr = rows[blockIdx.y];
   float* lg = logits + (size_t)blockIdx.y * row_stride;
   const int tid = threadIdx.x, from = blockIdx.x * FILTER_SLICE, to = min(vocab, from + FILTER_SLICE);
-  // additive bias per token id, before everything else (crates/cuda/kernels/sampler_kernel.cu:189-203);
-  // the caller lists every id once
-  if (fr.bias_len > 0) {
-    const int* bp = window + fr.bias_off;
-    for (int b = tid; b < fr.bias_len; b += FILTER_THREADS) {
-      const int tok = bp[2 * b];
-      if (tok < from || tok >= to) continue;
-      const float l = lg[tok];
-      if (isfinite(l)) lg[tok] = l + __int_as_float(bp[2 * b + 1]);
-    }
-    __syncthreads();
-  }
-  // penalties: the first occurrence of a token in the window carries its count
-  const bool pen = fr.repeat_penalty > 1.f || fr.frequency_penalty > 0.f || fr.presence_penalty > 0.f;
-  if (pen && fr.window_len > 0) {
+  float l[16];
+  filter_read(lg, from, to, l);              // asked for beside the row's options and its window
+  const bool pen = (fr.repeat_penalty > 1.f || fr.frequency_penalty > 0.f || fr.presence_penalty > 0.f) && fr.window_len > 0;
+  if (pen || fr.bias_len > 0) {
+    // the slice's logits change in LDS and, where they do, in the row
+#pragma unroll
+    for (int i = 0; i < 16; ++i) slice[filter_at(0, i >> 2) + (i & 3)] = l[i];
+    // a window of usual length is read once and counted in LDS
     const int* win = window + fr.window_off;
-    for (int w = tid; w < fr.window_len; w += FILTER_THREADS) {
-      const int tok = win[w];
-      if (tok < from || tok >= to) continue;
-      bool first = true;
-      int cnt = 0;
-      for (int x = 0; x < fr.window_len; ++x) {
-        if (win[x] == tok) {
-          if (x < w) { first = false; break; }
-          ++cnt;
-        }
-      }
-      if (!first) continue;
-      float l = lg[tok];
-      if (!isfinite(l)) continue;
-      l -= fr.frequency_penalty * (float)cnt + fr.presence_penalty;
-      if (fr.repeat_penalty > 1.f) l = l > 0.f ? l / fr.repeat_penalty : l * fr.repeat_penalty;
-      lg[tok] = l;
+    if (pen && fr.window_len <= FILTER_WINDOW) {
+      for (int w = tid; w < fr.window_len; w += FILTER_THREADS) near_window[w] = win[w];
+      win = near_window;
     }
     __syncthreads();
+    // additive bias per token id, before everything else (crates/cuda/kernels/sampler_kernel.cu:189-203);
+    // the caller lists every id once
+    if (fr.bias_len > 0) {
+      const int* bp = window + fr.bias_off;
+      for (int b = tid; b < fr.bias_len; b += FILTER_THREADS) {
+        const int tok = bp[2 * b];
+        if (tok < from || tok >= to) continue;
+        const float x = slice[tok - from];
+        if (isfinite(x)) lg[tok] = slice[tok - from] = x + __int_as_float(bp[2 * b + 1]);
+      }
+      __syncthreads();
+    }
+    // penalties: the first occurrence of a token in the window carries its count
+    if (pen) {
+      for (int w = tid; w < fr.window_len; w += FILTER_THREADS) {
+        const int tok = win[w];
+        if (tok < from || tok >= to) continue;
+        bool first = true;
+        int cnt = 0;
+        for (int x = 0; x < fr.window_len; ++x) {
+          if (win[x] == tok) {
+            if (x < w) { first = false; break; }
+            ++cnt;
+          }
+        }
+        if (!first) continue;
+        float x = slice[tok - from];
+        if (!isfinite(x)) continue;
+        x -= fr.frequency_penalty * (float)cnt + fr.presence_penalty;
+        if (fr.repeat_penalty > 1.f) x = x > 0.f ? x / fr.repeat_penalty : x * fr.repeat_penalty;
+        lg[tok] = slice[tok - from] = x;
+      }
+      __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) l[i] = slice[filter_at(0, i >> 2) + (i & 3)];
   }
   if (!filter_uses(fr, vocab)) return;
   float mx = -INFINITY;
-  for (int v = from + tid; v < to; v += FILTER_THREADS) {
-    const float l = lg[v];
-    if (isfinite(l)) mx = fmaxf(mx, l / fr.temperature);
-  }
+#pragma unroll
+  for (int i = 0; i < 16; ++i)
+    if (isfinite(l[i])) mx = fmaxf(mx, l[i] / fr.temperature);
   mx = wave_max(mx);
   if ((tid & (RA_WAVE - 1)) == 0) red[tid / RA_WAVE] = mx;
   __syncthreads();
@@ -355,10 +391,12 @@ filter_bins_kernel(const float* __restrict__ logits, int vocab, int row_stride, 
     c[b] = 0u;
   }
   __syncthreads();
-  for (int v = from + tid; v < to; v += FILTER_THREADS) {
-    const float l = lg[v];
-    if (!isfinite(l)) continue;
-    const float x = l / fr.temperature, e = __expf(x - mx);
+  float l[16];
+  filter_read(lg, from, to, l);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    if (!isfinite(l[i])) continue;
+    const float x = l[i] / fr.temperature, e = __expf(x - mx);
     const int b = filter_bin(x, mx);
     atomicAdd(&c[b], 1u);
     if (e >= e_min) atomicAdd(&m[b], (unsigned long long)(e * unit));
@@ -389,7 +427,7 @@ filter_plan_kernel(int vocab, const FilterRow* __restrict__ rows, const float* _
   unsigned long long ms = 0ull;
   unsigned cs = 0u;
   const size_t at = (size_t)blockIdx.x * slices * FILTER_BINS + b;
-#pragma unroll 8
+#pragma unroll 20
   for (int i = 0; i < slices; ++i) {
     ms += mass[at + (size_t)i * FILTER_BINS];
     cs += count[at + (size_t)i * FILTER_BINS];
@@ -444,17 +482,27 @@ filter_list_kernel(const float* __restrict__ logits, int vocab, int row_stride, 
   const int tid = threadIdx.x, from = blockIdx.x * FILTER_SLICE, to = min(vocab, from + FILTER_SLICE);
   if (tid == 0) found = 0u;
   __syncthreads();
-  for (int v = from + tid; v < to; v += FILTER_THREADS) {
-    const float l = lg[v];
-    if (!isfinite(l)) continue;
-    const int b = filter_bin(l / T, p.mx);
-    if (b == p.bin_k || (p.bin_p0 >= 0 && b >= p.bin_p0 && b <= p.bin_p1)) mine[atomicAdd(&found, 1u)] = v;
+  float l[16];
+  filter_read(lg, from, to, l);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    if (!isfinite(l[i])) continue;
+    const int b = filter_bin(l[i] / T, p.mx);
+    if (b == p.bin_k || (p.bin_p0 >= 0 && b >= p.bin_p0 && b <= p.bin_p1))
+      mine[atomicAdd(&found, 1u)] = filter_at(from, i >> 2) + (i & 3);
   }
   __syncthreads();
   if (found == 0u) return;
   if (tid == 0) base = atomicAdd(&plans[blockIdx.y].listed, found);
   __syncthreads();
   for (unsigned i = tid; i < found; i += FILTER_THREADS) list[(size_t)blockIdx.y * vocab + base + i] = mine[i];
+}
+
+// Sum over eight neighbouring threads, all of which are there; whole numbers, so in any order.
+template <typename T> __device__ __forceinline__ T eight_sum(T v) {
+#pragma unroll
+  for (int m = 4; m > 0; m >>= 1) v += __shfl_xor(v, m, RA_WAVE);
+  return v;
 }
 
 // One workgroup a row: the boundaries among the listed tokens, whose order on the list means nothing.
@@ -499,11 +547,13 @@ filter_select_kernel(const float* __restrict__ logits, int vocab, int row_stride
   __syncthreads();
   if (p.bin_k >= 0) {
     if (is_short) {
-      for (int i = tid; i < n; i += FILTER_ROW_THREADS) {
+      for (int i = tid >> 3; i < n; i += FILTER_ROW_THREADS >> 3) {      // eight threads a token
         if (bins[i] != p.bin_k) continue;
+        const unsigned long long key = keys[i];
         int above = 0;
-        for (int j = 0; j < n; ++j) above += bins[j] == p.bin_k && keys[j] > keys[i];
-        if (above == p.rank_k - 1) key_min = keys[i];      // keys differ: one thread
+        for (int j = tid & 7; j < n; j += 8) above += bins[j] == p.bin_k && keys[j] > key;
+        above = eight_sum(above);
+        if (above == p.rank_k - 1) key_min = key;            // keys differ: the threads of one token
       }
     } else {
       unsigned long long lo = 0ull, hi = ~0ull;            // count(key >= lo) >= rank > count(key >= hi)
@@ -534,11 +584,13 @@ filter_select_kernel(const float* __restrict__ logits, int vocab, int row_stride
     const double need = (double)fr.top_p * (double)left;
     auto counts = [&](int bin, unsigned long long key) { return bin >= p.bin_p0 && bin <= p.bin_p1 && key >= kmin; };
     if (is_short) {
-      for (int i = tid; i < n; i += FILTER_ROW_THREADS) {
+      for (int i = tid >> 3; i < n; i += FILTER_ROW_THREADS >> 3) {
         if (!counts(bins[i], keys[i]) || es[i] < p.e_min) continue;
-        unsigned long long s = p.mass_before_p;
-        for (int j = 0; j < n; ++j) s += es[j] >= es[i] && counts(bins[j], keys[j]) ? masses[j] : 0ull;
-        if ((double)s >= need) atomicMax(&theta_bits, __float_as_uint(es[i]));
+        const float e = es[i];
+        unsigned long long s = 0ull;
+        for (int j = tid & 7; j < n; j += 8) s += es[j] >= e && counts(bins[j], keys[j]) ? masses[j] : 0ull;
+        s = eight_sum(s) + p.mass_before_p;
+        if ((tid & 7) == 0 && (double)s >= need) atomicMax(&theta_bits, __float_as_uint(e));
       }
     } else {
       unsigned lo = 0u, hi = 0x3F800001u;                  // mass(e >= lo) >= need > mass(e >= hi); e is at most 1
@@ -569,11 +621,21 @@ filter_remove_kernel(float* __restrict__ logits, int vocab, int row_stride, cons
   float* lg = logits + (size_t)blockIdx.y * row_stride;
   const float T = rows[blockIdx.y].temperature;
   const int from = blockIdx.x * FILTER_SLICE, to = min(vocab, from + FILTER_SLICE);
-  for (int v = from + threadIdx.x; v < to; v += FILTER_THREADS) {
-    const float l = lg[v];
-    if (!isfinite(l)) continue;
-    const float x = l / T, e = __expf(x - p.mx);
-    if (!(e >= p.e_min && e >= p.theta && filter_key(v, x) >= p.key_min)) lg[v] = -INFINITY;
+  const bool whole = (uintptr_t)lg % 16 == 0;
+  float l[16];
+  filter_read(lg, from, to, l);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int v = filter_at(from, q);
+    f32x4_t o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float x = l[4 * q + i] / T, e = __expf(x - p.mx);
+      const bool keep = !isfinite(l[4 * q + i]) || (e >= p.e_min && e >= p.theta && filter_key(v + i, x) >= p.key_min);
+      o[i] = keep ? l[4 * q + i] : -INFINITY;
+      if (!keep && !(whole && v + 3 < to)) lg[v + i] = -INFINITY;
+    }
+    if (whole && v + 3 < to) *(f32x4_t*)(lg + v) = o;
   }
 }
 
