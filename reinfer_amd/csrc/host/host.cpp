@@ -26,6 +26,7 @@
 #include <pybind11/stl.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
@@ -1102,8 +1103,76 @@ struct Scheduler {
   }
 };
 
+// ------------------------------------------------------------------------------------------------- sampling options
+// The rows of ra_filter_logits (12 numbers of 4 bytes each, as `filter_logits` describes them) and behind them the tokens that
+// the rows' penalties look at, as one bytearray; None where an option or token is of a kind that is left to numpy (a bias, numbers
+// that are no plain float or int, ids past 32 bits), which then takes or refuses it.
+static py::object pack_filters(const py::sequence& params, const py::sequence& histories, int n) {
+  static PyObject* const names[9] = {
+      PyUnicode_InternFromString("temperature"),       PyUnicode_InternFromString("top_p"),
+      PyUnicode_InternFromString("min_p"),             PyUnicode_InternFromString("repeat_penalty"),
+      PyUnicode_InternFromString("frequency_penalty"), PyUnicode_InternFromString("presence_penalty"),
+      PyUnicode_InternFromString("top_k"),             PyUnicode_InternFromString("repeat_last_n"),
+      PyUnicode_InternFromString("logit_bias")};
+  const size_t rows = std::min(params.size(), histories.size());
+  if (n < 0 || rows > (size_t)n) return py::none();
+  std::vector<int32_t> out((size_t)n * 12, 0), window;
+  for (size_t r = 0; r < rows; ++r) {
+    const py::object p = params[r], hist = histories[r];
+    double f[6];
+    long k[2];
+    for (int a = 0; a < 9; ++a) {
+      const py::object v = py::reinterpret_steal<py::object>(PyObject_GetAttr(p.ptr(), names[a]));
+      if (!v) {
+        if (a == 8 && PyErr_ExceptionMatches(PyExc_AttributeError)) {      // options without a bias at all
+          PyErr_Clear();
+          continue;
+        }
+        throw py::error_already_set();
+      }
+      if (a == 8) {
+        if (!PyTuple_CheckExact(v.ptr()) || PyTuple_GET_SIZE(v.ptr()) != 0) return py::none();
+      } else if (a >= 6) {
+        int overflow = 0;
+        k[a - 6] = v.is_none() && a == 6 ? 0 : PyLong_CheckExact(v.ptr()) ? PyLong_AsLongAndOverflow(v.ptr(), &overflow) : -1;
+        if (overflow || k[a - 6] < 0 || k[a - 6] > INT32_MAX) return py::none();
+      } else if (PyFloat_CheckExact(v.ptr())) {
+        f[a] = PyFloat_AS_DOUBLE(v.ptr());
+      } else if (v.is_none() && a > 0) {
+        f[a] = 0.0;
+      } else {
+        return py::none();
+      }
+    }
+    const bool looks = k[1] > 0 && (f[3] > 1.0 || f[4] > 0.0 || f[5] > 0.0);
+    for (int a : {0, 4, 5}) f[a] = f[a] > 0.0 ? f[a] : 0.0;
+    int32_t* row = out.data() + r * 12;
+    for (int a = 0; a < 6; ++a) {
+      const float x = (float)f[a];
+      std::memcpy(row + a, &x, 4);
+    }
+    row[6] = (int32_t)k[0];
+    row[7] = (int32_t)window.size();
+    if (!looks) continue;
+    if (!PyList_CheckExact(hist.ptr())) return py::none();
+    const Py_ssize_t size = PyList_GET_SIZE(hist.ptr()), from = size > k[1] ? size - k[1] : 0;
+    for (Py_ssize_t i = from; i < size; ++i) {
+      PyObject* t = PyList_GET_ITEM(hist.ptr(), i);
+      int overflow = 0;
+      const long id = PyLong_CheckExact(t) ? PyLong_AsLongAndOverflow(t, &overflow) : LONG_MAX;
+      if (overflow || id > INT32_MAX || id < INT32_MIN) return py::none();
+      window.push_back((int32_t)id);
+    }
+    row[8] = (int32_t)(size - from);
+  }
+  window.push_back(0);                       // never empty
+  out.insert(out.end(), window.begin(), window.end());
+  return py::reinterpret_steal<py::object>(PyByteArray_FromStringAndSize((const char*)out.data(), (Py_ssize_t)(out.size() * 4)));
+}
+
 PYBIND11_MODULE(_host, m) {
   m.doc() = "host runtime of reinfer_amd: cache bookkeeping, step packing, scheduler";
+  m.def("pack_filters", &pack_filters, py::arg("params"), py::arg("histories"), py::arg("rows"));
   m.def("set_exceptions", [](py::object oob, py::object oos, py::object refused, py::object step) {
     E_OutOfBlocks = new py::object(std::move(oob));
     E_OutOfSlots = new py::object(std::move(oos));

@@ -12,6 +12,7 @@ from typing import Optional
 
 import torch
 
+from .._hostlib import host as _host
 from . import library
 from .upload import to_device
 
@@ -1943,14 +1944,10 @@ class HipKernels:
                      seeds.data_ptr(), positions.data_ptr(), val.data_ptr(), idx.data_ptr(),
                      tokens.data_ptr(), _stream())
 
-    def filter_logits(self, logits: torch.Tensor, params, histories) -> None:
-        """Logit bias, penalties and top-k / top-p / min-p of every row's SamplingParams, in
-        place (removed tokens become -inf); ``histories[i]`` are row i's tokens so far."""
+    @staticmethod
+    def _pack_filters(params, histories, n: int):
+        """The rows and windows of ``ra_filter_logits`` from options and tokens of any kind (and with biases)."""
         import numpy as np
-        _dev(logits)
-        n, V = logits.shape
-        if logits.dtype != torch.float32 or logits.stride(1) != 1:
-            raise TypeError("filter_logits: logits are float32 rows")
         floats, ints, window = [], [], []
         for p, hist in zip(params, histories):
             repeat, frequency, presence = p.repeat_penalty or 0.0, p.frequency_penalty or 0.0, p.presence_penalty or 0.0
@@ -1975,7 +1972,20 @@ class HipKernels:
             packed = np.frombuffer(struct.pack(f"{len(window)}i", *window), dtype=np.int32)     # half the time of an array of the list
         except struct.error:                 # numbers of another kind among the tokens
             packed = torch.tensor(window, dtype=torch.int32).numpy()
-        both = to_device(np.concatenate([rec.view(np.int32).reshape(-1), packed]), logits.device)
+        return np.concatenate([rec.view(np.int32).reshape(-1), packed])
+
+    def filter_logits(self, logits: torch.Tensor, params, histories) -> None:
+        """Logit bias, penalties and top-k / top-p / min-p of every row's SamplingParams, in
+        place (removed tokens become -inf); ``histories[i]`` are row i's tokens so far."""
+        import numpy as np
+        _dev(logits)
+        n, V = logits.shape
+        if logits.dtype != torch.float32 or logits.stride(1) != 1:
+            raise TypeError("filter_logits: logits are float32 rows")
+        lists = isinstance(params, (list, tuple)) and isinstance(histories, (list, tuple))
+        packed = _host.pack_filters(params, histories, n) if lists else None
+        packed = np.frombuffer(packed, dtype=np.int32) if packed is not None else self._pack_filters(params, histories, n)
+        both = to_device(packed, logits.device)
         rows_t, win_t = both[:12 * n], both[12 * n:]
         need = int(library.load().ra_filter_scratch(n, V))
         scratch = torch.empty(need, dtype=torch.uint8, device=logits.device)
