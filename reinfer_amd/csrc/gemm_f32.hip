@@ -6,10 +6,12 @@
 // element of it each.
 //
 // Up to 32 rows (gemm_f32_stream_kernel) the product is bound by reading the weights once. A workgroup has 16 features, its
-// waves share K out and add their sums through LDS in a fixed order; both operands go from memory to the matrix cores
-// without LDS. At 4 rows 19456 x 2560 takes 41 us (4.8 TB/s) and 151936 x 2560 277 us (5.6 TB/s), where the plain kernel
-// took 406 us for the first; with more rows the activations, which every workgroup reads again, cost as much as the weights
-// (19456 x 2560 at 32 rows 93 us).
+// waves share K out and add their sums through LDS in a fixed order. The activations go from memory to the matrix cores, the
+// weights by way of a piece of LDS of each wave's own: loaded in the products' order a load is 64 bytes of each of 16 rows, half a
+// line each, and takes twice the time of whole lines of 4 rows (weights from memory at 4 rows, straight / by way of LDS: 6144 x 2560
+// 23.6 / 20.0 us, 2560 x 4096 17.7 / 14.3, 19456 x 2560 45.8 / 41.6, 2560 x 9728 33.2 / 29.4, 151936 x 2560 298 / 265; at 32 rows
+// 19456 x 2560 100 / 82; a product of 1000 x 1028, all start and end, 10.2 / 11.0). Three or four runs in flight instead of two
+// change nothing. With more rows the activations, which every workgroup reads again, cost as much as the weights.
 //
 // From 33 rows on (gemm_f32_tile_kernel) tiles of both operands go through LDS, 32 k at a time, by loads that go straight
 // there; two stages and one barrier a step. The float matrix cores do 256 flops a clock and CU and bound it. Tiles of 64 x 128
@@ -49,7 +51,9 @@ gemm_f32_stream_kernel(const float* __restrict__ A, const float* __restrict__ W,
                        float* __restrict__ C, int M, int N, int K, int lda, int ldc, int block_k) {
   constexpr int SPAN = U * 32;             // k of one run of a wave
   constexpr unsigned NOWHERE = 0xFFFFFFF0u;
+  constexpr int CH = SPAN / 4;             // 16-byte pieces of a weight row in a run
   __shared__ f32x4_t sums[2][8][MT][RA_WAVE];            // of one tile while the next one's may already be written
+  __shared__ f32x4_t laid[8][16 * CH];                   // a wave's run of weights on its way into the products' order
   const int lane = threadIdx.x & 63, waves = blockDim.x >> 6;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, q = lane >> 4;
@@ -63,17 +67,24 @@ gemm_f32_stream_kernel(const float* __restrict__ A, const float* __restrict__ W,
       __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(W), 0, (int)((size_t)N * K * 4), 0x00020000);
   const __amdgpu_buffer_rsrc_t a_rsrc =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(A), 0, (int)(((size_t)(M - 1) * lda + K) * 4), 0x00020000);
-  f32x4_t w[DEPTH][U][2], a[DEPTH][U][MT][2];
-  int l_q = 0, l_step = 0, l_n = (int)blockIdx.x * 16 + r;         // where the loads are
+  // A load of weights takes whole lines of a few rows, lane after lane; piece c of row r of a run lies at place c ^ r in LDS, from
+  // where the products' rows are read without conflicts.
+  constexpr int LOADS = U * 2, LR = 16 / LOADS;          // loads of a run, rows of one
+  const int wr = lane / CH, wc = lane % CH;
+  f32x4_t w[DEPTH][LOADS], a[DEPTH][U][MT][2];
+  int l_q = 0, l_step = 0, l_n = (int)blockIdx.x * 16;             // where the loads are
 #define RA_F32_LOAD(d)                                                                                        \
   do {                                                                                                        \
     const bool live_ = l_q < total && l_step < n_steps;                                                       \
+    _Pragma("unroll") for (int i = 0; i < LOADS; ++i) {                                                       \
+      const int k_ = k0 + l_step * SPAN + wc * 4, n_ = l_n + i * LR + wr;                                     \
+      const unsigned off_ = live_ && k_ < k1 && n_ < N ? (unsigned)(((size_t)n_ * K + k_) * 4) : NOWHERE;     \
+      w[d][i] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, off_, 0, 0));       \
+    }                                                                                                         \
     _Pragma("unroll") for (int u = 0; u < U; ++u)                                                             \
       _Pragma("unroll") for (int j = 0; j < 2; ++j) {                                                         \
         const int k_ = k0 + l_step * SPAN + u * 32 + j * 16 + q * 4;                                          \
         const bool ok_ = live_ && k_ < k1;           /* a multiple of 4 */                                    \
-        const unsigned off_ = ok_ && l_n < N ? (unsigned)(((size_t)l_n * K + k_) * 4) : NOWHERE;              \
-        w[d][u][j] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, off_, 0, 0));  \
         _Pragma("unroll") for (int t = 0; t < MT; ++t) {                                                      \
           const int m_ = t * 16 + r;                                                                          \
           const unsigned at_ = ok_ && m_ < M ? (unsigned)(((size_t)m_ * lda + k_) * 4) : NOWHERE;             \
@@ -95,15 +106,20 @@ gemm_f32_stream_kernel(const float* __restrict__ A, const float* __restrict__ W,
   for (int base = 0; base < total; base += DEPTH) {
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d) {
+      f32x4_t* const mine = laid[wave];      // this wave's alone: LDS takes its accesses in their order
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) mine[(i * LR + wr) * CH + (wc ^ ((i * LR + wr) & (CH - 1)))] = w[d][i];
 #pragma unroll
       for (int u = 0; u < U; ++u)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < 2; ++j) {
+          const f32x4_t y = mine[r * CH + (((u * 2 + j) * 4 + q) ^ (r & (CH - 1)))];
 #pragma unroll
           for (int e = 0; e < 4; ++e)
 #pragma unroll
             for (int t = 0; t < MT; ++t)
-              acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[d][u][j][e], a[d][u][t][j][e], acc[t], 0, 0, 0);
+              acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(y[e], a[d][u][t][j][e], acc[t], 0, 0, 0);
+        }
       __builtin_amdgcn_sched_barrier(0);   // the run DEPTH ahead is asked for once this one's registers are free
       RA_F32_LOAD(d);
       __builtin_amdgcn_sched_barrier(0);
