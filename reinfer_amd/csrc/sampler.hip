@@ -427,7 +427,7 @@ filter_plan_kernel(int vocab, const FilterRow* __restrict__ rows, const float* _
   unsigned long long ms = 0ull;
   unsigned cs = 0u;
   const size_t at = (size_t)blockIdx.x * slices * FILTER_BINS + b;
-#pragma unroll 20
+#pragma unroll 8
   for (int i = 0; i < slices; ++i) {
     ms += mass[at + (size_t)i * FILTER_BINS];
     cs += count[at + (size_t)i * FILTER_BINS];
