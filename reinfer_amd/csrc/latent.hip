@@ -122,12 +122,13 @@ extern "C" int ra_latent_prep(const void* proj, int act_dtype, int ld, int q_off
 // owns 16 output columns of one head for MT tiles of 16 tokens and walks K in steps of 32; both operands come
 // straight from memory in operand layout (lane (r, g): row r, elements 8g .. 8g + 7 of the step, one 16-byte
 // load), the weights of a head being small enough to stay in the caches while the token tiles pass. The four
-// waves of a workgroup take four column tiles. Lane (r, g) ends with out[token r][column 4g .. 4g + 3], stored as one 8-byte
-// piece where rows allow it. Bound by memory: the rows in and out (1900 tokens, 16 heads, 128 -> 192 and back, 20 MB a
-// product: 22 us; with two-byte stores and each step's loads waited for, 30).
+// waves of a workgroup take four column tiles, or, with many tokens, four token tiles of 32 with four column tiles each, so that a
+// head's rows are read once for four column tiles. Lane (r, g) ends with out[token r][column 4g .. 4g + 3], stored as one 8-byte
+// piece where rows allow it. Bound by memory: the rows in and out (1900 tokens, 16 heads, 128 -> 192 and back with a gate, 20
+// and 27 MB: 17 and 20 us; with one column tile a wave 22 and 24, with two-byte stores and each step's loads waited for, 30).
 // Anything else (float, odd sizes): a plain kernel, 16 tokens of one head a workgroup, x in LDS as float.
 // ---------------------------------------------------------------------------
-template <int MT>
+template <int MT, int NT>
 __global__ void __launch_bounds__(256)
 head_linear_mfma_kernel(const bf16_t* __restrict__ x, int ldx, int x_head, const bf16_t* __restrict__ W,
                         bf16_t* __restrict__ out, int ldo, int o_head, const bf16_t* __restrict__ gate, int ldg,
@@ -136,67 +137,82 @@ head_linear_mfma_kernel(const bf16_t* __restrict__ x, int ldx, int x_head, const
   const int wave = threadIdx.x / RA_WAVE;
   const int r = lane & 15, g = lane >> 4;
   const int h = blockIdx.z;
-  const int n0 = (blockIdx.x * 4 + wave) * 16;
-  const int t0 = blockIdx.y * 16 * MT;
-  if (n0 >= N) return;
+  // with one column tile a wave the waves stand side by side along the columns, else along the tokens
+  const int n0 = NT == 1 ? (blockIdx.x * 4 + wave) * 16 : blockIdx.x * 16 * NT;
+  const int t0 = (NT == 1 ? blockIdx.y : blockIdx.y * 4 + wave) * 16 * MT;
+  if (n0 >= N || t0 >= T) return;
   // rows past the end are a row that is there: nobody stores what becomes of them
-  const bf16_t* wrow = W + ((size_t)h * N + (n0 + r < N ? n0 + r : 0)) * K;
-  const bf16_t* xrow[MT];
+  const bf16_t *wrow[NT], *xrow[MT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    const int n = n0 + nt * 16 + r;
+    wrow[nt] = W + ((size_t)h * N + (n < N ? n : 0)) * K;
+  }
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     const int t = t0 + mt * 16 + r;
     xrow[mt] = x + (size_t)(t < T ? t : 0) * ldx + (size_t)h * x_head;
   }
-  f32x4_t acc[MT];
+  f32x4_t acc[MT][NT];
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) acc[mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   const bf16x8_t zero = {0, 0, 0, 0, 0, 0, 0, 0};
   for (int k0 = 0; k0 < K; k0 += 64) {                // two steps' loads are on their way together
-    bf16x8_t a[2], b[2][MT];
+    bf16x8_t a[2][NT], b[2][MT];
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       const int k = k0 + s * 32 + g * 8;
       const bool k_ok = k < K;                        // K is a multiple of 8: a chunk is whole or absent
       const int at = k_ok ? k : 0;
-      a[s] = *(const bf16x8_t*)(wrow + at);
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) b[s][mt] = *(const bf16x8_t*)(xrow[mt] + at);
-      if (!k_ok) {
-        a[s] = zero;
+      for (int nt = 0; nt < NT; ++nt) {
+        a[s][nt] = *(const bf16x8_t*)(wrow[nt] + at);
+        if (!k_ok) a[s][nt] = zero;
+      }
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) b[s][mt] = zero;
+      for (int mt = 0; mt < MT; ++mt) {
+        b[s][mt] = *(const bf16x8_t*)(xrow[mt] + at);
+        if (!k_ok) b[s][mt] = zero;
       }
     }
 #pragma unroll
     for (int s = 0; s < 2; ++s)
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[s], b[s][mt], acc[mt], 0, 0, 0);
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+          acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[s][nt], b[s][mt], acc[mt][nt], 0, 0, 0);
   }
-  const int n = n0 + 4 * g;
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     const int t = t0 + mt * 16 + r;
     if (t >= T) continue;
-    bf16_t* o = out + (size_t)t * ldo + (size_t)h * o_head + n;
-    const bf16_t* gt = gate ? gate + (size_t)t * ldg + (gate_per_head ? (size_t)h : (size_t)h * N + n) : nullptr;
-    if (whole && n < N) {
-      f32x4_t v = acc[mt];
-      if (gate) {
-        bf16x4_t gv;
-        if (gate_per_head) gv = (bf16x4_t){gt[0], gt[0], gt[0], gt[0]};
-        else gv = *(const bf16x4_t*)gt;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] *= 1.f / (1.f + expf(-to_f32((bf16_t)gv[i])));
+    for (int nt = 0; nt < NT; ++nt) {
+      const int n = n0 + nt * 16 + 4 * g;
+      bf16_t* o = out + (size_t)t * ldo + (size_t)h * o_head + n;
+      const bf16_t* gt = gate ? gate + (size_t)t * ldg + (gate_per_head ? (size_t)h : (size_t)h * N + n) : nullptr;
+      if (whole && n < N) {
+        f32x4_t v = acc[mt][nt];
+        if (gate) {
+          bf16x4_t gv;
+          if (gate_per_head) gv = (bf16x4_t){gt[0], gt[0], gt[0], gt[0]};
+          else gv = *(const bf16x4_t*)gt;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[i] *= 1.f / (1.f + expf(-to_f32((bf16_t)gv[i])));
+        }
+        *(bf16x4_t*)o = (bf16x4_t){from_f32<bf16_t>(v[0]), from_f32<bf16_t>(v[1]), from_f32<bf16_t>(v[2]), from_f32<bf16_t>(v[3])};
+        continue;
       }
-      *(bf16x4_t*)o = (bf16x4_t){from_f32<bf16_t>(v[0]), from_f32<bf16_t>(v[1]), from_f32<bf16_t>(v[2]), from_f32<bf16_t>(v[3])};
-      continue;
-    }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if (n + i >= N) continue;
-      float v = acc[mt][i];
-      if (gate) v *= 1.f / (1.f + expf(-to_f32(gt[gate_per_head ? 0 : i])));
-      o[i] = from_f32<bf16_t>(v);
+      for (int i = 0; i < 4; ++i) {
+        if (n + i >= N) continue;
+        float v = acc[mt][nt][i];
+        if (gate) v *= 1.f / (1.f + expf(-to_f32(gt[gate_per_head ? 0 : i])));
+        o[i] = from_f32<bf16_t>(v);
+      }
     }
   }
 }
@@ -263,14 +279,21 @@ extern "C" int ra_head_linear(const void* x, int ldx, int x_head, const void* W,
                        (gate == nullptr || gate_per_head || (ldg % 4 == 0 && (uintptr_t)gate % 8 == 0));
     if (n_tokens <= 16) {
       dim3 grid(col_groups, 1, H);
-      head_linear_mfma_kernel<1><<<grid, 256, 0, stream>>>((const bf16_t*)x, ldx, x_head, (const bf16_t*)W,
+      head_linear_mfma_kernel<1, 1><<<grid, 256, 0, stream>>>((const bf16_t*)x, ldx, x_head, (const bf16_t*)W,
                                                            (bf16_t*)out, ldo, o_head, (const bf16_t*)gate, ldg,
                                                            gate_per_head, n_tokens, N, K, whole);
+    } else if ((long)((n_tokens + 31) / 32) * ((N + 63) / 64) * H >= 4 * ra_cu_count() && N % 64 == 0) {
+      // four column tiles a wave where that still leaves one wave a SIMD: with one, a wave loads five operands for four products
+      // and a head's rows as often as it has column tiles (1000 tokens, 128 -> 192: 13.8 us, so 12.6; at 520, 780 waves, the same)
+      dim3 grid(N / 64, (n_tokens + 127) / 128, H);
+      head_linear_mfma_kernel<2, 4><<<grid, 256, 0, stream>>>((const bf16_t*)x, ldx, x_head, (const bf16_t*)W,
+                                                              (bf16_t*)out, ldo, o_head, (const bf16_t*)gate, ldg,
+                                                              gate_per_head, n_tokens, N, K, whole);
     } else {
       const int tiles = (n_tokens + 63) / 64;
       RA_CHECK(tiles <= 65535, "head_linear: %d tokens in one launch", n_tokens);
       dim3 grid(col_groups, tiles, H);
-      head_linear_mfma_kernel<4><<<grid, 256, 0, stream>>>((const bf16_t*)x, ldx, x_head, (const bf16_t*)W,
+      head_linear_mfma_kernel<4, 1><<<grid, 256, 0, stream>>>((const bf16_t*)x, ldx, x_head, (const bf16_t*)W,
                                                            (bf16_t*)out, ldo, o_head, (const bf16_t*)gate, ldg,
                                                            gate_per_head, n_tokens, N, K, whole);
     }
