@@ -273,7 +273,8 @@ extern "C" int ra_head_linear(const void* x, int ldx, int x_head, const void* W,
   RA_CHECK(H <= 65535, "head_linear: %d heads in one launch", H);
   if (act_dtype == RA_BF16 && K % 8 == 0 && ldx % 8 == 0 && x_head % 8 == 0 && ((uintptr_t)x % 16) == 0 &&
       ((uintptr_t)W % 16) == 0) {
-    const int col_groups = (N + 63) / 64;
+    const int col_groups = (N + 63) / 64, tiles = (n_tokens + 63) / 64;
+    RA_CHECK(tiles <= 65535, "head_linear: %d tokens in one launch", n_tokens);
     // four columns of a result and of the gate in one access
     const bool whole = N % 4 == 0 && ldo % 4 == 0 && o_head % 4 == 0 && (uintptr_t)out % 8 == 0 &&
                        (gate == nullptr || gate_per_head || (ldg % 4 == 0 && (uintptr_t)gate % 8 == 0));
@@ -290,8 +291,6 @@ extern "C" int ra_head_linear(const void* x, int ldx, int x_head, const void* W,
                                                               (bf16_t*)out, ldo, o_head, (const bf16_t*)gate, ldg,
                                                               gate_per_head, n_tokens, N, K, whole);
     } else {
-      const int tiles = (n_tokens + 63) / 64;
-      RA_CHECK(tiles <= 65535, "head_linear: %d tokens in one launch", n_tokens);
       dim3 grid(col_groups, tiles, H);
       head_linear_mfma_kernel<4, 1><<<grid, 256, 0, stream>>>((const bf16_t*)x, ldx, x_head, (const bf16_t*)W,
                                                            (bf16_t*)out, ldo, o_head, (const bf16_t*)gate, ldg,
