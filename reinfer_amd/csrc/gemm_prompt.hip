@@ -442,72 +442,6 @@ int prompt_epilogue(const PromptArgs& g, int epilogue, hipStream_t stream) {
   }
 }
 
-// C[m] += alpha * (the ranges' planes, in order), and with norm_x the RMSNorm of the new row beside it. A row a workgroup, CH
-// chunks of 1024 columns; a plane's chunks are asked for together.
-template <int CH, typename TW>
-__global__ void __launch_bounds__(256) prompt_add_kernel(const float* __restrict__ planes, int ranges, float* __restrict__ C,
-                                                         int ldc, int M, int N, float alpha, const TW* __restrict__ norm_w,
-                                                         bf16_t* __restrict__ norm_x, int norm_ldx, float eps) {
-  __shared__ float red[17];
-  const int m = blockIdx.x;
-  f32x4_t v[CH], c[CH];
-#pragma unroll
-  for (int h = 0; h < CH; ++h) {
-    const int n = (h * 256 + threadIdx.x) * 4;
-    v[h] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-    c[h] = n < N ? *(const f32x4_t*)(C + (size_t)m * ldc + n) : v[h];
-  }
-#pragma unroll 2
-  for (int z = 0; z < ranges; ++z)
-#pragma unroll
-    for (int h = 0; h < CH; ++h) {
-      const int n = (h * 256 + threadIdx.x) * 4;
-      if (n < N) v[h] += *(const f32x4_t*)(planes + ((size_t)z * M + m) * N + n);
-    }
-  float ss = 0.f;
-#pragma unroll
-  for (int h = 0; h < CH; ++h) {
-    const int n = (h * 256 + threadIdx.x) * 4;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      c[h][i] = fmaf(alpha, v[h][i], c[h][i]);
-      ss += c[h][i] * c[h][i];
-    }
-    if (n < N) *(f32x4_t*)(C + (size_t)m * ldc + n) = c[h];
-  }
-  if (!norm_x) return;
-  const float rstd = rsqrtf(block_sum(ss, red) / (float)N + eps);
-#pragma unroll
-  for (int h = 0; h < CH; ++h) {
-    const int n = (h * 256 + threadIdx.x) * 4;
-    if (n >= N) continue;
-    bf16x4_t o;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) o[i] = (bf16_t)(c[h][i] * rstd * to_f32(norm_w[n + i]));
-    *(bf16x4_t*)(norm_x + (size_t)m * norm_ldx + n) = o;
-  }
-}
-
-template <typename TW>
-int prompt_add(const float* planes, int ranges, float* C, int ldc, int M, int N, float alpha, const void* norm_w, void* norm_x,
-               int norm_ldx, float eps, hipStream_t stream) {
-#define RA_PA(CH)                                                                                                            \
-  prompt_add_kernel<CH, TW><<<M, 256, 0, stream>>>(planes, ranges, C, ldc, M, N, alpha, (const TW*)norm_w, (bf16_t*)norm_x, \
-                                                   norm_ldx, eps)
-  if (N <= 2048) RA_PA(2);
-  else if (N <= 3072) RA_PA(3);
-  else if (N <= 4096) RA_PA(4);
-  else if (N <= 5120) RA_PA(5);
-  else if (N <= 8192) RA_PA(8);
-  else RA_PA(16);
-#undef RA_PA
-  RA_LAUNCH_CHECK("gemm_prompt add");
-  return 0;
-}
-
-// Bytes that a plane costs beside its product, in us: written with it, read by the adding kernel.
-float plane_cost(int M, int N) { return (float)M * N * 4.f / 4.5e6f; }
-
 }  // namespace
 
 // What a tile of `rows` x `cols` costs, measured on MI355X over products of 128 to 3000 rows (4096 to 25600 k, one to eight
@@ -624,60 +558,36 @@ int ra_prompt_experts(int rows, int cols, int kind, const void* a, long tokens, 
   return ra_fail("gemm_prompt: no tiles of %d x %d for experts", rows, cols);
 }
 
-// The K ranges of a product that adds into the stream (1: it adds in its epilogue), 1 for the others, 0 where the product is not
-// this kernel's. Up to 128 rows the weights' way from memory is the bound, and gemm_tile.hip's smaller stages are ahead. With a gate
-// it is ahead of the library and the gate's kernel from there on (160 rows of 24576 x 4096, weights from memory, 57 us against 60;
-// 512 rows of 19456 x 2560 60 / 65; 4096 rows of 24576 x 4096, the one size where it is not, 626 / 608). A plain product of up to
-// 512 rows, which the library cuts, is not (512 rows of 6144 x 4096 38 / 36; 700 rows of 6144 x 2560 29 / 31). One that adds into the
-// stream is priced beside the library's, whose time for weights from memory is its products at 1.45 PFLOP/s, 14 us and 2.5 ns a k,
-// within a tenth over 20 shapes of 600 to 3000 rows: 1024 rows of 2560 x 9728 in three ranges, with the adding kernel, 64 us against
-// 85, 1733 rows of 4096 x 12288 149 / 173, 2048 rows of 2560 x 4096 uncut 50 / 53, 3000 rows of 4096 x 4096 88 / 90. Above 3072 rows
-// the library multiplies without adding, which it does faster (4096 rows of 4096 x 4096 95 us; adding 117, here 121).
-extern "C" int ra_gemm_prompt_ranges(int epilogue, int M, int N, int K) {
+// Whether a product is this kernel's. Up to 128 rows the weights' way from memory is the bound, and gemm_tile.hip's smaller stages
+// are ahead. With a gate it is ahead of the library and the gate's kernel from there on (160 rows of 24576 x 4096, weights from
+// memory, 57 us against 60; 512 rows of 19456 x 2560 60 / 65; 4096 rows of 24576 x 4096, the one size where it is not, 626 / 608). A
+// plain product of up to 512 rows is not (512 rows of 6144 x 4096 38 / 36; 700 rows of 6144 x 2560 29 / 31). One that adds into
+// the stream is priced beside the library's, whose time for weights from memory is its products at 1.45 PFLOP/s, 14 us and 2.5 ns a
+// k, within a tenth over 20 shapes of 600 to 3000 rows: 2048 rows of 2560 x 4096 50 / 53, 3000 rows of 4096 x 4096 88 / 90. Above 3072
+// rows the library multiplies without adding, which it does faster (4096 rows of 4096 x 4096 95 us; adding 117, here 121).
+// K stays whole, though two to six ranges would be ahead up to 1500 rows (1024 rows of 2560 x 9728 64 us against 85 in the library):
+// a row's sums then do not depend on how many rows share the call, so that a prompt gives the same bits alone and among others.
+extern "C" int ra_gemm_prompt_takes(int epilogue, int M, int N, int K) {
   if (M <= 128 || !ra_prompt_shape(N, K) || (size_t)N * K < (4u << 20)) return 0;
   if (epilogue == GP_GATED) return 1;
   if (epilogue == GP_PLAIN) return M > 512;
-  if (epilogue != GP_ADD || M <= 256 || M > 3072 || N > 16384) return 0;
-  // the uncut product reads and writes the stream at its end; the cut one's adding kernel reads the planes, reads and writes the
-  // stream and saves the norm kernel's launch and reading; the library's
-  const float plane = plane_cost(M, N);
-  const RaPromptPlan one = ra_prompt_plan(M, N, K, 1, 1, 0.f), cut = ra_prompt_plan(M, N, K, 2, 16, plane);
-  const float whole = one.us + plane, parts = cut.us + plane - 3.f;
-  const float library = (float)((double)M * N * K * 2.0 / 1.45e9) + 14.f + 0.0025f * K;
-  if ((whole < parts ? whole : parts) > library) return 0;
-  return whole <= parts ? 1 : cut.ranges;
+  if (epilogue != GP_ADD || M <= 256 || M > 3072) return 0;
+  const float adding = (float)M * N * 4.f / 4.5e6f;        // the stream read and written at the end
+  return ra_prompt_plan(M, N, K, 1, 1, 0.f).us + adding <= (float)((double)M * N * K * 2.0 / 1.45e9) + 14.f + 0.0025f * K;
 }
 
-// bfloat16, many rows (ra_gemm_prompt_ranges): epilogue 0 C = A . W^T in bfloat16; 1 bfloat16 silu(gate) * up; 2 float C += alpha *
-// (A . W^T); 3 float C = A . W^T. A cut product needs ranges * M * N floats of scratch and may finish the RMSNorm that follows:
-// norm_x = bf16(C * rsqrt(mean(C^2) + eps) * norm_w). tile_rows 0: the plan's own choice.
+// bfloat16, many rows (ra_gemm_prompt_takes): epilogue 0 C = A . W^T in bfloat16; 1 bfloat16 silu(gate) * up; 2 float C += alpha *
+// (A . W^T); 3 float C = A . W^T, or with more than one range C[ranges][M][N]. tile_rows 0: the plan's own choice.
 extern "C" int ra_gemm_prompt(const void* A, const void* W, void* C, int epilogue, int M, int N, int K, int lda, int ldc,
-                              float alpha, float* scratch, long scratch_floats, const void* norm_w, int norm_w_dtype,
-                              void* norm_x, int norm_ldx, float norm_eps, int tile_rows, int tile_cols, int ranges,
-                              hipStream_t stream) {
+                              float alpha, int tile_rows, int tile_cols, int ranges, hipStream_t stream) {
   RA_CHECK(epilogue >= 0 && epilogue <= 3, "gemm_prompt: epilogue %d", epilogue);
   RA_CHECK(M > 0 && ra_prompt_shape(N, K), "gemm_prompt: a product of [%d, %d, %d]", M, N, K);
-  if (ranges < 1) ranges = epilogue == GP_ADD ? ra_gemm_prompt_ranges(epilogue, M, N, K) : 1;
-  if (ranges < 1) ranges = 1;
-  RA_CHECK(ranges == 1 || epilogue == GP_ADD, "gemm_prompt: only a product that adds is cut (%d ranges)", ranges);
+  RA_CHECK(ranges >= 1, "gemm_prompt: %d ranges", ranges);
   RaPromptPlan plan = ra_prompt_plan(M, N, K, ranges, ranges, 0.f);
+  RA_CHECK(plan.ranges == ranges, "gemm_prompt: K of %d does not cut into %d ranges", K, ranges);
   if (tile_rows) {
     plan.rows = tile_rows;
     plan.cols = tile_cols;
   }
-  RA_CHECK(plan.ranges == ranges, "gemm_prompt: K of %d does not cut into %d ranges", K, ranges);
-  if (ranges == 1) {
-    RA_CHECK(!norm_x, "gemm_prompt: only a cut product finishes a norm");
-    return ra_prompt_product(plan, epilogue, A, W, C, M, N, K, lda, ldc, alpha, stream);
-  }
-  RA_CHECK(scratch && scratch_floats >= (long)ranges * M * N && (uintptr_t)scratch % 16 == 0 && N <= 16384 && ldc % 4 == 0 &&
-               ldc >= N && (uintptr_t)C % 16 == 0,
-           "gemm_prompt: %d ranges of [%d, %d] need %ld floats, got %ld", ranges, M, N, (long)ranges * M * N, scratch_floats);
-  RA_CHECK(!norm_x || (norm_w && norm_ldx >= N && norm_ldx % 4 == 0 && (uintptr_t)norm_x % 8 == 0 &&
-                       (norm_w_dtype == RA_F32 || norm_w_dtype == RA_BF16)),
-           "gemm_prompt: the norm that follows takes a weight and rows of %d", N);
-  if (int rc = ra_prompt_product(plan, GP_FLOAT, A, W, scratch, M, N, K, lda, N, 1.f, stream)) return rc;
-  return norm_w_dtype == RA_F32
-             ? prompt_add<float>(scratch, ranges, (float*)C, ldc, M, N, alpha, norm_w, norm_x, norm_ldx, norm_eps, stream)
-             : prompt_add<bf16_t>(scratch, ranges, (float*)C, ldc, M, N, alpha, norm_w, norm_x, norm_ldx, norm_eps, stream);
+  return ra_prompt_product(plan, epilogue, A, W, C, M, N, K, lda, ldc, alpha, stream);
 }

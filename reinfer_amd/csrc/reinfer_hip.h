@@ -5,7 +5,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
-#define RA_ABI_VERSION 29
+#define RA_ABI_VERSION 30
 
 #ifdef __cplusplus
 extern "C" {
@@ -135,14 +135,12 @@ int ra_gemm_wide_normed(const void* A, const void* W, const void* bias, void* C,
                         int out_w_dtype, void* out_x, int out_ldx, float* out_ss, float out_eps,
                         hipStream_t stream);
 
-// bfloat16, more rows than the kernels above take, K a multiple of 64 and N of 16 (gemm_prompt.hip). ra_gemm_prompt_ranges: the K
-// ranges that a product is cut into (1: none; 0: not this kernel's). Epilogues 0 to 2 as above (2 with a factor on the product), 3
-// a float C = A . W^T; a cut product (epilogue 2) needs ranges * M * N floats of scratch, and with norm_x also writes
-// bf16(C_new * rsqrt(mean(C_new^2) + norm_eps) * norm_w). tile_rows, tile_cols and ranges 0: the library's own choice.
-int ra_gemm_prompt_ranges(int epilogue, int M, int N, int K);
+// bfloat16, more rows than the kernels above take, K a multiple of 64 and N of 16 (gemm_prompt.hip). ra_gemm_prompt_takes: whether
+// the product is this kernel's. Epilogues 0 to 2 as above (2 with a factor on the product), 3 a float C = A . W^T, whose K ranges, if
+// more than one, get a plane C[ranges][M][N] each. tile_rows and tile_cols 0: the library's own choice.
+int ra_gemm_prompt_takes(int epilogue, int M, int N, int K);
 int ra_gemm_prompt(const void* A, const void* W, void* C, int epilogue, int M, int N, int K, int lda, int ldc, float alpha,
-                   float* scratch, long scratch_floats, const void* norm_w, int norm_w_dtype, void* norm_x, int norm_ldx,
-                   float norm_eps, int tile_rows, int tile_cols, int ranges, hipStream_t stream);
+                   int tile_rows, int tile_cols, int ranges, hipStream_t stream);
 
 // The cache of a layer: K and V are [blocks][Hkv][block_size * d], every (block, KV head) slab
 // in tiles of 16 slots laid out in MFMA operand order (cache_k_index, cache_v_index in common.h);

@@ -15,7 +15,7 @@ import torch  # noqa: F401  (loads the HIP runtime the library links against)
 
 from ..csrc import build as _build
 
-ABI_VERSION = 29
+ABI_VERSION = 30
 
 
 class KernelLibraryError(RuntimeError):
@@ -44,7 +44,7 @@ _SIGNATURES = {
     "ra_gemm_wide_normed": [P, P, P, P, I, I, I, I, I, I, I, P, c_long, P, I, F, I, P, I, P, I, P, F, P],
     "ra_gemm_skinny_normed": [P, P, P, P, I, I, I, I, I, I, I, P, I, F, I, P, I, P, I, P, P],
     "ra_gemm_skinny_scaled": [P, P, P, I, I, I, I, I, F, P],
-    "ra_gemm_prompt": [P, P, P, I, I, I, I, I, I, F, P, c_long, P, I, P, I, F, I, I, I, P],
+    "ra_gemm_prompt": [P, P, P, I, I, I, I, I, I, F, I, I, I, P],
     "ra_gemm_wide_scaled": [P, P, P, I, I, I, I, I, P, c_long, F, P],
     "ra_gemm_plain": [P, P, P, P, I, I, I, I, I, I, I, P],
     "ra_moe_grouped": [P, I, P, P, I, P, P, I, I, I, I, I, I, I, P, P, I, P, P, F, P, c_long, P],
@@ -159,8 +159,8 @@ def load() -> ctypes.CDLL:
         lib.ra_gemm_wide_ranges.argtypes = [c_int, c_int, c_int]
         lib.ra_gemm_tile_takes.restype = c_int
         lib.ra_gemm_tile_takes.argtypes = [c_int, c_int, c_int, c_int]
-        lib.ra_gemm_prompt_ranges.restype = c_int
-        lib.ra_gemm_prompt_ranges.argtypes = [c_int, c_int, c_int, c_int]
+        lib.ra_gemm_prompt_takes.restype = c_int
+        lib.ra_gemm_prompt_takes.argtypes = [c_int, c_int, c_int, c_int]
         lib.ra_gemm_wide_preferred.restype = c_int
         lib.ra_gemm_wide_preferred.argtypes = [c_int, c_int, c_int, c_int]
         if lib.ra_abi_version() != ABI_VERSION:

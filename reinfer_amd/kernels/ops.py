@@ -703,7 +703,7 @@ class HipKernels:
 
         bfloat16 with up to 64 rows: the weight-streaming MFMA kernel; with up to
         512 rows the tiled one where it is ahead, with more the product of many rows
-        (``ra_gemm_prompt_ranges``). A bfloat16 result that these do not take (a bias, K in no steps
+        (``ra_gemm_prompt_takes``). A bfloat16 result that these do not take (a bias, K in no steps
         of 64): the library product (hipBLASLt through torch), as the reference calls cuBLAS for its
         prompt products (crates/cuda/src/gemm.rs:226-292). bfloat16 with more rows and a float
         result (the head's logits for more than 64 wanted rows): the library
@@ -720,7 +720,7 @@ class HipKernels:
             if self._tile_takes(0, x, weight, out):
                 self._check_linear(x, weight, out, bias)
                 return self._few_rows("linear output", x, weight, bias, out, 0, M, weight.shape[0], K, True)
-            if bias is None and out.dtype == torch.bfloat16 and self._prompt_ranges(0, x, weight, out):
+            if bias is None and out.dtype == torch.bfloat16 and self._prompt_takes(0, x, weight, out):
                 self._check_linear(x, weight, out, bias)
                 return self._prompt(0, x, weight, out)
             if out.dtype == torch.bfloat16 and x.is_cuda:
@@ -775,27 +775,21 @@ class HipKernels:
             and bool(library.load().ra_gemm_tile_takes(epilogue, M, N, K))
 
     @classmethod
-    def _prompt_ranges(cls, epilogue: int, x, weight, out) -> int:
-        """The K ranges in which the product of many rows takes this one (epilogues as ``ra_gemm_prompt``), 0 where it is the
-        library's or its rows cannot be read and written in whole 16-byte pieces."""
+    def _prompt_takes(cls, epilogue: int, x, weight, out) -> bool:
+        """True where the product of many rows takes this one (epilogues as ``ra_gemm_prompt``): where it is ahead of the
+        library's and its rows can be read and written in whole 16-byte pieces."""
         M, K = x.shape
-        if not (M > 128 and x.is_cuda and x.dtype == weight.dtype == torch.bfloat16 and x.stride(1) == 1 and x.stride(0) % 8 == 0
-                and K <= x.stride(0) < cls.TILE_ROW_STRIDE and weight.is_contiguous() and out.stride(1) == 1
-                and out.stride(0) % 8 == 0 and out.shape[1] <= out.stride(0) < cls.TILE_ROW_STRIDE
-                and all(t.data_ptr() % 16 == 0 for t in (x, weight, out))):
-            return 0
-        return int(library.load().ra_gemm_prompt_ranges(epilogue, M, weight.shape[0], K))
+        return M > 128 and x.is_cuda and x.dtype == weight.dtype == torch.bfloat16 and x.stride(1) == 1 and x.stride(0) % 8 == 0 \
+            and K <= x.stride(0) < cls.TILE_ROW_STRIDE and weight.is_contiguous() and out.stride(1) == 1 \
+            and out.stride(0) % 8 == 0 and out.shape[1] <= out.stride(0) < cls.TILE_ROW_STRIDE \
+            and all(t.data_ptr() % 16 == 0 for t in (x, weight, out)) \
+            and bool(library.load().ra_gemm_prompt_takes(epilogue, M, weight.shape[0], K))
 
     @staticmethod
-    def _prompt(epilogue: int, x, weight, out, alpha: float = 1.0, ranges: int = 1, finish=None, tile=(0, 0)) -> None:
+    def _prompt(epilogue: int, x, weight, out, alpha: float = 1.0, tile=(0, 0), ranges: int = 1) -> None:
         M, K = x.shape
-        N = weight.shape[0]
-        need = ranges * M * N if ranges > 1 else 0
-        scratch = torch.empty(need, dtype=torch.float32, device=x.device) if need else None
-        w, xo, eps = finish if finish is not None else (None, None, 0.0)
-        library.call("ra_gemm_prompt", x.data_ptr(), weight.data_ptr(), out.data_ptr(), epilogue, M, N, K, x.stride(0),
-                     out.stride(0), float(alpha), _ptr(scratch), need, _ptr(w), _tag(w, "norm weight") if w is not None else 0,
-                     _ptr(xo), xo.stride(0) if xo is not None else 0, float(eps), tile[0], tile[1], ranges, _stream())
+        library.call("ra_gemm_prompt", x.data_ptr(), weight.data_ptr(), out.data_ptr(), epilogue, M, weight.shape[0], K, x.stride(0),
+                     out.stride(-2), float(alpha), tile[0], tile[1], ranges, _stream())
 
     @staticmethod
     def _check_linear(x, weight, out, bias):
@@ -850,10 +844,8 @@ class HipKernels:
                 raise ValueError("linear_skinny: a factor rides on a plain accumulating bfloat16 product only")
             lib = library.load()
             if M > 64 and not self._tile_takes(2, x, weight, out):
-                ranges = self._prompt_ranges(2, x, weight, out)
-                if ranges:
-                    self._prompt(2, x, weight, out, alpha, ranges)
-                    return None
+                if self._prompt_takes(2, x, weight, out):
+                    return self._prompt(2, x, weight, out, alpha)
                 torch.addmm(out, x, weight.t(), alpha=float(alpha), out_dtype=torch.float32, out=out)
                 return None
             if wide is None:
@@ -877,18 +869,10 @@ class HipKernels:
             if self.can_finish_norm(M, N, K):
                 w, xo, eps = finish
                 _dev(w, xo)
-                if M > self.NORM_FINISHED_FEW_ROWS:
-                    ranges = 0 if bias is not None or wide is not None else self._prompt_ranges(2, x, weight, out)
-                    if ranges < 2 or xo.stride(0) % 4 or xo.data_ptr() % 8:
-                        self.linear_skinny(x, weight, out, bias, accumulate=True, wide=wide)
-                        return False
                 if w.shape != (N,) or not w.is_contiguous() or xo.dtype != torch.bfloat16 or xo.shape != (M, N) \
                         or xo.stride(1) != 1:
                     raise ValueError(f"linear_skinny: norm weight {tuple(w.shape)}, finished rows {tuple(xo.shape)} "
                                      f"{xo.dtype}; expected [{N}] and bfloat16 [{M}, {N}]")
-                if M > self.NORM_FINISHED_FEW_ROWS:
-                    self._prompt(2, x, weight, out, 1.0, ranges, finish)
-                    return True
                 need = int(library.load().ra_gemm_wide_scratch(2, M, N, K, 1))
                 scratch = torch.empty(need, dtype=torch.float32, device=x.device)
                 library.call("ra_gemm_wide_normed", x.data_ptr(), weight.data_ptr(), _ptr(bias), out.data_ptr(),
@@ -901,9 +885,8 @@ class HipKernels:
         if accumulate and M > 64 and bias is None and row_sums is None and emit is None and wide is None:
             if self._tile_takes(2, x, weight, out):
                 return self._few_rows("linear output", x, weight, None, out, 2, M, N, K, True)
-            ranges = self._prompt_ranges(2, x, weight, out)
-            if ranges:
-                return self._prompt(2, x, weight, out, 1.0, ranges)
+            if self._prompt_takes(2, x, weight, out):
+                return self._prompt(2, x, weight, out)
             # the library's product, adding in place
             torch.addmm(out, x, weight.t(), out_dtype=torch.float32, out=out)
             return None
@@ -919,18 +902,14 @@ class HipKernels:
     NORM_ON_PRODUCTS_ROWS = 64
     NORM_SKINNY_ROWS = 16
     # Rows up to which the adding kernel of a product cut into K ranges can finish the norm that follows
-    # (a whole row a workgroup): the steps above the weight-streaming products' rows, whose other
-    # products apply no row factor. Up to the first number wherever a product is cut, above it where the product of many
-    # rows is (``ra_gemm_prompt_ranges``).
-    NORM_FINISHED_FEW_ROWS = 128
-    NORM_FINISHED_ROWS = 3072
+    # (a whole row a workgroup): the decode steps above the weight-streaming products' rows, whose other
+    # products can apply no row factor.
+    NORM_FINISHED_ROWS = 128
 
     def can_finish_norm(self, M: int, N: int, K: int) -> bool:
         """True where ``linear_skinny(..., accumulate=True, finish=)`` writes the finished norm: the rows
         between the two limits, a product that the tiled kernel takes at these rows, rows of up to
         16384 columns in steps of 8."""
-        if self.NORM_FINISHED_FEW_ROWS < M <= self.NORM_FINISHED_ROWS:
-            return int(library.load().ra_gemm_prompt_ranges(2, M, N, K)) > 1
         return self.NORM_ON_PRODUCTS_ROWS < M <= self.NORM_FINISHED_ROWS and N % 8 == 0 and N <= 16384 \
             and K % 8 == 0 and bool(library.load().ra_gemm_wide_preferred(2, M, N, K))
 
@@ -1061,7 +1040,7 @@ class HipKernels:
         if row_sums is None and wide is None and weight.dtype == out.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 \
                 and out.stride(0) % 4 == 0 and self._tile_takes(1, x, weight, out):
             return self._few_rows("linear output", x, weight, None, out, 1, M, 2 * I, K, True)
-        if row_sums is None and wide is None and out.dtype == torch.bfloat16 and self._prompt_ranges(1, x, weight, out):
+        if row_sums is None and wide is None and out.dtype == torch.bfloat16 and self._prompt_takes(1, x, weight, out):
             return self._prompt(1, x, weight, out)
         if row_sums is not None:
             raise ValueError("gated_linear: row sums ride on the weight-streaming product only (bfloat16, <= 64 rows)")
