@@ -4,6 +4,7 @@ architectures is in the spec and in the parts the spec names.
 """
 from __future__ import annotations
 
+import contextlib
 from typing import Dict, List, Optional, Sequence
 
 import torch
@@ -67,6 +68,8 @@ class DecoderModel:
         # tied: the embedding matrix is the head (crates/cpu/src/model.rs:218-225)
         self.head = self.embed if spec.tie_embeddings else weights[spec.head_name]
         self.run_order = spec.run_order
+        # a router between two nearly equal experts decides by a sum's last bits: see HipKernels.library_products
+        self.routes = any(getattr(p, "router", None) is not None for p in self.parts())
 
     def cache_needs(self) -> List[Optional[object]]:
         """What each run-order entry keeps: KVNeed, PagedNeed, StateNeed, or None. The block arrangement
@@ -119,6 +122,11 @@ class DecoderModel:
         ``observer(i, hidden)``, if given, is called with the float32 hidden state [T, hidden] behind
         the embedding (i = 0) and behind run-order entry i - 1 (the reference reads activations back
         layer by layer the same way, crates/cuda/src/engine.rs:3744-3765)."""
+        products = getattr(kernels.current(), "library_products", None) if self.routes else None
+        with products() if products is not None else contextlib.nullcontext():
+            return self._forward_layers(batch, caches, observer, input_states)
+
+    def _forward_layers(self, batch, caches, observer, input_states):
         ops = kernels.current()
         resid = torch.empty((batch.num_tokens, self.spec.hidden), dtype=torch.float32, device=self.device)
         if self.spec.embed_scale != 1.0:
