@@ -10,8 +10,9 @@ struct RaPromptPlan {
 
 // Whether the kernel takes products of this shape: whole steps of 64 k, four or more, and weight rows in runs of 16.
 static inline bool ra_prompt_shape(int N, int K) { return N >= 16 && N % 16 == 0 && K % 64 == 0 && K >= 256 && K <= (1 << 22); }
-// The tile and ranges (from `least` to `most`) of the least expected time, plane_us for each range's float plane among it.
-RaPromptPlan ra_prompt_plan(int M, int N, int K, int least, int most, float plane_us);
+// The tile of the least expected time for a product in ranges of range_k (a multiple of 64) k; no ranges where the last one would
+// have fewer steps than the kernel's least.
+RaPromptPlan ra_prompt_plan(int M, int N, int K, int range_k);
 // C = A . W^T: epilogue 0 bfloat16, 1 bfloat16 silu(gate) * up over weight rows interleaved in runs of 8, 2 C += alpha * (float),
 // 3 float, with more than one range a plane [M, N] for each
 int ra_prompt_product(const RaPromptPlan& plan, int epilogue, const void* A, const void* W, void* C, int M, int N, int K, int lda,

@@ -448,41 +448,36 @@ int prompt_epilogue(const PromptArgs& g, int epilogue, hipStream_t stream) {
 // ranges; the tile so chosen is within 4 % of the fastest at each of 23 shapes): a start, then for each round of workgroups an
 // end that grows with the tile and the steps, each a part of its own (barrier, first operands) and one that grows with the tile,
 // the more the fuller the chip is (power and fetches).
-static RaPromptPlan prompt_plan(int M, int N, int K, int least, int most, float plane_us, int slots) {
+static RaPromptPlan prompt_plan(int M, int N, int K, int range_k, int slots) {
   static const int sides[10][2] = {{256, 256}, {224, 256}, {192, 256}, {160, 256}, {128, 256},
                                    {256, 128}, {224, 128}, {192, 128}, {160, 128}, {128, 128}};
   RaPromptPlan best = {0, 0, 0, 0, 1e30f};
-  const int steps = K / GP_BK;
-  for (const auto& side : sides)
-    for (int s = least; s <= most; ++s) {
-      const int each = (steps + s - 1) / s;
-      if ((long)(s - 1) * each + GP_STEPS > steps) break;
-      const long tiles = (long)((M + side[0] - 1) / side[0]) * ((N + side[1] - 1) / side[1]) * s;
-      const long rounds = ((tiles + RA_XCDS - 1) / RA_XCDS + slots - 1) / slots;
-      const float fill = (float)tiles / (float)(rounds * slots * RA_XCDS), area = (float)side[0] * side[1] / 65536.f;
-      const float us = 6.f + rounds * (11.2f * area + each * (0.227f + 0.623f * area + fill * (0.027f + 0.282f * area))) +
-                       s * plane_us;
-      if (us < best.us) best = {side[0], side[1], s, each * GP_BK, us};
-    }
+  const int steps = K / GP_BK, each = range_k / GP_BK, ranges = (steps + each - 1) / each;
+  if (steps - (ranges - 1) * each < GP_STEPS) return best;
+  for (const auto& side : sides) {
+    const long tiles = (long)((M + side[0] - 1) / side[0]) * ((N + side[1] - 1) / side[1]) * ranges;
+    const long rounds = ((tiles + RA_XCDS - 1) / RA_XCDS + slots - 1) / slots;
+    const float fill = (float)tiles / (float)(rounds * slots * RA_XCDS), area = (float)side[0] * side[1] / 65536.f;
+    const float us = 6.f + rounds * (11.2f * area + each * (0.227f + 0.623f * area + fill * (0.027f + 0.282f * area)));
+    if (us < best.us) best = {side[0], side[1], ranges, range_k, us};
+  }
   return best;
 }
 
-// A step asks for the same few plans layer after layer, several times a product (which kernel, how much scratch, the launch), and
-// a plan is up to 150 prices: a thread keeps those of the last shapes, 0.1 us instead of 2 (a prompt of 97 rows through 8 layers
-// lasts 1.3 ms).
-RaPromptPlan ra_prompt_plan(int M, int N, int K, int least, int most, float plane_us) {
+// A step asks for the same few plans layer after layer, twice a product (which kernel, the launch): a thread keeps those of the
+// last shapes.
+RaPromptPlan ra_prompt_plan(int M, int N, int K, int range_k) {
   struct Kept {
-    int M, N, K, least, most, slots;
-    float plane_us;
+    int M, N, K, range_k, slots;
     RaPromptPlan plan;
   };
   static thread_local Kept kept[64];
   const int slots = ra_cu_count() / RA_XCDS;
   const unsigned h = (unsigned)M * 2654435761u ^ (unsigned)N * 2246822519u ^ (unsigned)K * 3266489917u ^
-                     (unsigned)(least * 31 + most) * 668265263u;
+                     (unsigned)range_k * 668265263u;
   Kept& k = kept[h >> 26];
-  if (k.M != M || k.N != N || k.K != K || k.least != least || k.most != most || k.slots != slots || k.plane_us != plane_us)
-    k = {M, N, K, least, most, slots, plane_us, prompt_plan(M, N, K, least, most, plane_us, slots)};
+  if (k.M != M || k.N != N || k.K != K || k.range_k != range_k || k.slots != slots)
+    k = {M, N, K, range_k, slots, prompt_plan(M, N, K, range_k, slots)};
   return k.plan;
 }
 
@@ -573,7 +568,7 @@ extern "C" int ra_gemm_prompt_takes(int epilogue, int M, int N, int K) {
   if (epilogue == GP_PLAIN) return M > 512;
   if (epilogue != GP_ADD || M <= 256 || M > 3072) return 0;
   const float adding = (float)M * N * 4.f / 4.5e6f;        // the stream read and written at the end
-  return ra_prompt_plan(M, N, K, 1, 1, 0.f).us + adding <= (float)((double)M * N * K * 2.0 / 1.45e9) + 14.f + 0.0025f * K;
+  return ra_prompt_plan(M, N, K, K).us + adding <= (float)((double)M * N * K * 2.0 / 1.45e9) + 14.f + 0.0025f * K;
 }
 
 // bfloat16, many rows (ra_gemm_prompt_takes): epilogue 0 C = A . W^T in bfloat16; 1 bfloat16 silu(gate) * up; 2 float C += alpha *
@@ -583,7 +578,7 @@ extern "C" int ra_gemm_prompt(const void* A, const void* W, void* C, int epilogu
   RA_CHECK(epilogue >= 0 && epilogue <= 3, "gemm_prompt: epilogue %d", epilogue);
   RA_CHECK(M > 0 && ra_prompt_shape(N, K), "gemm_prompt: a product of [%d, %d, %d]", M, N, K);
   RA_CHECK(ranges >= 1, "gemm_prompt: %d ranges", ranges);
-  RaPromptPlan plan = ra_prompt_plan(M, N, K, ranges, ranges, 0.f);
+  RaPromptPlan plan = ra_prompt_plan(M, N, K, (K / GP_BK + ranges - 1) / ranges * GP_BK);
   RA_CHECK(plan.ranges == ranges, "gemm_prompt: K of %d does not cut into %d ranges", K, ranges);
   if (tile_rows) {
     plan.rows = tile_rows;

@@ -16,8 +16,10 @@
 // 203 tiles of 96 features 31.2 us, 152 of 128 34.5).
 //
 // With the adding kernel, 6144 x 4096 / 4096 x 4096 / 4096 x 12288, the library's product in brackets: 97 rows
-// 19 / 16 / 29 us (23 / 18 / 41), 128 rows 20 / 18 / 31 (26 / 24 / 66), 192 rows 29 / 21 / 43 (34 / 33 / 90), 256 rows
-// 31 / 23 / 45 (40 / 22 / 53). 24576 x 4096 with its gate at 97 rows 48 (54 with the gate's kernel).
+// 19 / 16 / 29 us (23 / 18 / 41), 128 rows 20 / 18 / 31 (26 / 24 / 66). 24576 x 4096 with its gate at 97 rows 48 (54 with the
+// gate's kernel). Above 128 rows these ranges run on gemm_prompt.hip's tiles where its shapes allow: 160 rows 24 / 19 / 36 us
+// (28 / 21 / 40 here; library 28 / 27 / 76), 193 rows 26 / 21 / 39 (28 / 22 / 41; 25 / 22 / 54), 256 rows 30 / 23 / 44
+// (30 / 24 / 45; 40 / 23 / 58).
 #include "common.h"
 #include "reinfer_hip.h"
 #include "gemm_tile.h"
@@ -188,24 +190,17 @@ int tile_launch(TileArgs g, hipStream_t stream) {
 static long tile_count(int M, int N) { return (long)((M + GT_SIDE - 1) / GT_SIDE) * ((N + GT_SIDE - 1) / GT_SIDE); }
 
 // As many K ranges as fill the chip once, of at least 512 k (shorter ones are all start and end), at most 16 (each is a float
-// plane to write and read again).
-static void tile_plan(int M, int N, int K, int* ranges, int* range_k) {
+// plane to write and read again). They follow from N, K and the rows of tiles alone, so that a row has the same sums at any of 129
+// to 256 rows (to 384, to 512). Ranges of the exact number of rows, which gemm_prompt.hip's tiles could have, would be faster (the two
+// at 5120 x 25600 with 160 rows 92 / 70 us, with 384 139 / 114, 4096 x 12288 with 512 74 / 63, most shapes within 5 %), but then one
+// more request in a step changes every row's last bits.
+void ra_tile_plan(int M, int N, int K, int* ranges, int* range_k) {
   long s = ra_cu_count() / tile_count(M, N);
   if (s > K / 512) s = K / 512;
   if (s > 16) s = 16;
   if (s < 1) s = 1;
   *range_k = ((K + (int)s - 1) / (int)s + GT_BK - 1) / GT_BK * GT_BK;
   *ranges = (K + *range_k - 1) / *range_k;
-}
-
-// The ranges of a product: above one row of tiles those of gemm_prompt.hip's, where its shape allows them (weights from memory,
-// with the adding kernel, these tiles / those: 160 rows of 6144 x 4096 32 / 25 us, 4096 x 12288 43 / 37; 300 rows 72 / 50; 256 rows
-// of 2560 x 9728 32.2 / 31.6; but 128 rows of 2560 x 4096 18.9 / 20.4, and of 24576 x 4096 with its gate 51 / 54).
-void ra_tile_plan(int M, int N, int K, int* ranges, int* range_k) {
-  const RaPromptPlan p = M > GT_SIDE && ra_prompt_shape(N, K) ? ra_prompt_plan(M, N, K, 2, 16, (float)M * N * 4.f / 4.5e6f) : RaPromptPlan();
-  if (p.ranges < 2) return tile_plan(M, N, K, ranges, range_k);
-  *ranges = p.ranges;
-  *range_k = p.range_k;
 }
 
 // Products that are cut and whose ranges fill three quarters of the chip, or that are small (the library has too few tiles for
@@ -221,7 +216,7 @@ extern "C" int ra_gemm_tile_takes(int epilogue, int M, int N, int K) {
   const long cus = ra_cu_count(), tiles = tile_count(M, N);
   if (epilogue == 1) return M <= GT_SIDE && tiles <= cus && tiles * 2 > cus;
   int ranges, range_k;
-  tile_plan(M, N, K, &ranges, &range_k);
+  ra_tile_plan(M, N, K, &ranges, &range_k);
   if (ranges < 2) return 0;
   if (M > 256) return K >= 8192 && tiles * ranges * 4 > cus * 3;
   return (epilogue == 2 && M <= GT_SIDE) || tiles * 4 <= cus || tiles * ranges * 4 >= cus * 3;
@@ -239,9 +234,8 @@ int ra_tile_ranges(const void* A, int lda, const void* W, float* planes, int M, 
                    hipStream_t stream) {
   if (int rc = tile_check(A, lda, W, M, N, K)) return rc;
   if (M > GT_SIDE && ra_prompt_shape(N, K)) {
-    const RaPromptPlan p = ra_prompt_plan(M, N, K, ranges, ranges, 0.f);
-    if (p.ranges == ranges && p.range_k == range_k)
-      return ra_prompt_product(p, 3, A, W, planes, M, N, K, lda, N, 1.f, stream);
+    const RaPromptPlan p = ra_prompt_plan(M, N, K, range_k);
+    if (p.ranges == ranges) return ra_prompt_product(p, 3, A, W, planes, M, N, K, lda, N, 1.f, stream);
   }
   TileArgs g = tile_args(A, lda, W, M, N, K, ranges, range_k);
   g.c = planes;

@@ -162,3 +162,23 @@ def test_small_products_are_left_in_ranges(M, N, K):
 @pytest.mark.parametrize("kind", ["spread", "one", "identity"])
 def test_experts_in_whole_steps(T, E, top, ff, width, gated_kind, kind):
     grouped.test_experts_over_sorted_tokens(T, E, top, ff, width, gated_kind, kind)
+
+
+@pytest.mark.parametrize("N,K", [(2560, 9728), (4096, 4096), (4096, 12288), (5120, 8192), (5120, 25600)])
+def test_products_cut_into_ranges_have_one_order_of_sums_a_row_of_tiles(N, K):
+    """129 to 256 rows (and the rows of further 128) share their ranges: a row's sums do not depend on the rows beside it. What is
+    not cut at these rows is the library's, here in one chain."""
+    x, w, g = operands(512, N, K, N + K)
+    stream = torch.randn(512, N, device=DEV, generator=g)
+    wq = w[:, :4096].repeat(3, 1)[:6144].contiguous()
+    for sizes in [(129, 150, 160, 161, 193, 240, 256), (257, 300, 321, 384), (385, 448, 481, 482, 512)]:
+        if kernels.library.load().ra_gemm_tile_takes(2, sizes[-1], N, K):
+            outs = []
+            for M in sizes:
+                outs.append(stream[:M].clone())
+                ops().linear_skinny(x[:M], w, outs[-1], accumulate=True)
+            assert all(torch.equal(o[:sizes[0]], outs[0]) for o in outs)
+        parts = [ops().linear_ranges(x[:M, :4096], wq) for M in sizes]
+        assert len({p is None for p in parts}) == 1
+        if parts[0] is not None:
+            assert all(p.shape[0] == parts[0].shape[0] and torch.equal(p[:, :sizes[0]], parts[0]) for p in parts)
