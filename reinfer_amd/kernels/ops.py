@@ -156,13 +156,12 @@ class HipKernels:
             return None
         M, K = x.shape
         N = weight.shape[0]
-        if not (self.NORM_SKINNY_ROWS < M <= 512) or K % 8 or x.stride(1) != 1 or x.stride(0) % 8 \
-                or weight.shape != (N, K) or not weight.is_contiguous():
+        if not (self.NORM_SKINNY_ROWS < M <= 512) or K % 8 or x.stride(1) != 1 or x.stride(0) % 8 or x.stride(0) < K \
+                or weight.shape != (N, K) or not weight.is_contiguous() or x.data_ptr() % 16 or weight.data_ptr() % 16:
             return None
         lib = library.load()
         S = int(lib.ra_gemm_wide_ranges(M, N, K))
-        if S < 2 or M > 64 and not lib.ra_gemm_tile_takes(0, M, N, K) \
-                or M > 64 and (not K <= x.stride(0) < self.TILE_ROW_STRIDE or x.data_ptr() % 16 or weight.data_ptr() % 16):
+        if S < 2 or M > 64 and not (x.stride(0) < self.TILE_ROW_STRIDE and lib.ra_gemm_tile_takes(0, M, N, K)):
             return None
         parts = torch.empty((S, M, N), dtype=torch.float32, device=x.device)
         library.call("ra_gemm_wide_partial", x.data_ptr(), weight.data_ptr(), parts.data_ptr(), parts.numel(),

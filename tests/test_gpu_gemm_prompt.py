@@ -182,3 +182,17 @@ def test_products_cut_into_ranges_have_one_order_of_sums_a_row_of_tiles(N, K):
         assert len({p is None for p in parts}) == 1
         if parts[0] is not None:
             assert all(p.shape[0] == parts[0].shape[0] and torch.equal(p[:, :sizes[0]], parts[0]) for p in parts)
+
+
+@pytest.mark.parametrize("M", [17, 64, 129])
+def test_rows_off_16_bytes_are_not_left_in_ranges(M):
+    """They are declined, as any product that the range kernels cannot read: the caller then asks for the whole product."""
+    N, K = 6144, 4096
+    x, w, _ = operands(M, N, K, M)
+    buf = torch.empty(M * (K + 8) + 4, device=DEV, dtype=torch.bfloat16)[4:].view(M, K + 8)[:, :K]
+    buf.copy_(x)
+    wide = torch.empty(N * K + 4, device=DEV, dtype=torch.bfloat16)[4:].view(N, K)
+    wide.copy_(w)
+    same = x[:1].expand(M, K)                  # one row M times: a stride below K
+    assert ops().linear_ranges(x, w) is not None
+    assert all(ops().linear_ranges(a, b) is None for a, b in ((buf, w), (x, wide), (same, w)))
