@@ -146,12 +146,18 @@ class HipKernels:
                      num_kv_heads, head_dim, 1 if values_are_keys else 0, qkv.stride(0), _stream())
 
     # ---- the q/k/v product left in K ranges for the kernel that consumes it
+    # Weights (elements) from which 17 to 64 rows leave a product in ranges that would else go, whole, to the kernel whose waves split
+    # K. Both with the q/k norm, 17 / 32 / 64 rows, in ranges : whole: 4096 x 1024 10.9 / 11.3 / 13.7 : 8.3 / 8.6 / 12.3 us,
+    # 4096 x 2048 11.6 / 13.2 / 15.5 : 10.6 / 11.0 / 15.3, but 2560 x 4096 13.0 / 13.1 / 16.5 : 12.4 / 13.5 / 19.5,
+    # 5120 x 2048 12.5 / 12.7 / 16.8 : 13.8 / 14.9 / 21.7, 6144 x 2560 14.5 / 14.9 / 17.3 : 16.3 / 18.4 / 26.6.
+    RANGES_WEIGHTS = 10 << 20
+
     def linear_ranges(self, x: torch.Tensor, weight: torch.Tensor):
         """x . weight^T as the float results of the K ranges it was cut into, [ranges, M, N], not yet
         added, or None where that does not pay: only the products the split kernels take (bfloat16,
         17 to 64 rows, or 512 where the tiled one is ahead) and cut (few output features), whose adding
-        kernel a consumer can save by adding the ranges itself (``qk_norm_rope_cache(..., ranges=)``): 6144 x 2560
-        at 48 rows 11.9 us beside 11.9 and 4.7 added by a kernel of its own, or 19.4 by the kernel whose waves split K."""
+        kernel a consumer can save by adding the ranges itself (``qk_norm_rope_cache(..., ranges=)``).
+        Where the kernel whose waves split K would take the whole product, the ranges pay from RANGES_WEIGHTS on."""
         if not (x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.dim() == 2):
             return None
         M, K = x.shape
@@ -161,7 +167,8 @@ class HipKernels:
             return None
         lib = library.load()
         S = int(lib.ra_gemm_wide_ranges(M, N, K))
-        if S < 2 or M > 64 and not (x.stride(0) < self.TILE_ROW_STRIDE and lib.ra_gemm_tile_takes(0, M, N, K)):
+        if S < 2 or not (x.stride(0) < self.TILE_ROW_STRIDE and lib.ra_gemm_tile_takes(0, M, N, K) if M > 64 else
+                         N * K >= self.RANGES_WEIGHTS or lib.ra_gemm_wide_preferred(0, M, N, K)):
             return None
         parts = torch.empty((S, M, N), dtype=torch.float32, device=x.device)
         library.call("ra_gemm_wide_partial", x.data_ptr(), weight.data_ptr(), parts.data_ptr(), parts.numel(),

@@ -146,10 +146,14 @@ def test_what_it_refuses():
 
 
 @pytest.mark.parametrize("M", [17, 48, 64])
-@pytest.mark.parametrize("N,K", [(6144, 2560), (1536, 1024), (4099, 4096)])
+@pytest.mark.parametrize("N,K", [(6144, 2560), (1536, 1024), (4096, 2552), (5120, 2048), (4099, 4096)])
 def test_small_products_are_left_in_ranges(M, N, K):
+    """From 10 M weights on; below, where the kernel whose waves split K takes them, the whole product is the faster one."""
     x, w, _ = operands(M, N, K, M + N)
     parts = ops().linear_ranges(x, w)
+    if N * K < 10 << 20 and not kernels.library.load().ra_gemm_wide_preferred(0, M, N, K):
+        assert parts is None
+        return
     assert parts.shape[0] == kernels.library.load().ra_gemm_wide_ranges(M, N, K) >= 2
     assert ((parts.double().sum(0) - x.double() @ w.double().T).abs() <= bound(x, w, K)).all()
 
