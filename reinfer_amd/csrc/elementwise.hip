@@ -938,8 +938,8 @@ __global__ void silu_mul_kernel(const TA* __restrict__ gu, TA* __restrict__ out,
 }
 
 // eight outputs a thread, 16-byte loads and stores; I a multiple of 8, group 0 or a multiple of 8
-template <typename TA>
-__global__ void silu_mul_vec_kernel(const TA* __restrict__ gu, TA* __restrict__ out, int I, int group, size_t total8, int act,
+template <typename TA, typename TO>
+__global__ void silu_mul_vec_kernel(const TA* __restrict__ gu, TO* __restrict__ out, int I, int group, size_t total8, int act,
                                     float lim) {
   size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   const size_t stride = (size_t)gridDim.x * blockDim.x;
@@ -957,8 +957,8 @@ __global__ void silu_mul_vec_kernel(const TA* __restrict__ gu, TA* __restrict__ 
       g0[e] = gated_value(g0[e], u0[e], act, lim);
       g1[e] = gated_value(g1[e], u1[e], act, lim);
     }
-    Vec4<TA>::store(out + idx * 8, g0);
-    Vec4<TA>::store(out + idx * 8 + 4, g1);
+    Vec4<TO>::store(out + idx * 8, g0);
+    Vec4<TO>::store(out + idx * 8 + 4, g1);
   }
 }
 
@@ -987,9 +987,9 @@ extern "C" int ra_act_mul_bounded(const void* gate_up, void* out, int act_dtype,
     size_t vb = (total8 + 255) / 256;
     if (vb > 65535 * 4) vb = 65535 * 4;
     if (act_dtype == RA_F32)
-      silu_mul_vec_kernel<float><<<(unsigned)vb, 256, 0, stream>>>((const float*)gate_up, (float*)out, intermediate, group, total8, act, lim);
+      silu_mul_vec_kernel<float, float><<<(unsigned)vb, 256, 0, stream>>>((const float*)gate_up, (float*)out, intermediate, group, total8, act, lim);
     else
-      silu_mul_vec_kernel<bf16_t><<<(unsigned)vb, 256, 0, stream>>>((const bf16_t*)gate_up, (bf16_t*)out, intermediate, group, total8, act, lim);
+      silu_mul_vec_kernel<bf16_t, bf16_t><<<(unsigned)vb, 256, 0, stream>>>((const bf16_t*)gate_up, (bf16_t*)out, intermediate, group, total8, act, lim);
     RA_LAUNCH_CHECK("silu_mul");
     return 0;
   }
@@ -1002,5 +1002,18 @@ extern "C" int ra_act_mul_bounded(const void* gate_up, void* out, int act_dtype,
   else
     return ra_fail("silu_mul: unknown dtype tag %d", act_dtype);
   RA_LAUNCH_CHECK("silu_mul");
+  return 0;
+}
+
+// The gate over float products, rounded once, at the end: the bits of a product that applies its gate itself
+extern "C" int ra_silu_mul_rounded(const float* gate_up, void* out, int n_tokens, int intermediate, int group, hipStream_t stream) {
+  RA_CHECK(n_tokens > 0 && intermediate > 0 && intermediate % 8 == 0 && group >= 0 && group % 8 == 0 &&
+               (group == 0 || intermediate % group == 0) && (uintptr_t)gate_up % 16 == 0 && (uintptr_t)out % 16 == 0,
+           "silu_mul: %d rows of %d in runs of %d, in whole pieces", n_tokens, intermediate, group);
+  const size_t total8 = (size_t)n_tokens * intermediate / 8;
+  size_t blocks = (total8 + 255) / 256;
+  if (blocks > 65535 * 4) blocks = 65535 * 4;
+  silu_mul_vec_kernel<float, bf16_t><<<(unsigned)blocks, 256, 0, stream>>>(gate_up, (bf16_t*)out, intermediate, group, total8, 0, 0.f);
+  RA_LAUNCH_CHECK("silu_mul (rounded)");
   return 0;
 }

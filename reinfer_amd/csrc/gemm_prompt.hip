@@ -553,20 +553,30 @@ int ra_prompt_experts(int rows, int cols, int kind, const void* a, long tokens, 
   return ra_fail("gemm_prompt: no tiles of %d x %d for experts", rows, cols);
 }
 
-// Whether a product is this kernel's. Up to 128 rows the weights' way from memory is the bound, and gemm_tile.hip's smaller stages
-// are ahead. With a gate it is ahead of the library and the gate's kernel from there on (160 rows of 24576 x 4096, weights from
-// memory, 57 us against 60; 512 rows of 19456 x 2560 60 / 65; 4096 rows of 24576 x 4096, the one size where it is not, 626 / 608). A
-// plain product of up to 512 rows is not (512 rows of 6144 x 4096 38 / 36; 700 rows of 6144 x 2560 29 / 31). One that adds into
-// the stream is priced beside the library's, whose time for weights from memory is its products at 1.45 PFLOP/s, 14 us and 2.5 ns a
-// k, within a tenth over 20 shapes of 600 to 3000 rows: 2048 rows of 2560 x 4096 50 / 53, 3000 rows of 4096 x 4096 88 / 90. Above 3072
-// rows the library multiplies without adding, which it does faster (4096 rows of 4096 x 4096 95 us; adding 117, here 121).
+// Whether a product is this kernel's: 0 no, 1 yes, 2 it could be, but few of its tiles are there and the library's product in float
+// with the gate's kernel behind it is ahead. (us, here / library, weights from memory.)
+// Up to 128 rows the weights' way from memory is the bound, and gemm_tile.hip's smaller stages are ahead. With a gate it is ahead of
+// the library and the gate's kernel from there on (129 rows of 24576 x 4096 51 / 59, 512 of 19456 x 2560 57 / 62, 4096 of 24576 x 4096
+// 577 / 593), a plain product from 513 rows on (513 rows of 6144 x 4096 31 / 36; below, wide ones would be, 300 rows of 12288 x 4096
+// 45 / 52, most not, 512 rows of 6144 x 4096 38 / 36).
+// A workgroup walks all of K at 0.35 to 0.45 us a step however few there are, and the library has smaller tiles: where tiles of
+// 128 x 128 fill less than half of the chip, it is ahead with K above 2048 (gated 256 rows of 2048 x 4096 38 / 19, of 4096 x 2560
+// 30 / 20, 512 of 4096 x 4096 38 / 33, but 513, 160 tiles, 31 / 38, and 256 rows of 8192 x 2048 23 / 29, of 6144 x 1024 14 / 19),
+// a plain product, which has no gate's kernel to save, up to three quarters (513 rows of 1024 x 8192 52 / 29, of 2048 x 4096
+// 29 / 24, 768 of 4096 x 4096 38 / 33; 1800 of 2048 x 4096, 240 tiles, 32 / 36), and with a shorter K up to half (1024 rows of 2048 x
+// 2048 21 / 17; 1280, 160 tiles, 21 / 21, 513 of 4096 x 1024 11 / 15).
+// One that adds into the stream, of more than half of the chip's tiles (1024 rows of 2048 x 2048 24 / 18), is priced beside the
+// library's, whose time for weights from memory is its products at 1.45 PFLOP/s, 14 us and 2.5 ns a k, within a tenth over 20 shapes
+// of 600 to 3000 rows: 2048 rows of 2560 x 4096 50 / 53, 3000 rows of 4096 x 4096 88 / 90. Above 3072 rows the library multiplies
+// without adding, which it does faster (4096 rows of 4096 x 4096 95 us; adding 117, here 121).
 // K stays whole, though two to six ranges would be ahead up to 1500 rows (1024 rows of 2560 x 9728 64 us against 85 in the library):
 // a row's sums then do not depend on how many rows share the call, so that a prompt gives the same bits alone and among others.
 extern "C" int ra_gemm_prompt_takes(int epilogue, int M, int N, int K) {
   if (M <= 128 || !ra_prompt_shape(N, K) || (size_t)N * K < (4u << 20)) return 0;
-  if (epilogue == GP_GATED) return 1;
-  if (epilogue == GP_PLAIN) return M > 512;
-  if (epilogue != GP_ADD || M <= 256 || M > 3072) return 0;
+  const long cus = ra_cu_count(), tiles = (long)((M + 127) / 128) * ((N + 127) / 128);
+  if (epilogue == GP_GATED) return K > 2048 && tiles * 2 <= cus ? 2 : 1;
+  if (epilogue == GP_PLAIN) return M > 512 && (K > 2048 ? tiles * 4 > cus * 3 : tiles * 2 > cus);
+  if (epilogue != GP_ADD || M <= 256 || M > 3072 || tiles * 2 <= cus) return 0;
   const float adding = (float)M * N * 4.f / 4.5e6f;        // the stream read and written at the end
   return ra_prompt_plan(M, N, K, K).us + adding <= (float)((double)M * N * K * 2.0 / 1.45e9) + 14.f + 0.0025f * K;
 }

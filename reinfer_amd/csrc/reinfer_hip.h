@@ -5,7 +5,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
-#define RA_ABI_VERSION 30
+#define RA_ABI_VERSION 31
 
 #ifdef __cplusplus
 extern "C" {
@@ -46,6 +46,8 @@ int ra_qk_norm_rope_cache_sums(const float* parts, int n_ranges, const float* in
 // up interleaved in runs of `group` columns (gate run, then the up run of the same features)
 int ra_silu_mul(const void* gate_up, void* out, int act_dtype, int n_tokens, int intermediate,
                 int group, hipStream_t stream);
+// float gate_up, bfloat16 out, rounded once: widths and runs of whole 16-byte pieces
+int ra_silu_mul_rounded(const float* gate_up, void* out, int n_tokens, int intermediate, int group, hipStream_t stream);
 // out = act(gate) * up; act 0: silu, act 1: the tanh form of gelu
 int ra_act_mul(const void* gate_up, void* out, int act_dtype, int n_tokens, int intermediate, int group, int act,
                hipStream_t stream);
@@ -136,8 +138,9 @@ int ra_gemm_wide_normed(const void* A, const void* W, const void* bias, void* C,
                         hipStream_t stream);
 
 // bfloat16, more rows than the kernels above take, K a multiple of 64 and N of 16 (gemm_prompt.hip). ra_gemm_prompt_takes: whether
-// the product is this kernel's. Epilogues 0 to 2 as above (2 with a factor on the product), 3 a float C = A . W^T, whose K ranges, if
-// more than one, get a plane C[ranges][M][N] each. tile_rows and tile_cols 0: the library's own choice.
+// the product is this kernel's (2, of a gated one: the library's float product and ra_silu_mul_rounded are ahead). Epilogues 0 to 2 as
+// above (2 with a factor on the product), 3 a float C = A . W^T, whose K ranges, if more than one, get a plane C[ranges][M][N] each.
+// tile_rows and tile_cols 0: the library's own choice; set ones, epilogue 3 and ranges are for tests of the tiles by themselves.
 int ra_gemm_prompt_takes(int epilogue, int M, int N, int K);
 int ra_gemm_prompt(const void* A, const void* W, void* C, int epilogue, int M, int N, int K, int lda, int ldc, float alpha,
                    int tile_rows, int tile_cols, int ranges, hipStream_t stream);

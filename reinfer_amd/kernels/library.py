@@ -15,7 +15,7 @@ import torch  # noqa: F401  (loads the HIP runtime the library links against)
 
 from ..csrc import build as _build
 
-ABI_VERSION = 30
+ABI_VERSION = 31
 
 
 class KernelLibraryError(RuntimeError):
@@ -35,6 +35,7 @@ _SIGNATURES = {
     "ra_qk_norm_rope_cache_sums": [P, I, P, I, F, I, P, I, I, P, P, I, F, P, P, I, I, P, P, P, I, I, I, I, I, I, P],
     "ra_gemm_wide_partial": [P, P, P, c_long, I, I, I, I, P],
     "ra_silu_mul": [P, P, I, I, I, I, P],
+    "ra_silu_mul_rounded": [P, P, I, I, I, P],
     "ra_attention_plain": [P, I, P, I, P, P, I, P, I, P, P, P, I, I, I, I, I, F, I, P],
     "ra_attention_decode": [P, I, P, I, P, P, P, I, P, P, P, I, I, I, I, I, F, I, I, I, I, P, P, P],
     "ra_attention_prefill": [P, I, P, I, P, P, P, I, P, I, I, I, I, I, F, I, P],

@@ -801,15 +801,16 @@ class HipKernels:
             _scope.library = was
 
     @classmethod
-    def _prompt_takes(cls, epilogue: int, x, weight, out) -> bool:
-        """True where the product of many rows takes this one (epilogues as ``ra_gemm_prompt``): where it is ahead of the
-        library's and its rows can be read and written in whole 16-byte pieces."""
+    def _prompt_takes(cls, epilogue: int, x, weight, out) -> int:
+        """Not 0 where the product of many rows takes this one (epilogues as ``ra_gemm_prompt``): where it is ahead of the
+        library's and its rows can be read and written in whole 16-byte pieces. 2 for a gated one of few tiles, where the
+        library's product in float and a gate's kernel that rounds once, the same sums, are ahead."""
         M, K = x.shape
-        return M > 128 and not getattr(_scope, "library", False) and x.is_cuda and x.dtype == weight.dtype == torch.bfloat16 \
+        return int(M > 128 and not getattr(_scope, "library", False) and x.is_cuda and x.dtype == weight.dtype == torch.bfloat16 \
             and x.stride(1) == 1 and x.stride(0) % 8 == 0 and K <= x.stride(0) < cls.TILE_ROW_STRIDE \
             and weight.is_contiguous() and out.stride(1) == 1 and out.stride(0) % 8 == 0 and out.shape[1] <= out.stride(0) < cls.TILE_ROW_STRIDE \
             and all(t.data_ptr() % 16 == 0 for t in (x, weight, out)) \
-            and bool(library.load().ra_gemm_prompt_takes(epilogue, M, weight.shape[0], K))
+            and library.load().ra_gemm_prompt_takes(epilogue, M, weight.shape[0], K))
 
     @staticmethod
     def _prompt(epilogue: int, x, weight, out, alpha: float = 1.0, tile=(0, 0), ranges: int = 1) -> None:
@@ -1066,8 +1067,15 @@ class HipKernels:
         if row_sums is None and wide is None and weight.dtype == out.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 \
                 and out.stride(0) % 4 == 0 and self._tile_takes(1, x, weight, out):
             return self._few_rows("linear output", x, weight, None, out, 1, M, 2 * I, K, True)
-        if row_sums is None and wide is None and out.dtype == torch.bfloat16 and self._prompt_takes(1, x, weight, out):
-            return self._prompt(1, x, weight, out)
+        if row_sums is None and wide is None and out.dtype == torch.bfloat16:
+            takes = self._prompt_takes(1, x, weight, out)
+            if takes == 2 and out.is_contiguous():
+                gu = torch.empty((M, 2 * I), dtype=torch.float32, device=x.device)
+                torch.mm(x, weight.t(), out_dtype=torch.float32, out=gu)
+                library.call("ra_silu_mul_rounded", gu.data_ptr(), out.data_ptr(), M, I, self.GATE_GROUP, _stream())
+                return
+            if takes:
+                return self._prompt(1, x, weight, out)
         if row_sums is not None:
             raise ValueError("gated_linear: row sums ride on the weight-streaming product only (bfloat16, <= 64 rows)")
         gu = torch.empty((M, 2 * I), dtype=out.dtype, device=x.device)

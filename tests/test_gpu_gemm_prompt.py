@@ -200,3 +200,35 @@ def test_rows_off_16_bytes_are_not_left_in_ranges(M):
     same = x[:1].expand(M, K)                  # one row M times: a stride below K
     assert ops().linear_ranges(x, w) is not None
     assert all(ops().linear_ranges(a, b) is None for a, b in ((buf, w), (x, wide), (same, w)))
+
+
+# both sides of every line of the rule: half of the chip's 256 CUs in tiles of 128 x 128, three quarters for plain products of a long K
+@pytest.mark.parametrize("epilogue,M,N,K,own", [
+    (1, 129, 2048, 4096, False), (1, 512, 4096, 2560, False), (1, 513, 4096, 2560, True), (1, 256, 8192, 2048, True),
+    (0, 768, 4096, 4096, False), (0, 769, 4096, 4096, True), (0, 513, 1024, 8192, False), (0, 1024, 2048, 2048, False),
+    (0, 1025, 2048, 2048, True), (2, 1024, 2048, 2560, False), (2, 3072, 2048, 4096, True)])
+def test_few_tiles_are_the_library_s(epilogue, M, N, K, own, monkeypatch):
+    x, w, g = operands(M, N, K, M + N)
+    ref, err = x.double() @ w.double().T, bound(x, w, K)
+    calls, call = [], kernels.library.call
+    monkeypatch.setattr(kernels.library, "call", lambda name, *a: (calls.append(name), call(name, *a))[1])
+    if epilogue == 0:
+        out = torch.full((M, N), float("nan"), device=DEV, dtype=torch.bfloat16)
+        ops().linear(x, w, out)
+        assert ((out.double() - ref).abs() <= err + ref.abs() * 2 ** -8).all()
+    elif epilogue == 2:
+        stream = torch.randn(M, N, device=DEV, generator=g)
+        want = stream.double() + ref
+        ops().linear_skinny(x, w, stream, accumulate=True)
+        assert ((stream.double() - want).abs() <= err + want.abs() * 2 ** -23).all()
+    else:
+        want, tol = gated(ref, err)                     # neither way rounds gate and up
+        for pad in (0, 8):
+            buf = torch.full((M + 1, N // 2 + pad), float("nan"), device=DEV, dtype=torch.bfloat16)
+            ops().gated_linear(x, w, buf[:M, :N // 2])
+            assert ((buf[:M, :N // 2].double() - want).abs() <= tol).all()
+            assert torch.isnan(buf[M]).all() and torch.isnan(buf[:, N // 2:]).all()
+            if pad == 0:
+                assert ("ra_silu_mul_rounded" in calls) != own
+        return
+    assert ("ra_gemm_prompt" in calls) == own
