@@ -5,6 +5,7 @@
 struct RaPromptPlan {
   int rows, cols;                // of a tile
   int ranges, range_k;           // K ranges, and the k of each (the last may have fewer)
+  int rounds;                    // of workgroups
   float us;                      // what the product is expected to take
 };
 

@@ -451,7 +451,7 @@ int prompt_epilogue(const PromptArgs& g, int epilogue, hipStream_t stream) {
 static RaPromptPlan prompt_plan(int M, int N, int K, int range_k, int slots) {
   static const int sides[10][2] = {{256, 256}, {224, 256}, {192, 256}, {160, 256}, {128, 256},
                                    {256, 128}, {224, 128}, {192, 128}, {160, 128}, {128, 128}};
-  RaPromptPlan best = {0, 0, 0, 0, 1e30f};
+  RaPromptPlan best = {0, 0, 0, 0, 0, 1e30f};
   const int steps = K / GP_BK, each = range_k / GP_BK, ranges = (steps + each - 1) / each;
   if (steps - (ranges - 1) * each < GP_STEPS) return best;
   for (const auto& side : sides) {
@@ -459,7 +459,7 @@ static RaPromptPlan prompt_plan(int M, int N, int K, int range_k, int slots) {
     const long rounds = ((tiles + RA_XCDS - 1) / RA_XCDS + slots - 1) / slots;
     const float fill = (float)tiles / (float)(rounds * slots * RA_XCDS), area = (float)side[0] * side[1] / 65536.f;
     const float us = 6.f + rounds * (11.2f * area + each * (0.227f + 0.623f * area + fill * (0.027f + 0.282f * area)));
-    if (us < best.us) best = {side[0], side[1], ranges, range_k, us};
+    if (us < best.us) best = {side[0], side[1], ranges, range_k, (int)rounds, us};
   }
   return best;
 }
@@ -565,20 +565,35 @@ int ra_prompt_experts(int rows, int cols, int kind, const void* a, long tokens, 
 // a plain product, which has no gate's kernel to save, up to three quarters (513 rows of 1024 x 8192 52 / 29, of 2048 x 4096
 // 29 / 24, 768 of 4096 x 4096 38 / 33; 1800 of 2048 x 4096, 240 tiles, 32 / 36), and with a shorter K up to half (1024 rows of 2048 x
 // 2048 21 / 17; 1280, 160 tiles, 21 / 21, 513 of 4096 x 1024 11 / 15).
+// Where tiles of 256 x 256 fill their rounds to 95 % and no column of them is padding, the library's product of that size is ahead of a
+// plain one here: 8192 rows of 6144 x 4096 282 / 267, 4096 of 12288 x 4096 287 / 270, 4096 of 4096 x 4096 96 / 90; beside such
+// numbers of rows it is behind, 6000 of 12288 x 4096 442 / 547, 3000 of 6144 x 4096 115 / 136. With a gate it is behind in both
+// (4096 of 24576 x 4096 577 / 593). Left are a few plain products that nothing here tells from others, 4 to 8 % (8192 of 5376 x 4096
+// 263 / 250, 513 of 16448 x 4096 77 / 71).
 // One that adds into the stream, of more than half of the chip's tiles (1024 rows of 2048 x 2048 24 / 18), is priced beside the
-// library's, whose time for weights from memory is its products at 1.45 PFLOP/s, 14 us and 2.5 ns a k, within a tenth over 20 shapes
-// of 600 to 3000 rows: 2048 rows of 2560 x 4096 50 / 53, 3000 rows of 4096 x 4096 88 / 90. Above 3072 rows the library multiplies
-// without adding, which it does faster (4096 rows of 4096 x 4096 95 us; adding 117, here 121).
+// library's. What a product takes here by that price is 5 % less in a single round and 12 % more in many, and 12 % more in any where
+// the rows fill every tile (all workgroups then walk K in step, where a row tile of few rows runs ahead and brings the weights into
+// the caches); the library's time for weights from memory is its products at 1.45 PFLOP/s, 12 us and 3 ns a k. Over 300 products of
+// 24 shapes the choice is 2.7 % ahead of the library alone and nowhere more than 8 % behind it (2048 rows of 5120 x 8192 148 / 137):
+// 2048 rows of 2560 x 4096 47 / 48, 3000 of 5120 x 8192 192 / 187, 1733 of 5120 x 25600 382 / 682, but 768 of 4096 x 4096 42 / 36,
+// 1536 of 2560 x 9728 94 / 89. Above 3072 rows the library multiplies without adding, which it does faster (4096 rows of 4096 x 4096
+// 95 us; adding 117, here 121).
 // K stays whole, though two to six ranges would be ahead up to 1500 rows (1024 rows of 2560 x 9728 64 us against 85 in the library):
 // a row's sums then do not depend on how many rows share the call, so that a prompt gives the same bits alone and among others.
 extern "C" int ra_gemm_prompt_takes(int epilogue, int M, int N, int K) {
   if (M <= 128 || !ra_prompt_shape(N, K) || (size_t)N * K < (4u << 20)) return 0;
   const long cus = ra_cu_count(), tiles = (long)((M + 127) / 128) * ((N + 127) / 128);
   if (epilogue == GP_GATED) return K > 2048 && tiles * 2 <= cus ? 2 : 1;
-  if (epilogue == GP_PLAIN) return M > 512 && (K > 2048 ? tiles * 4 > cus * 3 : tiles * 2 > cus);
+  if (epilogue == GP_PLAIN) {
+    if (M <= 512 || (K > 2048 ? tiles * 4 <= cus * 3 : tiles * 2 <= cus)) return 0;
+    const long large = (long)((M + 255) / 256) * (N / 256), rounds = (large + cus - 1) / cus;
+    return N % 256 != 0 || large * 100 < rounds * cus * 95;
+  }
   if (epilogue != GP_ADD || M <= 256 || M > 3072 || tiles * 2 <= cus) return 0;
+  const RaPromptPlan p = ra_prompt_plan(M, N, K, K);
   const float adding = (float)M * N * 4.f / 4.5e6f;        // the stream read and written at the end
-  return ra_prompt_plan(M, N, K, K).us + adding <= (float)((double)M * N * K * 2.0 / 1.45e9) + 14.f + 0.0025f * K;
+  return p.us * (M % p.rows == 0 ? 1.12f : 1.12f - 0.17f / p.rounds) + adding <=
+         (float)((double)M * N * K * 2.0 / 1.45e9) + 12.f + 0.003f * K;
 }
 
 // bfloat16, many rows (ra_gemm_prompt_takes): epilogue 0 C = A . W^T in bfloat16; 1 bfloat16 silu(gate) * up; 2 float C += alpha *

@@ -202,12 +202,15 @@ def test_rows_off_16_bytes_are_not_left_in_ranges(M):
     assert all(ops().linear_ranges(a, b) is None for a, b in ((buf, w), (x, wide), (same, w)))
 
 
-# both sides of every line of the rule: half of the chip's 256 CUs in tiles of 128 x 128, three quarters for plain products of a long K
+# both sides of every line of the rule: half of the chip's 256 CUs in tiles of 128 x 128, three quarters for plain products of a long K;
+# plain ones whose 256 x 256 tiles fill their rounds, without padding; rows that fill every tile, or not, of one that adds
 @pytest.mark.parametrize("epilogue,M,N,K,own", [
     (1, 129, 2048, 4096, False), (1, 512, 4096, 2560, False), (1, 513, 4096, 2560, True), (1, 256, 8192, 2048, True),
     (0, 768, 4096, 4096, False), (0, 769, 4096, 4096, True), (0, 513, 1024, 8192, False), (0, 1024, 2048, 2048, False),
-    (0, 1025, 2048, 2048, True), (2, 1024, 2048, 2560, False), (2, 3072, 2048, 4096, True)])
-def test_few_tiles_are_the_library_s(epilogue, M, N, K, own, monkeypatch):
+    (0, 1025, 2048, 2048, True), (2, 1024, 2048, 2560, False), (2, 3072, 2048, 4096, True),
+    (0, 3841, 4096, 2560, False), (0, 3840, 4096, 2560, True), (0, 4097, 4096, 2560, True), (0, 4096, 4112, 2560, True),
+    (2, 768, 4096, 4096, False), (2, 700, 4096, 4096, True)])
+def test_who_takes_a_product_of_many_rows(epilogue, M, N, K, own, monkeypatch):
     x, w, g = operands(M, N, K, M + N)
     ref, err = x.double() @ w.double().T, bound(x, w, K)
     calls, call = [], kernels.library.call
