@@ -45,6 +45,12 @@ KBlocks k_blocks(int K) {
 // its end returns zeros and touches no memory, so rows past N or M, pieces past the block and runs past the last tile count
 // like any other load and cost nothing. A tile's runs are padded to a multiple of DEPTH, so that it ends where a round of the
 // ring does.
+#define RA_WAVE_HANDOVER                                   \
+  do {                                                     \
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront"); \
+    __builtin_amdgcn_wave_barrier();                       \
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront"); \
+  } while (0)
 template <int MT, int U, int DEPTH>
 __global__ void __launch_bounds__(8 * RA_WAVE, 4)
 gemm_f32_stream_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
@@ -106,9 +112,13 @@ gemm_f32_stream_kernel(const float* __restrict__ A, const float* __restrict__ W,
   for (int base = 0; base < total; base += DEPTH) {
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d) {
-      f32x4_t* const mine = laid[wave];      // this wave's alone: LDS takes its accesses in their order
+      // this wave's alone: LDS takes its accesses in their order, and the fences have the compiler keep that order where lanes
+      // read what others wrote, and write what others have read
+      f32x4_t* const mine = laid[wave];
+      RA_WAVE_HANDOVER;
 #pragma unroll
       for (int i = 0; i < LOADS; ++i) mine[(i * LR + wr) * CH + (wc ^ ((i * LR + wr) & (CH - 1)))] = w[d][i];
+      RA_WAVE_HANDOVER;
 #pragma unroll
       for (int u = 0; u < U; ++u)
 #pragma unroll
