@@ -447,12 +447,13 @@ int prompt_epilogue(const PromptArgs& g, int epilogue, hipStream_t stream) {
 // What a tile of `rows` x `cols` costs, measured on MI355X over products of 128 to 3000 rows (4096 to 25600 k, one to eight
 // ranges; the tile so chosen is within 4 % of the fastest at each of 23 shapes): a start, then for each round of workgroups an
 // end that grows with the tile and the steps, each a part of its own (barrier, first operands) and one that grows with the tile,
-// the more the fuller the chip is (power and fetches).
-static RaPromptPlan prompt_plan(int M, int N, int K, int range_k, int slots) {
+// the more the fuller the chip is (power and fetches). It ranks tiles; beside the library's times it is corrected (below), as many
+// full rounds take a tenth longer. Ten prices, 0.1 us of the host.
+RaPromptPlan ra_prompt_plan(int M, int N, int K, int range_k) {
   static const int sides[10][2] = {{256, 256}, {224, 256}, {192, 256}, {160, 256}, {128, 256},
                                    {256, 128}, {224, 128}, {192, 128}, {160, 128}, {128, 128}};
   RaPromptPlan best = {0, 0, 0, 0, 0, 1e30f};
-  const int steps = K / GP_BK, each = range_k / GP_BK, ranges = (steps + each - 1) / each;
+  const int slots = ra_cu_count() / RA_XCDS, steps = K / GP_BK, each = range_k / GP_BK, ranges = (steps + each - 1) / each;
   if (steps - (ranges - 1) * each < GP_STEPS) return best;
   for (const auto& side : sides) {
     const long tiles = (long)((M + side[0] - 1) / side[0]) * ((N + side[1] - 1) / side[1]) * ranges;
@@ -462,23 +463,6 @@ static RaPromptPlan prompt_plan(int M, int N, int K, int range_k, int slots) {
     if (us < best.us) best = {side[0], side[1], ranges, range_k, (int)rounds, us};
   }
   return best;
-}
-
-// A step asks for the same few plans layer after layer, twice a product (which kernel, the launch): a thread keeps those of the
-// last shapes.
-RaPromptPlan ra_prompt_plan(int M, int N, int K, int range_k) {
-  struct Kept {
-    int M, N, K, range_k, slots;
-    RaPromptPlan plan;
-  };
-  static thread_local Kept kept[64];
-  const int slots = ra_cu_count() / RA_XCDS;
-  const unsigned h = (unsigned)M * 2654435761u ^ (unsigned)N * 2246822519u ^ (unsigned)K * 3266489917u ^
-                     (unsigned)range_k * 668265263u;
-  Kept& k = kept[h >> 26];
-  if (k.M != M || k.N != N || k.K != K || k.range_k != range_k || k.slots != slots)
-    k = {M, N, K, range_k, slots, prompt_plan(M, N, K, range_k, slots)};
-  return k.plan;
 }
 
 int ra_prompt_product(const RaPromptPlan& plan, int epilogue, const void* A, const void* W, void* C, int M, int N, int K, int lda,
