@@ -85,3 +85,31 @@ def test_tokens_of_other_number_kinds():
         kernels.current().filter_logits(logits, p, [history])
         want = logits.clone() if want is None else want
         assert torch.equal(logits, want) and logits[0, 3] == -2.0 and logits[0, 4] == 0.0
+
+
+@pytest.mark.parametrize("window", [1, 255, 257, 1024, 1025, 3000])
+@pytest.mark.parametrize("pad", [0, 3])
+@pytest.mark.parametrize("bias", [(), ((3, 1.0), (4097, -2.0), (12288, 0.5))])
+def test_penalties_over_windows_of_every_length(window, pad, bias):
+    """Windows that are counted in LDS and longer ones, shorter and longer than a workgroup, with tokens on both sides of the
+    window's start and in every slice; rows on 16 bytes and off. All numbers are exact in binary: so is the result."""
+    from reinfer_amd import kernels
+    from reinfer_amd.sampling import SamplingParams
+    V = 12289
+    g = torch.Generator().manual_seed(window)
+    rows = torch.randint(-64, 64, (4, V), generator=g) / 16.0
+    rows[:, [5, 9000]] = float("-inf")
+    kinds = [dict(frequency_penalty=0.25), dict(repeat_penalty=2.0, presence_penalty=0.5),
+             dict(temperature=1.0, top_k=40, repeat_penalty=4.0, frequency_penalty=0.125), dict(presence_penalty=0.5)]
+    # few different tokens, so that they come again across the window's start; the last row's are all one
+    histories = [torch.randint(0, 400, (3100,), generator=g).mul(V // 400).tolist() for _ in kinds[:3]] + [[12288] * 3100]
+    params = [SamplingParams(repeat_last_n=window, logit_bias=bias, **k) for k in kinds]
+    logits = torch.full((4, V + pad), 7.0, device=DEV)
+    logits[:, :V] = rows.to(DEV)
+    kernels.current().filter_logits(logits[:, :V], params, histories)
+    got = logits.cpu()
+    assert (got[:, V:] == 7.0).all()
+    for i, k in enumerate(kinds):
+        kw = {a: b for a, b in k.items() if a != "temperature"}
+        want = plain.filter_logits(rows[i], k.get("temperature", 0.0), window=histories[i][-window:], logit_bias=bias, **kw)
+        assert torch.equal(got[i, :V].double(), want), (i, (got[i, :V] != want).nonzero()[:5])
