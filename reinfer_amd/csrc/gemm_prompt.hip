@@ -13,10 +13,10 @@
 // policy (non-temporal): 2 to 50 % slower. The workgroups stay (one a CU) and ask for the next tile's first stages before they
 // write a tile's sums.
 //
-// The tile and the K ranges are chosen for the fewest part-filled rounds of workgroups, which is what the library's own product
-// loses on: with the gate 3000 x 24576 x 4096 466 us against 614 with the library and the gate's kernel, 2048 x 19456 x 2560 166
-// against 203, 512 x 51200 x 5120 234 against 288; 3000 x 6144 x 4096 127 against 146, but 8000 x 6144 x 4096, whose rounds are full
-// in any tile, 281 against 272. Weight rows of a tile are permuted (gp_row) so that a lane's sums are stored 16 bytes at a time.
+// The tile is chosen for the fewest part-filled rounds of workgroups, which is what the library's own product loses on: with the gate
+// 3000 x 24576 x 4096 459 us against 599 with the library and the gate's kernel, 2048 x 19456 x 2560 169 against 214, 512 x 51200 x
+// 5120 226 against 285; 3000 x 6144 x 4096 115 against 136, but 8192 x 6144 x 4096, whose rounds are full in any tile, 282 against 267
+// (ra_gemm_prompt_takes). Weight rows of a tile are permuted (gp_row) so that a lane's sums are stored 16 bytes at a time.
 #include <type_traits>
 #include <utility>
 #include <math.h>
