@@ -207,7 +207,8 @@ void ra_tile_plan(int M, int N, int K, int* ranges, int* range_k) {
 // those as well): 11264 x 4096 at 128 rows, 176 of 256 CUs, takes 34 us against the library's 32, 9216 x 4096, 216 CUs, 26
 // against 30; 22528 x 4096, whose tiles do not fill the chip and cannot be cut, 49 against 45. Above 256 rows only a long K,
 // where the planes are few beside the weights, and more than that share of the chip (4096 x 12288 at 384 rows, 192 CUs,
-// 68 us against 67; at 512 rows, all of them, 73 against 80); beyond 512 the library's larger tiles read less. What adds into
+// 70 us on gemm_prompt.hip's tiles against 69, though at 300 rows 57 against 69; at 512 rows, all of them, 74 against 80); the line
+// is the same for all rows of a row of tiles, as the sums are. Beyond 512 the library's larger tiles read less. What adds into
 // the stream with up to 128 rows also finishes the norm behind it, which outweighs a poor fill. A gated product, which is
 // not cut, where one row of tiles fills half of the chip. Below 8 MB of weights (a router, gates) both take the few us of
 // their launches, and the calls stay where they were.
