@@ -89,7 +89,7 @@ int ra_moe_grouped(const void* x, int ldx, const void* w_up, const void* w_down,
                    const float* more, const float* more_logit, int ld_logit, float* resid, void* out, float alpha,
                    void* scratch, long scratch_bytes, hipStream_t stream);
 
-// float operands and result on the float matrix cores, for rows that are whole 16-byte pieces (ra_gemm_f32_supports):
+// float operands and result, to float precision on the bfloat16 matrix cores (each float in three parts), for rows that are whole 16-byte pieces (ra_gemm_f32_supports):
 // C[M, N] = A . W^T (+ bias). scratch: ra_gemm_f32_scratch floats (0: none needed).
 int ra_gemm_f32_supports(const void* A, const void* W, int K, int lda);
 long ra_gemm_f32_scratch(int M, int N, int K);

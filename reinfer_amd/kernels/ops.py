@@ -720,7 +720,7 @@ class HipKernels:
         result (the head's logits for more than 64 wanted rows): the library
         product again, bfloat16 operands and a float result.
         float32 whose rows are whole 16-byte pieces: this library's product on the
-        float matrix cores. Everything else: the plain FMA kernel.
+        bfloat16 matrix cores, in three parts each. Everything else: the plain FMA kernel.
         """
         if bias is not None:
             bias = bias.contiguous()         # the kernels here read it as it lies
