@@ -80,6 +80,44 @@ struct ScanArgs {
   const int* positions; const float* inv_freq; int rot_dims;      // retention: the turn of q and k
 };
 
+// One token of the matrix memory and of the delta rule in a lane: the state (and normaliser) moves on, its column's read-out comes back.
+// The fused operations are written out: two kernels use these, and a token's bits are the same in both. (Of the delta rule's state the
+// first element has the other product fused; so the compiler had it, and a network's results keep their bits.)
+template <int R, int NPL>
+__device__ __forceinline__ float memory_step(float (&S)[NPL], float (&nrm)[NPL], const float (&k)[NPL], const float (&q)[NPL], float v,
+                                             float keep, float take, float least, float denom_eps) {
+  float ps[2] = {0.f, 0.f}, pn[2] = {0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < NPL; ++i) {
+    const float tk = take * k[i];
+    nrm[i] = fmaf(keep, nrm[i], tk);
+    S[i] = fmaf(tk, v, keep * S[i]);
+    ps[i & 1] = fmaf(S[i], q[i], ps[i & 1]);
+    pn[i & 1] = fmaf(nrm[i], q[i], pn[i & 1]);
+  }
+  const float s1 = group_sum<R>(ps[0] + ps[1]);
+  const float s2 = group_sum<R>(pn[0] + pn[1]);
+  return __fdividef(s1, fmaxf(fabsf(s2), least) + denom_eps);      // a reciprocal and a product: within an ulp or two
+}
+template <int R, int NPL>
+__device__ __forceinline__ float delta_step(float (&S)[NPL], const float (&k)[NPL], const float (&q)[NPL], float v, float beta,
+                                            float decay) {
+  float pa[2] = {0.f, 0.f}, pb[2] = {0.f, 0.f}, pkq[2] = {0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < NPL; ++i) {
+    pa[i & 1] = fmaf(S[i], k[i], pa[i & 1]);
+    pb[i & 1] = fmaf(S[i], q[i], pb[i & 1]);
+    pkq[i & 1] = fmaf(k[i], q[i], pkq[i & 1]);
+  }
+  const float sa = group_sum<R>(pa[0] + pa[1]);
+  const float sb = group_sum<R>(pb[0] + pb[1]);
+  const float skq = group_sum<R>(pkq[0] + pkq[1]);
+  const float u = beta * fmaf(-decay, sa, v);
+#pragma unroll
+  for (int i = 0; i < NPL; ++i) S[i] = i == 0 ? fmaf(decay, S[i], k[i] * u) : fmaf(k[i], u, decay * S[i]);
+  return fmaf(decay, sb, u * skq);
+}
+
 template <typename TA, int R, int NPL, int MODE>
 __global__ __launch_bounds__(256) void scan_kernel(ScanArgs p) {
   constexpr bool MEMORY = MODE == SCAN_MEMORY, WKV = MODE == SCAN_WKV, DECAY = MODE == SCAN_DECAY;
@@ -251,19 +289,7 @@ __global__ __launch_bounds__(256) void scan_kernel(ScanArgs p) {
       auto step = [&](int tt, const Operands& x) {   // one token: the state moves on, the read-out is stored
         float o;
         if (MEMORY) {
-          const float keep = x.g0, take = x.g1;
-          float ps[2] = {0.f, 0.f}, pn[2] = {0.f, 0.f};
-#pragma unroll
-          for (int i = 0; i < NPL; ++i) {
-            const float tk = take * x.k[i];
-            nrm[i] = keep * nrm[i] + tk;
-            S[i] = keep * S[i] + tk * x.v;
-            ps[i & 1] += S[i] * x.q[i];
-            pn[i & 1] += nrm[i] * x.q[i];
-          }
-          const float s1 = group_sum<R>(ps[0] + ps[1]);
-          const float s2 = group_sum<R>(pn[0] + pn[1]);
-          o = __fdividef(s1, fmaxf(fabsf(s2), x.g2) + p.denom_eps);      // a reciprocal and a product: within an ulp or two
+          o = memory_step<R, NPL>(S, nrm, x.k, x.q, x.v, x.g0, x.g1, x.g2, p.denom_eps);
         } else if (WKV) {
           // o = (S + diag(u) k v^T)^T q with the bonus for this token alone; then S <- diag(w) S + k v^T
           float po[2] = {0.f, 0.f};
@@ -291,20 +317,7 @@ __global__ __launch_bounds__(256) void scan_kernel(ScanArgs p) {
           }
           o = group_sum<R>(po[0] + po[1]);
         } else {
-          float pa[2] = {0.f, 0.f}, pb[2] = {0.f, 0.f}, pkq[2] = {0.f, 0.f};
-#pragma unroll
-          for (int i = 0; i < NPL; ++i) {
-            pa[i & 1] += S[i] * x.k[i];
-            pb[i & 1] += S[i] * x.q[i];
-            pkq[i & 1] += x.k[i] * x.q[i];
-          }
-          const float sa = group_sum<R>(pa[0] + pa[1]);
-          const float sb = group_sum<R>(pb[0] + pb[1]);
-          const float skq = group_sum<R>(pkq[0] + pkq[1]);
-          const float u = x.g0 * (x.v - x.g1 * sa);
-#pragma unroll
-          for (int i = 0; i < NPL; ++i) S[i] = x.g1 * S[i] + x.k[i] * u;
-          o = x.g1 * sb + u * skq;
+          o = delta_step<R, NPL>(S, x.k, x.q, x.v, x.g0, x.g1);
         }
         if (col_ok && r == 0) p.out[(size_t)(t0 + tt) * ow + head * dv + col] = o;
       };
@@ -333,33 +346,119 @@ __global__ __launch_bounds__(256) void scan_kernel(ScanArgs p) {
   }
 }
 
+// The matrix memory's log gates a (input) and b (forget) from their pre-activations, and the delta rule's beta and decay
+struct LogGates {
+  float a, b;
+};
+__device__ __forceinline__ LogGates memory_gates(float zi, float zf, float bias_i, float bias_f, float cap) {
+  zi += bias_i;
+  zf += bias_f;
+  if (cap > 0.f) { zi = cap * tanhf(zi / cap); zf = cap * tanhf(zf / cap); }
+  return {zi, ra_logsigmoid(zf)};
+}
+__device__ __forceinline__ float delta_beta(float z) { return 1.f / (1.f + expf(-z)); }
+__device__ __forceinline__ float delta_decay(float z, float a_log, float dt_bias) {
+  return expf(-expf(a_log) * ra_softplus(z + dt_bias));
+}
+
+// A step in which every request brings one token: nothing to stage and nothing to walk, so a lane reads its own run of k and q from
+// memory, works out the gates for itself and has its part of the state asked for at the same time; no LDS, no barrier, and no
+// kernels ahead that prepare gates. Bound by the state read and written, behind two trips to memory. Eight requests in a decode
+// step, 16 heads of 128 x 256: gates and scan_kernel 5.0 + 16.6 us, this one 12.4 (33 MB); the delta rule, 32 heads of 128 x 128:
+// 4.5 + 13.8, so 9.2, and 4.9 less for the filter's tail, which the kernel that prepares q, k and v moves on then.
+struct TokenGates {
+  const float* z;                                    // [T, 2 H] pre-activations
+  const float *first, *second;                       // their biases [2 H] (matrix memory); A_log, dt_bias [H] (delta rule)
+  float cap;
+  bool whole;                                        // k and q rows are whole 16-byte pieces of R NPL elements
+};
+template <typename TA, int R, int NPL, int MODE>
+__global__ __launch_bounds__(256) void scan_token_kernel(ScanArgs p, TokenGates g) {
+  constexpr bool MEMORY = MODE == SCAN_MEMORY;
+  constexpr int CPW = RA_WAVE / R;
+  const int seq = blockIdx.x, head = blockIdx.y, H = p.H;
+  const int lane = threadIdx.x & (RA_WAVE - 1), c = lane / R, r = lane % R;
+  const int w = blockIdx.z * (blockDim.x / RA_WAVE) + threadIdx.x / RA_WAVE, col = w * CPW + c;
+  const int t = p.cu_tokens[seq], end = p.cu_tokens[seq + 1], slot = p.state_slots[seq];
+  const bool zero = p.fresh[seq] != 0, col_ok = col < p.dv;
+  if (w >= p.waves_per_head || t >= end) return;
+  float* out = p.out + (size_t)t * H * p.dv + (size_t)head * p.dv + col;
+  if (slot < 0) {                                    // a padding row: no state, a defined result
+    if (col_ok && r == 0) *out = 0.f;
+    return;
+  }
+  float* st = p.state + (size_t)slot * p.slot_stride + (size_t)(head * p.waves_per_head + w) * p.wave_floats;
+  float* mp = st + NPL * RA_WAVE + NPL * R;          // this wave's copy of the running maximum
+  const size_t at = (size_t)t * p.ld + (size_t)(head / (H / p.q_heads)) * p.dk + r * NPL;
+  const TA *kr = (const TA*)p.k + at, *qr = (const TA*)p.q + at;
+  float S[NPL], nrm[NPL], k[NPL], q[NPL];
+#pragma unroll
+  for (int i = 0; i < NPL; ++i) {
+    S[i] = zero ? 0.f : st[i * RA_WAVE + lane];
+    nrm[i] = MEMORY && !zero ? st[NPL * RA_WAVE + i * R + r] : 0.f;
+  }
+  if constexpr (NPL == 8) {
+    if (g.whole) {
+      Vec8<TA>::load(kr, k);
+      Vec8<TA>::load(qr, q);
+    }
+  }
+  if (NPL != 8 || !g.whole) {
+#pragma unroll
+    for (int i = 0; i < NPL; ++i) {
+      const bool in = r * NPL + i < p.dk;
+      k[i] = in ? to_f32(kr[i]) : 0.f;
+      q[i] = in ? to_f32(qr[i]) : 0.f;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NPL; ++i) q[i] *= p.q_scale;
+  const float v = col_ok ? to_f32(((const TA*)p.v)[(size_t)t * p.ld + (size_t)head * p.dv + col]) : 0.f;
+  const float z0 = g.z[(size_t)t * 2 * H + head], z1 = g.z[(size_t)t * 2 * H + H + head];
+  float o;
+  if constexpr (MEMORY) {
+    const float m = zero ? 0.f : *mp;
+    const LogGates l = memory_gates(z0, z1, g.first[head], g.first[H + head], g.cap);
+    const float top = fmaxf(l.b + m, l.a);
+    o = memory_step<R, NPL>(S, nrm, k, q, v, expf(l.b + m - top), expf(l.a - top), expf(-top), p.denom_eps);
+    if (lane == 0) *mp = top;
+  } else {
+    o = delta_step<R, NPL>(S, k, q, v, delta_beta(z0), delta_decay(z1, g.first[head], g.second[head]));
+  }
+  if (col_ok && r == 0) *out = o;
+#pragma unroll
+  for (int i = 0; i < NPL; ++i) {
+    st[i * RA_WAVE + lane] = S[i];
+    if (MEMORY && c == 0) st[NPL * RA_WAVE + i * R + r] = nrm[i];
+  }
+}
+
 // The matrix memory's gates. z [T, 2 H] holds the pre-activations (input | forget); with a = cap tanh((z_i + bias) / cap)
 // and b = log sigmoid(cap tanh((z_f + bias) / cap)) the running maximum is m_t = max(b_t + m_{t-1}, a_t), a chain over
 // the request's tokens. The map m -> max(b + m, a) is the pair (a, b), and two such maps compose to
 // (max(a1 + b2, a2), b1 + b2), so a workgroup a (request, head) takes 256 tokens at a time through a prefix scan
 // in LDS. g3 [T, 3 H] gets keep = exp(b + m_{t-1} - m_t), take = exp(a - m_t) and exp(-m_t). The maximum itself
-// is kept in the request's state at `m_off` floats behind the head's first float (0 at a request's start).
+// is kept in the request's state `m_off` floats behind the first float of each wave's part of the head (0 at a request's start):
+// once a wave, so that the waves of a step of single tokens can move it on without waiting for each other.
 __global__ __launch_bounds__(256) void matrix_memory_gate_scan_kernel(
     const float* __restrict__ z, const float* __restrict__ bias, float cap, float* __restrict__ g3,
-    float* __restrict__ state, long slot_stride, long head_floats, long m_off, const int* __restrict__ cu_tokens,
+    float* __restrict__ state, long slot_stride, int waves, int wave_floats, int m_off, const int* __restrict__ cu_tokens,
     const int* __restrict__ state_slots, const int* __restrict__ fresh, int H) {
   __shared__ float sA[256], sB[256];
   const int seq = blockIdx.x, head = blockIdx.y, tid = threadIdx.x;
   const int first = cu_tokens[seq], last = cu_tokens[seq + 1];
   const int slot = state_slots[seq];
   if (slot < 0 || first >= last) return;       // the scan writes zeros for a padding row without reading its gates
-  float* mp = state + (size_t)slot * slot_stride + (size_t)head * head_floats + m_off;
+  float* mp = state + (size_t)slot * slot_stride + (size_t)head * waves * wave_floats + m_off;
   float m_run = fresh[seq] != 0 ? 0.f : *mp;
   for (int t0 = first; t0 < last; t0 += 256) {
     const int t = t0 + tid;
     const bool valid = t < last;
     float a = -INFINITY, b = 0.f;              // the identity map for rows past the end
     if (valid) {
-      float zi = z[(size_t)t * 2 * H + head] + bias[head];
-      float zf = z[(size_t)t * 2 * H + H + head] + bias[H + head];
-      if (cap > 0.f) { zi = cap * tanhf(zi / cap); zf = cap * tanhf(zf / cap); }
-      a = zi;
-      b = ra_logsigmoid(zf);
+      const LogGates l = memory_gates(z[(size_t)t * 2 * H + head], z[(size_t)t * 2 * H + H + head], bias[head], bias[H + head], cap);
+      a = l.a;
+      b = l.b;
     }
     float A = a, B = b;
     sA[tid] = A;
@@ -391,7 +490,7 @@ __global__ __launch_bounds__(256) void matrix_memory_gate_scan_kernel(
     __syncthreads();                           // before the next round overwrites the maps
     m_run = m_end;
   }
-  if (tid == 0) *mp = m_run;
+  for (int w = tid; w < waves; w += 256) mp[(size_t)w * wave_floats] = m_run;
 }
 
 // gb[t, h] <- sigmoid(b);  gb[t, H + h] <- exp(-exp(A_log[h]) softplus(a + dt_bias[h])), in place
@@ -401,8 +500,7 @@ __global__ void delta_rule_gates_kernel(float* __restrict__ gb, const float* __r
   if (i >= n) return;
   const int j = (int)(i % (2 * H));
   const float z = gb[i];
-  if (j < H) gb[i] = 1.f / (1.f + expf(-z));
-  else gb[i] = expf(-expf(a_log[j - H]) * ra_softplus(z + dt_bias[j - H]));
+  gb[i] = j < H ? delta_beta(z) : delta_decay(z, a_log[j - H], dt_bias[j - H]);
 }
 
 // ---------------------------------------------------------------------------
@@ -413,13 +511,16 @@ __global__ void delta_rule_gates_kernel(float* __restrict__ gb, const float* __r
 // ---------------------------------------------------------------------------
 #define PREP_WAVES 4
 #define PREP_HOLD 8          // values a lane keeps: heads up to 512 wide
+// `single`: every portion is one token, and the request's tail moves on here as well, each channel's by the one lane that read it.
+// Filters of up to PREP_TAPS taps have a channel's rows asked for together.
+#define PREP_TAPS 4
 template <typename TA>
 __global__ void delta_rule_prepare_kernel(const TA* __restrict__ proj, int ld, const float* __restrict__ filt,
-                                          const float* __restrict__ state, long slot_stride, long tail_off,
+                                          float* __restrict__ state, long slot_stride, long tail_off,
                                           const int* __restrict__ seq_of_token, const int* __restrict__ cu_tokens,
                                           const int* __restrict__ state_slots, const int* __restrict__ fresh, int G,
                                           int dk, int H, int dv, int taps, float unit_eps, float q_scale,
-                                          float* __restrict__ qkv, int T) {
+                                          float* __restrict__ qkv, int T, bool single) {
   const int lane = threadIdx.x & (RA_WAVE - 1);
   const int units = 2 * G + H;
   const long idx = (long)blockIdx.x * PREP_WAVES + threadIdx.x / RA_WAVE;
@@ -438,26 +539,57 @@ __global__ void delta_rule_prepare_kernel(const TA* __restrict__ proj, int ld, c
     return;
   }
   const bool zero = fresh[seq] != 0;
-  const float* tail = state + (size_t)slot * slot_stride + tail_off;      // [taps - 1, C], oldest first
+  float* tail = state + (size_t)slot * slot_stride + tail_off;            // [taps - 1, C], oldest first
+  auto row = [&](int p, int ch) {                          // of the filter's rows at this token
+    const int rel = t - first - (taps - 1) + p;            // row of the portion, negative: a row of the tail
+    if (rel >= 0) return to_f32(proj[(size_t)(first + rel) * ld + ch]);
+    return zero ? 0.f : tail[(size_t)(taps - 1 + rel) * C + ch];
+  };
   float y[PREP_HOLD];
   float ss = 0.f;
+  auto filtered = [&](int j, float acc) {
+    acc = acc / (1.f + expf(-acc));
+    y[j] = acc;
+    ss = fmaf(acc, acc, ss);
+  };
+  if (taps <= PREP_TAPS) {
+    float x[PREP_HOLD][PREP_TAPS], f[PREP_HOLD][PREP_TAPS];
 #pragma unroll
-  for (int j = 0; j < PREP_HOLD; ++j) {
-    const int e = lane + j * RA_WAVE;
-    y[j] = 0.f;
-    if (e < width) {
-      const int ch = base + e;
+    for (int j = 0; j < PREP_HOLD; ++j) {
+      const int ch = base + lane + j * RA_WAVE;
+#pragma unroll
+      for (int p = 0; p < PREP_TAPS; ++p) {
+        const bool in = lane + j * RA_WAVE < width && p < taps;
+        x[j][p] = in ? row(p, ch) : 0.f;
+        f[j][p] = in ? filt[(size_t)ch * taps + p] : 0.f;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < PREP_HOLD; ++j) {
+      y[j] = 0.f;
+      if (lane + j * RA_WAVE >= width) continue;
+      const int ch = base + lane + j * RA_WAVE;
+      float acc = 0.f;
+#pragma unroll
+      for (int p = 0; p < PREP_TAPS; ++p) {
+        if (p < taps) acc = fmaf(f[j][p], x[j][p], acc);
+        if (single && p > 0 && p < taps) tail[(size_t)(p - 1) * C + ch] = x[j][p];
+      }
+      filtered(j, acc);
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < PREP_HOLD; ++j) {
+      y[j] = 0.f;
+      if (lane + j * RA_WAVE >= width) continue;
+      const int ch = base + lane + j * RA_WAVE;
       float acc = 0.f;
       for (int p = 0; p < taps; ++p) {
-        const int rel = t - first - (taps - 1) + p;        // row of the portion, negative: a row of the tail
-        float x;
-        if (rel >= 0) x = to_f32(proj[(size_t)(first + rel) * ld + ch]);
-        else x = zero ? 0.f : tail[(size_t)(taps - 1 + rel) * C + ch];
+        const float x = row(p, ch);
         acc = fmaf(filt[(size_t)ch * taps + p], x, acc);
+        if (single && p > 0) tail[(size_t)(p - 1) * C + ch] = x;      // this row has been read
       }
-      acc = acc / (1.f + expf(-acc));
-      y[j] = acc;
-      ss = fmaf(acc, acc, ss);
+      filtered(j, acc);
     }
   }
   float f = 1.f;
@@ -479,7 +611,6 @@ __global__ void delta_rule_prepare_kernel(const TA* __restrict__ proj, int ld, c
 // order of the kernel above, so that a token's inputs do not depend on how many tokens stand beside it. Bound by its rows in and
 // results out: 1859 tokens of 8192 channels, four taps, 106 us in the kernel above, 43 here (40 with one sum a lane).
 #define PREP_RUN 8
-#define PREP_TAPS 4
 template <typename TA, int LANES>
 __global__ void __launch_bounds__(256)
 delta_rule_prepare_run_kernel(const TA* __restrict__ proj, int ld, const float* __restrict__ filt,
@@ -688,20 +819,46 @@ struct MeanInputs {
   const void* x[MEAN_MAX];
   const float* w[MEAN_MAX];
 };
-template <typename TA, int N>
+// HELD: rows that two runs of eight neighbouring elements a thread cover, read in 16-byte accesses, all asked for at once with the
+// weights and the stream's old values, and handed round in LDS for the sums, whose order is the other form's; else every element is
+// read twice, one a thread at a time. Eight rows of 4096, two inputs, in a decode step: 10.1 us read twice, 5.0 held.
+#define MEAN_LDS (64 * 1024)
+template <typename TA, int N, bool HELD>
 __global__ void normed_mean_kernel(MeanInputs in, float eps, int h, TA* __restrict__ out, float* __restrict__ resid,
                                    float scale) {
+  extern __shared__ __attribute__((aligned(16))) float held[];       // [N][h]
   __shared__ float red[N][17];
   const size_t row = (size_t)blockIdx.x * h;
   const int lane = threadIdx.x & (RA_WAVE - 1), wave = threadIdx.x / RA_WAVE, nwave = blockDim.x / RA_WAVE;
+  float x[2][N][8], wt[2][N][8], old[2][8];
   float ss[N];
 #pragma unroll
   for (int i = 0; i < N; ++i) ss[i] = 0.f;
+  if constexpr (HELD) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int at = (threadIdx.x + j * blockDim.x) * 8;
+      if (at >= h) break;
+#pragma unroll
+      for (int i = 0; i < N; ++i) Vec8<TA>::load((const TA*)in.x[i] + row + at, x[j][i]);
+#pragma unroll
+      for (int i = 0; i < N; ++i) Vec8<float>::load(in.w[i] + at, wt[j][i]);
+      if (resid) Vec8<float>::load(resid + row + at, old[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int at = (threadIdx.x + j * blockDim.x) * 8;
+      if (at >= h) break;
+#pragma unroll
+      for (int i = 0; i < N; ++i) Vec8<float>::store(held + i * h + at, x[j][i]);
+    }
+    __syncthreads();
+  }
   for (int e = threadIdx.x; e < h; e += blockDim.x) {
 #pragma unroll
     for (int i = 0; i < N; ++i) {
-      const float v = to_f32(((const TA*)in.x[i])[row + e]);
-      ss[i] += v * v;
+      const float v = HELD ? held[i * h + e] : to_f32(((const TA*)in.x[i])[row + e]);
+      ss[i] = fmaf(v, v, ss[i]);
     }
   }
 #pragma unroll
@@ -717,12 +874,30 @@ __global__ void normed_mean_kernel(MeanInputs in, float eps, int h, TA* __restri
     for (int w = 0; w < nwave; ++w) t += red[i][w];          // fixed order
     rstd[i] = 1.f / sqrtf(t / (float)h + eps) * (1.f / (float)N);
   }
-  for (int e = threadIdx.x; e < h; e += blockDim.x) {
-    float y = 0.f;
+  if constexpr (HELD) {
 #pragma unroll
-    for (int i = 0; i < N; ++i) y += to_f32(((const TA*)in.x[i])[row + e]) * rstd[i] * in.w[i][e];
-    if (resid) resid[row + e] += scale * y;
-    else out[row + e] = from_f32<TA>(y);
+    for (int j = 0; j < 2; ++j) {
+      const int at = (threadIdx.x + j * blockDim.x) * 8;
+      if (at >= h) return;
+      float y[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        y[e] = 0.f;
+#pragma unroll
+        for (int i = 0; i < N; ++i) y[e] = fmaf(x[j][i][e] * rstd[i], wt[j][i][e], y[e]);
+        old[j][e] = fmaf(scale, y[e], old[j][e]);
+      }
+      if (resid) Vec8<float>::store(resid + row + at, old[j]);
+      else Vec8<TA>::store(out + row + at, y);
+    }
+  } else {
+    for (int e = threadIdx.x; e < h; e += blockDim.x) {
+      float y = 0.f;
+#pragma unroll
+      for (int i = 0; i < N; ++i) y = fmaf(to_f32(((const TA*)in.x[i])[row + e]) * rstd[i], in.w[i][e], y);
+      if (resid) resid[row + e] = fmaf(scale, y, resid[row + e]);
+      else out[row + e] = from_f32<TA>(y);
+    }
   }
 }
 
@@ -762,9 +937,19 @@ ScanLaunch scan_launch(const ScanGeom& g, int n_seqs, int heads, int max_q_len, 
   return L;
 }
 
-template <typename TA, int MEMORY>
-int scan_dispatch(const ScanGeom& g, const ScanLaunch& L, const ScanArgs& a, hipStream_t stream) {
-#define RA_SCAN(R, NPL) scan_kernel<TA, R, NPL, MEMORY><<<L.grid, L.threads, L.lds, stream>>>(a)
+// With `tg` a step of single tokens.
+template <typename TA, int MODE>
+int scan_dispatch(const ScanGeom& g, const ScanLaunch& L, const ScanArgs& a, hipStream_t stream, const TokenGates* tg = nullptr) {
+#define RA_SCAN(R, NPL)                                                                               \
+  do {                                                                                                \
+    if constexpr (MODE == SCAN_MEMORY || MODE == SCAN_DELTA) {                                        \
+      if (tg) {                                                                                       \
+        scan_token_kernel<TA, R, NPL, MODE><<<L.grid, L.threads, 0, stream>>>(a, *tg);                \
+        break;                                                                                        \
+      }                                                                                               \
+    }                                                                                                 \
+    scan_kernel<TA, R, NPL, MODE><<<L.grid, L.threads, L.lds, stream>>>(a);                           \
+  } while (0)
 #define RA_SCAN_N(R)                               \
   do {                                             \
     if (g.NPL == 2) RA_SCAN(R, 2);                 \
@@ -797,12 +982,15 @@ extern "C" int ra_matrix_memory_scan(const void* proj, int act_dtype, int ld, in
            slot_stride, (long)heads * g.waves * g.wave_floats);
   RA_CHECK(heads <= 65535, "matrix_memory_scan: %d heads in one launch", heads);
   RA_CHECK(act_dtype == RA_F32 || act_dtype == RA_BF16, "matrix_memory_scan: unknown dtype tag %d", act_dtype);
-  // the running maximum lives where the first wave of each head has its spare floats
-  matrix_memory_gate_scan_kernel<<<dim3(n_seqs, heads), 256, 0, stream>>>(
-      gates, gate_bias, gate_cap, gates3, state, slot_stride, (long)g.waves * g.wave_floats,
-      (long)g.NPL * RA_WAVE + (long)g.NPL * g.R, cu_tokens, state_slots, fresh, heads);
-  RA_LAUNCH_CHECK("matrix_memory_gates");
-  if (scratch) {
+  const bool single = max_q_len == 1 && !(scratch && chunk_from <= 1);      // (chunks of every portion may be asked for)
+  if (!single) {
+    // the running maximum lives in the spare floats of each wave's part
+    matrix_memory_gate_scan_kernel<<<dim3(n_seqs, heads), 256, 0, stream>>>(
+        gates, gate_bias, gate_cap, gates3, state, slot_stride, g.waves, g.wave_floats, g.NPL * RA_WAVE + g.NPL * g.R,
+        cu_tokens, state_slots, fresh, heads);
+    RA_LAUNCH_CHECK("matrix_memory_gates");
+  }
+  if (scratch && !single) {
     const int rc = ra_matrix_memory_chunks(proj, act_dtype, ld, q_off, k_off, v_off, gates3, state, slot_stride, cu_tokens,
                                            state_slots, fresh, n_seqs, n_tokens, heads, key_dim, value_dim, q_scale, denom_eps,
                                            scratch, scratch_floats, chunk_from, out, stream);
@@ -818,16 +1006,19 @@ extern "C" int ra_matrix_memory_scan(const void* proj, int act_dtype, int ld, in
   a.ld = ld; a.q_heads = heads; a.gates = gates3; a.state = state; a.slot_stride = slot_stride;
   a.cu_tokens = cu_tokens; a.state_slots = state_slots; a.fresh = fresh;
   a.H = heads; a.dk = key_dim; a.dv = value_dim; a.waves_per_head = g.waves; a.wave_floats = g.wave_floats;
-  a.chunk = L.chunk; a.below = scratch ? chunk_from : 0; a.q_scale = q_scale; a.denom_eps = denom_eps; a.out = out;
-  if (act_dtype == RA_F32) scan_dispatch<float, SCAN_MEMORY>(g, L, a, stream);
-  else scan_dispatch<bf16_t, SCAN_MEMORY>(g, L, a, stream);
+  a.chunk = L.chunk; a.below = scratch && !single ? chunk_from : 0; a.q_scale = q_scale; a.denom_eps = denom_eps; a.out = out;
+  const TokenGates tg = {gates, gate_bias, nullptr, gate_cap,
+                         key_dim == g.R * g.NPL && ra_rows_16b(a.k, ld, (int)es) && ra_rows_16b(a.q, ld, (int)es) &&
+                             key_dim * es % 16 == 0};
+  if (act_dtype == RA_F32) scan_dispatch<float, SCAN_MEMORY>(g, L, a, stream, single ? &tg : nullptr);
+  else scan_dispatch<bf16_t, SCAN_MEMORY>(g, L, a, stream, single ? &tg : nullptr);
   RA_LAUNCH_CHECK("matrix_memory_scan");
   return 0;
 }
 
 extern "C" int ra_delta_rule_prepare(const void* proj, int act_dtype, int ld, const float* filt, float* state,
                                      long slot_stride, long tail_off, const int* seq_of_token, const int* cu_tokens,
-                                     const int* state_slots, const int* fresh, int n_seqs, int n_tokens,
+                                     const int* state_slots, const int* fresh, int n_seqs, int n_tokens, int max_q_len,
                                      int key_heads, int key_dim, int heads, int value_dim, int taps, float unit_eps,
                                      float q_scale, float* qkv, hipStream_t stream) {
   RA_CHECK(n_seqs > 0 && n_tokens > 0 && heads > 0 && key_heads > 0, "delta_rule_prepare: %d requests, %d tokens",
@@ -848,6 +1039,7 @@ extern "C" int ra_delta_rule_prepare(const void* proj, int act_dtype, int ld, co
   const bool in_runs = taps <= PREP_TAPS && widest <= 256 && key_dim % 4 == 0 && value_dim % 4 == 0 && ld % 4 == 0 &&
                        (uintptr_t)proj % (act_dtype == RA_F32 ? 16 : 8) == 0 && (uintptr_t)qkv % 16 == 0 &&
                        runs.y <= 65535 && (long)runs.x * runs.y >= 2L * ra_cu_count();
+  const bool single = max_q_len == 1 && !in_runs;
 #define RA_DR(TA, LANES)                                                                                            \
   delta_rule_prepare_run_kernel<TA, LANES><<<runs, 256, 0, stream>>>(                                               \
       (const TA*)proj, ld, filt, state, slot_stride, tail_off, seq_of_token, cu_tokens, state_slots, fresh, key_heads, \
@@ -859,8 +1051,8 @@ extern "C" int ra_delta_rule_prepare(const void* proj, int act_dtype, int ld, co
     else if (in_runs) RA_DR(TA, 64);                                                                                \
     else delta_rule_prepare_kernel<TA><<<blocks, PREP_WAVES * RA_WAVE, 0, stream>>>(                                     \
         (const TA*)proj, ld, filt, state, slot_stride, tail_off, seq_of_token, cu_tokens, state_slots, fresh,       \
-        key_heads, key_dim, heads, value_dim, taps, unit_eps, q_scale, qkv, n_tokens);                              \
-    if (taps > 1)                                                                                                   \
+        key_heads, key_dim, heads, value_dim, taps, unit_eps, q_scale, qkv, n_tokens, single);                      \
+    if (taps > 1 && !single)                                                                                                   \
       delta_rule_tail_kernel<TA><<<tail_grid, 256, 0, stream>>>((const TA*)proj, ld, state, slot_stride, tail_off,  \
                                                                 cu_tokens, state_slots, fresh, C, taps);            \
   } while (0)
@@ -885,10 +1077,13 @@ extern "C" int ra_delta_rule_scan(const float* qkv, int ld, float* gates, const 
   RA_CHECK(slot_stride >= (long)heads * g.waves * g.wave_floats, "delta_rule_scan: a state slot of %ld floats, need %ld",
            slot_stride, (long)heads * g.waves * g.wave_floats);
   RA_CHECK(heads <= 65535, "delta_rule_scan: %d heads in one launch", heads);
-  const long n = (long)n_tokens * 2 * heads;
-  delta_rule_gates_kernel<<<(unsigned)((n + 255) / 256), 256, 0, stream>>>(gates, a_log, dt_bias, heads, n);
-  RA_LAUNCH_CHECK("delta_rule_gates");
-  if (scratch) {
+  const bool single = max_q_len == 1 && !(scratch && chunk_from <= 1);      // (chunks of every portion may be asked for)
+  if (!single) {
+    const long n = (long)n_tokens * 2 * heads;
+    delta_rule_gates_kernel<<<(unsigned)((n + 255) / 256), 256, 0, stream>>>(gates, a_log, dt_bias, heads, n);
+    RA_LAUNCH_CHECK("delta_rule_gates");
+  }
+  if (scratch && !single) {
     const int rc = ra_delta_rule_chunks(qkv, ld, gates, state, slot_stride, cu_tokens, state_slots, fresh, n_seqs, n_tokens,
                                         heads, key_heads, key_dim, value_dim, scratch, scratch_floats, chunk_from, out, stream);
     if (rc != 0 || chunk_from <= 1) return rc;
@@ -902,8 +1097,10 @@ extern "C" int ra_delta_rule_scan(const float* qkv, int ld, float* gates, const 
   a.ld = ld; a.q_heads = key_heads; a.gates = gates; a.state = state; a.slot_stride = slot_stride;
   a.cu_tokens = cu_tokens; a.state_slots = state_slots; a.fresh = fresh;
   a.H = heads; a.dk = key_dim; a.dv = value_dim; a.waves_per_head = g.waves; a.wave_floats = g.wave_floats;
-  a.chunk = L.chunk; a.below = scratch ? chunk_from : 0; a.q_scale = 1.f; a.denom_eps = 0.f; a.out = out;
-  scan_dispatch<float, SCAN_DELTA>(g, L, a, stream);
+  a.chunk = L.chunk; a.below = scratch && !single ? chunk_from : 0; a.q_scale = 1.f; a.denom_eps = 0.f; a.out = out;
+  const TokenGates tg = {gates, a_log, dt_bias, 0.f,
+                         key_dim == g.R * g.NPL && ra_rows_16b(a.k, ld, 4) && ra_rows_16b(a.q, ld, 4) && key_dim % 4 == 0};
+  scan_dispatch<float, SCAN_DELTA>(g, L, a, stream, single ? &tg : nullptr);
   RA_LAUNCH_CHECK("delta_rule_scan");
   return 0;
 }
@@ -1105,7 +1302,16 @@ extern "C" int ra_normed_mean(const void* const* xs, const float* const* ws, int
     in.w[i] = i < n ? ws[i] : nullptr;
   }
   const int threads = hidden >= 2048 ? 512 : 256;
-#define RA_NM(TA, N) normed_mean_kernel<TA, N><<<n_tokens, threads, 0, stream>>>(in, eps, hidden, (TA*)out, resid, scale)
+  const long lds = (long)n * hidden * (long)sizeof(float);
+  bool held = hidden % 8 == 0 && hidden <= 16 * threads && lds <= MEAN_LDS && (uintptr_t)out % 16 == 0 && (uintptr_t)resid % 16 == 0;
+  for (int i = 0; i < n; ++i) held = held && (uintptr_t)xs[i] % 16 == 0 && (uintptr_t)ws[i] % 16 == 0;
+#define RA_NM(TA, N)                                                                                                       \
+  do {                                                                                                                     \
+    if (held)                                                                                                              \
+      normed_mean_kernel<TA, N, true><<<n_tokens, threads, (size_t)lds, stream>>>(in, eps, hidden, (TA*)out, resid, scale); \
+    else                                                                                                                   \
+      normed_mean_kernel<TA, N, false><<<n_tokens, threads, 0, stream>>>(in, eps, hidden, (TA*)out, resid, scale);         \
+  } while (0)
 #define RA_NM_N(TA)                 \
   do {                              \
     if (n == 1) RA_NM(TA, 1);       \

@@ -89,8 +89,8 @@ int ra_moe_grouped(const void* x, int ldx, const void* w_up, const void* w_down,
                    const float* more, const float* more_logit, int ld_logit, float* resid, void* out, float alpha,
                    void* scratch, long scratch_bytes, hipStream_t stream);
 
-// float operands and result, to float precision on the bfloat16 matrix cores (each float in three parts), for rows that are whole 16-byte pieces (ra_gemm_f32_supports):
-// C[M, N] = A . W^T (+ bias). scratch: ra_gemm_f32_scratch floats (0: none needed).
+// float operands and result, to float precision on the bfloat16 matrix cores (each float in three parts), for rows that are
+// whole 16-byte pieces (ra_gemm_f32_supports): C[M, N] = A . W^T (+ bias). scratch: ra_gemm_f32_scratch floats (0: none needed).
 int ra_gemm_f32_supports(const void* A, const void* W, int K, int lda);
 long ra_gemm_f32_scratch(int M, int N, int K);
 int ra_gemm_f32(const float* A, const float* W, const float* bias, float* C, int M, int N, int K, int lda, int ldc,
@@ -400,9 +400,10 @@ int ra_matrix_memory_scan(const void* proj, int act_dtype, int ld, int q_off, in
 // the filter's tail lies at tail_off floats in a request's state slot; qkv float [n_tokens, channels]
 int ra_delta_rule_prepare(const void* proj, int act_dtype, int ld, const float* filt, float* state, long slot_stride,
                           long tail_off, const int* seq_of_token, const int* cu_tokens, const int* state_slots,
-                          const int* fresh, int n_seqs, int n_tokens, int key_heads, int key_dim, int heads,
-                          int value_dim, int taps, float unit_eps, float q_scale, float* qkv, hipStream_t stream);
-// gates [n_tokens, 2 heads] float pre-activations (b | a), turned into (beta | decay) in place; scratch and chunk_from as above
+                          const int* fresh, int n_seqs, int n_tokens, int max_q_len, int key_heads, int key_dim,
+                          int heads, int value_dim, int taps, float unit_eps, float q_scale, float* qkv, hipStream_t stream);
+// gates [n_tokens, 2 heads] float pre-activations (b | a), turned into (beta | decay) in place where max_q_len is not 1; scratch and
+// chunk_from as above
 int ra_delta_rule_scan(const float* qkv, int ld, float* gates, const float* a_log, const float* dt_bias, float* state,
                        long slot_stride, const int* cu_tokens, const int* state_slots, const int* fresh, int n_seqs,
                        int n_tokens, int max_q_len, int heads, int key_heads, int key_dim, int value_dim, float* scratch,

@@ -1272,15 +1272,15 @@ class HipKernels:
         library.call("ra_delta_rule_prepare", proj.data_ptr(), _tag(proj, "delta_rule_prepare"), proj.stride(0),
                      filt.data_ptr(), state.data_ptr(), state.stride(0), int(tail_off), batch.seq_of_token.data_ptr(),
                      batch.cu_tokens.data_ptr(), batch.state_slots.data_ptr(), batch.fresh.data_ptr(), batch.num_seqs,
-                     T, int(key_heads), int(key_dim), int(heads), int(value_dim), int(taps), float(unit_eps),
-                     float(q_scale), qkv.data_ptr(), _stream())
+                     T, int(getattr(batch, "max_q_len", 0) or 0), int(key_heads), int(key_dim), int(heads), int(value_dim),
+                     int(taps), float(unit_eps), float(q_scale), qkv.data_ptr(), _stream())
 
     def delta_rule_scan(self, qkv: torch.Tensor, gates: torch.Tensor, a_log: torch.Tensor, dt_bias: torch.Tensor,
                         state: torch.Tensor, batch, heads: int, key_heads: int, key_dim: int, value_dim: int,
                         out: torch.Tensor, chunks: Optional[bool] = None) -> None:
         """The gated delta rule over the step's tokens from and into ``state``. ``qkv`` float32 [T, q | k | v]
         as ``delta_rule_prepare`` left it; ``gates`` float32 [T, 2 heads] holds the pre-activations of beta
-        and of the decay and is overwritten with both; ``out`` float32 [T, heads * value_dim]. ``chunks`` forces the form
+        and of the decay and is overwritten with both (left as it is in a step of single tokens); ``out`` float32 [T, heads * value_dim]. ``chunks`` forces the form
         (None: by a request's own portion)."""
         _dev(qkv, gates, a_log, dt_bias, state, out)
         T = qkv.shape[0]
