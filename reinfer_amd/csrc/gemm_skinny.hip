@@ -351,11 +351,21 @@ gemm_skinny_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __restri
 //  - the run DEPTH ahead is asked for as soon as a run's registers are free.
 // A tile's runs are padded to a multiple of DEPTH (runs of zeros), so that a tile ends where a round
 // of the ring ends. MROWS = rows of A that are loaded (4, 8 or 16: the least that holds M).
-template <int NT, int WAVES, int U, int DEPTH, int OCC, int MROWS, int EPI, typename TO>
+//
+// PAIR: a second matrix over the same rows, with a float result, whose tiles come behind the first one's: the few features beside a
+// wide projection that are kept in float (a router's logits, a recurrent layer's gates), which as a product of their own are
+// all start and end (32 or 16 features over 4096 at 8 rows in a decode step: 6.2 and 5.5 us; behind 12288 or 36864 others 0.3).
+// Both results have the bits of two launches.
+struct SkinnySecond {
+  const bf16_t* W;
+  float* C;
+  int N, ldc;
+};
+template <int NT, int WAVES, int U, int DEPTH, int OCC, int MROWS, int EPI, typename TO, bool PAIR = false>
 __global__ void __launch_bounds__(WAVES * RA_WAVE, OCC)
 gemm_skinny_deep_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
                         const bf16_t* __restrict__ bias, TO* __restrict__ C, int ldc, int M, int N, int K,
-                        SkinnyNorm nf) {
+                        SkinnyNorm nf, SkinnySecond second = {}) {
   constexpr int MT = (MROWS + 15) / 16;            // row tiles of A
   constexpr int KS = U * 32;
   constexpr int LPR = U * 4;
@@ -381,12 +391,14 @@ gemm_skinny_deep_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __r
   const int n_steps = (K + span - 1) / span;
   const int n_steps_p = (n_steps + DEPTH - 1) / DEPTH * DEPTH;
   const int n_tiles = (N + 16 * NT - 1) / (16 * NT);
+  const int tiles = PAIR ? n_tiles + (second.N + 16 * NT - 1) / (16 * NT) : n_tiles;
+  const int past = n_tiles * 16 * NT;                  // features from here on are the second matrix's
   const int stride_n = (int)gridDim.x * 16 * NT;
-  const int n_mine = (n_tiles - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;
+  const int n_mine = (tiles - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;
   const int total = n_mine * n_steps_p;
   // Workgroups start their walk over K at different runs and wrap round where many run side by side:
   // in step, the rows read at one moment, a whole K apart, fall on few memory channels.
-  const int rot = (n_tiles > 512 || K > 8192) ? (int)((blockIdx.x * 7u) % (unsigned)n_steps) : 0;
+  const int rot_own = (n_tiles > 512 || K > 8192) ? (int)((blockIdx.x * 7u) % (unsigned)n_steps) : 0;
 
   // Both operands are read through buffer descriptors: a load whose offset lies past the descriptor's end
   // returns zeros and touches no memory, so rows past N or M, chunks past K, padding runs and runs past
@@ -396,6 +408,8 @@ gemm_skinny_deep_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __r
       __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(W), 0, (int)((size_t)N * K * 2), 0x00020000);
   const __amdgpu_buffer_rsrc_t a_rsrc =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(A), 0, (int)(((size_t)(M - 1) * lda + K) * 2), 0x00020000);
+  const __amdgpu_buffer_rsrc_t w2_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<bf16_t*>(PAIR ? second.W : W), 0, (int)((size_t)(PAIR ? second.N : N) * K * 2), 0x00020000);
   unsigned a_off[MI];                      // byte offset of this lane's chunk in run 0, or NOWHERE
 #pragma unroll
   for (int i = 0; i < MI; ++i) {
@@ -461,6 +475,11 @@ gemm_skinny_deep_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __r
   // `d` is a constant after unrolling: the ring of registers is indexed statically
 #define RA_DEEP_LOAD(d)                                                                        \
   do {                                                                                         \
+    const bool two_ = PAIR && l_n0 >= past;                                                    \
+    /* the second matrix's walk starts where a launch of its own would have it start */        \
+    const int rot = !two_ ? rot_own : K > 8192 ? (int)((unsigned)((l_n0 - past) / (16 * NT)) * 7u % (unsigned)n_steps) : 0; \
+    const __amdgpu_buffer_rsrc_t rsrc_ = two_ ? w2_rsrc : w_rsrc;                              \
+    const int first_ = two_ ? l_n0 - past : l_n0, N_ = two_ ? second.N : N;                    \
     int kk_ = K;                          /* a padding run, or past the end: nothing is read */ \
     if (l_q < total && l_step < n_steps) {                                                     \
       const int q_ = l_step + rot < n_steps ? l_step + rot : l_step + rot - n_steps;           \
@@ -469,9 +488,9 @@ gemm_skinny_deep_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __r
     const bool ok_ = kk_ < K;             /* K is a multiple of 8: a chunk is in or out as a whole */ \
     _Pragma("unroll") for (int nt = 0; nt < NT; ++nt)                                          \
       _Pragma("unroll") for (int i = 0; i < NI; ++i) {                                         \
-        const int n_ = l_n0 + nt * 16 + i * RPI + lr;                                          \
-        const unsigned off_ = (ok_ && n_ < N) ? (unsigned)(((size_t)n_ * K + kk_) * 2) : NOWHERE; \
-        wr[d][nt][i] = __builtin_bit_cast(bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, off_, 0, 0)); \
+        const int n_ = first_ + nt * 16 + i * RPI + lr;                                        \
+        const unsigned off_ = (ok_ && n_ < N_) ? (unsigned)(((size_t)n_ * K + kk_) * 2) : NOWHERE; \
+        wr[d][nt][i] = __builtin_bit_cast(bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(rsrc_, off_, 0, 0)); \
       }                                                                                        \
     _Pragma("unroll") for (int i = 0; i < MI; ++i) {                                           \
       const unsigned off_ = (ok_ && a_off[i] != NOWHERE) ? a_off[i] + (unsigned)(kk_ - lc * 8) * 2u : NOWHERE; \
@@ -558,7 +577,11 @@ gemm_skinny_deep_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __r
     } else {
       pre.have_c = pre.have_w = false;      // only the first tile's values were asked for ahead
     }
-    skinny_finish<MT, NT, WAVES, EPI, TO>(acc, ss_held, pre, red, row_ss, bias, C, ldc, M, N, c_n0, nf);
+    if (PAIR && c_n0 >= past)
+      skinny_finish<MT, NT, WAVES, EPI_PLAIN, float>(acc, ss_held, pre, red, row_ss, nullptr, second.C, second.ldc, M, second.N,
+                                                     c_n0 - past, nf);
+    else
+      skinny_finish<MT, NT, WAVES, EPI, TO>(acc, ss_held, pre, red, row_ss, bias, C, ldc, M, N, c_n0, nf);
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
@@ -628,6 +651,24 @@ static int launch_deep_rows(const void* A, int lda, const void* W, const void* b
   if (runs64 * 512 < runs128 * 1024)
     return launch_deep<1, 8, 2, 2, 2, MROWS>(A, lda, W, bias, C, ldc, out_dtype, epilogue, M, N, K, nf, grid, stream);
   return launch_deep<1, 8, 4, 2, 2, MROWS>(A, lda, W, bias, C, ldc, out_dtype, epilogue, M, N, K, nf, grid, stream);
+}
+
+// The same with a second matrix behind the first one's features. The grid is what the first one alone gets where that fills the chip,
+// so a tile's walk over K starts where it would.
+template <int MROWS>
+static int launch_pair(const void* A, int lda, const void* W, void* C, int ldc, int M, int N, int K, const SkinnySecond& second,
+                       hipStream_t stream) {
+  const int tiles = (N + 15) / 16 + (second.N + 15) / 16, cus = skinny_cus(), grid = tiles < 2 * cus ? tiles : 2 * cus;
+  const SkinnyNorm nf = {};
+  const int runs128 = (K + 1023) / 1024, runs64 = (K + 511) / 512;
+  if (runs64 * 512 < runs128 * 1024)
+    gemm_skinny_deep_kernel<1, 8, 2, 2, 2, MROWS, EPI_PLAIN, bf16_t, true><<<grid, 8 * RA_WAVE, 0, stream>>>(
+        (const bf16_t*)A, lda, (const bf16_t*)W, nullptr, (bf16_t*)C, ldc, M, N, K, nf, second);
+  else
+    gemm_skinny_deep_kernel<1, 8, 4, 2, 2, MROWS, EPI_PLAIN, bf16_t, true><<<grid, 8 * RA_WAVE, 0, stream>>>(
+        (const bf16_t*)A, lda, (const bf16_t*)W, nullptr, (bf16_t*)C, ldc, M, N, K, nf, second);
+  RA_LAUNCH_CHECK("gemm_skinny_pair");
+  return 0;
 }
 
 extern "C" int ra_gemm_skinny_max_rows(void) { return 64; }
@@ -718,4 +759,24 @@ extern "C" int ra_gemm_skinny_scaled(const void* A, const void* W, float* C, int
                                      float acc_scale, hipStream_t stream) {
   return gemm_skinny_impl(A, W, nullptr, C, RA_F32, EPI_ACCUM, M, N, K, lda, ldc, nullptr, 0, 0.f, 0, nullptr,
                           0, nullptr, 0, nullptr, acc_scale, stream);
+}
+
+// C = A . W^T in bfloat16 and C2 = A . W2^T in float, in one launch: up to 16 rows.
+extern "C" int ra_gemm_skinny_pair(const void* A, const void* W, void* C, const void* W2, float* C2, int M, int N, int N2, int K,
+                                   int lda, int ldc, int ldc2, hipStream_t stream) {
+  RA_CHECK(M > 0 && N > 0 && N2 > 0 && K > 0, "gemm_skinny_pair: empty product (%d, %d and %d, %d)", M, N, N2, K);
+  RA_CHECK(M <= 16, "gemm_skinny_pair: %d rows; this kernel takes at most 16", M);
+  RA_CHECK(K % 8 == 0 && lda % 8 == 0, "gemm_skinny_pair: K (%d) and the row stride (%d) must be multiples of 8", K, lda);
+  RA_CHECK(lda >= K && ldc >= N && ldc2 >= N2, "gemm_skinny_pair: row strides (%d, %d, %d) below the row lengths (%d, %d, %d)", lda,
+           ldc, ldc2, K, N, N2);
+  RA_CHECK(((uintptr_t)A % 16) == 0 && ((uintptr_t)W % 16) == 0 && ((uintptr_t)W2 % 16) == 0,
+           "gemm_skinny_pair: operands must be 16-byte aligned");
+  // the second one's tiles must have a workgroup each in a launch of their own, whose starts they take over
+  RA_CHECK((N2 + 15) / 16 <= skinny_cus(), "gemm_skinny_pair: %d features of the second matrix", N2);
+  RA_CHECK(((size_t)N + N2) * K * 2 < 0xFFFFFF00ull && ((size_t)(M - 1) * lda + K) * 2 < 0xFFFFFF00ull,
+           "gemm_skinny_pair: [%d and %d, %d] is too large to address", N, N2, K);
+  const SkinnySecond second = {(const bf16_t*)W2, C2, N2, ldc2};
+  if (M <= 4) return launch_pair<4>(A, lda, W, C, ldc, M, N, K, second, stream);
+  if (M <= 8) return launch_pair<8>(A, lda, W, C, ldc, M, N, K, second, stream);
+  return launch_pair<16>(A, lda, W, C, ldc, M, N, K, second, stream);
 }

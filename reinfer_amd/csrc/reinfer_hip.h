@@ -281,6 +281,12 @@ int ra_moe_topk(const float* logits, int ld, int experts, int top, int* ids, flo
 // act[t, e * ff + j] = weight(t, e) * relu(up[t, e * ff + j])^2 for chosen experts, 0 for the others
 int ra_moe_relu2_scale(const void* up, void* act, int act_dtype, const int* ids, const float* weights, int top,
                        int experts, int ff, int n_tokens, hipStream_t stream);
+// The choice by float logits (rows ld apart) and the activation with its weights in one kernel: gated ([gate | up] of each expert, sigmoid
+// scores, groups, a shared expert) as ra_moe_route_sigmoid and ra_moe_silu_gate_scale, else as ra_moe_topk and ra_moe_relu2_scale
+int ra_moe_choose_scale_takes(const void* up, const void* act, int act_dtype, int top, int experts, int groups, int ff, int shared,
+                              int n_tokens);
+int ra_moe_choose_scale(const void* up, void* act, int act_dtype, int gated, const float* logits, int ld, int top, int experts,
+                        int groups, int kept, int group_top, float scale, int ff, int shared, int n_tokens, hipStream_t stream);
 
 // Few tokens: only the chosen experts' rows are read. w_up [experts * ff, width], w_down [width, experts * ff];
 // act[t * top + j, f] = weights[t, j] * relu(w_up[ids[t, j] * ff + f, :] . x[t, :])^2, then
@@ -350,6 +356,9 @@ int ra_turn_heads(void* x, int act_dtype, long ld, int n_tokens, int heads, int 
 // ra_gemm_skinny / ra_gemm_wide with the accumulating epilogue)
 int ra_gemm_skinny_scaled(const void* A, const void* W, float* C, int M, int N, int K, int lda, int ldc,
                           float acc_scale, hipStream_t stream);
+// up to 16 rows: C = A . W^T in bfloat16 and C2 = A . W2^T in float, W2 of at most 16 features a CU, in one launch
+int ra_gemm_skinny_pair(const void* A, const void* W, void* C, const void* W2, float* C2, int M, int N, int N2, int K, int lda,
+                        int ldc, int ldc2, hipStream_t stream);
 int ra_gemm_wide_scaled(const void* A, const void* W, float* C, int M, int N, int K, int lda, int ldc, float* scratch,
                         long scratch_floats, float acc_scale, hipStream_t stream);
 

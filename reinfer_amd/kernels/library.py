@@ -45,6 +45,7 @@ _SIGNATURES = {
     "ra_gemm_wide_normed": [P, P, P, P, I, I, I, I, I, I, I, P, c_long, P, I, F, I, P, I, P, I, P, F, P],
     "ra_gemm_skinny_normed": [P, P, P, P, I, I, I, I, I, I, I, P, I, F, I, P, I, P, I, P, P],
     "ra_gemm_skinny_scaled": [P, P, P, I, I, I, I, I, F, P],
+    "ra_gemm_skinny_pair": [P, P, P, P, P, I, I, I, I, I, I, I, P],
     "ra_gemm_prompt": [P, P, P, I, I, I, I, I, I, F, I, I, I, P],
     "ra_gemm_wide_scaled": [P, P, P, I, I, I, I, I, P, c_long, F, P],
     "ra_gemm_plain": [P, P, P, P, I, I, I, I, I, I, I, P],
@@ -70,6 +71,7 @@ _SIGNATURES = {
     "ra_tanh_rows": [P, I, c_long, P],
     "ra_moe_topk": [P, I, I, I, P, P, I, P],
     "ra_moe_relu2_scale": [P, P, I, P, P, I, I, I, I, P],
+    "ra_moe_choose_scale": [P, P, I, I, P, I, I, I, I, I, I, F, I, I, I, P],
     "ra_moe_up_chosen": [P, I, P, P, P, P, I, I, I, I, I, I, P],
     "ra_moe_down_chosen": [P, P, P, P, P, I, I, I, I, I, I, P],
     "ra_moe_gate_up_chosen": [P, I, P, P, P, P, I, P, I, I, I, I, I, I, I, P],
@@ -144,6 +146,8 @@ def load() -> ctypes.CDLL:
         lib.ra_scan_state_floats.argtypes = [c_int, c_int, c_int, c_int]
         lib.ra_moe_grouped_scratch.restype = c_long
         lib.ra_moe_grouped_scratch.argtypes = [I, I, I, I, I]
+        lib.ra_moe_choose_scale_takes.restype = c_int
+        lib.ra_moe_choose_scale_takes.argtypes = [P, P, I, I, I, I, I, I, I]
         lib.ra_gemm_f32_supports.restype = c_int
         lib.ra_gemm_f32_supports.argtypes = [P, P, I, I]
         lib.ra_gemm_f32_scratch.restype = c_long

@@ -753,6 +753,31 @@ class HipKernels:
             return self.linear_f32(x, weight, out, bias)
         self.linear_plain(x, weight, out, bias)
 
+    # Features of the second product of a pair up to which its tiles have a workgroup each, whatever the chip.
+    PAIR_FEATURES = 1024
+
+    def linear_pair(self, x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, weight2: torch.Tensor,
+                    out2: torch.Tensor) -> None:
+        """``linear(x, weight, out)`` and ``linear(x, weight2, out2)``, the same bits. With up to 16 rows a bfloat16 product and a narrow
+        one beside it with a float result (a router's logits, a recurrent layer's gates) are one launch: as one of its
+        own the narrow one is all start and end (8 rows of 4096, 32 features: 6.2 us in a decode step)."""
+        M, K = x.shape
+        if M <= 16 and x.is_cuda and x.dtype == weight.dtype == weight2.dtype == out.dtype == torch.bfloat16 \
+                and out2.dtype == torch.float32 and weight2.shape[0] <= self.PAIR_FEATURES and K % 8 == 0 \
+                and x.stride(0) % 8 == 0 and x.stride(0) >= K and all(t.data_ptr() % 16 == 0 for t in (x, weight, weight2)) \
+                and (weight.shape[0] + weight2.shape[0]) * K < 1 << 30 and x.stride(0) < 1 << 26:
+            self._check_linear(x, weight, out, None)
+            self._check_linear(x, weight2, out2, None)
+            lib = library.load()
+            N, N2 = weight.shape[0], weight2.shape[0]
+            if not lib.ra_gemm_wide_preferred(0, M, N, K) and not lib.ra_gemm_wide_preferred(0, M, N2, K) \
+                    and out.stride(0) >= N and out2.stride(0) >= N2:
+                library.call("ra_gemm_skinny_pair", x.data_ptr(), weight.data_ptr(), out.data_ptr(), weight2.data_ptr(),
+                             out2.data_ptr(), M, N, N2, K, x.stride(0), out.stride(0), out2.stride(0), _stream())
+                return
+        self.linear(x, weight, out)
+        self.linear(x, weight2, out2)
+
     def linear_columns(self, x: torch.Tensor, weight: torch.Tensor, first: int, out: torch.Tensor) -> None:
         """out = x . weight[:, first:]^T for bfloat16 ``x`` and ``weight`` and a float32 ``out``, by the library's product, which
         reads a range of a wider matrix's columns as fast as a matrix of their own (4096 x 2048 of 18432: 35 us at 1859 rows)."""
@@ -1765,6 +1790,39 @@ class HipKernels:
             raise ValueError("moe_relu2_scale: ids int32 and weights float32, both [T, top]")
         library.call("ra_moe_relu2_scale", up.data_ptr(), act.data_ptr(), _tag(up, "moe_relu2_scale"), ids.data_ptr(),
                      weights.data_ptr(), top, int(experts), int(ff), T, _stream())
+
+    def moe_choose_scale(self, up: torch.Tensor, act: torch.Tensor, logits: torch.Tensor, top: int, experts: int, ff: int,
+                         shared: int = 0, scoring: str = "softmax_chosen", scale: float = 1.0, groups: int = 1,
+                         groups_kept: int = 1, group_top: int = 2) -> None:
+        """The choice of :meth:`moe_route` by its float32 ``logits`` [T, >= experts] and the activation of all experts' products with
+        its weights, :meth:`moe_silu_gate_scale` ("sigmoid") or :meth:`moe_relu2_scale` ("softmax_chosen"): one kernel
+        where rows are 16-byte pieces, else two."""
+        gated = scoring == "sigmoid"
+        if not gated and (scoring != "softmax_chosen" or shared or groups != 1):
+            raise ValueError(f"moe_choose_scale: scoring {scoring!r}, shared {shared}, {groups} groups")
+        _dev(up, act, logits)
+        T, n = up.shape[0], experts * ff + shared
+        if up.shape != (T, (2 if gated else 1) * n) or act.shape != (T, n) or act.dtype != up.dtype or not up.is_contiguous() \
+                or not act.is_contiguous():
+            raise ValueError(f"moe_choose_scale: up {tuple(up.shape)}, act {tuple(act.shape)} for {experts} experts of {ff}, shared {shared}")
+        if logits.dtype != torch.float32 or logits.dim() != 2 or logits.shape[0] != T or logits.shape[1] < experts or logits.stride(1) != 1:
+            raise ValueError(f"moe_choose_scale: logits float32 [{T}, >= {experts}]")
+        tag = _tag(up, "moe_choose_scale")
+        if library.load().ra_moe_choose_scale_takes(up.data_ptr(), act.data_ptr(), tag, int(top), int(experts), int(groups), int(ff),
+                                                    int(shared), T):
+            library.call("ra_moe_choose_scale", up.data_ptr(), act.data_ptr(), tag, int(gated), logits.data_ptr(), logits.stride(0),
+                         int(top), int(experts), int(groups), int(groups_kept), int(group_top), float(scale), int(ff), int(shared),
+                         T, _stream())
+            return
+        ids = torch.empty((T, top), dtype=torch.int32, device=up.device)
+        weights = torch.empty((T, top), dtype=torch.float32, device=up.device)
+        if gated:
+            library.call("ra_moe_route_sigmoid", logits.data_ptr(), logits.stride(0), int(experts), int(top), int(groups),
+                         int(groups_kept), int(group_top), float(scale), ids.data_ptr(), weights.data_ptr(), T, _stream())
+            return self.moe_silu_gate_scale(up, act, ids, weights, experts, ff, shared)
+        library.call("ra_moe_topk", logits.data_ptr(), logits.stride(0), int(experts), int(top), ids.data_ptr(), weights.data_ptr(), T,
+                     _stream())
+        self.moe_relu2_scale(up, act, ids, weights, experts, ff)
 
     # Steps of so few tokens that their choices name at most this share of the experts read only the chosen
     # experts' rows (two kernels, a wave a row) instead of running every expert through the matrix cores

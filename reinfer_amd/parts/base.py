@@ -218,6 +218,15 @@ def project_out(ops, x: torch.Tensor, weight: torch.Tensor, resid: Optional[torc
     return out
 
 
+def linear_both(ops, x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, weight2: torch.Tensor, out2: torch.Tensor) -> None:
+    """Two products over the same rows, the second narrow and kept in float: one launch where the kernel set has it."""
+    if hasattr(ops, "linear_pair"):
+        ops.linear_pair(x, weight, out, weight2, out2)
+    else:
+        ops.linear(x, weight, out)
+        ops.linear(x, weight2, out2)
+
+
 def split_input(x):
     """(tensor, row sums or None) of a part's input, plain or :class:`RowScaled`."""
     if isinstance(x, RowScaled):

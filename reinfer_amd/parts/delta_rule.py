@@ -23,7 +23,7 @@ import torch
 from .. import kernels
 from ..config.schema import MixerSpec
 from ..weights import VECTOR, ParamDecl
-from .base import LayerCache, StateNeed
+from .base import LayerCache, StateNeed, linear_both
 from .registry import register_mixer
 
 
@@ -81,9 +81,8 @@ class GatedDeltaRule:
         T = x.shape[0]
         H, G, dk, dv = self.heads, self.key_heads, self.key_dim, self.value_dim
         proj = torch.empty((T, self.in_width), dtype=self.dtype, device=x.device)
-        ops.linear(x, self.w_in, proj)
         ba = torch.empty((T, 2 * H), dtype=torch.float32, device=x.device)
-        ops.linear(x, self.w_ba, ba)
+        linear_both(ops, x, self.w_in, proj, self.w_ba, ba)
         # filter + silu + unit norms -> float q | k | v; the filter's tail in the state moves on
         qkv = torch.empty((T, self.channels), dtype=torch.float32, device=x.device)
         ops.delta_rule_prepare(proj, self.filter, cache.state, self.scan_floats, batch, G, dk, H, dv, self.taps,

@@ -24,7 +24,7 @@ import torch
 from .. import kernels
 from ..config.schema import MixerSpec
 from ..weights import VECTOR, ParamDecl
-from .base import LayerCache, StateNeed
+from .base import LayerCache, StateNeed, linear_both
 from .registry import register_mixer
 
 
@@ -74,9 +74,8 @@ class MatrixMemory:
         T = x.shape[0]
         H, dk, dv = self.heads, self.key_dim, self.value_dim
         proj = torch.empty((T, self.in_width), dtype=self.dtype, device=x.device)
-        ops.linear(x, self.w_in, proj)
         gates = torch.empty((T, 2 * H), dtype=torch.float32, device=x.device)
-        ops.linear(x, self.w_gates, gates)
+        linear_both(ops, x, self.w_in, proj, self.w_gates, gates)
         read = torch.empty((T, H * dv), dtype=torch.float32, device=x.device)
         ops.matrix_memory_scan(proj, self.offsets[0], self.offsets[1], self.offsets[2], gates, self.b_gates,
                                cache.state, batch, H, dk, dv, self.gate_cap, dk ** -0.5, self.denom_eps, read)

@@ -43,6 +43,7 @@ import torch
 from .. import kernels
 from ..config.schema import FeedForwardSpec
 from ..weights import INT_TABLE, VECTOR, ParamDecl
+from .base import linear_both
 from .registry import register_feed_forward
 
 
@@ -138,6 +139,12 @@ class MixtureOfExperts:
         p = self.routing
         T = x.shape[0]
         n = self.experts * self.ff + self.shared
+        if p.weights == "sigmoid" and self._together(ops, x, self.w_gate_up, self.experts):
+            gu = torch.empty((T, 2 * n), dtype=self.dtype, device=x.device)
+            act = self._choose_and_scale(ops, x, self.w_gate_up, gu, n, shared=self.shared, scoring="sigmoid",
+                                         scale=float(p.weight_scale), groups=int(p.groups), groups_kept=int(p.groups_kept),
+                                         group_top=int(p.group_top))
+            return self._project_down(ops, act, resid, resid_scale)
         ids = torch.empty((T, self.top), dtype=torch.int32, device=x.device)
         weights = torch.empty((T, self.top), dtype=torch.float32, device=x.device)
         routed = self.experts + self.identity
@@ -178,6 +185,9 @@ class MixtureOfExperts:
             ops.linear(act, self.w_down, out)
             ops.moe_identity_add(out, x, ids, weights, self.experts)
             return out
+        return self._project_down(ops, act, resid, resid_scale)
+
+    def _project_down(self, ops, act, resid, resid_scale=1.0):
         can_add = getattr(ops, "can_accumulate", None)
         if resid is not None and can_add and can_add(act, self.w_down):
             if resid_scale != 1.0:
@@ -185,9 +195,24 @@ class MixtureOfExperts:
             else:
                 ops.linear_skinny(act, self.w_down, resid, accumulate=True)
             return None
-        out = torch.empty((T, self.spec.hidden), dtype=self.dtype, device=x.device)
+        out = torch.empty((act.shape[0], self.spec.hidden), dtype=self.dtype, device=act.device)
         ops.linear(act, self.w_down, out)
         return out
+
+    def _together(self, ops, x, w_up, routed: int) -> bool:
+        """Whether a step runs every expert, so that its products do not wait for the choice: the router's logits come with them, and the
+        choice is made where it weighs them."""
+        if not hasattr(ops, "moe_choose_scale"):
+            return False
+        chosen = getattr(ops, "moe_reads_chosen", None)
+        return not (chosen is not None and chosen(x.shape[0], self.top, routed)) and not self._grouped(ops, x, w_up, routed)
+
+    def _choose_and_scale(self, ops, x, w_up, up, n, **choice):
+        logits = torch.empty((x.shape[0], self.router.shape[0]), dtype=torch.float32, device=x.device)
+        linear_both(ops, x, w_up, up, self.router, logits)
+        act = torch.empty((x.shape[0], n), dtype=self.dtype, device=x.device)
+        ops.moe_choose_scale(up, act, logits, self.top, self.experts, self.ff, **choice)
+        return act
 
     def _grouped(self, ops, x, w_up, routed: int) -> bool:
         groups = getattr(ops, "moe_groups", None)
@@ -220,6 +245,9 @@ class MixtureOfExperts:
         ops = kernels.current()
         T = x.shape[0]
         n = self.experts * self.ff
+        if self._together(ops, x, self.w_up, self.experts):
+            up = torch.empty((T, n), dtype=self.dtype, device=x.device)
+            return self._project_down(ops, self._choose_and_scale(ops, x, self.w_up, up, n), resid)
         ids = torch.empty((T, self.top), dtype=torch.int32, device=x.device)
         weights = torch.empty((T, self.top), dtype=torch.float32, device=x.device)
         ops.moe_route(x, self.router, self.top, ids, weights)
@@ -240,10 +268,4 @@ class MixtureOfExperts:
         ops.linear(x, self.w_up, up)
         act = torch.empty((T, n), dtype=self.dtype, device=x.device)
         ops.moe_relu2_scale(up, act, ids, weights, self.experts, self.ff)
-        can_add = getattr(ops, "can_accumulate", None)
-        if resid is not None and can_add and can_add(act, self.w_down):
-            ops.linear_skinny(act, self.w_down, resid, accumulate=True)
-            return None
-        out = torch.empty((T, self.spec.hidden), dtype=self.dtype, device=x.device)
-        ops.linear(act, self.w_down, out)
-        return out
+        return self._project_down(ops, act, resid)
