@@ -234,6 +234,11 @@ int ra_sample_static(const float* logits, int n_rows, int vocab, int row_stride,
 long ra_filter_scratch(int n_rows, int vocab);
 int ra_filter_logits(float* logits, int n_rows, int vocab, int row_stride, const void* rows,
                      const int* window, void* scratch, long scratch_bytes, hipStream_t stream);
+// A token a row of what ra_filter_logits would leave, as ra_sample draws it; the logits stay as they are (rows that change: `changed`)
+int ra_filter_slices(int vocab);
+int ra_sample_filtered(const float* logits, int n_rows, int vocab, int row_stride, const void* rows, const int* window,
+                       float* changed, int changed_stride, void* scratch, long scratch_bytes, const long long* seeds,
+                       const int* positions, float* scratch_val, int* scratch_idx, int* tokens, hipStream_t stream);
 
 // What the machine gives at best (peaks.hip; for measurement, not on the product path): one read of
 // `bytes` of device memory, and `iters` iterations of bfloat16 matrix-core products on registers

@@ -55,6 +55,15 @@ __device__ __forceinline__ Best block_best(Best b, Best* red) {
   return r;
 }
 
+// A finite logit of token v as the draw compares it: itself at T <= 0, else over T and with its noise. False: it never wins.
+__device__ __forceinline__ bool sample_value(float& x, int v, float T, unsigned long long base) {
+  if (!(T > 0.f)) return true;
+  const float u = (float)(mix64(base ^ mix64((unsigned long long)v)) >> 40) * (1.0f / 16777216.0f);
+  if (u <= 0.f) return false;            // -ln(-ln 0) = -inf
+  x = x / T - logf(-logf(u));
+  return true;
+}
+
 __global__ void sample_stage1(const float* __restrict__ logits, int vocab, int row_stride,
                               const float* __restrict__ temperature,
                               const long long* __restrict__ seeds, const int* __restrict__ positions,
@@ -72,11 +81,7 @@ __global__ void sample_stage1(const float* __restrict__ logits, int vocab, int r
   for (int v = slice * SAMPLE_SLICE + threadIdx.x; v < end; v += SAMPLE_THREADS) {
     float x = lg[v];
     if (!isfinite(x)) continue;
-    if (T > 0.f) {
-      const float u = (float)(mix64(base ^ mix64((unsigned long long)v)) >> 40) * (1.0f / 16777216.0f);
-      if (u <= 0.f) continue;            // -ln(-ln 0) = -inf: never wins
-      x = x / T - logf(-logf(u));
-    }
+    if (!sample_value(x, v, T, base)) continue;
     Best c;
     c.val = x;
     c.idx = v;
@@ -217,8 +222,11 @@ extern "C" int ra_sample_static(const float* logits, int n_rows, int vocab, int 
 //   5  one workgroup a row finds the exact boundaries among them;
 //   6  every slice removes what lies below.
 // One workgroup a row that bisected over the whole row, up to 94 passes, took 3.15 ms for 24 rows of 151936 however many
-// rows there were; the six launches take 73 us for them, each bound by its own start and one trip over the row (the two
-// with one workgroup a row 9 and 21 us).
+// rows there were; the six launches take 46 us for them, each bound by its own start and one trip over the row.
+// Where a token is drawn from the row at once (ra_sample_filtered) nothing is removed: the draw passes over what a filter would have
+// taken, and only rows that penalties or a bias change are copied, in the first pass. For those 24 rows, half of them changed, that
+// saves the copy of all rows, the last pass and a trip over memory each: 83 us of kernels
+// and copies, so 59. Windows of 64 are counted eight tokens at a time: the first pass 13.8 -> 8.5 us.
 // ---------------------------------------------------------------------------
 #define FILTER_THREADS 256
 #define FILTER_SLICE 4096        // 16 tokens a thread
@@ -273,6 +281,20 @@ __device__ __forceinline__ bool filter_uses(const FilterRow& fr, int vocab) {
   return fr.temperature > 0.f && ((fr.top_k > 0 && fr.top_k < vocab) || (fr.top_p > 0.f && fr.top_p < 1.f) || fr.min_p > 0.f);
 }
 
+__device__ __forceinline__ bool filter_penalises(const FilterRow& fr) {
+  return (fr.repeat_penalty > 1.f || fr.frequency_penalty > 0.f || fr.presence_penalty > 0.f) && fr.window_len > 0;
+}
+// The rows as they came, and those that the first pass changes, in a buffer of their own (null: changed where they are).
+struct FilterLogits {
+  const float* given;
+  float* changed;
+  int given_stride, changed_stride;
+};
+__device__ __forceinline__ const float* filter_row(const FilterLogits& l, const FilterRow& fr, int row) {
+  return l.changed && (filter_penalises(fr) || fr.bias_len > 0) ? l.changed + (size_t)row * l.changed_stride
+                                                                : l.given + (size_t)row * l.given_stride;
+}
+
 // A thread's 16 values of a slice, all asked for at once: value 4 q + e is token filter_at(from, q) + e. Past the row's end they
 // are no numbers, which every pass leaves alone. Rows on a 16-byte boundary are read 16 bytes at a time.
 __device__ __forceinline__ int filter_at(int from, int q) { return from + (q * FILTER_THREADS + (int)threadIdx.x) * 4; }
@@ -292,18 +314,33 @@ __device__ __forceinline__ void filter_read(const float* lg, int from, int to, f
   }
 }
 
+// Whether any of the window's tokens before `w` is `tok`, and how many are. Read eight at a time: with a loop that ends at the first
+// one every read waits for the one before it.
+__device__ __forceinline__ int filter_count(const int* win, int n, int w, int tok, bool* before) {
+  int cnt = 0, early = 0;
+#pragma unroll 8
+  for (int x = 0; x < n; ++x) {
+    const int same = win[x] == tok;
+    cnt += same;
+    early += same && x < w;
+  }
+  *before = early != 0;
+  return cnt;
+}
+
 __global__ void __launch_bounds__(FILTER_THREADS)
-filter_max_kernel(float* __restrict__ logits, int vocab, int row_stride, const FilterRow* __restrict__ rows,
-                  const int* __restrict__ window, float* __restrict__ slice_max) {
+filter_max_kernel(FilterLogits logits, int vocab, const FilterRow* __restrict__ rows, const int* __restrict__ window,
+                  float* __restrict__ slice_max) {
   __shared__ float red[FILTER_THREADS / RA_WAVE];
   __shared__ int near_window[FILTER_WINDOW];
   __shared__ float slice[FILTER_SLICE];
   const FilterRow fr = rows[blockIdx.y];
-  float* lg = logits + (size_t)blockIdx.y * row_stride;
+  const float* lg = logits.given + (size_t)blockIdx.y * logits.given_stride;
+  float* to_row = logits.changed ? logits.changed + (size_t)blockIdx.y * logits.changed_stride : const_cast<float*>(lg);
   const int tid = threadIdx.x, from = blockIdx.x * FILTER_SLICE, to = min(vocab, from + FILTER_SLICE);
   float l[16];
   filter_read(lg, from, to, l);              // asked for beside the row's options and its window
-  const bool pen = (fr.repeat_penalty > 1.f || fr.frequency_penalty > 0.f || fr.presence_penalty > 0.f) && fr.window_len > 0;
+  const bool pen = filter_penalises(fr);
   if (pen || fr.bias_len > 0) {
     // the slice's logits change in LDS and, where they do, in the row
 #pragma unroll
@@ -323,7 +360,10 @@ filter_max_kernel(float* __restrict__ logits, int vocab, int row_stride, const F
         const int tok = bp[2 * b];
         if (tok < from || tok >= to) continue;
         const float x = slice[tok - from];
-        if (isfinite(x)) lg[tok] = slice[tok - from] = x + __int_as_float(bp[2 * b + 1]);
+        if (isfinite(x)) {
+          slice[tok - from] = x + __int_as_float(bp[2 * b + 1]);
+          if (!logits.changed) to_row[tok] = slice[tok - from];
+        }
       }
       __syncthreads();
     }
@@ -332,25 +372,30 @@ filter_max_kernel(float* __restrict__ logits, int vocab, int row_stride, const F
       for (int w = tid; w < fr.window_len; w += FILTER_THREADS) {
         const int tok = win[w];
         if (tok < from || tok >= to) continue;
-        bool first = true;
-        int cnt = 0;
-        for (int x = 0; x < fr.window_len; ++x) {
-          if (win[x] == tok) {
-            if (x < w) { first = false; break; }
-            ++cnt;
-          }
-        }
-        if (!first) continue;
+        bool before;
+        const int cnt = filter_count(win, fr.window_len, w, tok, &before);
+        if (before) continue;
         float x = slice[tok - from];
         if (!isfinite(x)) continue;
         x -= fr.frequency_penalty * (float)cnt + fr.presence_penalty;
         if (fr.repeat_penalty > 1.f) x = x > 0.f ? x / fr.repeat_penalty : x * fr.repeat_penalty;
-        lg[tok] = slice[tok - from] = x;
+        slice[tok - from] = x;
+        if (!logits.changed) to_row[tok] = x;
       }
       __syncthreads();
     }
 #pragma unroll
     for (int i = 0; i < 16; ++i) l[i] = slice[filter_at(0, i >> 2) + (i & 3)];
+    if (logits.changed) {
+      const bool whole = (uintptr_t)to_row % 16 == 0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int v = filter_at(from, q);
+        if (whole && v + 3 < to) *(f32x4_t*)(to_row + v) = (f32x4_t){l[4 * q], l[4 * q + 1], l[4 * q + 2], l[4 * q + 3]};
+        else
+          for (int e = 0; e < 4 && v + e < to; ++e) to_row[v + e] = l[4 * q + e];
+      }
+    }
   }
   if (!filter_uses(fr, vocab)) return;
   float mx = -INFINITY;
@@ -374,14 +419,14 @@ __device__ __forceinline__ float filter_row_max(const float* slice_max, int slic
 }
 
 __global__ void __launch_bounds__(FILTER_THREADS)
-filter_bins_kernel(const float* __restrict__ logits, int vocab, int row_stride, const FilterRow* __restrict__ rows,
+filter_bins_kernel(FilterLogits logits, int vocab, const FilterRow* __restrict__ rows,
                    const float* __restrict__ slice_max, unsigned long long* __restrict__ mass,
                    unsigned* __restrict__ count, float unit) {
   __shared__ unsigned long long m[FILTER_BINS];
   __shared__ unsigned c[FILTER_BINS];
   const FilterRow fr = rows[blockIdx.y];
   if (!filter_uses(fr, vocab)) return;
-  const float* lg = logits + (size_t)blockIdx.y * row_stride;
+  const float* lg = filter_row(logits, fr, blockIdx.y);
   const int tid = threadIdx.x, from = blockIdx.x * FILTER_SLICE, to = min(vocab, from + FILTER_SLICE);
   const float mx = filter_row_max(slice_max + (size_t)blockIdx.y * gridDim.x, gridDim.x);
   if (mx == -INFINITY) return;               // no finite logit: ra_sample reports it
@@ -471,14 +516,15 @@ filter_plan_kernel(int vocab, const FilterRow* __restrict__ rows, const float* _
 }
 
 __global__ void __launch_bounds__(FILTER_THREADS)
-filter_list_kernel(const float* __restrict__ logits, int vocab, int row_stride, const FilterRow* __restrict__ rows,
+filter_list_kernel(FilterLogits logits, int vocab, const FilterRow* __restrict__ rows,
                    FilterPlan* __restrict__ plans, int* __restrict__ list) {
   __shared__ unsigned found, base;
   __shared__ int mine[FILTER_SLICE];
   const FilterPlan p = plans[blockIdx.y];
   if (p.mx == -INFINITY || (p.bin_k < 0 && p.bin_p0 < 0)) return;
-  const float* lg = logits + (size_t)blockIdx.y * row_stride;
-  const float T = rows[blockIdx.y].temperature;
+  const FilterRow fr = rows[blockIdx.y];
+  const float* lg = filter_row(logits, fr, blockIdx.y);
+  const float T = fr.temperature;
   const int tid = threadIdx.x, from = blockIdx.x * FILTER_SLICE, to = min(vocab, from + FILTER_SLICE);
   if (tid == 0) found = 0u;
   __syncthreads();
@@ -507,7 +553,7 @@ template <typename T> __device__ __forceinline__ T eight_sum(T v) {
 
 // One workgroup a row: the boundaries among the listed tokens, whose order on the list means nothing.
 __global__ void __launch_bounds__(FILTER_ROW_THREADS)
-filter_select_kernel(const float* __restrict__ logits, int vocab, int row_stride, const FilterRow* __restrict__ rows,
+filter_select_kernel(FilterLogits logits, int vocab, const FilterRow* __restrict__ rows,
                      FilterPlan* __restrict__ plans, const int* __restrict__ list, float unit) {
   __shared__ unsigned long long red[FILTER_ROW_THREADS / RA_WAVE];
   __shared__ unsigned long long keys[FILTER_SHORT], masses[FILTER_SHORT];
@@ -518,7 +564,7 @@ filter_select_kernel(const float* __restrict__ logits, int vocab, int row_stride
   const FilterPlan p = plans[blockIdx.x];
   if (p.mx == -INFINITY || (p.bin_k < 0 && p.bin_p0 < 0)) return;
   const FilterRow fr = rows[blockIdx.x];
-  const float* lg = logits + (size_t)blockIdx.x * row_stride;
+  const float* lg = filter_row(logits, fr, blockIdx.x);
   const int* mine = list + (size_t)blockIdx.x * vocab;
   const int tid = threadIdx.x, n = (int)p.listed;
   const bool is_short = n <= FILTER_SHORT;
@@ -613,6 +659,42 @@ filter_select_kernel(const float* __restrict__ logits, int vocab, int row_stride
   }
 }
 
+// Whether the filters leave token v, whose logit is finite (x: over the temperature).
+__device__ __forceinline__ bool filter_keeps(const FilterPlan& p, int v, float x) {
+  const float e = __expf(x - p.mx);
+  return e >= p.e_min && e >= p.theta && filter_key(v, x) >= p.key_min;
+}
+
+// sample_stage1 over the tokens that the filters leave.
+__global__ void __launch_bounds__(FILTER_THREADS)
+filter_draw_kernel(FilterLogits logits, int vocab, const FilterRow* __restrict__ rows, const FilterPlan* __restrict__ plans,
+                   const long long* __restrict__ seeds, const int* __restrict__ positions, float* __restrict__ part_val,
+                   int* __restrict__ part_idx) {
+  __shared__ Best red[FILTER_THREADS / RA_WAVE];
+  const int row = blockIdx.y;
+  const FilterRow fr = rows[row];
+  const FilterPlan p = plans[row];
+  const unsigned long long base =
+      splitmix64((unsigned long long)seeds[row] ^ ((unsigned long long)positions[row] * 0x9E3779B97F4A7C15ull));
+  const int from = blockIdx.x * FILTER_SLICE, to = min(vocab, from + FILTER_SLICE);
+  const float T = fr.temperature;
+  float l[16];
+  filter_read(filter_row(logits, fr, row), from, to, l);
+  Best b = {-INFINITY, -1};
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    if (!isfinite(l[i])) continue;
+    const int v = filter_at(from, i >> 2) + (i & 3);
+    if (p.mx != -INFINITY && !filter_keeps(p, v, l[i] / T)) continue;
+    if (sample_value(l[i], v, T, base)) b = better(b, Best{l[i], v});
+  }
+  b = block_best(b, red);
+  if (threadIdx.x == 0) {
+    part_val[(size_t)row * gridDim.x + blockIdx.x] = b.val;
+    part_idx[(size_t)row * gridDim.x + blockIdx.x] = b.idx;
+  }
+}
+
 __global__ void __launch_bounds__(FILTER_THREADS)
 filter_remove_kernel(float* __restrict__ logits, int vocab, int row_stride, const FilterRow* __restrict__ rows,
                      const FilterPlan* __restrict__ plans) {
@@ -630,8 +712,7 @@ filter_remove_kernel(float* __restrict__ logits, int vocab, int row_stride, cons
     f32x4_t o;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const float x = l[4 * q + i] / T, e = __expf(x - p.mx);
-      const bool keep = !isfinite(l[4 * q + i]) || (e >= p.e_min && e >= p.theta && filter_key(v + i, x) >= p.key_min);
+      const bool keep = !isfinite(l[4 * q + i]) || filter_keeps(p, v + i, l[4 * q + i] / T);
       o[i] = keep ? l[4 * q + i] : -INFINITY;
       if (!keep && !(whole && v + 3 < to)) lg[v + i] = -INFINITY;
     }
@@ -657,6 +738,41 @@ extern "C" long ra_filter_scratch(int n_rows, int vocab) {
   return n_rows > 0 && vocab > 0 ? (long)filter_parts(n_rows, vocab, off) : 0;
 }
 
+static float filter_unit(int vocab) {
+  // e = 1 in whole numbers: a whole row of ones stays below 2^63
+  float unit = 1.f;
+  for (int bits = 62, v = vocab; bits > 0; --bits, v >>= 1)
+    if (v <= 1) {
+      unit = (float)(1ull << bits);
+      break;
+    }
+  return unit * 0.5f;
+}
+
+// Passes 1 to 5: the rows' plans.
+static int filter_plans(const FilterLogits& l, int n_rows, int vocab, const FilterRow* fr, const int* window, char* s,
+                        const size_t (&off)[5], hipStream_t stream) {
+  FilterPlan* plans = (FilterPlan*)(s + off[0]);
+  unsigned long long* mass = (unsigned long long*)(s + off[1]);
+  unsigned* count = (unsigned*)(s + off[2]);
+  float* slice_max = (float*)(s + off[3]);
+  int* list = (int*)(s + off[4]);
+  const int slices = (vocab + FILTER_SLICE - 1) / FILTER_SLICE;
+  const float unit = filter_unit(vocab);
+  const dim3 grid(slices, n_rows);
+  filter_max_kernel<<<grid, FILTER_THREADS, 0, stream>>>(l, vocab, fr, window, slice_max);
+  RA_LAUNCH_CHECK("filter_logits (maximum)");
+  filter_bins_kernel<<<grid, FILTER_THREADS, 0, stream>>>(l, vocab, fr, slice_max, mass, count, unit);
+  RA_LAUNCH_CHECK("filter_logits (bins)");
+  filter_plan_kernel<<<n_rows, FILTER_BINS, 0, stream>>>(vocab, fr, slice_max, slices, mass, count, plans);
+  RA_LAUNCH_CHECK("filter_logits (plan)");
+  filter_list_kernel<<<grid, FILTER_THREADS, 0, stream>>>(l, vocab, fr, plans, list);
+  RA_LAUNCH_CHECK("filter_logits (list)");
+  filter_select_kernel<<<n_rows, FILTER_ROW_THREADS, 0, stream>>>(l, vocab, fr, plans, list, unit);
+  RA_LAUNCH_CHECK("filter_logits (boundaries)");
+  return 0;
+}
+
 extern "C" int ra_filter_logits(float* logits, int n_rows, int vocab, int row_stride, const void* rows,
                                 const int* window, void* scratch, long scratch_bytes, hipStream_t stream) {
   RA_CHECK(n_rows > 0 && vocab > 0, "filter_logits: empty input (%d rows, vocabulary %d)", n_rows, vocab);
@@ -667,34 +783,40 @@ extern "C" int ra_filter_logits(float* logits, int n_rows, int vocab, int row_st
   const size_t need = filter_parts(n_rows, vocab, off);
   RA_CHECK(scratch != nullptr && scratch_bytes >= (long)need && (uintptr_t)scratch % 16 == 0,
            "filter_logits: scratch of %ld bytes, needs %zu on a 16-byte boundary", scratch_bytes, need);
-  char* s = (char*)scratch;
-  FilterPlan* plans = (FilterPlan*)(s + off[0]);
-  unsigned long long* mass = (unsigned long long*)(s + off[1]);
-  unsigned* count = (unsigned*)(s + off[2]);
-  float* slice_max = (float*)(s + off[3]);
-  int* list = (int*)(s + off[4]);
+  const FilterLogits l = {logits, nullptr, row_stride, 0};
   const FilterRow* fr = (const FilterRow*)rows;
-  const int slices = (vocab + FILTER_SLICE - 1) / FILTER_SLICE;
-  // e = 1 in whole numbers: a whole row of ones stays below 2^63
-  float unit = 1.f;
-  for (int bits = 62, v = vocab; bits > 0; --bits, v >>= 1)
-    if (v <= 1) {
-      unit = (float)(1ull << bits);
-      break;
-    }
-  unit *= 0.5f;
-  const dim3 grid(slices, n_rows);
-  filter_max_kernel<<<grid, FILTER_THREADS, 0, stream>>>(logits, vocab, row_stride, fr, window, slice_max);
-  RA_LAUNCH_CHECK("filter_logits (maximum)");
-  filter_bins_kernel<<<grid, FILTER_THREADS, 0, stream>>>(logits, vocab, row_stride, fr, slice_max, mass, count, unit);
-  RA_LAUNCH_CHECK("filter_logits (bins)");
-  filter_plan_kernel<<<n_rows, FILTER_BINS, 0, stream>>>(vocab, fr, slice_max, slices, mass, count, plans);
-  RA_LAUNCH_CHECK("filter_logits (plan)");
-  filter_list_kernel<<<grid, FILTER_THREADS, 0, stream>>>(logits, vocab, row_stride, fr, plans, list);
-  RA_LAUNCH_CHECK("filter_logits (list)");
-  filter_select_kernel<<<n_rows, FILTER_ROW_THREADS, 0, stream>>>(logits, vocab, row_stride, fr, plans, list, unit);
-  RA_LAUNCH_CHECK("filter_logits (boundaries)");
-  filter_remove_kernel<<<grid, FILTER_THREADS, 0, stream>>>(logits, vocab, row_stride, fr, plans);
+  if (filter_plans(l, n_rows, vocab, fr, window, (char*)scratch, off, stream) != 0) return 1;
+  filter_remove_kernel<<<dim3((vocab + FILTER_SLICE - 1) / FILTER_SLICE, n_rows), FILTER_THREADS, 0, stream>>>(
+      logits, vocab, row_stride, fr, (const FilterPlan*)((char*)scratch + off[0]));
   RA_LAUNCH_CHECK("filter_logits (removal)");
+  return 0;
+}
+
+// A token a row of what ra_filter_logits would leave, drawn as ra_sample draws it, the logits left as they are. changed: rows of
+// changed_stride floats for those that penalties and biases change; the slices' best go to scratch_val and scratch_idx,
+// ra_filter_slices a row. temperatures are the rows' own.
+extern "C" int ra_filter_slices(int vocab) { return (vocab + FILTER_SLICE - 1) / FILTER_SLICE; }
+
+extern "C" int ra_sample_filtered(const float* logits, int n_rows, int vocab, int row_stride, const void* rows, const int* window,
+                                  float* changed, int changed_stride, void* scratch, long scratch_bytes, const long long* seeds,
+                                  const int* positions, float* scratch_val, int* scratch_idx, int* tokens, hipStream_t stream) {
+  RA_CHECK(n_rows > 0 && vocab > 0, "sample_filtered: empty input (%d rows, vocabulary %d)", n_rows, vocab);
+  RA_CHECK(row_stride >= vocab && changed_stride >= vocab, "sample_filtered: row strides %d and %d below the vocabulary %d", row_stride,
+           changed_stride, vocab);
+  RA_CHECK(n_rows <= 65535, "sample_filtered: %d rows in one launch (max 65535)", n_rows);
+  RA_CHECK(rows != nullptr && changed != nullptr && changed != logits, "sample_filtered: no row parameters, or no rows of its own");
+  size_t off[5];
+  const size_t need = filter_parts(n_rows, vocab, off);
+  RA_CHECK(scratch != nullptr && scratch_bytes >= (long)need && (uintptr_t)scratch % 16 == 0,
+           "sample_filtered: scratch of %ld bytes, needs %zu on a 16-byte boundary", scratch_bytes, need);
+  const FilterLogits l = {logits, changed, row_stride, changed_stride};
+  const FilterRow* fr = (const FilterRow*)rows;
+  if (filter_plans(l, n_rows, vocab, fr, window, (char*)scratch, off, stream) != 0) return 1;
+  const int slices = ra_filter_slices(vocab);
+  filter_draw_kernel<<<dim3(slices, n_rows), FILTER_THREADS, 0, stream>>>(
+      l, vocab, fr, (const FilterPlan*)((char*)scratch + off[0]), seeds, positions, scratch_val, scratch_idx);
+  RA_LAUNCH_CHECK("sample_filtered (draw)");
+  sample_stage2<<<n_rows, SAMPLE_THREADS, 0, stream>>>(scratch_val, scratch_idx, slices, tokens);
+  RA_LAUNCH_CHECK("sample_filtered stage 2");
   return 0;
 }

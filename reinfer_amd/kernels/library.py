@@ -54,6 +54,7 @@ _SIGNATURES = {
     "ra_sample": [P, I, I, I, P, P, P, P, P, P, P],
     "ra_sample_static": [P, I, I, I, P, P, P, P, P],
     "ra_filter_logits": [P, I, I, I, P, P, P, c_long, P],
+    "ra_sample_filtered": [P, I, I, I, P, P, P, I, P, c_long, P, P, P, P, P, P],
     "ra_pair_hash_add": [P, P, I, P, P, P, P, P, P, I, c_longlong, c_longlong, I, I, P],
     "ra_stream_add": [P, P, I, P, P, I, I, I, F, P],
     "ra_tanh_cap": [P, I, I, I, F, P],
@@ -134,6 +135,8 @@ def load() -> ctypes.CDLL:
             getattr(lib, name).argtypes = [c_int, c_int, c_int]
         lib.ra_attention_prefill_part_floats.restype = c_long
         lib.ra_attention_prefill_part_floats.argtypes = [c_int, c_int, c_int, c_int, c_int]
+        lib.ra_filter_slices.restype = c_int
+        lib.ra_filter_slices.argtypes = [I]
         lib.ra_filter_scratch.restype = c_long
         lib.ra_filter_scratch.argtypes = [I, I]
         lib.ra_sample_static_max_pairs.restype = c_long

@@ -2045,18 +2045,48 @@ class HipKernels:
             packed = torch.tensor(window, dtype=torch.int32).numpy()
         return np.concatenate([rec.view(np.int32).reshape(-1), packed])
 
+    def _packed_filters(self, params, histories, n: int):
+        import numpy as np
+        lists = isinstance(params, (list, tuple)) and isinstance(histories, (list, tuple))
+        packed = _host.pack_filters(params, histories, n) if lists else None
+        return np.frombuffer(packed, dtype=np.int32) if packed is not None else self._pack_filters(params, histories, n)
+
+    def sample_filtered(self, logits: torch.Tensor, params, histories, seeds, positions, tokens: torch.Tensor) -> None:
+        """:meth:`filter_logits` and :meth:`sample` with the rows' own temperatures, the logits left as they are; ``seeds`` and
+        ``positions`` are a number a row, on the host: everything goes to the device in one transfer."""
+        import numpy as np
+        _dev(logits, tokens)
+        n, V = logits.shape
+        if logits.dtype != torch.float32 or logits.stride(1) != 1:
+            raise TypeError("sample_filtered: logits are float32 rows")
+        _int32(tokens, "sampled tokens", n)
+        if not (len(params) == len(seeds) == len(positions) == n):
+            raise ValueError("sample_filtered: one SamplingParams, seed and position per row")
+        packed = self._packed_filters(params, histories, n)
+        rows = np.empty(3 * n + packed.size, dtype=np.int32)
+        rows[:2 * n].view(np.int64)[:] = seeds
+        rows[2 * n:3 * n] = positions
+        rows[3 * n:] = packed
+        rows_t = to_device(rows, logits.device)
+        lib = library.load()
+        need, slices, stride = int(lib.ra_filter_scratch(n, V)), int(lib.ra_filter_slices(V)), (V + 3) // 4 * 4
+        # one allocation: the changed rows, the passes' scratch, the slices' best
+        at = 4 * n * stride
+        at += -at % 16
+        best = at + need + -need % 16
+        scratch = torch.empty(best + 8 * n * slices, dtype=torch.uint8, device=logits.device)
+        base, rows_p = scratch.data_ptr(), rows_t.data_ptr()
+        library.call("ra_sample_filtered", logits.data_ptr(), n, V, logits.stride(0), rows_p + 12 * n, rows_p + 60 * n, base, stride,
+                     base + at, need, rows_p, rows_p + 8 * n, base + best, base + best + 4 * n * slices, tokens.data_ptr(), _stream())
+
     def filter_logits(self, logits: torch.Tensor, params, histories) -> None:
         """Logit bias, penalties and top-k / top-p / min-p of every row's SamplingParams, in
         place (removed tokens become -inf); ``histories[i]`` are row i's tokens so far."""
-        import numpy as np
         _dev(logits)
         n, V = logits.shape
         if logits.dtype != torch.float32 or logits.stride(1) != 1:
             raise TypeError("filter_logits: logits are float32 rows")
-        lists = isinstance(params, (list, tuple)) and isinstance(histories, (list, tuple))
-        packed = _host.pack_filters(params, histories, n) if lists else None
-        packed = np.frombuffer(packed, dtype=np.int32) if packed is not None else self._pack_filters(params, histories, n)
-        both = to_device(packed, logits.device)
+        both = to_device(self._packed_filters(params, histories, n), logits.device)
         rows_t, win_t = both[:12 * n], both[12 * n:]
         need = int(library.load().ra_filter_scratch(n, V))
         scratch = torch.empty(need, dtype=torch.uint8, device=logits.device)

@@ -24,13 +24,13 @@ import torch
 
 # methods of the kernel set that launch work, and how their calls are classed
 _ROWS = {"embed": "embedding", "add_rmsnorm": "norm", "silu_mul": "gate", "sample": "sampler",
-         "filter_logits": "sampler"}
+         "filter_logits": "sampler", "sample_filtered": "sampler"}
 _QK = {"qk_norm_rope_cache", "qk_norm_rope_cache_ranges"}
 _ATTN = {"attention", "attention_plain", "attention_decode", "attention_prefill"}
-_LINEAR = {"linear", "linear_plain", "linear_skinny", "gated_linear", "linear_ranges"}
+_LINEAR = {"linear", "linear_plain", "linear_skinny", "gated_linear", "linear_ranges", "linear_pair"}
 # kernels of further mechanisms, each a class of its own
 _OTHER = {"latent_prep": "latent norm + rotation + cache write", "head_linear": "products head by head",
-          "moe_route": "router", "moe_relu2_scale": "expert activation",
+          "moe_route": "router", "moe_relu2_scale": "expert activation", "moe_choose_scale": "router + expert activation",
           "moe_grouped": "experts over sorted tokens", "linear_columns": "shared expert down", "moe_up_chosen": "chosen experts up", "moe_down_chosen": "chosen experts down",
           "moe_gate_up_chosen": "chosen experts up", "moe_down_gated_chosen": "chosen experts down", "stream_add": "stream add",
           "pair_hash_add": "embedding", "tanh_cap": "logit cap",

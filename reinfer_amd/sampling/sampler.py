@@ -56,6 +56,12 @@ class Sampler:
         if any(p.filters for p in params):
             if histories is None:
                 raise ValueError("penalties need the requests' tokens")
+            if hasattr(ops, "sample_filtered") and len(histories) == n:
+                if logits.stride(1) != 1 or logits.stride(0) < logits.shape[1]:
+                    logits = logits.clone()
+                tokens = torch.empty(n, dtype=torch.int32, device=self.device)
+                ops.sample_filtered(logits, params, histories, [as_int64(int(s)) for s in seeds], [int(p) for p in positions], tokens)
+                return self._drawn(tokens)
             logits = logits.clone()
             ops.filter_logits(logits, params, histories)
         # one transfer: seeds, temperatures, positions
@@ -67,6 +73,10 @@ class Sampler:
         tokens = torch.empty(n, dtype=torch.int32, device=self.device)
         ops.sample(logits, rows_t[8 * n:12 * n].view(torch.float32), rows_t[:8 * n].view(torch.int64),
                    rows_t[12 * n:].view(torch.int32), tokens)
+        return self._drawn(tokens)
+
+    @staticmethod
+    def _drawn(tokens: torch.Tensor) -> List[int]:
         out = tokens.tolist()
         for i, t in enumerate(out):
             if t < 0:
