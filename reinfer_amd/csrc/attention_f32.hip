@@ -1,18 +1,27 @@
 // Paged attention of the 32-bit path for head sizes 64, 128 and 256; attention_plain.hip says what it computes and keeps
 // the other sizes and the bfloat16 twin.
 //
-// A workgroup has one token and GH query heads of one KV head. The tiles of 16 keys are dealt out to eight shares, each with a
-// running maximum and sums of its own, that are added up through LDS at the end in their order; its waves, two or eight, take
-// the shares one after the other. So the order of a token's sums follows from its own position, whatever the step holds. Both
-// tiles are read in the order they are stored in, 16 bytes a lane, and once for all GH heads:
-//   keys    lane (slot = lane % 16, part = lane / 16) has the slot's pieces of 8 entries number part, part + 4, ...: its
-//           share of the scores is a product with queries that stay in registers, two exchanges add the four shares;
-//   values  lane (entry = lane % 16, four slots from 4 (lane / 16)) has four keys' values of one entry of every run of 16.
-// The plain kernel reads an element a lane and access and walks the values key by key: bound by the latency of those reads.
-// Four requests with prompts of 60 to 500 tokens and 12 further ones each, 32 heads of 128 on 8 KV heads: its calls take
-// 339 us on average there, 33 us here. (Eight shares whatever the step holds cost prompts the sums' ends: 497 tokens from their
-// start 169 us, 139 where each of two waves had one set of sums.) What bounds it now is the vector unit in prompts (every query reads the tiles from
-// the caches again) and the trips to memory of a short walk in decode steps.
+// Both products run on the float matrix cores, 16 rows a workgroup: the heads that share a KV head, times tokens. A float product of
+// 16x16x4 is a chain of four fused multiply-adds, in order and each rounded, so vector units can walk the same chains: few tokens, whose
+// products would be mostly empty columns, go there (attention_f32_token_kernel), and have the same bits. The tiles of 16 keys are dealt
+// out to eight shares by their number, each with a running maximum and sums of its own, that are added up through LDS at the end in
+// their order; waves take the shares one after the other. So a token's bits follow from its own position, whatever the step holds.
+// Both tiles are read in the order they are stored in, 16 bytes a lane, and once for all of a workgroup's rows:
+//   keys    are the products' rows and the queries their columns. Lane (slot = lane % 16, hi = lane / 16) has the slot's pieces of 8
+//           entries hi, hi + 4, ...; entry e of a half of piece hi + 4 c is step e of chain 2 c + half. (With half as many chains the
+//           error against 64 bits is 1.51e-7 of the norm in place of 1.35e-7; it was 1.46e-7 with a query a wave on the vector units);
+//   values  are the rows of the second product, lane (entry = lane % 16, four slots from 4 (lane / 16)). The first one's results lie as
+//           the second wants its columns: four keys of a row a lane. It starts from zero in every tile and is added to the sums so far.
+// What is read of a tile ahead of its turn goes into the registers of the one before: keys behind the first product, values behind the
+// second, through descriptors, whose loads past the last tile count like others. (Behind a branch all loads are waited for.)
+//
+// A query a workgroup on the vector units was bound by reading every tile again for each: four prompts of 60 to 500 tokens, 32 heads of
+// 128 on 8 KV heads, 335 us, now 85; one of 600 248 / 62; 300 tokens behind 1000 363 / 97; 500 and 400 of 16 heads of 256 on 4, 318 / 94. On
+// the bfloat16 cores, in three parts a float, it was 90 (keys and values split by every wave: 2800 cycles of vector instructions a wave
+// and 32 keys), and the decode step below 21.0. Bound now by the matrix cores, busy 30 % of the time, and by loads, which are a tile
+// ahead: 31 % of a wave's time; the next tile's scores beside this one's weights took a fifth longer (a wave's last are wasted). Decode
+// steps, a token a workgroup: 1 at 300 keys 12.2 / 8.9, 4 of 70 to 505 14.8 / 12.7, 1 at 4000 64.8 / 47.3: bound by trips to memory and
+// exchanges; through LDS each costs some hundred cycles, so they are the vector unit's own.
 #include "common.h"
 #include "reinfer_hip.h"
 
@@ -27,158 +36,476 @@ struct F32Attention {
   const int* block_tables;
   int max_blocks;
   const int *token_list, *seq_of_token, *positions;
-  int block_size, Hq, Hkv;
+  int n_tokens, heads;                     // heads: of a workgroup, a power of two
+  int block_size, tiles;                   // a block's tiles of 16 slots
+  unsigned long long share;                // i / tiles is i * share >> 32
+  int Hq, Hkv;
   float scale;
   int window, aligned, keep;
   RaScoreMod mod;
   RaHeadOut ho;
 };
 
-__device__ __forceinline__ float max16(float v) {
+// Over the four rows of 16 lanes, in the vector unit. (The builtins for the swaps give their first result twice. The waits are the two
+// that lie between a write by the vector unit and a swap, and as many behind it.)
+__device__ __forceinline__ float sum_rows(float v) {
+  float w = v;
+  asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(v), "+v"(w));
+  w = v += w;
+  asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(v), "+v"(w));
+  return v + w;
+}
+__device__ __forceinline__ float sum_rows_far(float v) {                // the far rows first: (first + third) + (second + fourth)
+  float w = v;
+  asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(v), "+v"(w));
+  w = v += w;
+  asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(v), "+v"(w));
+  return v + w;
+}
+__device__ __forceinline__ float max_rows(float v) {
+  float w = v;
+  asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(v), "+v"(w));
+  w = v = fmaxf(v, w);
+  asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(v), "+v"(w));
+  return fmaxf(v, w);
+}
+__device__ __forceinline__ int max16(int v) {
 #pragma unroll
-  for (int m = 8; m > 0; m >>= 1) v = fmaxf(v, __shfl_xor(v, m, RA_WAVE));
-  return v;
+  for (int m = 8; m > 0; m >>= 1) v = max(v, __shfl_xor(v, m, RA_WAVE));
+  return __builtin_amdgcn_readfirstlane(v);
+}
+
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
+// of 16 neighbouring lanes: pairs, quads, the mirrored half row and row
+__device__ __forceinline__ float max_row(float v) {
+  v = fmaxf(v, dpp<0xB1>(v));
+  v = fmaxf(v, dpp<0x4E>(v));
+  v = fmaxf(v, dpp<0x141>(v));
+  return fmaxf(v, dpp<0x140>(v));
 }
 
 #define SHARES 8
+#define ROWS 16
+// Where a chain of a tile's is cut in two, e 0 and 1, 2 and 3: where the error against 64 bits was not below that of the kernel before (64,
+// 1e-7 of the norm: a prompt of 600 1.33, whole chains 1.38, 1.25 so), or it costs nothing (values of 128: 1.35 / 1.30; of 256 they
+// are registers too many).
+#define SPLIT_KEYS(D) ((D) == 64)
+#define SPLIT_VALUES(D) ((D) <= 128)
 
+// The tiles of 16 keys that positions see: those with keys that are kept, then those from the first window's first key on. Tile i is share
+// i % SHARES's.
+struct F32Walk {
+  int early, first, last;
+  __device__ __forceinline__ int skip(int i) const {
+    return i >= early && i < first ? i + (first - i + SHARES - 1) / SHARES * SHARES : i;
+  }
+};
+__device__ __forceinline__ int block_of(const F32Attention& g, int i) { return (int)((unsigned)i * g.share >> 32); }
+__device__ __forceinline__ int id_of(const F32Attention& g, const int* table, int i) {
+  return ((const __attribute__((address_space(4))) int*)table)[block_of(g, i)];
+}
+__device__ __forceinline__ size_t base_of(const F32Attention& g, int kvh, int i, int id, int d) {
+  return (((size_t)id * g.Hkv + kvh) * g.tiles + (i - block_of(g, i) * g.tiles)) * 16 * d;
+}
+// The shares' sums of one entry or four, in their order.
+template <typename T>
+__device__ __forceinline__ T add_shares(const float* ends, int ends_step, const float* sums, int step, float sink, float gate) {
+  float top = -INFINITY, den = 0.f;
+  for (int w = 0; w < SHARES; ++w) top = fmaxf(top, ends[w * ends_step]);
+  T sum = {};
+  for (int w = 0; w < SHARES; ++w) {
+    const float lw = ends[w * ends_step + 1];
+    if (lw == 0.f) continue;               // nothing seen
+    const float f = expf(ends[w * ends_step] - top);
+    const T y = *(const T*)(sums + w * step);
+    if constexpr (sizeof(T) == 4) {
+      sum = fmaf(f, y, sum);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum[e] = fmaf(f, y[e], sum[e]);
+    }
+    den = fmaf(f, lw, den);
+  }
+  den += expf(sink - top);                 // no sink: minus infinity
+  return sum * (gate / den);
+}
+
+// One share of a token's walk for GH heads of one KV head, by a wave, in the order of the kernel below to the last bit. Its products' chains
+// of 16 are a lane each: chain 2 c + half takes entries half * 4 + e of pieces 4 c to 4 c + 3, e by e; chains c and c + w are added for w =
+// half of them, a quarter, ...; of the values' it is the keys 0, 4, 8, 12, 1, 5, .... sums [GH][D], ends [GH][2]: maximum and sum.
 template <int D, int GH>
-__global__ void __launch_bounds__(SHARES * RA_WAVE) attention_f32_kernel(F32Attention g) {
-  constexpr int KP = D / 32;               // pieces of 8 entries of a key a lane
-  constexpr int VP = D / 16;               // runs of 16 entries of the values
-  __shared__ float part[SHARES][GH][D + 2];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
-  const int lo16 = lane & 15, hi = lane >> 4;
-  const int h0 = blockIdx.x * GH, group = g.Hq / g.Hkv, kvh = h0 / group;
-  const int t = g.token_list ? g.token_list[blockIdx.y] : blockIdx.y;
-  const int p = g.positions[t];
-  const int* table = g.block_tables + (size_t)g.seq_of_token[t] * g.max_blocks;
-  float q[GH][KP][8];
+__device__ __forceinline__ void walk_share(const F32Attention& g, int t, int h0, const int* table, int share, float* sums, float* ends) {
+  constexpr int N = D / 64;                // chains, and entries of the values, of a lane: number lane / 16 + 4 j of the chains and runs
+  const int lane = threadIdx.x & 63, lo16 = lane & 15, hi = lane >> 4;
+  const int kvh = h0 / (g.Hq / g.Hkv), p = g.positions[t];
+  const int lo = ra_first_key(p, g.window, g.aligned), kept = g.keep < lo ? g.keep : lo;
+  const F32Walk walk = {(kept + 15) >> 4, lo >> 4, p >> 4};
+  int i = walk.skip(share);
+  float m[GH], l[GH], acc[GH][N];
 #pragma unroll
   for (int h = 0; h < GH; ++h) {
-    const float* qv = g.q + (size_t)t * g.q_stride + (size_t)(h0 + h) * D;
+    m[h] = -INFINITY;
+    l[h] = 0.f;
+#pragma unroll
+    for (int j = 0; j < N; ++j) acc[h][j] = 0.f;
+  }
+  if (i <= walk.last) {
+    f32x4_t q[GH][N][4];
+    const int piece = (hi >> 1) * 4, half = hi & 1;      // chain hi + 4 j: pieces piece + 8 j + 0 .. 3
+#pragma unroll
+    for (int h = 0; h < GH; ++h) {
+      const float* qv = g.q + (size_t)t * g.q_stride + (size_t)(h0 + h) * D + piece * 8 + half * 4;
+#pragma unroll
+      for (int j = 0; j < N; ++j)
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) q[h][j][x][e] = qv[j * 64 + x * 8 + e];
+    }
+    int id = id_of(g, table, i);
+    while (true) {
+      const int next = walk.skip(i + SHARES);
+      const size_t at = base_of(g, kvh, i, id, D);
+      f32x4_t k[N][4], v[N][4];
+#pragma unroll
+      for (int j = 0; j < N; ++j)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) k[j][x] = *(const f32x4_t*)(g.kcache + at + ((piece + j * 8 + x) * 16 + lo16) * 8 + half * 4);
+#pragma unroll
+      for (int j = 0; j < N; ++j)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) v[j][x] = *(const f32x4_t*)(g.vcache + at + (((hi + 4 * j) * 4 + x) * 16 + lo16) * 4);
+      id = id_of(g, table, min(next, walk.last));        // the next one's, beside this one's keys
+      const int key0 = i * 16, key = key0 + lo16;
+      const bool seen = key <= p && (key >= lo || key < kept);
+      // slots that nobody has written yet may hold anything: a probability of zero does not make a NaN harmless
+      if (key0 + 15 > p || key0 < lo) {
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int at_key = key0 + x * 4 + e;
+            const bool any = at_key <= p && (at_key >= lo || at_key < kept);
+#pragma unroll
+            for (int j = 0; j < N; ++j) v[j][x][e] = any ? v[j][x][e] : 0.f;
+          }
+      }
+#pragma unroll
+      for (int h = 0; h < GH; ++h) {
+        float z[N];
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+          float zz = z[j] = 0.f;
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int x = 0; x < 4; ++x) {
+              float& to = SPLIT_KEYS(D) && e > 1 ? zz : z[j];
+              to = fmaf(k[j][x][e], q[h][j][x][e], to);
+            }
+          if (SPLIT_KEYS(D)) z[j] += zz;
+        }
+#pragma unroll
+        for (int w = N / 2; w > 0; w >>= 1)
+#pragma unroll
+          for (int j = 0; j < w; ++j) z[j] += z[j + w];
+        const int a = h0 + h;
+        float s = sum_rows_far(z[0]) * g.scale;
+        if (g.mod.softcap > 0.f || g.mod.r1)
+          s = ra_mod_score(s, g.mod.softcap, g.mod.r1 != nullptr, g.mod.r1 ? g.mod.r1[a] : 0.f, g.mod.r1 ? g.mod.r2[a] : 0.f, p - key);
+        s = seen ? s : -INFINITY;
+        const float top = fmaxf(m[h], max_row(s));
+        const float corr = m[h] == -INFINITY ? 0.f : expf(m[h] - top), less = top == -INFINITY ? 0.f : top;      // all may be -inf
+        m[h] = top;
+        s = expf(s - less);
+        l[h] = fmaf(l[h], corr, dpp<0x00>(s)) + dpp<0x55>(s);
+        l[h] += dpp<0xAA>(s);
+        l[h] += dpp<0xFF>(s);
+        float y[2][N];
+#pragma unroll
+        for (int j = 0; j < N; ++j) y[0][j] = y[1][j] = 0.f;
+#define KEY(x, e)                      \
+  {                                    \
+    const float w = dpp<0x150 + x * 4 + e>(s); \
+    for (int j = 0; j < N; ++j) {      \
+      float& to = y[SPLIT_VALUES(D) ? e / 2 : 0][j]; \
+      to = fmaf(v[j][x][e], w, to);    \
+    }                                  \
+  }
+#define KEYS(e) KEY(0, e) KEY(1, e) KEY(2, e) KEY(3, e)
+        KEYS(0) KEYS(1) KEYS(2) KEYS(3)
+#undef KEYS
+#undef KEY
+#pragma unroll
+        for (int j = 0; j < N; ++j) acc[h][j] = fmaf(acc[h][j], corr, SPLIT_VALUES(D) ? y[0][j] + y[1][j] : y[0][j]);
+      }
+      if (next > walk.last) break;
+      i = next;
+    }
+#pragma unroll
+    for (int h = 0; h < GH; ++h) {
+      l[h] += __shfl_xor(l[h], 4, RA_WAVE);
+      l[h] += __shfl_xor(l[h], 8, RA_WAVE);
+#pragma unroll
+      for (int j = 0; j < N; ++j) sums[h * D + (hi + 4 * j) * 16 + lo16] = acc[h][j];
+    }
+  }
+  if (lane == 0) {
+#pragma unroll
+    for (int h = 0; h < GH; ++h) {
+      ends[h * 2] = m[h];
+      ends[h * 2 + 1] = l[h];
+    }
+  }
+}
+
+// 16 rows: tokens times the heads of a KV head. Tokens of several requests come one run of a request's after the other, or, with gridDim.z
+// over 1, a workgroup has the run that starts at its own token and ends at once where none does.
+template <int D, int WAVES>
+__global__ void __launch_bounds__(WAVES * RA_WAVE) attention_f32_kernel(F32Attention g) {
+  constexpr int KP = D / 32;               // pieces of 8 entries of a key a lane
+  constexpr int VP = D / 16;               // runs of 16 entries of the values
+  constexpr int LD = D + 4;
+  extern __shared__ __attribute__((aligned(16))) float part[];           // [SHARES][ROWS][LD], then maximum and sum [SHARES][ROWS][2]
+  float* const ends = part + SHARES * ROWS * LD;
+  __shared__ int off[ROWS];                // rows with a result that is no finite number
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+  const int lo16 = lane & 15, hi = lane >> 4;
+  const int gh = g.heads, nt = ROWS / gh;
+  const int h0 = blockIdx.x * gh, kvh = h0 / (g.Hq / g.Hkv), a = h0 + lo16 % gh;
+  // the last tokens first: theirs are the longest walks of a prompt
+  const int i0 = (gridDim.y - 1 - blockIdx.y) * nt, rows = min(ROWS, (g.n_tokens - i0) * gh);
+  const int at = i0 + min(lo16, rows - 1) / gh;
+  const int t = g.token_list ? g.token_list[at] : at;
+  const int seq = g.seq_of_token[t], pos = g.positions[t];
+  const int before = __shfl(seq, lo16 >= gh ? lo16 - gh : 0, RA_WAVE);
+  // the first rows of the requests' runs
+  const unsigned runs = __ballot(lane < rows && lo16 % gh == 0 && (lane == 0 || seq != before));
+  if (gridDim.z > 1 && !(runs >> (blockIdx.z * gh) & 1)) return;
+  float q[KP][8];                          // the products' columns
+  {
+    const float* qv = g.q + (size_t)t * g.q_stride + (size_t)a * D + hi * 8;
 #pragma unroll
     for (int c = 0; c < KP; ++c)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) q[h][c][e] = qv[(hi + 4 * c) * 8 + e];
+      for (int e = 0; e < 8; ++e) q[c][e] = qv[c * 32 + e];
   }
-  // tiles of the kept first keys, then those from the window's first key on; a tile that holds the end of the one and the
-  // start of the other comes twice, each time with its own keys alone
-  const int lo = ra_first_key(p, g.window, g.aligned);
-  const int kept = g.keep < lo ? g.keep : lo;
-  const int kept_tiles = (kept + 15) >> 4, first = lo >> 4;
-  const int tiles = kept_tiles + (p >> 4) - first + 1;
-  for (int share = wave; share < SHARES; share += waves) {
-    if (share >= tiles) {                    // a share without a tile
-      if (lane < GH) {
-        part[share][lane][D] = -INFINITY;
-        part[share][lane][D + 1] = 0.f;
+  const float d1 = g.mod.r1 ? g.mod.r1[a] : 0.f, d2 = g.mod.r1 ? g.mod.r2[a] : 0.f;
+
+  for (int r0 = 0, r1; r0 < rows; r0 = r1) {             // a run: rows r0 to r1
+    const unsigned rest = runs >> r0 >> 1;
+    r1 = rest ? r0 + __ffs(rest) : rows;
+    if (gridDim.z > 1 && r0 != (int)blockIdx.z * gh) continue;
+    const bool mine = lo16 >= r0 && lo16 < r1;
+    const int* table = g.block_tables + (size_t)__builtin_amdgcn_readlane(seq, r0) * g.max_blocks;
+    const int p = mine ? pos : -1;         // a row of another request sees nothing
+    const int lo = mine ? ra_first_key(p, g.window, g.aligned) : 0;
+    const int kept = mine ? (g.keep < lo ? g.keep : lo) : 0;
+    const int end = max16(p), from = -max16(mine ? -lo : -0x7fffffff), keeps = max16(kept);      // over the run's rows
+    const F32Walk walk = {(keeps + 15) >> 4, from >> 4, end >> 4};
+    const int last = walk.last;
+    for (int share = wave; share < SHARES; share += waves) {
+      int i = walk.skip(share);
+      if (i > last) {                      // a share without a tile
+        if (lane < ROWS) {
+          ends[(share * ROWS + lane) * 2] = -INFINITY;
+          ends[(share * ROWS + lane) * 2 + 1] = 0.f;
+        }
+        continue;
       }
-      continue;
-    }
-    float acc[GH][VP], m[GH], l[GH];
+      float m = -INFINITY, l = 0.f;
+      f32x4_t acc[VP], k[KP][2], v[VP];
 #pragma unroll
-    for (int h = 0; h < GH; ++h) {
-#pragma unroll
-      for (int b = 0; b < VP; ++b) acc[h][b] = 0.f;
-      m[h] = -INFINITY;
-      l[h] = 0.f;
-    }
-    for (int i = share; i < tiles; i += SHARES) {
-      const bool early = i < kept_tiles;
-      const int tile = early ? i : first + i - kept_tiles;
-      const int from = early ? 0 : lo, to = early ? kept : p + 1;      // the keys of this tile that are seen
-      const size_t at = ((size_t)table[tile * 16 / g.block_size] * g.Hkv + kvh) * g.block_size * D
-                        + (size_t)(tile * 16 % g.block_size) * D;
-      f32x4_t k[KP][2], v[VP];
-#pragma unroll
-      for (int c = 0; c < KP; ++c) {
-        const float* kr = g.kcache + at + ((hi + 4 * c) * 16 + lo16) * 8;
-        k[c][0] = *(const f32x4_t*)kr;
-        k[c][1] = *(const f32x4_t*)(kr + 4);
-      }
-#pragma unroll
-      for (int b = 0; b < VP; ++b) v[b] = *(const f32x4_t*)(g.vcache + at + ((b * 4 + hi) * 16 + lo16) * 4);
-      const int key = tile * 16 + lo16;
-      const bool seen = key >= from && key < to;
-      // slots that nobody has written yet may hold anything: a probability of zero does not make a NaN harmless
-      const int slot0 = tile * 16 + hi * 4;
-#pragma unroll
-      for (int b = 0; b < VP; ++b)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (slot0 + e < from || slot0 + e >= to) v[b][e] = 0.f;
-#pragma unroll
-      for (int h = 0; h < GH; ++h) {
-        float s = 0.f;
+      for (int b = 0; b < VP; ++b) acc[b] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+      // behind the last tile a load counts like any other, and neither reads memory nor makes the others' wait a longer one
+      auto load_keys = [&](int i, int id) {
+        const auto tile = __builtin_amdgcn_make_buffer_rsrc((void*)(g.kcache + base_of(g, kvh, i, id, D)), 0, i <= last ? 16 * D * 4 : 0, 0x00020000);
 #pragma unroll
         for (int c = 0; c < KP; ++c)
 #pragma unroll
-          for (int e = 0; e < 8; ++e) s = fmaf(q[h][c][e], k[c][e >> 2][e & 3], s);
-        s += __shfl_xor(s, 16, RA_WAVE);
-        s += __shfl_xor(s, 32, RA_WAVE);
-        const int a = h0 + h;
-        s = ra_mod_score(s * g.scale, g.mod.softcap, g.mod.r1 != nullptr, g.mod.r1 ? g.mod.r1[a] : 0.f,
-                         g.mod.r1 ? g.mod.r2[a] : 0.f, p - key);
-        if (!seen) s = -INFINITY;
-        const float top = fmaxf(m[h], max16(s));
-        const float corr = m[h] == -INFINITY ? 0.f : expf(m[h] - top);
-        const float pr = seen ? expf(s - (top == -INFINITY ? 0.f : top)) : 0.f;      // all of a tile's scores may be -inf
-        m[h] = top;
-        l[h] = l[h] * corr + pr;
-        float ps[4];
+          for (int e = 0; e < 2; ++e)
+            k[c][e] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(tile, (hi * 16 + lo16) * 32, c * 2048 + e * 16, 0));
+      };
+      auto load_values = [&](int i, int id) {
+        const auto tile = __builtin_amdgcn_make_buffer_rsrc((void*)(g.vcache + base_of(g, kvh, i, id, D)), 0, i <= last ? 16 * D * 4 : 0, 0x00020000);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) ps[e] = __shfl(pr, hi * 4 + e, RA_WAVE);
+        for (int b = 0; b < VP; ++b)
+          v[b] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(tile, (hi * 16 + lo16) * 16, b * 1024, 0));
+      };
+      int id = id_of(g, table, i), next = walk.skip(i + SHARES);
+      load_keys(i, id);
+      load_values(i, id);
+      id = id_of(g, table, min(next, last));
+      for (; i <= last;) {
+        const int then = walk.skip(next + SHARES), id2 = id_of(g, table, min(then, last));
+        f32x4_t z[2 * KP], zz[2 * KP];
 #pragma unroll
-        for (int b = 0; b < VP; ++b) {
-          float sum = acc[h][b] * corr;
+        for (int c = 0; c < 2 * KP; ++c) z[c] = zz[c] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int e = 0; e < 4; ++e) sum = fmaf(ps[e], v[b][e], sum);
-          acc[h][b] = sum;
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int c = 0; c < 2 * KP; ++c) {
+            f32x4_t& to = SPLIT_KEYS(D) && e > 1 ? zz[c] : z[c];
+            to = __builtin_amdgcn_mfma_f32_16x16x4f32(k[c >> 1][c & 1][e], q[c >> 1][(c & 1) * 4 + e], to, 0, 0, 0);
+          }
+        load_keys(next, id);
+        if (SPLIT_KEYS(D)) {
+#pragma unroll
+          for (int c = 0; c < 2 * KP; ++c) z[c] += zz[c];
         }
+#pragma unroll
+        for (int w = KP; w > 0; w >>= 1)
+#pragma unroll
+          for (int c = 0; c < w; ++c) z[c] += z[c + w];
+        const int key0 = i * 16 + hi * 4;
+        float s[4], top = m;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[e] = z[0][e] * g.scale;
+        if (g.mod.softcap > 0.f || g.mod.r1) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) s[e] = ra_mod_score(s[e], g.mod.softcap, g.mod.r1 != nullptr, d1, d2, p - key0 - e);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int key = key0 + e;
+          s[e] = key <= p && (key >= lo || key < kept) ? s[e] : -INFINITY;
+          top = fmaxf(top, s[e]);
+        }
+        top = max_rows(top);
+        const float corr = m == -INFINITY ? 0.f : expf(m - top), less = top == -INFINITY ? 0.f : top;      // all may be -inf
+        m = top;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          s[e] = expf(s[e] - less);
+          l = e == 0 ? fmaf(l, corr, s[0]) : l + s[e];
+        }
+        // slots that nobody has written yet may hold anything: a probability of zero does not make a NaN harmless
+        if (i * 16 + 15 > end || i * 16 < from) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int key = key0 + e;
+            const bool any = key <= end && (key >= from || key < keeps);
+#pragma unroll
+            for (int b = 0; b < VP; ++b) v[b][e] = any ? v[b][e] : 0.f;
+          }
+        }
+        f32x4_t y[2][VP];
+#pragma unroll
+        for (int b = 0; b < VP; ++b) y[0][b] = y[1][b] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int b = 0; b < VP; ++b) {
+            f32x4_t& to = y[SPLIT_VALUES(D) ? e / 2 : 0][b];
+            to = __builtin_amdgcn_mfma_f32_16x16x4f32(v[b][e], s[e], to, 0, 0, 0);
+          }
+        load_values(next, id);
+#pragma unroll
+        for (int b = 0; b < VP; ++b)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[b][e] = fmaf(acc[b][e], corr, SPLIT_VALUES(D) ? y[0][b][e] + y[1][b][e] : y[0][b][e]);
+        i = next;
+        next = then;
+        id = id2;
+      }
+      l = sum_rows(l);
+      float* row = part + (share * ROWS + lo16) * LD;
+#pragma unroll
+      for (int b = 0; b < VP; ++b) *(f32x4_t*)(row + b * 16 + hi * 4) = acc[b];
+      if (hi == 0) {
+        ends[(share * ROWS + lo16) * 2] = m;
+        ends[(share * ROWS + lo16) * 2 + 1] = l;
       }
     }
-    // a share's sums: l over its 16 slots, each entry over the four runs of slots
+    if (threadIdx.x < ROWS) off[threadIdx.x] = 0;
+    __syncthreads();
+    for (int x = threadIdx.x; x < (r1 - r0) * (D / 4); x += blockDim.x) {
+      const int r = r0 + x / (D / 4), e0 = x % (D / 4) * 4, head = h0 + r % gh, one = i0 + r / gh;
+      const int token = g.token_list ? g.token_list[one] : one;
+      const f32x4_t y = add_shares<f32x4_t>(ends + r * 2, ROWS * 2, part + r * LD + e0, ROWS * LD,
+                                            g.ho.sink ? g.ho.sink[head] : -INFINITY, ra_head_gate<float>(g.ho, token, head));
 #pragma unroll
-    for (int h = 0; h < GH; ++h) {
-#pragma unroll
-      for (int x = 8; x > 0; x >>= 1) l[h] += __shfl_xor(l[h], x, RA_WAVE);
-#pragma unroll
-      for (int b = 0; b < VP; ++b) {
-        acc[h][b] += __shfl_xor(acc[h][b], 16, RA_WAVE);
-        acc[h][b] += __shfl_xor(acc[h][b], 32, RA_WAVE);
-        if (hi == 0) part[share][h][b * 16 + lo16] = acc[h][b];
-      }
-      if (lane == 0) {
-        part[share][h][D] = m[h];
-        part[share][h][D + 1] = l[h];
+      for (int e = 0; e < 4; ++e) {
+        if (!(fabsf(y[e]) <= 3.402823466e38f)) off[r] = 1;
+        g.out[(size_t)token * g.out_stride + (size_t)head * D + e0 + e] = y[e];
       }
     }
+    __syncthreads();
+    // A key that a row does not see weighs zero there, and zero times a value that is no finite number is none: a row with such a result
+    // is worked out again, from the keys it sees alone.
+    for (int r = r0; r < r1; ++r) {
+      if (!off[r]) continue;
+      const int one = i0 + r / gh, head = h0 + r % gh, token = g.token_list ? g.token_list[one] : one;
+      __syncthreads();
+      for (int share = wave; share < SHARES; share += waves)
+        walk_share<D, 1>(g, token, head, table, share, part + share * D, ends + share * 2);
+      __syncthreads();
+      for (int e = threadIdx.x; e < D; e += blockDim.x)
+        g.out[(size_t)token * g.out_stride + (size_t)head * D + e] = add_shares<float>(
+            ends, 2, part + e, D, g.ho.sink ? g.ho.sink[head] : -INFINITY, ra_head_gate<float>(g.ho, token, head));
+    }
+    __syncthreads();
   }
+}
+
+// A token on its own, a share a wave.
+template <int D, int GH>
+__global__ void __launch_bounds__(SHARES * RA_WAVE) attention_f32_token_kernel(F32Attention g) {
+  __shared__ float part[SHARES][GH][D], ends[SHARES][GH][2];
+  const int share = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h0 = blockIdx.x * GH;
+  const int t = g.token_list ? g.token_list[blockIdx.y] : blockIdx.y;
+  walk_share<D, GH>(g, t, h0, g.block_tables + (size_t)g.seq_of_token[t] * g.max_blocks, share, part[share][0], ends[share][0]);
   __syncthreads();
-  for (int i = threadIdx.x; i < GH * D; i += blockDim.x) {
-    const int h = i / D, e = i % D, a = h0 + h;
-    float top = -INFINITY;
-    for (int w = 0; w < SHARES; ++w) top = fmaxf(top, part[w][h][D]);
-    float sum = 0.f, den = 0.f;
-    for (int w = 0; w < SHARES; ++w) {
-      if (part[w][h][D + 1] == 0.f) continue;      // nothing seen
-      const float f = expf(part[w][h][D] - top);
-      sum = fmaf(f, part[w][h][e], sum);
-      den = fmaf(f, part[w][h][D + 1], den);
-    }
-    if (g.ho.sink) den += expf(g.ho.sink[a] - top);
-    g.out[(size_t)t * g.out_stride + (size_t)a * D + e] = sum * (ra_head_gate<float>(g.ho, t, a) / den);
+  for (int x = threadIdx.x; x < GH * D; x += blockDim.x) {
+    const int h = x / D, e = x % D, a = h0 + h;
+    g.out[(size_t)t * g.out_stride + (size_t)a * D + e] = add_shares<float>(
+        &ends[0][h][0], GH * 2, &part[0][h][e], GH * D, g.ho.sink ? g.ho.sink[a] : -INFINITY, ra_head_gate<float>(g.ho, t, a));
   }
 }
 
 template <int D, int GH>
-int go(const F32Attention& g, int n_tokens, hipStream_t stream) {
-  const int pairs = g.Hq / GH;
-  // a wave a share where that fills the chip; with many tokens two, so that a short context still gives every wave a tile
-  // or two
-  const int waves = (long)pairs * n_tokens > 16L * ra_cu_count() ? 2 : 8;
-  attention_f32_kernel<D, GH><<<dim3(pairs, n_tokens), waves * RA_WAVE, 0, stream>>>(g);
+int go_tokens(const F32Attention& g, hipStream_t stream) {
+  attention_f32_token_kernel<D, GH><<<dim3(g.Hq / GH, g.n_tokens), SHARES * RA_WAVE, 0, stream>>>(g);
+  RA_LAUNCH_CHECK("attention_f32");
+  return 0;
+}
+
+template <int D>
+int go(F32Attention g, int n_requests, hipStream_t stream) {
+  const int group = g.Hq / g.Hkv;
+  const long cus = ra_cu_count();
+  g.heads = 1;
+  while (g.heads < ROWS && group % (2 * g.heads) == 0) g.heads *= 2;
+  // Tokens on their own while their workgroups find room at once, and where most of the products' 16 columns would stay empty; a request
+  // of several tokens up to twice as many, for its rows are one workgroup's. Two heads share what is read of a key they both read, but
+  // for so few that the chip has room for each. 32 heads of 128 on 8 KV heads, us, a head each / two / 16 rows: 1 token at 300 keys
+  // 8.9 / 10.4 / 15.4, 4 tokens of 4 requests at 600 18.0 / 15.3 / 22.2, 8 of 8 28.5 / 19.2 / 23.1, 16 of 16 at 500 43.0 / 25.5 / 21.5,
+  // 64 of 64 161 / 83 / 52; prompts of 16 6.7 / 7.0 / 10.2, 24 9.4 / 9.7 / 10.1, 40 11.9 / 12.9 / 10.5, 80 19.3 / 20.5 / 11.8; on 32 KV
+  // heads, 16 of 16 at 500 43.4 / - / 52.9, a prompt of 200 51.8 / - / 18.0.
+  const int each = n_requests > 0 && n_requests < g.n_tokens ? g.n_tokens / n_requests : 1;
+  const bool two = D <= 128 && group % 2 == 0;
+  const long alone = (long)g.Hq * g.n_tokens / (two ? 2 : 1);
+  if (g.heads * (each < ROWS ? each : ROWS) < 2 || alone <= (each > 1 ? cus : cus / 2)) {
+    if constexpr (D <= 128)
+      if (two && (long)g.Hq * g.n_tokens * 4 > cus) return go_tokens<D, 2>(g, stream);
+    return go_tokens<D, 1>(g, stream);
+  }
+  const long pairs = g.Hq / g.heads;
+  const int nt = ROWS / g.heads, tiles = (g.n_tokens + nt - 1) / nt;
+  // a workgroup a request's run of tokens where a workgroup a token would be a few rounds of the chip, else one for all runs of its rows
+  const int z = pairs * g.n_tokens <= 8 * cus ? (nt < g.n_tokens ? nt : g.n_tokens) : 1;
+  const int waves = D > 128 || pairs * tiles > cus ? 4 : 8;
+  constexpr size_t lds = (size_t)SHARES * ROWS * (D + 6) * sizeof(float);
+  constexpr int W = D <= 128 ? 8 : 4;
+  if (lds > 64 * 1024) {
+    const hipError_t e = hipFuncSetAttribute((const void*)attention_f32_kernel<D, W>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return ra_fail("attention_f32: %s", hipGetErrorString(e));
+  }
+  attention_f32_kernel<D, W><<<dim3(pairs, tiles, z), waves * RA_WAVE, lds, stream>>>(g);
   RA_LAUNCH_CHECK("attention_f32");
   return 0;
 }
@@ -186,19 +513,20 @@ int go(const F32Attention& g, int n_tokens, hipStream_t stream) {
 }  // namespace
 
 // Whether the kernel takes these sizes (16-byte reads of the cache besides; the queries are read element by element).
-bool ra_attention_f32_takes(const void* kcache, const void* vcache, int d) {
-  return (d == 64 || d == 128 || d == 256) && (uintptr_t)kcache % 16 == 0 && (uintptr_t)vcache % 16 == 0;
+bool ra_attention_f32_takes(const void* kcache, const void* vcache, int d, int block_size, int max_blocks) {
+  const long tiles = block_size / 16;      // a block's, and the range in which a product stands for a division by them
+  return (d == 64 || d == 128 || d == 256) && (uintptr_t)kcache % 16 == 0 && (uintptr_t)vcache % 16 == 0
+         && max_blocks * tiles * tiles < (1l << 32);
 }
 
 int ra_attention_f32(const float* q, int q_stride, float* out, int out_stride, const float* kcache, const float* vcache,
                      const int* block_tables, int max_blocks, const int* token_list, const int* seq_of_token,
-                     const int* positions, int n_tokens, int block_size, int Hq, int Hkv, int d, float scale, int window,
-                     int aligned, int keep, RaScoreMod mod, RaHeadOut ho, hipStream_t stream) {
+                     const int* positions, int n_tokens, int n_requests, int block_size, int Hq, int Hkv, int d, float scale,
+                     int window, int aligned, int keep, RaScoreMod mod, RaHeadOut ho, hipStream_t stream) {
   const F32Attention g = {q, q_stride, out, out_stride, kcache, vcache, block_tables, max_blocks, token_list, seq_of_token,
-                          positions, block_size, Hq, Hkv, scale, window, aligned, keep, mod, ho};
-  const bool even = Hq / Hkv % 2 == 0;     // two heads share what is read of a key where they read the same one
-  if (d == 64) return even ? go<64, 2>(g, n_tokens, stream) : go<64, 1>(g, n_tokens, stream);
-  if (d == 128) return even ? go<128, 2>(g, n_tokens, stream) : go<128, 1>(g, n_tokens, stream);
-  if (d == 256) return go<256, 1>(g, n_tokens, stream);
+                          positions, n_tokens, 1, block_size, block_size / 16, (1ull << 32) / (block_size / 16) + 1, Hq, Hkv, scale, window, aligned, keep, mod, ho};
+  if (d == 64) return go<64>(g, n_requests, stream);
+  if (d == 128) return go<128>(g, n_requests, stream);
+  if (d == 256) return go<256>(g, n_requests, stream);
   return ra_fail("attention_f32: head size %d", d);
 }
