@@ -139,7 +139,9 @@ class MixtureOfExperts:
         p = self.routing
         T = x.shape[0]
         n = self.experts * self.ff + self.shared
-        if p.weights == "sigmoid" and self._together(ops, x, self.w_gate_up, self.experts):
+        routed = self.experts + self.identity
+        way = self._way(ops, x, self.w_gate_up, routed, "moe_gate_up_chosen")
+        if way == "all" and p.weights == "sigmoid" and hasattr(ops, "moe_choose_scale"):
             gu = torch.empty((T, 2 * n), dtype=self.dtype, device=x.device)
             act = self._choose_and_scale(ops, x, self.w_gate_up, gu, n, shared=self.shared, scoring="sigmoid",
                                          scale=float(p.weight_scale), groups=int(p.groups), groups_kept=int(p.groups_kept),
@@ -147,7 +149,6 @@ class MixtureOfExperts:
             return self._project_down(ops, act, resid, resid_scale)
         ids = torch.empty((T, self.top), dtype=torch.int32, device=x.device)
         weights = torch.empty((T, self.top), dtype=torch.float32, device=x.device)
-        routed = self.experts + self.identity
         shared_logit = None
         if p.weights == "table":
             ops.moe_table_route(batch.token_ids, self.table, ids, weights)
@@ -160,8 +161,7 @@ class MixtureOfExperts:
         else:
             ops.moe_route(x, self.router, self.top, ids, weights, scoring="sigmoid", scale=float(p.weight_scale),
                           groups=int(p.groups), groups_kept=int(p.groups_kept), group_top=int(p.group_top))
-        chosen = getattr(ops, "moe_reads_chosen", None)
-        if chosen is not None and hasattr(ops, "moe_gate_up_chosen") and chosen(T, self.top, routed):
+        if way == "chosen":
             # so few tokens that most experts are not asked for: only the chosen experts' rows and the shared
             # expert's are read; the identity experts' share is added behind the down projection's sum
             act = torch.empty((T, self.top * self.ff + self.shared), dtype=self.dtype, device=x.device)
@@ -170,7 +170,7 @@ class MixtureOfExperts:
             out = torch.empty((T, self.spec.hidden), dtype=self.dtype, device=x.device)
             ops.moe_down_gated_chosen(act, self.w_down, ids, weights, x, out, self.experts, self.ff, self.shared)
             return out
-        if self._grouped(ops, x, self.w_gate_up, routed):
+        if way == "grouped":
             return self._forward_grouped(ops, x, self.w_gate_up, ids, weights, shared_logit, resid, resid_scale)
         gu = torch.empty((T, 2 * n), dtype=self.dtype, device=x.device)
         ops.linear(x, self.w_gate_up, gu)
@@ -199,13 +199,14 @@ class MixtureOfExperts:
         ops.linear(act, self.w_down, out)
         return out
 
-    def _together(self, ops, x, w_up, routed: int) -> bool:
-        """Whether a step runs every expert, so that its products do not wait for the choice: the router's logits come with them, and the
-        choice is made where it weighs them."""
-        if not hasattr(ops, "moe_choose_scale"):
-            return False
+    def _way(self, ops, x, w_up, routed: int, few: str) -> str:
+        """How a step's rows meet their experts: "chosen", few rows that read only these (the operation ``few``); "grouped", many, each
+        through its own; or "all", products that do not wait for the choice: the router's logits come with them, and the choice is made where
+        it weighs them. Asked once a layer: a step of some 150 rows waits for the host."""
         chosen = getattr(ops, "moe_reads_chosen", None)
-        return not (chosen is not None and chosen(x.shape[0], self.top, routed)) and not self._grouped(ops, x, w_up, routed)
+        if chosen is not None and hasattr(ops, few) and chosen(x.shape[0], self.top, routed):
+            return "chosen"
+        return "grouped" if self._grouped(ops, x, w_up, routed) else "all"
 
     def _choose_and_scale(self, ops, x, w_up, up, n, **choice):
         logits = torch.empty((x.shape[0], self.router.shape[0]), dtype=torch.float32, device=x.device)
@@ -245,14 +246,14 @@ class MixtureOfExperts:
         ops = kernels.current()
         T = x.shape[0]
         n = self.experts * self.ff
-        if self._together(ops, x, self.w_up, self.experts):
+        way = self._way(ops, x, self.w_up, self.experts, "moe_up_chosen")
+        if way == "all" and hasattr(ops, "moe_choose_scale"):
             up = torch.empty((T, n), dtype=self.dtype, device=x.device)
             return self._project_down(ops, self._choose_and_scale(ops, x, self.w_up, up, n), resid)
         ids = torch.empty((T, self.top), dtype=torch.int32, device=x.device)
         weights = torch.empty((T, self.top), dtype=torch.float32, device=x.device)
         ops.moe_route(x, self.router, self.top, ids, weights)
-        chosen = getattr(ops, "moe_reads_chosen", None)
-        if chosen is not None and chosen(T, self.top, self.experts):
+        if way == "chosen":
             # so few tokens that most experts are not asked for: only the chosen experts' rows are read
             act = torch.empty((T * self.top, self.ff), dtype=self.dtype, device=x.device)
             ops.moe_up_chosen(x, self.w_up, ids, weights, act, self.ff)
@@ -262,7 +263,7 @@ class MixtureOfExperts:
             out = torch.empty((T, self.spec.hidden), dtype=self.dtype, device=x.device)
             ops.moe_down_chosen(act, self.w_down, ids, self.ff, out=out)
             return out
-        if self._grouped(ops, x, self.w_up, self.experts):
+        if way == "grouped":
             return self._forward_grouped(ops, x, self.w_up, ids, weights, None, resid, 1.0)
         up = torch.empty((T, n), dtype=self.dtype, device=x.device)
         ops.linear(x, self.w_up, up)
