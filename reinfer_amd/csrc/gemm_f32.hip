@@ -1,26 +1,34 @@
 // Matrix products of the 32-bit path, C[M,N] = A[M,K] . W[N,K]^T (+ bias[N]), on the bfloat16 matrix cores, to float precision.
 //
-// A float is the sum of three bfloat16 numbers, exactly (but for bits below 2^-133): its value rounded, what that leaves rounded, and the
-// rest. Of the nine products of the parts the six largest are summed, in float; what is left out is below 2^-25 of a product, a
-// rounding of the sum 2^-24 of it. Measured against 64 bits over normal random numbers the sums are nearer than those of the
-// float matrix cores: K 2560 3.43e-7 of the result's norm against 4.08e-7, K 4096 3.47 / 4.09, K 9728 5.59 / 6.27 (a product of
-// 32 k is rounded into its sum once a term, where the float cores round for every four k).
+// A float is the sum of three bfloat16 numbers: its value rounded, what that leaves rounded, and the rest (Henry, Tang and Heinecke,
+// "Leveraging the bfloat16 Artificial Intelligence Datatype for Higher-Precision Computations", 2019). Split 2^24 times as large it is so
+// exactly down to the last subnormal bit. Of the nine products of the parts the six largest are summed, in float: the largest in a sum
+// of its own, the five others in a second one, 2^8 times smaller. What this keeps, U being 2^-24:
+//   one product   what is left out of it is below 1.001 U of it (2 2^-8 2^-17 and 2^-34; 0.99 for the mantissa 1 + 2^-8 - 2^-17), and one
+//                 rounding, below U: measured up to 0.94 of a last place, a float product 0.50;
+//   a sum         is rounded once for every eight k (a product of 32 k adds them eight at a time), where the float matrix cores round for every
+//                 one. Over normal random numbers the error against 64 bits is 1.35e-7 of the result's norm at K 2560 (float matrix cores
+//                 4.08e-7), 1.39e-7 at 4096 (4.09e-7) and 2.12e-7 at 9728 (6.27e-7). With all six products in one sum it was 3.43, 3.47
+//                 and 5.59e-7 and had a mean of -0.6, -0.7 and -1.7e-7, for these cores cut what lies below 2^-31 of the largest
+//                 that they add towards minus infinity, and did so six times for every eight k; now the mean is below 1e-9;
+//   magnitudes    all floats; rows of 2^-140 are as near as others. Sums past 2^80 and what is not finite are worked out again from the floats.
 //
 // Up to 32 rows (gemm_f32_stream_kernel) the product is bound by reading the weights once. A workgroup has 16 features, its
 // waves share K out and add their sums through LDS in a fixed order. The weights go by way of a piece of LDS of each wave's own:
 // loaded in the products' order a load is 64 bytes of each of 16 rows, half a line each, and takes twice the time of whole lines.
 // Splitting is issue time beside the loads' waits: with the next loads asked for behind it 15 % slower, with the rows split by every
-// lane that multiplies them 10 %. Weights from memory, float matrix cores / here, us: 4 rows 6144 x 2560 19.7 / 17.0, 2560 x 4096
-// 14.3 / 13.8, 19456 x 2560 41.4 / 39.1, 2560 x 9728 29.5 / 26.0, 151936 x 2560 265 / 271; 16 rows 23.5 / 21.7, 16.4 / 15.5, 51 / 48,
-// 36.7 / 33.0; 32 rows 36.6 / 34.0, 25.8 / 23.4, 80.5 / 79, 57 / 54.5. Runs of 64 k, or three or four in flight, are slower.
+// lane that multiplies them 10 %. Weights from memory, float matrix cores / here, us: 4 rows 6144 x 2560 19.7 / 17.4, 2560 x 4096
+// 15.8 / 14.3, 19456 x 2560 41.5 / 39.2, 2560 x 9728 29.3 / 26.2; 12 rows 21.8 / 20.9, 17.5 / 16.1, 46.9 / 45.0, 33.4 / 31.3; 32 rows
+// 37.5 / 33.0, 28.0 / 24.8, 80 / 73.5, 56.2 / 50.8. Where the stream is at memory rate splitting costs what it takes: 4 rows 151936 x 2560
+// 264 / 270 (5.8 TB/s), 12 rows 324 / 329, 32 rows 554 / 507; 20 or 24 waves a CU in place of 16 are no faster there, and a tenth
+// slower from 12 rows on. Runs of 64 k, or three or four in flight, are slower.
 //
 // From 33 rows on (gemm_f32_tile_kernel) tiles of both operands go through LDS, split on the way. Six bfloat16 products take 96 cycles
-// of a matrix core where the float ones take 256. What bounds them is issue: of a SIMD's time at 256 rows a tile 53 % are products, 27 %
-// other vector instructions, which find little room beside them, and 18 % waits; and the chip's power, whose clock is 1.95 GHz
-// (on zeros 2.35 and a sixth faster). In a loop over other weights, float matrix cores / here, us: 1119 x 19456 x 2560 880 / 620 (180
-// TFLOP/s), 1119 x 2560 x 9728 500 / 330, 2048 x 19456 x 2560 1520 / 1030, 300 x 6144 x 2560 103 / 84, 64 x 19456 x 2560 71 / 62. Tiles
-// split by every wave that multiplies them, the compiler's order, two waves a SIMD: 664 for the first. Dot products with (-1, 0) to take
-// a part off gave 1 %.
+// of a matrix core where the float ones take 256. What bounds them is the chip's power (the clock is 1.93 GHz; on zeros 2.4 and a quarter
+// faster) and issue: beside each product stand one and a half other vector instructions. In a loop over other weights, float matrix
+// cores / here, us: 1119 x 19456 x 2560 875 / 606 (184 TFLOP/s), 1119 x 2560 x 9728 470 / 317, 2048 x 19456 x 2560 1510 / 1052, 300 x 6144 x 2560
+// 96 / 68, 64 x 19456 x 2560 65 / 59. One wave a SIMD with tiles of 256 rows (one sum; with two they do not fit its registers) took 602, 303, 995,
+// 85 and 61; all eight products but the smallest 774 for the first where six took 677.
 #include <type_traits>
 
 #include "common.h"
@@ -33,18 +41,33 @@ struct F32Parts {
   bf16x8_t h, m, l;
 };
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-// Two floats rounded, as the low and the high half of a word; what that leaves of them stays behind. (The empty statement has the
-// compiler take the halves from the word: left to itself it converts each float once more for that.)
-__device__ __forceinline__ unsigned f32_part(float& a, float& b) {
+// Two floats rounded, as the low and the high half of a word (the empty statement has the compiler take the halves from the word: left to
+// itself it converts each float once more for that), and what that leaves of them.
+__device__ __forceinline__ unsigned f32_pack(float a, float b) {
   unsigned u = __builtin_bit_cast(unsigned, (bf16x2_t){(bf16_t)a, (bf16_t)b});
   asm("" : "+v"(u));
+  return u;
+}
+__device__ __forceinline__ void f32_rest(unsigned u, float& a, float& b) {
   a -= __builtin_bit_cast(float, u << 16);
   b -= __builtin_bit_cast(float, u & 0xFFFF0000u);
+}
+__device__ __forceinline__ unsigned f32_part(float& a, float& b) {
+  const unsigned u = f32_pack(a, b);
+  f32_rest(u, a, b);
   return u;
 }
 typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
+// Floats are split 2^24 times as large, so that the last bit of the smallest is no part's below what bfloat16 holds; a sum is 2^48 times as
+// large, then.
+#define F32_SCALE 0x1p24f
 __device__ __forceinline__ F32Parts f32_split(f32x4_t a, f32x4_t b) {
-  float v[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+  float v[8];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    v[e] = a[e] * F32_SCALE;
+    v[4 + e] = b[e] * F32_SCALE;
+  }
   u32x4_t p[3];
 #pragma unroll
   for (int i = 0; i < 3; ++i)
@@ -52,15 +75,38 @@ __device__ __forceinline__ F32Parts f32_split(f32x4_t a, f32x4_t b) {
     for (int e = 0; e < 4; ++e) p[i][e] = f32_part(v[2 * e], v[2 * e + 1]);
   return {__builtin_bit_cast(bf16x8_t, p[0]), __builtin_bit_cast(bf16x8_t, p[1]), __builtin_bit_cast(bf16x8_t, p[2])};
 }
-// Term t of the product of two floats in parts, the smallest first: every kernel adds them in this order.
+// Term t of the product of two floats in parts, the smallest first: every kernel adds them in this order. The largest has a sum of its own;
+// the others' sum is some 2^8 times smaller, and so are its roundings.
 #define F32_TERMS 6
 __device__ __forceinline__ f32x4_t f32_term(int t, const F32Parts& w, const F32Parts& a, f32x4_t c) {
   const bf16x8_t& x = t == 0 ? w.l : t == 2 || t == 3 ? w.m : w.h;
   const bf16x8_t& y = t == 1 ? a.l : t == 2 || t == 4 ? a.m : a.h;
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, y, c, 0, 0, 0);
 }
-// The parts of an infinity and of a float that rounds to one are no numbers, and a part that is zero times an infinity is none either: a
-// sum that is not finite is worked out again from the floats.
+struct F32Sum {
+  f32x4_t h, s;                            // of the largest term, of the others
+};
+__device__ __forceinline__ void f32_add_term(int t, const F32Parts& w, const F32Parts& a, F32Sum& c) {
+  if (t == F32_TERMS - 1) c.h = f32_term(t, w, a, c.h);
+  else c.s = f32_term(t, w, a, c.s);
+}
+// A block's sum; each operation is rounded by itself wherever it stands.
+__device__ __forceinline__ f32x4_t f32_block(const F32Sum& c) {
+#pragma clang fp contract(off)
+  f32x4_t v;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = (c.h[e] + c.s[e]) * (1.f / F32_SCALE / F32_SCALE);
+  return v;
+}
+__device__ __forceinline__ f32x4_t f32_plus(f32x4_t a, f32x4_t b) {
+#pragma clang fp contract(off)
+#pragma unroll
+  for (int e = 0; e < 4; ++e) a[e] += b[e];
+  return a;
+}
+
+// The parts of an infinity and of a float that is one 2^24 times as large are no numbers: a sum that is not finite is worked out again from
+// the floats.
 __device__ __forceinline__ bool f32_off(float v) { return !(fabsf(v) <= 3.402823466e38f); }
 __device__ __forceinline__ float f32_again(const float* __restrict__ a, const float* __restrict__ w, int K) {
   float s = 0.f;
@@ -73,10 +119,10 @@ __device__ __forceinline__ float f32_again(const float* __restrict__ a, const fl
 }
 
 // ------------------------------------------------------------------------------------------------ the order of the sums
-// K is summed in up to eight blocks of at least 512 k, whose number and length follow from K alone. A block is one chain of
-// 16x16x32 products over its pieces of 32 k, six a piece. The blocks' sums are added in their order, then the bias. Both kernels
-// keep this order, so a row's result does not depend on how many rows stand beside it: a request's 32-bit results are the same
-// bits alone and in any step.
+// K is summed in up to eight blocks of at least 512 k, whose number and length follow from K alone. A block is two chains of
+// 16x16x32 products over its pieces of 32 k, one and five a piece, that are added at its end. The blocks'
+// sums are added in their order, then the bias. Both kernels keep this order, so a row's result does not depend on how many rows stand
+// beside it: a request's 32-bit results are the same bits alone and in any step.
 struct KBlocks {
   int n, k;                                // how many, and k of one (a multiple of 64)
 };
@@ -170,9 +216,10 @@ gemm_f32_stream_kernel(const float* __restrict__ A, const float* __restrict__ W,
     load_w(d);
     load_a(d);
   }
-  f32x4_t acc[MT];
+  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+  F32Sum acc[MT];
 #pragma unroll
-  for (int t = 0; t < MT; ++t) acc[t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < MT; ++t) acc[t] = {zero, zero};
   int step = 0, n0 = (int)blockIdx.x * 16, buf = 0;                // where the products are
   for (int base = 0; base < total; base += DEPTH) {
 #pragma unroll
@@ -185,7 +232,7 @@ gemm_f32_stream_kernel(const float* __restrict__ A, const float* __restrict__ W,
       if constexpr (SHARED) {
 #pragma unroll
         for (int i = 0; i < A_LOADS; ++i) {
-          float v[4] = {a[d][i][0], a[d][i][1], a[d][i][2], a[d][i][3]};
+          float v[4] = {a[d][i][0] * F32_SCALE, a[d][i][1] * F32_SCALE, a[d][i][2] * F32_SCALE, a[d][i][3] * F32_SCALE};
 #pragma unroll
           for (int p = 0; p < 3; ++p) {
             const unsigned lo = f32_part(v[0], v[1]), hi = f32_part(v[2], v[3]);
@@ -211,7 +258,7 @@ gemm_f32_stream_kernel(const float* __restrict__ A, const float* __restrict__ W,
 #pragma unroll
       for (int e = 0; e < F32_TERMS; ++e)
 #pragma unroll
-        for (int t = 0; t < MT; ++t) acc[t] = f32_term(e, y, x[t], acc[t]);
+        for (int t = 0; t < MT; ++t) f32_add_term(e, y, x[t], acc[t]);
       if (!SHARED) {
         __builtin_amdgcn_sched_barrier(0);
         load_a(d);
@@ -224,15 +271,15 @@ gemm_f32_stream_kernel(const float* __restrict__ A, const float* __restrict__ W,
     // while the next tile's go to the other buffer, and a wave writes a buffer again only behind the next barrier.
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
-      sums[((buf * waves + wave) * MT + t) * RA_WAVE + lane] = acc[t];
-      acc[t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+      sums[((buf * waves + wave) * MT + t) * RA_WAVE + lane] = f32_block(acc[t]);
+      acc[t] = {zero, zero};
     }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     for (int t = wave; t < MT; t += waves) {
-      f32x4_t v = sums[(buf * waves * MT + t) * RA_WAVE + lane];
+      f32x4_t v = zero;
 #pragma unroll
-      for (int x = 1; x < 8; ++x)
-        if (x < waves) v += sums[((buf * waves + x) * MT + t) * RA_WAVE + lane];
+      for (int x = 0; x < 8; ++x)
+        if (x < waves) v = f32_plus(v, sums[((buf * waves + x) * MT + t) * RA_WAVE + lane]);
       const int m = t * 16 + r;
       if (m < M) {
 #pragma unroll
@@ -268,46 +315,37 @@ struct F32Tile {
   int block_k, range_blocks;               // k of a block (a multiple of 64), blocks of a range
 };
 
-// Large tiles' products are in assembly, so that a sum stays in its registers (of sums that fill the accumulation registers the
-// compiler moves some to and fro, and spills others at the ends of blocks). It then does not see the wait states that belong between a
-// product and an ordinary access to its sums, or between a copy of an operand, which it may make ahead of a block, and the product.
-__device__ __forceinline__ void f32_term_kept(int t, const F32Parts& w, const F32Parts& a, f32x4_t& c) {
-  const bf16x8_t& x = t == 0 ? w.l : t == 2 || t == 3 ? w.m : w.h;
-  const bf16x8_t& y = t == 1 ? a.l : t == 2 || t == 4 ? a.m : a.h;
-  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(x), "v"(y));
-}
-template <int TN, int TM>
-__device__ __forceinline__ void f32_settle(f32x4_t (&acc)[TN][TM]) {
-  f32x4_t* p = &acc[0][0];
-#pragma unroll
-  for (int i = 0; i < TN * TM; i += 4)
-    asm volatile("s_nop 15\n\ts_nop 3" : "+a"(p[i]), "+a"(p[i + 1]), "+a"(p[i + 2]), "+a"(p[i + 3]));
-}
-template <int TN>
-__device__ __forceinline__ void f32_ready(const F32Parts (&y)[TN], const F32Parts& x) {
-#pragma unroll
-  for (int i = 0; i < TN; ++i) asm volatile("s_nop 3" ::"v"(y[i].h), "v"(y[i].m), "v"(y[i].l));
-  asm volatile("s_nop 3" ::"v"(x.h), "v"(x.m), "v"(x.l));
-}
 // The instructions stay in the order that they are written in.
 #define F32_ORDER __builtin_amdgcn_sched_barrier(0)
 
-// A workgroup of four waves a tile of 32 TM rows and 128 features and range of k, in 2 x 2 quarters. A step is 32 k of both
-// operands: read from memory as floats, in whole lines, two steps ahead, into registers; split, each once a workgroup, and written to
+// Four neighbouring features of a row, n the first of N.
+__device__ __forceinline__ void f32_store(float* to, f32x4_t v, const float* bias, int n, int N, bool whole) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (bias && n + e < N) v[e] += bias[n + e];
+  if (whole) {
+    *(f32x4_t*)to = v;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (n + e < N) to[e] = v[e];
+  }
+}
+// A workgroup of WM x WN waves a tile of 32 WM rows and 128 features and range of k; a wave 32 rows and 16 TN features of it. A step is 32 k of
+// both operands: read from memory as floats, in whole lines, two steps ahead, into registers; split, each once a workgroup, and written to
 // LDS one step ahead, part by part in tiles of 16 rows in the products' order: the 16 bytes of row r, k 8 q .. + 7 lie at place
 // 16 q + r, or r ^ 8 for q 2 and 3; the lanes that write side by side hold pieces of q 0 and 2 of four rows and of q 1 and 3 of the
-// four behind them, which fall on all banks. A tile's operands have descriptors of their own, whose ends are those of the
-// matrices: rows past them are zeros.
+// four behind them. A tile's operands have descriptors of their own, whose ends are those of the matrices: rows past them are zeros.
 //
-// A step's products go row tile by row tile, all four columns' operands in registers and a row tile's read one ahead. The barrier stands
-// before the last row tile: there all of stage s has been read and all of stage s + 1 written, so that the next operands are
-// read, and the first pieces of stage s + 2 written, behind products that are still to issue. Splitting stands between the
-// products as well: a wave issues in order, and has the SIMD to itself but for tiles of 64 rows, of which a CU holds two.
-template <int TM, bool CUT>
-__global__ void __launch_bounds__(256, TM == 2 ? 2 : 1) gemm_f32_tile_kernel(F32Tile g) {
-  constexpr int TN = 4, BM = 32 * TM, BN = 128;
-  constexpr bool KEPT = TM >= 6;
-  constexpr int PA = BM / 32, PB = BN / 32, P = PA + PB;          // a thread's pieces of a stage: one of every 32 rows
+// A step's products go row tile by row tile, two columns in turn, with all columns' operands in registers. The barrier stands between the
+// row tiles: there all of stage s has been read and all of stage s + 1 written (a few products before: 4 % of the time), so that the next
+// operands are read, and the first pieces of stage s + 2 written, behind products that are still to issue. Splitting stands between the
+// products as well, two or three instructions at a time. Two waves a SIMD fill each other's gaps: one, with tiles of 128 rows in quarters
+// of 64 and four columns in turn, took 880 us where two take 774 (eight products, 1119 x 19456 x 2560).
+template <int WM, int WN, int TN, bool CUT>
+__global__ void __launch_bounds__(WM * WN * RA_WAVE, 2) gemm_f32_tile_kernel(F32Tile g) {
+  constexpr int TM = 2, BM = WM * TM * 16, BN = WN * TN * 16;
+  constexpr int ROWS = WM * WN * 8, PA = BM / ROWS, PB = BN / ROWS, P = PA + PB;     // a thread's pieces of a stage: one of every so many rows
   constexpr int EARLY = P / TM;                                   // of them, written behind the barrier
   constexpr int TILE = 3 * 1024, STAGE = (BM + BN) / 16 * TILE;   // bytes
   constexpr unsigned NOWHERE = 0xFFFFFFF0u;
@@ -327,12 +365,12 @@ __global__ void __launch_bounds__(256, TM == 2 ? 2 : 1) gemm_f32_tile_kernel(F32
       const_cast<float*>(g.a + (size_t)m0 * g.lda), 0, (int)(unsigned)(((size_t)(a_rows - 1) * g.lda + g.K) * 4), 0x00020000);
   const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<float*>(g.w + (size_t)n0 * g.K), 0, (int)(unsigned)((size_t)w_rows * g.K * 4), 0x00020000);
-  // piece c (16 bytes, 4 k) of row lr of each 32
+  // piece c (16 bytes, 4 k) of row lr of each ROWS
   const int c = lane & 7, lr = wave * 8 + ((lane >> 3) & 3) + 4 * ((lane >> 5) ^ ((c >> 1) & 1));
   unsigned off[P];
 #pragma unroll
   for (int i = 0; i < P; ++i) {
-    const int r = lr + (i < PA ? i : i - PA) * 32;
+    const int r = lr + (i < PA ? i : i - PA) * ROWS;
     off[i] = r < (i < PA ? a_rows : w_rows) ? ((unsigned)r * (unsigned)(i < PA ? g.lda : g.K) + c * 4) * 4u : 0x80000000u;
   }
   F32_LDS char* to[2];
@@ -345,34 +383,43 @@ __global__ void __launch_bounds__(256, TM == 2 ? 2 : 1) gemm_f32_tile_kernel(F32
     held[set][i] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(i < PA ? a_rsrc : w_rsrc, (int)o, 0, 0));
   };
   unsigned part[3][2];
-  // a piece's way to LDS in operations of about five instructions: its first and second two floats, the writes, the next load
-  constexpr int OPS = 6;
+  // a piece's way to LDS in operations of about three instructions, which is what there is room for beside a product: its first and second
+  // two floats, the writes, the next load
+  constexpr int OPS = 10;
   auto piece = [&](int i, int op, int set, int buf, int next) {
-    if (op < 4) {
+    if (op < 8) {
+      const int two = op >> 2;
       f32x4_t& v = held[set][i];
-      float a = v[op >> 1 << 1], b = v[(op >> 1 << 1) + 1];
-      if ((op & 1) == 0) {
-        part[0][op >> 1] = f32_part(a, b);
+      float a = v[2 * two], b = v[2 * two + 1];
+      if (op % 4 == 0) {
+        a *= F32_SCALE;
+        b *= F32_SCALE;
+        part[0][two] = f32_pack(a, b);
+      } else if (op % 4 == 1) {
+        f32_rest(part[0][two], a, b);
+      } else if (op % 4 == 2) {
+        part[1][two] = f32_pack(a, b);
       } else {
-        part[1][op >> 1] = f32_part(a, b);
-        part[2][op >> 1] = f32_part(a, b);
+        f32_rest(part[1][two], a, b);
+        part[2][two] = f32_pack(a, b);
       }
-      v[op >> 1 << 1] = a;
-      v[(op >> 1 << 1) + 1] = b;
-    } else if (op == 4) {
-      F32_LDS char* d = to[buf] + i * 2 * TILE;
+      v[2 * two] = a;
+      v[2 * two + 1] = b;
+    } else if (op == 8) {
+      F32_LDS char* d = to[buf] + i * (ROWS / 16) * TILE;
 #pragma unroll
       for (int x = 0; x < 3; ++x) *(F32_LDS unsigned long long*)(d + x * 1024) = part[x][0] | (unsigned long long)part[x][1] << 32;
     } else {
       load(next, i, set);
     }
   };
+  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
   f32x4_t sum[TN][TM];                       // of the blocks before this one
 #pragma unroll
   for (int i = 0; i < TN; ++i)
 #pragma unroll
-    for (int j = 0; j < TM; ++j) sum[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-  const int wm = (wave >> 1) * TM * 16, wn = (wave & 1) * 64;
+    for (int j = 0; j < TM; ++j) sum[i][j] = zero;
+  const int wm = wave / WN * TM * 16, wn = wave % WN * TN * 16;
   const int row = lane & 15, quarter = lane >> 4;
   const F32_LDS char* const from = (F32_LDS char*)lds + quarter * 256 + ((row ^ ((quarter >> 1) * 8)) * 16);
   const F32_LDS char *xs[2] = {from + wm / 16 * TILE}, *ys[2] = {from + (BM + wn) / 16 * TILE};
@@ -405,37 +452,34 @@ __global__ void __launch_bounds__(256, TM == 2 ? 2 : 1) gemm_f32_tile_kernel(F32
   const int ld = CUT ? g.N : g.ldc;
   const float* b = CUT ? nullptr : g.bias;
   const bool whole = g.N % 4 == 0 && ld % 4 == 0 && (uintptr_t)g.c % 16 == 0;
-  auto step = [&](int s, f32x4_t (&acc)[TN][TM], auto odd) {
-    constexpr int buf = odd, MF = TN * F32_TERMS;                 // products of a row tile
-    constexpr int LATE = (P - EARLY) * OPS, FIRST = MF * (TM - 1);
+  auto step = [&](int s, F32Sum (&acc)[TN][TM], auto odd) {
+    constexpr int buf = odd, MF = TN * F32_TERMS;                 // of a row tile
+    // the last write of stage s + 1 some products before the barrier, which waits for it
+    constexpr int LATE = (P - EARLY) * OPS, FIRST = MF * (TM - 1) - (TN == 4 ? 6 : 2);
     F32_ORDER;
 #pragma unroll
-    for (int j = 0; j < TM; ++j) {
-      if (j == TM - 1) {
+    for (int u = 0; u < TM; ++u) {
+      if (u == TM - 1) {
         // this wave's pieces of stage s + 1 are written and its reads of stage s done; behind the barrier that is so of all waves
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         F32_ORDER;
       }
 #pragma unroll
       for (int m = 0; m < MF; ++m) {
-        // all four columns in turn; in the last row tile two, as their operands are then free for the next stage's in the middle and
-        // at the end, and so in the first, where the other two are on their way
-        const bool two = j == 0 || j == TM - 1;
-        const int i = two ? m / (2 * F32_TERMS) * 2 + m % 2 : m % TN, t = two ? m % (2 * F32_TERMS) / 2 : m / TN;
-        if constexpr (KEPT) f32_term_kept(t, y[i], x[j & 1], acc[i][j]);
-        else acc[i][j] = f32_term(t, y[i], x[j & 1], acc[i][j]);
+        const int i = m / (2 * F32_TERMS) * 2 + m % 2;
+        f32_add_term(m % (2 * F32_TERMS) / 2, y[i], x[u], acc[i][u]);
         F32_ORDER;
-        if (j < TM - 1) {
-          const int at = j * MF + m;
-          if (m == 1) { x[(j + 1) & 1] = read(xs[buf] + (j + 1) * TILE); F32_ORDER; }
+        if (u < TM - 1) {
+          const int at = u * MF + m;
+          if (m == 1) { x[1] = read(xs[buf] + TILE); F32_ORDER; }
 #pragma unroll
-          for (int o = at * LATE / FIRST; o < (at + 1) * LATE / FIRST; ++o) {
+          for (int o = at * LATE / FIRST; o < LATE && o < (at + 1) * LATE / FIRST; ++o) {
             piece(EARLY + o / OPS, o % OPS, buf ^ 1, buf ^ 1, s + 3);
             F32_ORDER;
           }
         } else {
           if (m == 1) { x[0] = read(xs[buf ^ 1]); F32_ORDER; }
-          if (m == MF / 2) {
+          if (TN == 4 && m == MF / 2) {
             y[0] = read(ys[buf ^ 1]); F32_ORDER;
             y[1] = read(ys[buf ^ 1] + TILE); F32_ORDER;
           }
@@ -447,31 +491,24 @@ __global__ void __launch_bounds__(256, TM == 2 ? 2 : 1) gemm_f32_tile_kernel(F32
         }
       }
     }
-    y[2] = read(ys[buf ^ 1] + 2 * TILE); F32_ORDER;
-    y[3] = read(ys[buf ^ 1] + 3 * TILE); F32_ORDER;
+#pragma unroll
+    for (int i = TN - 2; i < TN; ++i) { y[i] = read(ys[buf ^ 1] + i * TILE); F32_ORDER; }
   };
   for (int s = 0, block = z * g.range_blocks; s < steps; ++block) {
-    f32x4_t acc[TN][TM];
+    F32Sum acc[TN][TM];
 #pragma unroll
     for (int i = 0; i < TN; ++i)
 #pragma unroll
-      for (int j = 0; j < TM; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-    if constexpr (KEPT) {
-      f32_settle(acc);
-      f32_ready(y, x[0]);
-    }
+      for (int j = 0; j < TM; ++j) acc[i][j] = {zero, zero};
     for (const int end = min(s + block_steps, steps); s < end; s += 2) {
       step(s, acc, std::integral_constant<int, 0>{});
       step(s + 1, acc, std::integral_constant<int, 1>{});
     }
-    if constexpr (KEPT) f32_settle(acc);
     if (!CUT) {                              // the blocks are added here, as the adding kernel does it
 #pragma unroll
       for (int i = 0; i < TN; ++i)
 #pragma unroll
-        for (int j = 0; j < TM; ++j)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) sum[i][j][e] += acc[i][j][e];
+        for (int j = 0; j < TM; ++j) sum[i][j] = f32_plus(sum[i][j], f32_block(acc[i][j]));
     }
     if (CUT || s == steps) {
       // a lane holds row lane % 16 of the tile, features 4 (lane / 16) .. + 3
@@ -487,20 +524,10 @@ __global__ void __launch_bounds__(256, TM == 2 ? 2 : 1) gemm_f32_tile_kernel(F32
         for (int i = 0; i < TN; ++i) {
           const int n = n0 + wn + i * 16 + quarter * 4;
           if (n >= g.N) continue;
-          f32x4_t v;
+          f32x4_t v = CUT ? f32_block(acc[i][j]) : sum[i][j];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            v[e] = CUT ? acc[i][j][e] : sum[i][j][e];
-            off |= f32_off(v[e]);
-            if (b && n + e < g.N) v[e] += b[n + e];
-          }
-          if (whole) {
-            *(f32x4_t*)(out + (size_t)m * ld + n) = v;
-          } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              if (n + e < g.N) out[(size_t)m * ld + n + e] = v[e];
-          }
+          for (int e = 0; e < 4; ++e) off |= f32_off(v[e]);
+          f32_store(out + (size_t)m * ld + n, v, b, n, g.N, whole);
         }
       }
       if (!CUT && off) {
@@ -526,50 +553,50 @@ gemm_f32_add_kernel(F32Tile g, int planes, float* __restrict__ C, const float* _
   if (n >= g.N) return;
   const size_t m = blockIdx.x, size = (size_t)g.M * g.N;
   const float* p = g.c + m * g.N + n;
-  float* c = C + m * g.ldc + n;
   f32x4_t v = {0.f, 0.f, 0.f, 0.f};
-  if (whole) {
-    v = *(const f32x4_t*)p;
-    for (int r = 1; r < planes; ++r) v += *(const f32x4_t*)(p + r * size);
-  } else {
-    for (int e = 0; e < 4 && n + e < g.N; ++e) {
-      v[e] = p[e];
-      for (int r = 1; r < planes; ++r) v[e] += p[r * size + e];
-    }
+  for (int r = 0; r < planes; ++r) {
+    f32x4_t x = {0.f, 0.f, 0.f, 0.f};
+    if (whole) x = *(const f32x4_t*)(p + r * size);
+    else
+      for (int e = 0; e < 4 && n + e < g.N; ++e) x[e] = p[r * size + e];
+    v = f32_plus(v, x);
   }
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    if (n + e >= g.N) break;
-    if (f32_off(v[e])) v[e] = f32_again(g.a + m * g.lda, g.w + (size_t)(n + e) * g.K, g.K);
-    if (bias) v[e] += bias[n + e];
-  }
-  if (whole) *(f32x4_t*)c = v;
-  else
-    for (int e = 0; e < 4 && n + e < g.N; ++e) c[e] = v[e];
+  for (int e = 0; e < 4; ++e)
+    if (n + e < g.N && f32_off(v[e])) v[e] = f32_again(g.a + m * g.lda, g.w + (size_t)(n + e) * g.K, g.K);
+  f32_store(C + m * g.ldc + n, v, bias, n, g.N, whole);
 }
 
-// The tile kernel's plan: rows of a tile, and how many of K's blocks a workgroup takes (it adds them in its registers; several ranges of
-// blocks go to planes that the adding kernel adds). The price is a CU's share of the workgroups at what a step takes in tiles of so
-// many rows (measured), and the planes written and read again.
+// The tile kernel's plan: the form of a tile, and how many of K's blocks a workgroup takes (it adds them in its registers; several ranges of
+// blocks go to planes that the adding kernel adds). The price is a CU's share of the workgroups at what a step of 32 k takes in
+// tiles of that form and a start of some 4 us (measured), and the planes written and read again.
 struct TilePlan {
-  int rows, blocks, block_k, range_blocks, ranges;
+  int form, blocks, block_k, range_blocks, ranges;
 };
+struct TileForm {
+  int rows;
+  double one, two;                         // us a step: of one workgroup on a CU, and of two, side by side or in turn
+  bool beside;
+};
+// 64 rows by eight waves are ahead while each CU has one tile, by four, two of them on a CU, from two tiles on: 64 x 2560 x 9728 41.5 / 48.1 us,
+// 160 x 6144 x 2560 55.1 / 52.9, 64 x 19456 x 2560 66.6 / 61; 128 rows from there on where they are there: 100 x 19456 x 2560 105 / 97.5
+// and 91, 300 x 2560 x 9728 - / 125 and 112.
+constexpr TileForm tile_forms[] = {{64, 0.85, 1.70, false}, {64, 1.03, 1.60, true}, {128, 1.38, 2.76, false}};
 TilePlan tile_plan(int M, int N, int K) {
   const long cus = ra_cu_count();
-  // us a step of 32 k: of one workgroup on a CU, and of two, side by side where there is room (tiles of 64 rows), else in turn
-  const struct { int rows; double one, two; } forms[] = {{64, 1.05, 1.42}, {128, 1.48, 2.96}, {192, 1.93, 3.86}, {256, 2.53, 5.06}};
   const KBlocks kb = k_blocks(K);
   TilePlan best = {};
-  double best_us = 0.0;
-  for (const auto& f : forms) {
+  double best_us = -1.0;
+  for (int form = 0; form < 3; ++form) {
+    const TileForm& f = tile_forms[form];
     const long tiles = (long)((M + f.rows - 1) / f.rows) * ((N + 127) / 128);
     for (int take = kb.n; take >= 1; --take) {
       const int ranges = (kb.n + take - 1) / take;
       const long load = (tiles * ranges + cus - 1) / cus;
-      double us = (load / 2 * f.two + load % 2 * f.one) * take * kb.k / F32_BK + load;
-      if (ranges > 1) us += 3.0 + (double)kb.n * M * N * 8.0 / 5e6;
-      if (best.rows == 0 || us < best_us) {
-        best = {f.rows, kb.n, kb.k, take, ranges};
+      double us = (load / 2 * f.two + load % 2 * f.one) * take * kb.k / F32_BK + 4.0 * (f.beside ? (load + 1) / 2 : load);
+      if (ranges > 1) us += 3.0 + (double)kb.n * M * N * 8.0 / 1e7;
+      if (best_us < 0.0 || us < best_us) {
+        best = {form, kb.n, kb.k, take, ranges};
         best_us = us;
       }
     }
@@ -577,23 +604,23 @@ TilePlan tile_plan(int M, int N, int K) {
   return best;
 }
 
-template <int TM>
+template <int WM, int WN, int TN>
 void tile_launch(const F32Tile& g, bool cut, unsigned blocks, hipStream_t stream) {
-  if (cut) gemm_f32_tile_kernel<TM, true><<<blocks, 256, 0, stream>>>(g);
-  else gemm_f32_tile_kernel<TM, false><<<blocks, 256, 0, stream>>>(g);
+  if (cut) gemm_f32_tile_kernel<WM, WN, TN, true><<<blocks, WM * WN * RA_WAVE, 0, stream>>>(g);
+  else gemm_f32_tile_kernel<WM, WN, TN, false><<<blocks, WM * WN * RA_WAVE, 0, stream>>>(g);
 }
 
 int tile_go(const TilePlan& p, const float* A, const float* W, const float* bias, float* C, int M, int N, int K, int lda,
             int ldc, float* scratch, hipStream_t stream) {
   const bool cut = p.ranges > 1;
-  F32Tile g = {A, W, bias, cut ? scratch : C, M, N, K, lda, ldc, (M + p.rows - 1) / p.rows, (N + 127) / 128, p.ranges,
+  const int rows = tile_forms[p.form].rows;
+  F32Tile g = {A, W, bias, cut ? scratch : C, M, N, K, lda, ldc, (M + rows - 1) / rows, (N + 127) / 128, p.ranges,
                p.block_k, p.range_blocks};
   const long total = (long)g.m_tiles * g.n_tiles * g.ranges, blocks = (total + RA_XCDS - 1) / RA_XCDS * RA_XCDS;
   RA_CHECK(blocks <= 0x7FFFFFFFL, "gemm_f32: [%d, %d] in one launch", M, N);
-  if (p.rows == 64) tile_launch<2>(g, cut, (unsigned)blocks, stream);
-  else if (p.rows == 128) tile_launch<4>(g, cut, (unsigned)blocks, stream);
-  else if (p.rows == 192) tile_launch<6>(g, cut, (unsigned)blocks, stream);
-  else tile_launch<8>(g, cut, (unsigned)blocks, stream);
+  if (p.form == 0) tile_launch<2, 4, 2>(g, cut, (unsigned)blocks, stream);
+  else if (p.form == 1) tile_launch<2, 2, 4>(g, cut, (unsigned)blocks, stream);
+  else tile_launch<4, 2, 4>(g, cut, (unsigned)blocks, stream);
   RA_LAUNCH_CHECK("gemm_f32");
   if (cut) {
     const bool whole = N % 4 == 0 && ldc % 4 == 0 && (uintptr_t)C % 16 == 0 && (uintptr_t)scratch % 16 == 0;
