@@ -105,24 +105,41 @@ __device__ __forceinline__ f32x4_t f32_plus(f32x4_t a, f32x4_t b) {
   return a;
 }
 
-// The parts of an infinity and of a float that is one 2^24 times as large are no numbers: a sum that is not finite is worked out again from
-// the floats.
-__device__ __forceinline__ bool f32_off(float v) { return !(fabsf(v) <= 3.402823466e38f); }
-__device__ __forceinline__ float f32_again(const float* __restrict__ a, const float* __restrict__ w, int K) {
-  float s = 0.f;
-  for (int k = 0; k < K; k += 4) {
-    const f32x4_t x = *(const f32x4_t*)(a + k), y = *(const f32x4_t*)(w + k);
+// The parts of an infinity and of a float that is one 2^24 times as large are no numbers: a block's sum that is not finite is worked out
+// again from the floats, on the float matrix cores, by a wave for 16 rows and 16 features: four products for every 16 k, of k 0, 4, 8, 12,
+// then 1, 5, 9, 13, .... a and w: the first row and feature, of `rows` and `features` that there are.
+// With a NaN in one row a product takes, us (without): 8 rows 2560 x 9728 35 (24), 300 x 6144 x 2560 168 (68), 1119 x 6144 x 2560 361 (196); 300
+// rows of NaN 391.
+__device__ __forceinline__ bool f32_off(f32x4_t v) {
+  return !(fabsf(v[0]) <= 3.402823466e38f && fabsf(v[1]) <= 3.402823466e38f && fabsf(v[2]) <= 3.402823466e38f && fabsf(v[3]) <= 3.402823466e38f);
+}
+__device__ __forceinline__ f32x4_t f32_again(const float* a, int lda, int rows, const float* w, int ldw, int features, int k0, int k1,
+                                             f32x4_t v) {
+  const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+  const float *x = a + (size_t)min(r, rows - 1) * lda, *y = w + (size_t)min(r, features - 1) * ldw;
+  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4_t c = zero;
+  for (int k = k0; k < k1; k += 64) {
+    f32x4_t f[4], g[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) s = fmaf(x[e], y[e], s);
+    for (int i = 0; i < 4; ++i) {
+      const int at = k + i * 16 + q * 4;
+      f[i] = at < k1 ? *(const f32x4_t*)(y + at) : zero;
+      g[i] = at < k1 ? *(const f32x4_t*)(x + at) : zero;
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) c = __builtin_amdgcn_mfma_f32_16x16x4f32(f[i / 4][i % 4], g[i / 4][i % 4], c, 0, 0, 0);
   }
-  return s;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = fabsf(v[e]) <= 3.402823466e38f ? v[e] : c[e];
+  return v;
 }
 
 // ------------------------------------------------------------------------------------------------ the order of the sums
 // K is summed in up to eight blocks of at least 512 k, whose number and length follow from K alone. A block is two chains of
-// 16x16x32 products over its pieces of 32 k, one and five a piece, that are added at its end. The blocks'
-// sums are added in their order, then the bias. Both kernels keep this order, so a row's result does not depend on how many rows stand
-// beside it: a request's 32-bit results are the same bits alone and in any step.
+// 16x16x32 products over its pieces of 32 k, one and five a piece, that are added at its end; where that is not finite, its sum from the
+// floats. The blocks' sums are added in their order, then the bias. Both kernels keep this order, so a row's result does not depend on
+// how many rows stand beside it: a request's 32-bit results are the same bits alone and in any step.
 struct KBlocks {
   int n, k;                                // how many, and k of one (a multiple of 64)
 };
@@ -271,7 +288,9 @@ gemm_f32_stream_kernel(const float* __restrict__ A, const float* __restrict__ W,
     // while the next tile's go to the other buffer, and a wave writes a buffer again only behind the next barrier.
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
-      sums[((buf * waves + wave) * MT + t) * RA_WAVE + lane] = f32_block(acc[t]);
+      f32x4_t v = f32_block(acc[t]);
+      if (__any(f32_off(v))) v = f32_again(A + (size_t)t * 16 * lda, lda, M - t * 16, W + (size_t)n0 * K, K, N - n0, k0, k1, v);
+      sums[((buf * waves + wave) * MT + t) * RA_WAVE + lane] = v;
       acc[t] = {zero, zero};
     }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -286,14 +305,6 @@ gemm_f32_stream_kernel(const float* __restrict__ A, const float* __restrict__ W,
         for (int i = 0; i < 4; ++i) {
           const int f = n0 + q * 4 + i;
           if (f < N) C[(size_t)m * ldc + f] = bias ? v[i] + bias[f] : v[i];
-        }
-        if (f32_off(v[0]) || f32_off(v[1]) || f32_off(v[2]) || f32_off(v[3])) {
-#pragma unroll 1
-          for (int f = n0 + q * 4; f < min(n0 + q * 4 + 4, N); ++f)
-            if (f32_off(C[(size_t)m * ldc + f])) {
-              const float u = f32_again(A + (size_t)m * lda, W + (size_t)f * K, K);
-              C[(size_t)m * ldc + f] = bias ? u + bias[f] : u;
-            }
         }
       }
     }
@@ -331,6 +342,40 @@ __device__ __forceinline__ void f32_store(float* to, f32x4_t v, const float* bia
       if (n + e < N) to[e] = v[e];
   }
 }
+// 16 rows and features by a wave, straight from memory: blocks first to past, each as the tiles have it, or from the floats where that
+// is not finite, added in their order. For tiles that hold a result that is not finite.
+__device__ __forceinline__ void f32_write_again(const F32Tile& g, int m0, int n0, int first, int past, float* out, int ld,
+                                                const float* bias, bool whole) {
+  const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4, rows = g.M - m0, features = g.N - n0;
+  const float *a = g.a + (size_t)m0 * g.lda, *w = g.w + (size_t)n0 * g.K;
+  const float *x = a + (size_t)min(r, rows - 1) * g.lda, *y = w + (size_t)min(r, features - 1) * g.K;
+  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4_t sum = zero;
+  for (int block = first; block < past; ++block) {
+    const int k0 = block * g.block_k, k1 = min(k0 + g.block_k, g.K);
+    F32Sum acc = {zero, zero};
+    for (int k = k0; k < k1; k += 64) {
+      f32x4_t f[4], h[4];                  // 8 k of each of two pieces
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int at = k + i / 2 * 32 + q * 8 + i % 2 * 4;
+        f[i] = at < k1 ? *(const f32x4_t*)(y + at) : zero;
+        h[i] = at < k1 ? *(const f32x4_t*)(x + at) : zero;
+      }
+#pragma unroll
+      for (int i = 0; i < 4; i += 2) {
+        const F32Parts wp = f32_split(f[i], f[i + 1]), ap = f32_split(h[i], h[i + 1]);
+#pragma unroll
+        for (int t = 0; t < F32_TERMS; ++t) f32_add_term(t, wp, ap, acc);
+      }
+    }
+    f32x4_t v = f32_block(acc);
+    if (__any(f32_off(v))) v = f32_again(a, g.lda, rows, w, g.K, features, k0, k1, v);
+    sum = f32_plus(sum, v);
+  }
+  if (r < rows && q * 4 < features) f32_store(out + (size_t)(m0 + r) * ld + n0 + q * 4, sum, bias, n0 + q * 4, g.N, whole);
+}
+
 // A workgroup of WM x WN waves a tile of 32 WM rows and 128 features and range of k; a wave 32 rows and 16 TN features of it. A step is 32 k of
 // both operands: read from memory as floats, in whole lines, two steps ahead, into registers; split, each once a workgroup, and written to
 // LDS one step ahead, part by part in tiles of 16 rows in the products' order: the 16 bytes of row r, k 8 q .. + 7 lie at place
@@ -515,7 +560,7 @@ __global__ void __launch_bounds__(WM * WN * RA_WAVE, 2) gemm_f32_tile_kernel(F32
       float* out = CUT ? g.c + (size_t)block * g.M * g.N : g.c;
       int m_at = m0 + wm + row;
       asm volatile("" : "+v"(m_at));         // addresses are worked out here and not kept in registers through the steps
-      bool off = false;
+      unsigned off = 0;                      // a bit for 16 rows and features that hold a result that is not finite
 #pragma unroll
       for (int j = 0; j < TM; ++j) {
         const int m = m_at + j * 16;
@@ -525,21 +570,16 @@ __global__ void __launch_bounds__(WM * WN * RA_WAVE, 2) gemm_f32_tile_kernel(F32
           const int n = n0 + wn + i * 16 + quarter * 4;
           if (n >= g.N) continue;
           f32x4_t v = CUT ? f32_block(acc[i][j]) : sum[i][j];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) off |= f32_off(v[e]);
+          off |= (unsigned)f32_off(v) << (j * TN + i);
           f32_store(out + (size_t)m * ld + n, v, b, n, g.N, whole);
         }
       }
-      if (!CUT && off) {
+      if (__any(off != 0)) {
+        const int first = CUT ? block : 0, past = CUT ? block + 1 : (g.K + g.block_k - 1) / g.block_k;
 #pragma unroll 1
-        for (int m = m_at; m < min(m_at + TM * 16, g.M); m += 16)
-#pragma unroll 1
-          for (int i = 0; i < TN * 4; ++i) {
-            const int n = n0 + wn + (i >> 2) * 16 + quarter * 4 + (i & 3);
-            if (n >= g.N || !f32_off(out[(size_t)m * ld + n])) continue;
-            const float u = f32_again(g.a + (size_t)m * g.lda, g.w + (size_t)n * g.K, g.K);
-            out[(size_t)m * ld + n] = b ? u + b[n] : u;
-          }
+        for (int j = 0; j < TM * TN; ++j)
+          if (__any(off >> j & 1))
+            f32_write_again(g, m0 + wm + j / TN * 16, n0 + wn + j % TN * 16, first, past, out, ld, b, whole);
       }
     }
   }
@@ -561,9 +601,6 @@ gemm_f32_add_kernel(F32Tile g, int planes, float* __restrict__ C, const float* _
       for (int e = 0; e < 4 && n + e < g.N; ++e) x[e] = p[r * size + e];
     v = f32_plus(v, x);
   }
-#pragma unroll
-  for (int e = 0; e < 4; ++e)
-    if (n + e < g.N && f32_off(v[e])) v[e] = f32_again(g.a + m * g.lda, g.w + (size_t)(n + e) * g.K, g.K);
   f32_store(C + m * g.ldc + n, v, bias, n, g.N, whole);
 }
 

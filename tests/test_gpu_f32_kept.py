@@ -1,5 +1,5 @@
 """What the 32-bit products keep of floats: numbers down to the smallest and up to the largest, mantissas that the six terms serve worst,
-errors without a mean; and a row's bits beside any others."""
+errors without a mean, many sums that are not finite; and a row's bits beside any others."""
 import pytest
 import torch
 
@@ -78,6 +78,28 @@ def test_worst_mantissas(M):
     assert ((product(x, w).double() - want).abs() <= (2 + 2.0 ** -6) * U * want).all()
 
 
+@pytest.mark.parametrize("M", ROWS)
+def test_many_that_are_not_finite(M):
+    """Whole rows, and all of them, that hold an infinity or a NaN; sums past 2^80, which are worked out from the floats."""
+    g = torch.Generator(device=DEV).manual_seed(M)
+    K, N = 1092, 140
+    x, w = torch.randn(M, K, generator=g, device=DEV), torch.randn(N, K, generator=g, device=DEV)
+    for rows in (slice(0, M, 3), slice(0, M)):
+        for value in (float("inf"), float("nan")):
+            y = x.clone()
+            y[rows, 700] = value
+            want = (y.double() @ w.double().t()).float()
+            got = product(y, w)
+            assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got[want.isinf()], want[want.isinf()])
+            keep = want.isfinite()
+            assert torch.equal(got[keep], product(x, w)[keep])
+    y = x.clone()
+    y[::2] *= 2.0 ** 90
+    want = y.double() @ w.double().t()
+    got = product(y, w)
+    assert ((got.double() - want).abs() <= (K + 8) * U * (y.double().abs() @ w.double().abs().t())).all()
+
+
 @pytest.mark.parametrize("N,K", [(2560, 1092), (200, 4096), (6144, 2560)])
 def test_a_rows_bits_beside_any_others(N, K):
     g = torch.Generator(device=DEV).manual_seed(N)
@@ -91,3 +113,26 @@ def test_a_rows_bits_beside_any_others(N, K):
         assert torch.equal(part.view(torch.int32), whole[:M].view(torch.int32)), M
     for m in (5, 6, 7, 1099):
         assert torch.equal(product(x[m:m + 1], w, b).view(torch.int32), whole[m:m + 1].view(torch.int32)), m
+
+
+@pytest.mark.parametrize("M,N,K,rows", [(8, 2560, 9728, 1), (4, 6144, 2560, 4), (300, 6144, 2560, 1), (300, 2560, 2560, 300)])
+def test_what_is_not_finite_costs_a_few_products(M, N, K, rows):
+    """What is worked out again is shared out over whole waves: some ten times the product at most, all of it NaN (3 to 6 measured; a lane a
+    sum took 20 to 50)."""
+    x, w = torch.randn(M, K, device=DEV), torch.randn(N, K, device=DEV)
+
+    def time(x):
+        out, best = torch.empty(M, N, device=DEV), float("inf")
+        from reinfer_amd import kernels
+        for _ in range(8):
+            first, last = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            first.record()
+            for _ in range(4):
+                kernels.current().linear(x, w, out, None)
+            last.record()
+            torch.cuda.synchronize()
+            best = min(best, first.elapsed_time(last))
+        return best
+    plain = time(x)
+    x[:rows, 5] = float("nan")
+    assert time(x) < 10 * plain
