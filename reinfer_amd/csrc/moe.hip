@@ -559,7 +559,7 @@ extern "C" int ra_moe_relu2_scale(const void* up, void* act, int act_dtype, cons
 // The choice and the activation in one kernel, for steps of few tokens, where a launch is most of the choice's time: every workgroup has
 // one wave choose for its token once more, while the others' rows are on their way. Sigmoid scores with gated experts, or the
 // softmax of the chosen with relu squared; rows of 16-byte pieces. Eight tokens, 16 experts of 1024 and a shared one of 2048, in a
-// decode step: route 7.4 and activation 4.7 us, this one 8.4.
+// decode step: route 7.4 and activation 4.7 us, this one 8.4 (in a trace; ra_moe_choose_scale_takes says up to how many tokens).
 // ---------------------------------------------------------------------------
 struct MoeChoice {
   const float* logits;
@@ -604,24 +604,36 @@ __global__ void moe_choose_scale_x8_kernel(const TA* __restrict__ up, TA* __rest
 }
 
 // Whether rows and sizes are whole 16-byte pieces and the choice fits LDS.
-extern "C" int ra_moe_choose_scale_takes(const void* up, const void* act, int act_dtype, int top, int experts, int groups, int ff,
-                                         int shared, int n_tokens) {
+static bool moe_choose_scale_can(const void* up, const void* act, int act_dtype, int top, int experts, int groups, int ff, int shared,
+                                 int n_tokens) {
   return (act_dtype == RA_F32 || act_dtype == RA_BF16) && ff > 0 && ff % 8 == 0 && shared >= 0 && shared % 8 == 0 &&
          (uintptr_t)up % 16 == 0 && (uintptr_t)act % 16 == 0 && top > 0 && top <= RA_WAVE && top <= experts &&
          (2L * experts + groups) * (long)sizeof(float) <= 64 * 1024 && n_tokens > 0 && n_tokens <= 65535;
+}
+static unsigned moe_choose_scale_groups(int experts, int ff, int shared) { return ((experts * ff + shared) / 8 + 255) / 256; }
+
+// Whether one kernel is the better one: while all workgroups have a place at once (8 a CU; the choice is made in each), us, one kernel / two,
+// bfloat16: 16 experts of 1024 and a shared one of 2048 (9 workgroups a token) 8 tokens 10.5 / 12.8, 64 11.4 / 13.9, 227 13.6 / 16.2, 256
+// 19.2 / 16.2, 2000 76 / 33; 64 of 512 (17) 64 tokens 17.4 / 18.8, 128 27.9 / 20.0, 2000 220 / 48; 16 of 1536 with relu squared (12) 170 tokens
+// 9.6 / 10.7, 192 12.7 / 11.4, 2000 59 / 26. Float activations with relu squared at any number, as their own kernel reads an
+// element a thread: 16 of 1536 192 tokens 16.3 / 18.2, 2000 73 / 107, 64 of 512 2000 tokens 108 / 143; gated 2000 87 / 52 and 225 / 93.
+extern "C" int ra_moe_choose_scale_takes(const void* up, const void* act, int act_dtype, int gated, int top, int experts, int groups,
+                                         int ff, int shared, int n_tokens) {
+  return moe_choose_scale_can(up, act, act_dtype, top, experts, groups, ff, shared, n_tokens) &&
+         ((!gated && act_dtype == RA_F32) || (long)moe_choose_scale_groups(experts, ff, shared) * n_tokens <= 8L * ra_cu_count());
 }
 
 extern "C" int ra_moe_choose_scale(const void* up, void* act, int act_dtype, int gated, const float* logits, int ld, int top,
                                    int experts, int groups, int kept, int group_top, float scale, int ff, int shared, int n_tokens,
                                    hipStream_t stream) {
-  RA_CHECK(ra_moe_choose_scale_takes(up, act, act_dtype, top, experts, groups, ff, shared, n_tokens),
+  RA_CHECK(moe_choose_scale_can(up, act, act_dtype, top, experts, groups, ff, shared, n_tokens),
            "moe_choose_scale: %d tokens, %d of %d experts of %d, shared %d", n_tokens, top, experts, ff, shared);
   RA_CHECK(ld >= experts, "moe_choose_scale: rows of %d for %d experts", ld, experts);
   RA_CHECK(groups >= 1 && experts % groups == 0 && kept >= 1 && kept <= groups && top <= kept * (experts / groups) && group_top >= 1,
            "moe_choose_scale: %d of %d groups, %d of %d experts", kept, groups, top, experts);
   RA_CHECK(gated || (groups == 1 && shared == 0), "moe_choose_scale: groups and a shared expert are the gated form's");
   const MoeChoice c = {logits, ld, top, groups, kept, group_top, scale};
-  const dim3 grid(((experts * ff + shared) / 8 + 255) / 256, n_tokens);
+  const dim3 grid(moe_choose_scale_groups(experts, ff, shared), n_tokens);
   const size_t lds = (size_t)(2 * experts + groups) * sizeof(float);
 #define RA_GO(TA, GATED) \
   moe_choose_scale_x8_kernel<TA, GATED><<<grid, 256, lds, stream>>>((const TA*)up, (TA*)act, c, experts, ff, shared)

@@ -288,8 +288,8 @@ int ra_moe_relu2_scale(const void* up, void* act, int act_dtype, const int* ids,
                        int experts, int ff, int n_tokens, hipStream_t stream);
 // The choice by float logits (rows ld apart) and the activation with its weights in one kernel: gated ([gate | up] of each expert, sigmoid
 // scores, groups, a shared expert) as ra_moe_route_sigmoid and ra_moe_silu_gate_scale, else as ra_moe_topk and ra_moe_relu2_scale
-int ra_moe_choose_scale_takes(const void* up, const void* act, int act_dtype, int top, int experts, int groups, int ff, int shared,
-                              int n_tokens);
+int ra_moe_choose_scale_takes(const void* up, const void* act, int act_dtype, int gated, int top, int experts, int groups, int ff,
+                              int shared, int n_tokens);
 int ra_moe_choose_scale(const void* up, void* act, int act_dtype, int gated, const float* logits, int ld, int top, int experts,
                         int groups, int kept, int group_top, float scale, int ff, int shared, int n_tokens, hipStream_t stream);
 

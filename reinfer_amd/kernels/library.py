@@ -150,7 +150,7 @@ def load() -> ctypes.CDLL:
         lib.ra_moe_grouped_scratch.restype = c_long
         lib.ra_moe_grouped_scratch.argtypes = [I, I, I, I, I]
         lib.ra_moe_choose_scale_takes.restype = c_int
-        lib.ra_moe_choose_scale_takes.argtypes = [P, P, I, I, I, I, I, I, I]
+        lib.ra_moe_choose_scale_takes.argtypes = [P, P, I, I, I, I, I, I, I, I]
         lib.ra_gemm_f32_supports.restype = c_int
         lib.ra_gemm_f32_supports.argtypes = [P, P, I, I]
         lib.ra_gemm_f32_scratch.restype = c_long

@@ -1797,7 +1797,7 @@ class HipKernels:
                          groups_kept: int = 1, group_top: int = 2) -> None:
         """The choice of :meth:`moe_route` by its float32 ``logits`` [T, >= experts] and the activation of all experts' products with
         its weights, :meth:`moe_silu_gate_scale` ("sigmoid") or :meth:`moe_relu2_scale` ("softmax_chosen"): one kernel
-        where rows are 16-byte pieces, else two."""
+        where rows are 16-byte pieces and few (``ra_moe_choose_scale_takes``), else two."""
         gated = scoring == "sigmoid"
         if not gated and (scoring != "softmax_chosen" or shared or groups != 1):
             raise ValueError(f"moe_choose_scale: scoring {scoring!r}, shared {shared}, {groups} groups")
@@ -1809,8 +1809,8 @@ class HipKernels:
         if logits.dtype != torch.float32 or logits.dim() != 2 or logits.shape[0] != T or logits.shape[1] < experts or logits.stride(1) != 1:
             raise ValueError(f"moe_choose_scale: logits float32 [{T}, >= {experts}]")
         tag = _tag(up, "moe_choose_scale")
-        if library.load().ra_moe_choose_scale_takes(up.data_ptr(), act.data_ptr(), tag, int(top), int(experts), int(groups), int(ff),
-                                                    int(shared), T):
+        if library.load().ra_moe_choose_scale_takes(up.data_ptr(), act.data_ptr(), tag, int(gated), int(top), int(experts), int(groups),
+                                                    int(ff), int(shared), T):
             library.call("ra_moe_choose_scale", up.data_ptr(), act.data_ptr(), tag, int(gated), logits.data_ptr(), logits.stride(0),
                          int(top), int(experts), int(groups), int(groups_kept), int(group_top), float(scale), int(ff), int(shared),
                          T, _stream())
