@@ -269,8 +269,8 @@ __global__ void __launch_bounds__(WAVES * RA_WAVE) attention_f32_kernel(F32Atten
   constexpr int KP = D / 32;               // pieces of 8 entries of a key a lane
   constexpr int VP = D / 16;               // runs of 16 entries of the values
   constexpr int LD = D + 4;
-  extern __shared__ __attribute__((aligned(16))) float part[];           // [SHARES][ROWS][LD], then maximum and sum [SHARES][ROWS][2]
-  float* const ends = part + SHARES * ROWS * LD;
+  // of a fixed size: one that is told at the launch and is above 64 KB is a host call more at each
+  __shared__ __attribute__((aligned(16))) float part[SHARES * ROWS * LD], ends[SHARES * ROWS * 2];       // maximum and sum
   __shared__ int off[ROWS];                // rows with a result that is no finite number
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
   const int lo16 = lane & 15, hi = lane >> 4;
@@ -499,13 +499,8 @@ int go(F32Attention g, int n_requests, hipStream_t stream) {
   // a workgroup a request's run of tokens where a workgroup a token would be a few rounds of the chip, else one for all runs of its rows
   const int z = pairs * g.n_tokens <= 8 * cus ? (nt < g.n_tokens ? nt : g.n_tokens) : 1;
   const int waves = D > 128 || pairs * tiles > cus ? 4 : 8;
-  constexpr size_t lds = (size_t)SHARES * ROWS * (D + 6) * sizeof(float);
   constexpr int W = D <= 128 ? 8 : 4;
-  if (lds > 64 * 1024) {
-    const hipError_t e = hipFuncSetAttribute((const void*)attention_f32_kernel<D, W>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) return ra_fail("attention_f32: %s", hipGetErrorString(e));
-  }
-  attention_f32_kernel<D, W><<<dim3(pairs, tiles, z), waves * RA_WAVE, lds, stream>>>(g);
+  attention_f32_kernel<D, W><<<dim3(pairs, tiles, z), waves * RA_WAVE, 0, stream>>>(g);
   RA_LAUNCH_CHECK("attention_f32");
   return 0;
 }
