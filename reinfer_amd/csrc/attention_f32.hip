@@ -37,7 +37,7 @@ struct F32Attention {
   int max_blocks;
   const int *token_list, *seq_of_token, *positions;
   int n_tokens, heads;                     // heads: of a workgroup, a power of two
-  int block_size, tiles;                   // a block's tiles of 16 slots
+  int tiles;                               // of 16 slots, of a block
   unsigned long long share;                // i / tiles is i * share >> 32
   int Hq, Hkv;
   float scale;
@@ -519,7 +519,7 @@ int ra_attention_f32(const float* q, int q_stride, float* out, int out_stride, c
                      const int* positions, int n_tokens, int n_requests, int block_size, int Hq, int Hkv, int d, float scale,
                      int window, int aligned, int keep, RaScoreMod mod, RaHeadOut ho, hipStream_t stream) {
   const F32Attention g = {q, q_stride, out, out_stride, kcache, vcache, block_tables, max_blocks, token_list, seq_of_token,
-                          positions, n_tokens, 1, block_size, block_size / 16, (1ull << 32) / (block_size / 16) + 1, Hq, Hkv, scale, window, aligned, keep, mod, ho};
+                          positions, n_tokens, 1, block_size / 16, (1ull << 32) / (block_size / 16) + 1, Hq, Hkv, scale, window, aligned, keep, mod, ho};
   if (d == 64) return go<64>(g, n_requests, stream);
   if (d == 128) return go<128>(g, n_requests, stream);
   if (d == 256) return go<256>(g, n_requests, stream);

@@ -62,6 +62,7 @@ class Sampler:
                 tokens = torch.empty(n, dtype=torch.int32, device=self.device)
                 ops.sample_filtered(logits, params, histories, [as_int64(int(s)) for s in seeds], [int(p) for p in positions], tokens)
                 return self._drawn(tokens)
+            # a kernel set without that, or fewer histories than rows (the others' options are not applied)
             logits = logits.clone()
             ops.filter_logits(logits, params, histories)
         # one transfer: seeds, temperatures, positions
