@@ -22,3 +22,17 @@ def pytest_collection_modifyitems(config, items):
     for item in items:
         if "gpu" in item.keywords:
             item.add_marker(skip)
+
+
+@pytest.fixture
+def library_calls(monkeypatch):
+    """``library_calls(run)``: the names of the kernel library's calls that ``run()`` makes."""
+    from reinfer_amd.kernels import library
+
+    def of(run):
+        names, call = [], library.call
+        with monkeypatch.context() as m:
+            m.setattr(library, "call", lambda name, *args: (names.append(name), call(name, *args))[1])
+            run()
+        return names
+    return of

@@ -8,22 +8,13 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-def calls_of(monkeypatch, run):
-    """The names of the library's calls that ``run`` makes."""
-    names, call = [], kernels.library.call
-    with monkeypatch.context() as m:
-        m.setattr(kernels.library, "call", lambda name, *args: (names.append(name), call(name, *args))[1])
-        run()
-    return names
-
-
 def places():
     return 8 * torch.cuda.get_device_properties(DEV).multi_processor_count
 
 
 @pytest.mark.parametrize("E,top,ff,shared,groups,kept", [(16, 4, 1024, 2048, 4, 2), (64, 8, 512, 512, 8, 4), (8, 3, 256, 8, 1, 1)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-def test_gated(monkeypatch, E, top, ff, shared, groups, kept, dtype):
+def test_gated(library_calls, E, top, ff, shared, groups, kept, dtype):
     ops = kernels.current()
     n = E * ff + shared
     line = places() // -(-(n // 8) // 256)
@@ -31,8 +22,8 @@ def test_gated(monkeypatch, E, top, ff, shared, groups, kept, dtype):
         g = torch.Generator(device=DEV).manual_seed(T + E)
         up, logits = torch.randn(T, 2 * n, generator=g, device=DEV).to(dtype), torch.randn(T, E, generator=g, device=DEV)
         act, want = torch.full((T, n), 7.0, device=DEV, dtype=dtype), torch.empty(T, n, device=DEV, dtype=dtype)
-        names = calls_of(monkeypatch, lambda: ops.moe_choose_scale(up, act, logits, top, E, ff, shared=shared, scoring="sigmoid", scale=2.5,
-                                                                   groups=groups, groups_kept=kept, group_top=2))
+        names = library_calls(lambda: ops.moe_choose_scale(up, act, logits, top, E, ff, shared=shared, scoring="sigmoid", scale=2.5,
+                                                           groups=groups, groups_kept=kept, group_top=2))
         assert names == (["ra_moe_choose_scale"] if T <= line else ["ra_moe_route_sigmoid", "ra_moe_silu_gate_scale_shared"])
         ids, weights = torch.empty(T, top, device=DEV, dtype=torch.int32), torch.empty(T, top, device=DEV)
         kernels.library.call("ra_moe_route_sigmoid", logits.data_ptr(), logits.stride(0), E, top, groups, kept, 2, 2.5, ids.data_ptr(),
@@ -43,7 +34,7 @@ def test_gated(monkeypatch, E, top, ff, shared, groups, kept, dtype):
 
 @pytest.mark.parametrize("E,top,ff", [(16, 4, 1536), (64, 6, 64)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-def test_squared(monkeypatch, E, top, ff, dtype):
+def test_squared(library_calls, E, top, ff, dtype):
     ops = kernels.current()
     n = E * ff
     line = places() // -(-(n // 8) // 256)
@@ -51,7 +42,7 @@ def test_squared(monkeypatch, E, top, ff, dtype):
         g = torch.Generator(device=DEV).manual_seed(T + E)
         up, logits = torch.randn(T, n, generator=g, device=DEV).to(dtype), torch.randn(T, E, generator=g, device=DEV)
         act, want = torch.full((T, n), 7.0, device=DEV, dtype=dtype), torch.empty(T, n, device=DEV, dtype=dtype)
-        names = calls_of(monkeypatch, lambda: ops.moe_choose_scale(up, act, logits, top, E, ff))
+        names = library_calls(lambda: ops.moe_choose_scale(up, act, logits, top, E, ff))
         assert names == (["ra_moe_choose_scale"] if T <= line or dtype == torch.float32 else ["ra_moe_topk", "ra_moe_relu2_scale"])
         ids, weights = torch.empty(T, top, device=DEV, dtype=torch.int32), torch.empty(T, top, device=DEV)
         kernels.library.call("ra_moe_topk", logits.data_ptr(), E, E, top, ids.data_ptr(), weights.data_ptr(), T, torch.cuda.current_stream().cuda_stream)

@@ -44,7 +44,8 @@ def test_what_is_not_finite_comes_out_as_of_floats(M, N, K):
 @pytest.mark.parametrize("M", ROWS)
 def test_exponents_of_all_sizes(M):
     """Rows and weights of 2^-60 .. 2^60: every product is a float's, and each is off by no more than its own roundings. What the six
-    terms leave out is below 2^-24 of a product, the sum's roundings are six for every 32 k and one for each of its blocks."""
+    terms leave out is some 2^-24 of a product, the sum's roundings are four for every 32 k and two for each of its blocks; six and one are
+    granted, twice over."""
     g = torch.Generator(device=DEV).manual_seed(M)
     K, N = 2052, 100
 

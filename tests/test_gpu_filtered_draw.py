@@ -35,7 +35,7 @@ def options(r, V, k):
 # less than a thread's four, a slice and more, off 16 bytes, the larger models'; windows of none to more than LDS holds
 @pytest.mark.parametrize("V,stride", [(5, 5), (4096, 4096), (4097, 4099), (32768, 32768), (50003, 50004), (151936, 151936)])
 @pytest.mark.parametrize("n", [1, 3, 24])
-def test_same_tokens_as_filter_then_draw(V, stride, n):
+def test_same_tokens_as_filter_then_draw(library_calls, V, stride, n):
     r = random.Random(V + n)
     g = torch.Generator(device=DEV).manual_seed(V + n)
     logits = (torch.randn(n, stride, generator=g, device=DEV) * 3)[:, :V]
@@ -48,8 +48,10 @@ def test_same_tokens_as_filter_then_draw(V, stride, n):
         params = [options(r, V, i + turn) for i in range(n)]
         histories = [[r.randrange(min(V, 40) if i % 2 else V) for _ in range(r.choice([0, 1, 64, 900, 3000]))] for i in range(n)]
         seeds, positions = [p.seed for p in params], [len(h) + 1 for h in histories]
-        assert Sampler(torch.device(DEV)).sample(logits, params, seeds, positions, histories) \
-            == two_steps(logits, params, seeds, positions, histories), turn
+        tokens = []
+        names = library_calls(lambda: tokens.extend(Sampler(torch.device(DEV)).sample(logits, params, seeds, positions, histories)))
+        assert names == ["ra_sample_filtered" if any(p.filters for p in params) else "ra_sample"]
+        assert tokens == two_steps(logits, params, seeds, positions, histories), turn
         assert torch.equal(logits.view(torch.int32), before.view(torch.int32)) if stride == V else torch.equal(logits.nan_to_num(9), before.nan_to_num(9))
 
 
