@@ -559,7 +559,7 @@ extern "C" int ra_moe_relu2_scale(const void* up, void* act, int act_dtype, cons
 // The choice and the activation in one kernel, for steps of few tokens, where a launch is most of the choice's time: every workgroup has
 // one wave choose for its token once more, while the others' rows are on their way. Sigmoid scores with gated experts, or the
 // softmax of the chosen with relu squared; rows of 16-byte pieces. Eight tokens, 16 experts of 1024 and a shared one of 2048, in a
-// decode step: route 7.4 and activation 4.7 us, this one 8.4 (in a trace; ra_moe_choose_scale_takes says up to how many tokens).
+// decode step: route 7.4 and activation 4.7 us, this one 8.3 (in a trace; ra_moe_choose_scale_takes says up to how many tokens).
 // ---------------------------------------------------------------------------
 struct MoeChoice {
   const float* logits;

@@ -364,8 +364,8 @@ __device__ __forceinline__ float delta_decay(float z, float a_log, float dt_bias
 // A step in which every request brings one token: nothing to stage and nothing to walk, so a lane reads its own run of k and q from
 // memory, works out the gates for itself and has its part of the state asked for at the same time; no LDS, no barrier, and no
 // kernels ahead that prepare gates. Bound by the state read and written, behind two trips to memory. Eight requests in a decode
-// step, 16 heads of 128 x 256: gates and scan_kernel 5.0 + 16.6 us, this one 12.4 (33 MB); the delta rule, 32 heads of 128 x 128:
-// 4.5 + 13.8, so 9.2, and 4.9 less for the filter's tail, which the kernel that prepares q, k and v moves on then.
+// step, 16 heads of 128 x 256, in a trace: gates and scan_kernel 4.9 + 16.6 us, this one 12.3 (33 MB); the delta rule, 32 heads of
+// 128 x 128: 4.7 + 13.7, so 9.3, and 4.8 less for the filter's tail, which the kernel that prepares q, k and v moves on then.
 struct TokenGates {
   const float* z;                                    // [T, 2 H] pre-activations
   const float *first, *second;                       // their biases [2 H] (matrix memory); A_log, dt_bias [H] (delta rule)

@@ -222,11 +222,11 @@ extern "C" int ra_sample_static(const float* logits, int n_rows, int vocab, int 
 //   5  one workgroup a row finds the exact boundaries among them;
 //   6  every slice removes what lies below.
 // One workgroup a row that bisected over the whole row, up to 94 passes, took 3.15 ms for 24 rows of 151936 however many
-// rows there were; the six launches take 46 us for them, each bound by its own start and one trip over the row.
+// rows there were; the six launches take 49 us for them (in a trace), each bound by its own start and one trip over the row.
 // Where a token is drawn from the row at once (ra_sample_filtered) nothing is removed: the draw passes over what a filter would have
 // taken, and only rows that penalties or a bias change are copied, in the first pass. For those 24 rows, half of them changed, that
-// saves the copy of all rows, the last pass and a trip over memory each: 83 us of kernels
-// and copies, so 59. Windows of 64 are counted eight tokens at a time: the first pass 13.8 -> 8.5 us.
+// saves the copy of all rows, the last pass and a trip over memory each: in a trace 66 us of kernels, 85 with copies, so 56 and 63.
+// Windows of 64 are counted eight tokens at a time: the first pass 14.1 -> 8.9 us.
 // ---------------------------------------------------------------------------
 #define FILTER_THREADS 256
 #define FILTER_SLICE 4096        // 16 tokens a thread
