@@ -1,7 +1,7 @@
 // Paged attention of the 32-bit path for head sizes 64, 128 and 256; attention_plain.hip says what it computes and keeps
 // the other sizes and the bfloat16 twin.
 //
-// Both products run on the float matrix cores, 16 rows a workgroup: the heads that share a KV head, times tokens. A float product of
+// Both products run on the float matrix cores, 16 rows a workgroup: the heads that share a KV head, times tokens of a request. A float product of
 // 16x16x4 is a chain of four fused multiply-adds, in order and each rounded, so vector units can walk the same chains: few tokens, whose
 // products would be mostly empty columns, go there (attention_f32_token_kernel), and have the same bits. The tiles of 16 keys are dealt
 // out to eight shares by their number, each with a running maximum and sums of its own, that are added up through LDS at the end in
@@ -36,7 +36,9 @@ struct F32Attention {
   const int* block_tables;
   int max_blocks;
   const int *token_list, *seq_of_token, *positions;
-  int n_tokens, heads;                     // heads: of a workgroup, a power of two
+  int n_tokens, heads;                     // heads: of a workgroup, of one KV head
+  const int* cu_tokens;                    // the requests' first tokens, and the number of tokens behind them
+  int n_requests;
   int tiles;                               // of 16 slots, of a block
   unsigned long long share;                // i / tiles is i * share >> 32
   int Hq, Hkv;
@@ -262,8 +264,36 @@ __device__ __forceinline__ void walk_share(const F32Attention& g, int t, int h0,
   }
 }
 
-// 16 rows: tokens times the heads of a KV head. Tokens of several requests come one run of a request's after the other, or, with gridDim.z
-// over 1, a workgroup has the run that starts at its own token and ends at once where none does.
+// The first token of tile y when each request's tokens lie in tiles of nt of their own, and how many it has: none behind the last tile.
+__device__ __forceinline__ int tile_of(const F32Attention& g, int nt, int y, int& tokens) {
+  const int lane = threadIdx.x & 63;
+  if (g.n_requests == 1) {                 // no trip to memory: a prompt of 700 73.7 us, with it 76.6
+    tokens = max(0, min(nt, g.n_tokens - y * nt));
+    return y * nt;
+  }
+  tokens = 0;
+  for (int s0 = 0; s0 < g.n_requests; s0 += RA_WAVE) {
+    const int s = s0 + lane, first = g.cu_tokens[min(s, g.n_requests)], past = g.cu_tokens[min(s + 1, g.n_requests)];
+    const int mine = (past - first + nt - 1) / nt;
+    int upto = mine;                       // of the requests up to the lane's
+#pragma unroll
+    for (int m = 1; m < RA_WAVE; m <<= 1) {
+      const int other = __shfl_up(upto, m, RA_WAVE);
+      upto += lane >= m ? other : 0;
+    }
+    const unsigned long long here = __ballot(y < upto);
+    if (here) {
+      const int l = __builtin_amdgcn_readfirstlane(__ffsll(here) - 1);
+      const int at = __builtin_amdgcn_readlane(first, l) + (y - __builtin_amdgcn_readlane(upto - mine, l)) * nt;
+      tokens = min(nt, __builtin_amdgcn_readlane(past, l) - at);
+      return at;
+    }
+    y -= __builtin_amdgcn_readlane(upto, RA_WAVE - 1);
+  }
+  return 0;
+}
+
+// 16 rows: tokens of a request times the heads of a KV head.
 template <int D, int WAVES>
 __global__ void __launch_bounds__(WAVES * RA_WAVE) attention_f32_kernel(F32Attention g) {
   constexpr int KP = D / 32;               // pieces of 8 entries of a key a lane
@@ -274,17 +304,12 @@ __global__ void __launch_bounds__(WAVES * RA_WAVE) attention_f32_kernel(F32Atten
   __shared__ int off[ROWS];                // rows with a result that is no finite number
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
   const int lo16 = lane & 15, hi = lane >> 4;
-  const int gh = g.heads, nt = ROWS / gh;
+  const int gh = g.heads;
   const int h0 = blockIdx.x * gh, kvh = h0 / (g.Hq / g.Hkv), a = h0 + lo16 % gh;
-  // the last tokens first: theirs are the longest walks of a prompt
-  const int i0 = (gridDim.y - 1 - blockIdx.y) * nt, rows = min(ROWS, (g.n_tokens - i0) * gh);
-  const int at = i0 + min(lo16, rows - 1) / gh;
-  const int t = g.token_list ? g.token_list[at] : at;
-  const int seq = g.seq_of_token[t], pos = g.positions[t];
-  const int before = __shfl(seq, lo16 >= gh ? lo16 - gh : 0, RA_WAVE);
-  // the first rows of the requests' runs
-  const unsigned runs = __ballot(lane < rows && lo16 % gh == 0 && (lane == 0 || seq != before));
-  if (gridDim.z > 1 && !(runs >> (blockIdx.z * gh) & 1)) return;
+  int tokens;                              // the last ones first: theirs are the longest walks of a prompt
+  const int i0 = tile_of(g, ROWS / gh, gridDim.y - 1 - blockIdx.y, tokens), rows = tokens * gh;
+  if (rows == 0) return;
+  const int t = i0 + min(lo16, rows - 1) / gh, pos = g.positions[t];
   float q[KP][8];                          // the products' columns
   {
     const float* qv = g.q + (size_t)t * g.q_stride + (size_t)a * D + hi * 8;
@@ -295,159 +320,152 @@ __global__ void __launch_bounds__(WAVES * RA_WAVE) attention_f32_kernel(F32Atten
   }
   const float d1 = g.mod.r1 ? g.mod.r1[a] : 0.f, d2 = g.mod.r1 ? g.mod.r2[a] : 0.f;
 
-  for (int r0 = 0, r1; r0 < rows; r0 = r1) {             // a run: rows r0 to r1
-    const unsigned rest = runs >> r0 >> 1;
-    r1 = rest ? r0 + __ffs(rest) : rows;
-    if (gridDim.z > 1 && r0 != (int)blockIdx.z * gh) continue;
-    const bool mine = lo16 >= r0 && lo16 < r1;
-    const int* table = g.block_tables + (size_t)__builtin_amdgcn_readlane(seq, r0) * g.max_blocks;
-    const int p = mine ? pos : -1;         // a row of another request sees nothing
-    const int lo = mine ? ra_first_key(p, g.window, g.aligned) : 0;
-    const int kept = mine ? (g.keep < lo ? g.keep : lo) : 0;
-    const int end = max16(p), from = -max16(mine ? -lo : -0x7fffffff), keeps = max16(kept);      // over the run's rows
-    const F32Walk walk = {(keeps + 15) >> 4, from >> 4, end >> 4};
-    const int last = walk.last;
-    for (int share = wave; share < SHARES; share += waves) {
-      int i = walk.skip(share);
-      if (i > last) {                      // a share without a tile
-        if (lane < ROWS) {
-          ends[(share * ROWS + lane) * 2] = -INFINITY;
-          ends[(share * ROWS + lane) * 2 + 1] = 0.f;
-        }
-        continue;
+  const bool mine = lo16 < rows;
+  const int* table = g.block_tables + (size_t)__builtin_amdgcn_readfirstlane(g.seq_of_token[i0]) * g.max_blocks;
+  const int p = mine ? pos : -1;         // a row that is not there sees nothing
+  const int lo = mine ? ra_first_key(p, g.window, g.aligned) : 0;
+  const int kept = mine ? (g.keep < lo ? g.keep : lo) : 0;
+  const int end = max16(p), from = -max16(mine ? -lo : -0x7fffffff), keeps = max16(kept);      // over the rows
+  const F32Walk walk = {(keeps + 15) >> 4, from >> 4, end >> 4};
+  const int last = walk.last;
+  for (int share = wave; share < SHARES; share += waves) {
+    int i = walk.skip(share);
+    if (i > last) {                      // a share without a tile
+      if (lane < ROWS) {
+        ends[(share * ROWS + lane) * 2] = -INFINITY;
+        ends[(share * ROWS + lane) * 2 + 1] = 0.f;
       }
-      float m = -INFINITY, l = 0.f;
-      f32x4_t acc[VP], k[KP][2], v[VP];
+      continue;
+    }
+    float m = -INFINITY, l = 0.f;
+    f32x4_t acc[VP], k[KP][2], v[VP];
 #pragma unroll
-      for (int b = 0; b < VP; ++b) acc[b] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-      // behind the last tile a load counts like any other, and neither reads memory nor makes the others' wait a longer one
-      auto load_keys = [&](int i, int id) {
-        const auto tile = __builtin_amdgcn_make_buffer_rsrc((void*)(g.kcache + base_of(g, kvh, i, id, D)), 0, i <= last ? 16 * D * 4 : 0, 0x00020000);
+    for (int b = 0; b < VP; ++b) acc[b] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    // behind the last tile a load counts like any other, and neither reads memory nor makes the others' wait a longer one
+    auto load_keys = [&](int i, int id) {
+      const auto tile = __builtin_amdgcn_make_buffer_rsrc((void*)(g.kcache + base_of(g, kvh, i, id, D)), 0, i <= last ? 16 * D * 4 : 0, 0x00020000);
 #pragma unroll
-        for (int c = 0; c < KP; ++c)
+      for (int c = 0; c < KP; ++c)
 #pragma unroll
-          for (int e = 0; e < 2; ++e)
-            k[c][e] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(tile, (hi * 16 + lo16) * 32, c * 2048 + e * 16, 0));
-      };
-      auto load_values = [&](int i, int id) {
-        const auto tile = __builtin_amdgcn_make_buffer_rsrc((void*)(g.vcache + base_of(g, kvh, i, id, D)), 0, i <= last ? 16 * D * 4 : 0, 0x00020000);
+        for (int e = 0; e < 2; ++e)
+          k[c][e] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(tile, (hi * 16 + lo16) * 32, c * 2048 + e * 16, 0));
+    };
+    auto load_values = [&](int i, int id) {
+      const auto tile = __builtin_amdgcn_make_buffer_rsrc((void*)(g.vcache + base_of(g, kvh, i, id, D)), 0, i <= last ? 16 * D * 4 : 0, 0x00020000);
 #pragma unroll
-        for (int b = 0; b < VP; ++b)
-          v[b] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(tile, (hi * 16 + lo16) * 16, b * 1024, 0));
-      };
-      int id = id_of(g, table, i), next = walk.skip(i + SHARES);
-      load_keys(i, id);
-      load_values(i, id);
-      id = id_of(g, table, min(next, last));
-      for (; i <= last;) {
-        const int then = walk.skip(next + SHARES), id2 = id_of(g, table, min(then, last));
-        f32x4_t z[2 * KP], zz[2 * KP];
+      for (int b = 0; b < VP; ++b)
+        v[b] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(tile, (hi * 16 + lo16) * 16, b * 1024, 0));
+    };
+    int id = id_of(g, table, i), next = walk.skip(i + SHARES);
+    load_keys(i, id);
+    load_values(i, id);
+    id = id_of(g, table, min(next, last));
+    for (; i <= last;) {
+      const int then = walk.skip(next + SHARES), id2 = id_of(g, table, min(then, last));
+      f32x4_t z[2 * KP], zz[2 * KP];
 #pragma unroll
-        for (int c = 0; c < 2 * KP; ++c) z[c] = zz[c] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+      for (int c = 0; c < 2 * KP; ++c) z[c] = zz[c] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
+      for (int e = 0; e < 4; ++e)
 #pragma unroll
-          for (int c = 0; c < 2 * KP; ++c) {
-            f32x4_t& to = SPLIT_KEYS(D) && e > 1 ? zz[c] : z[c];
-            to = __builtin_amdgcn_mfma_f32_16x16x4f32(k[c >> 1][c & 1][e], q[c >> 1][(c & 1) * 4 + e], to, 0, 0, 0);
-          }
-        load_keys(next, id);
-        if (SPLIT_KEYS(D)) {
-#pragma unroll
-          for (int c = 0; c < 2 * KP; ++c) z[c] += zz[c];
+        for (int c = 0; c < 2 * KP; ++c) {
+          f32x4_t& to = SPLIT_KEYS(D) && e > 1 ? zz[c] : z[c];
+          to = __builtin_amdgcn_mfma_f32_16x16x4f32(k[c >> 1][c & 1][e], q[c >> 1][(c & 1) * 4 + e], to, 0, 0, 0);
         }
+      load_keys(next, id);
+      if (SPLIT_KEYS(D)) {
 #pragma unroll
-        for (int w = KP; w > 0; w >>= 1)
+        for (int c = 0; c < 2 * KP; ++c) z[c] += zz[c];
+      }
 #pragma unroll
-          for (int c = 0; c < w; ++c) z[c] += z[c + w];
-        const int key0 = i * 16 + hi * 4;
-        float s[4], top = m;
+      for (int w = KP; w > 0; w >>= 1)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s[e] = z[0][e] * g.scale;
-        if (g.mod.softcap > 0.f || g.mod.r1) {
+        for (int c = 0; c < w; ++c) z[c] += z[c + w];
+      const int key0 = i * 16 + hi * 4;
+      float s[4], top = m;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) s[e] = ra_mod_score(s[e], g.mod.softcap, g.mod.r1 != nullptr, d1, d2, p - key0 - e);
-        }
+      for (int e = 0; e < 4; ++e) s[e] = z[0][e] * g.scale;
+      if (g.mod.softcap > 0.f || g.mod.r1) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[e] = ra_mod_score(s[e], g.mod.softcap, g.mod.r1 != nullptr, d1, d2, p - key0 - e);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int key = key0 + e;
+        s[e] = key <= p && (key >= lo || key < kept) ? s[e] : -INFINITY;
+        top = fmaxf(top, s[e]);
+      }
+      top = max_rows(top);
+      const float corr = m == -INFINITY ? 0.f : expf(m - top), less = top == -INFINITY ? 0.f : top;      // all may be -inf
+      m = top;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        s[e] = expf(s[e] - less);
+        l = e == 0 ? fmaf(l, corr, s[0]) : l + s[e];
+      }
+      // slots that nobody has written yet may hold anything: a probability of zero does not make a NaN harmless
+      if (i * 16 + 15 > end || i * 16 < from) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int key = key0 + e;
-          s[e] = key <= p && (key >= lo || key < kept) ? s[e] : -INFINITY;
-          top = fmaxf(top, s[e]);
+          const bool any = key <= end && (key >= from || key < keeps);
+#pragma unroll
+          for (int b = 0; b < VP; ++b) v[b][e] = any ? v[b][e] : 0.f;
         }
-        top = max_rows(top);
-        const float corr = m == -INFINITY ? 0.f : expf(m - top), less = top == -INFINITY ? 0.f : top;      // all may be -inf
-        m = top;
+      }
+      f32x4_t y[2][VP];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          s[e] = expf(s[e] - less);
-          l = e == 0 ? fmaf(l, corr, s[0]) : l + s[e];
+      for (int b = 0; b < VP; ++b) y[0][b] = y[1][b] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int b = 0; b < VP; ++b) {
+          f32x4_t& to = y[SPLIT_VALUES(D) ? e / 2 : 0][b];
+          to = __builtin_amdgcn_mfma_f32_16x16x4f32(v[b][e], s[e], to, 0, 0, 0);
         }
-        // slots that nobody has written yet may hold anything: a probability of zero does not make a NaN harmless
-        if (i * 16 + 15 > end || i * 16 < from) {
+      load_values(next, id);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int key = key0 + e;
-            const bool any = key <= end && (key >= from || key < keeps);
+      for (int b = 0; b < VP; ++b)
 #pragma unroll
-            for (int b = 0; b < VP; ++b) v[b][e] = any ? v[b][e] : 0.f;
-          }
-        }
-        f32x4_t y[2][VP];
-#pragma unroll
-        for (int b = 0; b < VP; ++b) y[0][b] = y[1][b] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-#pragma unroll
-          for (int b = 0; b < VP; ++b) {
-            f32x4_t& to = y[SPLIT_VALUES(D) ? e / 2 : 0][b];
-            to = __builtin_amdgcn_mfma_f32_16x16x4f32(v[b][e], s[e], to, 0, 0, 0);
-          }
-        load_values(next, id);
-#pragma unroll
-        for (int b = 0; b < VP; ++b)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) acc[b][e] = fmaf(acc[b][e], corr, SPLIT_VALUES(D) ? y[0][b][e] + y[1][b][e] : y[0][b][e]);
-        i = next;
-        next = then;
-        id = id2;
-      }
-      l = sum_rows(l);
-      float* row = part + (share * ROWS + lo16) * LD;
-#pragma unroll
-      for (int b = 0; b < VP; ++b) *(f32x4_t*)(row + b * 16 + hi * 4) = acc[b];
-      if (hi == 0) {
-        ends[(share * ROWS + lo16) * 2] = m;
-        ends[(share * ROWS + lo16) * 2 + 1] = l;
-      }
+        for (int e = 0; e < 4; ++e) acc[b][e] = fmaf(acc[b][e], corr, SPLIT_VALUES(D) ? y[0][b][e] + y[1][b][e] : y[0][b][e]);
+      i = next;
+      next = then;
+      id = id2;
     }
-    if (threadIdx.x < ROWS) off[threadIdx.x] = 0;
-    __syncthreads();
-    for (int x = threadIdx.x; x < (r1 - r0) * (D / 4); x += blockDim.x) {
-      const int r = r0 + x / (D / 4), e0 = x % (D / 4) * 4, head = h0 + r % gh, one = i0 + r / gh;
-      const int token = g.token_list ? g.token_list[one] : one;
-      const f32x4_t y = add_shares<f32x4_t>(ends + r * 2, ROWS * 2, part + r * LD + e0, ROWS * LD,
-                                            g.ho.sink ? g.ho.sink[head] : -INFINITY, ra_head_gate<float>(g.ho, token, head));
+    l = sum_rows(l);
+    float* row = part + (share * ROWS + lo16) * LD;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        if (!(fabsf(y[e]) <= 3.402823466e38f)) off[r] = 1;
-        g.out[(size_t)token * g.out_stride + (size_t)head * D + e0 + e] = y[e];
-      }
+    for (int b = 0; b < VP; ++b) *(f32x4_t*)(row + b * 16 + hi * 4) = acc[b];
+    if (hi == 0) {
+      ends[(share * ROWS + lo16) * 2] = m;
+      ends[(share * ROWS + lo16) * 2 + 1] = l;
     }
-    __syncthreads();
-    // A key that a row does not see weighs zero there, and zero times a value that is no finite number is none: a row with such a result
-    // is worked out again, from the keys it sees alone.
-    for (int r = r0; r < r1; ++r) {
-      if (!off[r]) continue;
-      const int one = i0 + r / gh, head = h0 + r % gh, token = g.token_list ? g.token_list[one] : one;
-      __syncthreads();
-      for (int share = wave; share < SHARES; share += waves)
-        walk_share<D, 1>(g, token, head, table, share, part + share * D, ends + share * 2);
-      __syncthreads();
-      for (int e = threadIdx.x; e < D; e += blockDim.x)
-        g.out[(size_t)token * g.out_stride + (size_t)head * D + e] = add_shares<float>(
-            ends, 2, part + e, D, g.ho.sink ? g.ho.sink[head] : -INFINITY, ra_head_gate<float>(g.ho, token, head));
+  }
+  if (threadIdx.x < ROWS) off[threadIdx.x] = 0;
+  __syncthreads();
+  for (int x = threadIdx.x; x < rows * (D / 4); x += blockDim.x) {
+    const int r = x / (D / 4), e0 = x % (D / 4) * 4, head = h0 + r % gh, token = i0 + r / gh;
+    const f32x4_t y = add_shares<f32x4_t>(ends + r * 2, ROWS * 2, part + r * LD + e0, ROWS * LD,
+                                          g.ho.sink ? g.ho.sink[head] : -INFINITY, ra_head_gate<float>(g.ho, token, head));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (!(fabsf(y[e]) <= 3.402823466e38f)) off[r] = 1;
+      g.out[(size_t)token * g.out_stride + (size_t)head * D + e0 + e] = y[e];
     }
+  }
+  __syncthreads();
+  // A key that a row does not see weighs zero there, and zero times a value that is no finite number is none: a row with such a result
+  // is worked out again, from the keys it sees alone.
+  for (int r = 0; r < rows; ++r) {
+    if (!off[r]) continue;
+    const int head = h0 + r % gh, token = i0 + r / gh;
     __syncthreads();
+    for (int share = wave; share < SHARES; share += waves)
+      walk_share<D, 1>(g, token, head, table, share, part + share * D, ends + share * 2);
+    __syncthreads();
+    for (int e = threadIdx.x; e < D; e += blockDim.x)
+      g.out[(size_t)token * g.out_stride + (size_t)head * D + e] = add_shares<float>(
+          ends, 2, part + e, D, g.ho.sink ? g.ho.sink[head] : -INFINITY, ra_head_gate<float>(g.ho, token, head));
   }
 }
 
@@ -475,32 +493,39 @@ int go_tokens(const F32Attention& g, hipStream_t stream) {
 }
 
 template <int D>
-int go(F32Attention g, int n_requests, hipStream_t stream) {
+int go(F32Attention g, hipStream_t stream) {
   const int group = g.Hq / g.Hkv;
   const long cus = ra_cu_count();
+  // all heads of a group, or as many of them as tokens fill 12 of the 16 rows with at least: keys and values are read once for them
   g.heads = 1;
-  while (g.heads < ROWS && group % (2 * g.heads) == 0) g.heads *= 2;
-  // Tokens on their own while their workgroups find room at once, and where most of the products' 16 columns would stay empty; a request
-  // of several tokens up to twice as many, for its rows are one workgroup's. Two heads share what is read of a key they both read, but
-  // for so few that the chip has room for each. 32 heads of 128 on 8 KV heads, us, a head each / two / 16 rows: 1 token at 300 keys
-  // 8.9 / 10.4 / 15.4, 4 tokens of 4 requests at 600 18.0 / 15.3 / 22.2, 8 of 8 28.5 / 19.2 / 23.1, 16 of 16 at 500 43.0 / 25.5 / 21.5,
-  // 64 of 64 161 / 83 / 52; prompts of 16 6.7 / 7.0 / 10.2, 24 9.4 / 9.7 / 10.1, 40 11.9 / 12.9 / 10.5, 80 19.3 / 20.5 / 11.8; on 32 KV
-  // heads, 16 of 16 at 500 43.4 / - / 52.9, a prompt of 200 51.8 / - / 18.0.
-  const int each = n_requests > 0 && n_requests < g.n_tokens ? g.n_tokens / n_requests : 1;
+  for (int h = 2; h <= ROWS; ++h)
+    if (group % h == 0 && ROWS / h * h >= 12) g.heads = h;
+  const int nt = ROWS / g.heads;
+  // Tokens on their own until their workgroups wait for one another, and where the products' 16 columns would stay all but empty; a request's
+  // tokens share what is read of its keys in the caches either way and go further so. Two heads of single tokens share what is read
+  // of a key they both read, but for so few that the chip has room for each. us, a head each / two / 16 rows: 32 heads of 128 on 8 KV
+  // heads at 300 keys, 4 tokens of 4 requests 12.4 / 10.5 / 16.0, 8 of 8 17.4 / 12.5 / 16.0, 16 of 16 29.5 / 17.9 / 17.6, 64 of 64 95 / 54 / 33; a
+  // prompt of 24 9.3 / 9.7 / 11.2, 33 11.5 / 12.6 / 11.2, 64 15.6 / 16.5 / 11.6, 250 69 / 76 / 21, 24 tokens behind 1000 36 / 34 / 32; 8 single
+  // ones beside a portion of 100 37 / 32 / 21 (of 40 heads 41 / - / 21). 32 on 32: 64 of 64 at 300 112 / - / 122, a prompt of 64 15.6 / -
+  // / 11.8. 16 of 64 on 16: prompts of 64 7.6 / - / 9.4, 128 11.5 / - / 10.6, 250 22 / - / 12.5. 16 of 256 on 2: 8 of 8 at 300 17.7 / - / 26,
+  // 16 of 16 27.8 / - / 26.3, 64 of 64 92 / - / 29. Over 29 steps of 13 shapes what is taken is nowhere more than 28 % behind the best (24 tokens
+  // behind 1000, two heads would be ahead), in 17 of 377 more than 10 %.
   const bool two = D <= 128 && group % 2 == 0;
-  const long alone = (long)g.Hq * g.n_tokens / (two ? 2 : 1);
-  if (g.heads * (each < ROWS ? each : ROWS) < 2 || alone <= (each > 1 ? cus : cus / 2)) {
+  const int each = g.n_requests > 0 ? g.n_tokens / g.n_requests : 1;        // tokens of a request, or so
+  const double alone = (double)g.Hq * g.n_tokens / cus;                    // workgroups of a head and token, a CU's share
+  const bool pair = two && each < 4 && alone > (D == 64 ? 0.75 : 0.35);
+  const double least = each < 2 ? (D == 64 ? 1.25 : 1.0) : each < 4 ? 2.0 : D == 64 ? 6.0 : D == 128 ? 3.5 : 2.8;
+  if (g.n_requests == 0 || g.heads * (each < nt ? each : nt) < 3 || alone < least * (pair ? 2 : 1)) {
     if constexpr (D <= 128)
-      if (two && (long)g.Hq * g.n_tokens * 4 > cus) return go_tokens<D, 2>(g, stream);
+      if (pair) return go_tokens<D, 2>(g, stream);
     return go_tokens<D, 1>(g, stream);
   }
-  const long pairs = g.Hq / g.heads;
-  const int nt = ROWS / g.heads, tiles = (g.n_tokens + nt - 1) / nt;
-  // a workgroup a request's run of tokens where a workgroup a token would be a few rounds of the chip, else one for all runs of its rows
-  const int z = pairs * g.n_tokens <= 8 * cus ? (nt < g.n_tokens ? nt : g.n_tokens) : 1;
+  // eight waves, a share each, while that leaves CUs without a workgroup: 33 tokens behind 300 18.4 us, of four waves 20.2; 250 from their start 24.5
+  // and 20.9
+  const long pairs = g.Hq / g.heads, tiles = (g.n_tokens - g.n_requests) / nt + g.n_requests;        // at most
   const int waves = D > 128 || pairs * tiles > cus ? 4 : 8;
   constexpr int W = D <= 128 ? 8 : 4;
-  attention_f32_kernel<D, W><<<dim3(pairs, tiles, z), waves * RA_WAVE, 0, stream>>>(g);
+  attention_f32_kernel<D, W><<<dim3(pairs, tiles), waves * RA_WAVE, 0, stream>>>(g);
   RA_LAUNCH_CHECK("attention_f32");
   return 0;
 }
@@ -516,12 +541,12 @@ bool ra_attention_f32_takes(const void* kcache, const void* vcache, int d, int b
 
 int ra_attention_f32(const float* q, int q_stride, float* out, int out_stride, const float* kcache, const float* vcache,
                      const int* block_tables, int max_blocks, const int* token_list, const int* seq_of_token,
-                     const int* positions, int n_tokens, int n_requests, int block_size, int Hq, int Hkv, int d, float scale,
+                     const int* positions, int n_tokens, const int* cu_tokens, int n_requests, int block_size, int Hq, int Hkv, int d, float scale,
                      int window, int aligned, int keep, RaScoreMod mod, RaHeadOut ho, hipStream_t stream) {
   const F32Attention g = {q, q_stride, out, out_stride, kcache, vcache, block_tables, max_blocks, token_list, seq_of_token,
-                          positions, n_tokens, 1, block_size / 16, (1ull << 32) / (block_size / 16) + 1, Hq, Hkv, scale, window, aligned, keep, mod, ho};
-  if (d == 64) return go<64>(g, n_requests, stream);
-  if (d == 128) return go<128>(g, n_requests, stream);
-  if (d == 256) return go<256>(g, n_requests, stream);
+                          positions, n_tokens, 1, cu_tokens, n_requests, block_size / 16, (1ull << 32) / (block_size / 16) + 1, Hq, Hkv, scale, window, aligned, keep, mod, ho};
+  if (d == 64) return go<64>(g, stream);
+  if (d == 128) return go<128>(g, stream);
+  if (d == 256) return go<256>(g, stream);
   return ra_fail("attention_f32: head size %d", d);
 }

@@ -21,8 +21,8 @@
 bool ra_attention_f32_takes(const void* kcache, const void* vcache, int d, int block_size, int max_blocks);
 int ra_attention_f32(const float* q, int q_stride, float* out, int out_stride, const float* kcache, const float* vcache,
                      const int* block_tables, int max_blocks, const int* token_list, const int* seq_of_token,
-                     const int* positions, int n_tokens, int n_requests, int block_size, int Hq, int Hkv, int d, float scale,
-                     int window, int aligned, int keep, RaScoreMod mod, RaHeadOut ho, hipStream_t stream);
+                     const int* positions, int n_tokens, const int* cu_tokens, int n_requests, int block_size, int Hq, int Hkv, int d,
+                     float scale, int window, int aligned, int keep, RaScoreMod mod, RaHeadOut ho, hipStream_t stream);
 
 template <typename TA>
 __global__ void attention_plain_kernel(const TA* __restrict__ q, int q_stride, TA* __restrict__ out,
@@ -117,15 +117,15 @@ extern "C" int ra_attention_plain(const void* q, int q_stride, void* out, int ou
                                   const int* seq_of_token, const int* positions, int n_tokens, int block_size, int Hq, int Hkv,
                                   int d, float scale, int window, hipStream_t stream) {
   return ra_attention_plain_mod(q, q_stride, out, out_stride, kcache, vcache, act_dtype, block_tables, max_blocks,
-                                token_list, seq_of_token, positions, n_tokens, 0, block_size, Hq, Hkv, d, scale, window,
+                                token_list, seq_of_token, positions, n_tokens, nullptr, 0, block_size, Hq, Hkv, d, scale, window,
                                 0, 0, 0.f, nullptr, nullptr, nullptr, nullptr, 0, stream);
 }
 
 extern "C" int ra_attention_plain_mod(const void* q, int q_stride, void* out, int out_stride,
                                       const void* kcache, const void* vcache, int act_dtype,
                                       const int* block_tables, int max_blocks, const int* token_list,
-                                      const int* seq_of_token, const int* positions, int n_tokens, int n_requests, int block_size,
-                                      int Hq, int Hkv, int d, float scale, int window, int aligned, int keep,
+                                      const int* seq_of_token, const int* positions, int n_tokens, const int* cu_tokens, int n_requests,
+                                      int block_size, int Hq, int Hkv, int d, float scale, int window, int aligned, int keep,
                                       float softcap, const float* r1, const float* r2, const float* sink,
                                       const void* gate, int gate_stride, hipStream_t stream) {
   RA_CHECK((r1 == nullptr) == (r2 == nullptr) && softcap >= 0.f,
@@ -141,10 +141,12 @@ extern "C" int ra_attention_plain_mod(const void* q, int q_stride, void* out, in
            block_size, d);
   RA_CHECK(window >= 0 && keep >= 0, "attention_plain: negative window or number of kept keys");
   RA_CHECK(n_tokens <= 65535, "attention_plain: %d tokens in one launch (max 65535)", n_tokens);
+  RA_CHECK(n_requests >= 0 && (n_requests == 0) == (cu_tokens == nullptr) && (n_requests == 0 || !token_list),
+           "attention_plain: %d requests' tokens", n_requests);
   if (act_dtype == RA_F32 && ra_attention_f32_takes(kcache, vcache, d, block_size, max_blocks))
     return ra_attention_f32((const float*)q, q_stride, (float*)out, out_stride, (const float*)kcache,
                             (const float*)vcache, block_tables, max_blocks, token_list, seq_of_token, positions, n_tokens,
-                            n_requests, block_size, Hq, Hkv, d, scale, window, aligned, keep, mod, ho, stream);
+                            cu_tokens, n_requests, block_size, Hq, Hkv, d, scale, window, aligned, keep, mod, ho, stream);
   dim3 grid(Hq, n_tokens);
   const size_t lds = (size_t)(d + RA_WAVE) * sizeof(float);
   if (act_dtype == RA_F32)

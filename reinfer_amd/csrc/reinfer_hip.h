@@ -63,11 +63,12 @@ int ra_attention_plain(const void* q, int q_stride, void* out, int out_stride, c
 // first keep keys are seen as well, however far the window has moved on. aligned: a query sees the keys of its own chunk,
 // the keys being cut into chunks of `window` from position 0. sink (float, one entry a query head, or null): one more term
 // exp(sink[h]) in the softmax's denominator. gate (activations' type, gate[t * gate_stride + h], or null): a head's result
-// times its sigmoid. n_requests: whose the tokens are, or 0 where that is not known; it chooses between ways to the same bits.
+// times its sigmoid. cu_tokens [n_requests + 1]: the step's tokens request by request, or null and 0 where that is not known or tokens are
+// listed; it allows a way to the same bits that is the faster one for many of them.
 int ra_attention_plain_mod(const void* q, int q_stride, void* out, int out_stride, const void* kcache,
                            const void* vcache, int act_dtype, const int* block_tables, int max_blocks,
-                           const int* token_list, const int* seq_of_token, const int* positions, int n_tokens, int n_requests,
-                           int block_size, int Hq, int Hkv, int d, float scale, int window, int aligned, int keep,
+                           const int* token_list, const int* seq_of_token, const int* positions, int n_tokens,
+                           const int* cu_tokens, int n_requests, int block_size, int Hq, int Hkv, int d, float scale, int window, int aligned, int keep,
                            float softcap, const float* r1, const float* r2, const float* sink, const void* gate,
                            int gate_stride, hipStream_t stream);
 // act 2 of ra_act_mul with its bound: g <- min(g, lim), u <- clamp(u, -lim, lim), out = g sigmoid(1.702 g) (u + 1)

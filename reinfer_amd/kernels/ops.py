@@ -578,9 +578,9 @@ class HipKernels:
         library.call("ra_attention_plain_mod", q.data_ptr(), q_stride, out.data_ptr(), out.stride(0),
                      kcache.data_ptr(), vcache.data_ptr(), _tag(q, "attention"), tables.data_ptr(),
                      tables.shape[1], _ptr(token_list), batch.seq_of_token.data_ptr(),
-                     batch.positions.data_ptr(), n, batch.num_seqs if token_list is None else 0, kcache.shape[2] * 16, num_heads,
-                     num_kv_heads, head_dim, float(scale), int(window), int(aligned), int(keep), mod[0], mod[1], mod[2], *head_out,
-                     _stream())
+                     batch.positions.data_ptr(), n, batch.cu_tokens.data_ptr() if token_list is None else None,
+                     batch.num_seqs if token_list is None else 0, kcache.shape[2] * 16, num_heads, num_kv_heads, head_dim,
+                     float(scale), int(window), int(aligned), int(keep), mod[0], mod[1], mod[2], *head_out, _stream())
 
     # The decode kernel runs in workgroups of 12 waves from this many (token, KV head) pairs on, or over
     # contexts longer than this; below both, in workgroups of 4 (measured with 32 query heads over 8 KV

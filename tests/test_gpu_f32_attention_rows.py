@@ -28,7 +28,7 @@ def exact(q, kc, vc, n, start, table, Hq, Hkv, d, window, keep, aligned):
     return torch.einsum("htk,khd->thd", torch.softmax(s, -1), V).reshape(n, -1)
 
 
-# groups of 1 (16 tokens a workgroup), 3 (as 1, all of a workgroup's requests in turn), 4, 8 and 16 (one); blocks of one tile and three
+# groups of 1 (16 tokens a workgroup), 3 (five), 4, 8 and 16 (one); blocks of one tile and three
 @pytest.mark.parametrize("Hq,Hkv,d,bs", [(6, 6, 64, 16), (24, 8, 128, 48), (16, 4, 128, 16), (16, 2, 256, 16), (32, 2, 64, 48)])
 @pytest.mark.parametrize("how", [{}, {"window": 37}, {"window": 100, "keep": 21}, {"window": 64, "aligned": True},
                                  {"softcap": 5.0}])
@@ -69,3 +69,44 @@ def test_a_value_that_is_no_finite_number_reaches_those_alone_that_see_it(bad):
     for t in (50, n - 1):
         one = attend(q[t:t + 1].contiguous(), kc, vc, [1], [t], tables, Hq, Hkv, d).view(Hkv, -1, d)
         assert torch.equal(out[t].nan_to_num(), one.nan_to_num()) and torch.equal(out[t].isnan(), one.isnan())
+
+
+# groups of 5, 7 and 14 (all heads a workgroup), 6 (two tokens), 24 (12 heads) and 11 (a head each); more requests than a wave has lanes
+@pytest.mark.parametrize("Hq,Hkv,d", [(40, 8, 128), (14, 2, 64), (28, 2, 64), (12, 2, 256), (24, 1, 128), (22, 2, 64)])
+def test_steps_of_many_requests(Hq, Hkv, d):
+    """Single tokens beside portions, a few tokens of many requests: tiles of each request's own, of which a step's first and last count."""
+    for q_lens in ([1] * 9 + [100] + [1] * 3, [1 + i % 5 for i in range(70)], [3] * 64 + [40], [1] * 130):
+        starts = [(37 * i) % 210 for i in range(len(q_lens))]
+        q, kc, vc, tables = make_paged_case("float32", Hq, Hkv, d, q_lens, starts, seed=len(q_lens))
+        whole = attend(q, kc, vc, q_lens, starts, tables, Hq, Hkv, d)
+        assert torch.isfinite(whole).all()
+        at = 0
+        for i, (n, s) in enumerate(zip(q_lens, starts)):
+            if i % 11 == 0 or n > 30 or i == len(q_lens) - 1:
+                for t in {0, n - 1}:
+                    one = attend(q[at + t:at + t + 1].contiguous(), kc, vc, [1], [s + t], tables[i:i + 1], Hq, Hkv, d)
+                    assert torch.equal(one, whole[at + t:at + t + 1]), (len(q_lens), i, t)
+            at += n
+
+
+def test_many_requests_beside_a_portion_take_what_their_workgroups_take():
+    """Eight single tokens and a portion of 100, 40 heads on 8 KV heads: a workgroup that took 16 tokens of nine requests one request after
+    the other made this four times the portion alone."""
+    Hq, Hkv, d = 40, 8, 128
+
+    def time(q_lens, starts):
+        q, kc, vc, tables = make_paged_case("float32", Hq, Hkv, d, q_lens, starts, seed=1)
+        out, batch, best = torch.empty(sum(q_lens), Hq * d, device=DEV), FakeBatch(q_lens, starts, tables), float("inf")
+        rows, k, v = q.reshape(sum(q_lens), Hq * d), kt(kc), vt(vc)
+        for _ in range(8):
+            first, last = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            torch.cuda._sleep(200000)
+            first.record()
+            for _ in range(4):
+                kernels.current().attention(rows, Hq * d, out, k, v, batch, Hq, Hkv, d, d ** -0.5, window=0, group=0)
+            last.record()
+            torch.cuda.synchronize()
+            best = min(best, first.elapsed_time(last))
+        return best
+    # as workgroups of their own the single ones add 64 to 56: 1.5 times (measured), with room for twice that
+    assert time([1] * 8 + [100], [300] * 8 + [0]) < 3 * time([100], [0])
