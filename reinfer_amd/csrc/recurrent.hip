@@ -821,10 +821,13 @@ struct MeanInputs {
 };
 // HELD: rows that two runs of eight neighbouring elements a thread cover, read in 16-byte accesses, all asked for at once with the
 // weights and the stream's old values, and handed round in LDS for the sums, whose order is the other form's; else every element is
-// read twice, one a thread at a time. Eight rows of 4096, two inputs, in a decode step: 10.1 us read twice, 5.0 held.
+// read twice, one a thread at a time. Eight rows of 4096, two inputs, in a decode step: 10.1 us read twice, 5.0 held. With four inputs
+// held rows take registers and LDS that many rows would share a CU by: held while each has a CU of its own. us, read twice / held,
+// four inputs of 4096, 8 rows 9.2 / 7.7, 64 9.2 / 7.7, 300 11.2 / 11.8, 2000 30 / 36; three of 4096 2000 rows 24 / 22, of 520 9.6 / 10.3; two
+// of 4096 1000 rows 16.0 / 12.6. (A workgroup is told to be of 512 threads at most: as if of 1024 four held inputs spilled, 8 rows 12.0.)
 #define MEAN_LDS (64 * 1024)
 template <typename TA, int N, bool HELD>
-__global__ void normed_mean_kernel(MeanInputs in, float eps, int h, TA* __restrict__ out, float* __restrict__ resid,
+__global__ void __launch_bounds__(512) normed_mean_kernel(MeanInputs in, float eps, int h, TA* __restrict__ out, float* __restrict__ resid,
                                    float scale) {
   extern __shared__ __attribute__((aligned(16))) float held[];       // [N][h]
   __shared__ float red[N][17];
@@ -1304,6 +1307,7 @@ extern "C" int ra_normed_mean(const void* const* xs, const float* const* ws, int
   const int threads = hidden >= 2048 ? 512 : 256;
   const long lds = (long)n * hidden * (long)sizeof(float);
   bool held = hidden % 8 == 0 && hidden <= 16 * threads && lds <= MEAN_LDS && (uintptr_t)out % 16 == 0 && (uintptr_t)resid % 16 == 0;
+  held = held && (n <= 3 || n_tokens <= ra_cu_count());
   for (int i = 0; i < n; ++i) held = held && (uintptr_t)xs[i] % 16 == 0 && (uintptr_t)ws[i] % 16 == 0;
 #define RA_NM(TA, N)                                                                                                       \
   do {                                                                                                                     \

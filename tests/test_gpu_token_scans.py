@@ -95,3 +95,23 @@ def test_mean_of_normed_rows(h, n, dtype):
     # sums of h squares: their relative error is below h 2^-24 at worst, half of it reaches the result; products of a few roundings
     assert (resid.double() - (base.double() + 0.5 * want)).abs().max() <= (h / 2 + 8) * 2.0 ** -24 * 8
     assert (out.double() - want).abs().max() <= ((h / 2 + 8) * 2.0 ** -24 + (2.0 ** -9 if dtype == torch.bfloat16 else 0.0)) * 8
+
+
+# whole runs of eight for each thread and for some; one row fewer, as many rows as CUs, and one more, where rows are read twice again
+@pytest.mark.parametrize("h", [520, 4096])
+@pytest.mark.parametrize("n", [2, 3, 4])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_mean_of_as_many_rows_as_cus(h, n, dtype):
+    cus = torch.cuda.get_device_properties(DEV).multi_processor_count
+    g = torch.Generator(device=DEV).manual_seed(h + n)
+    xs = [torch.randn(cus + 1, h, generator=g, device=DEV).to(dtype) for _ in range(n)]
+    ws = [torch.rand(h, generator=g, device=DEV) + 0.5 for _ in range(n)]
+    want = sum(x.double() / (x.double().pow(2).mean(-1, keepdim=True) + 1e-6).sqrt() * w.double() for x, w in zip(xs, ws)) / n
+    outs = []
+    for rows in (1, cus - 1, cus, cus + 1):
+        resid = torch.ones(rows, h, device=DEV)
+        kernels.current().normed_mean([x[:rows] for x in xs], ws, 1e-6, resid=resid, scale=0.5)
+        assert (resid.double() - 1 - 0.5 * want[:rows]).abs().max() <= (h / 2 + 8) * 2.0 ** -24 * 8
+        outs.append(resid)
+    for a in outs[:-1]:
+        assert torch.equal(a, outs[-1][:len(a)])
