@@ -575,6 +575,8 @@ class HipKernels:
         tables = self._check_attention(q, q_stride, out, kcache, vcache, batch, num_heads, num_kv_heads,
                                        head_dim, group)
         n = batch.num_tokens if token_list is None else int(n_listed)
+        if token_list is None:
+            _int32(batch.cu_tokens, "first token of each request", batch.num_seqs + 1)
         library.call("ra_attention_plain_mod", q.data_ptr(), q_stride, out.data_ptr(), out.stride(0),
                      kcache.data_ptr(), vcache.data_ptr(), _tag(q, "attention"), tables.data_ptr(),
                      tables.shape[1], _ptr(token_list), batch.seq_of_token.data_ptr(),

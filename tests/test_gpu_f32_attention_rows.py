@@ -110,3 +110,13 @@ def test_many_requests_beside_a_portion_take_what_their_workgroups_take():
         return best
     # as workgroups of their own the single ones add 64 to 56: 1.5 times (measured), with room for twice that
     assert time([1] * 8 + [100], [300] * 8 + [0]) < 3 * time([100], [0])
+
+
+def test_first_tokens_that_the_kernel_cannot_read_are_refused():
+    q, kc, vc, tables = make_paged_case("float32", 4, 2, 64, [3, 2], [0, 5], seed=0)
+    batch, out = FakeBatch([3, 2], [0, 5], tables), torch.empty(5, 256, device=DEV)
+    cu = batch.cu_tokens
+    for wrong, error in ((cu.long(), TypeError), (cu[:2], ValueError), (torch.stack([cu, cu], 1)[:, 0], TypeError)):
+        batch.cu_tokens = wrong
+        with pytest.raises(error):
+            kernels.current().attention(q.reshape(5, -1), 256, out, kt(kc), vt(vc), batch, 4, 2, 64, 0.125, window=0, group=0)
