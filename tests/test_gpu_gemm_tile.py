@@ -142,3 +142,64 @@ def test_rows_too_far_apart_to_address_stay_with_the_library():
         x = torch.empty((M - 1) * stride + K, device=DEV, dtype=torch.bfloat16).as_strided((M, K), (stride, 1))
         assert ops()._tile_takes(2, x, w, torch.empty(M, N, device=DEV)) == taken
         assert taken or ops().linear_ranges(x, w) is None
+
+
+# a width of tile each (64, 80, 96, 112, 128, 160 features; fewer tiles than CUs, one more than they are, and several rounds), N and K at
+# and off whole tiles, stages and pieces of four, rows on both sides of a tile of 16 and of the 32 and 64 that the kernel is built for
+@pytest.mark.parametrize("M", [16, 17, 32, 33, 49, 64])
+@pytest.mark.parametrize("N,K", [(19456, 264), (24576, 320), (51200, 128), (151936, 72), (40016, 640), (32896, 8), (6144, 2560), (2560, 4104)])
+def test_few_rows_in_tiles_of_every_width(M, N, K):
+    """Plain results in both types, with and without a bias and at a stride that is in no whole pieces; added; gated."""
+    x, w, g = operands(M, N, K, M + N + K)
+    ref, err = x.double() @ w.double().T, bound(x, w, K)
+    bias = torch.randn(N, device=DEV, generator=g).to(torch.bfloat16)
+    for kind, ulp in ((torch.float32, 2.0 ** -23), (torch.bfloat16, 2.0 ** -8)):
+        for wide, b in ((N + 8, None), (N + 8, bias), (N + 3, None)):
+            buf = torch.full((M, wide), float("nan"), device=DEV, dtype=kind)
+            ops().linear_skinny(x, w, buf[:, :N], b, wide=True)
+            want = ref if b is None else ref + b.double()
+            assert ((buf[:, :N].double() - want).abs() <= err + want.abs() * ulp).all()
+            assert torch.isnan(buf[:, N:]).all()
+    stream = torch.randn(M, N, device=DEV, generator=g)
+    want = stream.double() + ref
+    ops().linear_skinny(x, w, stream, accumulate=True, wide=True)
+    assert ((stream.double() - want).abs() <= err + want.abs() * 2 ** -23).all()
+    out = torch.full((M, N // 2), float("nan"), device=DEV, dtype=torch.bfloat16)
+    ops().gated_linear(x, w, out, wide=True)
+    rows = torch.arange(N, device=DEV).view(-1, 2, 8)
+    gate, up = ref[:, rows[:, 0].reshape(-1)], ref[:, rows[:, 1].reshape(-1)]
+    eg, eu = err[:, rows[:, 0].reshape(-1)], err[:, rows[:, 1].reshape(-1)]
+    want = gate * torch.sigmoid(gate) * up
+    assert ((out.double() - want).abs() <= 1.1 * eg * (up.abs() + eu) + gate.abs() * eu + want.abs() * (2 ** -8 + 2 ** -20)).all()
+
+
+@pytest.mark.parametrize("M", [17, 48, 64])
+@pytest.mark.parametrize("parts", [1, 4, 5, 8, 9, 160, 257])
+def test_a_carried_norm_of_any_number_of_parts(M, parts):
+    N, K, eps = 24576, 192, 1e-6
+    x, w, g = operands(M, N, K, parts)
+    ss = torch.rand(parts, M, device=DEV, generator=g) + 0.1
+    factor = torch.rsqrt(ss.double().sum(0) / K + eps)[:, None]
+    out = torch.full((M, N), float("nan"), device=DEV)
+    ops().linear_skinny(x, w, out, row_sums=(ss, eps, K))
+    want = x.double() @ w.double().T * factor
+    # the sums of the parts and the factor: parts + 4 roundings at most
+    assert ((out.double() - want).abs() <= bound(x, w, K) * factor + want.abs() * (parts + 4) * 2 ** -24).all()
+
+
+def test_a_gate_of_what_is_not_finite():
+    """silu of infinities and of what overflows: as the float formula has them."""
+    M, I, K = 17, 12288, 64
+    x, w = torch.zeros(M, K, device=DEV, dtype=torch.bfloat16), torch.zeros(2 * I, K, device=DEV, dtype=torch.bfloat16)
+    x[:, 0] = 1
+    gate = torch.tensor([0.0, 1e30, -1e30, 88.0, -88.0, 130.0, -130.0, float("inf"), float("-inf"), float("nan")], device=DEV).to(torch.bfloat16)
+    rows = torch.arange(2 * I, device=DEV).view(-1, 2, 8)
+    w[rows[:, 0].reshape(-1)[:len(gate)], 0] = gate
+    w[rows[:, 1].reshape(-1), 0] = 1
+    out = torch.empty(M, I, device=DEV, dtype=torch.bfloat16)
+    ops().gated_linear(x, w, out, wide=True)
+    v = gate.float()
+    want = torch.where(v <= -88, v * 0, v * torch.sigmoid(v))
+    want[8] = float("nan")                  # minus infinity over infinity
+    got = out[0, :len(gate)].float()
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.allclose(got.nan_to_num(0.0, 1e38, -1e38), want.nan_to_num(0.0, 1e38, -1e38), rtol=2 ** -8, atol=1e-30)
