@@ -448,6 +448,15 @@ static hipError_t fd_allow_lds(size_t lds) {
   return hipSuccess;
 }
 
+// the exact form of a head size needs a few registers more than the other: it is asked for
+template <int DM>
+static hipError_t fd_occupancy(int waves, size_t lds, int* per_cu) {
+  const hipError_t e = waves == 4 ? fd_allow_lds<DM, true, 4>(lds) : fd_allow_lds<DM, true, 12>(lds);
+  if (e != hipSuccess) return e;
+  return waves == 4 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, flash_decode_kernel<DM, true, 4, 0>, 4 * RA_WAVE, lds)
+                    : hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, flash_decode_kernel<DM, true, 12, 0>, 12 * RA_WAVE, lds);
+}
+
 static int fd_resident_workgroups(int variant, int waves, size_t lds) {
   static int cached[3][2] = {{0, 0}, {0, 0}, {0, 0}};
   static size_t cached_lds[3][2] = {{0, 0}, {0, 0}, {0, 0}};
@@ -457,16 +466,9 @@ static int fd_resident_workgroups(int variant, int waves, size_t lds) {
   if (hipGetDevice(&dev) != hipSuccess) return 0;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
   hipError_t e = hipSuccess;
-  // the exact form of a head size needs a few registers more than the other: ask for it
-#define RA_FD_OCC(DM)                                                                                                  \
-  e = waves == 4 ? fd_allow_lds<DM, true, 4>(lds) : fd_allow_lds<DM, true, 12>(lds);                                   \
-  if (e == hipSuccess)                                                                                                 \
-  e = waves == 4 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, flash_decode_kernel<DM, true, 4, 0>, 4 * RA_WAVE, lds) \
-                 : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, flash_decode_kernel<DM, true, 12, 0>, 12 * RA_WAVE, lds)
-  if (variant == 0) RA_FD_OCC(64);
-  else if (variant == 1) RA_FD_OCC(128);
-  else RA_FD_OCC(256);
-#undef RA_FD_OCC
+  if (variant == 0) e = fd_occupancy<64>(waves, lds, &per_cu);
+  else if (variant == 1) e = fd_occupancy<128>(waves, lds, &per_cu);
+  else e = fd_occupancy<256>(waves, lds, &per_cu);
   if (e != hipSuccess || cus <= 0 || per_cu <= 0) return 0;
   cached[variant][wi] = cus * per_cu;
   cached_lds[variant][wi] = lds;

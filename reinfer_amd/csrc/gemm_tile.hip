@@ -486,7 +486,7 @@ int ra_tile_product(int epilogue, const RaTilePlan& plan, const void* A, int lda
                     RaTileEnd end, hipStream_t stream) {
   RA_CHECK(M > 0 && N > 0 && K > 0 && K % 8 == 0 && lda % 8 == 0 && lda >= K && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0,
            "gemm_tile: [%d, %d, %d] with rows of stride %d must be whole 16-byte pieces", M, N, K, lda);
-  RA_CHECK((size_t)GT_SIDE * K * 2 < 0x7FFFFF00ull && ((size_t)(M - 1) * lda + K) * 2 < 0x7FFFFF00ull,
+  RA_CHECK((size_t)160 * K * 2 < 0x7FFFFF00ull && ((size_t)(M - 1) * lda + K) * 2 < 0x7FFFFF00ull,
            "gemm_tile: an operand of [%d, %d, %d] is larger than a descriptor covers", M, N, K);
   RA_CHECK(plan.ranges >= 1 && plan.range_k % GT_BK == 0 && (long)(plan.ranges - 1) * plan.range_k < K &&
                (long)plan.ranges * plan.range_k >= K && (plan.ranges == 1 || epilogue == GT_PART),

@@ -584,20 +584,13 @@ class HipKernels:
                      batch.num_seqs if token_list is None else 0, kcache.shape[2] * 16, num_heads, num_kv_heads, head_dim,
                      float(scale), int(window), int(aligned), int(keep), mod[0], mod[1], mod[2], *head_out, _stream())
 
-    # The decode kernel runs in workgroups of 12 waves from this many (token, KV head) pairs on, or over
-    # contexts longer than this; below both, in workgroups of 4 (measured with 32 query heads over 8 KV
-    # heads of 128, flash decode and merge together: 2200 keys a token, 1 / 4 / 8 / 16 / 32 / 64 tokens: 4 waves
-    # 10.6 / 13.1 / 23.3 / 40.4 / 61.3 / 107 us, 12 waves 13.6 / 14.5 / 21.5 / 33.8 / 56.2 / 107; 8000 keys,
-    # 1 / 4 / 16 / 64 tokens: 17.9 / 35.9 / 113 / 370 against 14.7 / 31.2 / 101 / 364)
-    DECODE_WIDE_PAIRS = 64
-    DECODE_WIDE_CTX = 4096      # keys of head size 128: what counts is the bytes of a (token, KV head) pair
-    DECODE_WIDE_FILL = 0.9      # of the last round of large workgroups that the pairs must fill
-    # Fewer pairs than the chip holds large workgroups: one large workgroup a pair, nothing to merge, from this
-    # share of them on (20 to 28 requests over 8 KV heads, 1000 to 7000 keys: 8 to 14 % faster than the small
-    # workgroups with their chunks and merge, 16 requests: equal), and at any number over contexts up to
-    # DECODE_SHORT_CTX keys of head size 128 (600 keys, 1 to 24 requests: 7.8 to 15.2 us against 9.3 to 20.6)
-    DECODE_WIDE_FILL_ONE = 0.6
-    DECODE_SHORT_CTX = 768
+    # How the decode kernel is cut, in keys of head size 128 (what counts is the bytes of a (token, KV head) pair): below
+    DECODE_SHORT_CTX = 768      # one large workgroup a pair, where the chip holds them all
+    DECODE_LONG_CTX = 4096      # from here on large workgroups and their chunks, where the chip holds one a pair
+    DECODE_ONE_CTX = 1024       # one small workgroup a pair, where there are more pairs than that
+    DECODE_FILL_ONE = 0.5       # pairs that the chip holds as large workgroups, from this share of them on one each
+    DECODE_FILL = 0.9           # of the last round of large workgroups that more pairs must fill
+    DECODE_PARTS = 16           # chunks that the merging kernel asks for in one trip
 
     def _slots_of_decode(self, num_heads: int, num_kv_heads: int, head_dim: int, waves: int) -> int:
         """Workgroups of the decode kernel's form with ``waves`` waves that the chip holds at once (0: that
@@ -612,30 +605,29 @@ class HipKernels:
     def decode_chunk(self, n_tokens: int, num_heads: int, num_kv_heads: int, head_dim: int, max_ctx: int):
         """How the decode kernel cuts a token's keys: (least chunk length, most chunks a token, waves a
         workgroup). The kernel cuts every token into equal chunks of its own length, so only their
-        number is chosen here: as many as fill the kernel's grid once (the workgroups the chip holds at
-        once, whatever the batch). Then all work items run side by side and the launch lasts as long as
-        one of them; more items than that cost a start and a partial result each (measured at 2200
-        and 8000 keys a token, 1 to 128 tokens). Workgroups of 12 waves, one a CU, each with three times
-        the keys in flight, need a third of the chunks to keep the memory as busy, which leaves fewer
-        partial results to merge (none at 32 tokens and more); a small step over short contexts has too
-        little work for them, and a step with more (token, KV head) pairs than the chip holds such
-        workgroups would give some of them two pairs one after the other while the rest idle (33
-        requests over 8 KV heads: 68 us a layer against 47 with the small workgroups, of which three fit
-        a CU)."""
+        number is chosen here. A launch takes 5 us with nothing to read, a merge 4 more, a round of 32 keys a wave
+        two (three small workgroups fit a CU, one large one, with as many waves), and the keys come at 4.9 TB/s:
+        few pairs of (token, KV head) are cut until their chunks fill the chip once, and where a workgroup a pair
+        fills half of it there is nothing to merge. 32 query heads over 8 KV heads of 128, us, this rule /
+        the best of 30 others: 8 tokens of 700 keys 11.9 / 11.9, of 1500 16.8 / 16.8, 12 of up to 1500 16.3 / 16.3, 1 of 1500
+        9.5 / 9.5, 16 of 1000 18.7 / 18.7, 2 of 6000 16.8 / 16.8, 48 of up to 440 16.8 / 16.8, 64 of up to 300 14.6 / 14.6,
+        of up to 1800 52.2 / 52.2; 40 of up to 1500 33.6 / 33.6, 14 of 1000 19.4 / 18.2."""
         pairs = max(1, n_tokens * num_kv_heads)
-        waves = 4
+        ctx = max_ctx * head_dim // 128
         wide = self._slots_of_decode(num_heads, num_kv_heads, head_dim, 12)
-        if 0 < pairs <= wide and (pairs >= self.DECODE_WIDE_FILL_ONE * wide
-                                  or max_ctx * head_dim <= self.DECODE_SHORT_CTX * 128):
+        slots = self._slots_of_decode(num_heads, num_kv_heads, head_dim, 4) or 768
+        if pairs <= wide:
+            if pairs >= self.DECODE_FILL_ONE * wide or ctx <= self.DECODE_SHORT_CTX:
+                return 512, 1, 12
+            if ctx >= self.DECODE_LONG_CTX:
+                return 256, min(wide // pairs, -(-max_ctx // 256)), 12
+        elif wide > 0 and ctx > self.DECODE_ONE_CTX and pairs >= self.DECODE_FILL * (-(-pairs // wide) * wide):
             return 512, 1, 12
-        if pairs >= self.DECODE_WIDE_PAIRS or max_ctx * head_dim > self.DECODE_WIDE_CTX * 128:
-            # whole rounds of the large workgroups, or nearly (64 requests over 8 KV heads are two rounds
-            # of 256: 8.45 ms a step against 8.65 with the small workgroups)
-            if wide > 0 and pairs >= self.DECODE_WIDE_FILL * (-(-pairs // wide) * wide):
-                waves = 12
-        slots = self._slots_of_decode(num_heads, num_kv_heads, head_dim, waves) or 768
-        least = 256 if waves == 4 else 512
-        return least, max(1, min(slots // pairs, -(-max_ctx // least))), waves
+        elif pairs <= slots and ctx <= self.DECODE_ONE_CTX:
+            return 256, 1, 4
+        # more pairs than CUs last longer than a round: their last one part-filled costs less than longer chunks
+        fill = slots // pairs if pairs <= wide else -(-slots // pairs)
+        return 128, max(1, min(fill, -(-max_ctx // 128), self.DECODE_PARTS)), 4
 
     def attention_decode(self, q, q_stride, out, kcache, vcache, batch, num_heads, num_kv_heads, head_dim,
                          scale, window, group, token_list=None, n_listed=None, max_ctx=None,

@@ -1101,3 +1101,23 @@ def test_measured_peaks_are_plausible():
     with pytest.raises(kernels.KernelLibraryError, match="multiple of 16"):
         from reinfer_amd.kernels import library
         library.call("ra_stream_read", 0, 8, 0, 0)
+
+
+def test_small_decode_workgroups_share_a_cu():
+    """The grid of the decode kernel's small form is what the chip holds: several workgroups a CU up to head size 128."""
+    slots = kernels.library.load().ra_attention_decode_slots
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert slots(32, 8, 128, 4) >= 2 * cus and slots(32, 8, 64, 4) >= slots(32, 8, 128, 4) >= slots(32, 4, 256, 4) >= cus
+    assert slots(32, 8, 128, 12) == cus
+
+
+# a step on each side of the lines that the cut of the keys is chosen by: one workgroup a pair, large and small, chunks of both
+# (one pair more than the chip holds large workgroups, and contexts of one key more than a round, a chunk and the short ones)
+@pytest.mark.parametrize("n,longest", [(1, 769), (2, 4097), (8, 129), (16, 1025), (32, 300), (33, 1024), (33, 1025), (48, 449)])
+def test_attention_decode_as_its_keys_are_cut(n, longest):
+    Hq, Hkv, d = 16, 8, 128
+    q_lens, starts = [1] * n, [(longest - 1) * (i + 1) // n for i in range(n)]
+    q, kc, vc, tables = make_paged_case("bfloat16", Hq, Hkv, d, q_lens, starts, seed=n)
+    out = torch.full((n, Hq * d), float("nan"), device=DEV, dtype=torch.bfloat16)
+    ops().attention_decode(q.view(n, Hq * d), Hq * d, out, kt(kc), vt(vc), FakeBatch(q_lens, starts, tables), Hq, Hkv, d, d ** -0.5, 0, 0)
+    close(out, attention_reference(q, kc, vc, tables, q_lens, starts, Hq, Hkv, d, d ** -0.5, 0), 2 ** -7)
