@@ -31,18 +31,14 @@
 // crates/cuda/kernels/fmha_kernels.cu:96); this one is written here and reads
 // earlier context from the cache, so a prompt can be cut anywhere.
 #include <type_traits>
-#include "common.h"
-#include "reinfer_hip.h"
+#include "attention_prefill.h"
 
 #define FP_THREADS 512
 #define FP_WAVES 8
-#define FP_KT 64          // keys per round
-
-__device__ __forceinline__ float fp_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // how the heads of a group and the queries are spread over a wave's column tiles
 struct FpShape {
-  int nc;      // column tiles a wave holds (template parameter)
+  int nc;      // column tiles a wave holds (template parameter; of 256 elements the wide form's four waves hold two each)
   int hg;      // heads of one KV head per workgroup: 4, 2 or 1
   int runs;    // runs of 16 queries per workgroup
 };
@@ -55,26 +51,7 @@ static FpShape fp_shape(int Hq, int Hkv, int d) {
   return s;
 }
 
-// A listed tile may be one of several parts of a query tile, each with a range of keys (split.ranges, three
-// ints a listed tile: first key, one past the last, both multiples of the round; and the part's slot, or -1
-// for a tile that is whole): a part leaves its float sums (the outputs before the division, the running
-// maximum and the sum of each column) in its slot, and a second kernel adds a tile's parts up. A portion
-// of few queries deep in a long prompt is a handful of tiles with thousands of keys each, and a 2048-token
-// prompt is one tile a CU of which the last has 32 times the keys of the first: cut by keys, the heavy
-// tiles spread over the CUs that would idle.
-struct FpSplit {
-  const int* ranges;       // [listed tiles][3], or null: every tile is whole
-  float* part_o;           // [slots][workgroups a tile][256 columns][DMAX]
-  float* part_ml;          // [slots][workgroups a tile][256 columns][2]
-};
-
 // EXACT: the head size is DMAX itself, so every test against it is decided when the kernel is compiled
-// FLAGS & FP_MOD: the scores are changed before the softmax (RaScoreMod: a tanh cap, a per-head distance term); the scaled
-// and changed score then replaces the product in the registers, and scale_log2 is log2(e) alone
-// FLAGS & FP_KEEP: a window that keeps the first `keep` keys; the rounds that hold them and lie below the window's
-// first round are walked before it.
-// FLAGS & FP_CHUNK: the window is the query's own chunk of `window` keys, counted from position 0.
-enum { FP_MOD = 1, FP_KEEP = 2, FP_CHUNK = 4 };
 template <int DMAX, int NC, bool EXACT, int FLAGS>
 __global__ void __launch_bounds__(FP_THREADS)
 flash_prefill_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, int out_stride,
@@ -652,7 +629,10 @@ static int fp_launch(const void* q, int q_stride, void* out, int out_stride,
   } while (0)
   if (d <= 64) RA_FP(64, 2);
   else if (d <= 128) RA_FP(128, 2);
-  else RA_FP(256, 1);
+  else if (d < FPW_D) RA_FP_GO(256, 1, false);
+  else ra_prefill_wide(n_tiles * gy, (const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)kcache,
+                       (const bf16_t*)vcache, block_tables, max_blocks, tile_info, block_size, Hq, Hkv, sh.hg, scale_log2, window,
+                       aligned, keep, sp, scale, mod, ho, stream);
 #undef RA_FP_GO
 #undef RA_FP
 #undef RA_FP_ARGS

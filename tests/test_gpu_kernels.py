@@ -1069,6 +1069,12 @@ def test_attention_dispatch_mixed_batch():
     close(out, attention_reference(q, kc, vc, tables, q_lens, starts, Hq, Hkv, d, d ** -0.5, 0), 2 ** -7)
 
 
+@pytest.mark.parametrize("Hq,Hkv,d", [(4, 1, 256), (2, 2, 256), (6, 3, 144), (4, 2, 192), (9, 1, 240)])
+def test_attention_prefill_of_wide_heads(Hq, Hkv, d):
+    """Above 128 elements: a kernel of its own; four, two and one head a workgroup, head sizes that end inside a tile of 32."""
+    test_attention_prefill(Hq, Hkv, d)
+
+
 def test_far_key_among_hundreds_decode_and_prefill():
     """One key far back matches the query much better than all others: losing it
     (a wrong block, a dropped split, a wrong running maximum) changes the output."""
