@@ -14,6 +14,14 @@ enum { RA_F32 = 0, RA_BF16 = 1 };
 // XCDs of the chip: workgroups are dealt round them in the order of their numbers, each XCD has an L2 of its own
 #define RA_XCDS 8
 
+// Weights that a launch reads once are asked for past the caches' usual policy (non-temporal): on their way through they would put out
+// what is there and be put out themselves before the next step reads them. Measured where the weights in turn are more than the
+// last-level cache (256 MB) holds: 4 to 10 % less for the products of a decode step (8 rows of 24576 x 4096 35.0 us, so 32.5; of 4096 x
+// 12288 20.9, 18.5; of 1024 x 2048 6.0, 5.6). Where a whole model stays in that cache it is the other way round (1 row of 4096 x 1024
+// 3.9, 4.5): models that small have products below this many bytes, and those keep the usual policy.
+#define RA_STREAM_BYTES (8u << 20)
+#define RA_STREAM 2                // the load's cache policy bits: non-temporal
+
 typedef __bf16 bf16_t;
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));

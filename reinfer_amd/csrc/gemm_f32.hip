@@ -174,7 +174,7 @@ struct F32Stream {
   static constexpr int SUM_BYTES = 2 * MT * RA_WAVE * 16;
   static constexpr int lds(int waves) { return waves * (W_BYTES + A_BYTES + SUM_BYTES); }
 };
-template <int ROWS>
+template <int ROWS, bool STREAM>
 __global__ void __launch_bounds__(8 * RA_WAVE, 4)
 gemm_f32_stream_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
                        float* __restrict__ C, int M, int N, int K, int lda, int ldc, int block_k) {
@@ -212,7 +212,7 @@ gemm_f32_stream_kernel(const float* __restrict__ A, const float* __restrict__ W,
     for (int i = 0; i < LOADS; ++i) {
       const int k = k0 + l_step * F32_BK + wc * 4, n = l_n + i * LR + wr;
       const unsigned off = l_q < total && k < k1 && n < N ? (unsigned)(((size_t)n * K + k) * 4) : NOWHERE;
-      w[d][i] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, off, 0, 0));
+      w[d][i] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, off, 0, STREAM ? RA_STREAM : 0));
     }
   };
   auto load_a = [&](int d) {                   // and on to the next run
@@ -700,8 +700,13 @@ extern "C" int ra_gemm_f32(const float* A, const float* W, const float* bias, fl
       const int tiles = (n + 15) / 16, cus = ra_cu_count();
       const float *w = W + (size_t)n0 * K, *b = bias ? bias + n0 : nullptr;
 #define RA_GO(ROWS) \
-  gemm_f32_stream_kernel<ROWS><<<grid < tiles ? grid : tiles, kb.n * RA_WAVE, F32Stream<ROWS>::lds(kb.n), stream>>>( \
-      A, w, b, C + n0, M, n, K, lda, ldc, kb.k)
+  do {                                                                                                                               \
+    if (past) gemm_f32_stream_kernel<ROWS, true><<<grid < tiles ? grid : tiles, kb.n * RA_WAVE, F32Stream<ROWS>::lds(kb.n), stream>>>( \
+        A, w, b, C + n0, M, n, K, lda, ldc, kb.k);                                                                                   \
+    else gemm_f32_stream_kernel<ROWS, false><<<grid < tiles ? grid : tiles, kb.n * RA_WAVE, F32Stream<ROWS>::lds(kb.n), stream>>>(    \
+        A, w, b, C + n0, M, n, K, lda, ldc, kb.k);                                                                                   \
+  } while (0)
+      const bool past = (size_t)N * K * sizeof(float) >= RA_STREAM_BYTES;
       // as many workgroups as the registers hold, 16 waves a CU
       const int grid = 16 / kb.n * cus;
       if (M > 16) RA_GO(32);

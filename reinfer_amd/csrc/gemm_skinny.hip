@@ -361,7 +361,7 @@ struct SkinnySecond {
   float* C;
   int N, ldc;
 };
-template <int NT, int WAVES, int U, int DEPTH, int OCC, int MROWS, int EPI, typename TO, bool PAIR = false>
+template <int NT, int WAVES, int U, int DEPTH, int OCC, int MROWS, int EPI, typename TO, bool STREAM, bool PAIR = false>
 __global__ void __launch_bounds__(WAVES * RA_WAVE, OCC)
 gemm_skinny_deep_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
                         const bf16_t* __restrict__ bias, TO* __restrict__ C, int ldc, int M, int N, int K,
@@ -396,9 +396,14 @@ gemm_skinny_deep_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __r
   const int stride_n = (int)gridDim.x * 16 * NT;
   const int n_mine = (tiles - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;
   const int total = n_mine * n_steps_p;
-  // Workgroups start their walk over K at different runs and wrap round where many run side by side:
-  // in step, the rows read at one moment, a whole K apart, fall on few memory channels.
-  const int rot_own = (n_tiles > 512 || K > 8192) ? (int)((blockIdx.x * 7u) % (unsigned)n_steps) : 0;
+  // Workgroups start their walk over K at different runs and wrap round: in step, the rows read at one moment, a whole K apart, fall
+  // on few memory channels. Neighbours start at the same run, as eight of them, on the eight XCDs, are the nearest in time (1 row, K
+  // a multiple of 4096, 4096 x 4096 9.1 us, so 8.7, all from the same start 9.1, each from another than its neighbour 9.2; 5120 x
+  // 8192 20.9, 19.8; 4096 x 12288 20.0, 19.5; other K within 2 % in all forms).
+  auto rot_of = [&](unsigned b, int own_tiles) -> int {           // of workgroup b in a launch of these tiles alone
+    return (int)(b * (unsigned)n_steps / (unsigned)min(own_tiles, (int)gridDim.x));
+  };
+  const int rot_own = (int)blockIdx.x < n_tiles ? rot_of(blockIdx.x, n_tiles) : 0;
 
   // Both operands are read through buffer descriptors: a load whose offset lies past the descriptor's end
   // returns zeros and touches no memory, so rows past N or M, chunks past K, padding runs and runs past
@@ -477,7 +482,7 @@ gemm_skinny_deep_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __r
   do {                                                                                         \
     const bool two_ = PAIR && l_n0 >= past;                                                    \
     /* the second matrix's walk starts where a launch of its own would have it start */        \
-    const int rot = !two_ ? rot_own : K > 8192 ? (int)((unsigned)((l_n0 - past) / (16 * NT)) * 7u % (unsigned)n_steps) : 0; \
+    const int rot = two_ ? rot_of((unsigned)((l_n0 - past) / (16 * NT)), tiles - n_tiles) : rot_own; \
     const __amdgpu_buffer_rsrc_t rsrc_ = two_ ? w2_rsrc : w_rsrc;                              \
     const int first_ = two_ ? l_n0 - past : l_n0, N_ = two_ ? second.N : N;                    \
     int kk_ = K;                          /* a padding run, or past the end: nothing is read */ \
@@ -490,7 +495,7 @@ gemm_skinny_deep_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __r
       _Pragma("unroll") for (int i = 0; i < NI; ++i) {                                         \
         const int n_ = first_ + nt * 16 + i * RPI + lr;                                        \
         const unsigned off_ = (ok_ && n_ < N_) ? (unsigned)(((size_t)n_ * K + kk_) * 2) : NOWHERE; \
-        wr[d][nt][i] = __builtin_bit_cast(bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(rsrc_, off_, 0, 0)); \
+        wr[d][nt][i] = __builtin_bit_cast(bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(rsrc_, off_, 0, STREAM ? RA_STREAM : 0)); \
       }                                                                                        \
     _Pragma("unroll") for (int i = 0; i < MI; ++i) {                                           \
       const unsigned off_ = (ok_ && a_off[i] != NOWHERE) ? a_off[i] + (unsigned)(kk_ - lc * 8) * 2u : NOWHERE; \
@@ -619,9 +624,14 @@ static int skinny_cus() { return ra_cu_count(); }
 template <int NT, int WAVES, int U, int DEPTH, int OCC, int MROWS>
 static int launch_deep(const void* A, int lda, const void* W, const void* bias, void* C, int ldc, int out_dtype,
                        int epilogue, int M, int N, int K, const SkinnyNorm& nf, int grid, hipStream_t stream) {
-#define RA_GO(EPI, TO)                                                                              \
-  gemm_skinny_deep_kernel<NT, WAVES, U, DEPTH, OCC, MROWS, EPI, TO><<<grid, WAVES * RA_WAVE, 0, stream>>>(  \
-      (const bf16_t*)A, lda, (const bf16_t*)W, (const bf16_t*)bias, (TO*)C, ldc, M, N, K, nf)
+  const bool past = (size_t)N * K * sizeof(bf16_t) >= RA_STREAM_BYTES;
+#define RA_GO(EPI, TO)                                                                                                       \
+  do {                                                                                                                       \
+    if (past) gemm_skinny_deep_kernel<NT, WAVES, U, DEPTH, OCC, MROWS, EPI, TO, true><<<grid, WAVES * RA_WAVE, 0, stream>>>( \
+        (const bf16_t*)A, lda, (const bf16_t*)W, (const bf16_t*)bias, (TO*)C, ldc, M, N, K, nf);                             \
+    else gemm_skinny_deep_kernel<NT, WAVES, U, DEPTH, OCC, MROWS, EPI, TO, false><<<grid, WAVES * RA_WAVE, 0, stream>>>(     \
+        (const bf16_t*)A, lda, (const bf16_t*)W, (const bf16_t*)bias, (TO*)C, ldc, M, N, K, nf);                             \
+  } while (0)
   if (epilogue == EPI_SILU_PAIRS) {
     if (out_dtype == RA_BF16) RA_GO(EPI_SILU_PAIRS, bf16_t);
     else RA_GO(EPI_SILU_PAIRS, float);
@@ -661,12 +671,18 @@ static int launch_pair(const void* A, int lda, const void* W, void* C, int ldc, 
   const int tiles = (N + 15) / 16 + (second.N + 15) / 16, cus = skinny_cus(), grid = tiles < 2 * cus ? tiles : 2 * cus;
   const SkinnyNorm nf = {};
   const int runs128 = (K + 1023) / 1024, runs64 = (K + 511) / 512;
-  if (runs64 * 512 < runs128 * 1024)
-    gemm_skinny_deep_kernel<1, 8, 2, 2, 2, MROWS, EPI_PLAIN, bf16_t, true><<<grid, 8 * RA_WAVE, 0, stream>>>(
-        (const bf16_t*)A, lda, (const bf16_t*)W, nullptr, (bf16_t*)C, ldc, M, N, K, nf, second);
-  else
-    gemm_skinny_deep_kernel<1, 8, 4, 2, 2, MROWS, EPI_PLAIN, bf16_t, true><<<grid, 8 * RA_WAVE, 0, stream>>>(
-        (const bf16_t*)A, lda, (const bf16_t*)W, nullptr, (bf16_t*)C, ldc, M, N, K, nf, second);
+#define RA_PAIR(U, STREAM)                                                                                          \
+  gemm_skinny_deep_kernel<1, 8, U, 2, 2, MROWS, EPI_PLAIN, bf16_t, STREAM, true><<<grid, 8 * RA_WAVE, 0, stream>>>( \
+      (const bf16_t*)A, lda, (const bf16_t*)W, nullptr, (bf16_t*)C, ldc, M, N, K, nf, second)
+  const bool past = (size_t)N * K * sizeof(bf16_t) >= RA_STREAM_BYTES;
+  if (runs64 * 512 < runs128 * 1024) {
+    if (past) RA_PAIR(2, true);
+    else RA_PAIR(2, false);
+  } else {
+    if (past) RA_PAIR(4, true);
+    else RA_PAIR(4, false);
+  }
+#undef RA_PAIR
   RA_LAUNCH_CHECK("gemm_skinny_pair");
   return 0;
 }

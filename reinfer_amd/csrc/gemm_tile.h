@@ -15,6 +15,7 @@ struct RaTileEnd {
   const bf16_t* bias;            // [N], plain and added
   float alpha;                   // added: alpha times the product
   int half;                      // plain and gated: the result is bfloat16
+  bool keep;                     // the weights by the caches' usual policy
 };
 
 extern "C" int ra_gemm_tile_takes(int epilogue, int M, int N, int K);
@@ -23,4 +24,5 @@ RaTilePlan ra_tile_plan(int M, int N, int K, bool cut);
 int ra_tile_product(int epilogue, const RaTilePlan& plan, const void* A, int lda, const void* W, void* C, int ldc, int M, int N, int K,
                     RaTileEnd end, hipStream_t stream);
 // planes[z][m][n] = A[m, range z] . W[n, range z]^T
-int ra_tile_ranges(const RaTilePlan& plan, const void* A, int lda, const void* W, float* planes, int M, int N, int K, hipStream_t stream);
+int ra_tile_ranges(const RaTilePlan& plan, const void* A, int lda, const void* W, float* planes, int M, int N, int K, bool keep,
+                   hipStream_t stream);

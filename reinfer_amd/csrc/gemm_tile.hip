@@ -72,7 +72,7 @@ __device__ __forceinline__ int gt_key(int row) { return (row >> 1) & 7; }
 // BMT x TN tiles of 16 rows x 16 features, shared out over WM x WN waves. QUICK: results whose rows start at whole pieces, no bias and, with
 // the gate, in bfloat16, so that an end is a few stores; what is left takes any end, in four times the code (a launch runs each line of
 // its code for the first time, from memory: with one end for all, 19456 x 2560 with its gate took 30.5 us at 97 rows, so 28.8).
-template <int BMT, int TN, int WM, int WN, int EPI, bool QUICK>
+template <int BMT, int TN, int WM, int WN, int EPI, bool QUICK, bool STREAM>
 __global__ void __launch_bounds__(64 * WM * WN) gemm_tile_kernel(TileArgs g) {
   constexpr int NW = WM * WN, MT = BMT / WM, NT = TN / WN;
   static_assert(BMT % WM == 0 && TN % WN == 0);
@@ -171,7 +171,7 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_tile_kernel(TileArgs g) {
       const int rows = i * NW + wave;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           rsrc, (__attribute__((address_space(3))) void*)(2 * TN % NW == 0 || rows < 2 * TN ? to + (BM + rows * 8) * GT_BK : lds + STAGES * SLOT),
-          16, (int)(w_off[i < PB ? i : 0] | f_past[i & 1]), f_k, 0, 0);
+          16, (int)(w_off[i < PB ? i : 0] | f_past[i & 1]), f_k, 0, STREAM ? RA_STREAM : 0);
     } else {
       const int j = i - PB, rows = j * NW + wave;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
@@ -353,6 +353,8 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_tile_kernel(TileArgs g) {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");           // loads that are still on their way to LDS
 }
 
+// With one row of tiles the weights are read once: past the caches' usual policy (RA_STREAM_BYTES in common.h; 48 rows of 24576 x 4096
+// with its gate 37.1 us, so 34.8, of 6144 x 4096 12.7, 12.0, 97 rows 15.3, 14.3).
 template <int BMT, int TN, int WM, int WN, int EPI, bool QUICK = true>
 int tile_launch(TileArgs g, hipStream_t stream) {
   g.m_tiles = (g.M + 16 * BMT - 1) / (16 * BMT);
@@ -361,7 +363,11 @@ int tile_launch(TileArgs g, hipStream_t stream) {
   RA_CHECK(total < 1L << 27 && g.ranges <= 16, "gemm_tile: too many tiles");         // where 2^32 over 16 divides exactly
   g.m_part = g.m_tiles > 1 ? 0xFFFFFFFFu / (unsigned)g.m_tiles + 1u : 0u;
   g.z_part = g.ranges > 1 ? 0xFFFFFFFFu / (unsigned)g.ranges + 1u : 0u;
-  gemm_tile_kernel<BMT, TN, WM, WN, EPI, QUICK><<<(unsigned)(total < cus ? total : cus), 64 * WM * WN, 0, stream>>>(g);
+  const unsigned grid = (unsigned)(total < cus ? total : cus);
+  if (QUICK && g.m_tiles == 1 && !g.end.keep && (size_t)g.N * g.K * sizeof(bf16_t) >= RA_STREAM_BYTES)
+    gemm_tile_kernel<BMT, TN, WM, WN, EPI, QUICK, QUICK><<<grid, 64 * WM * WN, 0, stream>>>(g);
+  else
+    gemm_tile_kernel<BMT, TN, WM, WN, EPI, QUICK, false><<<grid, 64 * WM * WN, 0, stream>>>(g);
   RA_LAUNCH_CHECK("gemm_tile");
   return 0;
 }
@@ -510,10 +516,13 @@ int ra_tile_product(int epilogue, const RaTilePlan& plan, const void* A, int lda
 }
 
 // planes[z][m][n] = A[m, range z] . W[n, range z]^T
-int ra_tile_ranges(const RaTilePlan& plan, const void* A, int lda, const void* W, float* planes, int M, int N, int K, hipStream_t stream) {
+int ra_tile_ranges(const RaTilePlan& plan, const void* A, int lda, const void* W, float* planes, int M, int N, int K, bool keep,
+                   hipStream_t stream) {
   if (M > GT_SIDE && ra_prompt_shape(N, K)) {
     const RaPromptPlan p = ra_prompt_plan(M, N, K, plan.range_k);
     if (p.ranges == plan.ranges) return ra_prompt_product(p, 3, A, W, planes, M, N, K, lda, N, 1.f, stream);
   }
-  return ra_tile_product(GT_PART, plan, A, lda, W, planes, N, M, N, K, RaTileEnd{}, stream);
+  RaTileEnd end = {};
+  end.keep = keep;
+  return ra_tile_product(GT_PART, plan, A, lda, W, planes, N, M, N, K, end, stream);
 }

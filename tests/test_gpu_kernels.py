@@ -795,6 +795,35 @@ def test_accumulating_product_finishes_the_norm_that_follows(M, N, K):
     close(s2, want2, 2 ** -8)
 
 
+@pytest.mark.parametrize("N", [4080, 4096])           # the first ends 32 KB below the size from which weights are streamed
+@pytest.mark.parametrize("M", [1, 7, 16, 17, 48, 64])
+def test_products_below_and_above_the_stream_size(M, N):
+    """Loads of weights past the caches' usual policy are another instance of each kernel: the same sums, on both sides of the rule."""
+    K = 1024
+    torch.manual_seed(M + N)
+    x = torch.randn(M, K, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(N, K, device=DEV) / 32).to(torch.bfloat16)
+    want = x.double() @ w.double().T
+    out = torch.full((M, N), float("nan"), device=DEV)
+    ops().linear(x, w, out)
+    close(out, want, 2 ** -8)
+    half = torch.empty(M, N, device=DEV, dtype=torch.bfloat16)
+    ops().linear(x, w, half)
+    close(half, want, OUT_TOL["bfloat16"])
+    total = torch.ones(M, N, device=DEV)
+    ops().linear_skinny(x, w, total, accumulate=True)
+    close(total, want + 1, 2 ** -8)
+    gated = torch.empty(M, N // 2, device=DEV, dtype=torch.bfloat16)
+    ops().gated_linear(x, w, gated)
+    both = want.view(M, N // 16, 2, 8)
+    close(gated, (torch.nn.functional.silu(both[:, :, 0]) * both[:, :, 1]).reshape(M, N // 2), OUT_TOL["bfloat16"])
+    f = (torch.randn(N // 2, K, device=DEV) / 32)      # the same sizes in float
+    xf = torch.randn(M, K, device=DEV)
+    out = torch.empty(M, N // 2, device=DEV)
+    ops().linear(xf, f, out)
+    close(out, xf.double() @ f.double().T, 1e-5)
+
+
 @pytest.mark.parametrize("M,N,K", [(129, 520, 264), (700, 96, 1000), (2048, 1024, 4096), (3072, 80, 176)])
 def test_accumulating_product_of_many_rows_adds_in_the_library(M, N, K):
     """More rows than the weight-streaming kernels take: the library's product reads and writes the float
