@@ -80,7 +80,16 @@ __device__ __forceinline__ int fd_kept(int keep, int lo) {
 // tile on a place is the key's own number, and the kept tiles take the places right below it.
 // FLAGS & FD_HEAD: the window may be the query's own chunk (aligned), and the head's result has a sink and / or a gate
 // (RaHeadOut); the other forms keep their scalar registers.
-enum { FD_MOD = 1, FD_KEEP = 2, FD_HEAD = 4 };
+// FLAGS & FD_STREAM: keys and values are read past the caches' usual policy (the plain form of a whole head size only). Where a layer's
+// are 32 MB or more, all layers' are more than the last-level cache keeps from one step to the next: 48 tokens of 60 to 440 keys (32
+// query heads, 8 KV heads of 128) 16.8 us, so 15.3, 8 of 1500 17.2, 15.5, 32 of 3000 72, 63.5; where they stay in it the usual policy
+// is ahead (1 of 4000, 16 MB a layer in 8 layers: 11.5, with this 12.3). The caller says which.
+enum { FD_MOD = 1, FD_KEEP = 2, FD_HEAD = 4, FD_STREAM = 8 };
+template <bool STREAM, typename V>
+__device__ __forceinline__ V fd_load(const bf16_t* p) {
+  if constexpr (STREAM) return __builtin_nontemporal_load((const V*)p);
+  else return *(const V*)p;
+}
 template <int DMAX, bool EXACT, int FD_WAVES, int FLAGS>
 __global__ void __launch_bounds__(FD_WAVES * RA_WAVE, (DMAX <= 128 && FD_WAVES == 4) ? 3 : 1)
 flash_decode_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, int out_stride,
@@ -91,7 +100,7 @@ flash_decode_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __restri
                     float scale_log2, int window, int keep, int chunk_shift, int max_chunks, int n_tokens,
                     int t_base, float* __restrict__ part_o, float* __restrict__ part_ml, float scale, RaScoreMod mod,
                     int aligned, RaHeadOut ho) {
-  constexpr bool MOD = (FLAGS & FD_MOD) != 0, KEEP = (FLAGS & FD_KEEP) != 0, HEAD = (FLAGS & FD_HEAD) != 0;
+  constexpr bool MOD = (FLAGS & FD_MOD) != 0, KEEP = (FLAGS & FD_KEEP) != 0, HEAD = (FLAGS & FD_HEAD) != 0, STREAM = (FLAGS & FD_STREAM) != 0;
   constexpr int FD_THREADS = FD_WAVES * RA_WAVE;
   const int d = EXACT ? DMAX : d_arg;
   constexpr int NDT = DMAX / 32;       // 32-wide d tiles of the score product
@@ -182,12 +191,12 @@ flash_decode_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __restri
 #pragma unroll
         for (int dt = 0; dt < NDT; ++dt) {
           kreg[tt][dt] = (bf16x8_t){0, 0, 0, 0, 0, 0, 0, 0};
-          if (live[tt] && dt * 32 + g * 8 < d) kreg[tt][dt] = *(const bf16x8_t*)(kb[tt] + dt * 512);
+          if (live[tt] && dt * 32 + g * 8 < d) kreg[tt][dt] = fd_load<STREAM, bf16x8_t>(kb[tt] + dt * 512);
         }
 #pragma unroll
         for (int ot = 0; ot < NOT; ++ot) {
           vreg[tt][ot] = (bf16x4_t){0, 0, 0, 0};
-          if (live[tt] && ot * 16 < d) vreg[tt][ot] = *(const bf16x4_t*)(vb[tt] + ot * 256);
+          if (live[tt] && ot * 16 < d) vreg[tt][ot] = fd_load<STREAM, bf16x4_t>(vb[tt] + ot * 256);
         }
       }
       f32x4_t s[2];
@@ -437,10 +446,11 @@ static size_t fd_lds_limit(void) {
 template <int DM, bool EX, int WV>
 static hipError_t fd_allow_lds(size_t lds) {
   if (lds <= 64 * 1024) return hipSuccess;
-  const void* forms[8] = {(const void*)flash_decode_kernel<DM, EX, WV, 0>, (const void*)flash_decode_kernel<DM, EX, WV, 1>,
+  const void* forms[9] = {(const void*)flash_decode_kernel<DM, EX, WV, 0>, (const void*)flash_decode_kernel<DM, EX, WV, 1>,
                           (const void*)flash_decode_kernel<DM, EX, WV, 2>, (const void*)flash_decode_kernel<DM, EX, WV, 3>,
                           (const void*)flash_decode_kernel<DM, EX, WV, 4>, (const void*)flash_decode_kernel<DM, EX, WV, 5>,
-                          (const void*)flash_decode_kernel<DM, EX, WV, 6>, (const void*)flash_decode_kernel<DM, EX, WV, 7>};
+                          (const void*)flash_decode_kernel<DM, EX, WV, 6>, (const void*)flash_decode_kernel<DM, EX, WV, 7>,
+                          (const void*)flash_decode_kernel<DM, EX, WV, EX ? FD_STREAM : 0>};
   for (const void* f : forms) {
     const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
@@ -505,19 +515,19 @@ extern "C" int ra_attention_decode(const void* q, int q_stride, void* out, int o
                                    float* part_o, float* part_ml, hipStream_t stream) {
   return ra_attention_decode_mod(q, q_stride, out, out_stride, kcache, vcache, block_tables, max_blocks, token_list,
                                  seq_of_token, positions, n_tokens, block_size, Hq, Hkv, d, scale, window, 0, 0, chunk,
-                                 max_chunks, waves, part_o, part_ml, 0.f, nullptr, nullptr, nullptr, nullptr, 0, stream);
+                                 max_chunks, waves, part_o, part_ml, 0.f, nullptr, nullptr, nullptr, nullptr, 0, 0, stream);
 }
 
 // The same with the scores changed before the softmax: softcap > 0 caps them by a tanh, r1 / r2 (one float a query
 // head each; both or neither) take r1 ln(1 + r2 (position - key)) off. aligned: the window is the query's chunk; sink
-// and gate as in RaHeadOut.
+// and gate as in RaHeadOut. past: the keys and values are too many to stay in the caches (a hint: FD_STREAM).
 extern "C" int ra_attention_decode_mod(const void* q, int q_stride, void* out, int out_stride,
                                        const void* kcache, const void* vcache, const int* block_tables,
                                        int max_blocks, const int* token_list, const int* seq_of_token,
                                        const int* positions, int n_tokens, int block_size, int Hq, int Hkv,
                                        int d, float scale, int window, int aligned, int keep, int chunk, int max_chunks,
                                        int waves, float* part_o, float* part_ml, float softcap, const float* r1,
-                                       const float* r2, const float* sink, const void* gate, int gate_stride,
+                                       const float* r2, const float* sink, const void* gate, int gate_stride, int past,
                                        hipStream_t stream) {
   RA_CHECK((r1 == nullptr) == (r2 == nullptr) && softcap >= 0.f,
            "attention_decode: the distance term takes both per-head vectors, the cap is not negative");
@@ -571,7 +581,10 @@ extern "C" int ra_attention_decode_mod(const void* q, int q_stride, void* out, i
       RA_FD_FORM(DM, EX, WV, 5)                                                                       \
       RA_FD_FORM(DM, EX, WV, 6)                                                                       \
       RA_FD_FORM(DM, EX, WV, 7)                                                                       \
-      default: flash_decode_kernel<DM, EX, WV, 0><<<grid, WV * RA_WAVE, lds, stream>>>(RA_FD_ARGS);   \
+      default:                                                                                        \
+        if (EX && past)                                                                               \
+          flash_decode_kernel<DM, EX, WV, EX ? FD_STREAM : 0><<<grid, WV * RA_WAVE, lds, stream>>>(RA_FD_ARGS); \
+        else flash_decode_kernel<DM, EX, WV, 0><<<grid, WV * RA_WAVE, lds, stream>>>(RA_FD_ARGS);     \
     }                                                                                                 \
   } while (0)
 #define RA_FD(DM)                                                                                     \

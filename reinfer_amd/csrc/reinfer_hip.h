@@ -174,7 +174,7 @@ int ra_attention_decode_mod(const void* q, int q_stride, void* out, int out_stri
                             int n_tokens, int block_size, int Hq, int Hkv, int d, float scale, int window,
                             int aligned, int keep, int chunk, int max_chunks, int waves, float* part_o, float* part_ml,
                             float softcap, const float* r1, const float* r2, const float* sink, const void* gate,
-                            int gate_stride, hipStream_t stream);
+                            int gate_stride, int past, hipStream_t stream);
 int ra_attention_prefill_supports(int Hq, int Hkv, int d, int block_size);
 int ra_attention_prefill_tile(int Hq, int Hkv, int d);
 int ra_attention_prefill_columns(int Hq, int Hkv, int d);

@@ -85,7 +85,7 @@ _SIGNATURES = {
     "ra_head_norm_gate": [P, P, I, P, I, I, I, F, I, I, I, P, P],
     "ra_normed_mean": [P, P, I, I, F, I, I, P, P, F, P],
     "ra_attention_plain_mod": [P, I, P, I, P, P, I, P, I, P, P, P, I, P, I, I, I, I, I, F, I, I, I, F, P, P, P, P, I, P],
-    "ra_attention_decode_mod": [P, I, P, I, P, P, P, I, P, P, P, I, I, I, I, I, F, I, I, I, I, I, I, P, P, F, P, P, P, P, I, P],
+    "ra_attention_decode_mod": [P, I, P, I, P, P, P, I, P, P, P, I, I, I, I, I, F, I, I, I, I, I, I, P, P, F, P, P, P, P, I, I, P],
     "ra_attention_prefill_mod": [P, I, P, I, P, P, P, I, P, I, I, I, I, I, F, I, I, I, F, P, P, P, P, I, P],
     "ra_attention_prefill_split_mod": [P, I, P, I, P, P, P, I, P, I, P, P, I, P, P, I, I, I, I, F, I, I, I, F, P, P, P, P, I, P],
     "ra_act_mul_bounded": [P, P, I, I, I, I, I, F, P],

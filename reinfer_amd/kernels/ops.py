@@ -591,6 +591,7 @@ class HipKernels:
     DECODE_FILL_ONE = 0.5       # pairs that the chip holds as large workgroups, from this share of them on one each
     DECODE_FILL = 0.9           # of the last round of large workgroups that more pairs must fill
     DECODE_PARTS = 16           # chunks that the merging kernel asks for in one trip
+    DECODE_PAST_CACHES = 32 << 20      # bytes of keys and values of the longest contexts, from which on the caches do not keep them
 
     def _slots_of_decode(self, num_heads: int, num_kv_heads: int, head_dim: int, waves: int) -> int:
         """Workgroups of the decode kernel's form with ``waves`` waves that the chip holds at once (0: that
@@ -658,6 +659,8 @@ class HipKernels:
             G = num_heads // num_kv_heads
             part_o = torch.empty((pairs, max_chunks, G, head_dim), dtype=torch.float32, device=q.device)
             part_ml = torch.empty((pairs, max_chunks, G, 2), dtype=torch.float32, device=q.device)
+        # keys and values of a layer that all layers' together do not stay in the caches
+        past = 4 * n * max_ctx * num_kv_heads * head_dim >= self.DECODE_PAST_CACHES
         # every request of the step brings one token: token t is request t, and the kernel need not look it up
         one_each = token_list is None and batch.num_tokens == batch.num_seqs
         library.call("ra_attention_decode_mod", q.data_ptr(), q_stride, out.data_ptr(), out.stride(0),
@@ -665,7 +668,7 @@ class HipKernels:
                      _ptr(token_list), None if one_each else batch.seq_of_token.data_ptr(), batch.positions.data_ptr(), n,
                      kcache.shape[2] * 16, num_heads, num_kv_heads, head_dim, float(scale), int(window), int(aligned),
                      int(keep), int(chunk), int(max_chunks), int(waves), _ptr(part_o), _ptr(part_ml), mod[0], mod[1], mod[2],
-                     *head_out, _stream())
+                     *head_out, int(past), _stream())
 
     def attention_prefill(self, q, q_stride, out, kcache, vcache, batch, num_heads, num_kv_heads, head_dim,
                           scale, window, group, tiles, n_tiles, ranges=None, merge=None, n_merge: int = 0,

@@ -1138,6 +1138,22 @@ def test_measured_peaks_are_plausible():
         library.call("ra_stream_read", 0, 8, 0, 0)
 
 
+@pytest.mark.parametrize("d,keys,n", [(128, 700, 3), (128, 2100, 2), (64, 333, 5), (256, 40, 9), (96, 700, 3)])
+def test_attention_decode_past_the_caches_reads_the_same(monkeypatch, d, keys, n):
+    """Keys and values by the other policy are another instance of the kernel (but for sizes that it is not made for): the same bits."""
+    q, kc, vc, tables = make_paged_case("bfloat16", 8, 2, d, [1] * n, [keys - 1 - 7 * i % keys for i in range(n)], seed=d)
+    batch = FakeBatch([1] * n, [keys - 1 - 7 * i % keys for i in range(n)], tables)
+    got = []
+    for least in (1 << 60, 0):
+        monkeypatch.setattr(ops(), "DECODE_PAST_CACHES", least)
+        for waves, chunk in ((4, 128), (12, 512)):
+            out = torch.full((n, 8 * d), float("nan"), device=DEV, dtype=torch.bfloat16)
+            ops().attention_decode(q.view(n, 8 * d), 8 * d, out, kt(kc), vt(vc), batch, 8, 2, d, d ** -0.5, 0, 0, chunk=chunk, waves=waves)
+            got.append(out)
+    assert torch.equal(got[0], got[2]) and torch.equal(got[1], got[3])
+    close(got[0], attention_reference(q, kc, vc, tables, [1] * n, [keys - 1 - 7 * i % keys for i in range(n)], 8, 2, d, d ** -0.5, 0), 2 ** -7)
+
+
 def test_small_decode_workgroups_share_a_cu():
     """The grid of the decode kernel's small form is what the chip holds: several workgroups a CU up to head size 128."""
     slots = kernels.library.load().ra_attention_decode_slots
