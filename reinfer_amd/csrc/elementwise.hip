@@ -30,6 +30,23 @@ int ra_cu_count(void) {
 }
 extern "C" int ra_abi_version(void) { return RA_ABI_VERSION; }
 
+typedef float f32x4_raw __attribute__((ext_vector_type(4)));
+
+template <typename T> struct Vec4;
+template <> struct Vec4<float> {
+  static __device__ __forceinline__ f32x4_raw load(const float* p) { return *(const f32x4_raw*)p; }
+  static __device__ __forceinline__ void store(float* p, f32x4_raw v) { *(f32x4_raw*)p = v; }
+};
+template <> struct Vec4<bf16_t> {
+  static __device__ __forceinline__ f32x4_raw load(const bf16_t* p) {
+    const bf16x4_t v = *(const bf16x4_t*)p;
+    return (f32x4_raw){(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
+  }
+  static __device__ __forceinline__ void store(bf16_t* p, f32x4_raw v) {
+    *(bf16x4_t*)p = (bf16x4_t){(bf16_t)v[0], (bf16_t)v[1], (bf16_t)v[2], (bf16_t)v[3]};
+  }
+};
+
 // ---------------------------------------------------------------------------
 // embedding rows into the float residual stream: out[t, :] = table[ids[t], :]
 // (reference: gather_row, crates/cuda/kernels/dense_kernels.cu:329-336)
@@ -43,15 +60,43 @@ __global__ void embed_kernel(const T* __restrict__ table, const int* __restrict_
   for (int i = threadIdx.x; i < h; i += blockDim.x) o[i] = to_f32(row[i]) * scale;
 }
 
+// The same for rows of whole chunks of 4 that fit the workgroup's registers: a row is asked for in one trip to memory instead of one an
+// element of a thread (rows of 4096, launches back to back: 1 row 3.3 us, so 2.3; 1733 rows 15.7, 10.6; 8000 57.9, 32.9).
+#define EMBED_CH 4      // chunks of 4 elements a thread keeps
+template <typename T>
+__global__ void embed_reg_kernel(const T* __restrict__ table, const int* __restrict__ ids,
+                                 float* __restrict__ out, int h, float scale) {
+  const int t = blockIdx.x;
+  const T* row = table + (size_t)ids[t] * h;
+  float* o = out + (size_t)t * h;
+  f32x4_raw v[EMBED_CH];
+#pragma unroll
+  for (int j = 0; j < EMBED_CH; ++j) {
+    const int i = (threadIdx.x + j * blockDim.x) * 4;
+    if (i < h) v[j] = Vec4<T>::load(row + i);
+  }
+#pragma unroll
+  for (int j = 0; j < EMBED_CH; ++j) {
+    const int i = (threadIdx.x + j * blockDim.x) * 4;
+    if (i < h) Vec4<float>::store(o + i, v[j] * scale);
+  }
+}
+
 extern "C" int ra_embed(const void* table, int table_dtype, const int* ids, float* out, int n_tokens,
                         int hidden, float scale, hipStream_t stream) {
   RA_CHECK(n_tokens > 0 && hidden > 0, "embed: empty input (%d tokens, width %d)", n_tokens, hidden);
-  if (table_dtype == RA_F32)
-    embed_kernel<float><<<n_tokens, 256, 0, stream>>>((const float*)table, ids, out, hidden, scale);
-  else if (table_dtype == RA_BF16)
-    embed_kernel<bf16_t><<<n_tokens, 256, 0, stream>>>((const bf16_t*)table, ids, out, hidden, scale);
-  else
-    return ra_fail("embed: unknown dtype tag %d", table_dtype);
+  const bool in_regs = hidden % 4 == 0 && hidden <= 1024 * 4 * EMBED_CH && ((uintptr_t)table % 16) == 0 && ((uintptr_t)out % 16) == 0;
+  int threads = 256;
+  while (in_regs && threads * 4 * EMBED_CH < hidden) threads *= 2;
+#define RA_GO(T)                                                                                        \
+  do {                                                                                                  \
+    if (in_regs) embed_reg_kernel<T><<<n_tokens, threads, 0, stream>>>((const T*)table, ids, out, hidden, scale); \
+    else embed_kernel<T><<<n_tokens, threads, 0, stream>>>((const T*)table, ids, out, hidden, scale);   \
+  } while (0)
+  if (table_dtype == RA_F32) RA_GO(float);
+  else if (table_dtype == RA_BF16) RA_GO(bf16_t);
+  else return ra_fail("embed: unknown dtype tag %d", table_dtype);
+#undef RA_GO
   RA_LAUNCH_CHECK("embed");
   return 0;
 }
@@ -95,23 +140,6 @@ __global__ void add_rmsnorm_kernel(float* __restrict__ resid, const TA* __restri
 // most threads * 16): one read of the row, the sum in registers, one write. A
 // decode step runs this on a handful of rows, so its time is the chain of memory
 // round trips, not bandwidth; the plain kernel above reads the row a second time.
-typedef float f32x4_raw __attribute__((ext_vector_type(4)));
-
-template <typename T> struct Vec4;
-template <> struct Vec4<float> {
-  static __device__ __forceinline__ f32x4_raw load(const float* p) { return *(const f32x4_raw*)p; }
-  static __device__ __forceinline__ void store(float* p, f32x4_raw v) { *(f32x4_raw*)p = v; }
-};
-template <> struct Vec4<bf16_t> {
-  static __device__ __forceinline__ f32x4_raw load(const bf16_t* p) {
-    const bf16x4_t v = *(const bf16x4_t*)p;
-    return (f32x4_raw){(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
-  }
-  static __device__ __forceinline__ void store(bf16_t* p, f32x4_raw v) {
-    *(bf16x4_t*)p = (bf16x4_t){(bf16_t)v[0], (bf16_t)v[1], (bf16_t)v[2], (bf16_t)v[3]};
-  }
-};
-
 #define NORM_CH 4       // chunks of 4 elements a thread keeps
 
 template <typename TA, typename TW>

@@ -77,9 +77,17 @@ __global__ void sample_stage1(const float* __restrict__ logits, int vocab, int r
   Best b;
   b.val = -INFINITY;
   b.idx = -1;
-  const int end = min(vocab, (slice + 1) * SAMPLE_SLICE);
-  for (int v = slice * SAMPLE_SLICE + threadIdx.x; v < end; v += SAMPLE_THREADS) {
-    float x = lg[v];
+  // a thread's logits are asked for in one trip to memory (one after the other, both stages: 1 row of
+  // 151936 6.8 us, so 5.9; 48 rows 14.1, 11.4)
+  constexpr int EACH = SAMPLE_SLICE / SAMPLE_THREADS;
+  const int first = slice * SAMPLE_SLICE + threadIdx.x;
+  float held[EACH];
+#pragma unroll
+  for (int j = 0; j < EACH; ++j) held[j] = first + j * SAMPLE_THREADS < vocab ? lg[first + j * SAMPLE_THREADS] : INFINITY;
+#pragma unroll
+  for (int j = 0; j < EACH; ++j) {
+    const int v = first + j * SAMPLE_THREADS;
+    float x = held[j];
     if (!isfinite(x)) continue;
     if (!sample_value(x, v, T, base)) continue;
     Best c;

@@ -74,6 +74,17 @@ def test_embed(dtype):
     assert torch.equal(out, table[ids.long()].float())
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("h", [4, 1020, 4096, 4098, 16380, 16384, 16388])
+def test_embed_widths(dtype, h):
+    """Rows kept in registers up to 16384 elements in chunks of 4, any others element by element: the same numbers."""
+    table = torch.randn(9, h, device=DEV).to(DT[dtype])
+    ids = torch.tensor([8, 0, 3], dtype=torch.int32, device=DEV)
+    out = torch.full((3, h), float("nan"), device=DEV)
+    ops().embed(table, ids, out, 1.75)
+    assert torch.equal(out, table[ids.long()].float() * 1.75)
+
+
 @pytest.mark.parametrize("dtype,wdtype", [("float32", "float32"), ("bfloat16", "bfloat16"), ("bfloat16", "float32")])
 @pytest.mark.parametrize("h", [100, 98, 4096, 4104, 20000])
 def test_add_rmsnorm(dtype, wdtype, h):
