@@ -23,6 +23,7 @@ int ra_prompt_product(const RaPromptPlan& plan, int epilogue, const void* A, con
 // the first pair, the expert's first tile, the expert's tiles. slots: pair (token * top + choice) by place in the sorted run.
 struct RaExpertsPlan {
   int rows, up_cols, down_cols;  // of a tile: sorted pairs, and weight rows of the up (and gate) and the down product
+  int past;                      // the weights are read once, past the caches' usual policy
 };
 // false: not a shape of this kernel (widths in steps of 64, operands within reach of a descriptor)
 bool ra_prompt_experts_plan(int pairs, int experts, int ff, int width, int gated, long tokens, long ldx, long ld_down,
@@ -30,4 +31,4 @@ bool ra_prompt_experts_plan(int pairs, int experts, int ff, int width, int gated
 // kind 0: relu(a . w^T)^2, 1: silu(gate) * up of an expert's gate rows and its up rows behind them, both of tokens' rows and times
 // the pair's weight, in bfloat16; 2: a . w^T of pairs' rows in float, an expert's K columns of w's rows side by side
 int ra_prompt_experts(int rows, int cols, int kind, const void* a, long tokens, int lda, const void* w, int ldw, void* out, int N,
-                      int K, const int* plan, const int* slots, const float* weights, int top, long most, hipStream_t stream);
+                      int K, const int* plan, const int* slots, const float* weights, int top, long most, int past, hipStream_t stream);

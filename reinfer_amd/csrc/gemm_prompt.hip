@@ -120,7 +120,8 @@ struct GpOps {
   }
 };
 
-template <int TM, int TN, int KIND>
+// STREAM: the weights past the caches' usual policy (experts of a tile each; RA_STREAM_BYTES in common.h)
+template <int TM, int TN, int KIND, bool STREAM = false>
 __global__ void __launch_bounds__(256, 1) gemm_prompt_kernel(PromptArgs g) {
   constexpr bool MOE = KIND >= GP_MOE_RELU2;
   constexpr int EPI = gp_form(KIND);
@@ -183,7 +184,7 @@ __global__ void __launch_bounds__(256, 1) gemm_prompt_kernel(PromptArgs g) {
   };
   auto fetch_w = [&](int i, int slot, __amdgpu_buffer_rsrc_t rs, int k) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(
-        rs, (__attribute__((address_space(3))) void*)(lw + slot + i * 8 * GP_BK), 16, (int)w_off[i], k, 0, 0);
+        rs, (__attribute__((address_space(3))) void*)(lw + slot + i * 8 * GP_BK), 16, (int)w_off[i], k, 0, STREAM ? RA_STREAM : 0);
   };
   // range by range, in a range bands of `band` row tiles, inside a band column by column
   auto place = [&](int at, int& m0, int& n0, int& z) {
@@ -420,14 +421,14 @@ int prompt_launch(PromptArgs g, hipStream_t stream) {
   return 0;
 }
 
-template <int TM, int TN>
+template <int TM, int TN, bool STREAM>
 int prompt_experts(PromptArgs g, int kind, long most, hipStream_t stream) {
   const int rows = kind == GP_MOE_GATED ? 2 * g.N : g.N;        // weight rows of an expert
   g.n_tiles = (rows + 32 * TN - 1) / (32 * TN);
   const unsigned blocks = (unsigned)((most * g.n_tiles + RA_XCDS - 1) / RA_XCDS * RA_XCDS);
-  if (kind == GP_MOE_RELU2) gemm_prompt_kernel<TM, TN, GP_MOE_RELU2><<<blocks, 256, 0, stream>>>(g);
-  else if (kind == GP_MOE_GATED) gemm_prompt_kernel<TM, TN, GP_MOE_GATED><<<blocks, 256, 0, stream>>>(g);
-  else gemm_prompt_kernel<TM, TN, GP_MOE_DOWN><<<blocks, 256, 0, stream>>>(g);
+  if (kind == GP_MOE_RELU2) gemm_prompt_kernel<TM, TN, GP_MOE_RELU2, STREAM><<<blocks, 256, 0, stream>>>(g);
+  else if (kind == GP_MOE_GATED) gemm_prompt_kernel<TM, TN, GP_MOE_GATED, STREAM><<<blocks, 256, 0, stream>>>(g);
+  else gemm_prompt_kernel<TM, TN, GP_MOE_DOWN, STREAM><<<blocks, 256, 0, stream>>>(g);
   RA_LAUNCH_CHECK("gemm_prompt (experts)");
   return 0;
 }
@@ -515,25 +516,31 @@ bool ra_prompt_experts_plan(int pairs, int experts, int ff, int width, int gated
     const float us = fminf(u[0], u[1]) + fminf(d[0], d[1]);
     if (us < best) {
       best = us;
-      *plan = {rows, u[0] < u[1] ? 128 : 256, d[0] < d[1] ? 128 : 256};
+      // An expert of one tile reads its weights once: they are asked for past the caches' usual policy. 16 experts of 1536 x 4096, four
+      // a token, with their gate, 300 tokens 157 us, so 142, 600 185, 167; with two tiles an expert, 1000 tokens, the other way
+      // round, 268 and 285. 128 experts of 768 x 2048, eight a token: 1000 tokens 333, 307, 3000 488, 449; 6000, two tiles, 858 and 891.
+      const bool once = tiles <= experts && (size_t)experts * ff * width * sizeof(bf16_t) >= RA_STREAM_BYTES;
+      *plan = {rows, u[0] < u[1] ? 128 : 256, d[0] < d[1] ? 128 : 256, once};
     }
   }
   return true;
 }
 
 int ra_prompt_experts(int rows, int cols, int kind, const void* a, long tokens, int lda, const void* w, int ldw, void* out, int N,
-                      int K, const int* plan, const int* slots, const float* weights, int top, long most, hipStream_t stream) {
+                      int K, const int* plan, const int* slots, const float* weights, int top, long most, int past, hipStream_t stream) {
   PromptArgs g = {(const bf16_t*)a, (const bf16_t*)w, out, (int)tokens, N, K, lda, ldw, N, 1.f, 0, 0, 1, 1, K / GP_BK,
                   plan, slots, weights, top};
   const int k = GP_MOE_RELU2 + kind;
+#define RA_EXPERTS(TM, TN) return past ? prompt_experts<TM, TN, true>(g, k, most, stream) : prompt_experts<TM, TN, false>(g, k, most, stream);
   switch (rows * 1000 + cols) {
-    case 256256: return prompt_experts<8, 8>(g, k, most, stream);
-    case 192256: return prompt_experts<6, 8>(g, k, most, stream);
-    case 128256: return prompt_experts<4, 8>(g, k, most, stream);
-    case 256128: return prompt_experts<8, 4>(g, k, most, stream);
-    case 192128: return prompt_experts<6, 4>(g, k, most, stream);
-    case 128128: return prompt_experts<4, 4>(g, k, most, stream);
+    case 256256: RA_EXPERTS(8, 8)
+    case 192256: RA_EXPERTS(6, 8)
+    case 128256: RA_EXPERTS(4, 8)
+    case 256128: RA_EXPERTS(8, 4)
+    case 192128: RA_EXPERTS(6, 4)
+    case 128128: RA_EXPERTS(4, 4)
   }
+#undef RA_EXPERTS
   return ra_fail("gemm_prompt: no tiles of %d x %d for experts", rows, cols);
 }
 

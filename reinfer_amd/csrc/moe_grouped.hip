@@ -341,10 +341,10 @@ extern "C" int ra_moe_grouped(const void* x, int ldx, const void* w_up, const vo
   const long most = most_tiles(pairs, experts);
   if (tiled) {
     if (int rc = ra_prompt_experts(tile.rows, tile.up_cols, gated ? 1 : 0, x, n_tokens, ldx, w_up, width, s + at.act, ff, width, plan,
-                                   slots, weights, top, most, stream))
+                                   slots, weights, top, most, tile.past, stream))
       return rc;
     if (int rc = ra_prompt_experts(tile.rows, tile.down_cols, 2, s + at.act, pairs, ff, w_down, ld_down, s + at.rows, width, ff, plan,
-                                   slots, weights, top, most, stream))
+                                   slots, weights, top, most, tile.past, stream))
       return rc;
   } else {
   // 256 weight rows a tile where that still leaves every CU two workgroups: half the reads of the slots' rows (gate and up

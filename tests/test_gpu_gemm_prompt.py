@@ -235,3 +235,12 @@ def test_who_takes_a_product_of_many_rows(epilogue, M, N, K, own, monkeypatch):
                 assert ("ra_silu_mul_rounded" in calls) != own
         return
     assert ("ra_gemm_prompt" in calls) == own
+
+
+# 16 MB of experts: one tile an expert by the mean, where their weights are read past the caches, and two; with all tokens at one
+# expert ("one") more than the mean says
+@pytest.mark.parametrize("T,E,top,ff,width", [(300, 16, 4, 512, 1024), (1100, 16, 4, 512, 1024)])
+@pytest.mark.parametrize("gated_kind", [False, True])
+@pytest.mark.parametrize("kind", ["spread", "one"])
+def test_experts_of_one_tile_each(T, E, top, ff, width, gated_kind, kind):
+    grouped.test_experts_over_sorted_tokens(T, E, top, ff, width, gated_kind, kind)
