@@ -114,11 +114,10 @@ int ra_gemm_skinny_normed(const void* A, const void* W, const void* bias, void* 
                           int in_parts, float in_eps, int in_width, const void* out_w, int out_w_dtype,
                           void* out_x, int out_ldx, float* out_ss, hipStream_t stream);
 
-// bfloat16, up to 64 rows: the same product and epilogues with the activations shared by a
-// workgroup's waves; ra_gemm_wide_preferred says where it is the faster of the two (17 rows and
-// more, not the smallest products). Small N cuts K into ranges whose float partial results need
-// `ra_gemm_wide_scratch(...)` floats of scratch (0: none needed). A product that is cut so may have up to
-// 128 rows (ra_gemm_wide_preferred says which are worth it: adding into the stream over a long K).
+// bfloat16, up to 128 rows (gated and cut products; plain and added whole ones up to 64): the same product and epilogues with the
+// activations shared by a workgroup's waves; ra_gemm_wide_preferred says where it is the faster of the two (17 rows and more, not the
+// smallest products). Small N cuts K into up to 16 ranges whose float partial results need `ra_gemm_wide_scratch(...)` floats of
+// scratch (0: none needed).
 int ra_gemm_wide_ranges(int M, int N, int K);          // K ranges of ra_gemm_wide_partial's result
 int ra_gemm_wide_partial(const void* A, const void* W, float* P, long p_floats, int M, int N, int K, int lda,
                          hipStream_t stream);         // P[range][m][n] float, for a consumer that adds the ranges
