@@ -5,7 +5,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
-#define RA_ABI_VERSION 31
+#define RA_ABI_VERSION 32
 
 #ifdef __cplusplus
 extern "C" {

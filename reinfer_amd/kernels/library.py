@@ -15,7 +15,7 @@ import torch  # noqa: F401  (loads the HIP runtime the library links against)
 
 from ..csrc import build as _build
 
-ABI_VERSION = 31
+ABI_VERSION = 32
 
 
 class KernelLibraryError(RuntimeError):
