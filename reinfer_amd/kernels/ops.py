@@ -617,18 +617,38 @@ class HipKernels:
         ctx = max_ctx * head_dim // 128
         wide = self._slots_of_decode(num_heads, num_kv_heads, head_dim, 12)
         slots = self._slots_of_decode(num_heads, num_kv_heads, head_dim, 4) or 768
+        if wide == 0:
+            return self._small_decode_chunk(pairs, head_dim, max_ctx, slots)
         if pairs <= wide:
             if pairs >= self.DECODE_FILL_ONE * wide or ctx <= self.DECODE_SHORT_CTX:
                 return 512, 1, 12
             if ctx >= self.DECODE_LONG_CTX:
                 return 256, min(wide // pairs, -(-max_ctx // 256)), 12
-        elif wide > 0 and ctx > self.DECODE_ONE_CTX and pairs >= self.DECODE_FILL * (-(-pairs // wide) * wide):
+        elif ctx > self.DECODE_ONE_CTX and pairs >= self.DECODE_FILL * (-(-pairs // wide) * wide):
             return 512, 1, 12
         elif pairs <= slots and ctx <= self.DECODE_ONE_CTX:
             return 256, 1, 4
         # more pairs than CUs last longer than a round: their last one part-filled costs less than longer chunks
         fill = slots // pairs if pairs <= wide else -(-slots // pairs)
         return 128, max(1, min(fill, -(-max_ctx // 128), self.DECODE_PARTS)), 4
+
+    def _small_decode_chunk(self, pairs: int, head_dim: int, max_ctx: int, slots: int):
+        """The same where the large form's sums do not fit its LDS (more than 10 query heads a KV head at head size 128,
+        more than 5 at 256): small workgroups at every size. A pair is one chunk over a few rounds of keys, and over
+        DECODE_ONE_CTX where the pairs are half of the CUs and more; else it is cut as finely as fills the chip. 1 and 8
+        tokens, us, in one chunk / in 4, 8, 16, 32, 64: 64 heads over 4 KV heads of 128, 300 keys 9.6 / 11.1 and 10.7 / 12.3,
+        1000 keys 19.3 / 12.5 / 11.1 and 19.9 / 14.8 / 14.3, 16000 keys (from 16 chunks) 27.4 / 24.9 / 27.2 and 51 / 56 / -;
+        16 over 1 of 256, 1000 keys (from 4) 18.5 / 16.0 and 20.1 / 17.5, 16000 keys (from 16) 36.6 / 30.1 / 30.0 and
+        48 / 43 / -."""
+        ctx = max_ctx * head_dim // 128
+        cus = self._slots_of_decode(1, 1, 128, 12)           # the large form is one workgroup a CU
+        if ctx <= self.DECODE_ONE_CTX // 2 or (ctx <= self.DECODE_ONE_CTX and pairs * 2 >= cus):
+            return 256, 1, 4
+        # where a pair has few chunks they are not short ones: 64 pairs of 1500 keys, 16 query heads each, 8 chunks 20.6, 12 22.0
+        least = 256 if pairs * 4 >= cus and head_dim <= 128 else 128
+        fill = slots // pairs if pairs <= cus else -(-slots // pairs)
+        most = self.DECODE_PARTS if pairs > 8 else max(self.DECODE_PARTS, ctx // 512)
+        return least, max(1, min(fill, -(-max_ctx // least), most)), 4
 
     def attention_decode(self, q, q_stride, out, kcache, vcache, batch, num_heads, num_kv_heads, head_dim,
                          scale, window, group, token_list=None, n_listed=None, max_ctx=None,

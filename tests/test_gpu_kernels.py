@@ -1183,3 +1183,19 @@ def test_attention_decode_as_its_keys_are_cut(n, longest):
     out = torch.full((n, Hq * d), float("nan"), device=DEV, dtype=torch.bfloat16)
     ops().attention_decode(q.view(n, Hq * d), Hq * d, out, kt(kc), vt(vc), FakeBatch(q_lens, starts, tables), Hq, Hkv, d, d ** -0.5, 0, 0)
     close(out, attention_reference(q, kc, vc, tables, q_lens, starts, Hq, Hkv, d, d ** -0.5, 0), 2 ** -7)
+
+
+# sizes whose sums do not fit the large workgroups' LDS: one chunk a pair, more than a trip of the merge, and the lines between
+@pytest.mark.parametrize("Hq,Hkv,d", [(64, 4, 128), (16, 1, 256), (12, 2, 256)])
+@pytest.mark.parametrize("n,longest", [(1, 256), (1, 1024), (3, 1025), (1, 16385), (32, 513), (64, 600)])
+def test_attention_decode_without_the_large_form(Hq, Hkv, d, n, longest):
+    assert kernels.library.load().ra_attention_decode_slots(Hq, Hkv, d, 12) == 0
+    starts = [(longest - 1) * (i + 1) // n for i in range(n)]
+    q, kc, vc, tables = make_paged_case("bfloat16", Hq, Hkv, d, [1] * n, starts, seed=n)
+    out = torch.full((n, Hq * d), float("nan"), device=DEV, dtype=torch.bfloat16)
+    ops().attention_decode(q.view(n, Hq * d), Hq * d, out, kt(kc), vt(vc), FakeBatch([1] * n, starts, tables), Hq, Hkv, d, d ** -0.5, 0, 0)
+    for i, start in enumerate(starts):          # one query a request: its keys in order
+        keys = torch.arange(start + 1, device=DEV)
+        k, v = (c.double()[tables[i, keys // 16].long(), :, keys % 16].repeat_interleave(Hq // Hkv, 1) for c in (kc, vc))
+        p = torch.softmax((q[i].double() * k).sum(-1) * d ** -0.5, 0)
+        close(out[i].view(Hq, d), (p[:, :, None] * v).sum(0), 2 ** -7)
