@@ -615,7 +615,7 @@ class HipKernels:
         of up to 1800 52.2 / 52.2; 40 of up to 1500 33.6 / 33.6, 14 of 1000 19.4 / 18.2."""
         pairs = max(1, n_tokens * num_kv_heads)
         ctx = max_ctx * head_dim // 128
-        wide = self._slots_of_decode(num_heads, num_kv_heads, head_dim, 12)
+        wide = self._slots_of_decode(num_heads, num_kv_heads, head_dim, 12) if head_dim <= 128 else 0
         slots = self._slots_of_decode(num_heads, num_kv_heads, head_dim, 4) or 768
         if wide == 0:
             return self._small_decode_chunk(pairs, head_dim, max_ctx, slots)
@@ -633,8 +633,10 @@ class HipKernels:
         return 128, max(1, min(fill, -(-max_ctx // 128), self.DECODE_PARTS)), 4
 
     def _small_decode_chunk(self, pairs: int, head_dim: int, max_ctx: int, slots: int):
-        """The same where the large form's sums do not fit its LDS (more than 10 query heads a KV head at head size 128,
-        more than 5 at 256): small workgroups at every size. A pair is one chunk over a few rounds of keys, and over
+        """The same in small workgroups alone: where the large form's sums do not fit its LDS (more than 10 query heads a KV
+        head at head size 128), and above 128 elements a head, where it keeps half of a wave's registers in memory (16
+        heads over 8 KV heads of 256, large / small, one chunk a pair: 16 tokens of 300 keys 40 / 16 us, of 1500 109 / 55;
+        32 chunks: 1 token of 6000 51 / 21). A pair is one chunk over a few rounds of keys, and over
         DECODE_ONE_CTX where the pairs are half of the CUs and more; else it is cut as finely as fills the chip. 1 and 8
         tokens, us, in one chunk / in 4, 8, 16, 32, 64: 64 heads over 4 KV heads of 128, 300 keys 9.6 / 11.1 and 10.7 / 12.3,
         1000 keys 19.3 / 12.5 / 11.1 and 19.9 / 14.8 / 14.3, 16000 keys (from 16 chunks) 27.4 / 24.9 / 27.2 and 51 / 56 / -;

@@ -1185,11 +1185,12 @@ def test_attention_decode_as_its_keys_are_cut(n, longest):
     close(out, attention_reference(q, kc, vc, tables, q_lens, starts, Hq, Hkv, d, d ** -0.5, 0), 2 ** -7)
 
 
-# sizes whose sums do not fit the large workgroups' LDS: one chunk a pair, more than a trip of the merge, and the lines between
-@pytest.mark.parametrize("Hq,Hkv,d", [(64, 4, 128), (16, 1, 256), (12, 2, 256)])
+# sizes whose sums do not fit the large workgroups' LDS, and heads too wide for their registers: one chunk a pair, more than a
+# trip of the merge, and the lines between
+@pytest.mark.parametrize("Hq,Hkv,d", [(64, 4, 128), (16, 1, 256), (12, 2, 256), (16, 8, 256), (8, 2, 192)])
 @pytest.mark.parametrize("n,longest", [(1, 256), (1, 1024), (3, 1025), (1, 16385), (32, 513), (64, 600)])
 def test_attention_decode_without_the_large_form(Hq, Hkv, d, n, longest):
-    assert kernels.library.load().ra_attention_decode_slots(Hq, Hkv, d, 12) == 0
+    assert ops().decode_chunk(n, Hq, Hkv, d, longest)[2] == 4
     starts = [(longest - 1) * (i + 1) // n for i in range(n)]
     q, kc, vc, tables = make_paged_case("bfloat16", Hq, Hkv, d, [1] * n, starts, seed=n)
     out = torch.full((n, Hq * d), float("nan"), device=DEV, dtype=torch.bfloat16)
