@@ -588,7 +588,7 @@ class HipKernels:
     DECODE_SHORT_CTX = 768      # one large workgroup a pair, where the chip holds them all
     DECODE_LONG_CTX = 4096      # from here on large workgroups and their chunks, where the chip holds one a pair
     DECODE_ONE_CTX = 1024       # one small workgroup a pair, where there are more pairs than that
-    DECODE_FILL_ONE = 0.5       # pairs that the chip holds as large workgroups, from this share of them on one each
+    DECODE_FILL_ONE = 0.6       # pairs that the chip holds as large workgroups, from this share of them on one each
     DECODE_FILL = 0.9           # of the last round of large workgroups that more pairs must fill
     DECODE_PARTS = 16           # chunks that the merging kernel asks for in one trip
     DECODE_PAST_CACHES = 32 << 20      # bytes of keys and values of the longest contexts, from which on the caches do not keep them
@@ -608,11 +608,13 @@ class HipKernels:
         workgroup). The kernel cuts every token into equal chunks of its own length, so only their
         number is chosen here. A launch takes 5 us with nothing to read, a merge 4 more, a round of 32 keys a wave
         two (three small workgroups fit a CU, one large one, with as many waves), and the keys come at 4.9 TB/s:
-        few pairs of (token, KV head) are cut until their chunks fill the chip once, and where a workgroup a pair
-        fills half of it there is nothing to merge. 32 query heads over 8 KV heads of 128, us, this rule /
-        the best of 30 others: 8 tokens of 700 keys 11.9 / 11.9, of 1500 16.8 / 16.8, 12 of up to 1500 16.3 / 16.3, 1 of 1500
-        9.5 / 9.5, 16 of 1000 18.7 / 18.7, 2 of 6000 16.8 / 16.8, 48 of up to 440 16.8 / 16.8, 64 of up to 300 14.6 / 14.6,
-        of up to 1800 52.2 / 52.2; 40 of up to 1500 33.6 / 33.6, 14 of 1000 19.4 / 18.2."""
+        few pairs of (token, KV head) are cut until their chunks fill the chip once, and where a large workgroup a pair
+        fills more than half of it there is nothing to merge, but over long contexts from DECODE_FILL_ONE on alone (17 tokens
+        of 2000 keys one / five small chunks 30.0 / 32.2 us, of 6000 79.0 / 73.6; with just half of it two large chunks:
+        16 of 1000 17.4 / 19.7, of 1500 24.1 / 22.8, of 6000 77.7 / 66.8). Over 7 cuts of each form, of 1 to 64 tokens of 300 to
+        16,000 keys, this rule is 1 to 3 % behind the best on average (32 heads over 8 of 128 and of 64, 28 over 4, 16 and 64
+        over 8, 8 over 8 of 96), 5 % with 14 over 2 of 64; 15 to 30 % at 1 to 12 pairs over 6,000 keys and more, where 16
+        large chunks are best."""
         pairs = max(1, n_tokens * num_kv_heads)
         ctx = max_ctx * head_dim // 128
         wide = self._slots_of_decode(num_heads, num_kv_heads, head_dim, 12) if head_dim <= 128 else 0
@@ -620,10 +622,12 @@ class HipKernels:
         if wide == 0:
             return self._small_decode_chunk(pairs, head_dim, max_ctx, slots)
         if pairs <= wide:
-            if pairs >= self.DECODE_FILL_ONE * wide or ctx <= self.DECODE_SHORT_CTX:
+            room, half = wide // pairs, pairs * 2 >= wide
+            if pairs >= self.DECODE_FILL_ONE * wide or ctx <= self.DECODE_SHORT_CTX \
+                    or half and (ctx <= self.DECODE_ONE_CTX if room > 1 else ctx < self.DECODE_LONG_CTX):
                 return 512, 1, 12
-            if ctx >= self.DECODE_LONG_CTX:
-                return 256, min(wide // pairs, -(-max_ctx // 256)), 12
+            if room > 1 and (half or ctx >= self.DECODE_LONG_CTX):
+                return 256, min(room, -(-max_ctx // 256)), 12
         elif ctx > self.DECODE_ONE_CTX and pairs >= self.DECODE_FILL * (-(-pairs // wide) * wide):
             return 512, 1, 12
         elif pairs <= slots and ctx <= self.DECODE_ONE_CTX:

@@ -37,3 +37,13 @@ def test_few_pairs_without_the_large_form_are_cut(Hq, Hkv, d):
                 assert most >= 4 or most == slots // pairs
             if pairs <= 8 and ctx * d >= 16384 * 128:          # no more than 1,024 keys of 128 elements one after the other
                 assert most * 1024 >= ctx * d // 128 or most == slots // pairs
+
+
+def test_pairs_that_fill_half_of_the_chip():
+    """Pairs that the chip holds twice as large workgroups are two such chunks each above 1,024 keys; a few more, which it holds
+    once, are one up to 4,096 keys and small chunks above."""
+    def cut(n, ctx):
+        return Chip().decode_chunk(n, 32, 8, 128, ctx)[1:]
+    assert cut(16, 1024) == (1, 12) and cut(16, 1025) == (2, 12) and cut(16, 16384) == (2, 12)
+    assert cut(17, 4095) == (1, 12) and cut(17, 4096) == (768 // 136, 4)
+    assert cut(20, 4096) == (1, 12) and cut(32, 16384) == (1, 12)

@@ -1195,8 +1195,25 @@ def test_attention_decode_without_the_large_form(Hq, Hkv, d, n, longest):
     q, kc, vc, tables = make_paged_case("bfloat16", Hq, Hkv, d, [1] * n, starts, seed=n)
     out = torch.full((n, Hq * d), float("nan"), device=DEV, dtype=torch.bfloat16)
     ops().attention_decode(q.view(n, Hq * d), Hq * d, out, kt(kc), vt(vc), FakeBatch([1] * n, starts, tables), Hq, Hkv, d, d ** -0.5, 0, 0)
-    for i, start in enumerate(starts):          # one query a request: its keys in order
+    one_query_each(out, q, kc, vc, tables, starts)
+
+
+def one_query_each(out, q, kc, vc, tables, starts):
+    """Decode attention of one query a request against a softmax over its keys in 64 bits."""
+    Hq, d, Hkv = q.shape[1], q.shape[2], kc.shape[1]
+    for i, start in enumerate(starts):
         keys = torch.arange(start + 1, device=DEV)
         k, v = (c.double()[tables[i, keys // 16].long(), :, keys % 16].repeat_interleave(Hq // Hkv, 1) for c in (kc, vc))
         p = torch.softmax((q[i].double() * k).sum(-1) * d ** -0.5, 0)
         close(out[i].view(Hq, d), (p[:, :, None] * v).sum(0), 2 ** -7)
+
+
+@pytest.mark.parametrize("n,longest", [(16, 1025), (16, 4096), (17, 4096)])
+def test_attention_decode_of_half_the_chip(n, longest):
+    """Two large chunks a pair, and five small ones where pairs are a few more."""
+    Hq, Hkv, d = 16, 8, 128
+    starts = [(longest - 1) * (i + 1) // n for i in range(n)]
+    q, kc, vc, tables = make_paged_case("bfloat16", Hq, Hkv, d, [1] * n, starts, seed=n)
+    out = torch.full((n, Hq * d), float("nan"), device=DEV, dtype=torch.bfloat16)
+    ops().attention_decode(q.view(n, Hq * d), Hq * d, out, kt(kc), vt(vc), FakeBatch([1] * n, starts, tables), Hq, Hkv, d, d ** -0.5, 0, 0)
+    one_query_each(out, q, kc, vc, tables, starts)
