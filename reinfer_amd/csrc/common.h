@@ -15,12 +15,16 @@ enum { RA_F32 = 0, RA_BF16 = 1 };
 #define RA_XCDS 8
 
 // Weights that a launch reads once are asked for past the caches' usual policy (non-temporal): on their way through they would put out
-// what is there and be put out themselves before the next step reads them. Measured where the weights in turn are more than the
-// last-level cache (256 MB) holds: 4 to 10 % less for the products of a decode step (8 rows of 24576 x 4096 35.0 us, so 32.5; of 4096 x
-// 12288 20.9, 18.5; of 1024 x 2048 6.0, 5.6). Where a whole model stays in that cache it is the other way round (1 row of 4096 x 1024
-// 3.9, 4.5): models that small have products below this many bytes, and those keep the usual policy.
+// what is there and be put out themselves before the next step reads them. Weights in turn that are more than the last-level cache
+// (256 MB) holds, 1 row, us by the usual policy / past it: 4096 x 1024 4.9 / 4.6, 6144 x 1024 6.6 / 6.1, 2560 x 4096 6.7 / 6.2, 4096 x
+// 4096 8.0 / 7.6, 4096 x 12288 18.7 / 17.4, 24576 x 4096 33.5 / 31.9.
+// Where all the weights, about 200 MB, are still in that cache when they are read again, it is the other way round: 6.2 / 6.4 for 6144 x
+// 1024, 6.6 / 7.6 for 2048 x 6144, 8.0 / 8.6 for 6144 x 2560, at 48 rows 13.8 / 18.2 for 2048 x 6144. What decides is the whole model, which
+// the caller knows: `keep` says that its weights stay (HipKernels.cached_weights), and then all are read by the usual policy. Below this
+// many bytes they always are: that small a model's products mostly are, and its caller may be one that does not say.
 #define RA_STREAM_BYTES (8u << 20)
 #define RA_STREAM 2                // the load's cache policy bits: non-temporal
+static inline bool ra_streams(size_t weight_bytes, int keep) { return !keep && weight_bytes >= RA_STREAM_BYTES; }
 
 typedef __bf16 bf16_t;
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));

@@ -686,7 +686,7 @@ extern "C" long ra_gemm_f32_scratch(int M, int N, int K) {
 }
 
 extern "C" int ra_gemm_f32(const float* A, const float* W, const float* bias, float* C, int M, int N, int K, int lda,
-                           int ldc, float* scratch, long scratch_floats, hipStream_t stream) {
+                           int ldc, float* scratch, long scratch_floats, int keep, hipStream_t stream) {
   RA_CHECK(M > 0 && N > 0 && K > 0, "gemm_f32: empty product (%d, %d, %d)", M, N, K);
   RA_CHECK(lda >= K && ldc >= N, "gemm_f32: row strides (%d, %d) below the row lengths (%d, %d)", lda, ldc, K, N);
   RA_CHECK(ra_gemm_f32_supports(A, W, K, lda), "gemm_f32: rows of %d (stride %d) are not 16-byte pieces", K, lda);
@@ -706,7 +706,7 @@ extern "C" int ra_gemm_f32(const float* A, const float* W, const float* bias, fl
     else gemm_f32_stream_kernel<ROWS, false><<<grid < tiles ? grid : tiles, kb.n * RA_WAVE, F32Stream<ROWS>::lds(kb.n), stream>>>(    \
         A, w, b, C + n0, M, n, K, lda, ldc, kb.k);                                                                                   \
   } while (0)
-      const bool past = (size_t)N * K * sizeof(float) >= RA_STREAM_BYTES;
+      const bool past = ra_streams((size_t)N * K * sizeof(float), keep);
       // as many workgroups as the registers hold, 16 waves a CU
       const int grid = 16 / kb.n * cus;
       if (M > 16) RA_GO(32);

@@ -623,8 +623,8 @@ static int skinny_cus() { return ra_cu_count(); }
 
 template <int NT, int WAVES, int U, int DEPTH, int OCC, int MROWS>
 static int launch_deep(const void* A, int lda, const void* W, const void* bias, void* C, int ldc, int out_dtype,
-                       int epilogue, int M, int N, int K, const SkinnyNorm& nf, int grid, hipStream_t stream) {
-  const bool past = (size_t)N * K * sizeof(bf16_t) >= RA_STREAM_BYTES;
+                       int epilogue, int M, int N, int K, const SkinnyNorm& nf, int grid, int keep, hipStream_t stream) {
+  const bool past = ra_streams((size_t)N * K * sizeof(bf16_t), keep);
 #define RA_GO(EPI, TO)                                                                                                       \
   do {                                                                                                                       \
     if (past) gemm_skinny_deep_kernel<NT, WAVES, U, DEPTH, OCC, MROWS, EPI, TO, true><<<grid, WAVES * RA_WAVE, 0, stream>>>( \
@@ -652,29 +652,29 @@ static int launch_deep(const void* A, int lda, const void* W, const void* bias, 
 // workgroup with four workgroups a CU, and sixteen waves: within 3 % of each other, this one ahead.)
 template <int MROWS>
 static int launch_deep_rows(const void* A, int lda, const void* W, const void* bias, void* C, int ldc, int out_dtype,
-                            int epilogue, int M, int N, int K, const SkinnyNorm& nf, hipStream_t stream) {
+                            int epilogue, int M, int N, int K, const SkinnyNorm& nf, int keep, hipStream_t stream) {
   const int n_tiles = (N + 15) / 16, cus = skinny_cus();
   const int grid = n_tiles < 2 * cus ? n_tiles : 2 * cus;
   // a wave's runs are 128 k long, or 64 where that splits K more evenly over the eight waves (2560 = 2.5
   // x 1024 would leave half of the waves idle in every tile's last run)
   const int runs128 = (K + 1023) / 1024, runs64 = (K + 511) / 512;
   if (runs64 * 512 < runs128 * 1024)
-    return launch_deep<1, 8, 2, 2, 2, MROWS>(A, lda, W, bias, C, ldc, out_dtype, epilogue, M, N, K, nf, grid, stream);
-  return launch_deep<1, 8, 4, 2, 2, MROWS>(A, lda, W, bias, C, ldc, out_dtype, epilogue, M, N, K, nf, grid, stream);
+    return launch_deep<1, 8, 2, 2, 2, MROWS>(A, lda, W, bias, C, ldc, out_dtype, epilogue, M, N, K, nf, grid, keep, stream);
+  return launch_deep<1, 8, 4, 2, 2, MROWS>(A, lda, W, bias, C, ldc, out_dtype, epilogue, M, N, K, nf, grid, keep, stream);
 }
 
 // The same with a second matrix behind the first one's features. The grid is what the first one alone gets where that fills the chip,
 // so a tile's walk over K starts where it would.
 template <int MROWS>
 static int launch_pair(const void* A, int lda, const void* W, void* C, int ldc, int M, int N, int K, const SkinnySecond& second,
-                       hipStream_t stream) {
+                       int keep, hipStream_t stream) {
   const int tiles = (N + 15) / 16 + (second.N + 15) / 16, cus = skinny_cus(), grid = tiles < 2 * cus ? tiles : 2 * cus;
   const SkinnyNorm nf = {};
   const int runs128 = (K + 1023) / 1024, runs64 = (K + 511) / 512;
 #define RA_PAIR(U, STREAM)                                                                                          \
   gemm_skinny_deep_kernel<1, 8, U, 2, 2, MROWS, EPI_PLAIN, bf16_t, STREAM, true><<<grid, 8 * RA_WAVE, 0, stream>>>( \
       (const bf16_t*)A, lda, (const bf16_t*)W, nullptr, (bf16_t*)C, ldc, M, N, K, nf, second)
-  const bool past = (size_t)N * K * sizeof(bf16_t) >= RA_STREAM_BYTES;
+  const bool past = ra_streams((size_t)N * K * sizeof(bf16_t), keep);
   if (runs64 * 512 < runs128 * 1024) {
     if (past) RA_PAIR(2, true);
     else RA_PAIR(2, false);
@@ -701,7 +701,7 @@ static int gemm_skinny_impl(const void* A, const void* W, const void* bias, void
                             int epilogue, int M, int N, int K, int lda, int ldc, const float* in_ss,
                             int in_parts, float in_eps, int in_width, const void* out_w,
                             int out_w_dtype, void* out_x, int out_ldx, float* out_ss, float acc_scale,
-                            hipStream_t stream) {
+                            int keep, hipStream_t stream) {
   RA_CHECK(M > 0 && N > 0 && K > 0, "gemm_skinny: empty product (%d, %d, %d)", M, N, K);
   RA_CHECK(M <= 64, "gemm_skinny: %d rows; this kernel takes at most 64", M);
   RA_CHECK(K % 8 == 0 && lda % 8 == 0, "gemm_skinny: K (%d) and the row stride (%d) must be multiples of 8", K, lda);
@@ -735,17 +735,17 @@ static int gemm_skinny_impl(const void* A, const void* W, const void* bias, void
   }
   // the kernel for up to 16 rows reads through buffer descriptors, whose offsets are 32 bits
   const bool small = (size_t)N * K * 2 < 0xFFFFFF00ull && ((size_t)(M - 1) * lda + K) * 2 < 0xFFFFFF00ull;
-  if (M <= 4 && small) return launch_deep_rows<4>(A, lda, W, bias, C, ldc, out_dtype, epilogue, M, N, K, nf, stream);
-  if (M <= 8 && small) return launch_deep_rows<8>(A, lda, W, bias, C, ldc, out_dtype, epilogue, M, N, K, nf, stream);
-  if (M <= 16 && small) return launch_deep_rows<16>(A, lda, W, bias, C, ldc, out_dtype, epilogue, M, N, K, nf, stream);
+  if (M <= 4 && small) return launch_deep_rows<4>(A, lda, W, bias, C, ldc, out_dtype, epilogue, M, N, K, nf, keep, stream);
+  if (M <= 8 && small) return launch_deep_rows<8>(A, lda, W, bias, C, ldc, out_dtype, epilogue, M, N, K, nf, keep, stream);
+  if (M <= 16 && small) return launch_deep_rows<16>(A, lda, W, bias, C, ldc, out_dtype, epilogue, M, N, K, nf, keep, stream);
   if (M <= 16) return launch_skinny<1, 1, 8, 4>(A, lda, W, bias, C, ldc, out_dtype, epilogue, M, N, K, nf, stream);
   if (small && skinny_features(M, N) == 16) {
     // 17..64 rows, 16 features a workgroup: one workgroup a CU, runs of 64 k
     const int n_tiles = (N + 15) / 16, cus = skinny_cus();
     const int grid = n_tiles < cus ? n_tiles : cus;
-    if (M <= 32) return launch_deep<1, 8, 2, 2, 1, 32>(A, lda, W, bias, C, ldc, out_dtype, epilogue, M, N, K, nf, grid, stream);
-    if (M <= 48) return launch_deep<1, 8, 2, 2, 1, 48>(A, lda, W, bias, C, ldc, out_dtype, epilogue, M, N, K, nf, grid, stream);
-    return launch_deep<1, 8, 2, 2, 1, 64>(A, lda, W, bias, C, ldc, out_dtype, epilogue, M, N, K, nf, grid, stream);
+    if (M <= 32) return launch_deep<1, 8, 2, 2, 1, 32>(A, lda, W, bias, C, ldc, out_dtype, epilogue, M, N, K, nf, grid, keep, stream);
+    if (M <= 48) return launch_deep<1, 8, 2, 2, 1, 48>(A, lda, W, bias, C, ldc, out_dtype, epilogue, M, N, K, nf, grid, keep, stream);
+    return launch_deep<1, 8, 2, 2, 1, 64>(A, lda, W, bias, C, ldc, out_dtype, epilogue, M, N, K, nf, grid, keep, stream);
   }
   if (M <= 32) return launch_skinny<2, 1, 8, 4>(A, lda, W, bias, C, ldc, out_dtype, epilogue, M, N, K, nf, stream);
   // 33..64 rows: with few output features, 16 a workgroup keep all CUs busy; with many, 32 a
@@ -759,27 +759,27 @@ extern "C" int ra_gemm_skinny_normed(const void* A, const void* W, const void* b
                                      int epilogue, int M, int N, int K, int lda, int ldc, const float* in_ss,
                                      int in_parts, float in_eps, int in_width, const void* out_w,
                                      int out_w_dtype, void* out_x, int out_ldx, float* out_ss,
-                                     hipStream_t stream) {
+                                     int keep, hipStream_t stream) {
   return gemm_skinny_impl(A, W, bias, C, out_dtype, epilogue, M, N, K, lda, ldc, in_ss, in_parts, in_eps, in_width,
-                          out_w, out_w_dtype, out_x, out_ldx, out_ss, 1.f, stream);
+                          out_w, out_w_dtype, out_x, out_ldx, out_ss, 1.f, keep, stream);
 }
 
 extern "C" int ra_gemm_skinny(const void* A, const void* W, const void* bias, void* C, int out_dtype,
-                              int epilogue, int M, int N, int K, int lda, int ldc, hipStream_t stream) {
+                              int epilogue, int M, int N, int K, int lda, int ldc, int keep, hipStream_t stream) {
   return gemm_skinny_impl(A, W, bias, C, out_dtype, epilogue, M, N, K, lda, ldc, nullptr, 0, 0.f, 0, nullptr,
-                          0, nullptr, 0, nullptr, 1.f, stream);
+                          0, nullptr, 0, nullptr, 1.f, keep, stream);
 }
 
 // C += acc_scale * (A . W^T): the accumulating epilogue with a factor on the product
 extern "C" int ra_gemm_skinny_scaled(const void* A, const void* W, float* C, int M, int N, int K, int lda, int ldc,
-                                     float acc_scale, hipStream_t stream) {
+                                     float acc_scale, int keep, hipStream_t stream) {
   return gemm_skinny_impl(A, W, nullptr, C, RA_F32, EPI_ACCUM, M, N, K, lda, ldc, nullptr, 0, 0.f, 0, nullptr,
-                          0, nullptr, 0, nullptr, acc_scale, stream);
+                          0, nullptr, 0, nullptr, acc_scale, keep, stream);
 }
 
 // C = A . W^T in bfloat16 and C2 = A . W2^T in float, in one launch: up to 16 rows.
 extern "C" int ra_gemm_skinny_pair(const void* A, const void* W, void* C, const void* W2, float* C2, int M, int N, int N2, int K,
-                                   int lda, int ldc, int ldc2, hipStream_t stream) {
+                                   int lda, int ldc, int ldc2, int keep, hipStream_t stream) {
   RA_CHECK(M > 0 && N > 0 && N2 > 0 && K > 0, "gemm_skinny_pair: empty product (%d, %d and %d, %d)", M, N, N2, K);
   RA_CHECK(M <= 16, "gemm_skinny_pair: %d rows; this kernel takes at most 16", M);
   RA_CHECK(K % 8 == 0 && lda % 8 == 0, "gemm_skinny_pair: K (%d) and the row stride (%d) must be multiples of 8", K, lda);
@@ -792,7 +792,7 @@ extern "C" int ra_gemm_skinny_pair(const void* A, const void* W, void* C, const 
   RA_CHECK(((size_t)N + N2) * K * 2 < 0xFFFFFF00ull && ((size_t)(M - 1) * lda + K) * 2 < 0xFFFFFF00ull,
            "gemm_skinny_pair: [%d and %d, %d] is too large to address", N, N2, K);
   const SkinnySecond second = {(const bf16_t*)W2, C2, N2, ldc2};
-  if (M <= 4) return launch_pair<4>(A, lda, W, C, ldc, M, N, K, second, stream);
-  if (M <= 8) return launch_pair<8>(A, lda, W, C, ldc, M, N, K, second, stream);
-  return launch_pair<16>(A, lda, W, C, ldc, M, N, K, second, stream);
+  if (M <= 4) return launch_pair<4>(A, lda, W, C, ldc, M, N, K, second, keep, stream);
+  if (M <= 8) return launch_pair<8>(A, lda, W, C, ldc, M, N, K, second, keep, stream);
+  return launch_pair<16>(A, lda, W, C, ldc, M, N, K, second, keep, stream);
 }

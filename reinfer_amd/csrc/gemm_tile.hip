@@ -364,7 +364,7 @@ int tile_launch(TileArgs g, hipStream_t stream) {
   g.m_part = g.m_tiles > 1 ? 0xFFFFFFFFu / (unsigned)g.m_tiles + 1u : 0u;
   g.z_part = g.ranges > 1 ? 0xFFFFFFFFu / (unsigned)g.ranges + 1u : 0u;
   const unsigned grid = (unsigned)(total < cus ? total : cus);
-  if (QUICK && g.m_tiles == 1 && !g.end.keep && (size_t)g.N * g.K * sizeof(bf16_t) >= RA_STREAM_BYTES)
+  if (QUICK && g.m_tiles == 1 && ra_streams((size_t)g.N * g.K * sizeof(bf16_t), g.end.keep))
     gemm_tile_kernel<BMT, TN, WM, WN, EPI, QUICK, QUICK><<<grid, 64 * WM * WN, 0, stream>>>(g);
   else
     gemm_tile_kernel<BMT, TN, WM, WN, EPI, QUICK, false><<<grid, 64 * WM * WN, 0, stream>>>(g);

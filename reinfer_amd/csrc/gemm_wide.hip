@@ -250,7 +250,7 @@ static int gemm_wide_impl(const void* A, const void* W, const void* bias, void* 
                           int epilogue, int M, int N, int K, int lda, int ldc, float* scratch,
                           long scratch_floats, const float* in_ss, int in_parts, float in_eps,
                           int in_width, const void* out_w, int out_w_dtype, void* out_x, int out_ldx,
-                          float* out_ss, float out_eps, float acc_scale, hipStream_t stream) {
+                          float* out_ss, float out_eps, float acc_scale, int keep, hipStream_t stream) {
   RA_CHECK(M > 0 && N > 0 && K > 0, "gemm_wide: empty product (%d, %d, %d)", M, N, K);
   RA_CHECK(M <= 128 || ra_gemm_tile_takes(epilogue, M, N, K),
            "gemm_wide: %d rows; at most 128, or 512 where the tiled product is ahead", M);
@@ -298,12 +298,12 @@ static int gemm_wide_impl(const void* A, const void* W, const void* bias, void* 
   if (p.partial) {
     // Above 48 rows the weights by the caches' usual policy: with the adding kernel behind it, 64 rows of 4096 x 4096 14.8 us (past it
     // 15.5), 128 of 2560 x 9728 22.5 (24.0), of 4096 x 12288 32.9 (33.9); at 24 rows 13.6 (12.5), 16.5 (15.4), 25.0 (23.3).
-    if (int rc = ra_tile_ranges(p.tile, A, lda, W, scratch, M, N, K, M > 48, stream)) return rc;
+    if (int rc = ra_tile_ranges(p.tile, A, lda, W, scratch, M, N, K, keep || M > 48, stream)) return rc;
     return launch_wide_reduce(bias, C, ldc, out_dtype, epilogue, M, N, p.tile.ranges, scratch, nf, stream);
   }
   RA_CHECK(M <= 64 || (!in_ss && out_dtype == RA_BF16 && ra_gemm_tile_takes(epilogue, M, N, K)),
            "gemm_wide: with %d rows a gated product only where its tiles fill the chip, with a bfloat16 result and no norm", M);
-  const RaTileEnd end = {nf.in_ss, nf.in_parts, nf.in_eps, nf.in_inv_width, (const bf16_t*)bias, acc_scale, out_dtype == RA_BF16};
+  const RaTileEnd end = {nf.in_ss, nf.in_parts, nf.in_eps, nf.in_inv_width, (const bf16_t*)bias, acc_scale, out_dtype == RA_BF16, keep != 0};
   return ra_tile_product(epilogue, p.tile, A, lda, W, C, ldc, M, N, K, end, stream);
 }
 
@@ -316,7 +316,7 @@ extern "C" int ra_gemm_wide_ranges(int M, int N, int K) {
 // Only the first half of a split product: P[s][m][n] = A[m, range s] . W[n, range s]^T, float, for a
 // consumer that adds the ranges itself (in range order) instead of the adding kernel.
 extern "C" int ra_gemm_wide_partial(const void* A, const void* W, float* P, long p_floats, int M, int N, int K,
-                                    int lda, hipStream_t stream) {
+                                    int lda, int keep, hipStream_t stream) {
   RA_CHECK(M > 0 && N > 0 && K > 0, "gemm_wide: empty product (%d, %d, %d)", M, N, K);
   RA_CHECK(M <= 64 || ra_gemm_tile_takes(WEPI_PLAIN, M, N, K),
            "gemm_wide: %d rows; at most 64, or 512 where the tiled product is ahead", M);
@@ -326,28 +326,30 @@ extern "C" int ra_gemm_wide_partial(const void* A, const void* W, float* P, long
   const RaTilePlan tile = gw_plan(WEPI_PLAIN, M, N, K, true).tile;
   RA_CHECK(P && p_floats >= (long)tile.ranges * M * N, "gemm_wide: %d ranges of [%d, %d] need %ld floats, got %ld", tile.ranges, M, N,
            (long)tile.ranges * M * N, p_floats);
-  return ra_tile_ranges(tile, A, lda, W, P, M, N, K, false, stream);
+  // past the caches at any number of rows (by the usual policy / past it, 64 rows 6144 x 2560 10.8 / 10.3 us, 4096 x 12288 21.8 / 20.2, 128
+  // rows 13.6 / 13.2 and 26.5 / 25.5): the planes' reader here does more than add
+  return ra_tile_ranges(tile, A, lda, W, P, M, N, K, keep != 0, stream);
 }
 
 extern "C" int ra_gemm_wide_normed(const void* A, const void* W, const void* bias, void* C, int out_dtype,
                                    int epilogue, int M, int N, int K, int lda, int ldc, float* scratch,
                                    long scratch_floats, const float* in_ss, int in_parts, float in_eps,
                                    int in_width, const void* out_w, int out_w_dtype, void* out_x, int out_ldx,
-                                   float* out_ss, float out_eps, hipStream_t stream) {
+                                   float* out_ss, float out_eps, int keep, hipStream_t stream) {
   return gemm_wide_impl(A, W, bias, C, out_dtype, epilogue, M, N, K, lda, ldc, scratch, scratch_floats, in_ss,
-                        in_parts, in_eps, in_width, out_w, out_w_dtype, out_x, out_ldx, out_ss, out_eps, 1.f, stream);
+                        in_parts, in_eps, in_width, out_w, out_w_dtype, out_x, out_ldx, out_ss, out_eps, 1.f, keep, stream);
 }
 
 extern "C" int ra_gemm_wide(const void* A, const void* W, const void* bias, void* C, int out_dtype, int epilogue,
                             int M, int N, int K, int lda, int ldc, float* scratch, long scratch_floats,
-                            hipStream_t stream) {
+                            int keep, hipStream_t stream) {
   return gemm_wide_impl(A, W, bias, C, out_dtype, epilogue, M, N, K, lda, ldc, scratch, scratch_floats,
-                        nullptr, 0, 0.f, 0, nullptr, 0, nullptr, 0, nullptr, -1.f, 1.f, stream);
+                        nullptr, 0, 0.f, 0, nullptr, 0, nullptr, 0, nullptr, -1.f, 1.f, keep, stream);
 }
 
 // C += acc_scale * (A . W^T): the accumulating epilogue with a factor on the product
 extern "C" int ra_gemm_wide_scaled(const void* A, const void* W, float* C, int M, int N, int K, int lda, int ldc,
-                                   float* scratch, long scratch_floats, float acc_scale, hipStream_t stream) {
+                                   float* scratch, long scratch_floats, float acc_scale, int keep, hipStream_t stream) {
   return gemm_wide_impl(A, W, nullptr, C, RA_F32, WEPI_ACCUM, M, N, K, lda, ldc, scratch, scratch_floats,
-                        nullptr, 0, 0.f, 0, nullptr, 0, nullptr, 0, nullptr, -1.f, acc_scale, stream);
+                        nullptr, 0, 0.f, 0, nullptr, 0, nullptr, 0, nullptr, -1.f, acc_scale, keep, stream);
 }

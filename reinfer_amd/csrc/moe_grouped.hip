@@ -316,7 +316,7 @@ extern "C" long ra_moe_grouped_scratch(int n_tokens, int top, int experts, int f
 extern "C" int ra_moe_grouped(const void* x, int ldx, const void* w_up, const void* w_down, int ld_down, const int* ids,
                               const float* weights, int top, int distinct, int experts, int ff, int gated, int n_tokens, int width,
                               const float* more, const float* more_logit, int ld_logit, float* resid, void* out, float alpha,
-                              void* scratch, long scratch_bytes, hipStream_t stream) {
+                              void* scratch, long scratch_bytes, int keep, hipStream_t stream) {
   RA_CHECK(n_tokens > 0 && top > 0 && experts > 0 && ff > 0 && width > 0, "moe_grouped: %d tokens, %d of %d experts of %d",
            n_tokens, top, experts, ff);
   RA_CHECK((long)n_tokens * top <= 1L << 24 && n_tokens <= 65535 && experts <= 4096, "moe_grouped: %d tokens, %d of %d experts",
@@ -341,10 +341,10 @@ extern "C" int ra_moe_grouped(const void* x, int ldx, const void* w_up, const vo
   const long most = most_tiles(pairs, experts);
   if (tiled) {
     if (int rc = ra_prompt_experts(tile.rows, tile.up_cols, gated ? 1 : 0, x, n_tokens, ldx, w_up, width, s + at.act, ff, width, plan,
-                                   slots, weights, top, most, tile.past, stream))
+                                   slots, weights, top, most, tile.past && !keep, stream))
       return rc;
     if (int rc = ra_prompt_experts(tile.rows, tile.down_cols, 2, s + at.act, pairs, ff, w_down, ld_down, s + at.rows, width, ff, plan,
-                                   slots, weights, top, most, tile.past, stream))
+                                   slots, weights, top, most, tile.past && !keep, stream))
       return rc;
   } else {
   // 256 weight rows a tile where that still leaves every CU two workgroups: half the reads of the slots' rows (gate and up

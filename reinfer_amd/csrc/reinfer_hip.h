@@ -5,7 +5,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
-#define RA_ABI_VERSION 32
+#define RA_ABI_VERSION 33
 
 #ifdef __cplusplus
 extern "C" {
@@ -88,21 +88,24 @@ long ra_moe_grouped_scratch(int n_tokens, int top, int experts, int ff, int widt
 int ra_moe_grouped(const void* x, int ldx, const void* w_up, const void* w_down, int ld_down, const int* ids,
                    const float* weights, int top, int distinct, int experts, int ff, int gated, int n_tokens, int width,
                    const float* more, const float* more_logit, int ld_logit, float* resid, void* out, float alpha,
-                   void* scratch, long scratch_bytes, hipStream_t stream);
+                   void* scratch, long scratch_bytes, int keep, hipStream_t stream);
 
 // float operands and result, to float precision on the bfloat16 matrix cores (each float in three parts), for rows that are
 // whole 16-byte pieces (ra_gemm_f32_supports): C[M, N] = A . W^T (+ bias). scratch: ra_gemm_f32_scratch floats (0: none needed).
 int ra_gemm_f32_supports(const void* A, const void* W, int K, int lda);
 long ra_gemm_f32_scratch(int M, int N, int K);
 int ra_gemm_f32(const float* A, const float* W, const float* bias, float* C, int M, int N, int K, int lda, int ldc,
-                float* scratch, long scratch_floats, hipStream_t stream);
+                float* scratch, long scratch_floats, int keep, hipStream_t stream);
+
+// `keep`, here and below: the weights are read by the caches' usual policy whatever their size (a hint: the caller knows that they
+// stay in the last-level cache from one call to the next; RA_STREAM_BYTES in common.h).
 
 // bfloat16, M <= 64, K and lda multiples of 8: weight-streaming MFMA product.
 // epilogue 0: C[M, N] = A . W^T (+ bias); epilogue 1: W rows are gate/up interleaved in runs of 8
 // and C[M, N/2] = silu(gate) * up; epilogue 2: C is float and C += A . W^T (+ bias)
 int ra_gemm_skinny_max_rows(void);
 int ra_gemm_skinny(const void* A, const void* W, const void* bias, void* C, int out_dtype, int epilogue,
-                   int M, int N, int K, int lda, int ldc, hipStream_t stream);
+                   int M, int N, int K, int lda, int ldc, int keep, hipStream_t stream);
 // The same with an RMSNorm carried by the products around it, y = rstd[m] * ((x .* w) . W^T):
 // in_ss float [in_parts, M], if given: partial sums of squares of the rows behind A; the result
 // rows are scaled by rsqrt(sum / in_width + in_eps). out_w / out_x / out_ss, if given (epilogue 2
@@ -112,7 +115,7 @@ int ra_gemm_skinny_row_parts(int M, int N);
 int ra_gemm_skinny_normed(const void* A, const void* W, const void* bias, void* C, int out_dtype,
                           int epilogue, int M, int N, int K, int lda, int ldc, const float* in_ss,
                           int in_parts, float in_eps, int in_width, const void* out_w, int out_w_dtype,
-                          void* out_x, int out_ldx, float* out_ss, hipStream_t stream);
+                          void* out_x, int out_ldx, float* out_ss, int keep, hipStream_t stream);
 
 // bfloat16, up to 128 rows (gated and cut products; plain and added whole ones up to 64): the same product and epilogues with the
 // activations shared by a workgroup's waves; ra_gemm_wide_preferred says where it is the faster of the two (17 rows and more, not the
@@ -120,12 +123,12 @@ int ra_gemm_skinny_normed(const void* A, const void* W, const void* bias, void* 
 // scratch (0: none needed).
 int ra_gemm_wide_ranges(int M, int N, int K);          // K ranges of ra_gemm_wide_partial's result
 int ra_gemm_wide_partial(const void* A, const void* W, float* P, long p_floats, int M, int N, int K, int lda,
-                         hipStream_t stream);         // P[range][m][n] float, for a consumer that adds the ranges
+                         int keep, hipStream_t stream);         // P[range][m][n] float, for a consumer that adds the ranges
 int ra_gemm_wide_preferred(int epilogue, int M, int N, int K);
 long ra_gemm_wide_scratch(int epilogue, int M, int N, int K, int emits);
 int ra_gemm_wide(const void* A, const void* W, const void* bias, void* C, int out_dtype, int epilogue,
                  int M, int N, int K, int lda, int ldc, float* scratch, long scratch_floats,
-                 hipStream_t stream);
+                 int keep, hipStream_t stream);
 // With a carried RMSNorm, as ra_gemm_skinny_normed; an emitting product always needs scratch
 // (ra_gemm_wide_scratch with emits = 1) and writes out_ss[ra_gemm_wide_row_parts(N), M]. With out_ss null and
 // out_eps >= 0 it finishes the norm that follows instead: out_x = bf16(norm(C_new, out_eps) * out_w), one
@@ -135,7 +138,7 @@ int ra_gemm_wide_normed(const void* A, const void* W, const void* bias, void* C,
                         int M, int N, int K, int lda, int ldc, float* scratch, long scratch_floats,
                         const float* in_ss, int in_parts, float in_eps, int in_width, const void* out_w,
                         int out_w_dtype, void* out_x, int out_ldx, float* out_ss, float out_eps,
-                        hipStream_t stream);
+                        int keep, hipStream_t stream);
 
 // bfloat16, more rows than the kernels above take, K a multiple of 64 and N of 16 (gemm_prompt.hip). ra_gemm_prompt_takes: whether
 // the product is this kernel's (2, of a gated one: the library's float product and ra_silu_mul_rounded are ahead). Epilogues 0 to 2 as
@@ -360,12 +363,12 @@ int ra_turn_heads(void* x, int act_dtype, long ld, int n_tokens, int heads, int 
 // C += acc_scale * (A . W^T) through the weight-streaming kernels (bfloat16 operands, float C; the limits of
 // ra_gemm_skinny / ra_gemm_wide with the accumulating epilogue)
 int ra_gemm_skinny_scaled(const void* A, const void* W, float* C, int M, int N, int K, int lda, int ldc,
-                          float acc_scale, hipStream_t stream);
+                          float acc_scale, int keep, hipStream_t stream);
 // up to 16 rows: C = A . W^T in bfloat16 and C2 = A . W2^T in float, W2 of at most 16 features a CU, in one launch
 int ra_gemm_skinny_pair(const void* A, const void* W, void* C, const void* W2, float* C2, int M, int N, int N2, int K, int lda,
-                        int ldc, int ldc2, hipStream_t stream);
+                        int ldc, int ldc2, int keep, hipStream_t stream);
 int ra_gemm_wide_scaled(const void* A, const void* W, float* C, int M, int N, int K, int lda, int ldc, float* scratch,
-                        long scratch_floats, float acc_scale, hipStream_t stream);
+                        long scratch_floats, float acc_scale, int keep, hipStream_t stream);
 
 // Retention: S <- decays[h] S + k v^T, o = S^T q, q and k turned by their position over their first rot_dims elements
 // (pairs (i, i + rot_dims / 2), angle position * inv_freq[i]), times q_scale and k_scale. State: ra_scan_state_floats kind 3.

@@ -15,7 +15,7 @@ import torch  # noqa: F401  (loads the HIP runtime the library links against)
 
 from ..csrc import build as _build
 
-ABI_VERSION = 32
+ABI_VERSION = 33
 
 
 class KernelLibraryError(RuntimeError):
@@ -33,24 +33,24 @@ _SIGNATURES = {
     "ra_add_rmsnorm": [P, P, P, I, P, I, P, I, I, F, F, P],
     "ra_qk_norm_rope_cache": [P, I, P, P, I, F, P, P, I, I, P, P, P, I, I, I, I, I, I, I, P],
     "ra_qk_norm_rope_cache_sums": [P, I, P, I, F, I, P, I, I, P, P, I, F, P, P, I, I, P, P, P, I, I, I, I, I, I, P],
-    "ra_gemm_wide_partial": [P, P, P, c_long, I, I, I, I, P],
+    "ra_gemm_wide_partial": [P, P, P, c_long, I, I, I, I, I, P],
     "ra_silu_mul": [P, P, I, I, I, I, P],
     "ra_silu_mul_rounded": [P, P, I, I, I, P],
     "ra_attention_plain": [P, I, P, I, P, P, I, P, I, P, P, P, I, I, I, I, I, F, I, P],
     "ra_attention_decode": [P, I, P, I, P, P, P, I, P, P, P, I, I, I, I, I, F, I, I, I, I, P, P, P],
     "ra_attention_prefill": [P, I, P, I, P, P, P, I, P, I, I, I, I, I, F, I, P],
     "ra_attention_prefill_split": [P, I, P, I, P, P, P, I, P, I, P, P, I, P, P, I, I, I, I, F, I, P],
-    "ra_gemm_skinny": [P, P, P, P, I, I, I, I, I, I, I, P],
-    "ra_gemm_wide": [P, P, P, P, I, I, I, I, I, I, I, P, c_long, P],
-    "ra_gemm_wide_normed": [P, P, P, P, I, I, I, I, I, I, I, P, c_long, P, I, F, I, P, I, P, I, P, F, P],
-    "ra_gemm_skinny_normed": [P, P, P, P, I, I, I, I, I, I, I, P, I, F, I, P, I, P, I, P, P],
-    "ra_gemm_skinny_scaled": [P, P, P, I, I, I, I, I, F, P],
-    "ra_gemm_skinny_pair": [P, P, P, P, P, I, I, I, I, I, I, I, P],
+    "ra_gemm_skinny": [P, P, P, P, I, I, I, I, I, I, I, I, P],
+    "ra_gemm_wide": [P, P, P, P, I, I, I, I, I, I, I, P, c_long, I, P],
+    "ra_gemm_wide_normed": [P, P, P, P, I, I, I, I, I, I, I, P, c_long, P, I, F, I, P, I, P, I, P, F, I, P],
+    "ra_gemm_skinny_normed": [P, P, P, P, I, I, I, I, I, I, I, P, I, F, I, P, I, P, I, P, I, P],
+    "ra_gemm_skinny_scaled": [P, P, P, I, I, I, I, I, F, I, P],
+    "ra_gemm_skinny_pair": [P, P, P, P, P, I, I, I, I, I, I, I, I, P],
     "ra_gemm_prompt": [P, P, P, I, I, I, I, I, I, F, I, I, I, P],
-    "ra_gemm_wide_scaled": [P, P, P, I, I, I, I, I, P, c_long, F, P],
+    "ra_gemm_wide_scaled": [P, P, P, I, I, I, I, I, P, c_long, F, I, P],
     "ra_gemm_plain": [P, P, P, P, I, I, I, I, I, I, I, P],
-    "ra_moe_grouped": [P, I, P, P, I, P, P, I, I, I, I, I, I, I, P, P, I, P, P, F, P, c_long, P],
-    "ra_gemm_f32": [P, P, P, P, I, I, I, I, I, P, c_long, P],
+    "ra_moe_grouped": [P, I, P, P, I, P, P, I, I, I, I, I, I, I, P, P, I, P, P, F, P, c_long, I, P],
+    "ra_gemm_f32": [P, P, P, P, I, I, I, I, I, P, c_long, I, P],
     "ra_sample": [P, I, I, I, P, P, P, P, P, P, P],
     "ra_sample_static": [P, I, I, I, P, P, P, P, P],
     "ra_filter_logits": [P, I, I, I, P, P, P, c_long, P],

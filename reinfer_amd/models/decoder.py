@@ -70,6 +70,9 @@ class DecoderModel:
         self.run_order = spec.run_order
         # a router between two nearly equal experts decides by a sum's last bits: see HipKernels.library_products
         self.routes = any(getattr(p, "router", None) is not None for p in self.parts())
+        # what a step may read of the weights (of an embedding that is not the head, a row a token): see HipKernels.cached_weights
+        aside = spec.head_name if spec.tie_embeddings else spec.embed_name
+        self.weight_bytes = sum(t.numel() * t.element_size() for name, t in weights.items() if name != aside)
 
     def cache_needs(self) -> List[Optional[object]]:
         """What each run-order entry keeps: KVNeed, PagedNeed, StateNeed, or None. The block arrangement
@@ -123,8 +126,14 @@ class DecoderModel:
         the embedding (i = 0) and behind run-order entry i - 1 (the reference reads activations back
         layer by layer the same way, crates/cuda/src/engine.rs:3744-3765)."""
         products = getattr(kernels.current(), "library_products", None) if self.routes else None
-        with products() if products is not None else contextlib.nullcontext():
+        with products() if products is not None else contextlib.nullcontext(), self._weights_in_cache():
             return self._forward_layers(batch, caches, observer, input_states)
+
+    def _weights_in_cache(self):
+        ops = kernels.current()
+        if self.weight_bytes > getattr(ops, "CACHED_WEIGHTS", -1):
+            return contextlib.nullcontext()
+        return ops.cached_weights()
 
     def _forward_layers(self, batch, caches, observer, input_states):
         ops = kernels.current()
@@ -191,7 +200,8 @@ class DecoderModel:
             xn = self.final_norm.add_norm(resid, delta, rows=batch.logit_rows)
         logits = torch.empty((batch.num_logit_rows, self.spec.vocab_size), dtype=torch.float32,
                              device=self.device)
-        kernels.current().linear(xn, self.head, logits)
+        with self._weights_in_cache():
+            kernels.current().linear(xn, self.head, logits)
         if self.spec.logit_softcap > 0.0:
             kernels.current().tanh_cap(logits, self.spec.logit_softcap)
         return logits
