@@ -203,3 +203,35 @@ def test_a_gate_of_what_is_not_finite():
     want[8] = float("nan")                  # minus infinity over infinity
     got = out[0, :len(gate)].float()
     assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.allclose(got.nan_to_num(0.0, 1e38, -1e38), want.nan_to_num(0.0, 1e38, -1e38), rtol=2 ** -8, atol=1e-30)
+
+
+# 65 to 128 rows, the first and the last N of a width of tile (80, 96, 112, 128 features)
+@pytest.mark.parametrize("M", [65, 113, 128])
+@pytest.mark.parametrize("I,K", [(8200, 1032), (10240, 1024), (10248, 1032), (12288, 1096), (12296, 1032), (14336, 1536), (14344, 1032)])
+def test_gated_in_tiles_of_every_width(M, I, K):
+    test_tiled_gated_product(M, I, K)
+
+
+# planes in tiles of 64, 80, 96, 112 and 128 features above 64 rows, and of 80, 96, 112, 128 and 160 below; N off a whole tile, ranges
+# that end inside a stage
+@pytest.mark.parametrize("M,N,K", [(M, N, K) for M in (65, 97, 128) for N, K in ((4096, 4104), (10236, 2568), (6144, 4104), (7168, 4104),
+                                                                               (2564, 12296), (7164, 2056))]
+                         + [(M, N, K) for M in (17, 33, 64) for N, K in ((2560, 4104), (4604, 2568), (7164, 2568), (6656, 4096), (10236, 4104),
+                                                                         (9216, 4096))])
+def test_planes_in_tiles_of_every_width(M, N, K):
+    lib = kernels.library.load()
+    x, w, g = operands(M, N, K, M * 5 + N)
+    ref, err = x.double() @ w.double().T, bound(x, w, K)
+    S = int(lib.ra_gemm_wide_ranges(M, N, K))
+    parts = torch.full((S, M, N), float("nan"), device=DEV)
+    for keep in (0, 1):
+        if M > 64 and not lib.ra_gemm_tile_takes(0, M, N, K):
+            break
+        kernels.library.call("ra_gemm_wide_partial", x.data_ptr(), w.data_ptr(), parts.data_ptr(), parts.numel(), M, N, K, K, keep,
+                             torch.cuda.current_stream().cuda_stream)
+        assert ((parts.double().sum(0) - ref).abs() <= err).all()
+        parts.fill_(float("nan"))
+    stream = torch.randn(M, N, device=DEV, generator=g)
+    want = stream.double() + ref
+    ops()._few_rows("linear output", x, w, None, stream, 2, M, N, K, True)
+    assert ((stream.double() - want).abs() <= err + want.abs() * 2 ** -23).all()
