@@ -1,7 +1,7 @@
 // Flash-decode attention over the paged cache, bfloat16, on the matrix cores:
 // one query token per (request, position); the query heads of one KV head are
 // the columns of the MFMA tiles, so every key and value is read once for the
-// whole group. The keys are cut into chunks; a workgroup (4 waves) takes one
+// whole group. The keys are cut into chunks; a workgroup (4 or 12 waves) takes one
 // (chunk, KV head, token), its waves take 32 keys at a time:
 //
 //   S^T[key][head]  = K . Q^T          v_mfma_f32_16x16x32_bf16 over d
@@ -38,9 +38,11 @@
 #include "common.h"
 #include "reinfer_hip.h"
 
-// Waves a workgroup: 4 where the step has (token, KV head) pairs enough to fill the chip with small
-// workgroups, 12 where it has few: a CU then has 192 KB of keys and values in flight for one work item,
-// few chunks a token are enough to keep the memory busy, and a token with one chunk needs no merge.
+// Waves a workgroup: 4, of which up to head size 128 three workgroups or more share a CU, or 12, one a CU with 192 KB of keys and values in
+// flight for one work item, so that few chunks a token keep the memory busy, and one needs no merge. The caller chooses, and the
+// chunks with it (HipKernels.decode_chunk): 12 where one such workgroup a (token, KV head) pair fills half of the chip and more, and
+// for fewer pairs over short contexts and over long ones; 4 for few pairs between those, for more pairs than CUs, and for all steps
+// where 12 do not fit their LDS or registers (many query heads a KV head, heads of more than 128 elements).
 
 __device__ __forceinline__ float fd_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
@@ -499,7 +501,7 @@ extern "C" int ra_attention_decode_supports(int Hq, int Hkv, int d, int block_si
 
 // Workgroups of the decode kernel, in its form with `waves` waves a workgroup (4 or 12), that the current
 // device holds at once for these sizes (its grid); 0 if the sizes are not taken or the device cannot be
-// asked. The caller cuts the keys so that the work items fill this grid once.
+// asked. The caller cuts the keys by it.
 extern "C" int ra_attention_decode_slots(int Hq, int Hkv, int d, int waves) {
   if (!ra_attention_decode_supports(Hq, Hkv, d, 16) || (waves != 4 && waves != 12)) return 0;
   const size_t lds = (size_t)waves * (Hq / Hkv) * (d + 2) * sizeof(float);

@@ -624,7 +624,7 @@ static int fp_launch(const void* q, int q_stride, void* out, int out_stride,
   } while (0)
 #define RA_FP(DM, NCC)                                                                                \
   do {                                                                                                \
-    if (d == DM && DM <= 128) RA_FP_GO(DM, NCC, true); /* at 256 the exact form spills registers */   \
+    if (d == DM) RA_FP_GO(DM, NCC, true);                                                             \
     else RA_FP_GO(DM, NCC, false);                                                                    \
   } while (0)
   if (d <= 64) RA_FP(64, 2);

@@ -372,8 +372,9 @@ int tile_launch(TileArgs g, hipStream_t stream) {
   return 0;
 }
 
-// Five to ten waves, which fetch rows faster than four (36 against 30 bytes a clock): 19456 x 2560 with its gate at 128 rows, 80
-// features, is the one shape measured where four were ahead (30.9 us against 31.0, at 97 rows 28.6 against 29.5).
+// Five to ten waves, which fetch rows faster than four (36 against 30 bytes a clock). Above 64 rows a gated tile of 80 features has
+// four, each with its two row tiles of all features. Of 16400 to 20480 features at 65 to 128 rows, four / ten waves, K of 1024 13.0 / 12.7
+// us, 1536 to 2560 the same within 1 % (19456 x 2560 27.7 / 27.9 at 97 rows), 4096 34.0 / 34.6, 5120 45.0 / 47.2, 8192 63.4 / 66.6.
 template <int EPI>
 int tile_cols(const TileArgs& g, int cols, hipStream_t stream) {
 #define RA_GT(BMT, TN, WM, WN) return tile_launch<BMT, TN, WM, WN, EPI>(g, stream)
@@ -469,8 +470,9 @@ RaTilePlan ra_tile_plan(int M, int N, int K, bool cut) {
 }
 
 // Of 65 to 512 rows. Products that are cut and whose ranges fill three quarters of the chip, or that are small (the library has too few
-// tiles for those as well): 11264 x 4096 at 128 rows, 176 of 256 CUs, takes 34 us against the library's 32, 9216 x 4096, 216 CUs, 26
-// against 30; 22528 x 4096, whose tiles do not fill the chip and cannot be cut, 49 against 45. Above 256 rows only a long K,
+// tiles for those as well): 9216 x 4096 at 128 rows, 216 of 256 CUs, takes 27 us against the library's 30. 11264 x 4096, 176 CUs, is
+// refused though it takes 29 against 32 now (this line was drawn with the tiles of before, which took 34); 22528 x 4096, whose tiles do
+// not fill the chip and cannot be cut, takes 40 against 46 at 65 rows, 49 against 47 at 128. Above 256 rows only a long K,
 // where the planes are few beside the weights, and more than that share of the chip (4096 x 12288 at 384 rows, 192 CUs,
 // 70 us on gemm_prompt.hip's tiles against 69, though at 300 rows 57 against 69; at 512 rows, all of them, 74 against 80); the line
 // is the same for all rows of a row of tiles, as the sums are. Beyond 512 the library's larger tiles read less. What adds into
@@ -498,7 +500,6 @@ int ra_tile_product(int epilogue, const RaTilePlan& plan, const void* A, int lda
                (long)plan.ranges * plan.range_k >= K && (plan.ranges == 1 || epilogue == GT_PART),
            "gemm_tile: %d ranges of %d k for %d", plan.ranges, plan.range_k, K);
   RA_CHECK(epilogue != GT_GATED || N % 16 == 0, "gemm_tile: the gate takes whole runs of 16 features");
-  const size_t piece = epilogue == GT_PART || epilogue == GT_ADD || !end.half ? 16 : 8;
   if (!end.in_ss) end.in_parts = 0;
   const int cols = epilogue == GT_GATED ? N / 2 : N;
   const bool half = end.half && (epilogue == GT_PLAIN || epilogue == GT_GATED);

@@ -326,8 +326,8 @@ extern "C" int ra_gemm_wide_partial(const void* A, const void* W, float* P, long
   const RaTilePlan tile = gw_plan(WEPI_PLAIN, M, N, K, true).tile;
   RA_CHECK(P && p_floats >= (long)tile.ranges * M * N, "gemm_wide: %d ranges of [%d, %d] need %ld floats, got %ld", tile.ranges, M, N,
            (long)tile.ranges * M * N, p_floats);
-  // past the caches at any number of rows (by the usual policy / past it, 64 rows 6144 x 2560 10.8 / 10.3 us, 4096 x 12288 21.8 / 20.2, 128
-  // rows 13.6 / 13.2 and 26.5 / 25.5): the planes' reader here does more than add
+  // past the caches at any number of rows: by the usual policy / past it, 64 rows 6144 x 2560 10.8 / 10.3 us, 4096 x 12288 21.8 / 20.2, 128
+  // rows 13.6 / 13.2 and 26.5 / 25.5
   return ra_tile_ranges(tile, A, lda, W, P, M, N, K, keep != 0, stream);
 }
 

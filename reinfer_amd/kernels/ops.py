@@ -151,9 +151,9 @@ class HipKernels:
 
     # ---- the q/k/v product left in K ranges for the kernel that consumes it
     # Weights (elements) from which 17 to 64 rows leave a product in ranges that would else go, whole, to the kernel whose waves split
-    # K. Both with the q/k norm, 17 / 32 / 64 rows, in ranges : whole: 4096 x 1024 10.9 / 11.3 / 13.7 : 8.3 / 8.6 / 12.3 us,
-    # 4096 x 2048 11.6 / 13.2 / 15.5 : 10.6 / 11.0 / 15.3, but 2560 x 4096 13.0 / 13.1 / 16.5 : 12.4 / 13.5 / 19.5,
-    # 5120 x 2048 12.5 / 12.7 / 16.8 : 13.8 / 14.9 / 21.7, 6144 x 2560 14.5 / 14.9 / 17.3 : 16.3 / 18.4 / 26.6.
+    # K. Both with the q/k norm, 17 / 32 / 64 rows, in ranges : whole: 4096 x 1024 9.1 / 9.6 / 11.1 : 7.6 / 8.6 / 12.3 us,
+    # 4096 x 2048 10.9 / 11.8 / 13.0 : 9.5 / 10.1 / 14.6, but 2560 x 4096 11.7 / 13.1 / 15.2 : 12.0 / 13.0 / 19.4,
+    # 5120 x 2048 11.2 / 12.4 / 14.3 : 12.6 / 14.2 / 21.4, 6144 x 2560 12.5 / 13.8 / 16.9 : 16.0 / 18.2 / 26.4.
     RANGES_WEIGHTS = 10 << 20
 
     def linear_ranges(self, x: torch.Tensor, weight: torch.Tensor):
@@ -817,9 +817,11 @@ class HipKernels:
             raise ValueError(f"linear_columns: x {tuple(x.shape)}, columns {tuple(part.shape)}, out {tuple(out.shape)}")
         torch.mm(x, part.t(), out_dtype=torch.float32, out=out)
 
-    # Weights (elements) from which a product that is cut, and then added up by a kernel of its own, is worth that: at 65 to 256
-    # rows, tiled / library, 8192 x 2048 14 to 22 / 11 to 20 us, 6144 x 2560 14 to 23 / 13 to 25, 4096 x 4096 14 to 22 / 14 to 26 in
-    # no order, but 6144 x 4096 18 to 30 / 18 to 40 and 4096 x 6144 17 to 28 / 19 to 43. A gated product is not cut, and what adds
+    # Weights (elements) from which a product that is cut, and then added up by a kernel of its own, is surely worth that: at 65 to
+    # 256 rows, tiled / library, 6144 x 4096 17 to 30 / 23 to 40 us, 4096 x 6144 17 to 28 / 23 to 36, 4096 x 12288 26 to 42 / 41 to
+    # 76; 8192 x 2048 15 to 22 / 14 to 25 and 6144 x 2560 14 to 25 / 16 to 31 in no order, 2048 x 2048 10 to 16 / 11 to 12.
+    # (4096 x 4096 and 2560 x 4096 are ahead at most rows as well, 13 to 21 / 16 to 27 and 12 to 19 / 13 to 24: the line was drawn
+    # with the tiles of before.) A gated product is not cut, and what adds
     # into the stream is launched here in a fraction of the host's time for the library's product (a 4b prompt of 160 rows with
     # its 2560 x 4096 in the library 1.70 ms, tiled 1.63).
     TILE_ADDED_WEIGHTS = 20 << 20
