@@ -33,6 +33,7 @@ namespace {
 #define GT_BK 64
 #define GT_SIDE 128
 #define GT_RING (128 * 1024)
+#define GT_SPAN 0x7FFFFF00ull      // bytes that a descriptor covers, from a tile's first row on
 
 typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
@@ -452,6 +453,7 @@ RaTilePlan ra_tile_plan(int M, int N, int K, bool cut) {
   const float rows = M <= 64 ? 48.f : 112.f;
   float least = 1e30f;
   for (int cols = M <= 64 ? 160 : 128; cols >= 64; cols -= cols > 128 ? 32 : 16) {
+    if (cols > GT_SIDE && (size_t)cols * K * 2 >= GT_SPAN) continue;
     const int tiles = (N + cols - 1) / cols;
     const int fits = tiles < cus ? cus / tiles : 1, top = fits < most ? fits : most;
     for (int s = top > 1 ? top : 1; s >= 1 && s + 1 >= top; --s) {       // as many ranges as fill the chip once, or one less
@@ -494,7 +496,7 @@ int ra_tile_product(int epilogue, const RaTilePlan& plan, const void* A, int lda
                     RaTileEnd end, hipStream_t stream) {
   RA_CHECK(M > 0 && N > 0 && K > 0 && K % 8 == 0 && lda % 8 == 0 && lda >= K && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0,
            "gemm_tile: [%d, %d, %d] with rows of stride %d must be whole 16-byte pieces", M, N, K, lda);
-  RA_CHECK((size_t)160 * K * 2 < 0x7FFFFF00ull && ((size_t)(M - 1) * lda + K) * 2 < 0x7FFFFF00ull,
+  RA_CHECK((size_t)(plan.cols > GT_SIDE ? plan.cols : GT_SIDE) * K * 2 < GT_SPAN && ((size_t)(M - 1) * lda + K) * 2 < GT_SPAN,
            "gemm_tile: an operand of [%d, %d, %d] is larger than a descriptor covers", M, N, K);
   RA_CHECK(plan.ranges >= 1 && plan.range_k % GT_BK == 0 && (long)(plan.ranges - 1) * plan.range_k < K &&
                (long)plan.ranges * plan.range_k >= K && (plan.ranges == 1 || epilogue == GT_PART),

@@ -235,3 +235,18 @@ def test_planes_in_tiles_of_every_width(M, N, K):
     want = stream.double() + ref
     ops()._few_rows("linear output", x, w, None, stream, 2, M, N, K, True)
     assert ((stream.double() - want).abs() <= err + want.abs() * 2 ** -23).all()
+
+
+@pytest.mark.parametrize("N", [16, 33000])          # one tile in ranges of K; tiles of 160 features where K allows them
+def test_rows_too_long_for_the_widest_tile(N):
+    """160 rows of weights span more than a descriptor covers, 128 do not: a narrower tile takes the product."""
+    M, K = 17, 6710912 if N == 16 else 128
+    x, w, _ = operands(M, N, K, 5)
+    out = torch.full((M, N), float("nan"), device=DEV)
+    ops().linear_skinny(x, w, out, wide=True)
+    for n in range(0, N, 4096):
+        part = slice(n, n + 4096)
+        want = sum(x[:, k:k + (1 << 20)].double() @ w[part, k:k + (1 << 20)].double().T for k in range(0, K, 1 << 20))
+        # sums of deviation 1, rounded K times at most by up to 2^-25 in either direction: eight deviations of their sum, a fifth of
+        # what a lost stage of 64 k would show
+        assert ((out[:, part].double() - want).abs() <= 8 * math.sqrt(K) * 2 ** -25 * (1 + want.abs())).all()
