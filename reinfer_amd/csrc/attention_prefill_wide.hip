@@ -84,7 +84,7 @@ flash_prefill_wide_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __
   const int kvh = by / n_hgrp, hgrp = by % n_hgrp;
   const int seq = tile_info[tile * 4 + 0];
   const int row0 = tile_info[tile * 4 + 1];
-  const int nq = tile_info[tile * 4 + 2];
+  const int nq = tile_info[tile * 4 + 2] & 0xffff;      // above it, which column tiles are computed: at 256 elements all are
   const int pos0 = tile_info[tile * 4 + 3];
   const int* table = block_tables + (size_t)seq * max_blocks;
 

@@ -1217,3 +1217,22 @@ def test_attention_decode_of_half_the_chip(n, longest):
     out = torch.full((n, Hq * d), float("nan"), device=DEV, dtype=torch.bfloat16)
     ops().attention_decode(q.view(n, Hq * d), Hq * d, out, kt(kc), vt(vc), FakeBatch([1] * n, starts, tables), Hq, Hkv, d, d ** -0.5, 0, 0)
     one_query_each(out, q, kc, vc, tables, starts)
+
+
+@pytest.mark.parametrize("d", [144, 256])
+def test_column_bits_of_a_tile_mean_nothing_where_a_wave_holds_one(d):
+    """Above 128 elements a tile is never given away by halves: the bits above its number of queries change nothing."""
+    Hq, Hkv, q_lens, starts = 4, 2, [70, 9], [3, 40]
+    lib = kernels.library.load()
+    assert lib.ra_attention_prefill_columns(Hq, Hkv, d) == 1
+    q, kc, vc, tables = make_paged_case("bfloat16", Hq, Hkv, d, q_lens, starts, seed=d)
+    tile, T, got = lib.ra_attention_prefill_tile(Hq, Hkv, d), sum(q_lens), []
+    for bits in (0, 1, 2, 3):
+        info = [v for i, row in enumerate((0, 70)) for q0 in range(0, q_lens[i], tile)
+                for v in (i, row + q0, min(tile, q_lens[i] - q0) | bits << 16, starts[i] + q0)]
+        out = torch.full((T, Hq * d), float("nan"), device=DEV, dtype=torch.bfloat16)
+        ops().attention_prefill(q.view(T, Hq * d), Hq * d, out, kt(kc), vt(vc), FakeBatch(q_lens, starts, tables), Hq, Hkv, d, d ** -0.5, 0, 0,
+                                torch.tensor(info, dtype=torch.int32, device=DEV), len(info) // 4)
+        got.append(out)
+    assert all(torch.equal(got[0], o) for o in got[1:])
+    close(got[0], attention_reference(q, kc, vc, tables, q_lens, starts, Hq, Hkv, d, d ** -0.5, 0), 2 ** -7)
