@@ -91,12 +91,18 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_tile_kernel(TileArgs g) {
   if (at >= total) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, q = lane >> 4;
-  // a tile: the row tiles of a panel and range of weights follow one another
+  // A tile: the row tiles of a panel and range of weights follow one another. Workgroups go round the XCDs, so that of eight ranges an
+  // XCD has one, and its L2 that part of the rows. Of four it would have one too, in every other panel, and where panels lie whole
+  // megabytes apart (128 rows of 4096) their loads come a quarter slower: there neighbouring pairs of panels start their ranges one on
+  // (8192 x 4096 at 17 / 48 / 97 rows 19.7 / 21.1 / 25.8 us, so 16.0 / 18.6 / 22.7, 8192 x 8192 31.7 / 32.8 / 39.5, 26.2 / 28.8 / 34.7;
+  // elsewhere 3 % either way, with eight ranges up to 17 % slower).
+  const bool turned = g.ranges == 4 && ((unsigned)BN * (unsigned)g.K & ((1u << 19) - 1)) == 0;
   auto place = [&](int tile, int& m0, int& z, int& n) {
     const int in = g.m_part ? (int)__umulhi((unsigned)tile, g.m_part) : tile;
     m0 = (tile - in * g.m_tiles) * BM;
     n = g.z_part ? (int)__umulhi((unsigned)in, g.z_part) : in;
     z = in - n * g.ranges;
+    if (turned) z = (z + n / 2) & 3;
   };
 
   // The carried norm's partial sums of squares. Up to eight a row (a product cut into ranges wrote them, one for 1024 columns): lane group

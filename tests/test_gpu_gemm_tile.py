@@ -250,3 +250,19 @@ def test_rows_too_long_for_the_widest_tile(N):
         # sums of deviation 1, rounded K times at most by up to 2^-25 in either direction: eight deviations of their sum, a fifth of
         # what a lost stage of 64 k would show
         assert ((out[:, part].double() - want).abs() <= 8 * math.sqrt(K) * 2 ** -25 * (1 + want.abs())).all()
+
+
+@pytest.mark.parametrize("M", [17, 64, 128])
+@pytest.mark.parametrize("N,K", [(8192, 4096), (4096, 4104), (7168, 4104), (6144, 4096)])
+def test_four_ranges_each_in_its_plane(M, N, K):
+    """Four ranges, which panels of weights start one on from one another, land where the adding kernels look for them."""
+    x, w, _ = operands(M, N, K, M + N)
+    S = int(kernels.library.load().ra_gemm_wide_ranges(M, N, K))
+    assert S == 4
+    parts = torch.full((S, M, N), float("nan"), device=DEV)
+    kernels.library.call("ra_gemm_wide_partial", x.data_ptr(), w.data_ptr(), parts.data_ptr(), parts.numel(), M, N, K, K, 0,
+                         torch.cuda.current_stream().cuda_stream)
+    each = (-(-K // S) + 63) // 64 * 64
+    for z in range(S):
+        xs, ws = x[:, z * each:(z + 1) * each], w[:, z * each:(z + 1) * each]
+        assert ((parts[z].double() - xs.double() @ ws.double().T).abs() <= bound(xs, ws, each)).all()
