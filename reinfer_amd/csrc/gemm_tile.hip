@@ -70,9 +70,10 @@ __device__ __forceinline__ float gt_exp(float x) {
 
 __device__ __forceinline__ int gt_key(int row) { return (row >> 1) & 7; }
 
-// BMT x TN tiles of 16 rows x 16 features, shared out over WM x WN waves. QUICK: results whose rows start at whole pieces, no bias and, with
-// the gate, in bfloat16, so that an end is a few stores; what is left takes any end, in four times the code (a launch runs each line of
-// its code for the first time, from memory: with one end for all, 19456 x 2560 with its gate took 30.5 us at 97 rows, so 28.8).
+// BMT x TN tiles of 16 rows x 16 features, shared out over WM x WN waves. QUICK: results whose rows start at whole pieces, a bias where
+// they are plain only and, with the gate, in bfloat16, so that an end is a few stores; what is left takes any end, in four times the code
+// (a launch runs each line of its code for the first time, from memory: with one end for all, 19456 x 2560 with its gate took 30.5 us at
+// 97 rows, so 28.8; with a bias 51200 x 5120 at 17 rows 101.7, so 81.5, without one 82.3 and 81.1).
 template <int BMT, int TN, int WM, int WN, int EPI, bool QUICK, bool STREAM>
 __global__ void __launch_bounds__(64 * WM * WN) gemm_tile_kernel(TileArgs g) {
   constexpr int NW = WM * WN, MT = BMT / WM, NT = TN / WN;
@@ -287,6 +288,14 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_tile_kernel(TileArgs g) {
       const __amdgpu_buffer_rsrc_t cr = __builtin_amdgcn_make_buffer_rsrc(
           (char*)g.c + ((size_t)(EPI == GT_PART ? z : 0) * g.M + m0) * g.ldc * SIZE, 0,
           (int)(((size_t)(left - 1) * g.ldc + cols) * SIZE), 0x00020000);
+      constexpr bool PLAIN = EPI == GT_PLAIN || EPI == GT_PLAIN_HALF;
+      f32x4_t bias[PLAIN ? NT : 1];
+      if (PLAIN && g.end.bias) {
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) bias[PLAIN ? i : 0][e] = to_f32(g.end.bias[min(n0 + (wn * NT + i) * 16 + q * 4 + e, cols - 1)]);
+      }
 #pragma unroll
       for (int j = 0; j < MT; ++j) {
         const int row = (wm * MT + j) * 16 + r;
@@ -297,6 +306,7 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_tile_kernel(TileArgs g) {
           const unsigned to = (row < left && n < cols && (EPI != GT_GATED || q < 2)) ? ((unsigned)row * (unsigned)g.ldc + n) * SIZE : 0xFFFFFFF0u;
           f32x4_t v = acc[i][j];
           if (SUMS) v *= rstd;
+          if (PLAIN && g.end.bias) v += bias[PLAIN ? i : 0];
           if constexpr (EPI == GT_GATED) {   // rows 0-7 of a tile are gate, 8-15 up of the same features: those sit two groups on
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
@@ -511,7 +521,7 @@ int ra_tile_product(int epilogue, const RaTilePlan& plan, const void* A, int lda
   if (!end.in_ss) end.in_parts = 0;
   const int cols = epilogue == GT_GATED ? N / 2 : N;
   const bool half = end.half && (epilogue == GT_PLAIN || epilogue == GT_GATED);
-  const bool quick = !end.bias && cols % 4 == 0 && ldc % 4 == 0 && ldc <= (1 << 22) && (uintptr_t)C % (half ? 8 : 16) == 0 &&
+  const bool quick = (!end.bias || epilogue == GT_PLAIN) && cols % 4 == 0 && ldc % 4 == 0 && ldc <= (1 << 22) && (uintptr_t)C % (half ? 8 : 16) == 0 &&
                      (half || epilogue != GT_GATED);
   TileArgs g = {(const bf16_t*)A, (const bf16_t*)W, C, M, N, K, lda, ldc, 0, 0, plan.ranges, plan.range_k, 0, 0, end};
   switch (epilogue) {

@@ -266,3 +266,21 @@ def test_four_ranges_each_in_its_plane(M, N, K):
     for z in range(S):
         xs, ws = x[:, z * each:(z + 1) * each], w[:, z * each:(z + 1) * each]
         assert ((parts[z].double() - xs.double() @ ws.double().T).abs() <= bound(xs, ws, each)).all()
+
+
+@pytest.mark.parametrize("M", [17, 33, 64])
+@pytest.mark.parametrize("N,K", [(32768, 1024), (40000, 264), (51201, 128), (24580, 320)])
+def test_a_bias_on_uncut_tiles(M, N, K):
+    """In the short end, where rows start at whole pieces, and in the other: off them by the stride, by N, by the result's address."""
+    x, w, g = operands(M, N, K, M + N)
+    biases = torch.randn(N + 1, device=DEV, generator=g).to(torch.bfloat16)
+    ref, err = x.double() @ w.double().T, bound(x, w, K)
+    for kind, ulp in ((torch.float32, 2.0 ** -23), (torch.bfloat16, 2.0 ** -8)):
+        for wide, first in ((N + 8, 0), (N + 3, 0), (N + 8, 1)):
+            bias = biases[first:first + N]                  # its address is off whole pieces too
+            buf = torch.full((M, wide), float("nan"), device=DEV, dtype=kind)
+            out = buf[:, first:first + N]
+            ops()._few_rows("linear output", x, w, bias, out, 0, M, N, K, True)
+            want = ref + bias.double()
+            assert ((out.double() - want).abs() <= err + want.abs() * ulp).all()
+            assert torch.isnan(buf[:, :first]).all() and torch.isnan(buf[:, first + N:]).all()
