@@ -590,7 +590,7 @@ class HipKernels:
 
     # How the decode kernel is cut, in keys of head size 128 (what counts is the bytes of a (token, KV head) pair): below
     DECODE_SHORT_CTX = 768      # one large workgroup a pair, where the chip holds them all
-    DECODE_LONG_CTX = 4096      # from here on large workgroups and their chunks, where the chip holds one a pair
+    DECODE_LONG_CTX = 4096      # from here on (8 pairs and fewer: beyond it) large workgroups and their chunks, where the chip holds one a pair
     DECODE_ONE_CTX = 1024       # one small workgroup a pair, where there are more pairs than that
     DECODE_FILL_ONE = 0.6       # pairs that the chip holds as large workgroups, from this share of them on one each
     DECODE_FILL = 0.9           # of the last round of large workgroups that more pairs must fill
@@ -615,7 +615,8 @@ class HipKernels:
         few pairs of (token, KV head) are cut until their chunks fill the chip once, and where a large workgroup a pair
         fills more than half of it there is nothing to merge, but over long contexts from DECODE_FILL_ONE on alone (17 tokens
         of 2000 keys one / five small chunks 30.0 / 32.2 us, of 6000 79.0 / 73.6; with just half of it two large chunks:
-        16 of 1000 17.4 / 19.7, of 1500 24.1 / 22.8, of 6000 77.7 / 66.8). Over 7 cuts of each form, of 1 to 64 tokens of 300 to
+        16 of 1000 17.4 / 19.7, of 1500 24.1 / 22.8, of 6000 77.7 / 66.8). 4,096 keys of 2 to 8 pairs are 16 small chunks, 11.4 to
+        12.9 us, 16 large ones 11.4 to 13.5, of 16 and 32 pairs 12.9 and 16.3 small, 12.9 and 15.4 large. Over 7 cuts of each form, of 1 to 64 tokens of 300 to
         16,000 keys, this rule is 1 to 3 % behind the best on average (32 heads over 8 of 128 and of 64, 28 over 4, 16 and 64
         over 8, 8 over 8 of 96), 5 % with 14 over 2 of 64; 15 to 30 % at 1 to 12 pairs over 6,000 keys and more, where 16
         large chunks are best."""
@@ -630,7 +631,7 @@ class HipKernels:
             if pairs >= self.DECODE_FILL_ONE * wide or ctx <= self.DECODE_SHORT_CTX \
                     or half and (ctx <= self.DECODE_ONE_CTX if room > 1 else ctx < self.DECODE_LONG_CTX):
                 return 512, 1, 12
-            if room > 1 and (half or ctx >= self.DECODE_LONG_CTX):
+            if room > 1 and (half or ctx >= self.DECODE_LONG_CTX + (pairs <= 8)):
                 return 256, min(room, -(-max_ctx // 256)), 12
         elif ctx > self.DECODE_ONE_CTX and pairs >= self.DECODE_FILL * (-(-pairs // wide) * wide):
             return 512, 1, 12

@@ -47,3 +47,12 @@ def test_pairs_that_fill_half_of_the_chip():
     assert cut(16, 1024) == (1, 12) and cut(16, 1025) == (2, 12) and cut(16, 16384) == (2, 12)
     assert cut(17, 4095) == (1, 12) and cut(17, 4096) == (768 // 136, 4)
     assert cut(20, 4096) == (1, 12) and cut(32, 16384) == (1, 12)
+
+
+@pytest.mark.parametrize("Hq,Hkv", [(20, 2), (28, 4), (64, 8)])
+def test_few_pairs_of_four_thousand_keys(Hq, Hkv):
+    """A captured step's bucket of 2,049 to 4,096 keys: small chunks for up to 8 pairs, large ones from there and from the next bucket on."""
+    chip = Chip()
+    assert chip.decode_chunk(1, Hq, Hkv, 128, 4096)[1:] == (16, 4)
+    assert chip.decode_chunk(1, Hq, Hkv, 128, 8192)[2] == 12
+    assert chip.decode_chunk(16 // Hkv, Hq, Hkv, 128, 4096)[2] == 12
