@@ -7,7 +7,11 @@
 #define FP_KT 64          // keys per round
 #define FPW_D 256         // the wide form: head size,
 #define FPW_WAVES 4       // waves of a workgroup
-#define FPW_NC 2          // and column tiles of a wave
+#define FPW_NC 2          // column tiles of a wave,
+// and keys up to which the other form's eight waves are ahead (the same bits). There / here, us, 16 query heads on 1 and on 8 KV heads:
+// one prompt of 5 tokens 7.9 / 10.6, 7.7 / 10.4; of 64 12.7 / 13.2, 11.5 / 13.1; of 112 15.9 / 16.1, 14.7 / 14.6; of 128 17.4 / 16.1,
+// 15.8 / 15.9; of 192 21.6 / 18.6, 20.2 / 18.6; a hundred of 100 tokens 99.7 / 106.9, 102.5 / 104.7
+#define FPW_FEW_KEYS 112
 
 __device__ __forceinline__ float fp_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 

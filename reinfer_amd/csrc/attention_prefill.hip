@@ -588,7 +588,7 @@ static int fp_launch(const void* q, int q_stride, void* out, int out_stride,
                      const void* kcache, const void* vcache, const int* block_tables,
                      int max_blocks, const int* tile_info, int n_tiles, int block_size,
                      int Hq, int Hkv, int d, float scale, int window, int aligned, int keep, const FpSplit& sp,
-                     const int* merge_info, int n_merge, const RaScoreMod& mod, const RaHeadOut& ho, hipStream_t stream) {
+                     const int* merge_info, int n_merge, const RaScoreMod& mod, const RaHeadOut& ho, int longest, hipStream_t stream) {
   RA_CHECK((mod.r1 == nullptr) == (mod.r2 == nullptr) && mod.softcap >= 0.f,
            "attention_prefill: the distance term takes both per-head vectors, the cap is not negative");
   RA_CHECK(ho.gate == nullptr || ho.gate_stride >= Hq, "attention_prefill: gate rows of %d for %d heads", ho.gate_stride, Hq);
@@ -629,7 +629,7 @@ static int fp_launch(const void* q, int q_stride, void* out, int out_stride,
   } while (0)
   if (d <= 64) RA_FP(64, 2);
   else if (d <= 128) RA_FP(128, 2);
-  else if (d < FPW_D) RA_FP_GO(256, 1, false);
+  else if (d < FPW_D || (longest > 0 && longest <= FPW_FEW_KEYS)) RA_FP_GO(256, 1, false);
   else ra_prefill_wide(n_tiles * gy, (const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)kcache,
                        (const bf16_t*)vcache, block_tables, max_blocks, tile_info, block_size, Hq, Hkv, sh.hg, scale_log2, window,
                        aligned, keep, sp, scale, mod, ho, stream);
@@ -658,7 +658,7 @@ extern "C" int ra_attention_prefill(const void* q, int q_stride, void* out, int 
                                     int Hq, int Hkv, int d, float scale, int window, hipStream_t stream) {
   return ra_attention_prefill_mod(q, q_stride, out, out_stride, kcache, vcache, block_tables, max_blocks, tile_info,
                                   n_tiles, block_size, Hq, Hkv, d, scale, window, 0, 0, 0.f, nullptr, nullptr, nullptr,
-                                  nullptr, 0, stream);
+                                  nullptr, 0, 0, stream);
 }
 
 // The same with the scores changed before the softmax: softcap > 0 caps them by a tanh, r1 / r2 (one float a query
@@ -669,12 +669,12 @@ extern "C" int ra_attention_prefill_mod(const void* q, int q_stride, void* out, 
                                         int max_blocks, const int* tile_info, int n_tiles, int block_size,
                                         int Hq, int Hkv, int d, float scale, int window, int aligned, int keep,
                                         float softcap, const float* r1, const float* r2, const float* sink,
-                                        const void* gate, int gate_stride, hipStream_t stream) {
+                                        const void* gate, int gate_stride, int longest, hipStream_t stream) {
   const FpSplit none = {};
   const RaHeadOut ho = {sink, gate, gate_stride};
   const RaScoreMod mod = {softcap, r1, r2};
   return fp_launch(q, q_stride, out, out_stride, kcache, vcache, block_tables, max_blocks, tile_info, n_tiles,
-                   block_size, Hq, Hkv, d, scale, window, aligned, keep, none, nullptr, 0, mod, ho, stream);
+                   block_size, Hq, Hkv, d, scale, window, aligned, keep, none, nullptr, 0, mod, ho, longest, stream);
 }
 
 // The same with query tiles cut by keys: `ranges` holds three ints a listed tile (first key and one past the
@@ -711,5 +711,5 @@ extern "C" int ra_attention_prefill_split_mod(const void* q, int q_stride, void*
   sp.part_o = part_o;
   sp.part_ml = part_ml;
   return fp_launch(q, q_stride, out, out_stride, kcache, vcache, block_tables, max_blocks, tile_info, n_tiles,
-                   block_size, Hq, Hkv, d, scale, window, aligned, keep, sp, merge_info, n_merge, mod, ho, stream);
+                   block_size, Hq, Hkv, d, scale, window, aligned, keep, sp, merge_info, n_merge, mod, ho, 0, stream);
 }

@@ -11,7 +11,7 @@
 // heads, 2000 tokens 140 -> 93; 16 and 4, 7000 tokens 896 -> 562. At 128 elements the same scheme is slower than eight waves (64 and 8 heads, 7901 tokens 1035 ->
 // 1483 us), and so are eight waves that take turns at products and exponentials between barriers (1100). Sizes of
 // 129 to 255 stay with the other form too: padded to 256 this one reads and loads more than they need (192 elements, 16 and 8 heads,
-// 2000 tokens 119 there, 127 here; 144 elements, 300 tokens 22 and 28).
+// 2000 tokens 119 there, 127 here; 144 elements, 300 tokens 22 and 28). So do steps of few keys (FPW_FEW_KEYS).
 #include <type_traits>
 #include <utility>
 #include "attention_prefill.h"

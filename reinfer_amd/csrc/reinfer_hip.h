@@ -5,7 +5,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
-#define RA_ABI_VERSION 33
+#define RA_ABI_VERSION 34
 
 #ifdef __cplusplus
 extern "C" {
@@ -196,11 +196,12 @@ int ra_attention_prefill_split(const void* q, int q_stride, void* out, int out_s
                                float* part_ml, int block_size, int Hq, int Hkv, int d, float scale, int window,
                                hipStream_t stream);
 
+// longest: keys that a query of these tiles sees at most, 0 where the caller does not say (a hint: the kernel for few keys).
 int ra_attention_prefill_mod(const void* q, int q_stride, void* out, int out_stride, const void* kcache,
                              const void* vcache, const int* block_tables, int max_blocks, const int* tile_info,
                              int n_tiles, int block_size, int Hq, int Hkv, int d, float scale, int window,
                              int aligned, int keep, float softcap, const float* r1, const float* r2, const float* sink,
-                             const void* gate, int gate_stride, hipStream_t stream);
+                             const void* gate, int gate_stride, int longest, hipStream_t stream);
 int ra_attention_prefill_split_mod(const void* q, int q_stride, void* out, int out_stride, const void* kcache,
                                    const void* vcache, const int* block_tables, int max_blocks, const int* tile_info,
                                    int n_tiles, const int* ranges, const int* merge_info, int n_merge, float* part_o,

@@ -15,7 +15,7 @@ import torch  # noqa: F401  (loads the HIP runtime the library links against)
 
 from ..csrc import build as _build
 
-ABI_VERSION = 33
+ABI_VERSION = 34
 
 
 class KernelLibraryError(RuntimeError):
@@ -86,7 +86,7 @@ _SIGNATURES = {
     "ra_normed_mean": [P, P, I, I, F, I, I, P, P, F, P],
     "ra_attention_plain_mod": [P, I, P, I, P, P, I, P, I, P, P, P, I, P, I, I, I, I, I, F, I, I, I, F, P, P, P, P, I, P],
     "ra_attention_decode_mod": [P, I, P, I, P, P, P, I, P, P, P, I, I, I, I, I, F, I, I, I, I, I, I, P, P, F, P, P, P, P, I, I, P],
-    "ra_attention_prefill_mod": [P, I, P, I, P, P, P, I, P, I, I, I, I, I, F, I, I, I, F, P, P, P, P, I, P],
+    "ra_attention_prefill_mod": [P, I, P, I, P, P, P, I, P, I, I, I, I, I, F, I, I, I, F, P, P, P, P, I, I, P],
     "ra_attention_prefill_split_mod": [P, I, P, I, P, P, P, I, P, I, P, P, I, P, P, I, I, I, I, F, I, I, I, F, P, P, P, P, I, P],
     "ra_act_mul_bounded": [P, P, I, I, I, I, I, F, P],
     "ra_decay_scan": [P, I, I, I, I, I, P, P, c_long, P, P, P, I, I, I, I, I, I, P, P],

@@ -323,7 +323,8 @@ class HipKernels:
                 self.attention_prefill(q, q_stride, out, kcache, vcache, batch, num_heads, num_kv_heads,
                                        head_dim, scale, window, group, plan["tiles"], plan["n_tiles"],
                                        plan.get("ranges"), plan.get("merge"), plan.get("n_merge", 0),
-                                       plan.get("n_slots", 0), **changed)
+                                       plan.get("n_slots", 0), longest=min(plan["longest"], window + keep + tile if window else plan["longest"]),
+                                       **changed)
             else:
                 self.attention_plain(q, q_stride, out, kcache, vcache, batch, num_heads, num_kv_heads,
                                      head_dim, scale, window, group, plan["prefill_list"], plan["n_prefill"], **changed)
@@ -538,6 +539,7 @@ class HipKernels:
             "ranges": dev[o_ranges:o_merge] if merge else None,
             "merge": dev[o_merge:] if merge else None,
             "n_merge": len(merge) // 4, "n_slots": n_slots,
+            "longest": max((q0 + n for _, _, n, q0 in tiles), default=0),
             "tile": tile,
         }
         batch.extra[("attention_plan", tile, room, halves, fixed, chunk)] = plan
@@ -704,9 +706,10 @@ class HipKernels:
     def attention_prefill(self, q, q_stride, out, kcache, vcache, batch, num_heads, num_kv_heads, head_dim,
                           scale, window, group, tiles, n_tiles, ranges=None, merge=None, n_merge: int = 0,
                           n_slots: int = 0, mod=(0.0, None, None), keep: int = 0, aligned: bool = False,
-                          head_out=(None, None, 0)) -> None:
+                          head_out=(None, None, 0), longest: int = 0) -> None:
         """``tiles``: four ints a listed query tile (request row, first token row, queries, first
-        position). With ``ranges`` (three ints a listed tile: first key, one past the last, the part's
+        position). ``longest``: keys that any of their queries sees at most (0: not said), for the choice
+        of kernel. With ``ranges`` (three ints a listed tile: first key, one past the last, the part's
         slot or -1) some tiles are listed in several parts by keys, and ``merge`` (four ints a cut tile:
         first token row, queries, first slot, parts) says which to add up."""
         tables = self._check_attention(q, q_stride, out, kcache, vcache, batch, num_heads, num_kv_heads,
@@ -734,7 +737,7 @@ class HipKernels:
         library.call("ra_attention_prefill_mod", q.data_ptr(), q_stride, out.data_ptr(), out.stride(0),
                      kcache.data_ptr(), vcache.data_ptr(), tables.data_ptr(), tables.shape[1],
                      tiles.data_ptr(), int(n_tiles), kcache.shape[2] * 16, num_heads, num_kv_heads, head_dim,
-                     float(scale), int(window), int(aligned), int(keep), mod[0], mod[1], mod[2], *head_out, _stream())
+                     float(scale), int(window), int(aligned), int(keep), mod[0], mod[1], mod[2], *head_out, int(longest), _stream())
 
     # ---------------------------------------------------------------- linear
     def linear(self, x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor,

@@ -1236,3 +1236,23 @@ def test_column_bits_of_a_tile_mean_nothing_where_a_wave_holds_one(d):
         got.append(out)
     assert all(torch.equal(got[0], o) for o in got[1:])
     close(got[0], attention_reference(q, kc, vc, tables, q_lens, starts, Hq, Hkv, d, d ** -0.5, 0), 2 ** -7)
+
+
+@pytest.mark.parametrize("Hq,Hkv", [(16, 1), (4, 2), (9, 3)])
+@pytest.mark.parametrize("q_lens,starts", [([5], [0]), ([60, 9], [40, 100]), ([112], [0]), ([113], [0])])
+def test_prompt_attention_of_few_keys_with_heads_of_256(monkeypatch, Hq, Hkv, q_lens, starts):
+    """The form of eight waves up to 112 keys, the wide one from 113 on: the same bits, and what the step tells of its longest context."""
+    d, T, said, call = 256, sum(q_lens), [], kernels.library.call
+    monkeypatch.setattr(kernels.library, "call", lambda name, *args: (said.append((name, args[-2])), call(name, *args))[1])
+    q, kc, vc, tables = make_paged_case("bfloat16", Hq, Hkv, d, q_lens, starts, seed=T)
+    args = (q.view(T, Hq * d), Hq * d), (kt(kc), vt(vc)), (Hq, Hkv, d, d ** -0.5, 0, 0)
+    out = torch.full((T, Hq * d), float("nan"), device=DEV, dtype=torch.bfloat16)
+    batch = FakeBatch(q_lens, starts, tables)
+    ops().attention(*args[0], out, *args[1], batch, *args[2])
+    assert said == [("ra_attention_prefill_mod", max(a + b for a, b in zip(q_lens, starts)))]
+    plan = next(p for k, p in batch.extra.items() if isinstance(k, tuple) and k[0] == "attention_plan")
+    for longest in (0, 112, 113):
+        again = torch.full((T, Hq * d), float("nan"), device=DEV, dtype=torch.bfloat16)
+        ops().attention_prefill(*args[0], again, *args[1], batch, *args[2], plan["tiles"], plan["n_tiles"], longest=longest)
+        assert torch.equal(out, again)
+    close(out, attention_reference(q, kc, vc, tables, q_lens, starts, Hq, Hkv, d, d ** -0.5, 0), 2 ** -7)

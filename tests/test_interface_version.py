@@ -8,7 +8,7 @@ from reinfer_amd.csrc import build
 from reinfer_amd.kernels import library
 
 # the prototypes' digest that goes with the version: where this fails, the interface has changed and needs the next version
-VERSION, DIGEST = 33, "ee17f59afa0ce07a"
+VERSION, DIGEST = 34, "8c522cd3c913a08c"
 
 
 def prototypes():
