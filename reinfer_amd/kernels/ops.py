@@ -320,11 +320,13 @@ class HipKernels:
                                      head_dim, scale, window, group, plan["decode_list"], plan["n_decode"], **changed)
         if plan["n_tiles"]:
             if pre_ok:
+                said = {}
+                if head_dim == 256 and plan["ranges"] is None:      # the one size with two kernels to choose from
+                    said["longest"] = min(plan["longest"], window + keep + tile) if window else plan["longest"]
                 self.attention_prefill(q, q_stride, out, kcache, vcache, batch, num_heads, num_kv_heads,
                                        head_dim, scale, window, group, plan["tiles"], plan["n_tiles"],
                                        plan.get("ranges"), plan.get("merge"), plan.get("n_merge", 0),
-                                       plan.get("n_slots", 0), longest=min(plan["longest"], window + keep + tile if window else plan["longest"]),
-                                       **changed)
+                                       plan.get("n_slots", 0), **said, **changed)
             else:
                 self.attention_plain(q, q_stride, out, kcache, vcache, batch, num_heads, num_kv_heads,
                                      head_dim, scale, window, group, plan["prefill_list"], plan["n_prefill"], **changed)
